@@ -9,7 +9,7 @@ public entry point runs it:
   logits have nothing in common.
 * ``generate``: the whole greedy generation of the 32-bit model, prompts in, tokens and logits out.
 
-``sizes`` names layer sizes of ``SIZES`` below.  Models have the full depth where three of them fit the card, and fewer layers of
+``sizes`` names layer sizes given below.  Models have the full depth where three of them fit the card, and fewer layers of
 the full size elsewhere.  Weights are random, as ``from_config`` draws them.  Routed experts are in no case: in bfloat16 the
 choice between two experts of nearly the same score is an accident, and outputs of two correct implementations cannot be compared.
 """
