@@ -1,82 +1,365 @@
-// C[M,N] = act(A[M,K] . W[N,K]^T + bias) + add1 + add2 in true 32-bit: plain FMA on
-// the vector units, no matrix-core mode of reduced precision.  Every output element
-// sums its K products in the order k = 0 .. K-1 in one accumulator, whatever M is and
-// wherever the element lies in the grid, so a row's result is bitwise the same alone
-// and in any batch.  The 32-bit path of the whole model runs its projections, MLP and
-// output head through this kernel.
+// C[M,N] = act(A[M,K] . W[N,K]^T + bias) + add1 + add2 in true 32-bit, on the 32-bit matrix instruction
+// (v_mfma_f32_16x16x4_f32: products and sums in 32-bit, 154 TFLOP/s dense on this chip; the vector units give half).
+// The 32-bit path of the whole model runs its projections, feed-forwards and output head through here.
+//
+// Order of summation.  A row's result is bitwise the same alone and in any batch, so every kernel here sums the products
+// of an output in one order, which K alone decides: K is walked in blocks of sixteen elements (the last one filled up with
+// zeros), the blocks are cut into up to eight segments of equal length, a segment is one chain of matrix instructions
+// (instruction j of a block takes elements j, 4 + j, 8 + j and 12 + j of it, so that a lane's four operands are sixteen
+// consecutive bytes of a row), and the segments' sums are added in order.  Where a row lies in the grid, which kernel runs
+// and how many workgroups share the segments changes nothing.
+//
+// Measured at 4,544 / 18,176 features (one kernel of 64 x 64 tiles on the vector units before): one row of A 986 -> 56 us a
+// product on average (28 us for 83 MB, 71 us = 4.7 TB/s for 330 MB); 2,053 rows 26 -> 98 to 110 TFLOP/s.
+//
+// Three ways to the same numbers, by what bounds them:
+//   few rows (M <= 64): every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight
+//     waves a segment each; W goes from memory straight into the instruction's operands, the sums meet in LDS.
+//   many rows: tiles of 128 x 128 or 64 x 64 through two LDS buffers, bound by the matrix instruction.
+//   in between, or N small: too few tiles to fill the chip, so the segments of a tile are shared out over workgroups, whose
+//     sums go to memory and are added by a small launch.
 #include "common.h"
 #include "pta_kernels.h"
 
-#define G_BM 64
-#define G_BN 64
-#define G_BK 16
+typedef float f32x4 __attribute__((ext_vector_type(4)));
 
-__global__ __launch_bounds__(256) void gemm_f32_kernel(float* __restrict__ C, const float* __restrict__ A,
-                                                       const float* __restrict__ W,
-                                                       const float* __restrict__ bias,
-                                                       const float* __restrict__ add1,
-                                                       const float* __restrict__ add2, int M, int N, int K,
-                                                       int act) {
-    __shared__ float As[G_BK][G_BM + 4];
-    __shared__ float Ws[G_BK][G_BN + 4];
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-    const int m0 = blockIdx.y * G_BM, n0 = blockIdx.x * G_BN;
-    float acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = 0.f;
+#define SEGS 8          // segments of K, at most
+#define SKINNY_ROWS 64  // rows of A up to which the kernel for few rows runs
 
-    for (int k0 = 0; k0 < K; k0 += G_BK) {
+struct F32Epilogue {
+    const float* bias;
+    const float* add1;
+    const float* add2;
+    int act;
+};
+
+__device__ __forceinline__ float finish(float v, const F32Epilogue& e, int n, long at) {
+    if (e.bias) v += e.bias[n];
+    if (e.act) v = apply_act(v, e.act);
+    if (e.add1) v += e.add1[at];
+    if (e.add2) v += e.add2[at];
+    return v;
+}
+
+// How rows are read: element by element; sixteen bytes at a time (rows sixteen-byte aligned, K a multiple of 4); the same
+// without a look at the end (K a multiple of 16, what every published size is).
+enum RowLoads { ROW_ELEMENTS, ROW_VECTORS, ROW_WHOLE };
+
+// four consecutive elements of a row from k on, zeros beyond K (ROW_WHOLE: k + 4 <= K is the caller's)
+template <int ROWS>
+__device__ __forceinline__ f32x4 load4(const float* row, int k, int K) {
+    if (ROWS == ROW_WHOLE) return *(const f32x4*)(row + k);
+    f32x4 v = {0.f, 0.f, 0.f, 0.f};
+    if (ROWS == ROW_VECTORS) {
+        if (k < K) v = *(const f32x4*)(row + k);
+    } else {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + i * 256;
-            const int r = idx >> 4, kk = idx & 15;
-            const int gk = k0 + kk;
-            const int gm = m0 + r, gn = n0 + r;
-            As[kk][r] = (gm < M && gk < K) ? A[(long)gm * K + gk] : 0.f;
-            Ws[kk][r] = (gn < N && gk < K) ? W[(long)gn * K + gk] : 0.f;
+        for (int j = 0; j < 4; ++j)
+            if (k + j < K) v[j] = row[k + j];
+    }
+    return v;
+}
+
+__host__ __device__ static inline int seg_blocks(int K) { return ((K + 15) / 16 + SEGS - 1) / SEGS; }
+
+// ---- few rows ---------------------------------------------------------------------------------------------------------
+// CT: tiles of sixteen rows of A, RT: tiles of sixteen rows of W.  D blocks of K are asked for while the D before them are
+// multiplied: at K = 4,544 and one row of A a compute unit then has some 60 KB on its way.
+template <int CT, int RT, int D, int ROWS>
+__global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel(
+    float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, F32Epilogue epi, int M, int N, int K) {
+    __shared__ f32x4 part[SEGS][RT * CT][64];
+    const int lane = threadIdx.x & 63, seg = threadIdx.x >> 6;
+    const int r16 = lane & 15, kq = 4 * (lane >> 4);
+    // the rows of W are shared out evenly: a launch takes as long as the compute unit with the most of them
+    const int n0 = (int)((long)blockIdx.x * N / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * N / gridDim.x);
+    const int m0 = blockIdx.y * SKINNY_ROWS;
+    const int nb = (K + 15) / 16, sb = seg_blocks(K);
+    const int b0 = seg * sb, b1 = min(nb, b0 + sb);
+    const float* wr[RT];
+    const float* xr[CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r) wr[r] = W + (long)min(n0 + 16 * r + r16, n1 - 1) * K;  // rows past the end: read again, not kept
+#pragma unroll
+    for (int c = 0; c < CT; ++c) xr[c] = A + (long)min(m0 + 16 * c + r16, M - 1) * K;
+    f32x4 acc[RT][CT];
+#pragma unroll
+    for (int r = 0; r < RT; ++r)
+#pragma unroll
+        for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    f32x4 w[2][D][RT], x[2][D][CT];
+    auto fetch = [&](int buf, int b) {
+#pragma unroll
+        for (int i = 0; i < D; ++i) {
+            const int k = 16 * min(b + i, nb - 1) + kq;  // past the segment: read again, not used
+#pragma unroll
+            for (int r = 0; r < RT; ++r) w[buf][i][r] = load4<ROWS>(wr[r], k, K);
+#pragma unroll
+            for (int c = 0; c < CT; ++c) x[buf][i][c] = load4<ROWS>(xr[c], k, K);
         }
-        __syncthreads();
+    };
+    auto multiply = [&](int buf, int b) {
 #pragma unroll
-        for (int kk = 0; kk < G_BK; ++kk) {
-            float a[4], w[4];
+        for (int i = 0; i < D; ++i) {
+            if (b + i < b1) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) { a[i] = As[kk][ty * 4 + i]; w[i] = Ws[kk][tx * 4 + i]; }
+                for (int j = 0; j < 4; ++j)
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+                    for (int r = 0; r < RT; ++r)
 #pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], w[j], acc[i][j]);
+                        for (int c = 0; c < CT; ++c)
+                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[buf][i][r][j], x[buf][i][c][j], acc[r][c], 0, 0, 0);
+            }
         }
-        __syncthreads();
+    };
+    if (b0 < b1) {
+        fetch(0, b0);
+        for (int b = b0; b < b1; b += 2 * D) {
+            fetch(1, b + D);
+            multiply(0, b);
+            fetch(0, b + 2 * D);
+            multiply(1, b + D);
+        }
     }
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int gm = m0 + ty * 4 + i;
-        if (gm >= M) continue;
+    for (int r = 0; r < RT; ++r)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int gn = n0 + tx * 4 + j;
-            if (gn >= N) continue;
-            float v = acc[i][j];
-            if (bias) v += bias[gn];
-            if (act) v = apply_act(v, act);
-            const long o = (long)gm * N + gn;
-            if (add1) v += add1[o];
-            if (add2) v += add2[o];
-            C[o] = v;
+        for (int c = 0; c < CT; ++c) part[seg][r * CT + c][lane] = acc[r][c];
+    __syncthreads();
+    const int used = (nb + sb - 1) / sb;
+    for (int i = threadIdx.x; i < RT * CT * 64; i += 512) {
+        const int t = i >> 6, l = i & 63;
+        f32x4 v = part[0][t][l];
+        for (int s = 1; s < used; ++s) {
+            const f32x4 p = part[s][t][l];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] += p[j];
+        }
+        const int m = m0 + 16 * (t % CT) + (l & 15);
+        const int n = n0 + 16 * (t / CT) + 4 * (l >> 4);
+        if (m < M) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < n1) C[(long)m * N + n + j] = finish(v[j], epi, n + j, (long)m * N + n + j);
         }
     }
 }
 
+// ---- many rows ----------------------------------------------------------------------------------------------------------
+// A workgroup of four waves, two by two, on a tile of T x T.  A row of a tile is 32 elements of K in LDS, 36 apart: the eight
+// lanes that read together (rows next to each other, sixteen bytes each) then cover every bank once.
+#define BK 32
+#define PITCH 36
+
+template <int T, int ROWS, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ A,
+                                                               const float* __restrict__ W, F32Epilogue epi, int M, int N,
+                                                               int K, int tiles_m, int tiles_n) {
+    constexpr int F = T / 32;        // tiles of sixteen rows per wave and side
+    constexpr int L = T * 8 / 256;   // sixteen-byte loads per thread and side
+    __shared__ float As[2][T * PITCH];
+    __shared__ float Ws[2][T * PITCH];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int r16 = lane & 15, kq = 4 * (lane >> 4);
+    // workgroups go to the eight dies in turn: give each die a run of tiles that share rows of W, which its L2 then holds
+    const int tiles = tiles_m * tiles_n;
+    const int per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * T, n0 = (tile / tiles_m) * T;
+    const int wn = (wave & 1) * (T / 2), wm = (wave >> 1) * (T / 2);
+    const int nb = (K + 15) / 16, sb = seg_blocks(K);
+    // SPLIT: this workgroup's share of the segments
+    const int used = (nb + sb - 1) / sb;
+    const int s0 = SPLIT ? (int)((long)blockIdx.y * used / gridDim.y) : 0;
+    const int s1 = SPLIT ? (int)((long)(blockIdx.y + 1) * used / gridDim.y) : used;
+    const int b_first = s0 * sb, b_last = min(nb, s1 * sb);
+
+    f32x4 acc[F][F], total[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    f32x4 ra[L], rw[L];
+    const float* pa[L];
+    const float* pw[L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+        const int row = (tid + 256 * i) >> 3;
+        pa[i] = A + (long)min(m0 + row, M - 1) * K;
+        pw[i] = W + (long)min(n0 + row, N - 1) * K;
+    }
+    const int kc = 4 * (tid & 7);
+    auto fetch = [&](int b) {  // blocks b and b + 1 (whole blocks: the second may lie past K, is read from before it and not used)
+        const int k = ROWS == ROW_WHOLE ? min(16 * b + kc, K - 4) : 16 * b + kc;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            ra[i] = load4<ROWS>(pa[i], k, K);
+            rw[i] = load4<ROWS>(pw[i], k, K);
+        }
+    };
+    auto stage = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int at = ((tid + 256 * i) >> 3) * PITCH + kc;
+            *(f32x4*)&As[buf][at] = ra[i];
+            *(f32x4*)&Ws[buf][at] = rw[i];
+        }
+    };
+    auto store_all = [&](const f32x4 (&v)[F][F], float* to, bool last) {
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+            for (int j = 0; j < F; ++j) {
+                const int n = n0 + wn + 16 * i + kq, m = m0 + wm + 16 * j + r16;
+                if (m >= M) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) to[(long)m * N + n + e] = last ? finish(v[i][j][e], epi, n + e, (long)m * N + n + e) : v[i][j][e];
+            }
+    };
+    if (b_first < b_last) {
+        fetch(b_first);
+        stage(0);
+        __syncthreads();
+    }
+    int left = sb, segs = 0, buf = 0;  // blocks left of the segment, segments finished
+    for (int b = b_first; b < b_last; b += 2, buf ^= 1) {
+        const bool more = b + 2 < b_last;
+        if (more) fetch(b + 2);
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            if (b + h < b_last) {
+                f32x4 w[F], x[F];
+#pragma unroll
+                for (int i = 0; i < F; ++i) {
+                    w[i] = *(const f32x4*)&Ws[buf][(wn + 16 * i + r16) * PITCH + 16 * h + kq];
+                    x[i] = *(const f32x4*)&As[buf][(wm + 16 * i + r16) * PITCH + 16 * h + kq];
+                }
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int i = 0; i < F; ++i)
+#pragma unroll
+                        for (int c = 0; c < F; ++c)
+                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][j], x[c][j], acc[i][c], 0, 0, 0);
+                if (--left == 0 || b + h + 1 == b_last) {  // the segment ends: its sum joins the others in their order
+                    if (SPLIT) {
+                        store_all(acc, C + (long)(s0 + segs) * M * N, false);
+                    } else if (segs == 0) {
+#pragma unroll
+                        for (int i = 0; i < F; ++i)
+#pragma unroll
+                            for (int c = 0; c < F; ++c) total[i][c] = acc[i][c];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < F; ++i)
+#pragma unroll
+                            for (int c = 0; c < F; ++c)
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) total[i][c][e] += acc[i][c][e];
+                    }
+#pragma unroll
+                    for (int i = 0; i < F; ++i)
+#pragma unroll
+                        for (int c = 0; c < F; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+                    ++segs;
+                    left = sb;
+                }
+            }
+        }
+        if (more) {
+            stage(buf ^ 1);  // the other buffer: everyone is past reading it since the last barrier
+            __syncthreads();
+        }
+    }
+    if (!SPLIT) store_all(total, C, true);
+}
+
+// the segments' sums added in order, and the epilogue
+__global__ void gemm_f32_add_kernel(float* __restrict__ C, const float* __restrict__ part, F32Epilogue epi, int segs, long MN, int N) {
+    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= MN) return;
+    float v = part[i];
+    for (int s = 1; s < segs; ++s) v += part[(long)s * MN + i];
+    C[i] = finish(v, epi, (int)(i % N), i);
+}
+
+// How a product runs: the tile's side (0: the kernel for few rows) and over how many workgroups a tile's segments are shared.
+static void f32_plan(int M, int N, int K, int* tile, int* share) {
+    *tile = 0, *share = 1;
+    if (M <= SKINNY_ROWS) return;
+    const int cus = 256;
+    auto tiles = [&](long t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
+    auto rounds = [&](long n) { return (double)((n + cus - 1) / cus); };
+    // time of a round: a tile of 128 is four of 64; the smaller tile reads twice as much per product
+    const double big = 4.0 * rounds(tiles(128)), small = 1.1 * rounds(tiles(64));
+    *tile = big <= small ? 128 : 64;
+    const int used = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
+    if (*tile == 64 && K >= 1024)  // a chip that is not filled twice: share the segments out
+        while (*share < used && tiles(64) * *share < 2 * cus) *share *= 2;
+    if (*share > used) *share = used;
+}
+
+// 32-bit values of scratch memory that pta_gemm_f32 needs for this product (0: none)
+extern "C" long pta_gemm_f32_scratch(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    int tile, share;
+    f32_plan(M, N, K, &tile, &share);
+    if (share <= 1) return 0;
+    return (long)(((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K)) * M * N;
+}
+
+template <int ROWS>
+static void launch_few(float* C, const float* A, const float* W, const F32Epilogue& epi, int M, int N, int K, hipStream_t s) {
+    // whole rounds of the 256 compute units, up to 32 rows of W each; small matrices: four rows a workgroup
+    int groups = 256 * ((N + 256 * 32 - 1) / (256 * 32));
+    if (groups > (N + 3) / 4) groups = (N + 3) / 4;
+    const bool two = (N + groups - 1) / groups > 16;
+    const dim3 grid(groups, (M + SKINNY_ROWS - 1) / SKINNY_ROWS);
+    const int ct = (M < SKINNY_ROWS ? M : SKINNY_ROWS) <= 16 ? 1 : M <= 32 ? 2 : 4;
+#define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), grid, dim3(512), 0, s, C, A, W, epi, M, N, K)
+    if (ct == 1) { if (two) FEW(1, 2, 4); else FEW(1, 1, 4); }
+    else if (ct == 2) { if (two) FEW(2, 2, 4); else FEW(2, 1, 4); }
+    else { if (two) FEW(4, 2, 2); else FEW(4, 1, 2); }
+#undef FEW
+}
+
+template <int ROWS>
+static void launch_tiles(float* C, float* scratch, const float* A, const float* W, const F32Epilogue& epi, int M, int N, int K,
+                         int tile, int share, hipStream_t s) {
+    const int tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
+    const int groups = 8 * ((tm * tn + 7) / 8);
+#define TILE(T, SPLIT, OUT) \
+    hipLaunchKernelGGL((gemm_f32_tile_kernel<T, ROWS, SPLIT>), dim3(groups, SPLIT ? share : 1), dim3(256), 0, s, OUT, A, W, epi, M, N, K, tm, tn)
+    if (share > 1) TILE(64, true, scratch);
+    else if (tile == 128) TILE(128, false, C);
+    else TILE(64, false, C);
+#undef TILE
+    if (share > 1) {
+        const long mn = (long)M * N;
+        const int segs = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
+        hipLaunchKernelGGL(gemm_f32_add_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, C, scratch, epi, segs, mn, N);
+    }
+}
+
 extern "C" int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, const float* add1,
-                            const float* add2, int M, int N, int K, int act, void* stream) {
+                            const float* add2, int M, int N, int K, int act, float* scratch, void* stream) {
     PTA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: sizes must be positive (M=%d N=%d K=%d)", M, N, K);
     PTA_REQUIRE(C && A && W, "gemm_f32: null pointer");
     PTA_REQUIRE(pta_act_known(act), "gemm_f32: unknown activation %d", act);
-    const int gy = (M + G_BM - 1) / G_BM, gx = (N + G_BN - 1) / G_BN;
-    PTA_REQUIRE(gy <= 65535, "gemm_f32: M=%d is too large for one launch", M);
-    hipLaunchKernelGGL(gemm_f32_kernel, dim3(gx, gy), dim3(256), 0, (hipStream_t)stream, C, A, W, bias, add1, add2,
-                       M, N, K, act);
+    PTA_REQUIRE(M <= 65535 * 64, "gemm_f32: M=%d is too large for one launch", M);
+    int tile, share;
+    f32_plan(M, N, K, &tile, &share);
+    PTA_REQUIRE(share <= 1 || scratch, "gemm_f32: this product needs scratch memory (pta_gemm_f32_scratch)");
+    const F32Epilogue epi{bias, add1, add2, act};
+    const bool vec = K % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+    hipStream_t s = (hipStream_t)stream;
+#define BY_ROWS(FN, ...) (vec && K % 16 == 0 ? FN<ROW_WHOLE>(__VA_ARGS__) : vec ? FN<ROW_VECTORS>(__VA_ARGS__) : FN<ROW_ELEMENTS>(__VA_ARGS__))
+    if (tile == 0) BY_ROWS(launch_few, C, A, W, epi, M, N, K, s);
+    else BY_ROWS(launch_tiles, C, scratch, A, W, epi, M, N, K, tile, share, s);
+#undef BY_ROWS
     return pta_check_launch("gemm_f32");
 }

@@ -14,7 +14,7 @@
 
 #include <stdint.h>
 
-#define PTA_ABI_VERSION 16
+#define PTA_ABI_VERSION 17
 
 #ifdef __cplusplus
 extern "C" {
@@ -128,9 +128,11 @@ int pta_attn_mfma(void* out, const void* q, const void* k_pool, const void* v_po
                   float* pm, float* pl, int window, int chunk, int decode_tiles, int decode_waves, int prompt_wide,
                   const float* sink, const PtaHeadRows* head_rows, void* stream);
 
-// C = act(A . W^T + bias) + add1 + add2, all 32-bit, fixed summation order
+// C = act(A . W^T + bias) + add1 + add2, all 32-bit, in an order of summation that K alone decides.  scratch: as many 32-bit
+// values as pta_gemm_f32_scratch says (0: may be null)
+long pta_gemm_f32_scratch(int M, int N, int K);
 int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, const float* add1, const float* add2,
-                 int M, int N, int K, int act, void* stream);
+                 int M, int N, int K, int act, float* scratch, void* stream);
 
 // y = act(x . W^T + bias) + add1 + add2 for M <= 64 rows of bfloat16; y is bfloat16, or 32-bit if out_f32.
 // variant and waves are tuning knobs (0: chosen from N and K): row tiles per wave, waves per workgroup

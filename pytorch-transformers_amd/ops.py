@@ -24,7 +24,7 @@ QKV_LAYOUT_CODES = {"grouped": 0, "tail": 1, "interleaved": 2}
 ACT_CODES = {None: 0, "none": 0, "linear": 0, "gelu": 1, "gelu_python": 1, "gelu_new": 2, "gelu_pytorch_tanh": 2,
              "gelu_fast": 2, "gelu_accurate": 2, "quick_gelu": 3, "relu": 4, "relu2": 5, "relu6": 6, "silu": 7, "swish": 7,
              "sigmoid": 8, "tanh": 9, "leaky_relu": 10, "mish": 11, "gelu_10": 12, "laplace": 13}
-ABI_VERSION = 16
+ABI_VERSION = 17
 PAIRING_CODES = {"half": 0, "interleaved": 1}  # PtaPairing: elements (i, i + rotary_dim / 2) or (2i, 2i + 1)
 BIAS_OF_CODES = {"key": 0, "distance": 1}  # PtaBiasOf: the slope times the key's position, or times key - query position
 
@@ -87,6 +87,7 @@ def load_library(build_if_missing: bool = True):
             path = b.build(verbose=True)
         lib = ctypes.CDLL(path)
         lib.pta_last_error.restype = ctypes.c_char_p
+        lib.pta_gemm_f32_scratch.restype = ctypes.c_long
         if lib.pta_abi_version() != ABI_VERSION:
             raise KernelError(f"{path} has ABI {lib.pta_abi_version()}, this package needs {ABI_VERSION}; rebuild it")
         _lib = lib
@@ -668,8 +669,10 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, a
         if t is not None:
             _need(t, name, torch.float32, (M, N))
     out = torch.empty((M, N), dtype=torch.float32, device=a.device)
+    need = load_library().pta_gemm_f32_scratch(M, N, K)
+    scratch = torch.empty(need, dtype=torch.float32, device=a.device) if need else None
     _call("pta_gemm_f32", _ptr(out), _ptr(a), _ptr(w), _ptr(bias), _ptr(add1), _ptr(add2), M, N, K, ACT_CODES[act],
-          _stream())
+          _ptr(scratch), _stream())
     return out
 
 
