@@ -1,0 +1,383 @@
+// Causal attention over the paged cache in true 32-bit, on the 32-bit matrix instruction (v_mfma_f32_16x16x4_f32: products
+// and sums in 32-bit), for head sizes that are a multiple of 4.  What it computes is what attn_generic.hip says.
+//
+// Sixteen (token, head) pairs that share a KV head are the sixteen columns of a tile.  A page of 64 keys is one unit of work:
+// scores = K . q^T (four tiles of sixteen keys), the columns' maxima, weights and their sums, and V^T . weights.  The scores'
+// registers are the second product's operand as they are (a lane holds four keys of its column in both), so nothing goes
+// through LDS on the way.  A page's result (maximum, sum, weighted values) is joined to what the pages before it gave, page
+// by page in order, whoever computed them: what a token gets does not depend on the step's cut, on its batch or on the kernel.
+//
+// 71 heads of 64 on one KV head, four prompts of 90 to 700 tokens in a launch: 5,952 us with a wave per (token, head), 245 us.
+//
+//   prompts: a wave owns one or two tiles and walks their pages.  Bound by the matrix instruction and by L2 (a page of heads
+//     of 64 is 32 KB a tile); the tiles with the most keys start first.
+//   one token per sequence: the waves of a workgroup share the pages of a tile out and meet in LDS.
+#include "common.h"
+#include "pta_kernels.h"
+#include "score_bias.h"
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct AttnF32 {
+    float* out;
+    const float* q;
+    const float* k_pool;
+    const float* v_pool;
+    const int* block_table;
+    int bt_stride;
+    const int* token_seq;
+    const int* token_pos;
+    const float* slopes;
+    int bias_mode;
+    float bias_scale;
+    int M, nh, nkv, d;
+    float scale;
+    int window, chunk;
+    const float* sink;
+    PtaHeadRows rows;
+    int vec;  // heads may be written sixteen bytes at a time
+};
+
+// a column: its token's keys first .. nkeys - 1 of sequence seq (nkeys 0: no such column)
+struct Column {
+    int token, head, seq, first, nkeys;
+    float slope;
+};
+
+__device__ __forceinline__ Column column_of(const AttnF32& a, int token, int head, bool there) {
+    Column c{0, 0, -1, 0, 0, 0.f};
+    if (!there) return c;
+    c.token = token, c.head = head, c.seq = a.token_seq[token], c.nkeys = a.token_pos[token] + 1;
+    if (a.window > 0) c.first = max(0, c.nkeys - a.window);
+    if (a.chunk > 0) c.first = max(c.first, (c.nkeys - 1) / a.chunk * a.chunk);
+    if (a.slopes) c.slope = a.slopes[head];
+    return c;
+}
+
+// query operands of a column: four elements from 16 b + kq on, zeros past the head
+template <int DT>
+__device__ __forceinline__ void load_query(const AttnF32& a, const Column& c, int kq, f32x4 (&q)[DT]) {
+    const float* row = a.q + ((long)c.token * a.nh + c.head) * a.d;
+#pragma unroll
+    for (int b = 0; b < DT; ++b) {
+        q[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c.nkeys > 0 && 16 * b + kq < a.d) q[b] = *(const f32x4*)(row + 16 * b + kq);
+    }
+}
+
+__device__ __forceinline__ float across_max(float v) {  // over the four lanes of a column
+    v = fmaxf(v, __shfl_xor(v, 16));
+    return fmaxf(v, __shfl_xor(v, 32));
+}
+__device__ __forceinline__ float across_sum(float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+}
+
+// One page for CT tiles: m, l and o of its keys alone.  ``seen[c]``: whether column c looks at this page's sequence at all.
+// ``end``: keys of the sequence that any column of the wave sees (what lies behind is whatever the page held before).
+template <int DT, int CT>
+__device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, const float* vp, int j0, int end, const f32x4 (&q)[CT][DT],
+                                          const Column (&col)[CT], const bool (&seen)[CT], float (&m)[CT], float (&l)[CT],
+                                          f32x4 (&o)[CT][DT]) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
+    f32x4 s[CT][4];
+#pragma unroll
+    for (int c = 0; c < CT; ++c)
+#pragma unroll
+        for (int t = 0; t < 4; ++t) s[c][t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+        const float* row = kp + (16 * t + r16) * a.d + kq;
+        f32x4 k[DT];
+#pragma unroll
+        for (int b = 0; b < DT; ++b) {
+            k[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+            if (16 * b + kq < a.d) k[b] = *(const f32x4*)(row + 16 * b);
+        }
+#pragma unroll
+        for (int b = 0; b < DT; ++b)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) s[c][t] = __builtin_amdgcn_mfma_f32_16x16x4f32(k[b][e], q[c][b][e], s[c][t], 0, 0, 0);
+    }
+    bool whole = true;  // every column sees every key of the page
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const int first = seen[c] ? col[c].first : 0, n = seen[c] ? col[c].nkeys : 0;
+        whole = whole && first <= j0 && n >= j0 + PTA_PAGE;
+        float top = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = j0 + 16 * t + kq + e;
+                float v = s[c][t][e] * a.scale;
+                if (a.slopes)  // slope x key position as the reference rounds it (0), exact (1), or x the distance from the query (2)
+                    v += (a.bias_mode == 0 ? round_to_bf16(col[c].slope * round_to_bf16((float)j))
+                                           : col[c].slope * (float)(a.bias_mode == 2 ? j - (col[c].nkeys - 1) : j)) * a.bias_scale;
+                v = j >= first && j < n ? v : -INFINITY;
+                s[c][t][e] = v;
+                top = fmaxf(top, v);
+            }
+        top = across_max(top);
+        const float base = top == -INFINITY ? 0.f : top;
+        float sum = 0.f;
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int j = j0 + 16 * t + kq + e;
+                const float p = j >= first && j < n ? expf(s[c][t][e] - base) : 0.f;
+                s[c][t][e] = p;
+                sum += p;
+            }
+        m[c] = top, l[c] = across_sum(sum);
+    }
+    const bool ragged = __ballot(!whole) != 0;
+#pragma unroll
+    for (int b = 0; b < DT; ++b) {
+        const int row = min(16 * b + r16, a.d - 1);  // rows past the head: read again, not kept
+        f32x4 v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) v[t] = *(const f32x4*)(vp + row * PTA_PAGE + 16 * t + kq);
+#pragma unroll
+        for (int c = 0; c < CT; ++c) o[c][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (ragged) {
+            // A weight of 0 must hide its value whatever that is: keys behind the end are cleared; an infinite or undefined
+            // value of a key that only some columns see takes the page one key at a time.
+            float odd = 0.f;
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (j0 + 16 * t + kq + e >= end) v[t][e] = 0.f;
+                    odd += v[t][e] * 0.f;
+                }
+            if (__ballot(!(odd == 0.f))) {
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const int first = seen[c] ? col[c].first : 0, n = seen[c] ? col[c].nkeys : 0;
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e)
+                            for (int g = 0; g < 4; ++g) {
+                                const int jj = 16 * t + 4 * g + e;
+                                const float p = __shfl(s[c][t][e], 16 * g + r16);
+                                if (j0 + jj >= first && j0 + jj < n) {
+#pragma unroll
+                                    for (int i = 0; i < 4; ++i)
+                                        o[c][b][i] += p * vp[min(16 * b + kq + i, a.d - 1) * PTA_PAGE + jj];
+                                }
+                            }
+                }
+                continue;
+            }
+        }
+#pragma unroll
+        for (int t = 0; t < 4; ++t)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int c = 0; c < CT; ++c) o[c][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][e], s[c][t][e], o[c][b], 0, 0, 0);
+    }
+}
+
+// what the pages so far gave (M, L, O) takes in one more page's result; a page with no key of the column changes nothing
+__device__ __forceinline__ bool join(float& M, float& L, float m, float l, float& keep, float& take) {
+    if (m == -INFINITY && l == 0.f) return false;
+    const float top = fmaxf(M, m);
+    keep = expf(M - top), take = expf(m - top);  // the first page: M is -infinity, keep 0
+    L = L * keep + l * take;
+    M = top;
+    return true;
+}
+
+__device__ __forceinline__ void store_heads(const AttnF32& a, const Column& c, int dim, f32x4 v) {
+    float* to = a.out + (long)c.token * a.rows.ld + (long)c.head * a.rows.head + dim;
+    if (a.vec) {
+        if (dim < a.rows.keep) *(f32x4*)to = v;
+    } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (dim + i < a.rows.keep) to[i] = v[i];
+    }
+}
+
+// a learned number per head: its exponential joins the sum of the weights once, with no key and no value
+__device__ __forceinline__ float last_factor(const AttnF32& a, const Column& c, float M, float L) {
+    float last = 1.f;
+    if (a.sink) {
+        const float top = fmaxf(M, a.sink[c.head]);
+        last = expf(M - top);
+        L = L * last + expf(a.sink[c.head] - top);
+    }
+    return last / L * a.rows.mult;
+}
+
+template <int DT, int CT>
+__global__ __launch_bounds__(256, DT <= 6 ? 2 : 1) void attn_f32_prompt_kernel(AttnF32 a) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
+    const int per = a.nh / a.nkv, kvh = blockIdx.y;
+    // columns are (token, head of the group) pairs in a row; the last tiles have the most keys and start first
+    const long cols = (long)a.M * per;
+    const long tile = ((long)(gridDim.x - 1 - blockIdx.x) * 4 + (threadIdx.x >> 6)) * CT;
+    Column col[CT];
+    f32x4 q[CT][DT], O[CT][DT];
+    float M[CT], L[CT];
+    bool todo[CT];
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        const long at = (tile + c) * 16 + r16;
+        todo[c] = at < cols;
+        col[c] = column_of(a, (int)(at / per), kvh * per + (int)(at % per), todo[c]);
+        load_query<DT>(a, col[c], kq, q[c]);
+        M[c] = -INFINITY, L[c] = 0.f;
+#pragma unroll
+        for (int b = 0; b < DT; ++b) O[c][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+    for (;;) {  // one sequence after the other of those that the columns belong to: at least one column is done each time
+        unsigned long long left = 0;
+        int seq = 0;
+#pragma unroll
+        for (int c = CT - 1; c >= 0; --c) {
+            const unsigned long long here = __ballot(todo[c]);
+            if (here) left = here, seq = __shfl(col[c].seq, __ffsll(here) - 1);
+        }
+        if (!left) break;
+        bool seen[CT];
+        int from = 0x7fffffff, end = 0;
+#pragma unroll
+        for (int c = 0; c < CT; ++c) {
+            seen[c] = todo[c] && col[c].seq == seq;
+            if (seen[c]) from = min(from, col[c].first), end = max(end, col[c].nkeys), todo[c] = false;
+        }
+#pragma unroll
+        for (int x = 1; x < 16; x <<= 1) from = min(from, __shfl_xor(from, x)), end = max(end, __shfl_xor(end, x));
+        from = __builtin_amdgcn_readfirstlane(from), end = __builtin_amdgcn_readfirstlane(end);
+        const int* bt = a.block_table + (long)__builtin_amdgcn_readfirstlane(seq) * a.bt_stride;
+        for (int p = from / PTA_PAGE; p * PTA_PAGE < end; ++p) {
+            const long at = ((long)bt[p] * a.nkv + kvh) * PTA_PAGE * a.d;
+            float m[CT], l[CT], keep, take;
+            f32x4 o[CT][DT];
+            page_pass<DT, CT>(a, a.k_pool + at, a.v_pool + at, p * PTA_PAGE, end, q, col, seen, m, l, o);
+#pragma unroll
+            for (int c = 0; c < CT; ++c)
+                if (join(M[c], L[c], m[c], l[c], keep, take)) {
+#pragma unroll
+                    for (int b = 0; b < DT; ++b)
+#pragma unroll
+                        for (int i = 0; i < 4; ++i) O[c][b][i] = fmaf(O[c][b][i], keep, o[c][b][i] * take);
+                }
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < CT; ++c) {
+        if (col[c].nkeys == 0) continue;
+        const float f = last_factor(a, col[c], M[c], L[c]);
+#pragma unroll
+        for (int b = 0; b < DT; ++b) store_heads(a, col[c], 16 * b + kq, O[c][b] * f);
+    }
+}
+
+template <int DT, int NW>
+__global__ __launch_bounds__(NW * 64) void attn_f32_decode_kernel(AttnF32 a) {
+    __shared__ f32x4 po[NW][DT][64];
+    __shared__ float pm[NW][16], pl[NW][16];
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4), wave = threadIdx.x >> 6;
+    const int per = a.nh / a.nkv, kvh = blockIdx.y, token = blockIdx.z;
+    const int hh = blockIdx.x * 16 + r16;
+    Column col[1] = {column_of(a, token, kvh * per + hh, hh < per)};
+    f32x4 q[1][DT], O[(DT + NW - 1) / NW];
+    load_query<DT>(a, col[0], kq, q[0]);
+    const bool seen[1] = {col[0].nkeys > 0};
+    // one token: the same keys for every column that is there, and column 0 always is
+    const int end = __shfl(col[0].nkeys, 0), from = __shfl(col[0].first, 0), seq = __shfl(col[0].seq, 0);
+    const int* bt = a.block_table + (long)__builtin_amdgcn_readfirstlane(seq) * a.bt_stride;
+    const int p0 = __builtin_amdgcn_readfirstlane(from / PTA_PAGE), p1 = __builtin_amdgcn_readfirstlane((end + PTA_PAGE - 1) / PTA_PAGE);
+    float M = -INFINITY, L = 0.f;
+#pragma unroll
+    for (int i = 0; i < (DT + NW - 1) / NW; ++i) O[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int p = p0; p < p1; p += NW) {
+        const int n = min(NW, p1 - p);
+        if (wave < n) {
+            const long at = ((long)bt[p + wave] * a.nkv + kvh) * PTA_PAGE * a.d;
+            float m[1], l[1];
+            f32x4 o[1][DT];
+            page_pass<DT, 1>(a, a.k_pool + at, a.v_pool + at, (p + wave) * PTA_PAGE, end, q, col, seen, m, l, o);
+#pragma unroll
+            for (int b = 0; b < DT; ++b) po[wave][b][lane] = o[0][b];
+            if (lane < 16) pm[wave][lane] = m[0], pl[wave][lane] = l[0];
+        }
+        __syncthreads();
+        for (int w = 0; w < n; ++w) {  // in the pages' order; every wave the rows that it will write
+            float keep, take;
+            if (join(M, L, pm[w][r16], pl[w][r16], keep, take)) {
+#pragma unroll
+                for (int i = 0; i < (DT + NW - 1) / NW; ++i) {
+                    const int b = wave + i * NW;
+                    if (b < DT) {
+                        const f32x4 o = po[w][b][lane];
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) O[i][e] = fmaf(O[i][e], keep, o[e] * take);
+                    }
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (col[0].nkeys == 0) return;
+    const float f = last_factor(a, col[0], M, L);
+#pragma unroll
+    for (int i = 0; i < (DT + NW - 1) / NW; ++i) {
+        const int b = wave + i * NW;
+        if (b < DT) store_heads(a, col[0], 16 * b + kq, O[i] * f);
+    }
+}
+
+template <int DT>
+static void launch(const AttnF32& a, int one_each, hipStream_t s) {
+    constexpr int CT = DT <= 4 ? 2 : 1;   // a second tile halves the reads of a page per tile while the registers hold it
+    constexpr int NW = DT <= 4 ? 8 : DT <= 8 ? 4 : 2;
+    const int per = a.nh / a.nkv;
+    if (one_each) {
+        hipLaunchKernelGGL((attn_f32_decode_kernel<DT, NW>), dim3((per + 15) / 16, a.nkv, a.M), dim3(NW * 64), 0, s, a);
+    } else {
+        const long tiles = ((long)a.M * per + 16 * CT - 1) / (16 * CT);
+        hipLaunchKernelGGL((attn_f32_prompt_kernel<DT, CT>), dim3((unsigned)((tiles + 3) / 4), a.nkv), dim3(256), 0, s, a);
+    }
+}
+
+extern "C" int pta_attn_f32(float* out, const float* q, const float* k_pool, const float* v_pool, const int* block_table,
+                            int bt_stride, const int* token_seq, const int* token_pos, const PtaScoreBias* score_bias, int M,
+                            int nh, int nkv, int d, float scale, int window, int chunk, const float* sink,
+                            const PtaHeadRows* head_rows, int one_each, void* stream) {
+    int bias_mode = 0;
+    if (pta_score_bias_mode("attn_f32", score_bias, &bias_mode)) return 1;
+    const float* slopes = score_bias ? score_bias->slopes : nullptr;
+    PTA_REQUIRE(M > 0 && nh > 0 && nkv > 0 && nh % nkv == 0, "attn_f32: sizes must be positive and heads a multiple of kv heads (M=%d nh=%d nkv=%d)",
+                M, nh, nkv);
+    PTA_REQUIRE(d > 0 && d <= 256 && d % 4 == 0, "attn_f32: head size %d is no multiple of 4 up to 256", d);
+    PTA_REQUIRE(nkv <= 65535 && (!one_each || M <= 65535), "attn_f32: at most 65535 kv heads and decoded tokens, got %d and %d", nkv, M);
+    PTA_REQUIRE(window >= 0 && chunk >= 0, "attn_f32: window and chunk must be 0 (none) or positive, got %d and %d", window, chunk);
+    PTA_REQUIRE((uintptr_t)q % 16 == 0 && (uintptr_t)k_pool % 16 == 0 && (uintptr_t)v_pool % 16 == 0,
+                "attn_f32: queries and pages must be sixteen-byte aligned");
+    const PtaHeadRows rows = pta_head_rows_of(head_rows, nh, d);
+    if (pta_check_head_rows("attn_f32", rows, nh, d, out, 1)) return 1;
+    const int vec = rows.keep % 4 == 0 && rows.head % 4 == 0 && rows.ld % 4 == 0 && (uintptr_t)out % 16 == 0;
+    const AttnF32 a{out, q, k_pool, v_pool, block_table, bt_stride, token_seq, token_pos, slopes, bias_mode,
+                    slopes ? score_bias->scale : 0.f, M, nh, nkv, d, scale, window, chunk, sink, rows, vec};
+    hipStream_t s = (hipStream_t)stream;
+    const int dt = (d + 15) / 16;
+    if (dt <= 1) launch<1>(a, one_each, s);
+    else if (dt <= 2) launch<2>(a, one_each, s);
+    else if (dt <= 3) launch<3>(a, one_each, s);
+    else if (dt <= 4) launch<4>(a, one_each, s);
+    else if (dt <= 5) launch<5>(a, one_each, s);
+    else if (dt <= 6) launch<6>(a, one_each, s);
+    else if (dt <= 8) launch<8>(a, one_each, s);
+    else launch<16>(a, one_each, s);
+    return pta_check_launch("attn_f32");
+}

@@ -2,8 +2,8 @@
 // all arithmetic in 32-bit.  One wave per (token, head): keys are taken a page
 // (64) at a time from position 0 in a running softmax, so what a token computes
 // does not depend on how the sequence was cut into steps or on the rest of the
-// batch.  This is the engine's 32-bit path and the fallback for sizes the MFMA
-// kernels refuse.
+// batch.  For bfloat16 heads of sizes the matrix-core kernel is not built for, and
+// 32-bit heads that are no multiple of four (attn_f32.hip takes the others).
 //
 // score[j] = q . k_j / sqrt(d) + bias_j, keys 0 .. pos (or the last `window` of them)
 // (src/transformers/models/falcon/modeling_falcon.py:371-386, :407-422).

@@ -134,6 +134,12 @@ long pta_gemm_f32_scratch(int M, int N, int K);
 int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, const float* add1, const float* add2,
                  int M, int N, int K, int act, float* scratch, void* stream);
 
+// Attention of 32-bit heads of up to 256 elements, a multiple of 4, on the 32-bit matrix instruction: the arguments of
+// pta_attn_generic, and one_each: every token is its sequence's only one (a decode step)
+int pta_attn_f32(float* out, const float* q, const float* k_pool, const float* v_pool, const int* block_table, int bt_stride,
+                 const int* token_seq, const int* token_pos, const PtaScoreBias* score_bias, int M, int nh, int nkv, int d,
+                 float scale, int window, int chunk, const float* sink, const PtaHeadRows* head_rows, int one_each, void* stream);
+
 // y = act(x . W^T + bias) + add1 + add2 for M <= 64 rows of bfloat16; y is bfloat16, or 32-bit if out_f32.
 // variant and waves are tuning knobs (0: chosen from N and K): row tiles per wave, waves per workgroup
 int pta_gemm_skinny_bf16(void* y, const void* x, const void* W, const float* bias, const void* add1, const void* add2,

@@ -179,7 +179,7 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[6], a[7], a[8], 4)
     if name == "pta_layernorm_sum":
         return ((a[4] + a[7]) * float(a[17]) * a[19] * 4, 0.0)
-    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_latent_mfma", "pta_attn_latent", "pta_attn_talk",
+    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_attn_latent_mfma", "pta_attn_latent", "pta_attn_talk",
                 "pta_attn_talk_mfma"):
         # (a model with two kinds of attention says each kind's figures under the entry point's name)
         return (float(timing_hint.get("attn_bytes:" + name, timing_hint.get("attn_bytes", 0))),
@@ -584,13 +584,17 @@ def head_rows_ok(out: torch.Tensor, keep: int) -> bool:
 
 def attn_generic(q: torch.Tensor, k_pool, v_pool, block_table, token_seq, token_pos, slopes, scale: float,
                  window: int = 0, alibi_exact: bool = False, bias_of: str = "key", bias_scale: Optional[float] = None,
-                 chunk: int = 0, sink: Optional[torch.Tensor] = None, into=None):
+                 chunk: int = 0, sink: Optional[torch.Tensor] = None, into=None, one_each: bool = False):
     """Causal attention of every token over its sequence's cache (the last ``window`` positions of it, itself
     included, if ``window`` > 0; the positions of its own block of ``chunk``, counted from the sequence's start, if
     ``chunk`` > 0); out [M, nh*d].  ``slopes`` (None: no bias), ``bias_of``, ``alibi_exact`` (no
     rounding to bfloat16) and ``bias_scale`` (None: 1 / sqrt(head size), as the reference folds its bias into the
     mask) describe a bias on the scores (``_score_bias_arg``).  ``sink`` (``[nh]`` 32-bit): ``exp(sink[h])`` joins the
-    sum that head h's weights are divided by.  ``into = (out, keep, mult)``: see ``_head_rows``."""
+    sum that head h's weights are divided by.  ``into = (out, keep, mult)``: see ``_head_rows``.  ``one_each``: every
+    token is its sequence's only one in the step (says how the work is shared out, not what comes of it).
+
+    32-bit heads of a multiple of four elements run on the 32-bit matrix instruction (``pta_attn_f32``); bfloat16 heads of
+    sizes that the matrix-core kernel is not built for, and other 32-bit ones, a wave per token and head."""
     _need(q, "q")
     if sink is not None:
         _need(sink, "sink", torch.float32, (q.shape[1],))
@@ -604,6 +608,11 @@ def attn_generic(q: torch.Tensor, k_pool, v_pool, block_table, token_seq, token_
     out, rows = _head_rows(into, M, nh, d, q.dtype)
     if out is None:
         out = torch.empty((M, nh * d), dtype=q.dtype, device=q.device)
+    if q.dtype == torch.float32 and d % 4 == 0 and q.data_ptr() % 16 == 0 and k_pool.data_ptr() % 16 == 0 and v_pool.data_ptr() % 16 == 0:
+        _call("pta_attn_f32", _ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table), block_table.shape[1],
+              _ptr(token_seq), _ptr(token_pos), bias, M, nh, nkv, d, ctypes.c_float(scale), int(window), int(chunk), _ptr(sink),
+              rows, int(one_each and M <= 65535), _stream())
+        return out
     _call("pta_attn_generic", _ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
           block_table.shape[1], _ptr(token_seq), _ptr(token_pos), bias, M, nh, nkv, d,
           ctypes.c_float(scale), int(window), int(chunk), _ptr(sink), rows, dtype_code(q.dtype), _stream())
@@ -761,7 +770,7 @@ def attention(q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: 
                          decode_tiles=tiles, decode_waves=waves, alibi_exact=alibi_exact, bias_of=bias_of,
                          bias_scale=bias_scale, chunk=chunk, sink=sink, into=into)
     return attn_generic(q, k_pool, v_pool, block_table, ctx.token_seq, ctx.token_pos, slopes, scale, window, alibi_exact,
-                        bias_of, bias_scale, chunk, sink, into)
+                        bias_of, bias_scale, chunk, sink, into, one_each=ctx.is_decode)
 
 
 def attn_talk_mfma_ok(q: torch.Tensor, nkv: int, mixed: bool = True) -> bool:

@@ -1,5 +1,5 @@
-"""The 32-bit kernels alone, against 64-bit references: every way a product runs (few rows, tiles, shared segments),
-at the edges of their tiles, and the same bits for a row whichever of them it runs in."""
+"""The 32-bit kernels alone, against 64-bit references: every way a product runs (few rows, tiles, shared segments) and both
+attention kernels, at the edges of their tiles, and the same bits for a row whichever of them it runs in."""
 import math
 
 import pytest
@@ -39,3 +39,88 @@ def test_products(N, K):
     for m in (1, 2, 16, 17, 33, 64, 65, 128, 300):
         assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w), plain[:m]), f"{m} rows alone and in a batch"
         assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w, bias, "gelu", a1[:m].contiguous(), a2[:m].contiguous()), full[:m])
+
+
+def _attention_case(nh, nkv, d, starts, news, window=0, chunk=0, sink=False, slopes=None, spoil=False):
+    """(queries, pools, table, token arrays, 64-bit result); pages hold NaN where nothing was written."""
+    g = torch.Generator().manual_seed(nh * 100 + d)
+    lens = [s + n for s, n in zip(starts, news)]
+    pages = [(n + 63) // 64 for n in lens]
+    k_pool = torch.full((sum(pages) + 1, nkv, 64, d), float("nan"))
+    v_pool = torch.full((sum(pages) + 1, nkv, d, 64), float("nan"))
+    table = torch.zeros((len(lens), max(pages)), dtype=torch.int32)
+    order = torch.randperm(sum(pages), generator=g).tolist()
+    qs, outs = [], []
+    sinks = torch.randn(nh, generator=g) if sink else None
+    for i, (s0, n, L) in enumerate(zip(starts, news, lens)):
+        k, v, q = (torch.randn(m, h, d, generator=g) for m, h in ((L, nkv), (L, nkv), (n, nh)))
+        for p in range(pages[i]):
+            page = order.pop()
+            table[i, p] = page
+            m = min(64, L - 64 * p)
+            k_pool[page, :, :m] = k[64 * p:64 * p + m].transpose(0, 1)
+            v_pool[page, :, :, :m] = v[64 * p:64 * p + m].permute(1, 2, 0)
+        qs.append(q)
+        j = torch.arange(L)[None, :]
+        t = torch.arange(s0, L)[:, None]
+        seen = j <= t
+        if window:
+            seen &= j > t - window
+        if chunk:
+            seen &= j >= t // chunk * chunk
+        o = torch.empty(n, nh, d, dtype=torch.float64)
+        for h in range(nh):
+            sc = q[:, h].double() @ k[:, h * nkv // nh].double().T * d ** -0.5
+            if slopes is not None:
+                sc = sc + slopes[h].double() * j * d ** -0.5
+            sc = sc.masked_fill(~seen, float("-inf"))
+            if sink:
+                sc = torch.cat([sc, sinks[h].double().expand(n, 1)], 1)
+            o[:, h] = torch.softmax(sc, -1)[:, :L] @ v[:, h * nkv // nh].double()
+        outs.append(o.reshape(n, nh * d))
+    seq = torch.tensor([i for i, n in enumerate(news) for _ in range(n)], dtype=torch.int32).cuda()
+    pos = torch.tensor([s + j for s, n in zip(starts, news) for j in range(n)], dtype=torch.int32).cuda()
+    args = (torch.cat(qs).cuda(), k_pool.cuda(), v_pool.cuda(), table.cuda(), seq, pos, None if slopes is None else slopes.cuda(), d ** -0.5)
+    kw = dict(window=window, chunk=chunk, sink=None if sinks is None else sinks.cuda(), alibi_exact=True)
+    return args, kw, torch.cat(outs)
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(71, 1, 64), (4, 2, 16), (6, 6, 24), (3, 1, 4), (5, 5, 80), (8, 2, 128), (4, 1, 256), (2, 2, 100), (7, 1, 40)])
+@pytest.mark.parametrize("how", ["plain", "window", "chunk", "sink", "slopes"])
+def test_attention(nh, nkv, d, how):
+    """Prompts, single tokens and continuations of several sequences in one launch, against 64 bits, and one token after the
+    other through the kernel for single tokens: the same bits."""
+    ops = _ops()
+    more = {"window": dict(window=70), "chunk": dict(chunk=96), "sink": dict(sink=True),
+            "slopes": dict(slopes=-torch.rand(nh, generator=torch.Generator().manual_seed(3)))}.get(how, {})
+    args, kw, want = _attention_case(nh, nkv, d, [0, 63, 700, 0, 127, 64], [70, 1, 5, 1, 2, 200], **more)
+    got = ops.attn_generic(*args, **kw)
+    assert (got.double().cpu() - want).abs().max().item() <= 2e-5 * max(1.0, want.abs().max().item())
+    q, kp, vp, table, seq, pos, slopes, scale = args
+    one = ops.attn_generic(*args, **kw, one_each=True)
+    assert torch.equal(one, got)
+    pick = [0, 69, 70, 75, len(seq) - 1]  # rows of several sequences, each alone
+    for r in pick:
+        alone = ops.attn_generic(q[r:r + 1].contiguous(), kp, vp, table, seq[r:r + 1].contiguous(), pos[r:r + 1].contiguous(), slopes, scale, **kw)
+        assert torch.equal(alone[0], got[r])
+    big = torch.full((len(seq), nh * d + 3), 7.0, device="cuda")
+    ops.attn_generic(*args, **kw, into=(big[:, 1:1 + nh * d], d, 2.0))
+    assert torch.equal(big[:, 1:1 + nh * d], got * 2.0) and bool((big[:, 0] == 7.0).all()) and bool((big[:, -2:] == 7.0).all())
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(4, 1, 64), (3, 3, 24)])
+def test_attention_hides_values_that_a_token_does_not_see(nh, nkv, d):
+    """An infinite value or an undefined key of a later token, or of another sequence, changes no earlier token's bits."""
+    ops = _ops()
+    args, kw, _ = _attention_case(nh, nkv, d, [0, 0], [50, 30])
+    got = ops.attn_generic(*args, **kw)
+    q, kp, vp, table, *rest = args
+    kp, vp = kp.clone(), vp.clone()
+    vp[table[0, 0].item(), :, :, 40] = float("inf")
+    kp[table[0, 0].item(), :, 40] = float("nan")
+    bad = ops.attn_generic(q, kp, vp, table, *rest, **kw)
+    # (a page with such a value is summed in another order)
+    assert (bad[:40] - got[:40]).abs().max().item() <= 1e-5 and torch.equal(bad[50:], got[50:]) or \
+        (bad[50:] - got[50:]).abs().max().item() <= 1e-5
+    assert bool(torch.isfinite(bad[:40]).all()) and bool(torch.isfinite(bad[50:]).all())
+    assert bool(torch.isnan(bad[40:50]).all())
