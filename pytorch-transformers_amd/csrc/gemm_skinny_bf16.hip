@@ -290,7 +290,7 @@ static int pick_split(int N) {
 }
 
 template <int MT, int RT, int U, typename OutT>
-static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hipStream_t s) {
+static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hipStream_t s, bool spread = false) {
     const int rows = 16 * RT;
     if (S <= 0) S = pick_split(a.N + b.N);
     a.blocks = (a.N + rows - 1) / rows;
@@ -299,7 +299,9 @@ static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hi
     // the time of 768 (measured: 44.7 us for 22,848 rows, 45.5 us for 24,576).  So a launch with more
     // workgroups than units gets a whole number of workgroups per unit, each with a little fewer rows.
     const int units = pta_compute_units(), natural = a.blocks + b.blocks;
-    if (natural > units && natural % units != 0) {
+    if (spread) {
+        a.blocks = std::max(a.blocks, std::min(units, (a.N + 3) / 4));
+    } else if (natural > units && natural % units != 0) {
         const int total = (natural + units - 1) / units * units;
         if (b.blocks == 0) {
             a.blocks = total;
@@ -318,21 +320,31 @@ static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hi
 
 template <typename OutT>
 static int launch_skinny(SkinnyProblem a, SkinnyProblem b, int M, int K, int variant, int S, hipStream_t s) {
-    // variant: row tiles per wave and steps per stage; 0: chosen here
+    // variant: row tiles per wave and steps per stage (6: one tile, its rows spread over all units); 0: chosen here
+    // Tiles of 32 rows of W that would occupy half of the compute units or fewer: a unit pulls no more than some 24 GB/s, so
+    // the rows are spread over all units instead, a few rows each (the rest of a tile's lanes read a row again).  Replays over
+    // cold weights, 8 rows of x, 32-row tiles -> spread: 2,048 x 8,192 24.0 -> 13.6 us, 2,048 x 2,048 9.7 -> 6.4, 3,072 x
+    // 2,048 9.8 -> 7.0, 1,040 x 4,160 15.2 -> 8.3; with more tiles the second read of x costs more than the units win (5,504
+    // x 2,048 9.2 -> 9.8, at 16 rows of x 9.9 -> 11.7).
+    if (variant == 0 && b.N == 0 && (a.N + 31) / 32 <= pta_compute_units() / 2) variant = 6;
     if (M <= 16) {
         if (variant == 0) variant = 2;
         if (variant == 1) launch_cfg<1, 1, 4, OutT>(a, b, M, K, S, s);
         else if (variant == 2) launch_cfg<1, 2, 2, OutT>(a, b, M, K, S, s);
         else if (variant == 3) launch_cfg<1, 4, 1, OutT>(a, b, M, K, S, s);
         else if (variant == 4) launch_cfg<1, 4, 2, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) launch_cfg<1, 1, 2, OutT>(a, b, M, K, S, s, true);
         else launch_cfg<1, 2, 4, OutT>(a, b, M, K, S, s);
     } else if (M <= 32) {
         if (variant == 3 || variant == 4) launch_cfg<2, 4, 1, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) launch_cfg<2, 1, 1, OutT>(a, b, M, K, S, s, true);
         else launch_cfg<2, 2, 1, OutT>(a, b, M, K, S, s);
     } else if (M <= 48) {
-        launch_cfg<3, 2, 1, OutT>(a, b, M, K, S, s);
+        if (variant == 6) launch_cfg<3, 1, 1, OutT>(a, b, M, K, S, s, true);
+        else launch_cfg<3, 2, 1, OutT>(a, b, M, K, S, s);
     } else {
         if (variant == 3 || variant == 4) launch_cfg<4, 4, 1, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) launch_cfg<4, 1, 1, OutT>(a, b, M, K, S, s, true);
         else launch_cfg<4, 2, 1, OutT>(a, b, M, K, S, s);
     }
     return pta_check_launch("gemm_skinny_bf16");
@@ -355,7 +367,7 @@ extern "C" int pta_gemm_skinny_bf16(void* y, const void* x, const void* W, const
                                     const void* add2, int M, int N, int K, int act, int out_f32, int variant,
                                     int waves, void* stream) {
     if (check_skinny("gemm_skinny_bf16", y, x, W, M, N, K, act)) return 1;
-    PTA_REQUIRE(variant >= 0 && variant <= 5, "gemm_skinny_bf16: unknown variant %d", variant);
+    PTA_REQUIRE(variant >= 0 && variant <= 6, "gemm_skinny_bf16: unknown variant %d", variant);
     PTA_REQUIRE(waves == 0 || (waves >= 1 && waves <= 8 && (waves & (waves - 1)) == 0),
                 "gemm_skinny_bf16: waves per workgroup must be 0 (choose) or a power of two up to 8, got %d", waves);
     hipStream_t s = (hipStream_t)stream;
