@@ -67,12 +67,11 @@ def _require_gpu(device) -> torch.device:
     return device
 
 
-GRAPH_LEN_STEP = 1024  # a decode graph serves contexts up to the next multiple of this ...
-GRAPH_MEAN_STEP = 512  # ... whose mean is at most a multiple of this
+GRAPH_MEAN_STEP = 512  # a decode graph serves contexts up to a bound (``_len_bound``) whose mean is at most a multiple of this
 
 
 def _len_bound(max_len: int) -> int:
-    return (max_len + GRAPH_LEN_STEP - 1) // GRAPH_LEN_STEP * GRAPH_LEN_STEP
+    return tuning.context_bound(max_len)
 
 
 def mean_len_bound(total_len: int, n_seqs: int, len_bound: int) -> int:

@@ -760,10 +760,13 @@ def attention(q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: 
     if attn_mfma_ok(q):
         n_splits, size, tiles, waves = 1, ATTN_SPLIT_KEYS, 0, 1
         if ctx.is_decode:
-            shape = (ctx.n_seqs, q.shape[1], k_pool.shape[1], q.shape[2], ctx.max_len, getattr(ctx, "mean_len", 0))
-            if window == 0 and chunk == 0:
-                tuning.note_decode_launch(*shape)
-            tiles, size, waves = tuning.decode_plan(*shape)
+            cut = tuning.short_cut(ctx.max_len)
+            if cut is None:
+                shape = (ctx.n_seqs, q.shape[1], k_pool.shape[1], q.shape[2], ctx.max_len, getattr(ctx, "mean_len", 0))
+                if window == 0 and chunk == 0:
+                    tuning.note_decode_launch(*shape)
+                cut = tuning.decode_plan(*shape)
+            tiles, size, waves = cut
             n_splits = (ctx.max_len + size - 1) // size
         return attn_mfma(q, k_pool, v_pool, block_table, ctx.cu_tokens, ctx.seq_start, slopes, scale,
                          max_new=max(ctx.new_tokens), n_splits=n_splits, split_size=size, window=window,

@@ -233,6 +233,30 @@ def _decode_plan(n: int, n_heads: int, n_kv_heads: int, head_dim: int, bound: in
 
 
 
+# Decode launches over contexts up to here walk the whole context with one wave per sequence and group of sixteen heads, which
+# leaves no ranges to merge; nothing is timed and no table is asked there.  Launch and merge, replayed over sixteen caches in
+# turn, the ranges of ``decode_plan`` -> whole: 71 heads on 1 KV head of 64, 8 sequences of 64 / 130 / 300 / 500 keys 6.9 ->
+# 3.5, 7.9 -> 4.9, 8.3 -> 7.1, 8.6 -> 9.2 us, 64 sequences 9.7 -> 4.8, 11.7 -> 6.5, 13.0 -> 8.4, 13.5 -> 11.5; 13 on 13 of 80, 5
+# sequences 7.0 -> 4.1, 8.6 -> 6.2, 8.9 -> 7.9, 9.3 -> 10.2; 16 on 8 of 128, 2 sequences 6.6 -> 4.0, 7.4 -> 5.6, 8.6 -> 8.5,
+# 8.7 -> 11.4; 128 on 8 of 64, 32 sequences 8.7 -> 4.3, 10.0 -> 5.7, 12.7 -> 8.9, 15.4 -> 13.2: the merge costs a launch,
+# which few keys do not win back.  In whole steps, where keys come from memory, a lone wave on 300 keys is no longer the faster
+# one (24 layers of 13 heads of 80 with ALiBi, 17 to 325 keys: 34.7 ms a request with ranges, 35.4 with whole contexts up to
+# 320), at 60 keys it is by what the merge costs (32 layers of 71 heads, one sequence: 79.7 -> 77.1 ms).
+SHORT_CONTEXT = 192
+
+
+def context_bound(max_len: int) -> int:
+    """The context that a captured decode step is sized for: ``SHORT_CONTEXT``, or the next multiple of 1,024."""
+    return SHORT_CONTEXT if max_len <= SHORT_CONTEXT else (max_len + 1023) // 1024 * 1024
+
+
+def short_cut(max_len: int):
+    """The cut of a decode launch over so short a context (as ``decode_plan`` gives cuts), or None where it is longer."""
+    if max_len > SHORT_CONTEXT or ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
+        return None
+    return (1, SHORT_CONTEXT, 1)
+
+
 def decode_key(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int):
     n = 1
     while n < n_seqs:
