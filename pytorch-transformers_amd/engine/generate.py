@@ -231,7 +231,7 @@ def generate(model, prompts: Sequence[Sequence[int]], generation_config: Optiona
                     if want_scores:
                         out_scores[i].append(scores[row].clone())
                     if want_logits:
-                        out_logits[i].append(logits[row].clone())
+                        out_logits[i].append(logits[row])  # (a step's logits are a tensor of their own)
                     if puts:
                         streamer.put(_ids_tensor([tok]))
                     elif streamer is not None:

@@ -80,6 +80,19 @@ def mean_len_bound(total_len: int, n_seqs: int, len_bound: int) -> int:
     return min(len_bound, -(-mean // GRAPH_MEAN_STEP) * GRAPH_MEAN_STEP)
 
 
+_capture_streams: Dict[int, "torch.cuda.Stream"] = {}
+
+
+def _capture_stream(device: torch.device) -> "torch.cuda.Stream":
+    """The stream of a device that steps are captured on: one for all captures, because libraries keep a workspace per
+    stream."""
+    index = torch.cuda.current_device() if device.index is None else device.index
+    stream = _capture_streams.get(index)
+    if stream is None:
+        stream = _capture_streams[index] = torch.cuda.Stream(device=index)
+    return stream
+
+
 class _DecodeGraph:
     """One decode step of ``n`` sequences with contexts up to ``len_bound`` (``mean_bound`` on average),
     captured once and replayed.
@@ -205,8 +218,17 @@ class _DecodeGraph:
         collecting = gc.isenabled()
         gc.disable()  # no finalizer of a dead cycle may call into the runtime while the capture lasts
         try:
-            with torch.cuda.graph(graph):
-                self.logits = self.model.forward_tokens(*self._context())  # a context of its own: nothing cached per step is shared
+            # on a stream of its own, without the wait for the GPU and the emptying of torch's memory cache that
+            # ``torch.cuda.graph`` begins with: the step just launched goes on meanwhile, and the memory that a program's
+            # next tensors would take stays where it is
+            stream = _capture_stream(self.model.device)
+            stream.wait_stream(torch.cuda.current_stream(self.model.device))
+            with torch.cuda.stream(stream):
+                graph.capture_begin()
+                try:
+                    self.logits = self.model.forward_tokens(*self._context())  # a context of its own: nothing cached per step is shared
+                finally:
+                    graph.capture_end()
         finally:
             if collecting:
                 gc.enable()

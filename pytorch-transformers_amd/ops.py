@@ -271,7 +271,8 @@ def _entry_cost(name: str, a) -> tuple:
 
 
 def _stream() -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    # (the handle alone: a Stream object around it costs more than a launch does)
+    return ctypes.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
 
 
 def dtype_code(dt: torch.dtype) -> int:
