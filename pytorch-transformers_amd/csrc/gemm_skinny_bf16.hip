@@ -278,6 +278,53 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     }
 }
 
+// A fused query_key_value product on its own, taken to its end by its epilogue (qkv_tail.h), for matrices whose rows are spread
+// over all compute units (``launch_skinny``): a workgroup has up to eight neighbouring rotation pairs, the first elements as
+// rows 0 .. 7 of its one tile, their partners as rows 8 .. 15.  Bound by the launch, not by W: at 3,120 x 1,040 and 5 rows it
+// takes what the product alone takes, and the launch that split, rotated and wrote the cache (4 us a layer) is gone: a
+// model of 24 such layers, 5 sequences, 24 steps and their prompts 34.5 -> 32.2 ms.
+__global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
+                                                               const float* __restrict__ bias, int M, int K, int rot_stride,
+                                                               QkvTail tail) {
+    extern __shared__ f32x4_t part[];  // [S][64]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const int r = lane & 15, g = lane >> 4, half = tail.d >> 1;
+    const int pairs = (tail.nh + 2 * tail.nkv) * half;
+    const int p0 = (int)((long)blockIdx.x * pairs / gridDim.x), p1 = (int)((long)(blockIdx.x + 1) * pairs / gridDim.x);
+    const int mine = min(p0 + (r & 7), p1 - 1);  // (places past the end read a pair again)
+    int ea, eb;
+    bool rotated;
+    qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
+    const bf16_t* wrow[1] = {W + (long)(mine / half * tail.d + (r < 8 ? ea : eb)) * K};
+    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
+    f32x4_t acc[1][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}};
+    const int nsteps = (K + 63) >> 6;
+    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
+    Stage<1, 1, 2> s0, s1;
+    load_stage<1, 1, 2>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
+    for (int step = wave; step < nsteps; step += 4 * S) {
+        load_stage<1, 1, 2>(s1, wrow, xres, r, step + 2 * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<1, 1, 2>(s0, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        load_stage<1, 1, 2>(s0, wrow, xres, r, step + 4 * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<1, 1, 2>(s1, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    part[wave * 64 + lane] = acc[0][0];
+    __syncthreads();
+    const float* sums = (const float*)part;  // row i of the tile, column m: lane (i / 4) * 16 + m, element i % 4
+    for (int item = threadIdx.x; item < 128; item += blockDim.x) {
+        const int m = item & 15, i = item >> 4, pair = p0 + i;
+        if (m >= M || pair >= p1) continue;
+        const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
+        float a = sums[at], b = sums[at + 2 * 16 * 4];
+        for (int w = 1; w < S; ++w) a += sums[w * 256 + at], b += sums[w * 256 + at + 2 * 16 * 4];
+        qkv_tail_pair(tail, bias, m, pair / half, pair % half, round_to_bf16(a), round_to_bf16(b));
+    }
+}
+
 // Waves per workgroup, i.e. how many ways K is split.  Measured on MI355X: long streams per wave beat
 // many short ones, so K is split only when N alone gives too few waves.  It depends on N only, never
 // on M or on the tile variant, so the order of summation is the same for every batch.
@@ -326,7 +373,7 @@ static int launch_skinny(SkinnyProblem a, SkinnyProblem b, int M, int K, int var
     // cold weights, 8 rows of x, 32-row tiles -> spread: 2,048 x 8,192 24.0 -> 13.6 us, 2,048 x 2,048 9.7 -> 6.4, 3,072 x
     // 2,048 9.8 -> 7.0, 1,040 x 4,160 15.2 -> 8.3; with more tiles the second read of x costs more than the units win (5,504
     // x 2,048 9.2 -> 9.8, at 16 rows of x 9.9 -> 11.7).
-    if (variant == 0 && b.N == 0 && (a.N + 31) / 32 <= pta_compute_units() / 2) variant = 6;
+    if (variant == 0 && b.N == 0 && pta_gemm_skinny_spread(a.N)) variant = 6;
     if (M <= 16) {
         if (variant == 0) variant = 2;
         if (variant == 1) launch_cfg<1, 1, 4, OutT>(a, b, M, K, S, s);
@@ -430,6 +477,40 @@ extern "C" int pta_gemm_skinny_pair_qkv_bf16(void* q_out, const void* x1, const 
     if (pta_check_launch("gemm_skinny_pair_qkv_bf16")) return 1;
     if (!in_kernel(act2)) return pta_epilogue(y2, N2, nullptr, nullptr, nullptr, M, N2, act2, PTA_BF16, stream);
     return 0;
+}
+
+// Whether pta_gemm_skinny_qkv_bf16 is the launch for a fused product of so many rows of W: where they are spread over the units
+extern "C" int pta_gemm_skinny_spread(int N) { return N > 0 && (N + 31) / 32 <= pta_compute_units() / 2; }
+
+// A fused query_key_value projection on its own for up to 16 rows, with the tail of pta_gemm_skinny_pair_qkv_bf16; any even
+// head size up to 256, N = (nh + 2 nkv) d within pta_gemm_skinny_spread.
+extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const float* bias, const PtaRotation* rotation,
+                                        const int* token_pos, const int* token_seq, const int* block_table, int bt_stride,
+                                        void* k_pool, void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K,
+                                        void* stream) {
+    PTA_REQUIRE(nh > 0 && nkv > 0 && d > 0 && nh % nkv == 0, "gemm_skinny_qkv_bf16: heads %d, kv heads %d, head size %d", nh, nkv, d);
+    const int N = (nh + 2 * nkv) * d;
+    if (check_skinny("gemm_skinny_qkv_bf16", q_out, x, W, M, N, K, PTA_ACT_NONE)) return 1;
+    PTA_REQUIRE(M <= 16, "gemm_skinny_qkv_bf16: at most 16 rows, got %d", M);
+    PTA_REQUIRE(d % 2 == 0 && d <= 256, "gemm_skinny_qkv_bf16: head size %d must be even and at most 256", d);
+    PTA_REQUIRE(pta_gemm_skinny_spread(N), "gemm_skinny_qkv_bf16: %d rows of W are too many for this launch", N);
+    PTA_REQUIRE(layout >= 0 && layout <= 2, "gemm_skinny_qkv_bf16: unknown layout %d", layout);
+    PTA_REQUIRE(layout != PTA_QKV_TAIL || nkv == 1, "gemm_skinny_qkv_bf16: the tail layout has one kv head, got %d", nkv);
+    PTA_REQUIRE(layout != PTA_QKV_INTERLEAVED || nkv == nh, "gemm_skinny_qkv_bf16: the interleaved layout needs kv heads == heads");
+    PTA_REQUIRE(token_pos, "gemm_skinny_qkv_bf16: null token positions");
+    const PtaRotation rot = pta_rotation_of(rotation);
+    if (pta_check_rotation("gemm_skinny_qkv_bf16", rot, d, token_seq)) return 1;
+    PTA_REQUIRE(!write_cache || (k_pool && v_pool && block_table && token_seq), "gemm_skinny_qkv_bf16: null cache pointer");
+    const QkvTail tail{(bf16_t*)q_out, rot, token_pos, token_seq, block_table, bt_stride, (bf16_t*)k_pool,
+                       (bf16_t*)v_pool, nh, nkv, d, layout, write_cache};
+    const int pairs = N / 2;
+    const int blocks = std::max((pairs + 7) / 8, std::min(pta_compute_units(), (pairs + 1) / 2));
+    const int S = pick_split(N);
+    static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
+    const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
+    hipLaunchKernelGGL(gemm_skinny_tail_kernel, dim3(blocks), dim3(S * 64), (size_t)S * 64 * sizeof(f32x4_t), (hipStream_t)stream,
+                       (const bf16_t*)x, (const bf16_t*)W, bias, M, K, rot_stride, tail);
+    return pta_check_launch("gemm_skinny_qkv_bf16");
 }
 
 // Two products of one launch: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2), both [M, *] in

@@ -14,7 +14,7 @@
 
 #include <stdint.h>
 
-#define PTA_ABI_VERSION 17
+#define PTA_ABI_VERSION 18
 
 #ifdef __cplusplus
 extern "C" {
@@ -159,6 +159,13 @@ int pta_gemm_skinny_pair_qkv_bf16(void* q_out, const void* x1, const void* W1, c
                                   const int* block_table, int bt_stride, void* k_pool, void* v_pool, int nh, int nkv,
                                   int d, int layout, int write_cache, void* y2, const void* x2, const void* W2,
                                   const float* bias2, int N2, int act2, int M, int K, void* stream);
+
+// whether a matrix of N rows has them spread over all compute units in steps of up to 16 rows; and, for those, the fused
+// query_key_value product on its own with the same tail (any even head size)
+int pta_gemm_skinny_spread(int N);
+int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const float* bias, const PtaRotation* rotation,
+                             const int* token_pos, const int* token_seq, const int* block_table, int bt_stride, void* k_pool,
+                             void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K, void* stream);
 
 // The same product for a batch of up to 128 rows that shares x through LDS and may split K over workgroups:
 // `part` is a 32-bit workspace [parts, M, N], needed when parts > 1 or reduce = 0.  rt (row tiles per wave),

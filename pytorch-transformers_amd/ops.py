@@ -24,7 +24,7 @@ QKV_LAYOUT_CODES = {"grouped": 0, "tail": 1, "interleaved": 2}
 ACT_CODES = {None: 0, "none": 0, "linear": 0, "gelu": 1, "gelu_python": 1, "gelu_new": 2, "gelu_pytorch_tanh": 2,
              "gelu_fast": 2, "gelu_accurate": 2, "quick_gelu": 3, "relu": 4, "relu2": 5, "relu6": 6, "silu": 7, "swish": 7,
              "sigmoid": 8, "tanh": 9, "leaky_relu": 10, "mish": 11, "gelu_10": 12, "laplace": 13}
-ABI_VERSION = 17
+ABI_VERSION = 18
 PAIRING_CODES = {"half": 0, "interleaved": 1}  # PtaPairing: elements (i, i + rotary_dim / 2) or (2i, 2i + 1)
 BIAS_OF_CODES = {"key": 0, "distance": 1}  # PtaBiasOf: the slope times the key's position, or times key - query position
 
@@ -165,6 +165,8 @@ def _entry_cost(name: str, a) -> tuple:
         return both(gemm(a[12], a[4], a[13]), gemm(a[12], a[10], a[13]))
     if name == "pta_gemm_skinny_pair_qkv_bf16":
         return both(gemm(a[22], (a[11] + 2 * a[12]) * a[13], a[23]), gemm(a[22], a[20], a[23]))
+    if name == "pta_gemm_skinny_qkv_bf16":
+        return gemm(a[16], (a[11] + 2 * a[12]) * a[13], a[17])
     if name == "pta_gemm_splitk_bf16":
         return gemm(a[7], a[8], a[9])
     if name == "pta_gemm_splitk_pair_bf16":
@@ -1200,12 +1202,31 @@ def gemm_splitk_pair_qkv(x1: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_fr
     return q, y2
 
 
-def gemm_splitk_qkv(x: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_freq, cs_scale: float, token_pos, token_seq,
+def gemm_skinny_qkv_ok(x: torch.Tensor, w_qkv: torch.Tensor, d: int) -> bool:
+    """Whether the product of few rows takes a fused query_key_value projection on its own to its end: matrices whose rows
+    are spread over all compute units (larger ones keep their tiles, and the launch behind them)."""
+    return (QKV_TAIL and gemm_skinny_ok(x, w_qkv) and d % 2 == 0 and d <= 256
+            and bool(load_library().pta_gemm_skinny_spread(int(w_qkv.shape[0]))))
+
+
+def gemm_skinny_qkv(x: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_freq, cs_scale: float, token_pos, token_seq,
                     block_table, k_pool, v_pool, nh: int, nkv: int, d: int, layout: str, write_cache: bool,
                     rotary_dim: Optional[int] = None, pairing: str = "half"):
-    """A fused query_key_value projection of a decode batch (17 to 256 rows) on its own, taken to its end by the
-    launch that adds its partial sums: returns the queries [M, nh, d] rotated; keys and values are in the cache
-    pages, as ``qkv_rope_cache`` leaves them."""
+    """A fused query_key_value projection of at most 16 rows on its own (``gemm_skinny_qkv_ok``), taken to its end by the
+    launch that makes it: returns the queries [M, nh, d] rotated; keys and values are in the cache pages, as
+    ``qkv_rope_cache`` leaves them."""
+    rot = _check_qkv(x, w_qkv, bias_qkv, inv_freq, cs_scale, token_pos, token_seq, block_table, k_pool, v_pool, nh, nkv, d,
+                     rotary_dim, pairing)
+    M, K = x.shape
+    q = torch.empty((M, nh, d), dtype=torch.bfloat16, device=x.device)
+    _call("pta_gemm_skinny_qkv_bf16", _ptr(q), _ptr(x), _ptr(w_qkv), _ptr(bias_qkv), rot, _ptr(token_pos), _ptr(token_seq),
+          _ptr(block_table), block_table.shape[1], _ptr(k_pool), _ptr(v_pool), nh, nkv, d, QKV_LAYOUT_CODES[layout],
+          int(write_cache), M, K, _stream())
+    return q
+
+
+def _check_qkv(x, w_qkv, bias_qkv, inv_freq, cs_scale, token_pos, token_seq, block_table, k_pool, v_pool, nh, nkv, d, rotary_dim, pairing):
+    """The operands of a fused query_key_value product with its tail, checked; returns the rotation for the entry point."""
     _need(x, "x", torch.bfloat16)
     _need(w_qkv, "w_qkv", torch.bfloat16)
     M, K = x.shape
@@ -1221,8 +1242,20 @@ def gemm_splitk_qkv(x: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_freq, cs
     _need(block_table, "block_table", torch.int32)
     if block_table.dim() != 2:
         raise KernelError("block_table must be [sequences, pages]")
-    rot = _rotation_arg(inv_freq, cs_scale, d, block_table.shape[0], rotary_dim, pairing)
     _need_pools(k_pool, v_pool, torch.bfloat16, nkv, d)
+    return _rotation_arg(inv_freq, cs_scale, d, block_table.shape[0], rotary_dim, pairing)
+
+
+def gemm_splitk_qkv(x: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_freq, cs_scale: float, token_pos, token_seq,
+                    block_table, k_pool, v_pool, nh: int, nkv: int, d: int, layout: str, write_cache: bool,
+                    rotary_dim: Optional[int] = None, pairing: str = "half"):
+    """A fused query_key_value projection of a decode batch (17 to 256 rows) on its own, taken to its end by the
+    launch that adds its partial sums: returns the queries [M, nh, d] rotated; keys and values are in the cache
+    pages, as ``qkv_rope_cache`` leaves them."""
+    rot = _check_qkv(x, w_qkv, bias_qkv, inv_freq, cs_scale, token_pos, token_seq, block_table, k_pool, v_pool, nh, nkv, d,
+                     rotary_dim, pairing)
+    M, K = x.shape
+    N = (nh + 2 * nkv) * d
     part = torch.empty((int(load_library().pta_gemm_splitk_parts(N, K, 0, 0)), M, N), dtype=torch.float32, device=x.device)
     q = torch.empty((M, nh, d), dtype=torch.bfloat16, device=x.device)
     _call("pta_gemm_splitk_reduced_qkv_bf16", _ptr(q), _ptr(part), _ptr(x), _ptr(w_qkv), _ptr(bias_qkv), K,

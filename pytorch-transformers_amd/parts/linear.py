@@ -122,12 +122,17 @@ class Linear(Part):
         return y
 
     def with_tail(self, x: torch.Tensor, tail: "QkvTail") -> Optional["TailDone"]:
-        """This product as a fused query_key_value projection whose launch also runs ``tail`` (a decode batch of
-        17 rows and more, where the product is the split-K kernel's); else None, and the caller runs the two."""
-        if not (ops.QKV_TAIL and x.dtype == torch.bfloat16 and tail.head_dim % 2 == 0
-                and not ops.gemm_skinny_ok(x, self.weight) and ops.gemm_splitk_ok(x, self.weight)):
+        """This product as a fused query_key_value projection whose launch also runs ``tail`` (a small matrix in a step of
+        few rows, or a decode batch of 17 rows and more where the product is the split-K kernel's); else None, and the
+        caller runs the two."""
+        if ops.gemm_skinny_qkv_ok(x, self.weight, tail.head_dim):
+            launch = ops.gemm_skinny_qkv
+        elif (ops.QKV_TAIL and x.dtype == torch.bfloat16 and tail.head_dim % 2 == 0
+              and not ops.gemm_skinny_ok(x, self.weight) and ops.gemm_splitk_ok(x, self.weight)):
+            launch = ops.gemm_splitk_qkv
+        else:
             return None
-        return TailDone(ops.gemm_splitk_qkv(
+        return TailDone(launch(
             x, self.weight, tail.bias, tail.inv_freq, tail.cs_scale, tail.token_pos, tail.token_seq, tail.table,
             tail.k_pool, tail.v_pool, tail.num_heads, tail.kv_heads, tail.head_dim, tail.layout, tail.write_cache,
             **tail.how))

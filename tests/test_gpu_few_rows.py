@@ -23,3 +23,37 @@ def test_rows_spread_over_the_units(N, K):
     assert (whole.double() - want).abs().max().item() <= tol
     for m in (1, 8, 16, 17, 33, 48):
         assert torch.equal(ops.gemm_skinny_bf16(x[:m].contiguous(), w, out_f32=True), whole[:m])
+
+
+@pytest.mark.parametrize("layout,nh,nkv,d", [("interleaved", 13, 13, 80), ("grouped", 4, 2, 6), ("tail", 7, 1, 64), ("grouped", 8, 2, 128), ("tail", 1, 1, 2)])
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("rotation", ["none", "half", "interleaved part", "per sequence"])
+def test_fused_rows_to_their_end(layout, nh, nkv, d, M, rotation):
+    """The fused product on its own with the tail in its epilogue against the product and the kernel that splits, rotates and
+    writes: the same bits (K no multiple of 2,048), nothing written elsewhere, nothing at all with write_cache off."""
+    from pytorch_transformers_amd import ops
+
+    if not ops.QKV_TAIL:
+        pytest.skip("switched off by PTA_QKV_TAIL=0")
+    K, N = 264, (nh + 2 * nkv) * d
+    g = torch.Generator().manual_seed(M + d)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    x, w, bias = r(M, K).bfloat16(), (0.05 * r(N, K)).bfloat16(), r(N)
+    part = d // 2 if rotation == "interleaved part" and d >= 4 else d
+    part -= part % 2
+    how = dict(rotary_dim=part, pairing="interleaved") if rotation == "interleaved part" else {}
+    inv = None if rotation == "none" else 10000.0 ** (-torch.arange(part // 2, device="cuda").float() * 2 / part)
+    if rotation == "per sequence":
+        inv = (inv[None] * torch.arange(1, M + 1, device="cuda")[:, None]).contiguous()
+    pos = torch.randint(0, 190, (M,), generator=g).int().cuda()
+    seq, table = torch.arange(M).int().cuda(), torch.randperm(3 * M, generator=g).view(M, 3).int().cuda()
+    assert ops.gemm_skinny_qkv_ok(x, w, d)
+    new = lambda: (torch.full((3 * M, nkv, 64, d), 7.0).bfloat16().cuda(), torch.full((3 * M, nkv, d, 64), 7.0).bfloat16().cuda())
+    k0, v0 = new()
+    q0 = ops.qkv_rope_cache(ops.gemm_skinny_bf16(x, w), bias, inv, 0.9, pos, seq, table, k0, v0, nh, nkv, d, layout, **how)
+    k1, v1 = new()
+    q1 = ops.gemm_skinny_qkv(x, w, bias, inv, 0.9, pos, seq, table, k1, v1, nh, nkv, d, layout, True, **how)
+    assert torch.equal(q0, q1) and torch.equal(k0, k1) and torch.equal(v0, v1)
+    k2, v2 = new()
+    ops.gemm_skinny_qkv(x, w, bias, inv, 0.9, pos, seq, table, k2, v2, nh, nkv, d, layout, False, **how)
+    assert bool((k2 == 7.0).all()) and bool((v2 == 7.0).all())
