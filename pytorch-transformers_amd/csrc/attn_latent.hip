@@ -8,52 +8,14 @@
 // so the attention itself runs over the cache rows as they lie: every head is a query of R + dr elements against
 // one shared key row, and the values are the first R elements of the same row.  Queries and the latent results
 // stay in 32-bit between the three launches (latent_prep, head_project, attn_latent).
-#include "common.h"
-#include "pta_kernels.h"
+#include "attn_latent_token.h"
 
-// One workgroup per token.  q_rows[t] = H * (dn + dr) query elements (row stride q_ld), down_rows[t] = R + dr (row stride ld).
-//  - latent c = down[:R] / sqrt(mean(down[:R]^2) + eps) * w_norm -> cache row [0, R)
-//  - shared key part down[R:], its first rot->rotary_dim elements rotated by the token's position -> cache row [R, R + dr)
-//  - each head's rotated query part, rotated likewise -> q_full[t, h, R:]  (32-bit)
+// One workgroup per token.
 template <typename T>
-__global__ void latent_prep_kernel(float* __restrict__ q_full, T* __restrict__ k_pool, const T* __restrict__ q_rows,
-                                   long q_ld, const T* __restrict__ down_rows, long ld, const float* __restrict__ w_norm, float eps,
-                                   const float* __restrict__ inv_freq, int inv_freq_ld, float cs_scale, int rot_n,
-                                   int pairing, const int* __restrict__ token_pos, const int* __restrict__ token_seq,
-                                   const int* __restrict__ block_table, int bt_stride, int H, int dn, int dr, int R,
-                                   int write_cache) {
+__global__ void latent_prep_kernel(float* __restrict__ q_full, T* __restrict__ k_pool, const T* __restrict__ q_rows, long q_ld, LatentToken t) {
     __shared__ float red[16];
-    const int m = blockIdx.x;
-    const int pos = token_pos[m], seq = token_seq[m];
-    const T* row = q_rows + (long)m * q_ld;
-    const T* down = down_rows + (long)m * ld;
-    const float* freq = inv_freq ? inv_freq + (inv_freq_ld ? (long)seq * inv_freq_ld : 0) : nullptr;
-    const int D = R + dr;
-    // the element that element i of a rotated part is paired with, and the sign of the sine term
-    auto rotated = [&](const T* v, int i) -> float {
-        const float a = Io<T>::ld(v + i);
-        if (!freq || i >= rot_n) return a;
-        int pair, fi;
-        float sign;
-        if (pairing == PTA_PAIR_INTERLEAVED) { pair = i ^ 1; fi = i >> 1; sign = (i & 1) ? 1.f : -1.f; }
-        else { const int half = rot_n >> 1; pair = i < half ? i + half : i - half; fi = i < half ? i : i - half; sign = i < half ? -1.f : 1.f; }
-        const float ang = (float)pos * freq[fi];
-        return a * (cosf(ang) * cs_scale) + sign * Io<T>::ld(v + pair) * (sinf(ang) * cs_scale);
-    };
-    if (write_cache) {
-        float ss = 0.f;
-        for (int i = threadIdx.x; i < R; i += blockDim.x) { const float v = Io<T>::ld(down + i); ss += v * v; }
-        ss = block_sum(ss, red);
-        const float inv = 1.0f / sqrtf(ss / (float)R + eps);
-        const long page = block_table[(long)seq * bt_stride + pos / PTA_PAGE];
-        T* dst = k_pool + (page * PTA_PAGE + pos % PTA_PAGE) * (long)D;
-        for (int i = threadIdx.x; i < R; i += blockDim.x) Io<T>::st(dst + i, Io<T>::ld(down + i) * inv * w_norm[i]);
-        for (int i = threadIdx.x; i < dr; i += blockDim.x) Io<T>::st(dst + R + i, rotated(down + R, i));
-    }
-    for (int i = threadIdx.x; i < H * dr; i += blockDim.x) {
-        const int h = i / dr, e = i - h * dr;
-        q_full[((long)m * H + h) * D + R + e] = rotated(row + (long)h * (dn + dr) + dn, e);
-    }
+    if (t.write_cache) latent_row<T>(t, blockIdx.x, k_pool, red);
+    latent_rotations<T>(t, blockIdx.x, q_full, q_rows, q_ld);
 }
 
 // q_rows [M, H * (dn + dr)] rows q_ld apart; down_rows [M, R + dr] rows ld apart (the two may be blocks of columns of
@@ -63,27 +25,15 @@ extern "C" int pta_latent_prep(float* q_full, void* k_pool, const void* q_rows, 
                                const PtaRotation* rot, const int* token_pos, const int* token_seq,
                                const int* block_table, int bt_stride, int M, int H, int dn, int dr, int R,
                                int write_cache, int dtype, void* stream) {
-    PTA_REQUIRE(M > 0 && H > 0 && dn > 0 && dr >= 0 && R > 0, "latent_prep: sizes must be positive");
-    PTA_REQUIRE(q_full && q_rows && token_pos && token_seq && (!write_cache || (k_pool && proj && w_norm && block_table)), "latent_prep: null pointer");
-    PTA_REQUIRE(q_ld >= (long)H * (dn + dr) && (!write_cache || ld >= (long)R + dr), "latent_prep: rows lie closer together than they are long");
-    const float* inv_freq = rot ? rot->inv_freq : nullptr;
-    int rot_n = 0, pairing = PTA_PAIR_HALF, freq_ld = 0;
-    float cs = 1.f;
-    if (inv_freq) {
-        rot_n = rot->rotary_dim, pairing = rot->pairing, freq_ld = rot->inv_freq_ld, cs = rot->cs_scale;
-        PTA_REQUIRE(rot_n >= 2 && rot_n % 2 == 0 && rot_n <= dr,
-                    "latent_prep: %d rotated elements must be even and at most the rotated part's %d", rot_n, dr);
-        PTA_REQUIRE(pairing == PTA_PAIR_HALF || pairing == PTA_PAIR_INTERLEAVED, "latent_prep: unknown pairing %d", pairing);
-    }
+    LatentToken t;
+    if (latent_token_args("latent_prep", t, q_full, k_pool, q_rows, q_ld, proj, ld, w_norm, eps, rot, token_pos, token_seq, block_table, bt_stride,
+                          M, H, dn, dr, R, write_cache))
+        return 1;
     hipStream_t s = (hipStream_t)stream;
     if (dtype == PTA_F32)
-        hipLaunchKernelGGL(latent_prep_kernel<float>, dim3(M), dim3(256), 0, s, q_full, (float*)k_pool, (const float*)q_rows,
-                           q_ld, (const float*)proj, ld, w_norm, eps, inv_freq, freq_ld, cs, rot_n, pairing, token_pos, token_seq, block_table,
-                           bt_stride, H, dn, dr, R, write_cache);
+        hipLaunchKernelGGL(latent_prep_kernel<float>, dim3(M), dim3(256), 0, s, q_full, (float*)k_pool, (const float*)q_rows, q_ld, t);
     else if (dtype == PTA_BF16)
-        hipLaunchKernelGGL(latent_prep_kernel<bf16_t>, dim3(M), dim3(256), 0, s, q_full, (bf16_t*)k_pool,
-                           (const bf16_t*)q_rows, q_ld, (const bf16_t*)proj, ld, w_norm, eps, inv_freq, freq_ld, cs, rot_n, pairing, token_pos,
-                           token_seq, block_table, bt_stride, H, dn, dr, R, write_cache);
+        hipLaunchKernelGGL(latent_prep_kernel<bf16_t>, dim3(M), dim3(256), 0, s, q_full, (bf16_t*)k_pool, (const bf16_t*)q_rows, q_ld, t);
     else
         return pta_fail("latent_prep: unknown dtype %d", dtype);
     return pta_check_launch("latent_prep");

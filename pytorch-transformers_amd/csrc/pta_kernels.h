@@ -14,7 +14,7 @@
 
 #include <stdint.h>
 
-#define PTA_ABI_VERSION 18
+#define PTA_ABI_VERSION 19
 
 #ifdef __cplusplus
 extern "C" {
@@ -302,6 +302,19 @@ int pta_latent_prep(float* q_full, void* k_pool, const void* q_rows, long q_ld, 
                     const float* w_norm, float eps,
                     const PtaRotation* rot, const int* token_pos, const int* token_seq, const int* block_table,
                     int bt_stride, int M, int H, int dn, int dr, int R, int write_cache, int dtype, void* stream);
+
+// Decode steps over bfloat16 latents in three launches, for the sizes of pta_latent_decode_ok: what pta_latent_prep does and
+// the queries' frames filled with the plain queries through kt [H][R][dn] (the key expansion, a head's rows its outputs); then
+// the attention over `splits` ranges of `size` keys (po [M, H, splits, R], pm and pl [M, H, splits] are scratch) and the value
+// expansion up_v [H][V][R], out bfloat16 [M, H * V]
+int pta_latent_decode_ok(int H, int dn, int dr, int R, int V);
+int pta_latent_queries(float* q_full, void* k_pool, const void* q_rows, long q_ld, const void* down_rows, long ld,
+                       const float* w_norm, float eps, const PtaRotation* rot, const int* token_pos, const int* token_seq,
+                       const int* block_table, int bt_stride, const void* kt, int M, int H, int dn, int dr, int R, int write_cache,
+                       void* stream);
+int pta_latent_decode(void* out, float* po, float* pm, float* pl, const float* q, const void* k_pool, const int* block_table,
+                      int bt_stride, const int* seq_start, const void* up_v, int M, int H, int R, int dr, int V, float scale, int size,
+                      int splits, void* stream);
 int pta_head_project(void* out, int out_wide, long out_ld, long out_head, const void* in, int in_wide, long in_ld,
                      long in_head, const void* w, int M, int H, int K, int O, int dtype, void* stream);
 int pta_attn_latent(float* out, const float* q, const void* k_pool, const int* block_table, int bt_stride,

@@ -24,7 +24,7 @@ QKV_LAYOUT_CODES = {"grouped": 0, "tail": 1, "interleaved": 2}
 ACT_CODES = {None: 0, "none": 0, "linear": 0, "gelu": 1, "gelu_python": 1, "gelu_new": 2, "gelu_pytorch_tanh": 2,
              "gelu_fast": 2, "gelu_accurate": 2, "quick_gelu": 3, "relu": 4, "relu2": 5, "relu6": 6, "silu": 7, "swish": 7,
              "sigmoid": 8, "tanh": 9, "leaky_relu": 10, "mish": 11, "gelu_10": 12, "laplace": 13}
-ABI_VERSION = 18
+ABI_VERSION = 19
 PAIRING_CODES = {"half": 0, "interleaved": 1}  # PtaPairing: elements (i, i + rotary_dim / 2) or (2i, 2i + 1)
 BIAS_OF_CODES = {"key": 0, "distance": 1}  # PtaBiasOf: the slope times the key's position, or times key - query position
 
@@ -181,7 +181,7 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[6], a[7], a[8], 4)
     if name == "pta_layernorm_sum":
         return ((a[4] + a[7]) * float(a[17]) * a[19] * 4, 0.0)
-    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_attn_latent_mfma", "pta_attn_latent", "pta_attn_talk",
+    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_latent_decode", "pta_attn_latent_mfma", "pta_attn_latent", "pta_attn_talk",
                 "pta_attn_talk_mfma"):
         # (a model with two kinds of attention says each kind's figures under the entry point's name)
         return (float(timing_hint.get("attn_bytes:" + name, timing_hint.get("attn_bytes", 0))),
@@ -1617,15 +1617,10 @@ def latent_sizes_problem(heads: int, dim: int, rot_dim: int, rank: int) -> Optio
     return lib.pta_last_error().decode("utf-8", "replace")
 
 
-def latent_prep(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor], eps: float, inv_freq, cs_scale: float, rotary_dim, pairing: str,
-                token_pos, token_seq, block_table, k_pool, heads: int, dim: int, rot_dim: int, rank: int,
-                write_cache: bool = True, q: Optional[torch.Tensor] = None) -> torch.Tensor:
-    """From ``proj`` ``[tokens, heads * (dim + rot_dim) + rank + rot_dim]`` (the queries, then the down-projection), or
-    with the queries ``q`` ``[tokens, heads * (dim + rot_dim)]`` given apart from ``proj`` ``[tokens, rank + rot_dim]``
-    (each may be a block of columns): the normed latent and the rotated shared key part go into the token's cache row
-    ``[rank + rot_dim]``; returns the queries' frame ``[tokens, heads, rank + rot_dim]`` in 32-bit with the rotated
-    parts filled in (the first ``rank`` of each head are for ``head_project``).  ``write_cache`` False with ``q`` given:
-    the queries alone (``proj`` and ``w_norm`` None), for a layer that reads rows another layer has written."""
+def _latent_rows(proj, w_norm, inv_freq, cs_scale, rotary_dim, pairing, token_pos, token_seq, block_table, k_pool, heads, dim, rot_dim,
+                 rank, write_cache, q):
+    """``latent_prep``'s operands checked: ``(tokens, queries, their row distance, down rows, their row distance, rotation, an empty
+    frame of the queries)``."""
     M = (q if proj is None else proj).shape[0]
     q_cols = heads * (dim + rot_dim)
     if q is None:
@@ -1651,11 +1646,24 @@ def latent_prep(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor], ep
         raise KernelError(f"k_pool must be [pages, 1, 64, {D}], got {tuple(k_pool.shape)}")
     rot = _rotation_arg(inv_freq, cs_scale, rot_dim, block_table.shape[0], rotary_dim, pairing) if rot_dim else None
     q_full = torch.empty((M, heads, D), dtype=torch.float32, device=ref.device)
+    return M, ctypes.c_void_p(q_ptr), ctypes.c_long(q_ld), ctypes.c_void_p(down_ptr), ctypes.c_long(ld), rot, q_full
+
+
+def latent_prep(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor], eps: float, inv_freq, cs_scale: float, rotary_dim, pairing: str,
+                token_pos, token_seq, block_table, k_pool, heads: int, dim: int, rot_dim: int, rank: int,
+                write_cache: bool = True, q: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """From ``proj`` ``[tokens, heads * (dim + rot_dim) + rank + rot_dim]`` (the queries, then the down-projection), or
+    with the queries ``q`` ``[tokens, heads * (dim + rot_dim)]`` given apart from ``proj`` ``[tokens, rank + rot_dim]``
+    (each may be a block of columns): the normed latent and the rotated shared key part go into the token's cache row
+    ``[rank + rot_dim]``; returns the queries' frame ``[tokens, heads, rank + rot_dim]`` in 32-bit with the rotated
+    parts filled in (the first ``rank`` of each head are for ``head_project``).  ``write_cache`` False with ``q`` given:
+    the queries alone (``proj`` and ``w_norm`` None), for a layer that reads rows another layer has written."""
+    M, q_ptr, q_ld, down_ptr, ld, rot, q_full = _latent_rows(proj, w_norm, inv_freq, cs_scale, rotary_dim, pairing, token_pos, token_seq,
+                                                             block_table, k_pool, heads, dim, rot_dim, rank, write_cache, q)
     if M:
-        _call("pta_latent_prep", _ptr(q_full), _ptr(k_pool), ctypes.c_void_p(q_ptr), ctypes.c_long(q_ld),
-              ctypes.c_void_p(down_ptr), ctypes.c_long(ld), _ptr(w_norm),
+        _call("pta_latent_prep", _ptr(q_full), _ptr(k_pool), q_ptr, q_ld, down_ptr, ld, _ptr(w_norm),
               ctypes.c_float(eps), rot, _ptr(token_pos), _ptr(token_seq), _ptr(block_table), block_table.shape[1], M,
-              heads, dim, rot_dim, rank, int(write_cache), dtype_code(ref.dtype), _stream())
+              heads, dim, rot_dim, rank, int(write_cache), dtype_code((q if proj is None else proj).dtype), _stream())
     return q_full
 
 
@@ -1714,6 +1722,65 @@ def latent_decode_split(n_seqs: int, heads: int, max_len: int):
     want = max(1, min((max_len + 63) // 64, LATENT_SPLIT_WORKGROUPS // max(1, n_seqs * tiles)))
     size = ((max_len + want - 1) // want + 63) // 64 * 64
     return size, (max_len + size - 1) // size
+
+
+LATENT_DECODE = os.environ.get("PTA_LATENT_DECODE", "1") != "0"
+
+
+def latent_decode_ok(x: torch.Tensor, heads: int, dim: int, rot_dim: int, rank: int, value_dim: int) -> bool:
+    """Whether a decode step over latents runs in the three launches that are built for it (``latent_queries``,
+    ``latent_decode``): bfloat16, whole pieces of 32 elements, latents of up to 512.  PTA_LATENT_DECODE=0 switches it off."""
+    return (LATENT_DECODE and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= 65535
+            and bool(load_library().pta_latent_decode_ok(int(heads), int(dim), int(rot_dim), int(rank), int(value_dim))))
+
+
+def latent_queries(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor], eps: float, inv_freq, cs_scale: float, rotary_dim, pairing: str,
+                   token_pos, token_seq, block_table, k_pool, k_turned: torch.Tensor, heads: int, dim: int, rot_dim: int, rank: int,
+                   write_cache: bool, q: torch.Tensor) -> Optional[torch.Tensor]:
+    """``latent_prep`` of a decode step with the rest of the queries' frames filled in the same launch: ``k_turned`` ``[heads, rank,
+    dim]`` takes a head's plain query into the first ``rank`` of its frame.  None where the queries' rows do not lie as
+    sixteen-byte loads want them."""
+    _need(k_turned, "k_turned", torch.bfloat16, (heads, rank, dim))
+    M, q_ptr, q_ld, down_ptr, ld, rot, q_full = _latent_rows(proj, w_norm, inv_freq, cs_scale, rotary_dim, pairing, token_pos, token_seq,
+                                                             block_table, k_pool, heads, dim, rot_dim, rank, write_cache, q)
+    if q_ld.value % 8 or q_ptr.value % 16:
+        return None
+    _call("pta_latent_queries", _ptr(q_full), _ptr(k_pool), q_ptr, q_ld, down_ptr, ld, _ptr(w_norm), ctypes.c_float(eps), rot, _ptr(token_pos),
+          _ptr(token_seq), _ptr(block_table), block_table.shape[1], _ptr(k_turned), M, heads, dim, rot_dim, rank, int(write_cache), _stream())
+    return q_full
+
+
+def latent_ranges(n_seqs: int, heads: int, max_len: int) -> tuple:
+    """(keys per range, ranges) of ``latent_decode``: whole pages, as many ranges as give every compute unit a workgroup.  The
+    batch counts by its next power of two and the context by its bound, as a captured step has them."""
+    pages = (tuning.context_bound(int(max_len)) + 63) // 64
+    workgroups = (1 << max(int(n_seqs) - 1, 0).bit_length()) * ((heads + 15) // 16)
+    size = -(-pages // max(1, min(pages, 256 // workgroups, 1024)))
+    return 64 * size, -(-pages // size)
+
+
+def latent_decode(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, up_v: torch.Tensor, rank: int, scale: float, ctx) -> torch.Tensor:
+    """Attention of a decode step's tokens (one per sequence) over their cache rows and the value expansion ``up_v`` ``[heads,
+    value_dim, rank]``: ``q_full`` ``[tokens, heads, rank + rot_dim]`` (32-bit) -> ``[tokens, heads * value_dim]`` bfloat16."""
+    _need(q_full, "q_full", torch.float32)
+    M, H, D = q_full.shape
+    V = up_v.shape[1]
+    _need(up_v, "up_v", torch.bfloat16, (H, V, rank))
+    _need(k_pool, "k_pool", torch.bfloat16)
+    if k_pool.dim() != 4 or tuple(k_pool.shape[1:]) != (1, 64, D):
+        raise KernelError(f"k_pool must be [pages, 1, 64, {D}], got {tuple(k_pool.shape)}")
+    _need(block_table, "block_table", torch.int32)
+    _need(ctx.seq_start, "seq_start", torch.int32, (M,))
+    if block_table.shape[0] != M:
+        raise KernelError(f"{M} tokens of {block_table.shape[0]} sequences: a decode step has one token a sequence")
+    size, splits = latent_ranges(M, H, ctx.max_len)
+    out = torch.empty((M, H * V), dtype=torch.bfloat16, device=q_full.device)
+    po = torch.empty((M, H, splits, rank), dtype=torch.float32, device=q_full.device)
+    stats = torch.empty((2, M, H, splits), dtype=torch.float32, device=q_full.device)
+    _call("pta_latent_decode", _ptr(out), _ptr(po), _ptr(stats[0]), _ptr(stats[1]), _ptr(q_full), _ptr(k_pool), _ptr(block_table),
+          block_table.shape[1], _ptr(ctx.seq_start), _ptr(up_v), M, H, int(rank), D - int(rank), V, ctypes.c_float(scale), size, splits,
+          _stream())
+    return out
 
 
 def attn_latent(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, token_seq, token_pos, rank: int,

@@ -79,6 +79,8 @@ class LatentAttentionMixer(Part):
         # per head, with a head's rows its inputs: the key expansion as the file has it, the value expansion turned
         self.k_side = self.up_k.view(self.heads, self.dim, self.rank)
         self.v_side = self.up_v.view(self.heads, self.value_dim, self.rank).transpose(1, 2).contiguous()
+        # decode steps want the rows of both to be outputs
+        self.k_turned = self.k_side.transpose(1, 2).contiguous() if self.up_k.dtype == torch.bfloat16 else None
 
     def check_sizes(self) -> None:
         problem = ops.latent_sizes_problem(self.heads, self.dim, self.rot_dim, self.rank)
@@ -104,12 +106,32 @@ class LatentAttentionMixer(Part):
             queries, at = self.q(lat_q), self.q_rank
         else:
             queries, at = proj[:, :q_cols], q_cols
-        q_full = ops.latent_prep(proj[:, at:at + D] if made else None, self.norm_w, self.eps, None if rot is None else rot.inv_freq,
-                                 1.0 if rot is None else rot.scale, None if rot is None else rot.rotary_dim,
-                                 "half" if rot is None else rot.pairing, ctx.token_pos, ctx.token_seq, table, k_pool,
-                                 self.heads, self.dim, self.rot_dim, self.rank, write_cache=call.write_cache and not self.reads_other, q=queries)
+        rows = (proj[:, at:at + D] if made else None, self.norm_w, self.eps, None if rot is None else rot.inv_freq,
+                1.0 if rot is None else rot.scale, None if rot is None else rot.rotary_dim, "half" if rot is None else rot.pairing,
+                ctx.token_pos, ctx.token_seq, table, k_pool)
+        write = call.write_cache and not self.reads_other
         gate = proj[:, at + made:at + made + H * self.value_dim] if self.gate else None
-        library = x.dtype == torch.bfloat16 and M > ops.HEAD_PROJECT_LIBRARY_ROWS
+        o = self._decode(queries, rows, write, ctx) if ctx.is_decode else None
+        if o is None:
+            o = self._attend(queries, rows, write, ctx)
+        if gate is not None:
+            o = ops.gated_heads(o, self.value_dim, gate, H, self.value_dim, x.dtype)
+        return self.out(o, add1=residual)
+
+    def _decode(self, queries: torch.Tensor, rows, write: bool, ctx: StepContext) -> Optional[torch.Tensor]:
+        """The heads' results of a step of one token per sequence in three launches, where they are built for these sizes."""
+        if not ops.latent_decode_ok(queries, self.heads, self.dim, self.rot_dim, self.rank, self.value_dim):
+            return None
+        q_full = ops.latent_queries(*rows, self.k_turned, self.heads, self.dim, self.rot_dim, self.rank, write_cache=write, q=queries)
+        if q_full is None:
+            return None
+        return ops.latent_decode(q_full, rows[-1], rows[-2], self.up_v.view(self.heads, self.value_dim, self.rank), self.rank, self.scale, ctx)
+
+    def _attend(self, queries: torch.Tensor, rows, write: bool, ctx: StepContext) -> torch.Tensor:
+        """The heads' results of any step."""
+        H, D, M, dtype, k_pool = self.heads, self.cache_row, queries.shape[0], queries.dtype, rows[-1]
+        q_full = ops.latent_prep(*rows, H, self.dim, self.rot_dim, self.rank, write_cache=write, q=queries)
+        library = dtype == torch.bfloat16 and M > ops.HEAD_PROJECT_LIBRARY_ROWS
         # each head's plain query through the transpose of its key expansion: the first `rank` of its frame
         if library:
             plain = queries.unflatten(1, (H, self.dim + self.rot_dim))[:, :, :self.dim]
@@ -117,15 +139,10 @@ class LatentAttentionMixer(Part):
         else:
             ops.head_project(queries, self.dim + self.rot_dim, self.k_side, H, self.dim, self.rank,
                              out=q_full.view(M, H * D), out_head=D)
-        lat = ops.attn_latent(q_full, k_pool, table, ctx.token_seq, ctx.token_pos, self.rank, self.scale, ctx=ctx)
+        lat = ops.attn_latent(q_full, k_pool, rows[-2], ctx.token_seq, ctx.token_pos, self.rank, self.scale, ctx=ctx)
         if library:
-            o = ops.head_project_library(lat.to(x.dtype), self.v_side).transpose(0, 1).reshape(M, H * self.value_dim)
-        else:
-            o = ops.head_project(lat.view(M, H * self.rank), self.rank, self.v_side, H, self.rank, self.value_dim,
-                                 out_dtype=x.dtype)
-        if gate is not None:
-            o = ops.gated_heads(o, self.value_dim, gate, H, self.value_dim, x.dtype)
-        return self.out(o, add1=residual)
+            return ops.head_project_library(lat.to(dtype), self.v_side).transpose(0, 1).reshape(M, H * self.value_dim)
+        return ops.head_project(lat.view(M, H * self.rank), self.rank, self.v_side, H, self.rank, self.value_dim, out_dtype=dtype)
 
 
 register_part("mixer", "latent_attention", LatentAttentionMixer)
