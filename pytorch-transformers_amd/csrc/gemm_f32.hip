@@ -10,12 +10,13 @@
 // and how many workgroups share the segments changes nothing.
 //
 // Measured at 4,544 / 18,176 features (one kernel of 64 x 64 tiles on the vector units before): one row of A 986 -> 56 us a
-// product on average (28 us for 83 MB, 71 us = 4.7 TB/s for 330 MB); 2,053 rows 26 -> 98 to 110 TFLOP/s.
+// product on average (28 us for 83 MB, 71 us = 4.7 TB/s for 330 MB); 2,053 rows 26 -> 103 to 131 TFLOP/s.
 //
 // Three ways to the same numbers, by what bounds them:
-//   few rows (M <= 64): every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight
+//   few rows (M <= 32, with a short K 64): every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight
 //     waves a segment each; W goes from memory straight into the instruction's operands, the sums meet in LDS.
-//   many rows: tiles of 128 x 128 or 64 x 64 through two LDS buffers, bound by the matrix instruction.
+//   many rows: tiles of 128 x 128 or 64 x 64 through two LDS buffers, bound by the matrix instruction (loads straight to LDS
+//     where rows are sixteen-byte aligned, else through registers).
 //   in between, or N small: too few tiles to fill the chip, so the segments of a tile are shared out over workgroups, whose
 //     sums go to memory and are added by a small launch.
 #include "common.h"
@@ -24,7 +25,8 @@
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
 #define SEGS 8          // segments of K, at most
-#define SKINNY_ROWS 64  // rows of A up to which the kernel for few rows runs
+#define SKINNY_ROWS 32  // rows of A up to which the kernel for few rows runs
+#define SHARE_K 1024    // K from which segments may be shared out over workgroups
 
 struct F32Epilogue {
     const float* bias;
@@ -73,7 +75,6 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
     const int r16 = lane & 15, kq = 4 * (lane >> 4);
     // the rows of W are shared out evenly: a launch takes as long as the compute unit with the most of them
     const int n0 = (int)((long)blockIdx.x * N / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * N / gridDim.x);
-    const int m0 = blockIdx.y * SKINNY_ROWS;
     const int nb = (K + 15) / 16, sb = seg_blocks(K);
     const int b0 = seg * sb, b1 = min(nb, b0 + sb);
     const float* wr[RT];
@@ -81,7 +82,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 #pragma unroll
     for (int r = 0; r < RT; ++r) wr[r] = W + (long)min(n0 + 16 * r + r16, n1 - 1) * K;  // rows past the end: read again, not kept
 #pragma unroll
-    for (int c = 0; c < CT; ++c) xr[c] = A + (long)min(m0 + 16 * c + r16, M - 1) * K;
+    for (int c = 0; c < CT; ++c) xr[c] = A + (long)min(16 * c + r16, M - 1) * K;
     f32x4 acc[RT][CT];
 #pragma unroll
     for (int r = 0; r < RT; ++r)
@@ -136,7 +137,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 #pragma unroll
             for (int j = 0; j < 4; ++j) v[j] += p[j];
         }
-        const int m = m0 + 16 * (t % CT) + (l & 15);
+        const int m = 16 * (t % CT) + (l & 15);
         const int n = n0 + 16 * (t / CT) + 4 * (l >> 4);
         if (m < M) {
 #pragma unroll
@@ -152,7 +153,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 #define BK 32
 #define PITCH 36
 
-template <int T, int ROWS, bool SPLIT>
+template <int T, bool SPLIT>
 __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ A,
                                                                const float* __restrict__ W, F32Epilogue epi, int M, int N,
                                                                int K, int tiles_m, int tiles_n) {
@@ -192,12 +193,12 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict
         pw[i] = W + (long)min(n0 + row, N - 1) * K;
     }
     const int kc = 4 * (tid & 7);
-    auto fetch = [&](int b) {  // blocks b and b + 1 (whole blocks: the second may lie past K, is read from before it and not used)
-        const int k = ROWS == ROW_WHOLE ? min(16 * b + kc, K - 4) : 16 * b + kc;
+    auto fetch = [&](int b) {  // blocks b and b + 1
+        const int k = 16 * b + kc;
 #pragma unroll
         for (int i = 0; i < L; ++i) {
-            ra[i] = load4<ROWS>(pa[i], k, K);
-            rw[i] = load4<ROWS>(pw[i], k, K);
+            ra[i] = load4<ROW_ELEMENTS>(pa[i], k, K);
+            rw[i] = load4<ROW_ELEMENTS>(pw[i], k, K);
         }
     };
     auto stage = [&](int buf) {
@@ -278,6 +279,149 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict
     if (!SPLIT) store_all(total, C, true);
 }
 
+// The same tiles where rows can be read sixteen bytes at a time (rows sixteen-byte aligned, K a multiple of 4), loads going
+// straight to LDS.  A row of a tile is 32 elements of K, 128 bytes without a gap: sixteen bytes c of row r lie at place
+// c ^ (r % 8), so that the eight lanes that read together cover every bank once.
+//
+// What bounds it is the matrix instruction (32 cycles each); the kernel above, which stages through registers and reads a
+// block's operands right before their products, keeps it busy 80 % of the time a workgroup is there.  Here operands of a
+// block are read while the block before is multiplied, and the loads of a step have the whole step before it to arrive:
+// 8,192 x 8,192 x 4,096 124 -> 139 TFLOP/s, 2,053 rows by 4,544 x 4,544 90 -> 113, by 18,176 x 4,544 110 -> 131.
+// TAIL: K is no multiple of 16, what a block holds past it has to be zero.
+
+// sixteen bytes a lane from byte `at` of an array of `bytes` into LDS, one lane after the other; zeros from its end on
+__device__ __forceinline__ void to_lds(const float* src, int bytes, float* dst, int at) {
+    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, bytes, 0x00020000);
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, at, 0, 0, 0);
+}
+
+template <int T, bool TAIL, bool SPLIT>
+__global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(float* __restrict__ C, const float* __restrict__ A,
+                                                                 const float* __restrict__ W, F32Epilogue epi, int M, int N,
+                                                                 int K, int tiles_m, int tiles_n) {
+    constexpr int F = T / 32;       // tiles of sixteen rows per wave and side
+    constexpr int L = T * 8 / 256;  // sixteen-byte loads per thread and side
+    // A's rows, then W's; two arrays, so that the compiler sees which of them a load is on its way to
+    __shared__ __attribute__((aligned(1024))) float lds0[2 * T * BK];
+    __shared__ __attribute__((aligned(1024))) float lds1[2 * T * BK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int r16 = lane & 15, kq = 4 * (lane >> 4);
+    const int tiles = tiles_m * tiles_n;
+    const int per = (tiles + 7) / 8;
+    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
+    if ((int)(blockIdx.x >> 3) >= per || tile >= tiles) return;
+    const int m0 = (tile % tiles_m) * T, n0 = (tile / tiles_m) * T;
+    const int wn = (wave & 1) * (T / 2), wm = (wave >> 1) * (T / 2);
+    const int nb = (K + 15) / 16, sb = seg_blocks(K);
+    const int used = (nb + sb - 1) / sb;
+    const int s0 = SPLIT ? (int)((long)blockIdx.y * used / gridDim.y) : 0;
+    const int s1 = SPLIT ? (int)((long)(blockIdx.y + 1) * used / gridDim.y) : used;
+    const int b_first = s0 * sb, b_last = min(nb, s1 * sb);
+
+    f32x4 acc[F][F], total[F][F];
+#pragma unroll
+    for (int i = 0; i < F; ++i)
+#pragma unroll
+        for (int j = 0; j < F; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const float* at_a = A + (long)m0 * K;
+    const float* at_w = W + (long)n0 * K;
+    const int bytes_a = min(T, M - m0) * K * 4, bytes_w = min(T, N - n0) * K * 4;
+    const int trow = tid >> 3, kc = 4 * ((tid & 7) ^ (trow & 7));
+    // blocks b and b + 1; rows past the last are zeros, what the second block holds past K is not used; past b_last nothing is read
+    auto fetch = [&](float* buf, int b) __attribute__((always_inline)) {
+        const int k = 16 * b + kc;
+#pragma unroll
+        for (int i = 0; i < L; ++i) {
+            const int at = TAIL && k >= K ? -16 : ((trow + 32 * i) * K + k) * 4;
+            to_lds(at_a, b < b_last ? bytes_a : 0, buf + (32 * i + 8 * wave) * BK, at);
+            to_lds(at_w, b < b_last ? bytes_w : 0, buf + (T + 32 * i + 8 * wave) * BK, at);
+        }
+    };
+    f32x4 w[2][F], x[2][F];
+    const int place[2] = {4 * ((lane >> 4) ^ (r16 & 7)), 4 * ((4 + (lane >> 4)) ^ (r16 & 7))};
+    auto read = [&](const float* buf, int h) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < F; ++i) {
+            x[h][i] = *(const f32x4*)&buf[(wm + 16 * i + r16) * BK + place[h]];
+            w[h][i] = *(const f32x4*)&buf[(T + wn + 16 * i + r16) * BK + place[h]];
+        }
+    };
+    auto store_all = [&](const f32x4 (&v)[F][F], float* to, bool last) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < F; ++i)
+#pragma unroll
+            for (int j = 0; j < F; ++j) {
+                const int n = n0 + wn + 16 * i + kq, m = m0 + wm + 16 * j + r16;
+                if (m >= M) continue;
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    if (n + e < N) to[(long)m * N + n + e] = last ? finish(v[i][j][e], epi, n + e, (long)m * N + n + e) : v[i][j][e];
+            }
+    };
+    int left = sb, segs = 0;  // blocks left of the segment, segments finished
+    auto multiply = [&](int h, int b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int c = 0; c < F; ++c)
+                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][i][j], x[h][c][j], acc[i][c], 0, 0, 0);
+        if (--left == 0 || b + 1 == b_last) {  // the segment ends: its sum joins the others in their order
+            if (SPLIT) {
+                store_all(acc, C + (long)(s0 + segs) * M * N, false);
+            } else {
+                const bool first = segs == 0;
+#pragma unroll
+                for (int i = 0; i < F; ++i)
+#pragma unroll
+                    for (int c = 0; c < F; ++c)
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) total[i][c][e] = first ? acc[i][c][e] : total[i][c][e] + acc[i][c][e];
+            }
+#pragma unroll
+            for (int i = 0; i < F; ++i)
+#pragma unroll
+                for (int c = 0; c < F; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+            ++segs;
+            left = sb;
+        }
+    };
+    // Blocks b and b + 1 out of `cur`.  Everyone has read all of it when its second block is multiplied: then it takes the loads
+    // of the step after next, and the next step's first block is read.
+    auto step = [&](float* cur, const float* next, int b) __attribute__((always_inline)) {
+        read(cur, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b < b_last) multiply(0, b);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070);  // this wave's reads of `cur` are done, its loads into `next` have landed
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        fetch(cur, b + 4);
+        read(next, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        if (b + 1 < b_last) multiply(1, b + 1);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    if (b_first < b_last) {
+        fetch(lds0, b_first);
+        fetch(lds1, b_first + 2);
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0x0070);
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        read(lds0, 0);
+        for (int b = b_first; b < b_last; b += 4) {
+            step(lds0, lds1, b);
+            step(lds1, lds0, b + 2);
+        }
+        __builtin_amdgcn_s_waitcnt(0x0070);  // nothing is on its way to LDS when the workgroup ends
+    }
+    if (!SPLIT) store_all(total, C, true);
+}
+
 // the segments' sums added in order, and the epilogue
 __global__ void gemm_f32_add_kernel(float* __restrict__ C, const float* __restrict__ part, F32Epilogue epi, int segs, long MN, int N) {
     const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
@@ -290,15 +434,18 @@ __global__ void gemm_f32_add_kernel(float* __restrict__ C, const float* __restri
 // How a product runs: the tile's side (0: the kernel for few rows) and over how many workgroups a tile's segments are shared.
 static void f32_plan(int M, int N, int K, int* tile, int* share) {
     *tile = 0, *share = 1;
-    if (M <= SKINNY_ROWS) return;
+    // 33 rows by 4,544 x 4,544: 61 us with the kernel for few rows, 36 with shared tiles; 17 rows: 35 and 51; 33 rows by 256 x
+    // 512, whose segments are too short to be shared: 7 and 13
+    if (M <= (K < SHARE_K ? 2 * SKINNY_ROWS : SKINNY_ROWS)) return;
     const int cus = 256;
     auto tiles = [&](long t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
     auto rounds = [&](long n) { return (double)((n + cus - 1) / cus); };
-    // time of a round: a tile of 128 is four of 64; the smaller tile reads twice as much per product
-    const double big = 4.0 * rounds(tiles(128)), small = 1.1 * rounds(tiles(64));
+    // time of a round: a tile of 128 is four of 64, which read twice as much per product (8,192 x 8,192 x 4,096: 139 and
+    // 134 TFLOP/s; 2,053 x 4,544 x 4,544, where 128 leaves the last round half empty: 101 and 119)
+    const double big = 4.0 * rounds(tiles(128)), small = 1.04 * rounds(tiles(64));
     *tile = big <= small ? 128 : 64;
     const int used = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
-    if (*tile == 64 && K >= 1024)  // a chip that is not filled twice: share the segments out
+    if (*tile == 64 && K >= SHARE_K)  // a chip that is not filled twice: share the segments out
         while (*share < used && tiles(64) * *share < 2 * cus) *share *= 2;
     if (*share > used) *share = used;
 }
@@ -318,26 +465,32 @@ static void launch_few(float* C, const float* A, const float* W, const F32Epilog
     int groups = 256 * ((N + 256 * 32 - 1) / (256 * 32));
     if (groups > (N + 3) / 4) groups = (N + 3) / 4;
     const bool two = (N + groups - 1) / groups > 16;
-    const dim3 grid(groups, (M + SKINNY_ROWS - 1) / SKINNY_ROWS);
-    const int ct = (M < SKINNY_ROWS ? M : SKINNY_ROWS) <= 16 ? 1 : M <= 32 ? 2 : 4;
-#define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), grid, dim3(512), 0, s, C, A, W, epi, M, N, K)
-    if (ct == 1) { if (two) FEW(1, 2, 4); else FEW(1, 1, 4); }
-    else if (ct == 2) { if (two) FEW(2, 2, 4); else FEW(2, 1, 4); }
+#define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), dim3(groups), dim3(512), 0, s, C, A, W, epi, M, N, K)
+    if (M <= 16) { if (two) FEW(1, 2, 4); else FEW(1, 1, 4); }
+    else if (M <= 32) { if (two) FEW(2, 2, 4); else FEW(2, 1, 4); }
     else { if (two) FEW(4, 2, 2); else FEW(4, 1, 2); }
 #undef FEW
 }
 
-template <int ROWS>
 static void launch_tiles(float* C, float* scratch, const float* A, const float* W, const F32Epilogue& epi, int M, int N, int K,
-                         int tile, int share, hipStream_t s) {
+                         int tile, int share, bool vec, hipStream_t s) {
     const int tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
     const int groups = 8 * ((tm * tn + 7) / 8);
+    // offsets within a tile's rows are 32-bit bytes
+    const bool stream = vec && (long)(128 + 2) * K * 4 < (1L << 31);
+#define LAUNCH(KERNEL, SPLIT, OUT) \
+    hipLaunchKernelGGL(KERNEL, dim3(groups, SPLIT ? share : 1), dim3(256), 0, s, OUT, A, W, epi, M, N, K, tm, tn)
 #define TILE(T, SPLIT, OUT) \
-    hipLaunchKernelGGL((gemm_f32_tile_kernel<T, ROWS, SPLIT>), dim3(groups, SPLIT ? share : 1), dim3(256), 0, s, OUT, A, W, epi, M, N, K, tm, tn)
+    do { \
+        if (!stream) LAUNCH((gemm_f32_tile_kernel<T, SPLIT>), SPLIT, OUT); \
+        else if (K % 16) LAUNCH((gemm_f32_stream_kernel<T, true, SPLIT>), SPLIT, OUT); \
+        else LAUNCH((gemm_f32_stream_kernel<T, false, SPLIT>), SPLIT, OUT); \
+    } while (0)
     if (share > 1) TILE(64, true, scratch);
     else if (tile == 128) TILE(128, false, C);
     else TILE(64, false, C);
 #undef TILE
+#undef LAUNCH
     if (share > 1) {
         const long mn = (long)M * N;
         const int segs = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
@@ -359,7 +512,7 @@ extern "C" int pta_gemm_f32(float* C, const float* A, const float* W, const floa
     hipStream_t s = (hipStream_t)stream;
 #define BY_ROWS(FN, ...) (vec && K % 16 == 0 ? FN<ROW_WHOLE>(__VA_ARGS__) : vec ? FN<ROW_VECTORS>(__VA_ARGS__) : FN<ROW_ELEMENTS>(__VA_ARGS__))
     if (tile == 0) BY_ROWS(launch_few, C, A, W, epi, M, N, K, s);
-    else BY_ROWS(launch_tiles, C, scratch, A, W, epi, M, N, K, tile, share, s);
+    else launch_tiles(C, scratch, A, W, epi, M, N, K, tile, share, vec, s);
 #undef BY_ROWS
     return pta_check_launch("gemm_f32");
 }

@@ -19,9 +19,10 @@ def _rand(*shape, seed=0):
     return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).cuda()
 
 
-@pytest.mark.parametrize("N,K", [(1, 1), (40, 15), (129, 16), (260, 100), (64, 1040), (4544, 576), (8200, 300), (96, 2050)])
+@pytest.mark.parametrize("N,K", [(1, 1), (40, 15), (129, 16), (260, 100), (64, 1040), (4544, 576), (8200, 300), (96, 2050),
+                                 (5376, 100), (5376, 48), (70, 1044)])
 def test_products(N, K):
-    """Rows 1 .. 700 (few rows with one, two and four tiles; 64 and 128 tiles; shared segments), K with and without a last
+    """Rows 1 .. 700 (few rows with one, two and four tiles; 64 and, at 5376 columns, 128 tiles; shared segments), K with and without a last
     block and rows that are no multiple of sixteen bytes."""
     ops = _ops()
     M = 700
