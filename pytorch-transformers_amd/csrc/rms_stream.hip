@@ -134,6 +134,91 @@ __global__ void rmsnorm_reg_kernel(T* __restrict__ out_narrow, float* __restrict
     }
 }
 
+// four neighbouring elements, loaded and stored at once
+__device__ __forceinline__ void ld4(const float* p, float (&v)[4]) {
+    const float4 q = *reinterpret_cast<const float4*>(p);
+    v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w;
+}
+__device__ __forceinline__ void ld4(const bf16_t* p, float (&v)[4]) {
+    const uint2 q = *reinterpret_cast<const uint2*>(p);
+    v[0] = bf16_bits_to_f32((bf16_t)(q.x & 0xffffu)); v[1] = bf16_bits_to_f32((bf16_t)(q.x >> 16));
+    v[2] = bf16_bits_to_f32((bf16_t)(q.y & 0xffffu)); v[3] = bf16_bits_to_f32((bf16_t)(q.y >> 16));
+}
+__device__ __forceinline__ void st4(float* p, const float (&v)[4]) { *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]); }
+__device__ __forceinline__ void st4(bf16_t* p, const float (&v)[4]) {
+    *reinterpret_cast<uint2*>(p) = make_uint2((uint32_t)f32_to_bf16_bits(v[0]) | ((uint32_t)f32_to_bf16_bits(v[1]) << 16),
+                                              (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
+}
+
+// The same where rows can be read four elements at a time (C times four a thread, at most 8,192 a group).  In a step of a
+// few rows the launch is one chain (load, sum over the workgroup, store) and its length is instructions as much as trips to
+// memory: 2,048 features of 8 rows 3.4 -> 2.4 us (with a gate 4.5 -> 2.9); of 2,000 rows 9.5 -> 6.0 us.
+template <typename TI, typename T, int C>
+__global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(T* __restrict__ out_narrow, float* __restrict__ out_wide,
+                                                           const TI* __restrict__ x, long x_ld, const T* __restrict__ gate,
+                                                           long gate_ld, const int* __restrict__ rows, const float* __restrict__ w,
+                                                           float offset, int group_len, float eps,
+                                                           const float* __restrict__ residual, float mult, int H,
+                                                           const float* __restrict__ planes, long plane,
+                                                           const float* __restrict__ coef, int count, float* __restrict__ mix_wide) {
+    __shared__ float red[16];
+    const int m = blockIdx.x, g = blockIdx.y;
+    const long src = rows ? rows[m] : m;
+    const TI* xr = x + src * x_ld + (long)g * group_len;
+    const T* gr = gate ? gate + src * gate_ld + (long)g * group_len : nullptr;
+    const float* wr = w + (long)g * group_len;
+    const float* rr = residual ? residual + src * H + (long)g * group_len : nullptr;
+    const long o = (long)m * H + (long)g * group_len;
+    float v[C][4], z[C][4], wv[C][4], rv[C][4];
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int i = 4 * (threadIdx.x + c * blockDim.x);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[c][e] = z[c][e] = 0.f;
+        if (i < group_len) {
+            ld4(xr + i, v[c]);
+            if (gr) ld4(gr + i, z[c]);
+            ld4(wr + i, wv[c]);
+            if (rr) ld4(rr + i, rv[c]);
+        }
+    }
+    float ss = 0.f;
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (gr) v[c][e] *= z[c][e] / (1.0f + expf(-z[c][e]));
+            ss += v[c][e] * v[c][e];
+        }
+    ss = block_sum(ss, red);
+    const float inv = 1.0f / sqrtf(ss / (float)group_len + eps);
+#pragma unroll
+    for (int c = 0; c < C; ++c) {
+        const int i = 4 * (threadIdx.x + c * blockDim.x);
+        if (i >= group_len) continue;
+        float n[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            n[e] = v[c][e] * inv * (offset + wv[c][e]);
+            if (rr) n[e] = rv[c][e] + mult * n[e];
+        }
+        if (out_wide) st4(out_wide + o + i, n);
+        if (planes) {
+            float acc[4] = {0.f, 0.f, 0.f, 0.f}, pv[4];
+#pragma unroll 8
+            for (int j = 0; j + 1 < count; ++j) {
+                ld4(planes + (long)j * plane + o + i, pv);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[e] += coef[j] * pv[e];
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) n[e] = acc[e] + coef[count - 1] * n[e];
+            st4(mix_wide + o + i, n);
+        }
+        if (out_narrow) st4(out_narrow + o + i, n);
+    }
+}
+
 extern "C" int pta_rmsnorm(void* out_narrow, float* out_wide, const void* x, int x_wide, long x_ld, const void* gate,
                            long gate_ld, const int* rows, const float* w, float offset, int groups, float eps,
                            const float* residual, float mult, const float* planes, long plane, const float* coef,
@@ -151,6 +236,23 @@ extern "C" int pta_rmsnorm(void* out_narrow, float* out_wide, const void* x, int
     const dim3 grid(M, groups), block(L >= 2048 ? 512 : L > 64 ? 256 : 64);
 #define RMS_ARGS(TN, TX, TG) (TN*)out_narrow, out_wide, (const TX*)x, x_ld, (const TG*)gate, gate_ld, rows, w, offset, L, eps, \
                              residual, mult, H, planes, plane, coef, count, mix_wide
+    // rows, groups and planes start at a multiple of four elements: what every width in use gives.  Groups beyond 8,192 take
+    // the kernel that reads its row twice, rows that start anywhere the one above it.
+    auto on = [](const void* p, size_t bytes) { return (uintptr_t)p % bytes == 0; };
+    const size_t narrow = dtype == PTA_F32 ? 16 : 8;
+    if (L % 4 == 0 && L <= 8192 && x_ld % 4 == 0 && (!gate || gate_ld % 4 == 0) && plane % 4 == 0 && on(w, 16) && on(residual, 16) &&
+        on(out_wide, 16) && on(planes, 16) && on(mix_wide, 16) && on(gate, narrow) && on(out_narrow, narrow) &&
+        on(x, x_wide ? 16 : narrow)) {
+        const int threads = (L / 4 + 63) / 64 * 64;
+#define RMS_VEC(TX, T, C) hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, T, C>), grid, dim3((threads / C + 63) / 64 * 64), 0, s, RMS_ARGS(T, TX, T))
+#define RMS_VEC_C(TX, T) if (threads <= 1024) RMS_VEC(TX, T, 1); else RMS_VEC(TX, T, 2)
+        if (dtype == PTA_F32) { RMS_VEC_C(float, float); }
+        else if (x_wide) { RMS_VEC_C(float, bf16_t); }
+        else { RMS_VEC_C(bf16_t, bf16_t); }
+#undef RMS_VEC_C
+#undef RMS_VEC
+        return pta_check_launch("rmsnorm");
+    }
     if (L <= 8 * (int)block.x) {  // the group fits the threads' registers
         if (dtype == PTA_F32) hipLaunchKernelGGL((rmsnorm_reg_kernel<float, float, 8>), grid, block, 0, s, RMS_ARGS(float, float, float));
         else if (x_wide) hipLaunchKernelGGL((rmsnorm_reg_kernel<float, bf16_t, 8>), grid, block, 0, s, RMS_ARGS(bf16_t, float, bf16_t));
