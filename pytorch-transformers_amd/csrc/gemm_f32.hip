@@ -5,8 +5,8 @@
 // Order of summation.  A row's result is bitwise the same alone and in any batch, so every kernel here sums the products
 // of an output in one order, which K alone decides: K is walked in blocks of sixteen elements (the last one filled up with
 // zeros), the blocks are cut into up to eight segments of equal length, a segment is one chain of matrix instructions
-// (instruction j of a block takes elements j, 4 + j, 8 + j and 12 + j of it, so that a lane's four operands are sixteen
-// consecutive bytes of a row), and the segments' sums are added in order.  Where a row lies in the grid, which kernel runs
+// (a block is four instructions; each takes one element in four, from 3, 7, 11 and 15 down to 0, 4, 8 and 12, so that a
+// lane's four operands are sixteen consecutive bytes of a row), and the segments' sums are added in order.  Where a row lies in the grid, which kernel runs
 // and how many workgroups share the segments changes nothing.
 //
 // Measured at 4,544 / 18,176 features (one kernel of 64 x 64 tiles on the vector units before): one row of A 986 -> 56 us a
@@ -110,7 +110,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
                     for (int r = 0; r < RT; ++r)
 #pragma unroll
                         for (int c = 0; c < CT; ++c)
-                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[buf][i][r][j], x[buf][i][c][j], acc[r][c], 0, 0, 0);
+                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[buf][i][r][3 - j], x[buf][i][c][3 - j], acc[r][c], 0, 0, 0);
             }
         }
     };
@@ -245,7 +245,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict
                     for (int i = 0; i < F; ++i)
 #pragma unroll
                         for (int c = 0; c < F; ++c)
-                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][j], x[c][j], acc[i][c], 0, 0, 0);
+                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][3 - j], x[c][3 - j], acc[i][c], 0, 0, 0);
                 if (--left == 0 || b + h + 1 == b_last) {  // the segment ends: its sum joins the others in their order
                     if (SPLIT) {
                         store_all(acc, C + (long)(s0 + segs) * M * N, false);
@@ -367,7 +367,7 @@ __global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(float* __restri
             for (int i = 0; i < F; ++i)
 #pragma unroll
                 for (int c = 0; c < F; ++c)
-                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][i][j], x[h][c][j], acc[i][c], 0, 0, 0);
+                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][i][3 - j], x[h][c][3 - j], acc[i][c], 0, 0, 0);
         if (--left == 0 || b + 1 == b_last) {  // the segment ends: its sum joins the others in their order
             if (SPLIT) {
                 store_all(acc, C + (long)(s0 + segs) * M * N, false);
