@@ -184,12 +184,12 @@ __global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(T* __restrict__ out_n
     }
     float ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < C; ++c)
+    for (int c = 0; c < C; ++c) {
 #pragma unroll
-        for (int e = 0; e < 4; ++e) {
+        for (int e = 0; e < 4; ++e)
             if (gr) v[c][e] *= z[c][e] / (1.0f + expf(-z[c][e]));
-            ss += v[c][e] * v[c][e];
-        }
+        ss += (v[c][0] * v[c][0] + v[c][1] * v[c][1]) + (v[c][2] * v[c][2] + v[c][3] * v[c][3]);
+    }
     ss = block_sum(ss, red);
     const float inv = 1.0f / sqrtf(ss / (float)group_len + eps);
 #pragma unroll
@@ -236,11 +236,12 @@ extern "C" int pta_rmsnorm(void* out_narrow, float* out_wide, const void* x, int
     const dim3 grid(M, groups), block(L >= 2048 ? 512 : L > 64 ? 256 : 64);
 #define RMS_ARGS(TN, TX, TG) (TN*)out_narrow, out_wide, (const TX*)x, x_ld, (const TG*)gate, gate_ld, rows, w, offset, L, eps, \
                              residual, mult, H, planes, plane, coef, count, mix_wide
-    // rows, groups and planes start at a multiple of four elements: what every width in use gives.  Groups beyond 8,192 take
-    // the kernel that reads its row twice, rows that start anywhere the one above it.
+    // Rows, groups and planes start at a multiple of four elements: what every width in use gives.  Groups below 512 elements
+    // are one or two a thread in the kernel for rows that start anywhere and stay there, groups beyond 8,192 take the one that
+    // reads its row twice.
     auto on = [](const void* p, size_t bytes) { return (uintptr_t)p % bytes == 0; };
     const size_t narrow = dtype == PTA_F32 ? 16 : 8;
-    if (L % 4 == 0 && L <= 8192 && x_ld % 4 == 0 && (!gate || gate_ld % 4 == 0) && plane % 4 == 0 && on(w, 16) && on(residual, 16) &&
+    if (L % 4 == 0 && L >= 512 && L <= 8192 && x_ld % 4 == 0 && (!gate || gate_ld % 4 == 0) && plane % 4 == 0 && on(w, 16) && on(residual, 16) &&
         on(out_wide, 16) && on(planes, 16) && on(mix_wide, 16) && on(gate, narrow) && on(out_narrow, narrow) &&
         on(x, x_wide ? 16 : narrow)) {
         const int threads = (L / 4 + 63) / 64 * 64;
