@@ -12,26 +12,71 @@
 // Key pages are [kv_head][64 positions][d]; value pages are transposed, [kv_head][d][64 positions].
 //
 // One workgroup per token: the cosines and sines of the token's position are computed once into
-// LDS and used by every head; then the threads walk (head, element) items of the whole fused row.
+// LDS and used by every head; then the threads walk (head, element) items of the whole fused row.  In steps of many tokens
+// the values go by a launch of their own (value_pages_kernel).
 #include "common.h"
 #include "pta_kernels.h"
 #include "qkv_tail.h"
 
+#include <algorithm>
+
 #define RC_THREADS 256
+// Values of a step (tokens x kv heads x head size) from which they go by a launch of their own: below some two million it
+// costs what it gives (2,048 tokens of 1 x 64: 10 us in one launch, 16 in two; 1,000 of 8 x 128: 13 and 13; 4,800 of 8 x 64:
+// 38 and 36; 24,000 of 8 x 128: 338 and 156).
+#define VALUES_APART (1L << 21)
+
+// which head of a fused row holds query (kind 0), key (1) or value (2) `head`; g: heads / kv heads
+__device__ __forceinline__ int fused_head(int layout, int nh, int g, int kind, int head) {
+    if (layout == PTA_QKV_GROUPED) return kind == 0 ? (head / g) * (g + 2) + (head % g) : head * (g + 2) + g + (kind ? kind - 1 : 0);
+    if (layout == PTA_QKV_TAIL) return kind == 0 ? head : nh + kind - 1;
+    return head * 3 + kind;
+}
+
+// Values of many tokens into their pages.  A page holds an element's 64 positions side by side, so a token alone writes
+// single elements 128 bytes apart, and neighbouring tokens, on other dies, write into the same lines.  Here a workgroup
+// takes 64 tokens (of any sequences) and 64 elements of a head through LDS and a lane keeps to a token: a store is
+// 64 tokens' worth of one element, whole lines where the tokens are neighbours.
+template <typename T>
+__global__ __launch_bounds__(RC_THREADS) void value_pages_kernel(const T* __restrict__ fused, long fused_ld,
+                                                                 const float* __restrict__ bias, const int* __restrict__ token_pos,
+                                                                 const int* __restrict__ token_seq,
+                                                                 const int* __restrict__ block_table, int bt_stride,
+                                                                 T* __restrict__ v_pool, int M, int nh, int nkv, int d, int layout) {
+    constexpr int PITCH = sizeof(T) == 2 ? 66 : 65;  // rows an odd number of banks apart
+    __shared__ T tile[64 * PITCH];
+    const int chunks = (d + 63) / 64, head = blockIdx.y / chunks, i0 = (blockIdx.y % chunks) * 64, n = min(64, d - i0);
+    const int m0 = blockIdx.x * 64, tokens = min(64, M - m0);
+    const int src = fused_head(layout, nh, nh / nkv, 2, head) * d + i0;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    for (int t = wave; t < tokens; t += RC_THREADS / 64)
+        if (lane < n) {
+            float a = Io<T>::ld(fused + (long)(m0 + t) * fused_ld + src + lane);
+            if (bias) a = Io<T>::round(a + bias[src + lane]);
+            Io<T>::st(&tile[t * PITCH + lane], a);
+        }
+    const int m = m0 + min(lane, tokens - 1), pos = token_pos[m];
+    const long page = block_table[(long)token_seq[m] * bt_stride + pos / PTA_PAGE];
+    T* to = v_pool + ((page * nkv + head) * (long)d + i0) * PTA_PAGE + pos % PTA_PAGE;
+    __syncthreads();
+    if (lane >= tokens) return;
+#pragma unroll 4
+    for (int i = wave; i < n; i += RC_THREADS / 64) to[i * PTA_PAGE] = tile[lane * PITCH + i];
+}
 
 template <typename T>
 __global__ __launch_bounds__(RC_THREADS) void qkv_rope_cache_kernel(
     T* __restrict__ q_out, const T* __restrict__ fused, long fused_ld, const float* __restrict__ bias,
     PtaRotation rot, const int* __restrict__ token_pos,
     const int* __restrict__ token_seq, const int* __restrict__ block_table, int bt_stride, T* __restrict__ k_pool,
-    T* __restrict__ v_pool, int nh, int nkv, int d, int layout, int write_cache) {
+    T* __restrict__ v_pool, int nh, int nkv, int d, int layout, int write_cache, int write_values) {
     __shared__ float cos_s[128], sin_s[128];
     const int m = blockIdx.x, tid = threadIdx.x;
     const int g = nh / nkv;
     const int R = rot.inv_freq ? rot.rotary_dim : 0, half = R >> 1;  // rotated elements of a head, and their pairs
     const int pos = token_pos[m];
     const T* row = fused + (long)m * fused_ld;  // rows of the fused projection may lie apart
-    const int n_slots = write_cache ? nh + 2 * nkv : nh;  // queries, then keys, then values
+    const int n_slots = write_cache ? nh + nkv + (write_values ? nkv : 0) : nh;  // queries, then keys, then values
     // rotated items: (slot < nh + nkv, pair i < half); plain items: every other element of every slot
     const int rot_slots = R ? min(n_slots, nh + nkv) : 0;
     // gridDim.y workgroups share a token's items (a decode step has few tokens and many heads)
@@ -39,11 +84,7 @@ __global__ __launch_bounds__(RC_THREADS) void qkv_rope_cache_kernel(
     // bfloat16, half-split pairs whose halves are multiples of eight: eight pairs per item, sixteen bytes per access
     const bool wide = sizeof(T) == 2 && rot.pairing == PTA_PAIR_HALF && half > 0 && (half & 7) == 0 && (d & 7) == 0;
     const int h8 = half >> 3;
-    auto source_head = [&](int kind, int head) {
-        if (layout == PTA_QKV_GROUPED) return kind == 0 ? (head / g) * (g + 2) + (head % g) : head * (g + 2) + g + (kind ? kind - 1 : 0);
-        if (layout == PTA_QKV_TAIL) return kind == 0 ? head : nh + kind - 1;
-        return head * 3 + kind;
-    };
+    auto source_head = [&](int kind, int head) { return fused_head(layout, nh, g, kind, head); };
     // A thread's first two items are asked for before anything else, so that the table of angles is made and the
     // page looked up while they are on their way: a token's row is read in one round trip to memory, not three.
     constexpr int AHEAD = 2;
@@ -166,16 +207,24 @@ extern "C" int pta_qkv_rope_cache(void* q_out, const void* fused, int fused_ld, 
     hipStream_t s = (hipStream_t)stream;
     int slices = 1;  // enough workgroups to occupy the chip when the step has few tokens
     while (slices < 16 && M * slices < 512 && slices * RC_THREADS < (nh + 2 * nkv) * d) slices *= 2;
+    const dim3 tiles((M + 63) / 64, (unsigned)std::min(65536L, (long)nkv * ((d + 63) / 64)));
+    const bool apart = write_cache && (long)M * nkv * d >= VALUES_APART && tiles.y <= 65535;
     if (dtype == PTA_F32)
         hipLaunchKernelGGL(qkv_rope_cache_kernel<float>, dim3(M, slices), dim3(RC_THREADS), 0, s, (float*)q_out,
                            (const float*)fused, fused_ld, bias, rot, token_pos, token_seq, block_table, bt_stride,
-                           (float*)k_pool, (float*)v_pool, nh, nkv, d, layout, write_cache);
+                           (float*)k_pool, (float*)v_pool, nh, nkv, d, layout, write_cache, !apart);
     else if (dtype == PTA_BF16)
         hipLaunchKernelGGL(qkv_rope_cache_kernel<bf16_t>, dim3(M, slices), dim3(RC_THREADS), 0, s, (bf16_t*)q_out,
                            (const bf16_t*)fused, fused_ld, bias, rot, token_pos, token_seq, block_table,
-                           bt_stride, (bf16_t*)k_pool, (bf16_t*)v_pool, nh, nkv, d, layout, write_cache);
+                           bt_stride, (bf16_t*)k_pool, (bf16_t*)v_pool, nh, nkv, d, layout, write_cache, !apart);
     else
         return pta_fail("qkv_rope_cache: unknown dtype %d", dtype);
+    if (apart && dtype == PTA_F32)
+        hipLaunchKernelGGL(value_pages_kernel<float>, tiles, dim3(RC_THREADS), 0, s, (const float*)fused, fused_ld, bias, token_pos,
+                           token_seq, block_table, bt_stride, (float*)v_pool, M, nh, nkv, d, layout);
+    else if (apart)
+        hipLaunchKernelGGL(value_pages_kernel<bf16_t>, tiles, dim3(RC_THREADS), 0, s, (const bf16_t*)fused, fused_ld, bias, token_pos,
+                           token_seq, block_table, bt_stride, (bf16_t*)v_pool, M, nh, nkv, d, layout);
     return pta_check_launch("qkv_rope_cache");
 }
 
