@@ -1,0 +1,68 @@
+"""Memory of captured decode steps: what dropped steps held is given back, and a capture that finds none left tries once more
+with torch's cache emptied."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _model():
+    from pytorch_transformers_amd import AutoModelForCausalLM, FalconConfig
+
+    cfg = FalconConfig(num_hidden_layers=2, hidden_size=64, num_attention_heads=4, num_kv_heads=2, new_decoder_architecture=True,
+                       vocab_size=512, ffn_hidden_size=256, alibi=False, bias=False)
+    return AutoModelForCausalLM.from_config(cfg, seed=0, std=0.2, dtype="float32", device="cuda:0")
+
+
+def test_generating_again_and_again_keeps_no_memory():
+    """Each call makes a cache of its own and captures steps in it: the memory torch holds goes up and down, and not up alone."""
+    from pytorch_transformers_amd.engine import model as engine
+
+    model, held = _model(), []
+    for _ in range(5 * engine.DROPPED_GRAPHS):
+        model.generate([[1, 2, 3]], max_new_tokens=4, do_sample=False, eos_token_id=None)
+        held.append(torch.cuda.memory_reserved())
+    half = len(held) // 2
+    assert max(held[half:]) <= max(held[:half])
+    assert held[-1] < held[0] + (engine.DROPPED_GRAPHS + 2) * (4 << 20)  # a step's pool here: 2 MiB
+
+
+def _steps(model, count=4):
+    cache = model.new_cache(256, max_slots=2)
+    slots = [cache.alloc(), cache.alloc()]
+    rows = [model.step(cache, slots, [[5, 6, 7], [8]], "last")]
+    rows += [model.step(cache, slots, [[9 + i], [20 + i]], "last") for i in range(count)]
+    return torch.stack(rows), cache
+
+
+@pytest.mark.parametrize("failures", [1, 2])
+def test_a_capture_without_memory(monkeypatch, failures):
+    """The first capture runs out half way: it is taken again and every step's logits are the plain steps'.  Where the second
+    attempt runs out too, the error is the caller's, the step is not committed, and the next one works."""
+    model = _model()
+    model.use_graphs = False
+    want, _ = _steps(model)
+    model.use_graphs = True
+    forward, left = model.forward_tokens, [failures]
+
+    def short_of_memory(*args):
+        out = forward(*args)
+        if torch.cuda.is_current_stream_capturing() and left[0]:
+            left[0] -= 1
+            raise torch.cuda.OutOfMemoryError("no memory")
+        return out
+
+    monkeypatch.setattr(model, "forward_tokens", short_of_memory)
+    if failures == 1:
+        got, cache = _steps(model)
+        assert torch.equal(got, want) and left == [0]
+        assert [g.graph is not None for g in cache._decode_graphs.values()] == [True]
+        return
+    cache = model.new_cache(256, max_slots=2)
+    slots = [cache.alloc(), cache.alloc()]
+    model.step(cache, slots, [[5, 6, 7], [8]], "last")
+    with pytest.raises(torch.cuda.OutOfMemoryError):
+        model.step(cache, slots, [[9], [20]], "last")
+    assert [cache.length(s) for s in slots] == [3, 1]
+    assert torch.equal(model.step(cache, slots, [[9], [20]], "last"), want[1])
+    assert torch.equal(model.step(cache, slots, [[10], [21]], "last"), want[2])
