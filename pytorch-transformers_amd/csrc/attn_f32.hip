@@ -144,36 +144,25 @@ __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, con
         for (int t = 0; t < 4; ++t) v[t] = *(const f32x4*)(vp + row * PTA_PAGE + 16 * t + kq);
 #pragma unroll
         for (int c = 0; c < CT; ++c) o[c][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+        bool odd = false;
         if (ragged) {
-            // A weight of 0 must hide its value whatever that is: keys behind the end are cleared; an infinite or undefined
-            // value of a key that only some columns see takes the page one key at a time.
-            float odd = 0.f;
+            // A weight of 0 must hide its value whatever that is.  Keys behind the end are cleared; an infinite or undefined
+            // value is cleared too and joins below those columns alone that see its key.
+            float zero = 0.f;
 #pragma unroll
             for (int t = 0; t < 4; ++t)
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if (j0 + 16 * t + kq + e >= end) v[t][e] = 0.f;
-                    odd += v[t][e] * 0.f;
+                    zero += v[t][e] * 0.f;
                 }
-            if (__ballot(!(odd == 0.f))) {
+            odd = __ballot(!(zero == 0.f)) != 0;
+            if (odd) {
 #pragma unroll
-                for (int c = 0; c < CT; ++c) {
-                    const int first = seen[c] ? col[c].first : 0, n = seen[c] ? col[c].nkeys : 0;
+                for (int t = 0; t < 4; ++t)
 #pragma unroll
-                    for (int t = 0; t < 4; ++t)
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            for (int g = 0; g < 4; ++g) {
-                                const int jj = 16 * t + 4 * g + e;
-                                const float p = __shfl(s[c][t][e], 16 * g + r16);
-                                if (j0 + jj >= first && j0 + jj < n) {
-#pragma unroll
-                                    for (int i = 0; i < 4; ++i)
-                                        o[c][b][i] += p * vp[min(16 * b + kq + i, a.d - 1) * PTA_PAGE + jj];
-                                }
-                            }
-                }
-                continue;
+                    for (int e = 0; e < 4; ++e)
+                        if (!(v[t][e] * 0.f == 0.f)) v[t][e] = 0.f;
             }
         }
 #pragma unroll
@@ -182,6 +171,27 @@ __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, con
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int c = 0; c < CT; ++c) o[c][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][e], s[c][t][e], o[c][b], 0, 0, 0);
+        if (odd) {
+#pragma unroll
+            for (int c = 0; c < CT; ++c) {
+                const int first = seen[c] ? col[c].first : 0, n = seen[c] ? col[c].nkeys : 0;
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e)
+                        for (int g = 0; g < 4; ++g) {
+                            const int jj = 16 * t + 4 * g + e;
+                            const float p = __shfl(s[c][t][e], 16 * g + r16);
+                            if (j0 + jj >= first && j0 + jj < n) {
+#pragma unroll
+                                for (int i = 0; i < 4; ++i) {
+                                    const float x = vp[min(16 * b + kq + i, a.d - 1) * PTA_PAGE + jj];
+                                    if (!(x * 0.f == 0.f)) o[c][b][i] += p * x;
+                                }
+                            }
+                        }
+            }
+        }
     }
 }
 

@@ -110,18 +110,21 @@ def test_attention(nh, nkv, d, how):
 
 
 @pytest.mark.parametrize("nh,nkv,d", [(4, 1, 64), (3, 3, 24)])
-def test_attention_hides_values_that_a_token_does_not_see(nh, nkv, d):
-    """An infinite value or an undefined key of a later token, or of another sequence, changes no earlier token's bits."""
+@pytest.mark.parametrize("window", [0, 5])
+@pytest.mark.parametrize("key", [True, False])
+def test_attention_hides_values_that_a_token_does_not_see(nh, nkv, d, window, key):
+    """An infinite value, and with ``key`` an undefined key, of one token changes no bit of a token that does not see it: earlier
+    ones, later ones behind the window, another sequence's; in one launch and token by token.  Whoever sees it shows it."""
     ops = _ops()
-    args, kw, _ = _attention_case(nh, nkv, d, [0, 0], [50, 30])
+    args, kw, _ = _attention_case(nh, nkv, d, [0, 0], [50, 30], window=window)
     got = ops.attn_generic(*args, **kw)
     q, kp, vp, table, *rest = args
     kp, vp = kp.clone(), vp.clone()
     vp[table[0, 0].item(), :, :, 40] = float("inf")
-    kp[table[0, 0].item(), :, 40] = float("nan")
-    bad = ops.attn_generic(q, kp, vp, table, *rest, **kw)
-    # (a page with such a value is summed in another order)
-    assert (bad[:40] - got[:40]).abs().max().item() <= 1e-5 and torch.equal(bad[50:], got[50:]) or \
-        (bad[50:] - got[50:]).abs().max().item() <= 1e-5
-    assert bool(torch.isfinite(bad[:40]).all()) and bool(torch.isfinite(bad[50:]).all())
-    assert bool(torch.isnan(bad[40:50]).all())
+    if key:
+        kp[table[0, 0].item(), :, 40] = float("nan")
+    sees = slice(40, 40 + window if window else 50)
+    for one_each in (False, True):
+        bad = ops.attn_generic(q, kp, vp, table, *rest, **kw, one_each=one_each)
+        assert torch.equal(bad[:40], got[:40]) and torch.equal(bad[sees.stop:], got[sees.stop:])
+        assert bool(torch.isnan(bad[sees]).all() if key else (bad[sees] == float("inf")).all())
