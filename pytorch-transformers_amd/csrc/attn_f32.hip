@@ -75,11 +75,12 @@ __device__ __forceinline__ float across_sum(float v) {
 }
 
 // One page for CT tiles: m, l and o of its keys alone.  ``seen[c]``: whether column c looks at this page's sequence at all.
-// ``end``: keys of the sequence that any column of the wave sees (what lies behind is whatever the page held before).
+// ``end``: keys of the sequence that any column of the wave sees (what lies behind is whatever the page held before).  ``spare``:
+// LDS of the wave's own for the weights of the page.
 template <int DT, int CT>
 __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, const float* vp, int j0, int end, const f32x4 (&q)[CT][DT],
                                           const Column (&col)[CT], const bool (&seen)[CT], float (&m)[CT], float (&l)[CT],
-                                          f32x4 (&o)[CT][DT]) {
+                                          f32x4 (&o)[CT][DT], float* spare) {
     const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
     f32x4 s[CT][4];
 #pragma unroll
@@ -171,26 +172,31 @@ __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, con
             for (int e = 0; e < 4; ++e)
 #pragma unroll
                 for (int c = 0; c < CT; ++c) o[c][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[t][e], s[c][t][e], o[c][b], 0, 0, 0);
-        if (odd) {
+        if (odd) {  // (rare: the columns' weights go through LDS, so that this is a loop and little code)
 #pragma unroll
-            for (int c = 0; c < CT; ++c) {
-                const int first = seen[c] ? col[c].first : 0, n = seen[c] ? col[c].nkeys : 0;
+            for (int c = 0; c < CT; ++c)
 #pragma unroll
                 for (int t = 0; t < 4; ++t)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e)
-                        for (int g = 0; g < 4; ++g) {
-                            const int jj = 16 * t + 4 * g + e;
-                            const float p = __shfl(s[c][t][e], 16 * g + r16);
-                            if (j0 + jj >= first && j0 + jj < n) {
+                    for (int e = 0; e < 4; ++e) spare[(c * PTA_PAGE + 16 * t + kq + e) * 16 + r16] = s[c][t][e];
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+#pragma unroll 1
+            for (int j = 0; j < PTA_PAGE; ++j) {
+                float x[4];
 #pragma unroll
-                                for (int i = 0; i < 4; ++i) {
-                                    const float x = vp[min(16 * b + kq + i, a.d - 1) * PTA_PAGE + jj];
-                                    if (!(x * 0.f == 0.f)) o[c][b][i] += p * x;
-                                }
-                            }
-                        }
+                for (int i = 0; i < 4; ++i) x[i] = vp[min(16 * b + kq + i, a.d - 1) * PTA_PAGE + j];
+#pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    if (!seen[c] || j0 + j < col[c].first || j0 + j >= col[c].nkeys) continue;
+                    const float p = spare[(c * PTA_PAGE + j) * 16 + r16];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (!(x[i] * 0.f == 0.f)) o[c][b][i] += p * x[i];
+                }
             }
+            __builtin_amdgcn_wave_barrier();
         }
     }
 }
@@ -229,6 +235,8 @@ __device__ __forceinline__ float last_factor(const AttnF32& a, const Column& c, 
 
 template <int DT, int CT>
 __global__ __launch_bounds__(256, DT <= 6 ? 2 : 1) void attn_f32_prompt_kernel(AttnF32 a) {
+    __shared__ float weights[4][CT * PTA_PAGE * 16];
+    float* spare = weights[threadIdx.x >> 6];
     const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
     const int per = a.nh / a.nkv, kvh = blockIdx.y;
     // columns are (token, head of the group) pairs in a row; the last tiles have the most keys and start first
@@ -272,7 +280,7 @@ __global__ __launch_bounds__(256, DT <= 6 ? 2 : 1) void attn_f32_prompt_kernel(A
             const long at = ((long)bt[p] * a.nkv + kvh) * PTA_PAGE * a.d;
             float m[CT], l[CT], keep, take;
             f32x4 o[CT][DT];
-            page_pass<DT, CT>(a, a.k_pool + at, a.v_pool + at, p * PTA_PAGE, end, q, col, seen, m, l, o);
+            page_pass<DT, CT>(a, a.k_pool + at, a.v_pool + at, p * PTA_PAGE, end, q, col, seen, m, l, o, spare);
 #pragma unroll
             for (int c = 0; c < CT; ++c)
                 if (join(M[c], L[c], m[c], l[c], keep, take)) {
@@ -296,7 +304,9 @@ template <int DT, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_f32_decode_kernel(AttnF32 a) {
     __shared__ f32x4 po[NW][DT][64];
     __shared__ float pm[NW][16], pl[NW][16];
+    __shared__ float weights[NW][PTA_PAGE * 16];
     const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4), wave = threadIdx.x >> 6;
+    float* spare = weights[wave];
     const int per = a.nh / a.nkv, kvh = blockIdx.y, token = blockIdx.z;
     const int hh = blockIdx.x * 16 + r16;
     Column col[1] = {column_of(a, token, kvh * per + hh, hh < per)};
@@ -316,7 +326,7 @@ __global__ __launch_bounds__(NW * 64) void attn_f32_decode_kernel(AttnF32 a) {
             const long at = ((long)bt[p + wave] * a.nkv + kvh) * PTA_PAGE * a.d;
             float m[1], l[1];
             f32x4 o[1][DT];
-            page_pass<DT, 1>(a, a.k_pool + at, a.v_pool + at, (p + wave) * PTA_PAGE, end, q, col, seen, m, l, o);
+            page_pass<DT, 1>(a, a.k_pool + at, a.v_pool + at, (p + wave) * PTA_PAGE, end, q, col, seen, m, l, o, spare);
 #pragma unroll
             for (int b = 0; b < DT; ++b) po[wave][b][lane] = o[0][b];
             if (lane < 16) pm[wave][lane] = m[0], pl[wave][lane] = l[0];
