@@ -14,7 +14,7 @@
 
 #include <stdint.h>
 
-#define PTA_ABI_VERSION 19
+#define PTA_ABI_VERSION 20
 
 #ifdef __cplusplus
 extern "C" {
@@ -135,10 +135,18 @@ int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, co
                  int M, int N, int K, int act, float* scratch, void* stream);
 
 // Attention of 32-bit heads of up to 256 elements, a multiple of 4, on the 32-bit matrix instruction: the arguments of
-// pta_attn_generic, and one_each: every token is its sequence's only one (a decode step)
+// pta_attn_generic, and the step's sequences in the tokens' order (cu_tokens null: every token is taken by itself, in any
+// order) with what pta_attn_f32_plan says of them, which looks at host copies of their new and cached tokens: up to how many
+// new tokens a sequence's tiles share their pages out over a workgroup, tiles of the largest of these; waves of the others
+// (per KV head), and tiles of a wave
+typedef struct {
+    int share_new, shared_tiles, prompt_waves, wave_tiles;
+} PtaAttnF32Plan;
+int pta_attn_f32_plan(const int* new_tokens, const int* starts, int n_seqs, int nh, int nkv, int d, PtaAttnF32Plan* plan);
 int pta_attn_f32(float* out, const float* q, const float* k_pool, const float* v_pool, const int* block_table, int bt_stride,
                  const int* token_seq, const int* token_pos, const PtaScoreBias* score_bias, int M, int nh, int nkv, int d,
-                 float scale, int window, int chunk, const float* sink, const PtaHeadRows* head_rows, int one_each, void* stream);
+                 float scale, int window, int chunk, const float* sink, const PtaHeadRows* head_rows, const int* cu_tokens,
+                 int n_seqs, const PtaAttnF32Plan* plan, void* stream);
 
 // y = act(x . W^T + bias) + add1 + add2 for M <= 64 rows of bfloat16; y is bfloat16, or 32-bit if out_f32.
 // variant and waves are tuning knobs (0: chosen from N and K): row tiles per wave, waves per workgroup

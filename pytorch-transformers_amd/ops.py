@@ -24,7 +24,7 @@ QKV_LAYOUT_CODES = {"grouped": 0, "tail": 1, "interleaved": 2}
 ACT_CODES = {None: 0, "none": 0, "linear": 0, "gelu": 1, "gelu_python": 1, "gelu_new": 2, "gelu_pytorch_tanh": 2,
              "gelu_fast": 2, "gelu_accurate": 2, "quick_gelu": 3, "relu": 4, "relu2": 5, "relu6": 6, "silu": 7, "swish": 7,
              "sigmoid": 8, "tanh": 9, "leaky_relu": 10, "mish": 11, "gelu_10": 12, "laplace": 13}
-ABI_VERSION = 19
+ABI_VERSION = 20
 PAIRING_CODES = {"half": 0, "interleaved": 1}  # PtaPairing: elements (i, i + rotary_dim / 2) or (2i, 2i + 1)
 BIAS_OF_CODES = {"key": 0, "distance": 1}  # PtaBiasOf: the slope times the key's position, or times key - query position
 
@@ -112,7 +112,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_gemm_splitk_pair_parts", "pta_gemm_stationary_rule")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_stationary_rule")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -585,16 +585,38 @@ def head_rows_ok(out: torch.Tensor, keep: int) -> bool:
     return out.dtype == torch.float32 or (keep % 4 == 0 and out.stride(0) % 4 == 0 and out.data_ptr() % 8 == 0)
 
 
+class _F32Plan(ctypes.Structure):  # PtaAttnF32Plan
+    _fields_ = [(name, ctypes.c_int) for name in ("share_new", "shared_tiles", "prompt_waves", "wave_tiles")]
+
+
+def _f32_runs(ctx, M: int, nh: int, nkv: int, d: int) -> tuple:
+    """``pta_attn_f32``'s arguments on the step's sequences, which are looked at once a step; none of them where the tokens
+    are not the step's."""
+    n, key = ctx.n_seqs, ("attn_f32", nh, nkv, d)
+    if M != (n if ctx.is_decode else sum(ctx.new_tokens)):
+        return (None, 0, None)
+    plan = ctx.extras.get(key)
+    if plan is None:
+        # (a captured step is sized for its bound)
+        starts = [ctx.max_len - 1] * n if ctx.is_decode else ctx.starts
+        plan = _F32Plan()
+        _call("pta_attn_f32_plan", (ctypes.c_int * n)(*ctx.new_tokens), (ctypes.c_int * n)(*starts), n, nh, nkv, d, ctypes.byref(plan))
+        ctx.extras[key] = plan
+    _need(ctx.cu_tokens, "cu_tokens", torch.int32, (n + 1,))
+    return (_ptr(ctx.cu_tokens), n, ctypes.byref(plan))
+
+
 def attn_generic(q: torch.Tensor, k_pool, v_pool, block_table, token_seq, token_pos, slopes, scale: float,
                  window: int = 0, alibi_exact: bool = False, bias_of: str = "key", bias_scale: Optional[float] = None,
-                 chunk: int = 0, sink: Optional[torch.Tensor] = None, into=None, one_each: bool = False):
+                 chunk: int = 0, sink: Optional[torch.Tensor] = None, into=None, one_each: bool = False, ctx=None):
     """Causal attention of every token over its sequence's cache (the last ``window`` positions of it, itself
     included, if ``window`` > 0; the positions of its own block of ``chunk``, counted from the sequence's start, if
     ``chunk`` > 0); out [M, nh*d].  ``slopes`` (None: no bias), ``bias_of``, ``alibi_exact`` (no
     rounding to bfloat16) and ``bias_scale`` (None: 1 / sqrt(head size), as the reference folds its bias into the
     mask) describe a bias on the scores (``_score_bias_arg``).  ``sink`` (``[nh]`` 32-bit): ``exp(sink[h])`` joins the
-    sum that head h's weights are divided by.  ``into = (out, keep, mult)``: see ``_head_rows``.  ``one_each``: every
-    token is its sequence's only one in the step (says how the work is shared out, not what comes of it).
+    sum that head h's weights are divided by.  ``into = (out, keep, mult)``: see ``_head_rows``.  ``ctx``: the
+    step that the tokens are, in its order (it says how the work is shared out, not what comes of it; without it, as with
+    ``one_each``, every token is taken by itself).
 
     32-bit heads of a multiple of four elements run on the 32-bit matrix instruction (``pta_attn_f32``); bfloat16 heads of
     sizes that the matrix-core kernel is not built for, and other 32-bit ones, a wave per token and head."""
@@ -612,9 +634,10 @@ def attn_generic(q: torch.Tensor, k_pool, v_pool, block_table, token_seq, token_
     if out is None:
         out = torch.empty((M, nh * d), dtype=q.dtype, device=q.device)
     if q.dtype == torch.float32 and d % 4 == 0 and q.data_ptr() % 16 == 0 and k_pool.data_ptr() % 16 == 0 and v_pool.data_ptr() % 16 == 0:
+        runs = (None, 0, None) if ctx is None or one_each else _f32_runs(ctx, M, nh, nkv, d)
         _call("pta_attn_f32", _ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table), block_table.shape[1],
               _ptr(token_seq), _ptr(token_pos), bias, M, nh, nkv, d, ctypes.c_float(scale), int(window), int(chunk), _ptr(sink),
-              rows, int(one_each and M <= 65535), _stream())
+              rows, *runs, _stream())
         return out
     _call("pta_attn_generic", _ptr(out), _ptr(q), _ptr(k_pool), _ptr(v_pool), _ptr(block_table),
           block_table.shape[1], _ptr(token_seq), _ptr(token_pos), bias, M, nh, nkv, d,
@@ -776,7 +799,7 @@ def attention(q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: 
                          decode_tiles=tiles, decode_waves=waves, alibi_exact=alibi_exact, bias_of=bias_of,
                          bias_scale=bias_scale, chunk=chunk, sink=sink, into=into)
     return attn_generic(q, k_pool, v_pool, block_table, ctx.token_seq, ctx.token_pos, slopes, scale, window, alibi_exact,
-                        bias_of, bias_scale, chunk, sink, into, one_each=ctx.is_decode)
+                        bias_of, bias_scale, chunk, sink, into, ctx=ctx)
 
 
 def attn_talk_mfma_ok(q: torch.Tensor, nkv: int, mixed: bool = True) -> bool:

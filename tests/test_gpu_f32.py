@@ -128,3 +128,79 @@ def test_attention_hides_values_that_a_token_does_not_see(nh, nkv, d, window, ke
         bad = ops.attn_generic(q, kp, vp, table, *rest, **kw, one_each=one_each)
         assert torch.equal(bad[:40], got[:40]) and torch.equal(bad[sees.stop:], got[sees.stop:])
         assert bool(torch.isnan(bad[sees]).all() if key else (bad[sees] == float("inf")).all())
+
+
+def _step(runs, nh, nkv, d, seed=0):
+    """(attn_generic's arguments, the step's context) for sequences of (cached, new) tokens with random keys and values."""
+    from types import SimpleNamespace
+
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    starts, news = [a for a, _ in runs], [b for _, b in runs]
+    pages = [(a + b + 63) // 64 for a, b in runs]
+    order = torch.randperm(sum(pages), generator=torch.Generator().manual_seed(seed)).int()
+    table, at = torch.zeros((len(runs), max(pages)), dtype=torch.int32), 0
+    for i, n in enumerate(pages):
+        table[i, :n] = order[at:at + n]
+        at += n
+    new = lambda *shape: torch.randn(*shape, generator=g, device="cuda")
+    ints = lambda v: torch.tensor(v, dtype=torch.int32).cuda()
+    cu = [0]
+    for n in news:
+        cu.append(cu[-1] + n)
+    ctx = SimpleNamespace(is_decode=all(n == 1 for n in news), n_seqs=len(runs), new_tokens=news, starts=starts, cu_tokens=ints(cu),
+                          max_len=max(a + b for a, b in runs), extras={})
+    args = (new(cu[-1], nh, d), new(sum(pages), nkv, 64, d), new(sum(pages), nkv, d, 64), table.cuda(),
+            ints([i for i, n in enumerate(news) for _ in range(n)]), ints([a + j for a, n in runs for j in range(n)]), None, d ** -0.5)
+    return args, ctx
+
+
+@pytest.mark.parametrize("nh,nkv,d", [(71, 1, 64), (16, 16, 64), (3, 1, 100), (4, 2, 256), (6, 2, 16)])
+@pytest.mark.parametrize("runs", [
+    [(600, 1)] * 70 + [(0, 1200)] + [(64, 1)] * 3,      # single tokens beside a prompt, more than 64 sequences
+    [(500, 3), (0, 1), (130, 40), (0, 129)],            # a few tokens behind many
+    [(0, 33)] * 130 + [(0, 700)],                       # short prompts, more than 128 of them
+    [(0, 1)] * 5 + [(63, 1), (64, 1), (900, 1)],        # one token each
+    [(40 * i, 1) for i in range(300)],                  # so many of them that a wave takes each
+])
+def test_attention_of_steps(nh, nkv, d, runs):
+    """A step's launches, however its sequences are shared out, against every token by itself: the same bits, with and without a
+    window."""
+    ops = _ops()
+    args, ctx = _step(runs, nh, nkv, d)
+    for kw in ({}, {"window": 70}):
+        assert torch.equal(ops.attn_generic(*args, **kw, ctx=ctx), ops.attn_generic(*args, **kw))
+
+
+def test_attention_of_steps_takes_both_kernels():
+    """A mixed step shares the single tokens' pages out and not the prompt's, and a large batch of prompts has
+    two tiles a wave."""
+    ops = _ops()
+    for runs, shared, prompts, tiles in (([(600, 1)] * 40 + [(0, 1200)], True, True, 2), ([(0, 256)] * 8, False, True, 2),
+                                         ([(0, 1)] * 300, False, True, 1), ([(900, 3), (70, 1)], True, False, 1)):
+        args, ctx = _step(runs, 71, 1, 64)
+        assert torch.equal(ops.attn_generic(*args, ctx=ctx), ops.attn_generic(*args))
+        plan = next(iter(ctx.extras.values()))
+        assert (plan.shared_tiles > 0, plan.prompt_waves > 0, plan.wave_tiles) == (shared, prompts, tiles)
+
+
+def test_a_prompt_beside_single_tokens_costs_what_the_two_cost():
+    """32 single tokens behind 1,000 keys and a prompt of 64 tokens in one step, 16 heads on as many KV heads: no more than a few
+    times the two steps apart (a wave that walks one sequence after the other for its sixteen heads took a hundred times as long)."""
+    ops = _ops()
+
+    def us(runs):
+        args, ctx = _step(runs, 16, 16, 64)
+        ctx.seq_start = torch.tensor(ctx.starts, dtype=torch.int32).cuda()
+        ctx.block_tables, ctx.token_seq, ctx.token_pos, best = None, args[4], args[5], float("inf")
+        for _ in range(5):
+            a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            a.record()
+            for _ in range(10):
+                ops.attention(*args[:4], ctx, None, args[7])
+            b.record()
+            b.synchronize()
+            best = min(best, a.elapsed_time(b) * 100)
+        return best
+
+    apart = us([(1000, 1)] * 32) + us([(0, 64)])
+    assert us([(1000, 1)] * 32 + [(0, 64)]) <= 4 * apart + 50
