@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import importlib.util
+import math
 import os
 import threading
 from typing import Optional
@@ -1750,11 +1751,32 @@ def latent_decode_split(n_seqs: int, heads: int, max_len: int):
 LATENT_DECODE = os.environ.get("PTA_LATENT_DECODE", "1") != "0"
 
 
-def latent_decode_ok(x: torch.Tensor, heads: int, dim: int, rot_dim: int, rank: int, value_dim: int) -> bool:
-    """Whether a decode step over latents runs in the three launches that are built for it (``latent_queries``,
-    ``latent_decode``): bfloat16, whole pieces of 32 elements, latents of up to 512.  PTA_LATENT_DECODE=0 switches it off."""
-    return (LATENT_DECODE and x.dtype == torch.bfloat16 and 0 < x.shape[0] <= 65535
+def latent_decode_sizes_ok(dtype: torch.dtype, heads: int, dim: int, rot_dim: int, rank: int, value_dim: int) -> bool:
+    """Whether the three launches for decode steps over latents (``latent_queries``, ``latent_decode``) are built for a layer:
+    bfloat16, whole pieces of 32 elements, latents of up to 512.  PTA_LATENT_DECODE=0 switches them off."""
+    return (LATENT_DECODE and dtype == torch.bfloat16
             and bool(load_library().pta_latent_decode_ok(int(heads), int(dim), int(rot_dim), int(rank), int(value_dim))))
+
+
+def _latent_page_visits(n_seqs: int, heads: int, max_len: int) -> tuple:
+    """(pages of a sequence, workgroups of ``latent_decode`` that each of them is staged by, over all sequences), as a captured
+    step has them: the batch by its next power of two, the context by its bound."""
+    return (tuning.context_bound(int(max_len)) + 63) // 64, (1 << max(int(n_seqs) - 1, 0).bit_length()) * ((heads + 15) // 16)
+
+
+def latent_decode_ok(x: torch.Tensor, heads: int, dim: int, rot_dim: int, rank: int, value_dim: int, max_len: int = 1) -> bool:
+    """Whether a decode step of ``x.shape[0]`` sequences over contexts up to ``max_len`` runs in the three launches
+    (``latent_decode_sizes_ok``).  They save launches, but stage a page for sixteen heads where the general kernel stages it for
+    64, and read its values element by element: with many heads over many keys that costs more, the sooner the smaller rows are.
+    Three launches / general, us, at so many visits of a page by a workgroup.  Rows of 512 + 64: 16 heads, 64 sequences of 1,000 keys
+    (1,024) 62 / 133, of 16,000 (16,384) 633 / 676, 128 of 16,000 (32,768) 1,245 / 1,238; 32 heads, 128 of 1,000 (4,096) 184 / 201, 64
+    of 4,000 (8,192) 336 / 278; 128 heads, 8 of 4,000 (4,096) 193 / 208, 64 of 1,000 (8,192) 365 / 272.  Rows of 256 + 32: 16 heads, 128
+    of 1,000 (2,048) 58 / 80, 64 of 4,000 (4,096) 96 / 97; 40 heads, 64 of 1,000 (3,072) 101 / 89; 128 heads, 128 of 180 (3,072) 81 / 137.
+    Of 128 + 64: 16 heads, 32 of 4,000 (2,048) 46 / 57, 64 of 4,000 (4,096) 75 / 71."""
+    pages, workgroups = _latent_page_visits(x.shape[0], heads, max_len)
+    most = 16384 if rank > 256 and heads <= 16 else 4096 if rank > 256 or pages <= 3 else 2048
+    return (0 < x.shape[0] <= 65535 and pages * workgroups <= most
+            and latent_decode_sizes_ok(x.dtype, heads, dim, rot_dim, rank, value_dim))
 
 
 def latent_queries(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor], eps: float, inv_freq, cs_scale: float, rotary_dim, pairing: str,
@@ -1774,11 +1796,10 @@ def latent_queries(proj: Optional[torch.Tensor], w_norm: Optional[torch.Tensor],
 
 
 def latent_ranges(n_seqs: int, heads: int, max_len: int) -> tuple:
-    """(keys per range, ranges) of ``latent_decode``: whole pages, as many ranges as give every compute unit a workgroup.  The
-    batch counts by its next power of two and the context by its bound, as a captured step has them."""
-    pages = (tuning.context_bound(int(max_len)) + 63) // 64
-    workgroups = (1 << max(int(n_seqs) - 1, 0).bit_length()) * ((heads + 15) // 16)
-    size = -(-pages // max(1, min(pages, 256 // workgroups, 1024)))
+    """(keys per range, ranges) of ``latent_decode``: whole pages, as many ranges as give every compute unit a workgroup, but
+    no more than six times the root of the pages: a page more in a range costs some 10 us, a range more to merge 0.3."""
+    pages, workgroups = _latent_page_visits(n_seqs, heads, max_len)
+    size = -(-pages // max(1, min(pages, 256 // workgroups, math.isqrt(36 * pages))))
     return 64 * size, -(-pages // size)
 
 

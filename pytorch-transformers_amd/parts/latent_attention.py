@@ -79,8 +79,9 @@ class LatentAttentionMixer(Part):
         # per head, with a head's rows its inputs: the key expansion as the file has it, the value expansion turned
         self.k_side = self.up_k.view(self.heads, self.dim, self.rank)
         self.v_side = self.up_v.view(self.heads, self.value_dim, self.rank).transpose(1, 2).contiguous()
-        # decode steps want the rows of both to be outputs
-        self.k_turned = self.k_side.transpose(1, 2).contiguous() if self.up_k.dtype == torch.bfloat16 else None
+        # decode steps in three launches want the rows of both to be outputs
+        built = ops.latent_decode_sizes_ok(self.up_k.dtype, self.heads, self.dim, self.rot_dim, self.rank, self.value_dim)
+        self.k_turned = self.k_side.transpose(1, 2).contiguous() if built else None
 
     def check_sizes(self) -> None:
         problem = ops.latent_sizes_problem(self.heads, self.dim, self.rot_dim, self.rank)
@@ -119,8 +120,9 @@ class LatentAttentionMixer(Part):
         return self.out(o, add1=residual)
 
     def _decode(self, queries: torch.Tensor, rows, write: bool, ctx: StepContext) -> Optional[torch.Tensor]:
-        """The heads' results of a step of one token per sequence in three launches, where they are built for these sizes."""
-        if not ops.latent_decode_ok(queries, self.heads, self.dim, self.rot_dim, self.rank, self.value_dim):
+        """The heads' results of a step of one token per sequence in three launches, where they are built and the faster way."""
+        if self.k_turned is None or not ops.latent_decode_ok(queries, self.heads, self.dim, self.rot_dim, self.rank, self.value_dim,
+                                                             ctx.max_len):
             return None
         q_full = ops.latent_queries(*rows, self.k_turned, self.heads, self.dim, self.rot_dim, self.rank, write_cache=write, q=queries)
         if q_full is None:
