@@ -10,7 +10,7 @@
 // and how many workgroups share the segments changes nothing.
 //
 // Measured at 4,544 / 18,176 features (one kernel of 64 x 64 tiles on the vector units before): one row of A 986 -> 56 us a
-// product on average (28 us for 83 MB, 71 us = 4.7 TB/s for 330 MB); 2,053 rows 26 -> 103 to 131 TFLOP/s.
+// product on average (22 us = 3.7 TB/s for 83 MB, 70 to 75 us = 4.4 to 4.7 TB/s for 330 MB); 2,053 rows 26 -> 103 to 131 TFLOP/s.
 //
 // Three ways to the same numbers, by what bounds them:
 //   few rows (M <= 32, with a short K 64): every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight
@@ -66,7 +66,9 @@ __host__ __device__ static inline int seg_blocks(int K) { return ((K + 15) / 16 
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------
 // CT: tiles of sixteen rows of A, RT: tiles of sixteen rows of W.  D blocks of K are asked for while the D before them are
-// multiplied: at K = 4,544 and one row of A a compute unit then has some 60 KB on its way.
+// multiplied: at K = 4,544 and one row of A a compute unit then has some 60 KB on its way.  What is asked for past a segment's
+// end is its last block again, which a cache has (the next segment's first blocks, long gone from the caches, were a fifth of all
+// that came from memory at 4,544 x 4,544; the launch takes 22 us either way).
 template <int CT, int RT, int D, int ROWS>
 __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel(
     float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W, F32Epilogue epi, int M, int N, int K) {
@@ -93,7 +95,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
     auto fetch = [&](int buf, int b) {
 #pragma unroll
         for (int i = 0; i < D; ++i) {
-            const int k = 16 * min(b + i, nb - 1) + kq;  // past the segment: read again, not used
+            const int k = 16 * min(b + i, b1 - 1) + kq;  // past the segment: its last block again, not used
 #pragma unroll
             for (int r = 0; r < RT; ++r) w[buf][i][r] = load4<ROWS>(wr[r], k, K);
 #pragma unroll
