@@ -1,5 +1,6 @@
 """The decode launches over a cache of latents against 64 bits, at the edges of their tiles: heads beyond sixteen, latents from
-one piece of 32 elements to 512, no rotated part, outputs that fill no tile, contexts around a page and a range."""
+one piece of 32 elements to 512, no rotated part, outputs that fill no tile, contexts around a page and a range, ranges of one
+page and of several."""
 from types import SimpleNamespace
 
 import pytest
@@ -9,13 +10,14 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("H,dn,dr,R,V", [(16, 128, 64, 512, 128), (1, 32, 0, 32, 16), (17, 64, 32, 96, 40), (40, 256, 64, 192, 100), (3, 96, 128, 512, 33)])
-@pytest.mark.parametrize("lens", [[1], [64, 65, 1], [700, 3, 130], [100] * 17])
+@pytest.mark.parametrize("lens", [[1], [64, 65, 1], [700, 3, 130], [100] * 17, [max(1, 700 - 23 * i) for i in range(33)]])
 def test_against_64_bits(H, dn, dr, R, V, lens):
     from pytorch_transformers_amd import ops
 
     g = torch.Generator().manual_seed(H + dn + len(lens))
     r = lambda *s: torch.randn(*s, generator=g)
     M, D, width = len(lens), R + dr, (max(lens) + 63) // 64
+    assert M < 33 or ops.latent_ranges(M, H, max(lens))[0] > 64  # ranges of several pages, which end inside one
     assert ops.latent_decode_ok(torch.empty(M, 1, dtype=torch.bfloat16), H, dn, dr, R, V)
     table = torch.randperm(M * width, generator=g).view(M, width).int()
     pool = torch.full((M * width + 1, 1, 64, D), float("nan"))
