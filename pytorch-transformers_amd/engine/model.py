@@ -103,6 +103,7 @@ def _capture_stream(index: int) -> "torch.cuda.Stream":
 # 2.0 to 2.2 ms with it before every capture, 1.87 to 1.88 before every eighth, 1.84 to 1.88 without (and 2 MiB more a call).
 _dropped_graphs: Dict[int, int] = {}
 DROPPED_GRAPHS = 8
+DIRECT_STEPS = 64  # steps of a shape that are launched directly after a capture that found no memory, before the next attempt
 
 
 def _give_back_memory(index: int) -> None:
@@ -155,6 +156,7 @@ class _DecodeGraph:
         self.copied = torch.cuda.Event()
         self.graph = None
         self.logits = None
+        self.direct = 0  # steps still to be launched directly before a capture is tried
 
     @property
     def cache(self) -> PagedCache:
@@ -234,6 +236,9 @@ class _DecodeGraph:
         # the first step of this shape: launched directly, which also lets libraries set themselves up outside a
         # capture; its result is the step's result.  The capture that follows records launches and runs nothing.
         logits = self.model.forward_tokens(*self._context())
+        if self.direct > 0:
+            self.direct -= 1
+            return logits
         if _dropped_graphs.get(self.index, 0) >= DROPPED_GRAPHS:
             _give_back_memory(self.index)
         collecting = gc.isenabled()
@@ -242,14 +247,16 @@ class _DecodeGraph:
             if not self._capture():
                 # during a capture torch's allocator gives none of its cached blocks back: all are given back here, and once more
                 _give_back_memory(self.index)
-                self._capture(again=True)
+                if not self._capture():
+                    # the step itself is done, and states that layers keep have moved on with it: its result stands
+                    self.direct = DIRECT_STEPS
         finally:
             if collecting:
                 gc.enable()
         return logits
 
-    def _capture(self, again: bool = False) -> bool:
-        """Record the step.  Memory that runs out is False (nothing is kept of the attempt), or, ``again``, an error."""
+    def _capture(self) -> bool:
+        """Record the step; False (and nothing is kept of the attempt) where memory runs out."""
         # on a stream of its own, without the wait for the GPU and the emptying of torch's memory cache that
         # ``torch.cuda.graph`` begins with: the step just launched goes on meanwhile, and the memory that a program's
         # next tensors would take stays where it is
@@ -264,8 +271,6 @@ class _DecodeGraph:
                 finally:
                     graph.capture_end()
         except torch.cuda.OutOfMemoryError:
-            if again:
-                raise
             return False
         self.graph, self.logits = graph, logits
         return True

@@ -35,34 +35,42 @@ def _steps(model, count=4):
     return torch.stack(rows), cache
 
 
+def _stateful():
+    from pytorch_transformers_amd import AutoModelForCausalLM, PavodraConfig
+
+    mlp = {"kind": "dense", "ff": 128}
+    attention = {"heads": 2, "dim": 32, "rot_dim": 16, "vdim": 32, "kv_rank": 64, "scale": 0.15, "rot": {"base": 10000.0, "dims": 16}}
+    cfg = PavodraConfig(vocab=512, width=64, layers=[{"type": "latent_attention", "mixer": attention, "mlp": mlp},
+                                                     {"type": "mingru", "mixer": {"width": 64}, "mlp": mlp}])
+    return AutoModelForCausalLM.from_config(cfg, seed=0, std=0.2, dtype="bfloat16", device="cuda:0")
+
+
+@pytest.mark.parametrize("make", [_model, _stateful])
 @pytest.mark.parametrize("failures", [1, 2])
-def test_a_capture_without_memory(monkeypatch, failures):
-    """The first capture runs out half way: it is taken again and every step's logits are the plain steps'.  Where the second
-    attempt runs out too, the error is the caller's, the step is not committed, and the next one works."""
-    model = _model()
+def test_a_capture_without_memory(monkeypatch, make, failures):
+    """The first capture runs out half way: it is taken again.  Where the second attempt runs out too, the step's result stands, as
+    the states that layers keep have moved on, and some steps follow without a capture.  Every step's logits are the plain
+    steps'."""
+    from pytorch_transformers_amd.engine import model as engine
+
+    model = make()
     model.use_graphs = False
-    want, _ = _steps(model)
+    want, _ = _steps(model, 6)
     model.use_graphs = True
-    forward, left = model.forward_tokens, [failures]
+    monkeypatch.setattr(engine, "DIRECT_STEPS", 2)
+    forward, left, captures = model.forward_tokens, [failures], []
 
     def short_of_memory(*args):
         out = forward(*args)
-        if torch.cuda.is_current_stream_capturing() and left[0]:
-            left[0] -= 1
-            raise torch.cuda.OutOfMemoryError("no memory")
+        if torch.cuda.is_current_stream_capturing():
+            captures.append(1)
+            if left[0]:
+                left[0] -= 1
+                raise torch.cuda.OutOfMemoryError("no memory")
         return out
 
     monkeypatch.setattr(model, "forward_tokens", short_of_memory)
-    if failures == 1:
-        got, cache = _steps(model)
-        assert torch.equal(got, want) and left == [0]
-        assert [g.graph is not None for g in cache._decode_graphs.values()] == [True]
-        return
-    cache = model.new_cache(256, max_slots=2)
-    slots = [cache.alloc(), cache.alloc()]
-    model.step(cache, slots, [[5, 6, 7], [8]], "last")
-    with pytest.raises(torch.cuda.OutOfMemoryError):
-        model.step(cache, slots, [[9], [20]], "last")
-    assert [cache.length(s) for s in slots] == [3, 1]
-    assert torch.equal(model.step(cache, slots, [[9], [20]], "last"), want[1])
-    assert torch.equal(model.step(cache, slots, [[10], [21]], "last"), want[2])
+    got, cache = _steps(model, 6)
+    assert torch.equal(got, want) and len(captures) == failures + 1
+    assert [(g.graph is not None, g.direct) for g in cache._decode_graphs.values()] == [(True, 0)]
+    assert sorted(cache.length(s) for s in range(2)) == [7, 9]
