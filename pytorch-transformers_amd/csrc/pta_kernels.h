@@ -211,6 +211,14 @@ int pta_gemm_splitk_reduced_qkv_bf16(void* q_out, float* part, const void* x, co
 int pta_rope_dynamic_table(float* out, const int* seq_start, const int* cu_tokens, int n_seqs, int d, float theta,
                            float factor, int max_pos, void* stream);
 
+// y[M, N] = act(x[M, K] . W[N, K]^T + bias) + add1 + add2 for many rows (gemm_tile_bf16.hip): bfloat16, 32-bit sums, rows of
+// x and y ldx and ldy apart, N, K, ldx and ldy multiples of 8; act: none, exact GELU or squared ReLU.  pta_gemm_tile_plan says how a
+// product is shared out (tiles of 256 by 32 fq; the first `whole` of them over all of K, the others in `split` ranges of
+// K) and how many 32-bit values of `part` the cut ones need; any plan within the bounds that are checked is taken.
+int pta_gemm_tile_plan(int M, int N, int K, int* fq, int* whole, int* split, long* part_values);
+int pta_gemm_tile_bf16(void* y, int ldy, const void* x, int ldx, const void* W, const float* bias, const void* add1,
+                       const void* add2, int M, int N, int K, int act, int fq, int whole, int split, float* part,
+                       long part_values, void* stream);
 // y[M, N] = act(sum of part[P, M, N] over P, in order, + bias) + add1 + add2: the reduction of the products above
 // on its own, for 32-bit partial sums over ranges of K that the vendor library's batched product made
 int pta_gemm_reduce_parts(void* y, const float* part, const float* bias, const void* add1, const void* add2, int M,

@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_stationary_rule")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_stationary_rule", "pta_gemm_tile_plan")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -178,6 +178,8 @@ def _entry_cost(name: str, a) -> tuple:
         return both(gemm(a[26], (a[13] + 2 * a[14]) * a[15], a[5]), gemm(a[26], a[23], a[24]))
     if name == "pta_gemm_splitk_reduced_qkv_bf16":
         return gemm(a[18], (a[13] + 2 * a[14]) * a[15], a[5])
+    if name == "pta_gemm_tile_bf16":
+        return gemm(a[8], a[9], a[10])
     if name == "pta_gemm_f32":
         return gemm(a[6], a[7], a[8], 4)
     if name == "pta_layernorm_sum":
@@ -966,6 +968,91 @@ def library_mm(x: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
 
 
 
+# ---- products of many rows, hand-written ----------------------------------------------------------------------------------
+GEMM_TILE = os.environ.get("PTA_GEMM_TILE", "1") != "0"
+GEMM_TILE_ROWS = 16
+GEMM_TILE_MOST = 0x7ffffff0 // 2  # elements of a matrix whose bytes 32 bits can say
+GEMM_TILE_ACTS = (0, 1, 5)  # the activations (ACT_CODES) that its epilogue applies
+
+
+def _library_fills(M: int, N: int) -> bool:
+    """Whether tiles of 256 by 256 fill the chip to 97 % in whole rounds: there the vendor library's kernel, which has fewer
+    and larger waves, is 5 to 12 % faster (4,096 x 4,096 x 4,096 89 us against 97, 2,048 x 8,192 x 8,192 173 against 191, 25,148 x
+    16,384 x 4,096 2,282 against 2,397).  Elsewhere, over 260 products of 150 to 25,148 rows, the hand-written kernel takes 0.3 to
+    1.1 times as long (672 x 4,544 x 18,176 101 us against 205, 2,317 x 18,176 x 4,544 299 against 416), 0.9 in the middle."""
+    units = compute_units()
+    tiles = -(-M // 256) * -(-N // 256)
+    return M * N >= 0.97 * 65536 * units * -(-tiles // units)
+
+
+def gemm_tile_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the hand-written kernel for many rows takes this product and is the choice for it, where the kernels for few
+    rows (up to 16, and to 128 and more unless W has at least twice as many rows as columns) are not.  Up to 256 rows such
+    a tall W whose rows lie a multiple of 8 KiB apart is the library's: 32,768 x 8,192 by 64 to 192 rows 115 to 133 us against
+    135 to 151, 16,384 x 4,096 equal or up to 15 % faster; 18,176 x 4,544 46 to 58 us against 38 to 53, 8,192 x 2,048 20 against 16."""
+    M, K = x.shape
+    N = w.shape[0]
+    if M <= 256 and K % 4096 == 0 and N >= 2 * K:
+        return False
+    return (GEMM_TILE and M > GEMM_TILE_ROWS and _bf16_rows_ok(x, w) and N % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and (N + 256) * K < GEMM_TILE_MOST and (M + 256) * x.stride(0) < GEMM_TILE_MOST
+            and not _library_fills(M, N))
+
+
+@functools.lru_cache(maxsize=None)
+def compute_units() -> int:
+    return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_tile_plan(M: int, N: int, K: int) -> tuple:
+    """(32-row groups of a tile, tiles over all of K, ranges of K of the others, 32-bit values that their sums need)."""
+    fq, whole, split, values = ctypes.c_int(), ctypes.c_int(), ctypes.c_int(), ctypes.c_long()
+    _call("pta_gemm_tile_plan", M, N, K, ctypes.byref(fq), ctypes.byref(whole), ctypes.byref(split), ctypes.byref(values))
+    return fq.value, whole.value, split.value, values.value
+
+
+def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None, plan=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 for many rows of bfloat16; rows of ``x`` may lie apart.  ``plan``: another sharing out
+    than ``gemm_tile_plan``'s (without the last number)."""
+    M, K = x.shape
+    N = w.shape[0]
+    _need_rows(x, "x", torch.bfloat16, (M, K))
+    _need(w, "w", torch.bfloat16, (N, K))
+    if bias is not None:
+        _need(bias, "bias", torch.float32, (N,))
+    for name, a in (("add1", add1), ("add2", add2)):
+        if a is not None:
+            _need(a, name, torch.bfloat16, (M, N))
+    if plan is None:
+        fq, whole, split, values = gemm_tile_plan(M, N, K)
+    else:
+        fq, whole, split = plan
+        values = (-(-M // (32 * fq)) * -(-N // 256) - whole) * split * fq * 8192
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    part = torch.empty(values, dtype=torch.float32, device=x.device) if values > 0 else None
+    _call("pta_gemm_tile_bf16", _ptr(y), N, _ptr(x), int(x.stride(0)), _ptr(w), _ptr(bias), _ptr(add1), _ptr(add2), M, N, K,
+          ACT_CODES[act], fq, whole, split, _ptr(part), ctypes.c_long(values), _stream())
+    return y
+
+
+def mm_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 of many rows: the library's product over ranges of K where that was timed faster, else
+    the hand-written kernel or, where ``gemm_tile_ok`` leaves it to it, the library's plain product."""
+    y = library_mm_ksplit(x, w, bias, act, add1, add2)
+    if y is not None:
+        return y
+    if gemm_tile_ok(x, w):
+        if ACT_CODES[act] in GEMM_TILE_ACTS:
+            return gemm_tile_bf16(x, w, bias, act, add1, add2)
+        y = gemm_tile_bf16(x, w)
+    else:
+        y = library_mm(x, w)
+    if bias is not None or act is not None or add1 is not None or add2 is not None:
+        epilogue_(y, bias, act, add1, add2)
+    return y
+
+
 # ---- the vendor library's product with K cut into a batch ------------------------------------------------
 # Where K is long against N (the feed-forward's second matrix) and the rows are a few hundred, the library's
 # kernel choice has too few tiles of the result to fill the chip: with K = 18,176 and N = 4,544, 512 rows take 225
@@ -985,7 +1072,7 @@ def _k_batch(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
 
 def library_mm_ksplit(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None):
     """``act(x @ w.T + bias) + add1 + add2`` through the library's batched product over ranges of K, where that
-    was timed faster than its plain product (once per shape, by 64 rows); else None."""
+    was timed faster than the product in one (once per shape, by 64 rows); else None."""
     M, (N, K) = x.shape[0], w.shape
     if (not MM_KSPLIT or K < 2 * N or not (tuning.SPLITK_MAX_ROWS < M <= MM_KSPLIT_MAX_ROWS) or K % 32 or x.stride(1) != 1
             or not w.is_contiguous()):
@@ -995,7 +1082,8 @@ def library_mm_ksplit(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add
     if S is None:
         if not tuning.may_time():
             return None
-        ways = [(1, lambda: library_mm(x, w))] + [(s, (lambda s=s: _k_batch(x, w, s))) for s in (2, 4) if K % (s * 8) == 0]
+        plain = gemm_tile_bf16 if gemm_tile_ok(x, w) else library_mm
+        ways = [(1, lambda: plain(x, w))] + [(s, (lambda s=s: _k_batch(x, w, s))) for s in (2, 4) if K % (s * 8) == 0]
         best = tuning.time_ways_cold([run for _, run in ways], x.device)
         pick = min(range(len(ways)), key=lambda i: best[i])
         S = ways[pick][0] if best[pick] < 0.9 * best[0] else 1

@@ -7,9 +7,10 @@ layer, with activation and residual additions, is one hand-written kernel with a
 fixed summation order.  In bfloat16, steps of at most 128 tokens (decoding, short
 prompts), and up to 256 where that was timed faster, run a hand-written kernel
 that streams the weights once and applies bias, activation and additions in its
-epilogue; larger steps use the vendor library's matrix
-product (as the reference uses torch's), followed by one fused kernel for bias,
-activation and additions.
+epilogue; larger steps use a hand-written kernel of large tiles with the same
+epilogue or, where its tiles fill the chip evenly, the vendor library's matrix product
+(as the reference uses torch's), followed by one fused kernel for bias, activation
+and additions (``ops.mm_rows``).
 """
 from __future__ import annotations
 
@@ -113,13 +114,7 @@ class Linear(Part):
             return ops.gemm_skinny_bf16(x, self.weight, bias, act, add1, add2)
         if ops.gemm_splitk_ok(x, self.weight):
             return ops.gemm_splitk_bf16(x, self.weight, bias, act, add1, add2)
-        y = ops.library_mm_ksplit(x, self.weight, bias, act, add1, add2)
-        if y is not None:
-            return y
-        y = ops.library_mm(x, self.weight)
-        if bias is not None or act is not None or add1 is not None or add2 is not None:
-            ops.epilogue_(y, bias, act, add1, add2)
-        return y
+        return ops.mm_rows(x, self.weight, bias, act, add1, add2)
 
     def with_tail(self, x: torch.Tensor, tail: "QkvTail") -> Optional["TailDone"]:
         """This product as a fused query_key_value projection whose launch also runs ``tail`` (a small matrix in a step of
@@ -163,7 +158,7 @@ class Linear(Part):
                 and ops.joined_mm_pays(x1, first.joined[0], first.out_features)):
             # many rows, one input, the matrices side by side in memory: one library product where it was measured
             # faster than two; the results are blocks of columns of its output, each with its own epilogue
-            y = ops.library_mm(x1, first.joined[0])
+            y = ops.mm_rows(x1, first.joined[0])
             y1, y2 = y[:, :first.out_features], y[:, first.out_features:]
             for yi, bias, act in ((y1, b1, kw1.get("act")), (y2, b2, kw2.get("act"))):
                 if bias is not None or act is not None:

@@ -434,8 +434,7 @@ def time_ways_cold(ways, device, rounds: int = 3):
 def splitk_row_limit(*ws: torch.Tensor) -> int:
     """Rows up to which the decode batch kernel is the faster way to the product with ``w`` (or, for two weights, to
     the two products of a pair launch).  Up to 128 rows it always was (one chunk of rows per workgroup); with two
-    chunks it depends on how well the library does at the shape (at 256 rows it wins with K = 4,544, 9.5 against
-    11.4 ms a step of 32 layers, and loses with K = 4,096, 22.1 against 20.2 ms of 60 layers), so both are timed once
+    chunks it depends on how well the product of many rows (``ops.mm_rows``) does at the shape, so both are timed once
     per shape at 192 and 256 rows, when timing is on; without an entry the kernel stops at 128 rows."""
     if SPLITK_MAX_ROWS <= SPLITK_SURE_ROWS:
         return SPLITK_MAX_ROWS
@@ -446,7 +445,6 @@ def splitk_row_limit(*ws: torch.Tensor) -> int:
             return SPLITK_SURE_ROWS
         dev = ws[0].device
         xs = [torch.randn((256, w.shape[1]), dtype=torch.float32, device=dev).to(torch.bfloat16) for w in ws]
-        outs = [torch.empty((256, w.shape[0]), dtype=torch.bfloat16, device=dev) for w in ws]
         limit = SPLITK_SURE_ROWS
         for rows in (192, 256):
             if rows > SPLITK_MAX_ROWS:
@@ -459,11 +457,11 @@ def splitk_row_limit(*ws: torch.Tensor) -> int:
                 else:
                     ops.gemm_splitk_pair_bf16(xr[0], ws[0], xr[1], ws[1])
 
-            def library():
-                for x, w, out in zip(xr, ws, outs):
-                    torch.mm(x, w.t(), out=out[:rows])
+            def product():
+                for x, w in zip(xr, ws):
+                    ops.mm_rows(x, w)
 
-            best = time_ways_cold((kernel, library), dev)
+            best = time_ways_cold((kernel, product), dev)
             if best[0] < SPLITK_MARGIN * best[1]:
                 limit = rows
             else:
@@ -538,10 +536,9 @@ def mm_plan(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor):
 
 
 def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int) -> bool:
-    """Whether ``x @ joined.T`` in one library product beats the products with its first ``n_first`` rows and
-    with the rest on their own.  The library's kernel choice decides, so both ways are timed once per shape when
-    timing is on (2,048 rows, K = 4,544, N = 4,672 + 18,176: 308 us against 87 + 286; K = 4,096, N = 6,144 + 16,384:
-    311 against 80 + 179); without an entry the two stay apart."""
+    """Whether ``x @ joined.T`` in one product beats the products with its first ``n_first`` rows and
+    with the rest on their own.  How evenly the tiles of each fill the chip decides (and where it is the library's product,
+    its kernel choice), so both ways are timed once per shape when timing is on; without an entry the two stay apart."""
     M, (N, K) = x.shape[0], joined.shape
     if not MM_JOIN or not MM_CHUNKS or M < 512:
         return False
@@ -551,7 +548,7 @@ def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int) -> bool:
         if not may_time():
             return False
         first, rest = joined[:n_first], joined[n_first:]
-        ways = (lambda: ops.library_mm(x, joined), lambda: (ops.library_mm(x, first), ops.library_mm(x, rest)))
+        ways = (lambda: ops.mm_rows(x, joined), lambda: (ops.mm_rows(x, first), ops.mm_rows(x, rest)))
         best = [float("inf"), float("inf")]
         for run in ways:  # plans are made and the library set up before anything is timed
             run()
