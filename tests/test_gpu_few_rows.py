@@ -57,3 +57,18 @@ def test_fused_rows_to_their_end(layout, nh, nkv, d, M, rotation):
     k2, v2 = new()
     ops.gemm_skinny_qkv(x, w, bias, inv, 0.9, pos, seq, table, k2, v2, nh, nkv, d, layout, False, **how)
     assert bool((k2 == 7.0).all()) and bool((v2 == 7.0).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(1, 40, 72), (8, 8192, 2048), (16, 1048, 520)])
+def test_squared_relu_in_the_epilogue(M, N, K):
+    """Bias, squared ReLU and an addition in the launch itself: the bits of the product with its bias, taken to its end by hand."""
+    from pytorch_transformers_amd import ops
+
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), torch.randn(N, K, generator=g).bfloat16().cuda()
+    bias, add = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).bfloat16().cuda()
+    z = ops.gemm_skinny_bf16(x, w, bias).float().clamp_min(0)
+    assert torch.equal(ops.gemm_skinny_bf16(x, w, bias, "relu2"), (z * z).bfloat16())
+    want = (z.double() * z.double() + add.double()).float()  # one rounding at the end, whether or not the two are one instruction
+    got = ops.gemm_skinny_bf16(x, w, bias, "relu2", add)
+    assert bool(((got.float() - want).abs() <= want.abs() * 2.0 ** -8 + z * z * 2.0 ** -23).all())
