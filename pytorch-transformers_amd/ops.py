@@ -794,7 +794,7 @@ def attention(q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: 
                 shape = (ctx.n_seqs, q.shape[1], k_pool.shape[1], q.shape[2], ctx.max_len, getattr(ctx, "mean_len", 0))
                 if window == 0 and chunk == 0:
                     tuning.note_decode_launch(*shape)
-                cut = tuning.decode_plan(*shape)
+                cut = tuning.several_waves_cut(*shape) or tuning.decode_plan(*shape)
             tiles, size, waves = cut
             n_splits = (ctx.max_len + size - 1) // size
         return attn_mfma(q, k_pool, v_pool, block_table, ctx.cu_tokens, ctx.seq_start, slopes, scale,

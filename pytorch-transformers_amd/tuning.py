@@ -290,6 +290,27 @@ def decode_plan(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_l
     return _decode_plan(n, n_heads, n_kv_heads, head_dim, bound, mean, most) + (1,)
 
 
+def several_waves_cut(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0):
+    """The cut of an untuned decode launch whose contexts are at most 1,024 keys and 512 on average: four waves of a workgroup
+    walk the whole context between them and merge in LDS, which leaves no ranges to merge by a launch of their own; or None,
+    where ``decode_plan`` decides.  Launch and merge, replayed over twelve caches in turn, the rule's ranges -> this, at 210
+    / 320 / 500 keys: 13 heads on 13 of 80, 5 sequences 10.8 -> 8.1, 11.1 -> 9.5, 11.6 -> 11.0 us, 16 sequences 11.8 -> 9.0, 12.5 ->
+    10.9, 15.8 -> 14.2, 32 (416 workgroups) 13.4 -> 13.7, 16.1 -> 17.2, 22.5 -> 20.5; 71 on 1 of 64, 8 sequences 7.9 -> 6.2,
+    8.5 -> 7.9, 9.1 -> 9.1; 128 on 8 of 64, 32 sequences 11.1 -> 7.7, 12.5 -> 9.3, 15.2 -> 13.2, 64 (512 workgroups) 10.1 -> 11.4, 11.7 ->
+    14.0, 16.6 -> 19.5.  Heads of 128 carry twice the sums through LDS: 32 on 8, 16 sequences 10.0 -> 9.8, 11.4 -> 12.1, 14.8 ->
+    16.2, 32 sequences 14.6 -> 12.9, 16.2 -> 15.3, 21.9 -> 20.6."""
+    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
+        return None
+    key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
+    n, _, _, _, bound, mean = key
+    if bound > 1024 or mean > 512 or key in _active.decode_plans:
+        return None
+    groups = n * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)  # workgroups of the launch
+    if groups > 320 or (head_dim > 80 and groups < 192) or not ops.load_library().pta_attn_decode_waves_ok(head_dim, 1, 4):
+        return None
+    return (1, bound, 4)
+
+
 def _shared_keys_rule(n: int, n_heads: int, n_kv_heads: int, head_dim: int, bound: int, mean: int):
     """The cut with keys shared through LDS where it is built (many heads on a KV head) and the launch walks keys
     enough to fill the chip with such workgroups, else None.  Measured with 71 heads on one KV head of 64, launch
