@@ -172,7 +172,7 @@ __global__ void epilogue_kernel(T* __restrict__ y, const float* __restrict__ bia
         T* at = y + (i / N) * ld + i % N;
         float v = Io<T>::ld(at);
         if (bias) v = Io<T>::round(v + bias[i % N]);
-        if (act) v = apply_act(v, act);
+        if (act) v = sizeof(T) == 2 ? apply_act_bf16(v, act) : apply_act(v, act);
         if (add1) v += Io<T>::ld(add1 + i);
         if (add2) v += Io<T>::ld(add2 + i);
         Io<T>::st(at, v);
@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256) void epilogue_bf16x8_kernel(bf16_t* __restrict
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (bias) v[e] = round_to_bf16(v[e] + b[e]);
-            if (ACT != PTA_ACT_NONE) v[e] = apply_act(v[e], ACT);
+            if (ACT != PTA_ACT_NONE) v[e] = apply_act_bf16(v[e], ACT);
             v[e] += x1[e];  // an absent addend was loaded as zeros
             v[e] += x2[e];
         }

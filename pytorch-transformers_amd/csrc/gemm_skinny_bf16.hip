@@ -269,8 +269,8 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
                 float v = OutIo<OutT>::round(sum[i]);
                 if (bias) v = OutIo<OutT>::round(v + bias[n]);
                 // other activations run as a pass of their own (4.7 us of a step's 10 us product with squared ReLU, 8,192 x 2,048)
-                if (act == PTA_ACT_GELU) v = gelu_erf(v);
-                else if (act == PTA_ACT_RELU2) v = apply_act(v, PTA_ACT_RELU2);
+                if (act == PTA_ACT_GELU) v = sizeof(OutT) == 2 ? gelu_bf16(v) : gelu_erf(v);
+                else if (act == PTA_ACT_RELU2) v = apply_act_bf16(v, PTA_ACT_RELU2);
                 const long o = (long)m * N + n;
                 if (add1) v += bf16_bits_to_f32(add1[o]);
                 if (add2) v += bf16_bits_to_f32(add2[o]);

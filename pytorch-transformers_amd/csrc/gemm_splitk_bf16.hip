@@ -219,7 +219,7 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
                 float v = acc[t][mt][i];
                 if (!out_f32) v = round_to_bf16(v);
                 if (bias) { v += bias[n + i]; if (!out_f32) v = round_to_bf16(v); }
-                if (act == PTA_ACT_GELU) v = gelu_erf(v);  // other activations: see pta_gemm_splitk_bf16
+                if (act == PTA_ACT_GELU) v = out_f32 ? gelu_erf(v) : gelu_bf16(v);  // other activations: see pta_gemm_splitk_bf16
                 if (add1) v += bf16_bits_to_f32(add1[o + i]);
                 if (add2) v += bf16_bits_to_f32(add2[o + i]);
                 if (out_f32) ((float*)y)[o + i] = v;
@@ -241,7 +241,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(void* __restric
     const int n = (int)(o % N);
     if (!out_f32) v = round_to_bf16(v);
     if (bias) { v += bias[n]; if (!out_f32) v = round_to_bf16(v); }
-    if (act) v = apply_act(v, act);
+    if (act) v = out_f32 ? apply_act(v, act) : apply_act_bf16(v, act);
     if (add1) v += bf16_bits_to_f32(add1[o]);
     if (add2) v += bf16_bits_to_f32(add2[o]);
     if (out_f32) ((float*)y)[o] = v;
@@ -267,7 +267,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce2_kernel(bf16_t* __rest
     for (int p = 1; p < P; ++p) v += part[(long)p * MN + o];
     v = round_to_bf16(v);
     if (bias) v = round_to_bf16(v + bias[(int)(o % N)]);
-    if (act) v = apply_act(v, act);
+    if (act) v = apply_act_bf16(v, act);
     (second ? y2 : y1)[o] = f32_to_bf16_bits(v);
 }
 
@@ -314,7 +314,7 @@ __global__ __launch_bounds__(256) void gemm_splitk_reduce2_qkv_kernel(QkvTail ta
     for (int q = 1; q < P2; ++q) v += part2[(long)q * MN2 + o];
     v = round_to_bf16(v);
     if (bias2) v = round_to_bf16(v + bias2[(int)(o % N2)]);
-    if (act2) v = apply_act(v, act2);
+    if (act2) v = apply_act_bf16(v, act2);
     y2[o] = f32_to_bf16_bits(v);
 }
 

@@ -95,19 +95,25 @@ __device__ __forceinline__ void tile_at(const TileJob& job, int t, int& tp, int&
 template <int ACT>
 __device__ __forceinline__ void store8(const TileJob& job, int m, int n, uint4 u) {
     if (ACT != PTA_ACT_NONE || job.bias || job.add1 || job.add2) {
-        const uint4 none = make_uint4(0u, 0u, 0u, 0u);
-        const uint4 u1 = job.add1 ? *reinterpret_cast<const uint4*>(job.add1 + (long)m * job.N + n) : none;
-        const uint4 u2 = job.add2 ? *reinterpret_cast<const uint4*>(job.add2 + (long)m * job.N + n) : none;
-        float v[8], x1[8], x2[8];
+        float v[8];
         unpack8(u, v);
-        unpack8(u1, x1);
-        unpack8(u2, x2);
 #pragma unroll
         for (int e = 0; e < 8; ++e) {
             if (job.bias) v[e] = round_to_bf16(v[e] + job.bias[n + e]);
-            if (ACT != PTA_ACT_NONE) v[e] = apply_act(v[e], ACT);
-            v[e] += x1[e];  // an absent addend is zeros: the arithmetic is epilogue_bf16x8_kernel's
-            v[e] += x2[e];
+            if (ACT != PTA_ACT_NONE) v[e] = apply_act_bf16(v[e], ACT);
+        }
+        if (job.add1 || job.add2) {
+            const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+            const uint4 u1 = job.add1 ? *reinterpret_cast<const uint4*>(job.add1 + (long)m * job.N + n) : none;
+            const uint4 u2 = job.add2 ? *reinterpret_cast<const uint4*>(job.add2 + (long)m * job.N + n) : none;
+            float x1[8], x2[8];
+            unpack8(u1, x1);
+            unpack8(u2, x2);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[e] += x1[e];  // an absent addend is zeros: the arithmetic is epilogue_bf16x8_kernel's
+                v[e] += x2[e];
+            }
         }
         u = pack8(v);
     }
