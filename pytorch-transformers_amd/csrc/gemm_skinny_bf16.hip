@@ -106,6 +106,21 @@ struct SkinnyProblem {
     int blocks;  // workgroups of this product
 };
 
+// what follows the product, for one feature: bias, activation, additions
+template <typename OutT>
+__device__ __forceinline__ void store_feature(OutT* y, const float* bias, int act, const bf16_t* add1, const bf16_t* add2, int N, int m,
+                                              int n, float sum) {
+    float v = OutIo<OutT>::round(sum);
+    if (bias) v = OutIo<OutT>::round(v + bias[n]);
+    // other activations run as a pass of their own (4.7 us of a step's 10 us product with squared ReLU, 8,192 x 2,048)
+    if (act == PTA_ACT_GELU) v = sizeof(OutT) == 2 ? gelu_bf16(v) : gelu_erf(v);
+    else if (act == PTA_ACT_RELU2) v = apply_act_bf16(v, PTA_ACT_RELU2);
+    const long o = (long)m * N + n;
+    if (add1) v += bf16_bits_to_f32(add1[o]);
+    if (add2) v += bf16_bits_to_f32(add2[o]);
+    OutIo<OutT>::st(y + o, v);
+}
+
 // With a QkvTail (qkv_tail.h) the first product's rows are not stored: they are split into heads, rotated and written
 // as queries and into the cache pages.  The rotation works on pairs of a head's elements, so a workgroup takes the
 // first elements of sixteen pairs as its first row tile and their partners as its second (TAIL 1: whole heads in
@@ -265,17 +280,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int n = n0 + rt * 16 + (ln >> 4) * 4 + i;
-            if (n < n1) {
-                float v = OutIo<OutT>::round(sum[i]);
-                if (bias) v = OutIo<OutT>::round(v + bias[n]);
-                // other activations run as a pass of their own (4.7 us of a step's 10 us product with squared ReLU, 8,192 x 2,048)
-                if (act == PTA_ACT_GELU) v = sizeof(OutT) == 2 ? gelu_bf16(v) : gelu_erf(v);
-                else if (act == PTA_ACT_RELU2) v = apply_act_bf16(v, PTA_ACT_RELU2);
-                const long o = (long)m * N + n;
-                if (add1) v += bf16_bits_to_f32(add1[o]);
-                if (add2) v += bf16_bits_to_f32(add2[o]);
-                OutIo<OutT>::st(y + o, v);
-            }
+            if (n < n1) store_feature<OutT>(y, bias, act, add1, add2, N, m, n, sum[i]);
         }
     }
 }
@@ -327,6 +332,112 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
     }
 }
 
+// Small matrices, eight rows of W or fewer a workgroup (N up to eight times the compute units): what bounds such a launch, apart
+// from its start, is not memory but the compute units' address paths, a wave's load taking sixteen cycles whatever it fetches,
+// and with eight rows in a tile of sixteen half of W's loads fetched nothing new.  So a tile is eight rows at two places of K:
+// lanes of rows 0 .. 7 carry 64 elements of a step of 128, lanes of rows 8 .. 15 the 64 behind them.  With up to eight rows
+// of x (DIAG) x is laid out the same way, and one matrix instruction makes both halves' sums, in the blocks on its
+// diagonal; with more, two instructions do, and of each the half that belongs together is kept.  Either way a sum is that of
+// the first halves of its wave's steps plus that of the second, the waves' in order: the same bits for any number of rows.
+// TAIL: a fused query_key_value product taken to its end as by gemm_skinny_tail_kernel; rows 0 .. 3 are the first elements of up
+// to four rotation pairs, rows 4 .. 7 their partners.
+template <int MT, bool DIAG, int U, typename OutT, bool TAIL>
+__global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p, int M, int K, int rot_stride, QkvTail tail) {
+    static_assert(!DIAG || MT == 1, "both halves of K in a tile: eight rows of x");
+    constexpr int BT = DIAG ? 1 : 2 * MT;  // fragments of x a half step
+    extern __shared__ f32x4_t part[];      // [S][MT][64]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const int r = lane & 15, g = lane >> 4, row = r & 7, sub = r >> 3;
+    const int half = TAIL ? tail.d >> 1 : 1;
+    const int items = TAIL ? (tail.nh + 2 * tail.nkv) * half : p.N;  // pairs, or rows, that the workgroups share evenly
+    const int n0 = (int)((long)blockIdx.x * items / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * items / gridDim.x);
+    int w_row = min(n0 + row, n1 - 1);
+    if (TAIL) {
+        const int mine = min(n0 + (row & 3), n1 - 1);  // (places past the end read a pair again)
+        int ea, eb;
+        bool rotated;
+        qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
+        w_row = mine / half * tail.d + (row < 4 ? ea : eb);
+    }
+    const bf16_t* wrow = p.W + (long)w_row * K;
+    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, M * K * 2, 0x00020000);
+    const int nsteps = (K + 127) >> 7;
+    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
+    struct Halves {
+        Frag a[U][2], b[U][2][BT];
+        uint32_t keep[U][2];
+    } s0, s1;
+    auto load = [&](Halves& st, int first) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            int step = first + u * S;
+            if (step < nsteps) { step += rot; step -= step >= nsteps ? nsteps : 0; }
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                const int at = step * 128 + hf * 32 + g * 8, k = at + sub * 64, kc = min(k, K - 8);
+                st.keep[u][hf] = k < K ? 0xffffffffu : 0u;
+                st.a[u][hf].u = *reinterpret_cast<const uint4*>(wrow + kc);
+#pragma unroll
+                for (int t = 0; t < BT; ++t) {  // a row past M lies outside the buffer's bounds: zeros, and no traffic
+                    const int m = DIAG ? row : (t >> 1) * 16 + r, kx = DIAG ? kc : min(at + (t & 1) * 64, K - 8);
+                    st.b[u][hf][t].i = __builtin_amdgcn_raw_buffer_load_b128(xres, (m * K + kx) * 2, 0, 0);
+                }
+            }
+        }
+    };
+    f32x4_t acc[BT];
+#pragma unroll
+    for (int t = 0; t < BT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](const Halves& st) {
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int hf = 0; hf < 2; ++hf) {
+                Frag a = st.a[u][hf];
+                const uint32_t keep = st.keep[u][hf];
+                a.u.x &= keep; a.u.y &= keep; a.u.z &= keep; a.u.w &= keep;
+#pragma unroll
+                for (int t = 0; t < BT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.v, st.b[u][hf][t].v, acc[t], 0, 0, 0);
+            }
+    };
+    load(s0, wave);
+    for (int step = wave; step < nsteps; step += 2 * U * S) {
+        load(s1, step + U * S);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(s0);
+        __builtin_amdgcn_sched_barrier(0);
+        load(s0, step + 2 * U * S);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(s1);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) part[(wave * MT + mt) * 64 + lane] = DIAG ? acc[0] : (g < 2 ? acc[mt * 2] : acc[BT > 1 ? mt * 2 + 1 : 0]);
+    __syncthreads();
+    const float* sums = (const float*)part;
+    auto sum_of = [&](int m, int i) {  // row i of the eight for row m of x
+        constexpr int OTHER = (32 + (DIAG ? 8 : 0)) * 4;
+        const int at = ((m >> 4) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
+        float v = sums[at] + sums[at + OTHER];
+        for (int w = 1; w < S; ++w) {
+            v += sums[w * MT * 256 + at];
+            v += sums[w * MT * 256 + at + OTHER];
+        }
+        return v;
+    };
+    if constexpr (TAIL) {
+        for (int item = threadIdx.x; item < 4 * M; item += blockDim.x) {
+            const int m = item >> 2, i = item & 3, pair = n0 + i;
+            if (pair < n1) qkv_tail_pair(tail, p.bias, m, pair / half, pair % half, round_to_bf16(sum_of(m, i)), round_to_bf16(sum_of(m, i + 4)));
+        }
+    } else {
+        for (int item = threadIdx.x; item < 8 * M; item += blockDim.x) {
+            const int m = item >> 3, i = item & 7;
+            if (n0 + i < n1) store_feature<OutT>((OutT*)p.y, p.bias, p.act, p.add1, p.add2, p.N, m, n0 + i, sum_of(m, i));
+        }
+    }
+}
+
 // Waves per workgroup, i.e. how many ways K is split.  Measured on MI355X: long streams per wave beat
 // many short ones, so K is split only when N alone gives too few waves.  It depends on N only, never
 // on M or on the tile variant, so the order of summation is the same for every batch.
@@ -367,14 +478,36 @@ static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hi
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, RT, U, OutT>), grid, block, lds, s, a, b, M, K, rot_stride, QkvTail{});
 }
 
+// where a workgroup has eight rows of W or fewer (N alone decides: one order of summation for any number of rows of x)
+static bool by_halves(int N) { return N <= 8 * pta_compute_units(); }
+
+template <typename OutT, bool TAIL = false>
+static int launch_halves(const SkinnyProblem& p, int M, int K, int S, hipStream_t s, const QkvTail& tail = QkvTail{}) {
+    const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 4 : 8, units = pta_compute_units();
+    if (S <= 0) S = 2;  // four waves 5.9 us at 2,048 x 2,048 and 8 rows, 7.6 at 16, two 5.4 and 6.7; longer rows within 2 %
+    const dim3 grid(std::max((items + most - 1) / most, std::min(units, (items + most / 2 - 1) / (most / 2)))), block(S * 64);
+    static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
+    const int rot = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 3 : 0);
+    auto go = [&](auto kernel, int tiles) { hipLaunchKernelGGL(kernel, grid, block, (size_t)S * tiles * 64 * sizeof(f32x4_t), s, p, M, K, rot, tail); };
+    if (M <= 8) go(gemm_skinny_halves_kernel<1, true, 2, OutT, TAIL>, 1);
+    else if (M <= 16) go(gemm_skinny_halves_kernel<1, false, 2, OutT, TAIL>, 1);
+    else if constexpr (!TAIL) {
+        if (M <= 32) go(gemm_skinny_halves_kernel<2, false, 1, OutT, false>, 2);
+        else if (M <= 48) go(gemm_skinny_halves_kernel<3, false, 1, OutT, false>, 3);
+        else go(gemm_skinny_halves_kernel<4, false, 1, OutT, false>, 4);
+    }
+    return pta_check_launch("gemm_skinny_bf16");
+}
+
 template <typename OutT>
 static int launch_skinny(SkinnyProblem a, SkinnyProblem b, int M, int K, int variant, int S, hipStream_t s) {
     // variant: row tiles per wave and steps per stage (6: one tile, its rows spread over all units); 0: chosen here
     // Tiles of 32 rows of W that would occupy half of the compute units or fewer: a unit pulls no more than some 24 GB/s, so
     // the rows are spread over all units instead, a few rows each (the rest of a tile's lanes read a row again).  Replays over
-    // cold weights, 8 rows of x, 32-row tiles -> spread: 2,048 x 8,192 24.0 -> 13.6 us, 2,048 x 2,048 9.7 -> 6.4, 3,072 x
-    // 2,048 9.8 -> 7.0, 1,040 x 4,160 15.2 -> 8.3; with more tiles the second read of x costs more than the units win (5,504
+    // cold weights, 8 rows of x, 32-row tiles -> spread: 3,072 x 2,048 9.8 -> 7.0 us (up to eight rows a unit:
+    // gemm_skinny_halves_kernel); with more tiles the second read of x costs more than the units win (5,504
     // x 2,048 9.2 -> 9.8, at 16 rows of x 9.9 -> 11.7).
+    if (variant == 7 || (variant == 0 && b.N == 0 && by_halves(a.N))) return launch_halves<OutT>(a, M, K, S, s);
     if (variant == 0 && b.N == 0 && pta_gemm_skinny_spread(a.N)) variant = 6;
     if (M <= 16) {
         if (variant == 0) variant = 2;
@@ -416,7 +549,7 @@ extern "C" int pta_gemm_skinny_bf16(void* y, const void* x, const void* W, const
                                     const void* add2, int M, int N, int K, int act, int out_f32, int variant,
                                     int waves, void* stream) {
     if (check_skinny("gemm_skinny_bf16", y, x, W, M, N, K, act)) return 1;
-    PTA_REQUIRE(variant >= 0 && variant <= 6, "gemm_skinny_bf16: unknown variant %d", variant);
+    PTA_REQUIRE(variant >= 0 && variant <= 7, "gemm_skinny_bf16: unknown variant %d", variant);
     PTA_REQUIRE(waves == 0 || (waves >= 1 && waves <= 8 && (waves & (waves - 1)) == 0),
                 "gemm_skinny_bf16: waves per workgroup must be 0 (choose) or a power of two up to 8, got %d", waves);
     hipStream_t s = (hipStream_t)stream;
@@ -505,6 +638,10 @@ extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* 
     PTA_REQUIRE(!write_cache || (k_pool && v_pool && block_table && token_seq), "gemm_skinny_qkv_bf16: null cache pointer");
     const QkvTail tail{(bf16_t*)q_out, rot, token_pos, token_seq, block_table, bt_stride, (bf16_t*)k_pool,
                        (bf16_t*)v_pool, nh, nkv, d, layout, write_cache};
+    if (by_halves(N)) {
+        const SkinnyProblem p{nullptr, (const bf16_t*)x, (const bf16_t*)W, bias, nullptr, nullptr, N, PTA_ACT_NONE, 0};
+        return launch_halves<bf16_t, true>(p, M, K, 0, (hipStream_t)stream, tail);
+    }
     const int pairs = N / 2;
     const int blocks = std::max((pairs + 7) / 8, std::min(pta_compute_units(), (pairs + 1) / 2));
     const int S = pick_split(N);
