@@ -19,6 +19,7 @@
 #include <stdlib.h>
 
 #include <algorithm>
+#include <type_traits>
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
@@ -438,6 +439,142 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
     }
 }
 
+// The product of few rows together with the LayerNorm in front of it, y = act(LN(x) . W^T + bias), rows of up to 2,048
+// elements.  As launches of their own a norm of a few rows takes 4.7 us, nearly all of it what any launch costs; here every
+// workgroup norms the rows for itself while its rows of W are on their way: rows of x are asked for first, then the norm's
+// vectors, then all of the workgroup's W (a range of up to 2,048 elements: 16 loads a lane), so that the norm waits for its own
+// loads alone.  Normed rows lie in LDS, rounded to bfloat16 as the norm's own launch stores them, and are read from there as the
+// B operand: x passes the address path once a workgroup, not once a wave.  Statistics in 32-bit, mean first.
+// TAIL: a fused query_key_value product taken to its end as by gemm_skinny_tail_kernel.
+// Replays over cold weights, norm and product -> this: 5 rows, 3,120 x 1,040 8.2 -> 5.1 us, 4,160 x 1,040 8.8 -> 6.3, 3,072 x 2,048
+// 10.2 -> 6.7, 8,192 x 2,048 13.6 -> 11.7; 16 rows, 3,072 x 768 9.2 -> 5.4, 3,072 x 2,048 11.4 -> 8.3, 8,192 x 2,048 14.7 -> 15.4.  Eight waves
+// finish the norm sooner, four leave room for a second workgroup on the unit (8,192 x 2,048 at 5 rows: 12.4 and 11.7).
+template <int NORMED_WAVES, int CH, int RW, bool TAIL>  // CH: groups of 512 elements of a row; RW: rows of x a wave norms
+__global__ __launch_bounds__(NORMED_WAVES * 64) void gemm_normed_kernel(SkinnyProblem p, const float* __restrict__ ln_w,
+                                                                       const float* __restrict__ ln_b, float eps, int M, int K,
+                                                                       QkvTail tail) {
+    constexpr int STEPS = 8 * CH / NORMED_WAVES;  // steps of 64 elements of K a wave takes
+    extern __shared__ f32x4_t part[];  // [waves][64], then the normed rows [M][K + 8]
+    bf16_t* rows = (bf16_t*)(part + NORMED_WAVES * 64);
+    const int pitch = K + 8;  // sixteen bytes between rows keep the reads of sixteen rows on distinct banks
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int r = lane & 15, g = lane >> 4, half = TAIL ? tail.d >> 1 : 1;
+    const int items = TAIL ? (tail.nh + 2 * tail.nkv) * half : p.N;
+    const int n0 = (int)((long)blockIdx.x * items / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * items / gridDim.x);
+    int w_row = min(n0 + r, n1 - 1);
+    if (TAIL) {  // as in gemm_skinny_tail_kernel
+        const int mine = min(n0 + (r & 7), n1 - 1);
+        int ea, eb;
+        bool rotated;
+        qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
+        w_row = mine / half * tail.d + (r < 8 ? ea : eb);
+    }
+    const bf16_t* wrow = p.W + (long)w_row * K;
+    const int chunks = K >> 3;
+    uint4 xv[RW][CH];
+    float gain[CH][8], shift[CH][8];
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+            xv[i][j] = *reinterpret_cast<const uint4*>(p.x + (long)min(wave + i * NORMED_WAVES, M - 1) * K + min(lane + j * 64, chunks - 1) * 8);
+#pragma unroll
+    for (int j = 0; j < CH; ++j) {
+        const int at = min(lane + j * 64, chunks - 1) * 8;
+#pragma unroll
+        for (int e = 0; e < 8; e += 4) {
+            *reinterpret_cast<float4*>(&gain[j][e]) = *reinterpret_cast<const float4*>(ln_w + at + e);
+            *reinterpret_cast<float4*>(&shift[j][e]) = *reinterpret_cast<const float4*>(ln_b + at + e);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    Frag a[STEPS][2];
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+            a[u][hf].u = *reinterpret_cast<const uint4*>(wrow + min((wave + u * NORMED_WAVES) * 64 + hf * 32 + g * 8, K - 8));
+    __builtin_amdgcn_sched_barrier(0);
+    float v[RW][CH][8], sum[RW], mean[RW];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        sum[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            unpack8(xv[i][j], v[i][j]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) sum[i] += lane + j * 64 < chunks ? v[i][j][e] : 0.f;
+        }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < RW; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        mean[i] = sum[i] / (float)K;
+        sum[i] = 0.f;
+#pragma unroll
+        for (int j = 0; j < CH; ++j)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                v[i][j][e] -= mean[i];
+                sum[i] += lane + j * 64 < chunks ? v[i][j][e] * v[i][j][e] : 0.f;
+            }
+    }
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+        for (int i = 0; i < RW; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+        const int m = wave + i * NORMED_WAVES;
+        if (m >= M) break;
+        const float rstd = 1.0f / sqrtf(sum[i] / (float)K + eps);
+#pragma unroll
+        for (int j = 0; j < CH; ++j) {
+            float o[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = v[i][j][e] * rstd * gain[j][e] + shift[j][e];
+            if (lane + j * 64 < chunks) *reinterpret_cast<uint4*>(rows + m * pitch + (lane + j * 64) * 8) = pack8(o);
+        }
+    }
+    // the barrier waits for LDS alone: W stays on its way
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const bf16_t* mine = rows + min(r, M - 1) * pitch;  // (columns past M repeat the last row and are not stored)
+#pragma unroll
+    for (int u = 0; u < STEPS; ++u)
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const int k = (wave + u * NORMED_WAVES) * 64 + hf * 32 + g * 8;
+            const uint32_t keep = k < K ? 0xffffffffu : 0u;
+            Frag b;
+            b.u = *reinterpret_cast<const uint4*>(mine + min(k, K - 8));
+            a[u][hf].u.x &= keep; a[u][hf].u.y &= keep; a[u][hf].u.z &= keep; a[u][hf].u.w &= keep;
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][hf].v, b.v, acc, 0, 0, 0);
+        }
+    part[wave * 64 + lane] = acc;
+    __syncthreads();
+    const float* sums = (const float*)part;  // row i of the tile, column m: lane (i / 4) * 16 + m, element i % 4
+    auto sum_of = [&](int m, int i) {
+        const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
+        float s = sums[at];
+#pragma unroll
+        for (int w = 1; w < NORMED_WAVES; ++w) s += sums[w * 256 + at];
+        return s;
+    };
+    const int per = TAIL ? 8 : 16;
+    for (int item = threadIdx.x; item < per * M; item += NORMED_WAVES * 64) {
+        const int m = item / per, i = item % per, n = n0 + i;
+        if (n >= n1) continue;
+        if constexpr (TAIL) qkv_tail_pair(tail, p.bias, m, n / half, n % half, round_to_bf16(sum_of(m, i)), round_to_bf16(sum_of(m, i + 8)));
+        else store_feature<bf16_t>((bf16_t*)p.y, p.bias, p.act, nullptr, nullptr, p.N, m, n, sum_of(m, i));
+    }
+}
+
 // Waves per workgroup, i.e. how many ways K is split.  Measured on MI355X: long streams per wave beat
 // many short ones, so K is split only when N alone gives too few waves.  It depends on N only, never
 // on M or on the tile variant, so the order of summation is the same for every batch.
@@ -617,39 +754,106 @@ extern "C" int pta_gemm_skinny_pair_qkv_bf16(void* q_out, const void* x1, const 
 // Whether pta_gemm_skinny_qkv_bf16 is the launch for a fused product of so many rows of W: where they are spread over the units
 extern "C" int pta_gemm_skinny_spread(int N) { return N > 0 && (N + 31) / 32 <= pta_compute_units() / 2; }
 
+// The operands of a fused query_key_value projection on its own, checked: up to 16 rows, any even head size up to 256
+static int make_tail_problem(const char* what, void* q_out, const void* x, const void* W, const float* bias, const PtaRotation* rotation,
+                             const int* token_pos, const int* token_seq, const int* block_table, int bt_stride, void* k_pool, void* v_pool,
+                             int nh, int nkv, int d, int layout, int write_cache, int M, int K, SkinnyProblem& p, QkvTail& tail) {
+    PTA_REQUIRE(nh > 0 && nkv > 0 && d > 0 && nh % nkv == 0, "%s: heads %d, kv heads %d, head size %d", what, nh, nkv, d);
+    const int N = (nh + 2 * nkv) * d;
+    if (check_skinny(what, q_out, x, W, M, N, K, PTA_ACT_NONE)) return 1;
+    PTA_REQUIRE(M <= 16, "%s: at most 16 rows, got %d", what, M);
+    PTA_REQUIRE(d % 2 == 0 && d <= 256, "%s: head size %d must be even and at most 256", what, d);
+    PTA_REQUIRE(layout >= 0 && layout <= 2, "%s: unknown layout %d", what, layout);
+    PTA_REQUIRE(layout != PTA_QKV_TAIL || nkv == 1, "%s: the tail layout has one kv head, got %d", what, nkv);
+    PTA_REQUIRE(layout != PTA_QKV_INTERLEAVED || nkv == nh, "%s: the interleaved layout needs kv heads == heads", what);
+    PTA_REQUIRE(token_pos, "%s: null token positions", what);
+    const PtaRotation rot = pta_rotation_of(rotation);
+    if (pta_check_rotation(what, rot, d, token_seq)) return 1;
+    PTA_REQUIRE(!write_cache || (k_pool && v_pool && block_table && token_seq), "%s: null cache pointer", what);
+    p = SkinnyProblem{nullptr, (const bf16_t*)x, (const bf16_t*)W, bias, nullptr, nullptr, N, PTA_ACT_NONE, 0};
+    tail = QkvTail{(bf16_t*)q_out, rot, token_pos, token_seq, block_table, bt_stride, (bf16_t*)k_pool,
+                   (bf16_t*)v_pool, nh, nkv, d, layout, write_cache};
+    return 0;
+}
+
 // A fused query_key_value projection on its own for up to 16 rows, with the tail of pta_gemm_skinny_pair_qkv_bf16; any even
 // head size up to 256, N = (nh + 2 nkv) d within pta_gemm_skinny_spread.
 extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const float* bias, const PtaRotation* rotation,
                                         const int* token_pos, const int* token_seq, const int* block_table, int bt_stride,
                                         void* k_pool, void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K,
                                         void* stream) {
-    PTA_REQUIRE(nh > 0 && nkv > 0 && d > 0 && nh % nkv == 0, "gemm_skinny_qkv_bf16: heads %d, kv heads %d, head size %d", nh, nkv, d);
-    const int N = (nh + 2 * nkv) * d;
-    if (check_skinny("gemm_skinny_qkv_bf16", q_out, x, W, M, N, K, PTA_ACT_NONE)) return 1;
-    PTA_REQUIRE(M <= 16, "gemm_skinny_qkv_bf16: at most 16 rows, got %d", M);
-    PTA_REQUIRE(d % 2 == 0 && d <= 256, "gemm_skinny_qkv_bf16: head size %d must be even and at most 256", d);
+    SkinnyProblem p;
+    QkvTail tail;
+    if (make_tail_problem("gemm_skinny_qkv_bf16", q_out, x, W, bias, rotation, token_pos, token_seq, block_table, bt_stride, k_pool,
+                          v_pool, nh, nkv, d, layout, write_cache, M, K, p, tail)) return 1;
+    const int N = p.N;
     PTA_REQUIRE(pta_gemm_skinny_spread(N), "gemm_skinny_qkv_bf16: %d rows of W are too many for this launch", N);
-    PTA_REQUIRE(layout >= 0 && layout <= 2, "gemm_skinny_qkv_bf16: unknown layout %d", layout);
-    PTA_REQUIRE(layout != PTA_QKV_TAIL || nkv == 1, "gemm_skinny_qkv_bf16: the tail layout has one kv head, got %d", nkv);
-    PTA_REQUIRE(layout != PTA_QKV_INTERLEAVED || nkv == nh, "gemm_skinny_qkv_bf16: the interleaved layout needs kv heads == heads");
-    PTA_REQUIRE(token_pos, "gemm_skinny_qkv_bf16: null token positions");
-    const PtaRotation rot = pta_rotation_of(rotation);
-    if (pta_check_rotation("gemm_skinny_qkv_bf16", rot, d, token_seq)) return 1;
-    PTA_REQUIRE(!write_cache || (k_pool && v_pool && block_table && token_seq), "gemm_skinny_qkv_bf16: null cache pointer");
-    const QkvTail tail{(bf16_t*)q_out, rot, token_pos, token_seq, block_table, bt_stride, (bf16_t*)k_pool,
-                       (bf16_t*)v_pool, nh, nkv, d, layout, write_cache};
-    if (by_halves(N)) {
-        const SkinnyProblem p{nullptr, (const bf16_t*)x, (const bf16_t*)W, bias, nullptr, nullptr, N, PTA_ACT_NONE, 0};
-        return launch_halves<bf16_t, true>(p, M, K, 0, (hipStream_t)stream, tail);
-    }
+    if (by_halves(N)) return launch_halves<bf16_t, true>(p, M, K, 0, (hipStream_t)stream, tail);
     const int pairs = N / 2;
     const int blocks = std::max((pairs + 7) / 8, std::min(pta_compute_units(), (pairs + 1) / 2));
     const int S = pick_split(N);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
     hipLaunchKernelGGL(gemm_skinny_tail_kernel, dim3(blocks), dim3(S * 64), (size_t)S * 64 * sizeof(f32x4_t), (hipStream_t)stream,
-                       (const bf16_t*)x, (const bf16_t*)W, bias, M, K, rot_stride, tail);
+                       p.x, p.W, bias, M, K, rot_stride, tail);
     return pta_check_launch("gemm_skinny_qkv_bf16");
+}
+
+// Whether the two entry points below take so many rows of x, elements of K and rows of W: each workgroup norms the rows again, which
+// pays with two workgroups a compute unit up to eight rows of x, with one up to sixteen
+extern "C" int pta_gemm_normed_ok(int M, int N, int K) {
+    return M > 0 && M <= 16 && K > 0 && K % 8 == 0 && K <= 2048 && N > 0 && N <= (M <= 8 ? 32 : 16) * pta_compute_units();
+}
+
+template <bool TAIL>
+static int launch_normed(const char* what, const SkinnyProblem& p, const float* ln_w, const float* ln_b, float eps, int M, int K,
+                         const QkvTail& tail, hipStream_t s) {
+    PTA_REQUIRE(pta_gemm_normed_ok(M, p.N, K), "%s: M=%d N=%d K=%d are not for this launch", what, M, p.N, K);
+    PTA_REQUIRE(ln_w && ln_b && ((uintptr_t)ln_w % 16) == 0 && ((uintptr_t)ln_b % 16) == 0, "%s: the norm's vectors must be there and 16-byte aligned", what);
+    const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 8 : 16, units = pta_compute_units();
+    const int groups = std::max((items + most - 1) / most, std::min(units, (items + most / 4 - 1) / (most / 4)));
+    const bool eight = groups <= units + units / 16;
+    const int waves = eight ? 8 : 4;
+    const size_t lds = waves * 64 * sizeof(f32x4_t) + (size_t)M * (K + 8) * sizeof(bf16_t);
+    bool refused = false;
+    auto go = [&](auto kernel) {
+        if (lds > 64 * 1024) refused = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess;
+        if (!refused) hipLaunchKernelGGL(kernel, dim3(groups), dim3(waves * 64), lds, s, p, ln_w, ln_b, eps, M, K, tail);
+    };
+    auto by_rows = [&](auto ch) {
+        constexpr int CH = decltype(ch)::value;
+        if (eight && M <= 8) go(gemm_normed_kernel<8, CH, 1, TAIL>);
+        else if (eight) go(gemm_normed_kernel<8, CH, 2, TAIL>);
+        else go(gemm_normed_kernel<4, CH, 2, TAIL>);  // (more workgroups than units: up to eight rows)
+    };
+    switch ((K + 511) / 512) {
+        case 1: by_rows(std::integral_constant<int, 1>{}); break;
+        case 2: by_rows(std::integral_constant<int, 2>{}); break;
+        case 3: by_rows(std::integral_constant<int, 3>{}); break;
+        default: by_rows(std::integral_constant<int, 4>{}); break;
+    }
+    PTA_REQUIRE(!refused, "%s: %zu bytes of LDS were refused", what, lds);
+    return pta_check_launch(what);
+}
+
+extern "C" int pta_gemm_normed_bf16(void* y, const void* x, const float* ln_w, const float* ln_b, float eps, const void* W,
+                                    const float* bias, int M, int N, int K, int act, void* stream) {
+    if (check_skinny("gemm_normed_bf16", y, x, W, M, N, K, act)) return 1;
+    const SkinnyProblem p{y, (const bf16_t*)x, (const bf16_t*)W, bias, nullptr, nullptr, N, in_kernel(act) ? act : PTA_ACT_NONE, 0};
+    if (launch_normed<false>("gemm_normed_bf16", p, ln_w, ln_b, eps, M, K, QkvTail{}, (hipStream_t)stream)) return 1;
+    return in_kernel(act) ? 0 : pta_epilogue(y, N, nullptr, nullptr, nullptr, M, N, act, PTA_BF16, stream);
+}
+
+// The same with the tail of pta_gemm_skinny_qkv_bf16
+extern "C" int pta_gemm_normed_qkv_bf16(void* q_out, const void* x, const float* ln_w, const float* ln_b, float eps, const void* W,
+                                        const float* bias, const PtaRotation* rotation, const int* token_pos, const int* token_seq,
+                                        const int* block_table, int bt_stride, void* k_pool, void* v_pool, int nh, int nkv, int d,
+                                        int layout, int write_cache, int M, int K, void* stream) {
+    SkinnyProblem p;
+    QkvTail tail;
+    if (make_tail_problem("gemm_normed_qkv_bf16", q_out, x, W, bias, rotation, token_pos, token_seq, block_table, bt_stride, k_pool,
+                          v_pool, nh, nkv, d, layout, write_cache, M, K, p, tail)) return 1;
+    return launch_normed<true>("gemm_normed_qkv_bf16", p, ln_w, ln_b, eps, M, K, tail, (hipStream_t)stream);
 }
 
 // Two products of one launch: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2), both [M, *] in

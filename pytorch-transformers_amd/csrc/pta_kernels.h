@@ -175,6 +175,16 @@ int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const fl
                              const int* token_pos, const int* token_seq, const int* block_table, int bt_stride, void* k_pool,
                              void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K, void* stream);
 
+// the product of up to 16 rows of up to 2,048 elements with the LayerNorm in front of it, y = act(LN(x) . W^T + bias), and the
+// fused query_key_value product likewise; _ok says whether the launch takes the sizes
+int pta_gemm_normed_ok(int M, int N, int K);
+int pta_gemm_normed_bf16(void* y, const void* x, const float* ln_w, const float* ln_b, float eps, const void* W, const float* bias,
+                         int M, int N, int K, int act, void* stream);
+int pta_gemm_normed_qkv_bf16(void* q_out, const void* x, const float* ln_w, const float* ln_b, float eps, const void* W,
+                             const float* bias, const PtaRotation* rotation, const int* token_pos, const int* token_seq,
+                             const int* block_table, int bt_stride, void* k_pool, void* v_pool, int nh, int nkv, int d, int layout,
+                             int write_cache, int M, int K, void* stream);
+
 // The same product for a batch of up to 128 rows that shares x through LDS and may split K over workgroups:
 // `part` is a 32-bit workspace [parts, M, N], needed when parts > 1 or reduce = 0.  rt (row tiles per wave),
 // parts, stage_blocks (64-element blocks of K per stage) and depth (stages in flight) are tuning knobs (0:

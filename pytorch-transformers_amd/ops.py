@@ -180,6 +180,10 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[18], (a[13] + 2 * a[14]) * a[15], a[5])
     if name == "pta_gemm_tile_bf16":
         return gemm(a[8], a[9], a[10])
+    if name == "pta_gemm_normed_bf16":
+        return gemm(a[7], a[8], a[9])
+    if name == "pta_gemm_normed_qkv_bf16":
+        return gemm(a[19], (a[14] + 2 * a[15]) * a[16], a[20])
     if name == "pta_gemm_f32":
         return gemm(a[6], a[7], a[8], 4)
     if name == "pta_layernorm_sum":
@@ -1334,6 +1338,50 @@ def gemm_skinny_qkv(x: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_freq, cs
     _call("pta_gemm_skinny_qkv_bf16", _ptr(q), _ptr(x), _ptr(w_qkv), _ptr(bias_qkv), rot, _ptr(token_pos), _ptr(token_seq),
           _ptr(block_table), block_table.shape[1], _ptr(k_pool), _ptr(v_pool), nh, nkv, d, QKV_LAYOUT_CODES[layout],
           int(write_cache), M, K, _stream())
+    return q
+
+
+GEMM_NORMED = os.environ.get("PTA_GEMM_NORMED", "1") != "0"
+
+
+def gemm_normed_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the LayerNorm of ``x`` rides in the launch of its product with ``w``: up to 16 rows of bfloat16 of up to 2,048
+    elements, and matrices of so few rows that the norm is not done over too often (the figures are at ``gemm_normed_kernel``)."""
+    return (GEMM_NORMED and _bf16_rows_ok(x, w) and x.is_contiguous() and w.is_contiguous()
+            and bool(load_library().pta_gemm_normed_ok(int(x.shape[0]), int(w.shape[0]), int(x.shape[1]))))
+
+
+def gemm_normed(x: torch.Tensor, ln_w: torch.Tensor, ln_b: torch.Tensor, eps: float, w: torch.Tensor, bias=None, act=None) -> torch.Tensor:
+    """act(LayerNorm(x) @ w.T + bias), the normed rows rounded to bfloat16 on the way (``gemm_normed_ok``)."""
+    _need(x, "x", torch.bfloat16)
+    _need(w, "w", torch.bfloat16)
+    M, K = x.shape
+    N = w.shape[0]
+    if w.shape[1] != K:
+        raise KernelError(f"x is [{M}, {K}] but w is {tuple(w.shape)}; w must be [N, {K}]")
+    _need(ln_w, "norm weight", torch.float32, (K,))
+    _need(ln_b, "norm bias", torch.float32, (K,))
+    if bias is not None:
+        _need(bias, "bias", torch.float32, (N,))
+    y = torch.empty((M, N), dtype=torch.bfloat16, device=x.device)
+    _call("pta_gemm_normed_bf16", _ptr(y), _ptr(x), _ptr(ln_w), _ptr(ln_b), ctypes.c_float(eps), _ptr(w), _ptr(bias), M, N, K,
+          ACT_CODES[act], _stream())
+    return y
+
+
+def gemm_normed_qkv(x: torch.Tensor, ln_w: torch.Tensor, ln_b: torch.Tensor, eps: float, w_qkv: torch.Tensor, bias_qkv, inv_freq,
+                    cs_scale: float, token_pos, token_seq, block_table, k_pool, v_pool, nh: int, nkv: int, d: int, layout: str,
+                    write_cache: bool, rotary_dim: Optional[int] = None, pairing: str = "half"):
+    """``gemm_skinny_qkv`` of LayerNorm(x), the norm in the same launch (``gemm_normed_ok``)."""
+    rot = _check_qkv(x, w_qkv, bias_qkv, inv_freq, cs_scale, token_pos, token_seq, block_table, k_pool, v_pool, nh, nkv, d,
+                     rotary_dim, pairing)
+    M, K = x.shape
+    _need(ln_w, "norm weight", torch.float32, (K,))
+    _need(ln_b, "norm bias", torch.float32, (K,))
+    q = torch.empty((M, nh, d), dtype=torch.bfloat16, device=x.device)
+    _call("pta_gemm_normed_qkv_bf16", _ptr(q), _ptr(x), _ptr(ln_w), _ptr(ln_b), ctypes.c_float(eps), _ptr(w_qkv), _ptr(bias_qkv), rot,
+          _ptr(token_pos), _ptr(token_seq), _ptr(block_table), block_table.shape[1], _ptr(k_pool), _ptr(v_pool), nh, nkv, d,
+          QKV_LAYOUT_CODES[layout], int(write_cache), M, K, _stream())
     return q
 
 

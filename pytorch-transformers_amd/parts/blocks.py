@@ -116,15 +116,33 @@ class SequentialBlock(Part):
         return (self.norm_in, self.norm_post, self.mixer, self.feed_forward)
 
     def forward(self, x, ctx: StepContext, call):
-        x, a, _ = _normed(x, self.norm_in)
-        if _can_defer(self.mixer):
-            r = _sum_sequential(self.mixer.forward(a, ctx, call, defer=True), x)
+        # in steps of few tokens each norm rides in the launch of the product behind it
+        kw, projected = {}, None
+        if isinstance(x, torch.Tensor) and hasattr(self.mixer, "projection_tail"):
+            projected = self.mixer.input_projection()[0].normed(x, self.norm_in, tail=lambda: self.mixer.projection_tail(ctx, call))
+        if projected is not None:
+            a, kw["projected"] = x, projected
         else:
-            r = self.mixer.forward(a, ctx, call, residual=x)
-        r, m, _ = _normed(r, self.norm_post)
+            x, a, _ = _normed(x, self.norm_in)
+        if _can_defer(self.mixer):
+            r = _sum_sequential(self.mixer.forward(a, ctx, call, defer=True, **kw), x)
+        else:
+            r = self.mixer.forward(a, ctx, call, residual=x, **kw)
+        kw = {}
+        if isinstance(r, torch.Tensor) and hasattr(self.feed_forward, "input_projection"):
+            linear, how = self.feed_forward.input_projection()
+            projected = linear.normed(r, self.norm_post, **how)
+            if projected is not None:
+                kw["projected"] = projected
+        if kw:
+            m = r
+        else:
+            r, m, _ = _normed(r, self.norm_post)
         if _can_defer(self.feed_forward):
-            return _sum_sequential(self.feed_forward.forward(m, ctx, defer=True), r)
-        return self.feed_forward.forward(m, ctx, add1=r)
+            # a sum left to the next norm (the next block's first) would keep that norm out of its product's launch
+            out = self.feed_forward.forward(m, ctx, defer=True, **kw)
+            return out.run(add1=r) if kw else _sum_sequential(out, r)
+        return self.feed_forward.forward(m, ctx, add1=r, **kw)
 
 
 class PostNormBlock(Part):

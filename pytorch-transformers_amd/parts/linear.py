@@ -132,6 +132,21 @@ class Linear(Part):
             tail.k_pool, tail.v_pool, tail.num_heads, tail.kv_heads, tail.head_dim, tail.layout, tail.write_cache,
             **tail.how))
 
+    def normed(self, x: torch.Tensor, norm, *, act: Optional[str] = None, apply_bias: bool = True, tail=None):
+        """``self(norm(x))`` from one launch, where ``norm`` offers itself to it (``LayerNorm.fused``), else None.  ``tail``: a
+        function that makes the ``QkvTail`` by which the launch takes the product to its end, as in ``with_tail``."""
+        how = norm.fused(x, self) if hasattr(norm, "fused") else None
+        if how is None:
+            return None
+        if tail is None:
+            return ops.gemm_normed(x, *how, self.weight, self.bias if apply_bias else None, act)
+        tail = tail()
+        if not (ops.QKV_TAIL and tail.head_dim % 2 == 0 and tail.head_dim <= 256):
+            return None
+        return TailDone(ops.gemm_normed_qkv(
+            x, *how, self.weight, tail.bias, tail.inv_freq, tail.cs_scale, tail.token_pos, tail.token_seq, tail.table,
+            tail.k_pool, tail.v_pool, tail.num_heads, tail.kv_heads, tail.head_dim, tail.layout, tail.write_cache, **tail.how))
+
     @staticmethod
     def pair(first: "Linear", x1: torch.Tensor, kw1: dict, second: "Linear", x2: torch.Tensor, kw2: dict, tail=None):
         """``(first(x1, **kw1), second(x2, **kw2))`` from one matrix launch, in steps small enough for the

@@ -79,6 +79,13 @@ class LayerNorm(Part):
         return self.forward(x), other.forward(x)
 
 
+    def fused(self, x: torch.Tensor, linear) -> Optional[tuple]:
+        """(weight, bias, eps) for a launch that norms ``x`` and multiplies it with ``linear`` at once, or None where it is not
+        built or not the faster way; the product must be the norm's only reader."""
+        if type(self).forward is LayerNorm.forward and x.dtype == torch.bfloat16 and x.shape[1] == self.hidden_size and ops.gemm_normed_ok(x, linear.weight):
+            return self.weight, self.bias, self.eps
+        return None
+
     def forward_sum(self, total: ResidualSum, rows: Optional[torch.Tensor] = None, other: Optional["Part"] = None,
                     want_x: bool = True):
         """``(x, self(x), other(x))`` for the unformed sum ``total``: x is formed, rounded and normalised in

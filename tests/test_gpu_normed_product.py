@@ -1,0 +1,73 @@
+"""The product of few rows with the LayerNorm in front of it in one launch, against 64 bits and against the launches it stands
+for, at the edges of its sizes."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _draw(M, N, K, seed):
+    g = torch.Generator().manual_seed(seed)
+    r = lambda *s: torch.randn(*s, generator=g).cuda()
+    x = (r(M, K) * 3 + 1).bfloat16()
+    return x, (0.05 * r(N, K)).bfloat16(), 1 + 0.2 * r(K), 0.2 * r(K), r(N)
+
+
+@pytest.mark.parametrize("M", [1, 4, 5, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(1, 8), (17, 64), (300, 504), (4160, 512), (1040, 520), (4160, 1040), (2304, 768), (8192, 2048), (33, 2040)])
+@pytest.mark.parametrize("act", [None, "gelu", "silu"])
+def test_norm_and_product(M, N, K, act):
+    from pytorch_transformers_amd import ops
+
+    x, w, gain, shift, bias = _draw(M, N, K, M + N + K)
+    if N > 4096 and M > 8:
+        assert not ops.gemm_normed_ok(x, w)
+        return
+    assert ops.gemm_normed_ok(x, w)
+    got = ops.gemm_normed(x, gain, shift, 1e-5, w, bias, act).double()
+    rows = torch.nn.functional.layer_norm(x.double(), (K,), gain.double(), shift.double(), 1e-5).bfloat16().double()
+    z = rows @ w.double().T
+    z = (z.bfloat16().double() + bias.double()).bfloat16().double()
+    want = z if act is None else getattr(torch.nn.functional, act)(z)
+    # normed rows may be rounded to the neighbour where 32-bit statistics are a little off (2^-8 of an element, in few places);
+    # the product and the sum with the bias are rounded to 2^-8 of themselves each
+    size = (rows.abs() @ w.double().abs().T).max()
+    tol = 2.0 ** -7 * (z.abs() + bias.double().abs()) + 2.0 ** -8 * size / K ** 0.5 + 2.0 ** -8 * want.abs() + 1e-6
+    assert bool(((got - want).abs() <= 1.2 * tol).all())
+    assert (got - want).norm() <= 2.0 ** -8 * want.norm() + 1e-6
+    plain = ops.gemm_skinny_bf16(ops.layernorm(x, gain, shift, 1e-5), w, bias, act).double()
+    assert (plain - got).norm() <= 2.0 ** -8 * want.norm() + 1e-6
+
+
+@pytest.mark.parametrize("layout,nh,nkv,d", [("interleaved", 13, 13, 80), ("grouped", 4, 2, 6), ("tail", 7, 1, 64), ("tail", 1, 1, 2)])
+@pytest.mark.parametrize("M", [1, 5, 16])
+@pytest.mark.parametrize("rotated", [False, True])
+def test_norm_and_fused_rows_to_their_end(layout, nh, nkv, d, M, rotated):
+    """Queries and cache of the launch with the norm in it against the norm and the launch without: what differs comes from a
+    normed element rounded to its neighbour."""
+    from pytorch_transformers_amd import ops
+
+    K, N = 1040, (nh + 2 * nkv) * d
+    x, w, gain, shift, bias = _draw(M, N, K, M + d)
+    g = torch.Generator().manual_seed(d)
+    inv = 10000.0 ** (-torch.arange(d // 2, device="cuda").float() * 2 / d) if rotated else None
+    pos = torch.randint(0, 190, (M,), generator=g).int().cuda()
+    seq, table = torch.arange(M).int().cuda(), torch.randperm(3 * M, generator=g).view(M, 3).int().cuda()
+    new = lambda: (torch.full((3 * M, nkv, 64, d), 7.0).bfloat16().cuda(), torch.full((3 * M, nkv, d, 64), 7.0).bfloat16().cuda())
+    k0, v0 = new()
+    q0 = ops.gemm_skinny_qkv(ops.layernorm(x, gain, shift, 1e-5), w, bias, inv, 0.9, pos, seq, table, k0, v0, nh, nkv, d, layout, True)
+    k1, v1 = new()
+    q1 = ops.gemm_normed_qkv(x, gain, shift, 1e-5, w, bias, inv, 0.9, pos, seq, table, k1, v1, nh, nkv, d, layout, True)
+    for a, b in ((q0, q1), (k0, k1), (v0, v1)):
+        assert (a.float() - b.float()).norm() <= 2.0 ** -8 * a.float().norm()
+        assert torch.equal(a == 7.0, b == 7.0) or (a.float() - b.float()).abs().max() <= 0.1
+    k2, v2 = new()
+    ops.gemm_normed_qkv(x, gain, shift, 1e-5, w, bias, inv, 0.9, pos, seq, table, k2, v2, nh, nkv, d, layout, False)
+    assert bool((k2 == 7.0).all()) and bool((v2 == 7.0).all())
+
+
+def test_sizes_it_leaves_to_others():
+    from pytorch_transformers_amd import ops
+
+    ok = lambda M, N, K: ops.gemm_normed_ok(torch.empty(M, K, dtype=torch.bfloat16, device="cuda"), torch.empty(N, K, dtype=torch.bfloat16, device="cuda"))
+    assert ok(8, 8192, 2048) and ok(16, 4096, 2048) and not ok(9, 4097, 2048) and not ok(17, 64, 64) and not ok(1, 64, 2056) and not ok(1, 64, 12) and not ok(1, 8193, 64)
