@@ -373,6 +373,7 @@ PAVODRA_KERNEL_LABELS = {
     "pta_latent_prep": "latent norm, rotation, cache write",
     "pta_head_project": "per-head products with the key / value expansions",
     "pta_attn_latent_mfma": "attention over the latent cache (+ merge of key ranges)",
+    "pta_attn_latent_prompt": "attention over the latent cache, prompts",
     "pta_attn_latent": "attention over the latent cache, 32-bit kernel",
 }
 

@@ -188,7 +188,7 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[6], a[7], a[8], 4)
     if name == "pta_layernorm_sum":
         return ((a[4] + a[7]) * float(a[17]) * a[19] * 4, 0.0)
-    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_latent_decode", "pta_attn_latent_mfma", "pta_attn_latent", "pta_attn_talk",
+    if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_latent_decode", "pta_attn_latent_mfma", "pta_attn_latent_prompt", "pta_attn_latent", "pta_attn_talk",
                 "pta_attn_talk_mfma"):
         # (a model with two kinds of attention says each kind's figures under the entry point's name)
         return (float(timing_hint.get("attn_bytes:" + name, timing_hint.get("attn_bytes", 0))),
@@ -1963,12 +1963,16 @@ def latent_decode(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, up_v:
     return out
 
 
+LATENT_PROMPT = os.environ.get("PTA_LATENT_PROMPT", "1") != "0"
+
+
 def attn_latent(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, token_seq, token_pos, rank: int,
-                scale: float, ctx=None) -> torch.Tensor:
+                scale: float, ctx=None, out_dtype=torch.float32) -> torch.Tensor:
     """Causal attention of every token over its sequence's cache rows ``[rank + rot_dim]``, whose first ``rank``
     elements are also the values: ``q_full`` ``[tokens, heads, rank + rot_dim]`` (32-bit) -> ``[tokens, heads,
     rank]`` (32-bit).  With the step's context (``ctx``) and a bfloat16 cache of a size that is built, the kernel on
-    the matrix cores runs, its keys cut into ranges when every sequence brings one token; else the 32-bit kernel."""
+    the matrix cores runs, its keys cut into ranges when every sequence brings one token; else the 32-bit kernel.  ``out_dtype``:
+    the type that the 32-bit result is rounded to."""
     _need(q_full, "q_full", torch.float32)
     M, H, D = q_full.shape
     if k_pool.dim() != 4 or tuple(k_pool.shape[1:]) != (1, 64, D) or not k_pool.is_cuda or not k_pool.is_contiguous():
@@ -1976,14 +1980,21 @@ def attn_latent(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, token_s
     _need(block_table, "block_table", torch.int32)
     _need(token_seq, "token_seq", torch.int32, (M,))
     _need(token_pos, "token_pos", torch.int32, (M,))
-    out = torch.empty((M, H, rank), dtype=torch.float32, device=q_full.device)
     if M == 0:
-        return out
+        return torch.empty((M, H, rank), dtype=out_dtype, device=q_full.device)
     if ctx is not None and attn_latent_mfma_ok(k_pool, rank):
         n = block_table.shape[0]
         _need(ctx.cu_tokens, "cu_tokens", torch.int32, (n + 1,))
         _need(ctx.seq_start, "seq_start", torch.int32, (n,))
+        if (LATENT_PROMPT and not ctx.is_decode and out_dtype in (torch.float32, torch.bfloat16)
+                and load_library().pta_attn_latent_prompt_ok(int(rank), D)):
+            out = torch.empty((M, H, rank), dtype=out_dtype, device=q_full.device)
+            _call("pta_attn_latent_prompt", _ptr(out), int(out_dtype == torch.bfloat16), _ptr(q_full), _ptr(k_pool), _ptr(block_table),
+                  block_table.shape[1], _ptr(ctx.cu_tokens), _ptr(ctx.seq_start), n, int(max(ctx.new_tokens)), M, H, int(rank),
+                  D - int(rank), ctypes.c_float(scale), _stream())
+            return out
         size, splits = latent_decode_split(n, H, ctx.max_len) if ctx.is_decode else (0, 1)
+        out = torch.empty((M, H, rank), dtype=torch.float32, device=q_full.device)
         po = pm = pl = None
         if splits > 1:
             po = torch.empty((M, H, splits, rank), dtype=torch.float32, device=q_full.device)
@@ -1992,11 +2003,12 @@ def attn_latent(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, token_s
         _call("pta_attn_latent_mfma", _ptr(out), _ptr(po), _ptr(pm), _ptr(pl), _ptr(q_full), _ptr(k_pool), _ptr(block_table),
               block_table.shape[1], _ptr(ctx.cu_tokens), _ptr(ctx.seq_start), n, int(max(ctx.new_tokens)), M, H, int(rank),
               D - int(rank), ctypes.c_float(scale), int(size), int(splits), _stream())
-        return out
+        return out.to(out_dtype)
+    out = torch.empty((M, H, rank), dtype=torch.float32, device=q_full.device)
     _call("pta_attn_latent", _ptr(out), _ptr(q_full), _ptr(k_pool), _ptr(block_table), block_table.shape[1],
           _ptr(token_seq), _ptr(token_pos), M, H, int(rank), D - int(rank), ctypes.c_float(scale),
           dtype_code(k_pool.dtype), _stream())
-    return out
+    return out.to(out_dtype)
 
 
 # ---- a 32-bit stream with a token-shifted norm at the head of a block ---------------------------------------------

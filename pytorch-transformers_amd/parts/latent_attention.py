@@ -141,9 +141,10 @@ class LatentAttentionMixer(Part):
         else:
             ops.head_project(queries, self.dim + self.rot_dim, self.k_side, H, self.dim, self.rank,
                              out=q_full.view(M, H * D), out_head=D)
-        lat = ops.attn_latent(q_full, k_pool, rows[-2], ctx.token_seq, ctx.token_pos, self.rank, self.scale, ctx=ctx)
+        lat = ops.attn_latent(q_full, k_pool, rows[-2], ctx.token_seq, ctx.token_pos, self.rank, self.scale, ctx=ctx,
+                              out_dtype=dtype if library else torch.float32)
         if library:
-            return ops.head_project_library(lat.to(dtype), self.v_side).transpose(0, 1).reshape(M, H * self.value_dim)
+            return ops.head_project_library(lat, self.v_side).transpose(0, 1).reshape(M, H * self.value_dim)
         return ops.head_project(lat.view(M, H * self.rank), self.rank, self.v_side, H, self.rank, self.value_dim, out_dtype=dtype)
 
 

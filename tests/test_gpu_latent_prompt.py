@@ -1,0 +1,69 @@
+"""The latent attention of prompts with two waves a tile of 32 columns, against the 32-bit kernel on the same bfloat16 cache."""
+import types
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("heads", [1, 3, 16, 70])
+@pytest.mark.parametrize("starts,news", [([0], [2]), ([0, 0, 63, 64], [4, 64, 1, 1]), ([0, 5, 127], [65, 60, 2]), ([500, 0], [3, 131]), ([640], [33])])
+def test_prompts_on_top_of_cached_tokens(heads, starts, news):
+    """Ends of pages and of column groups, single tokens beside prompts, rows past a sequence's end that hold no numbers; the
+    result in 32-bit and rounded."""
+    from pytorch_transformers_amd import ops
+
+    rank, D, n = 512, 576, len(starts)
+    g = torch.Generator().manual_seed(heads + sum(news))
+    pages = [(s + k + 63) // 64 for s, k in zip(starts, news)]
+    pool = torch.full((sum(pages) + 1, 1, 64, D), float("nan"), dtype=torch.bfloat16)
+    table = torch.full((n, max(pages) + 1), -1, dtype=torch.int32)
+    order, at = torch.randperm(sum(pages) + 1, generator=g).tolist(), 0
+    for i, (s, k) in enumerate(zip(starts, news)):
+        for p in range(pages[i]):
+            page, at = order[at], at + 1
+            table[i, p] = page
+            rows = min(64, s + k - 64 * p)
+            pool[page, 0, :rows] = (torch.randn(rows, D, generator=g) * 0.7).to(torch.bfloat16)
+    pool, table = pool.cuda(), table.cuda()
+    cu = [0]
+    for k in news:
+        cu.append(cu[-1] + k)
+    seq = torch.tensor([i for i, k in enumerate(news) for _ in range(k)], dtype=torch.int32).cuda()
+    pos = torch.tensor([s + t for s, k in zip(starts, news) for t in range(k)], dtype=torch.int32).cuda()
+    q = (torch.randn(cu[-1], heads, D, generator=g) * 1.5).cuda()
+    ctx = types.SimpleNamespace(cu_tokens=torch.tensor(cu, dtype=torch.int32).cuda(), seq_start=torch.tensor(starts, dtype=torch.int32).cuda(),
+                                new_tokens=news, max_len=max(s + k for s, k in zip(starts, news)), is_decode=False)
+    # scores of size 0.05 sqrt(576) * 1.05 = 1.3, a few of several times that: no column is one key alone
+    want = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05)
+    got = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05, ctx=ctx)
+    assert got.dtype == torch.float32 and torch.isfinite(got).all()
+    # queries and weights are rounded to bfloat16 (2^-9 each): a score moves by 2^-9 of its terms' size, a result by 2^-8 or so of
+    # the values it averages
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()
+    assert (got - want).abs().max() <= 0.06
+    assert torch.equal(ops.attn_latent(q, pool, table, seq, pos, rank, 0.05, ctx=ctx, out_dtype=torch.bfloat16), got.to(torch.bfloat16))
+
+
+def test_scores_that_climb(monkeypatch):
+    """Every page's scores lie far above the last one's, so that the reference of the exponentials is brought up page after page;
+    and the other way round, where it stays."""
+    from pytorch_transformers_amd import ops
+
+    rank, D, T = 512, 576, 300
+    g = torch.Generator().manual_seed(5)
+    for sign in (1.0, -1.0):
+        rows = torch.randn(5 * 64, D, generator=g) * 0.2
+        rows[:, -1] = sign * torch.arange(5 * 64) / 64.0
+        pool = rows.view(5, 1, 64, D).to(torch.bfloat16).cuda()
+        table = torch.arange(5, dtype=torch.int32).view(1, 5).cuda()
+        seq, pos = torch.zeros(T, dtype=torch.int32).cuda(), torch.arange(T, dtype=torch.int32).cuda()
+        q = torch.randn(T, 16, D, generator=g)
+        q[:, :, -1] = 320.0
+        q = q.cuda()
+        ctx = types.SimpleNamespace(cu_tokens=torch.tensor([0, T], dtype=torch.int32).cuda(), seq_start=torch.zeros(1, dtype=torch.int32).cuda(),
+                                    new_tokens=[T], max_len=T, is_decode=False)
+        want = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05)
+        got = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05, ctx=ctx)
+        assert (got - want).norm() <= 2.0 ** -6 * want.norm()
