@@ -8,16 +8,18 @@
 //   latent_values    merges a token's ranges and takes the result through the head's value expansion
 //
 // What bounds a layer here is launches and chains of dependent loads, not bytes: 16 heads, R = 512, dr = 64, 8 sequences of 64 to
-// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 29 in three (4.7, 16 and 8).
+// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 27 in three (4.7,
+// 15 and 6.8).
 #include "attn_latent_token.h"
 
 typedef __bf16 ld_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float ld_f32x4 __attribute__((ext_vector_type(4)));
+typedef short ld_i16x4 __attribute__((ext_vector_type(4)));
 
 union LdFrag {
     uint4 u;
     ld_bf16x8 v;
-    bf16_t s[8];
+    ld_i16x4 half[2];
 };
 
 // ---- queries ------------------------------------------------------------------------------------------------------------
@@ -175,10 +177,14 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
             pf[1].u = *(const uint4*)(Ps + r16 * 72 + 32 + g * 8);
 #pragma unroll
             for (int i = 0; i < TILES; ++i) {
-                const bf16_t* vr = Ks + (g * 8) * P + min((wave * TILES + i) * 16 + r16, a.R - 1);
+                // by the transposing read: sixteen lanes give the addresses of four rows of sixteen elements and get an element of
+                // the four rows each, lanes g keys 8 g .. + 3, then + 4 .. + 7 (R is whole tiles; one past it reads the last again)
+                const bf16_t* vr = Ks + (g * 8 + (r16 >> 2)) * P + min((wave * TILES + i) * 16, a.R - 16) + (r16 & 3) * 4;
                 LdFrag v[2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[0].s[e] = vr[e * P], v[1].s[e] = vr[(32 + e) * P];
+                for (int e = 0; e < 4; ++e)
+                    v[e >> 1].half[e & 1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                        (__attribute__((address_space(3))) ld_i16x4*)(vr + ((e >> 1) * 32 + (e & 1) * 4) * P));
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[i][e] *= corr;
                 acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v[0].v, pf[0].v, acc[i], 0, 0, 0);
@@ -200,8 +206,12 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
 // ---- values -------------------------------------------------------------------------------------------------------------
 // A workgroup has 32 outputs of one head for TOK tokens (fewer tokens a workgroup where there are few: what it reads is the
 // ranges' sums, and one compute unit pulls some 24 GB/s): the ranges merged into LDS, then the product with 32 rows of the
-// value expansion [H][V][R], two tiles of sixteen rows over two halves of R.
+// value expansion [H][V][R], two tiles of sixteen rows over two halves of R.  It is a chain of round trips: the expansion's rows are
+// asked for before anything else, and LV_AHEAD ranges' sums at once (2 sequences of 1,900 keys, 30 ranges, 16 heads: 14.8 -> 8.1 us
+// against four at once behind a branch each; 8 sequences of 64 to 700: 8.0 -> 6.8).
 #define LV_SPLITS 1024
+#define LV_STEPS 8   // of 32 elements, half of a latent of 512
+#define LV_AHEAD 16
 
 template <int TOK>
 __global__ __launch_bounds__(256) void latent_values_kernel(bf16_t* __restrict__ out, const float* __restrict__ po,
@@ -211,17 +221,32 @@ __global__ __launch_bounds__(256) void latent_values_kernel(bf16_t* __restrict__
     const int P = R + 8, h = blockIdx.x, v0 = blockIdx.y * 32, m0 = blockIdx.z * TOK;
     float* w_s = (float*)(lat + TOK * P);
     __shared__ ld_f32x4 part[2][64];
+    __shared__ int live[TOK];  // ranges of a token that hold sums: those before the sequence's end
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
+    // the wave's rows of the expansion are on their way while the ranges are merged
+    const int tile = wave & 1, half = wave >> 1, steps = R / 32;
+    const int c0 = half ? (steps + 1) / 2 : 0, c1 = half ? steps : (steps + 1) / 2;
+    const bf16_t* wr = up_v + ((long)h * V + min(v0 + 16 * tile + r16, V - 1)) * R + g * 8;
+    LdFrag w[LV_STEPS];
+#pragma unroll
+    for (int c = 0; c < LV_STEPS; ++c) w[c].u = *(const uint4*)(wr + 32 * min(c0 + c, steps - 1));
     // a wave a token: e^(m_s - max) / sum
     for (int t = wave; t < TOK; t += 4) {
         const long row = (long)min(m0 + t, M - 1) * H + h;
         float top = -INFINITY, sum = 0.f;
-        for (int s = lane; s < splits; s += 64) top = fmaxf(top, pm[row * splits + s]);
-        top = wave_max(top);
+        int last = 0;
         for (int s = lane; s < splits; s += 64) {
-            const float m = pm[row * splits + s], w = m == -INFINITY ? 0.f : expf(m - top);
-            w_s[t * splits + s] = w;
-            sum += w * pl[row * splits + s];
+            const float m = pm[row * splits + s];
+            top = fmaxf(top, m);
+            if (m != -INFINITY) last = s + 1;
+        }
+        top = wave_max(top);
+        last = (int)wave_max((float)last);
+        if (lane == 0) live[t] = last;
+        for (int s = lane; s < splits; s += 64) {
+            const float m = pm[row * splits + s], e = m == -INFINITY ? 0.f : expf(m - top);
+            w_s[t * splits + s] = e;
+            sum += e * pl[row * splits + s];
         }
         sum = wave_sum(sum);
         for (int s = lane; s < splits; s += 64) w_s[t * splits + s] *= 1.0f / sum;
@@ -229,33 +254,34 @@ __global__ __launch_bounds__(256) void latent_values_kernel(bf16_t* __restrict__
     __syncthreads();
     const int quads = R / 4;
     for (int i = tid; i < TOK * quads; i += 256) {
-        const int t = i / quads, el = (i - t * quads) * 4;
+        const int t = i / quads, el = (i - t * quads) * 4, n = live[t];
         const long row = (long)min(m0 + t, M - 1) * H + h;
         const float* src = po + row * splits * R + el;
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll 4
-        for (int s = 0; s < splits; ++s) {
-            const float w = w_s[t * splits + s];
-            if (w == 0.f) continue;  // (a range past the sequence's end holds no sums)
-            const float4 v = *(const float4*)(src + (long)s * R);
-            acc.x += w * v.x, acc.y += w * v.y, acc.z += w * v.z, acc.w += w * v.w;
+        for (int s0 = 0; s0 < n; s0 += LV_AHEAD) {  // so many ranges' sums on their way at once
+            float4 v[LV_AHEAD];
+#pragma unroll
+            for (int u = 0; u < LV_AHEAD; ++u) v[u] = *(const float4*)(src + (long)min(s0 + u, n - 1) * R);
+#pragma unroll
+            for (int u = 0; u < LV_AHEAD; ++u) {
+                const float e = s0 + u < n ? w_s[t * splits + s0 + u] : 0.f;
+                if (e == 0.f) continue;  // (a range whose keys weigh nothing)
+                acc.x += e * v[u].x, acc.y += e * v[u].y, acc.z += e * v[u].z, acc.w += e * v[u].w;
+            }
         }
         union { uint2 u; bf16_t b[4]; } o;
         o.b[0] = f32_to_bf16_bits(acc.x), o.b[1] = f32_to_bf16_bits(acc.y), o.b[2] = f32_to_bf16_bits(acc.z), o.b[3] = f32_to_bf16_bits(acc.w);
         *(uint2*)(lat + t * P + el) = o.u;
     }
     __syncthreads();
-    const int tile = wave & 1, half = wave >> 1, steps = R / 32;
-    const int c0 = half ? (steps + 1) / 2 : 0, c1 = half ? steps : (steps + 1) / 2;
-    const bf16_t* wr = up_v + ((long)h * V + min(v0 + 16 * tile + r16, V - 1)) * R + g * 8;
     const bf16_t* lr = lat + (r16 % TOK) * P + g * 8;
     ld_f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll 8
-    for (int c = c0; c < c1; ++c) {
-        LdFrag w, l;
-        w.u = *(const uint4*)(wr + 32 * c);
-        l.u = *(const uint4*)(lr + 32 * c);
-        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w.v, l.v, acc, 0, 0, 0);
+#pragma unroll
+    for (int c = 0; c < LV_STEPS; ++c) {
+        if (c0 + c >= c1) break;
+        LdFrag l;
+        l.u = *(const uint4*)(lr + 32 * (c0 + c));
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[c].v, l.v, acc, 0, 0, 0);
     }
     if (half) part[tile][lane] = acc;
     __syncthreads();
