@@ -15,6 +15,7 @@
 //                   sigmoid or silu.
 // Arithmetic in 32-bit, results in the compute type.
 #include "common.h"
+#include "glu.h"
 #include "pta_kernels.h"
 
 #include <algorithm>
@@ -97,15 +98,7 @@ __global__ void glu_bf16x8_kernel(bf16_t* __restrict__ out, const bf16_t* __rest
     unpack8(*reinterpret_cast<const uint4*>(gate + m * in_ld + f), g);
     unpack8(*reinterpret_cast<const uint4*>(up + m * in_ld + f), u);
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        if constexpr (KIND == PTA_GLU_SILU) {
-            g[j] = g[j] / (1.0f + __expf(-g[j])) * u[j];
-            continue;
-        }
-        // tanh(z) = 1 - 2 / (1 + e^(2z)): both ends saturate without a branch (e^(2z) to infinity or to zero)
-        const float z = 0.79788456080286535588f * (g[j] + 0.044715f * g[j] * g[j] * g[j]);
-        g[j] = g[j] * (1.0f - 1.0f / (1.0f + __expf(2.0f * z))) * u[j];
-    }
+    for (int j = 0; j < 8; ++j) g[j] = glu_value(KIND, g[j], u[j], 0.f, 0.f);
     *reinterpret_cast<uint4*>(out + i * 8) = pack8(g);
 }
 

@@ -13,6 +13,7 @@
 // activation and additions are applied and the tile is stored.  S is chosen from N and K alone, so
 // the order of summation never depends on M or on what else is in the batch.
 #include "common.h"
+#include "glu.h"
 #include "pta_kernels.h"
 #include "qkv_tail.h"
 
@@ -439,6 +440,48 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
     }
 }
 
+// The input product of a gated feed-forward, W = [gate rows, up rows], with the gate in its epilogue: y[M, F] = glu(x . Wg^T, x . Wu^T)
+// for up to 16 rows.  A workgroup's two row tiles are the same rows of the gate and of the up matrix.  As a pass of its own
+// the gate took 4.5 us behind a product of 13 (2 rows, 2 x 5,504 x 2,048).
+__global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
+                                                              const bf16_t* __restrict__ W, int M, int F, int K, int rot_stride, int kind,
+                                                              float alpha, float limit) {
+    extern __shared__ f32x4_t part[];  // [S][2][64]
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const int r = lane & 15, g = lane >> 4;
+    const int n0 = (int)((long)blockIdx.x * F / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * F / gridDim.x);
+    const int row = min(n0 + r, n1 - 1);
+    const bf16_t* wrow[2] = {W + (long)row * K, W + (long)(F + row) * K};
+    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
+    f32x4_t acc[2][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}, {f32x4_t{0.f, 0.f, 0.f, 0.f}}};
+    const int nsteps = (K + 63) >> 6;
+    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
+    Stage<1, 2, 2> s0, s1;
+    load_stage<1, 2, 2>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
+    for (int step = wave; step < nsteps; step += 4 * S) {
+        load_stage<1, 2, 2>(s1, wrow, xres, r, step + 2 * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<1, 2, 2>(s0, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        load_stage<1, 2, 2>(s0, wrow, xres, r, step + 4 * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<1, 2, 2>(s1, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) part[(wave * 2 + rt) * 64 + lane] = acc[rt][0];
+    __syncthreads();
+    const float* sums = (const float*)part;  // feature i of a tile, row m of x: lane (i / 4) * 16 + m, element i % 4
+    for (int item = threadIdx.x; item < 16 * M; item += blockDim.x) {
+        const int m = item >> 4, i = item & 15;
+        if (n0 + i >= n1) continue;
+        const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
+        float gate = sums[at], up = sums[256 + at];
+        for (int w = 1; w < S; ++w) gate += sums[w * 512 + at], up += sums[w * 512 + 256 + at];
+        y[(long)m * F + n0 + i] = f32_to_bf16_bits(glu_value(kind, round_to_bf16(gate), round_to_bf16(up), alpha, limit));
+    }
+}
+
 // The product of few rows together with the LayerNorm in front of it, y = act(LN(x) . W^T + bias), rows of up to 2,048
 // elements.  As launches of their own a norm of a few rows takes 4.7 us, nearly all of it what any launch costs; here every
 // workgroup norms the rows for itself while its rows of W are on their way: rows of x are asked for first, then the norm's
@@ -854,6 +897,22 @@ extern "C" int pta_gemm_normed_qkv_bf16(void* q_out, const void* x, const float*
     if (make_tail_problem("gemm_normed_qkv_bf16", q_out, x, W, bias, rotation, token_pos, token_seq, block_table, bt_stride, k_pool,
                           v_pool, nh, nkv, d, layout, write_cache, M, K, p, tail)) return 1;
     return launch_normed<true>("gemm_normed_qkv_bf16", p, ln_w, ln_b, eps, M, K, tail, (hipStream_t)stream);
+}
+
+extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, int M, int F, int K, int kind, float alpha, float limit,
+                                        void* stream) {
+    if (check_skinny("gemm_skinny_glu_bf16", y, x, W, M, F, K, PTA_ACT_NONE)) return 1;
+    PTA_REQUIRE(M <= 16, "gemm_skinny_glu_bf16: at most 16 rows, got %d", M);
+    PTA_REQUIRE(F < (1 << 30), "gemm_skinny_glu_bf16: %d features are too many", F);
+    PTA_REQUIRE(kind == PTA_GLU_SILU || kind == PTA_GLU_CLAMPED || kind == PTA_GLU_GELU_TANH, "gemm_skinny_glu_bf16: kind %d is not built", kind);
+    const int S = pick_split(2 * F), units = pta_compute_units();
+    int blocks = (F + 15) / 16;
+    if (blocks > units) blocks = (blocks + units - 1) / units * units;  // a whole number of workgroups per unit (launch_cfg)
+    static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
+    const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
+    hipLaunchKernelGGL(gemm_skinny_glu_kernel, dim3(blocks), dim3(S * 64), (size_t)S * 2 * 64 * sizeof(f32x4_t), (hipStream_t)stream,
+                       (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)W, M, F, K, rot_stride, kind, alpha, limit);
+    return pta_check_launch("gemm_skinny_glu_bf16");
 }
 
 // Two products of one launch: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2), both [M, *] in

@@ -175,6 +175,9 @@ int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const fl
                              const int* token_pos, const int* token_seq, const int* block_table, int bt_stride, void* k_pool,
                              void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K, void* stream);
 
+// y [M, F] = glu(x . Wg^T, x . Wu^T), W = [Wg, Wu] [2 F, K], for up to 16 rows; kinds as pta_glu's
+int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, int M, int F, int K, int kind, float alpha, float limit, void* stream);
+
 // the product of up to 16 rows of up to 2,048 elements with the LayerNorm in front of it, y = act(LN(x) . W^T + bias), and the
 // fused query_key_value product likewise; _ok says whether the launch takes the sizes
 int pta_gemm_normed_ok(int M, int N, int K);

@@ -180,6 +180,8 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[18], (a[13] + 2 * a[14]) * a[15], a[5])
     if name == "pta_gemm_tile_bf16":
         return gemm(a[8], a[9], a[10])
+    if name == "pta_gemm_skinny_glu_bf16":
+        return gemm(a[3], 2 * a[4], a[5])
     if name == "pta_gemm_normed_bf16":
         return gemm(a[7], a[8], a[9])
     if name == "pta_gemm_normed_qkv_bf16":
@@ -2139,6 +2141,25 @@ def glu(gate: torch.Tensor, up: torch.Tensor, kind: str = "silu", alpha: float =
     if M:
         _call("pta_glu", _ptr(out), _ptr(gate), _ptr(up), ctypes.c_long(ld), M, F, GLU_CODES[kind], ctypes.c_float(alpha),
               ctypes.c_float(limit), dtype_code(gate.dtype), _stream())
+    return out
+
+
+def gemm_skinny_glu_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the product of few rows forms the gate of a feed-forward itself: ``w`` the gate's rows, then as many of the other."""
+    return gemm_skinny_ok(x, w) and w.shape[0] % 2 == 0 and w.shape[0] > 0
+
+
+def gemm_skinny_glu(x: torch.Tensor, w: torch.Tensor, kind: str = "silu", alpha: float = 1.0, limit: float = 0.0) -> torch.Tensor:
+    """``glu`` of the two halves of ``x @ w.T`` (each rounded to bfloat16), at most 16 rows, in one launch."""
+    _need(x, "x", torch.bfloat16)
+    _need(w, "w", torch.bfloat16)
+    M, K = x.shape
+    if w.shape[1] != K or w.shape[0] % 2:
+        raise KernelError(f"x is [{M}, {K}] but w is {tuple(w.shape)}; w must be [2 F, {K}]")
+    F = w.shape[0] // 2
+    out = torch.empty((M, F), dtype=torch.bfloat16, device=x.device)
+    _call("pta_gemm_skinny_glu_bf16", _ptr(out), _ptr(x), _ptr(w), M, F, K, GLU_CODES[kind], ctypes.c_float(alpha), ctypes.c_float(limit),
+          _stream())
     return out
 
 

@@ -72,3 +72,23 @@ def test_squared_relu_in_the_epilogue(M, N, K):
     want = (z.double() * z.double() + add.double()).float()  # one rounding at the end, whether or not the two are one instruction
     got = ops.gemm_skinny_bf16(x, w, bias, "relu2", add)
     assert bool(((got.float() - want).abs() <= want.abs() * 2.0 ** -8 + z * z * 2.0 ** -23).all())
+
+
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh", "clamped"])
+@pytest.mark.parametrize("M,F,K", [(1, 1, 8), (16, 15, 72), (2, 5504, 2048), (9, 1040, 1040), (16, 4099, 264)])
+def test_the_gate_in_the_epilogue(kind, M, F, K):
+    """The gate of a feed-forward in the launch of its input product against the product and the gate's own launch.  Sums may
+    be taken in another order (a half is then rounded to its neighbour), nothing else differs."""
+    from pytorch_transformers_amd import ops
+
+    g = torch.Generator().manual_seed(M + F)
+    x, w = torch.randn(M, K, generator=g).bfloat16().cuda(), (0.05 * torch.randn(2 * F, K, generator=g)).bfloat16().cuda()
+    assert ops.gemm_skinny_glu_ok(x, w)
+    got = ops.gemm_skinny_glu(x, w, kind, 1.7, 3.0)
+    both = ops.gemm_skinny_bf16(x, w)
+    want = ops.glu(both[:, :F], both[:, F:], kind, 1.7, 3.0).float()
+    gate, up = both[:, :F].float(), both[:, F:].float()
+    # a neighbour of either half is 2^-7 of it away at most; the gates' slopes stay under 1.2 (1.3 at alpha 1.7)
+    tol = 2.0 ** -7 * (1.3 * gate.abs() * (up.abs() + 1) + gate.abs() * up.abs() + want.abs()) + 1e-6
+    assert bool(((got.float() - want).abs() <= tol).all())
+    assert (got.float() != want).float().mean() <= 0.05
