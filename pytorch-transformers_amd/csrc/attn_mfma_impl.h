@@ -81,11 +81,10 @@ struct KvBlock {
 // Keys and values of the 32-key block at kb, straight into matrix-operand registers.  Nothing here
 // depends on the loaded data, so the loads of the next block stay in flight while this one is used.
 template <int DT>
-__device__ __forceinline__ void load_block(KvBlock<DT>& b, int kb, const int* __restrict__ bt,
+__device__ __forceinline__ void load_block(KvBlock<DT>& b, int kb, long page,
                                            const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
                                            int nkv, int kvh, int c, int gq) {
     constexpr int D = DT * 16, DS = (DT + 1) / 2, CHUNKS = D / 8;
-    const long page = bt[kb >> 6];
     const int in_page = kb & 63;
     const bf16_t* kpage = k_pool + (page * nkv + kvh) * (long)(PTA_PAGE * D);
     const bf16_t* vpage = v_pool + (page * nkv + kvh) * (long)(PTA_PAGE * D);
@@ -134,7 +133,7 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
     static_assert(KS == 1 || W == 1, "waves either share key blocks or divide them");
     const int lane = threadIdx.x & 63, c = lane & 15, gq = lane >> 4;
     const int wave = KS > 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // which columns of the workgroup
-    const int kw = KS > 1 ? threadIdx.x >> 6 : 0;     // which blocks of the keys
+    const int kw = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;     // which blocks of the keys
     // Ranges of keys are handed out range-major: the first ranges of every sequence, which all of them have whole,
     // start first, and the last ones, which are short or empty for most sequences, fill the launch's end.  (Sequence-
     // major, 32 sequences of 16,405 keys in ranges of 1,024 left two whole ranges to start when the first ones ended:
@@ -142,7 +141,17 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
     const int n_seqs_z = gridDim.z / n_splits;
     const int seq = blockIdx.z % n_seqs_z, split = blockIdx.z / n_seqs_z;
     const int kvh = blockIdx.y, g = nh / nkv;
+    // The pages of a lone wave's first two blocks are looked up beside the sequence's length, not behind it: one round trip less in
+    // a decode step's chain of them (an entry past the sequence's pages is read but not used).
+    const int* bt = block_table + (long)seq * bt_stride;
+    const int first_key = (n_splits > 1 ? split * split_size : 0) + 32 * kw;
+    int first_page = 0, next_page = 0;
+    if constexpr (W == 1 && !WIN) {
+        first_page = bt[min(first_key >> 6, bt_stride - 1)];
+        next_page = bt[min((first_key + 32 * KS) >> 6, bt_stride - 1)];
+    }
     const int t0 = cu_tokens[seq], n_new = cu_tokens[seq + 1] - t0, start = seq_start[seq];
+    if constexpr (W == 1 && !WIN) asm volatile("" : "+s"(first_page), "+s"(next_page));
     const int ncols = n_new * g, n_groups = (ncols + 16 * CT * W - 1) / (16 * CT * W);
     // Column groups are handed out last first: late tokens see the most keys, and the longest work should
     // start first so that the launch ends evenly.  A paired launch has half the workgroups, and each takes a
@@ -212,8 +221,6 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
     }
     AFrag ones;
     ones.u = make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u);
-
-    const int* bt = block_table + (long)seq * bt_stride;
 
     // AL says at compile time whether there is ALiBi (0: none, 1: there is; 2: whatever the launch brings), so
     // that the kernels for prompts, which are bound by their instruction stream, branch on nothing in it.
@@ -359,14 +366,21 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
         const int k_first = k_begin + 32 * kw;
         const int n_mine = k_first < k_end ? (k_end - k_first + STEP - 1) / STEP : 0;  // blocks of this wave
         auto blk = [&](int j) { return j < n_mine ? min(k_first + STEP * j, kb_last) : kb_last; };
+        auto page_of = [&](int kb) {
+            if constexpr (!WIN) {
+                if (kb >> 6 == first_key >> 6) return (long)first_page;
+                if (kb >> 6 == (first_key + STEP) >> 6) return (long)next_page;
+            }
+            return (long)bt[kb >> 6];
+        };
         if (n_mine > 0) {
 #pragma unroll
-            for (int i = 0; i < NB - 1; ++i) load_block<DT>(b[i], blk(i), bt, k_pool, v_pool, nkv, kvh, c, gq);
+            for (int i = 0; i < NB - 1; ++i) load_block<DT>(b[i], blk(i), page_of(blk(i)), k_pool, v_pool, nkv, kvh, c, gq);
         }
         for (int j = 0; j < n_mine; j += NB) {
 #pragma unroll
             for (int i = 0; i < NB; ++i) {
-                load_block<DT>(b[(i + NB - 1) % NB], blk(j + i + NB - 1), bt, k_pool, v_pool, nkv, kvh, c, gq);
+                load_block<DT>(b[(i + NB - 1) % NB], blk(j + i + NB - 1), page_of(blk(j + i + NB - 1)), k_pool, v_pool, nkv, kvh, c, gq);
                 __builtin_amdgcn_sched_barrier(0);
                 if (j + i < n_mine) use_block(b[i], blk(j + i));
                 __builtin_amdgcn_sched_barrier(0);
