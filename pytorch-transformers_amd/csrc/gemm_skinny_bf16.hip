@@ -681,7 +681,8 @@ static int launch_halves(const SkinnyProblem& p, int M, int K, int S, hipStream_
 
 template <typename OutT>
 static int launch_skinny(SkinnyProblem a, SkinnyProblem b, int M, int K, int variant, int S, hipStream_t s) {
-    // variant: row tiles per wave and steps per stage (6: one tile, its rows spread over all units); 0: chosen here
+    // variant: row tiles per wave and steps per stage (6: one tile, its rows spread over all units; 7: eight rows at two places of
+    // K); 0: chosen here
     // Tiles of 32 rows of W that would occupy half of the compute units or fewer: a unit pulls no more than some 24 GB/s, so
     // the rows are spread over all units instead, a few rows each (the rest of a tile's lanes read a row again).  Replays over
     // cold weights, 8 rows of x, 32-row tiles -> spread: 3,072 x 2,048 9.8 -> 7.0 us (up to eight rows a unit:
