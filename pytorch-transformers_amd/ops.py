@@ -991,18 +991,27 @@ def _library_fills(M: int, N: int) -> bool:
     return M * N >= 0.97 * 65536 * units * -(-tiles // units)
 
 
-def gemm_tile_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether the hand-written kernel for many rows takes this product and is the choice for it, where the kernels for few
+def gemm_tile_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the hand-written kernel for many rows can run this product."""
+    M, K = x.shape
+    N = w.shape[0]
+    return (GEMM_TILE and M > GEMM_TILE_ROWS and _bf16_rows_ok(x, w) and N % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+            and w.is_contiguous() and (N + 256) * K < GEMM_TILE_MOST and (M + 256) * x.stride(0) < GEMM_TILE_MOST)
+
+
+def gemm_tile_rule(M: int, N: int, K: int) -> bool:
+    """Whether the hand-written kernel is the choice for a product that was not timed (``tuning.tile_pays``), where the kernels for few
     rows (up to 16, and to 128 and more unless W has at least twice as many rows as columns) are not.  Up to 256 rows such
     a tall W whose rows lie a multiple of 8 KiB apart is the library's: 32,768 x 8,192 by 64 to 192 rows 115 to 133 us against
     135 to 151, 16,384 x 4,096 equal or up to 15 % faster; 18,176 x 4,544 46 to 58 us against 38 to 53, 8,192 x 2,048 20 against 16."""
-    M, K = x.shape
-    N = w.shape[0]
     if M <= 256 and K % 4096 == 0 and N >= 2 * K:
         return False
-    return (GEMM_TILE and M > GEMM_TILE_ROWS and _bf16_rows_ok(x, w) and N % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
-            and w.is_contiguous() and (N + 256) * K < GEMM_TILE_MOST and (M + 256) * x.stride(0) < GEMM_TILE_MOST
-            and not _library_fills(M, N))
+    return not _library_fills(M, N)
+
+
+def gemm_tile_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether an untuned product of many rows runs in the hand-written kernel."""
+    return gemm_tile_takes(x, w) and gemm_tile_rule(x.shape[0], w.shape[0], x.shape[1])
 
 
 @functools.lru_cache(maxsize=None)
@@ -1042,21 +1051,34 @@ def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=N
     return y
 
 
-def mm_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
-    """act(x @ w.T + bias) + add1 + add2 of many rows: the library's product over ranges of K where that was timed faster, else
-    the hand-written kernel or, where ``gemm_tile_ok`` leaves it to it, the library's plain product."""
-    y = library_mm_ksplit(x, w, bias, act, add1, add2)
-    if y is not None:
-        return y
-    if gemm_tile_ok(x, w):
-        if ACT_CODES[act] in GEMM_TILE_ACTS:
-            return gemm_tile_bf16(x, w, bias, act, add1, add2)
-        y = gemm_tile_bf16(x, w)
-    else:
-        y = library_mm(x, w)
+def tile_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 through the hand-written kernel, what its epilogue does not apply in a pass behind it."""
+    if ACT_CODES[act] in GEMM_TILE_ACTS:
+        return gemm_tile_bf16(x, w, bias, act, add1, add2)
+    return epilogue_(gemm_tile_bf16(x, w), bias, act, add1, add2)
+
+
+def library_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 through the library's product and a pass behind it."""
+    y = library_mm(x, w)
     if bias is not None or act is not None or add1 is not None or add2 is not None:
         epilogue_(y, bias, act, add1, add2)
     return y
+
+
+def whole_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 over all of K at once: the hand-written kernel or the library's product, as timed
+    (``tuning.tile_pays``) or, where nothing was, as ``gemm_tile_rule`` has it."""
+    if gemm_tile_takes(x, w) and tuning.tile_pays(x, w, bias, act, add1, add2):
+        return tile_rows(x, w, bias, act, add1, add2)
+    return library_rows(x, w, bias, act, add1, add2)
+
+
+def mm_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
+    """act(x @ w.T + bias) + add1 + add2 of many rows: the library's product over ranges of K where that was timed faster, else
+    ``whole_rows``."""
+    y = library_mm_ksplit(x, w, bias, act, add1, add2)
+    return whole_rows(x, w, bias, act, add1, add2) if y is None else y
 
 
 # ---- the vendor library's product with K cut into a batch ------------------------------------------------

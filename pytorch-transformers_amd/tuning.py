@@ -31,7 +31,7 @@ class TuningTable:
     nor overwrite each other's choices.  The ranges of K of pair launches are also kept inside the kernel library,
     by shape; ``activate`` takes the old table's out of it and puts the new one's in."""
 
-    FIELDS = ("pair_parts", "pair_stationary", "splitk_rows", "mm_plans", "mm_joined", "mm_ksplit", "decode_plans")
+    FIELDS = ("pair_parts", "pair_stationary", "splitk_rows", "mm_plans", "mm_joined", "mm_ksplit", "mm_tiles", "decode_plans")
 
     def __init__(self, data: Optional[dict] = None):
         self.pair_parts: dict = {}  # (shape of w1, shape of w2) -> (ranges, ranges, row tiles per wave) in use
@@ -44,6 +44,8 @@ class TuningTable:
         self.mm_costs: dict = {}  # (N, K, M bucket) -> microseconds of that plan, as measured piece by piece
         self.mm_joined: dict = {}  # (N1, N2, K, M bucket) -> whether one product with both matrices beats the two
         self.mm_ksplit: dict = {}  # (N, K, M bucket) -> ranges of K (1: the plain product)
+        # (N, K, M bucket, activation, bias, additions) -> whether the hand-written kernel beats the library's product
+        self.mm_tiles: dict = {}
         self.decode_plans: dict = {}  # (batch, heads, KV heads, head size, longest, mean) as counted -> a timed cut
         if data:
             self.load(data)
@@ -59,6 +61,7 @@ class TuningTable:
             "mm_plans": {key(k): list(v) for k, v in self.mm_plans.items()},
             "mm_joined": {key(k): bool(v) for k, v in self.mm_joined.items()},
             "mm_ksplit": {key(k): int(v) for k, v in self.mm_ksplit.items()},
+            "mm_tiles": {key(k): bool(v) for k, v in self.mm_tiles.items()},
             "decode_plans": {key(k): list(v) for k, v in self.decode_plans.items()},  # tiles, keys per workgroup, waves
         }
 
@@ -90,6 +93,8 @@ class TuningTable:
             self.mm_joined[flat(k)] = bool(v)
         for k, v in data.get("mm_ksplit", {}).items():
             self.mm_ksplit[flat(k)] = int(v)
+        for k, v in data.get("mm_tiles", {}).items():
+            self.mm_tiles[flat(k)] = bool(v)
         for k, v in data.get("decode_plans", {}).items():
             self.decode_plans[flat(k)] = tuple(int(p) for p in v)
 
@@ -98,7 +103,7 @@ class TuningTable:
         if self is _active:
             _release(self)
         for d in (self.pair_stationary, self.pair_parts, self.splitk_rows, self.mm_plans, self.mm_costs, self.mm_times,
-                  self.mm_joined, self.mm_ksplit, self.decode_plans):
+                  self.mm_joined, self.mm_ksplit, self.mm_tiles, self.decode_plans):
             d.clear()
 
 
@@ -554,6 +559,30 @@ def mm_plan(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor):
     _active.mm_plans[(N, K, bucket)] = plan
     _active.mm_costs[(N, K, bucket)] = cost if plan is pieces else times[M]
     return plan
+
+
+TILE_MARGIN = 0.98  # a way replaces the rule's only if it is faster by more than two runs of one way differ
+
+
+def tile_pays(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> bool:
+    """Whether ``act(x @ w.T + bias) + add1 + add2`` of many rows runs in the hand-written kernel, which can take it, or through the
+    library's product in the pieces of ``mm_plan``.  When timing is on, both are timed to their end once per shape and kind
+    of epilogue (the hand-written kernel's own, a pass behind the library's); without an entry pieces that were timed for the
+    shape hold (a table from before there was this choice), and else the rule (``ops.gemm_tile_rule``)."""
+    M, (N, K) = x.shape[0], w.shape
+    bucket = (M + 63) // 64
+    key = (N, K, bucket, ops.ACT_CODES[act], int(bias is not None), (add1 is not None) + (add2 is not None))
+    pays = _active.mm_tiles.get(key)
+    if pays is not None:
+        return pays
+    rule = ops.gemm_tile_rule(M, N, K)
+    if not may_time():
+        return rule and not (MM_CHUNKS and (N, K, bucket) in _active.mm_plans)
+    rest = (bias, act, add1, add2)
+    tile, library = time_ways_cold((lambda: ops.tile_rows(x, w, *rest), lambda: ops.library_rows(x, w, *rest)), x.device)
+    pays = not library < TILE_MARGIN * tile if rule else tile < TILE_MARGIN * library
+    _active.mm_tiles[key] = pays
+    return pays
 
 
 def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int) -> bool:
