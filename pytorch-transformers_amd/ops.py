@@ -1081,6 +1081,17 @@ def mm_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, ad
     return whole_rows(x, w, bias, act, add1, add2) if y is None else y
 
 
+def joined_rows(x: torch.Tensor, joined: torch.Tensor, n_first: int, bias1=None, act1=None, bias2=None, act2=None):
+    """The products of many rows with the first ``n_first`` rows of ``joined`` and with the rest as one product: blocks of columns
+    of its result, bias and activation a pass over each block that has any."""
+    y = mm_rows(x, joined)
+    y1, y2 = y[:, :n_first], y[:, n_first:]
+    for yi, bias, act in ((y1, bias1, act1), (y2, bias2, act2)):
+        if bias is not None or act is not None:
+            epilogue_(yi, bias, act)
+    return y1, y2
+
+
 # ---- the vendor library's product with K cut into a batch ------------------------------------------------
 # Where K is long against N (the feed-forward's second matrix) and the rows are a few hundred, the library's
 # kernel choice has too few tiles of the result to fill the chip: with K = 18,176 and N = 4,544, 512 rows take 225

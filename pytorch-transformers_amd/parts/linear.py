@@ -88,7 +88,7 @@ class Linear(Part):
     @staticmethod
     def join(first: "Linear", second: "Linear") -> bool:
         """Lay the two weight matrices out as one, ``first``'s rows then ``second``'s, if they are bfloat16 with
-        one K: products of many rows with the same input can then run as one library product (``pair``).  The
+        one K: products of many rows with the same input can then run as one product (``pair``).  The
         matrices themselves become views of the joined one, so nothing is held twice."""
         if first.joined is not None and first.joined[1] is second:
             return True
@@ -170,15 +170,10 @@ class Linear(Part):
         if x1.shape == x2.shape and ops.gemm_skinny_ok(x1, first.weight) and ops.gemm_skinny_ok(x2, second.weight):
             return ops.gemm_skinny_pair_bf16(*args)
         if (x1 is x2 and x1.shape[0] > ops.SPLITK_MAX_ROWS and first.joined is not None and first.joined[1] is second
-                and ops.joined_mm_pays(x1, first.joined[0], first.out_features)):
-            # many rows, one input, the matrices side by side in memory: one library product where it was measured
-            # faster than two; the results are blocks of columns of its output, each with its own epilogue
-            y = ops.mm_rows(x1, first.joined[0])
-            y1, y2 = y[:, :first.out_features], y[:, first.out_features:]
-            for yi, bias, act in ((y1, b1, kw1.get("act")), (y2, b2, kw2.get("act"))):
-                if bias is not None or act is not None:
-                    ops.epilogue_(yi, bias, act)
-            return y1, y2
+                and ops.joined_mm_pays(x1, first.joined[0], first.out_features, b1, kw1.get("act"), b2, kw2.get("act"))):
+            # many rows, one input, the matrices side by side in memory: one product where it was measured faster than two;
+            # the results are blocks of columns of its output
+            return ops.joined_rows(x1, first.joined[0], first.out_features, b1, kw1.get("act"), b2, kw2.get("act"))
         # 17 rows and more: the pair launch where it beats the products on their own (``ops.pair_launch_pays``)
         if ops.pair_launch_pays(x1.shape[0], first.weight, second.weight) and \
                 ops.gemm_splitk_pair_ok(x1, first.weight, x2, second.weight):

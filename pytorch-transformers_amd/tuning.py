@@ -42,7 +42,9 @@ class TuningTable:
         self.mm_times: dict = {}  # (N, K) -> {rows: microseconds}; measurements, not part of the table as data
         self.mm_plans: dict = {}  # (N, K, M bucket) -> [rows, ...]
         self.mm_costs: dict = {}  # (N, K, M bucket) -> microseconds of that plan, as measured piece by piece
-        self.mm_joined: dict = {}  # (N1, N2, K, M bucket) -> whether one product with both matrices beats the two
+        # (N1, N2, K, M bucket), then (activation, bias) of each where there is any -> whether one product with both
+        # matrices beats the two
+        self.mm_joined: dict = {}
         self.mm_ksplit: dict = {}  # (N, K, M bucket) -> ranges of K (1: the plain product)
         # (N, K, M bucket, activation, bias, additions) -> whether the hand-written kernel beats the library's product
         self.mm_tiles: dict = {}
@@ -585,20 +587,25 @@ def tile_pays(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, 
     return pays
 
 
-def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int) -> bool:
-    """Whether ``x @ joined.T`` in one product beats the products with its first ``n_first`` rows and
-    with the rest on their own.  How evenly the tiles of each fill the chip decides (and where it is the library's product,
-    its kernel choice), so both ways are timed once per shape when timing is on; without an entry the two stay apart."""
+def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int, bias1=None, act1=None, bias2=None, act2=None) -> bool:
+    """Whether the products with the first ``n_first`` rows of ``joined`` and with the rest, each with its bias and
+    activation, are faster as one product (``ops.joined_rows``: bias and activation are passes behind it) than on their own
+    (``ops.mm_rows``).  How evenly the tiles of each fill the chip decides (and where it is the library's product,
+    its kernel choice), so both ways are timed to their end once per shape when timing is on; without an entry the two
+    stay apart."""
     M, (N, K) = x.shape[0], joined.shape
     if not MM_JOIN or not MM_CHUNKS or M < 512:
         return False
     bucket = (M + 63) // 64
-    key = (n_first, N - n_first, K, bucket)
+    key = bare = (n_first, N - n_first, K, bucket)
+    if not (bias1 is None and act1 is None and bias2 is None and act2 is None):
+        key += (ops.ACT_CODES[act1], int(bias1 is not None), ops.ACT_CODES[act2], int(bias2 is not None))
     if key not in _active.mm_joined:
         if not may_time():
-            return False
+            return _active.mm_joined.get(bare, False)  # (a table from before the epilogues counted says it by the shape alone)
         first, rest = joined[:n_first], joined[n_first:]
-        ways = (lambda: ops.mm_rows(x, joined), lambda: (ops.mm_rows(x, first), ops.mm_rows(x, rest)))
+        ways = (lambda: ops.joined_rows(x, joined, n_first, bias1, act1, bias2, act2),
+                lambda: (ops.mm_rows(x, first, bias1, act1), ops.mm_rows(x, rest, bias2, act2)))
         best = [float("inf"), float("inf")]
         for run in ways:  # plans are made and the library set up before anything is timed
             run()

@@ -82,3 +82,45 @@ def test_both_ways_are_timed_to_their_end(ways, monkeypatch, act, with_bias, add
         seen.clear()
         ops.mm_rows(x, w, bias, act, *extra)
         assert seen == (["tile"] if pick == 0 else [300])
+
+
+@pytest.mark.parametrize("act,with_bias", [("gelu", False), (None, True), (None, False)])
+def test_joined_matrices_are_timed_with_what_follows_them(ways, monkeypatch, act, with_bias):
+    """Two matrices of one input, in one product or each in its own: on either side bias and activation are part of what is
+    timed, and the answer counts for that epilogue; a table that knows the shape alone still holds."""
+    from pytorch_transformers_amd.parts import Linear
+
+    ops, tuning, _ = ways
+    M, N1, N2, K = 600, 72, 136, 200
+    g = torch.Generator().manual_seed(2)
+    first, second = Linear("a", K, N1, False), Linear("b", K, N2, False)
+    first.weight, second.weight = ((0.05 * torch.randn(n, K, generator=g)).bfloat16().cuda() for n in (N1, N2))
+    first.bias = second.bias = first.joined = second.joined = None
+    if with_bias:
+        second.bias = torch.randn(N2, generator=g).cuda()
+    assert Linear.join(first, second)
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    work = []  # (rows of the matrix, whether its epilogue came with it), and the passes
+    mm_rows, epilogue = ops.mm_rows, ops.epilogue_
+    monkeypatch.setattr(ops, "mm_rows", lambda x, w, b=None, a=None, *r: (work.append((w.shape[0], a is not None or b is not None)), mm_rows(x, w, b, a, *r))[1])
+    monkeypatch.setattr(ops, "epilogue_", lambda y, *a: (work.append((y.shape[1], "pass")), epilogue(y, *a))[1])
+    monkeypatch.setattr(tuning, "tile_pays", lambda *a: True)  # (the products' own choice is another test's)
+    with ops.live_tuning():
+        both = Linear.pair(first, x, {}, second, x, {"act": act})
+    ep = act is not None or with_bias
+    joined, apart = [(N1 + N2, False)] + [(N2, "pass")] * ep, [(N1, False), (N2, ep)]
+    assert work[:5 * len(joined + apart)] == (joined + apart) * 5  # one run each before the timing, four in it
+    key = (N1, N2, K, 10) + ((0, 0, ops.ACT_CODES[act], int(with_bias)) if ep else ())
+    pays = tuning.active().mm_joined.get(key)
+    assert list(tuning.active().mm_joined) == [key] and (both is not None) == pays
+    # a loaded table: by the whole key, or by the shape alone as older tables have it
+    for k in (key, key[:4]):
+        for pays in (True, False):
+            tuning.clear_tuning()
+            tuning.load_tuning({"mm_joined": {",".join(map(str, k)): pays}})
+            both = Linear.pair(first, x, {}, second, x, {"act": act})
+            assert (both is not None) == pays
+            if pays:
+                want = x.double() @ second.weight.double().T + (second.bias.double() if with_bias else 0.0)
+                want = torch.nn.functional.gelu(want) if act else want
+                assert float((both[1].double() - want).norm()) <= 2.0 ** -7 * float(want.norm())
