@@ -1109,26 +1109,8 @@ def _k_batch(x: torch.Tensor, w: torch.Tensor, S: int) -> torch.Tensor:
     return torch.bmm(xb, wb, out_dtype=torch.float32)
 
 
-def library_mm_ksplit(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None):
-    """``act(x @ w.T + bias) + add1 + add2`` through the library's batched product over ranges of K, where that
-    was timed faster than the product in one (once per shape, by 64 rows); else None."""
+def _ksplit_rows(x: torch.Tensor, w: torch.Tensor, S: int, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
     M, (N, K) = x.shape[0], w.shape
-    if (not MM_KSPLIT or K < 2 * N or not (tuning.SPLITK_MAX_ROWS < M <= MM_KSPLIT_MAX_ROWS) or K % 32 or x.stride(1) != 1
-            or not w.is_contiguous()):
-        return None
-    key = (N, K, (M + 63) // 64)
-    S = tuning.active().mm_ksplit.get(key)
-    if S is None:
-        if not tuning.may_time():
-            return None
-        plain = gemm_tile_bf16 if gemm_tile_ok(x, w) else library_mm
-        ways = [(1, lambda: plain(x, w))] + [(s, (lambda s=s: _k_batch(x, w, s))) for s in (2, 4) if K % (s * 8) == 0]
-        best = tuning.time_ways_cold([run for _, run in ways], x.device)
-        pick = min(range(len(ways)), key=lambda i: best[i])
-        S = ways[pick][0] if best[pick] < 0.9 * best[0] else 1
-        tuning.active().mm_ksplit[key] = S
-    if S == 1:
-        return None
     with timed("library_mm", float(w.numel()) * 2, 2.0 * M * N * K):
         part = _k_batch(x, w, S)
     if bias is not None:
@@ -1140,6 +1122,27 @@ def library_mm_ksplit(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add
     _call("pta_gemm_reduce_parts", _ptr(y), _ptr(part), _ptr(bias), _ptr(add1), _ptr(add2), M, N, S, ACT_CODES[act], 0,
           _stream())
     return y
+
+
+def library_mm_ksplit(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None):
+    """``act(x @ w.T + bias) + add1 + add2`` through the library's batched product over ranges of K, where that
+    was timed faster than the product in one (once per shape, by 64 rows, both to their end); else None."""
+    M, (N, K) = x.shape[0], w.shape
+    if (not MM_KSPLIT or K < 2 * N or not (tuning.SPLITK_MAX_ROWS < M <= MM_KSPLIT_MAX_ROWS) or K % 32 or x.stride(1) != 1
+            or not w.is_contiguous()):
+        return None
+    key = (N, K, (M + 63) // 64)
+    S = tuning.active().mm_ksplit.get(key)
+    if S is None:
+        if not tuning.may_time():
+            return None
+        rest = (bias, act, add1, add2)
+        ways = [(1, lambda: whole_rows(x, w, *rest))] + [(s, (lambda s=s: _ksplit_rows(x, w, s, *rest))) for s in (2, 4) if K % (s * 8) == 0]
+        best = tuning.time_ways_cold([run for _, run in ways], x.device)
+        pick = min(range(len(ways)), key=lambda i: best[i])
+        S = ways[pick][0] if best[pick] < 0.9 * best[0] else 1
+        tuning.active().mm_ksplit[key] = S
+    return None if S == 1 else _ksplit_rows(x, w, S, bias, act, add1, add2)
 
 
 def gemm_skinny_pair_bf16(x1: torch.Tensor, w1: torch.Tensor, x2: torch.Tensor, w2: torch.Tensor, bias1=None, act1=None,

@@ -124,3 +124,29 @@ def test_joined_matrices_are_timed_with_what_follows_them(ways, monkeypatch, act
                 want = x.double() @ second.weight.double().T + (second.bias.double() if with_bias else 0.0)
                 want = torch.nn.functional.gelu(want) if act else want
                 assert float((both[1].double() - want).norm()) <= 2.0 ** -7 * float(want.norm())
+
+
+def test_ranges_of_k_are_timed_to_their_end(ways, monkeypatch):
+    """The product over ranges of K and the one in one, each with its bias, activation and additions; and the one in one is
+    whichever ``whole_rows`` is."""
+    ops, tuning, _ = ways
+    if not ops.MM_KSPLIT:
+        pytest.skip("switched off by PTA_MM_KSPLIT=0")
+    M, N, K = 300, 136, 640
+    x, w = _draw(M, N, K)
+    g = torch.Generator().manual_seed(3)
+    bias, add = torch.randn(N, generator=g).cuda(), torch.randn(M, N, generator=g).bfloat16().cuda()
+    want = torch.nn.functional.gelu(x.double() @ w.double().T + bias.double()) + add.double()
+    monkeypatch.setattr(tuning, "tile_pays", lambda *a: True)
+    for pick in range(3):
+        tuning.clear_tuning()
+
+        def times(runs, device):
+            got = [run() for run in runs]
+            assert len(got) == 3 and all(float((y.double() - want).norm()) <= 2.0 ** -7 * float(want.norm()) for y in got)
+            return [1.0 - 0.5 * (i == pick) for i in range(3)]
+
+        monkeypatch.setattr(tuning, "time_ways_cold", times)
+        with ops.live_tuning():
+            assert (ops.library_mm_ksplit(x, w, bias, "gelu", add) is None) == (pick == 0)
+        assert tuning.active().mm_ksplit == {(N, K, 5): (1, 2, 4)[pick]}
