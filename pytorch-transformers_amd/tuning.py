@@ -305,12 +305,17 @@ def several_waves_cut(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int,
     10.9, 15.8 -> 14.2, 32 (416 workgroups) 13.4 -> 13.7, 16.1 -> 17.2, 22.5 -> 20.5; 71 on 1 of 64, 8 sequences 7.9 -> 6.2,
     8.5 -> 7.9, 9.1 -> 9.1; 128 on 8 of 64, 32 sequences 11.1 -> 7.7, 12.5 -> 9.3, 15.2 -> 13.2, 64 (512 workgroups) 10.1 -> 11.4, 11.7 ->
     14.0, 16.6 -> 19.5.  Heads of 128 carry twice the sums through LDS: 32 on 8, 16 sequences 10.0 -> 9.8, 11.4 -> 12.1, 14.8 ->
-    16.2, 32 sequences 14.6 -> 12.9, 16.2 -> 15.3, 21.9 -> 20.6."""
-    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
-        return None
+    16.2, 32 sequences 14.6 -> 12.9, 16.2 -> 15.3, 21.9 -> 20.6.  Shared keys (``_shared_keys_rule``) -> this where both
+    apply: 71 on 1 of 64, 33 sequences 7.9 -> 6.6, 11.8 -> 7.4, 12.3 -> 8.4, 48 sequences 7.9 -> 7.1, 12.4 -> 8.1, 12.8 -> 9.4, 64
+    (320 workgroups) 8.0 -> 9.9, 13.1 -> 11.6, 13.5 -> 13.9; 64 on 1 of 128, 33 sequences 10.1 -> 9.4, 14.5 -> 11.0, 15.0 ->
+    13.3, 64 sequences 10.2 -> 10.7, 16.0 -> 13.0, 16.6 -> 15.8.  One answer for 33 to 64 sequences (``decode_key``): it wins
+    everywhere but at the most sequences of one range of 256 keys."""
     key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
-    n, _, _, _, bound, mean = key
-    if bound > 1024 or mean > 512 or key in _active.decode_plans:
+    return None if key in _active.decode_plans else _several_waves_rule(*key)
+
+
+def _several_waves_rule(n: int, n_heads: int, n_kv_heads: int, head_dim: int, bound: int, mean: int):
+    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES or bound > 1024 or mean > 512:
         return None
     groups = n * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)  # workgroups of the launch
     if groups > 320 or (head_dim > 80 and groups < 192) or not ops.load_library().pta_attn_decode_waves_ok(head_dim, 1, 4):
@@ -352,7 +357,8 @@ def take_decode_keys() -> list:
 
 
 def decode_plan_candidates(key) -> list:
-    """Cuts of the decode launch that ``key`` counts, the rule's first: the one-wave rule's neighbours,
+    """Cuts of the decode launch that ``key`` counts, first the one that runs where none is fixed
+    (``several_waves_cut``'s, else ``decode_plan``'s): the rules', the one-wave rule's neighbours,
     workgroups of four and eight waves over the whole context and over ranges of 512 and 1,024 keys, and, where
     they are built, workgroups that share their keys over ranges of 256 to 1,024 keys and the whole context.  A workgroup of several waves needs no second launch when it walks the whole context, but all its keys
     pass through one compute unit; which wins depends on how many sequences and KV heads there are to fill the
@@ -364,8 +370,8 @@ def decode_plan_candidates(key) -> list:
     groups = (nh // nkv + 15) // 16
     most = min(groups, int(lib.pta_attn_decode_max_tiles(d)))
     rule = _decode_plan(n, nh, nkv, d, bound, mean, most) + (1,)
-    shared = _shared_keys_rule(n, nh, nkv, d, bound, mean)
-    cuts = [rule] if shared is None else [shared, rule]
+    # what runs where nothing was timed comes first: the caller measures the others against it
+    cuts = [c for c in (_several_waves_rule(*key), _shared_keys_rule(*key), rule) if c is not None]
     want = [(rule[0], rule[1] * 2, 1), (rule[0], rule[1] // 2, 1), (max(1, rule[0] - 1), rule[1], 1),
             (min(most, rule[0] + 1), rule[1], 1)]
     want += [(t, size, w) for t in (1, min(2, most)) for w in (4, 8) for size in (bound, 1024, 512)]

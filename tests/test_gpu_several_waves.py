@@ -53,3 +53,30 @@ def test_where_it_applies():
         assert tuning.several_waves_cut(5, 13, 13, 80, 325, 300) is None and ops.decode_plan(5, 13, 13, 80, 325, 300) == (1, 128, 1)
     finally:
         ops.set_decode_plan(key, None)
+
+
+@pytest.mark.parametrize("n,nh,nkv,d,max_len,mean", [(5, 13, 13, 80, 325, 300), (64, 71, 1, 64, 500, 400), (64, 71, 1, 64, 1100, 1000), (8, 32, 8, 128, 300, 300)])
+def test_what_is_measured_first_is_what_runs_untuned(monkeypatch, n, nh, nkv, d, max_len, mean):
+    """``CausalLM.tune`` keeps no entry where the first candidate was the fastest: it has to be the cut of the launch without one."""
+    width = (max_len + 63) // 64
+    pool = torch.zeros(n * width, nkv, 64, d, dtype=torch.bfloat16, device="cuda")
+    table = torch.arange(n * width, dtype=torch.int32, device="cuda").view(n, width)
+    pos = torch.full((n,), max_len - 1, dtype=torch.int32, device="cuda")
+    ctx = SimpleNamespace(is_decode=True, n_seqs=n, max_len=max_len, mean_len=mean, new_tokens=[1] * n, token_pos=pos, seq_start=pos,
+                          cu_tokens=torch.arange(n + 1, dtype=torch.int32).cuda(), token_seq=torch.arange(n, dtype=torch.int32).cuda())
+    ran, attn = [], ops.attn_mfma
+    monkeypatch.setattr(ops, "attn_mfma", lambda *a, **k: (ran.append(k), attn(*a, **k))[1])
+    launch = lambda: (ops.attention(torch.zeros(n, nh, d, dtype=torch.bfloat16, device="cuda"), pool, pool.view(-1, nkv, d, 64), table, ctx, None, 1.0),
+                      ran.pop())[1]
+    key = ops.decode_key(n, nh, nkv, d, max_len, mean)
+    ops.set_decode_plan(key, None)
+    cuts, untuned = ops.decode_plan_candidates(key), launch()
+    assert len(set(cuts)) == len(cuts) and (tuning.several_waves_cut(n, nh, nkv, d, max_len, mean) or ops.decode_plan(n, nh, nkv, d, max_len, mean)) == cuts[0]
+    try:
+        ops.set_decode_plan(key, cuts[0])
+        assert launch() == untuned
+        ops.set_decode_plan(key, cuts[1])
+        assert launch() != untuned
+    finally:
+        ops.set_decode_plan(key, None)
+    assert launch() == untuned
