@@ -984,8 +984,10 @@ GEMM_TILE_ACTS = (0, 1, 5)  # the activations (ACT_CODES) that its epilogue appl
 def _library_fills(M: int, N: int) -> bool:
     """Whether tiles of 256 by 256 fill the chip to 97 % in whole rounds: there the vendor library's kernel, which has fewer
     and larger waves, is 5 to 12 % faster (4,096 x 4,096 x 4,096 89 us against 97, 2,048 x 8,192 x 8,192 173 against 191, 25,148 x
-    16,384 x 4,096 2,282 against 2,397).  Elsewhere, over 260 products of 150 to 25,148 rows, the hand-written kernel takes 0.3 to
-    1.1 times as long (672 x 4,544 x 18,176 101 us against 205, 2,317 x 18,176 x 4,544 299 against 416), 0.9 in the middle."""
+    16,384 x 4,096 2,282 against 2,397).  Elsewhere, over 4,500 products of 17 to 6,000 rows and K
+    of 768 to 32,768, replayed over cold weights, the hand-written kernel runs with GELU in 0.91 of the time of library and pass in
+    the middle (0.59 and 1.08 at the 5th and 95th of a hundred; 672 x 4,544 x 18,176 101 us against 205, 2,317 x 18,176 x 4,544
+    299 against 416)."""
     units = compute_units()
     tiles = -(-M // 256) * -(-N // 256)
     return M * N >= 0.97 * 65536 * units * -(-tiles // units)
@@ -1002,16 +1004,17 @@ def gemm_tile_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
 def gemm_tile_rule(M: int, N: int, K: int) -> bool:
     """Whether the hand-written kernel is the choice for a product that was not timed (``tuning.tile_pays``), where the kernels for few
     rows (up to 16, and to 128 and more unless W has at least twice as many rows as columns) are not.  Up to 256 rows such
-    a tall W whose rows lie a multiple of 8 KiB apart is the library's: 32,768 x 8,192 by 64 to 192 rows 115 to 133 us against
-    135 to 151, 16,384 x 4,096 equal or up to 15 % faster; 18,176 x 4,544 46 to 58 us against 38 to 53, 8,192 x 2,048 20 against 16."""
+    a tall W whose rows lie a multiple of 8 KiB apart is the library's: over ten such shapes it takes 0.91 to 0.99 of this kernel's
+    time in the middle up to 160 rows, 1.0 at 192 and 1.1 at 256 (16,384 x 8,192 by 64 rows 55 us against 76, 24,576 x 12,288 by 192 148
+    against 193; but 8,192 x 4,096 by 192 34 against 28); 18,176 x 4,544 46 to 58 us against 38 to 53.
+    Products that nothing follows are this kernel's too, though many small ones are faster in the library's when replayed (24 x
+    11,008 x 2,048 14.8 us against 17.6, 1,024 x 1,024 x 2,048 10.8 against 20.4: its tiles are smaller, nothing is added up in a
+    second launch): launched directly, as in every prompt, a product of the library's costs the host 20 us and this one 13,
+    and small prompts are bound by that.  With those of up to 128 rows left to the library, six layers of the latent, delta-rule and
+    attention kind took 1.6 -> 1.8 ms for a prompt of 40 tokens and 0.77 -> 0.75 ms for a decode step of 20 sequences."""
     if M <= 256 and K % 4096 == 0 and N >= 2 * K:
         return False
     return not _library_fills(M, N)
-
-
-def gemm_tile_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
-    """Whether an untuned product of many rows runs in the hand-written kernel."""
-    return gemm_tile_takes(x, w) and gemm_tile_rule(x.shape[0], w.shape[0], x.shape[1])
 
 
 @functools.lru_cache(maxsize=None)

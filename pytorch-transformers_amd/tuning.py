@@ -578,6 +578,8 @@ def tile_pays(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, 
     of epilogue (the hand-written kernel's own, a pass behind the library's); without an entry pieces that were timed for the
     shape hold (a table from before there was this choice), and else the rule (``ops.gemm_tile_rule``)."""
     M, (N, K) = x.shape[0], w.shape
+    if not (_active.mm_tiles or _active.mm_plans or TUNE_LIVE):  # nothing was timed: steps launched directly are bound by the host
+        return ops.gemm_tile_rule(M, N, K)
     bucket = (M + 63) // 64
     key = (N, K, bucket, ops.ACT_CODES[act], int(bias is not None), (add1 is not None) + (add2 is not None))
     pays = _active.mm_tiles.get(key)

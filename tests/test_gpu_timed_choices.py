@@ -36,15 +36,19 @@ def test_pieces_of_a_table_are_run(ways):
     M, N, K = 1030, 136, 264
     x, w = _draw(M, N, K)
     want = x.double() @ w.double().T
-    close = lambda y: float((y.double() - want).norm()) <= 2.0 ** -7 * float(want.norm())
-    assert ops.gemm_tile_ok(x, w) and close(ops.mm_rows(x, w)) and seen == ["tile"]
+
+    def runs():
+        seen.clear()
+        y = ops.mm_rows(x, w)
+        assert float((y.double() - want).norm()) <= 2.0 ** -7 * float(want.norm())
+        return list(seen)
+
+    assert runs() == ["tile"]
     tuning.load_tuning({"mm_plans": {f"{N},{K},17": [256, 256, 518]}})
-    seen.clear()
-    assert close(ops.mm_rows(x, w)) and seen == [256, 256, 518]
+    assert runs() == [256, 256, 518]
     for pays in (True, False):
         tuning.load_tuning({"mm_tiles": {f"{N},{K},17,0,0,0": pays}})
-        seen.clear()
-        assert close(ops.mm_rows(x, w)) and seen == (["tile"] if pays else [256, 256, 518])
+        assert runs() == (["tile"] if pays else [256, 256, 518])
     assert tuning.tuning_table()["mm_tiles"] == {f"{N},{K},17,0,0,0": False}
 
 
