@@ -2188,6 +2188,22 @@ def gemm_skinny_glu_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     return gemm_skinny_ok(x, w) and w.shape[0] % 2 == 0 and w.shape[0] > 0
 
 
+def gemm_skinny_glu_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether that launch is the choice for a feed-forward.  It gives up what the plain product of few rows of W does for the
+    compute units (``launch_skinny``: eight rows a unit up to 8 units, a few rows a unit up to 16 units), which loses where K is
+    long against what the gate's own launch costs (4 us).  Product and gate -> this, 1 / 8 / 16 rows, replayed over cold weights: F
+    512 x K 1,024 5.2 -> 5.7, 6.0 -> 6.1, 7.2 -> 6.7 us, 1,024 x 2,048 6.5 -> 7.7, 7.4 -> 8.5, 9.2 -> 9.4, 1,024 x 8,192 12.2 -> 20.6,
+    13.6 -> 23.5, 17.9 -> 26.3; 1,280 x 1,024 6.4 -> 5.7, 7.2 -> 6.3, 7.8 -> 6.8, 1,536 x 2,048 8.3 -> 8.2, 9.2 -> 9.1, 10.0 -> 10.0, 1,536 x
+    2,560 9.4 -> 11.0, 10.4 -> 12.4, 11.9 -> 13.7, 2,048 x 2,048 9.3 -> 7.8, 9.9 -> 8.4, 10.3 -> 9.4, 2,048 x 8,192 21.0 -> 23.8, 20.6 -> 22.5,
+    21.9 -> 25.4; 2,304 x 5,120 20.4 -> 17.2, 20.1 -> 17.2, 22.1 -> 19.4, 2,816 x 8,192 26.2 -> 23.3, 26.6 -> 23.4, 29.3 -> 26.4, 5,504 x
+    2,048 15.2 -> 12.3, 15.9 -> 12.9, 17.7 -> 14.8, 14,336 x 4,096 50.5 -> 48.4, 52.1 -> 50.4, 56.5 -> 54.6.  Sizes of W alone decide: one
+    order of summation for up to 16 rows."""
+    if not gemm_skinny_glu_ok(x, w):
+        return False
+    F, units = w.shape[0] // 2, compute_units()
+    return F > 8 * units or (F > 4 * units and w.shape[1] <= 2048)
+
+
 def gemm_skinny_glu(x: torch.Tensor, w: torch.Tensor, kind: str = "silu", alpha: float = 1.0, limit: float = 0.0) -> torch.Tensor:
     """``glu`` of the two halves of ``x @ w.T`` (each rounded to bfloat16), at most 16 rows, in one launch."""
     _need(x, "x", torch.bfloat16)

@@ -126,7 +126,7 @@ class GatedFeedForward(Part):
         return self.inp, {}
 
     def forward(self, x: torch.Tensor, ctx: StepContext, add1=None, add2=None, projected=None):
-        if projected is None and ops.gemm_skinny_glu_ok(x, self.inp.weight):
+        if projected is None and ops.gemm_skinny_glu_pays(x, self.inp.weight):
             y = ops.gemm_skinny_glu(x, self.inp.weight, self.kind, self.alpha, self.limit)
             return self.down(y, add1=as_tensor(add1), add2=as_tensor(add2))
         both = projected if projected is not None else self.inp(x)

@@ -92,3 +92,28 @@ def test_the_gate_in_the_epilogue(kind, M, F, K):
     tol = 2.0 ** -7 * (1.3 * gate.abs() * (up.abs() + 1) + gate.abs() * up.abs() + want.abs()) + 1e-6
     assert bool(((got.float() - want).abs() <= tol).all())
     assert (got.float() != want).float().mean() <= 0.05
+
+
+@pytest.mark.parametrize("F,K,fused", [(8, 64, False), (1024, 1024, False), (1032, 1024, True), (1536, 2048, True), (1536, 2056, False), (2048, 2056, False),
+                                       (2056, 2056, True), (5504, 2048, True)])
+@pytest.mark.parametrize("M", [1, 16])
+def test_where_the_gate_rides_in_the_launch(monkeypatch, F, K, fused, M):
+    """A feed-forward of 256 compute units' sizes: small matrices keep the product that spreads its rows over all of them."""
+    from pytorch_transformers_amd import ops
+    from pytorch_transformers_amd.parts import GatedFeedForward
+
+    if ops.compute_units() != 256:
+        pytest.skip("the lines are multiples of the compute units")
+    g = torch.Generator().manual_seed(M + F)
+    ff = GatedFeedForward("f", K, F)
+    draw = {s.name: (0.05 * torch.randn(*s.shape, generator=g)).bfloat16().cuda() for s in ff.all_tensor_specs()}
+    ff.load_all(draw)
+    ff.after_load()
+    x = torch.randn(M, K, generator=g).bfloat16().cuda()
+    seen, call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: (seen.append(name), call(name, *a))[1])
+    got = ff.forward(x, None)
+    assert seen[:-1] == (["pta_gemm_skinny_glu_bf16"] if fused else ["pta_gemm_skinny_bf16", "pta_glu"])
+    both = ff.inp(x)
+    want = ff.down(ops.glu(both[:, :F], both[:, F:])).float()
+    assert (got.float() - want).norm() <= 2.0 ** -7 * want.norm()
