@@ -1,4 +1,6 @@
-// The gate of a feed-forward on a pair of its input product's results, bfloat16 arithmetic as every launch that forms it has it.
+// The gate of a feed-forward on a pair of its input product's results, for bfloat16 rows of a multiple of eight elements: the
+// gate's own launch (glu_bf16x8_kernel; the clamped kind glu_kernel, with the same expf) and the few-row product's epilogue.
+// Rows of other lengths are glu_kernel's, silu with expf and the tanh form with tanhf.
 #pragma once
 
 #include "common.h"

@@ -2197,8 +2197,9 @@ def gemm_skinny_glu_pays(x: torch.Tensor, w: torch.Tensor) -> bool:
     2,560 9.4 -> 11.0, 10.4 -> 12.4, 11.9 -> 13.7, 2,048 x 2,048 9.3 -> 7.8, 9.9 -> 8.4, 10.3 -> 9.4, 2,048 x 8,192 21.0 -> 23.8, 20.6 -> 22.5,
     21.9 -> 25.4; 2,304 x 5,120 20.4 -> 17.2, 20.1 -> 17.2, 22.1 -> 19.4, 2,816 x 8,192 26.2 -> 23.3, 26.6 -> 23.4, 29.3 -> 26.4, 5,504 x
     2,048 15.2 -> 12.3, 15.9 -> 12.9, 17.7 -> 14.8, 14,336 x 4,096 50.5 -> 48.4, 52.1 -> 50.4, 56.5 -> 54.6.  Sizes of W alone decide: one
-    order of summation for up to 16 rows."""
-    if not gemm_skinny_glu_ok(x, w):
+    order of summation for up to 16 rows.  Rows of F that are no multiple of eight elements keep the gate's own launch, whose
+    arithmetic for them is another (``glu_kernel``: ``expf``), so that it is one for any number of rows of x."""
+    if not gemm_skinny_glu_ok(x, w) or w.shape[0] % 16:
         return False
     F, units = w.shape[0] // 2, compute_units()
     return F > 8 * units or (F > 4 * units and w.shape[1] <= 2048)

@@ -117,3 +117,19 @@ def test_where_the_gate_rides_in_the_launch(monkeypatch, F, K, fused, M):
     both = ff.inp(x)
     want = ff.down(ops.glu(both[:, :F], both[:, F:])).float()
     assert (got.float() - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh", "clamped"])
+@pytest.mark.parametrize("F", [2052, 2057, 2064])
+def test_one_arithmetic_of_the_gate_for_any_rows(kind, F):
+    """A gate has the exponential of its own launch, which is another for rows that are no multiple of eight elements: sixteen
+    rows of a feed-forward are formed as seventeen are."""
+    from pytorch_transformers_amd import ops
+
+    g = torch.Generator().manual_seed(F)
+    x, w = torch.randn(17, 64, generator=g).bfloat16().cuda(), torch.randn(2 * F, 64, generator=g).bfloat16().cuda()
+    assert ops.gemm_skinny_glu_pays(x[:16], w) == (F % 8 == 0)
+    if F % 8 == 0:  # the same exponential on both sides: what differs is the product's sums
+        both = ops.gemm_skinny_bf16(x[:16], w)
+        got, want = ops.gemm_skinny_glu(x[:16], w, kind, 1.7, 3.0), ops.glu(both[:, :F], both[:, F:], kind, 1.7, 3.0)
+        assert (got != want).float().mean() <= 0.01
