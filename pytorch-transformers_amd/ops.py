@@ -1055,8 +1055,9 @@ def gemm_tile_bf16(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=N
 
 
 def tile_rows(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
-    """act(x @ w.T + bias) + add1 + add2 through the hand-written kernel, what its epilogue does not apply in a pass behind it."""
-    if ACT_CODES[act] in GEMM_TILE_ACTS:
+    """act(x @ w.T + bias) + add1 + add2 through the hand-written kernel, what its epilogue does not take (other activations,
+    additions that are not at sixteen-byte addresses) in a pass behind it."""
+    if ACT_CODES[act] in GEMM_TILE_ACTS and all(a is None or a.data_ptr() % 16 == 0 for a in (add1, add2)):
         return gemm_tile_bf16(x, w, bias, act, add1, add2)
     return epilogue_(gemm_tile_bf16(x, w), bias, act, add1, add2)
 

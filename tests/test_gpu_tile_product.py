@@ -92,3 +92,18 @@ def test_refused(what):
             ops.gemm_tile_bf16(x, w, plan=(9, 0, 1))
         else:
             ops.gemm_tile_bf16(x.float(), w)
+
+
+def test_additions_at_any_address():
+    """The kernel's epilogue adds sixteen bytes at a time; additions that lie elsewhere are added behind it, to the same bits."""
+    M, N, K = 300, 264, 72
+    x, w = _draw(M, N, K, 5)
+    bias = torch.randn(N, generator=torch.Generator().manual_seed(6)).to(DEV)
+    wide = torch.randn(2 * M * N + 1, generator=torch.Generator().manual_seed(7)).bfloat16().to(DEV)
+    at = lambda off: wide[off:off + M * N].view(M, N)
+    assert ops.gemm_tile_takes(x, w) and ops.gemm_tile_rule(M, N, K)
+    for act in (None, "gelu"):
+        for add1, add2 in ((at(1), None), (at(0), at(M * N + 1)), (at(3), at(5))):
+            got = ops.mm_rows(x, w, bias, act, add1, add2)
+            want = ops.mm_rows(x, w, bias, act, add1.clone(), None if add2 is None else add2.clone())
+            assert torch.equal(got, want)
