@@ -997,7 +997,7 @@ def gemm_tile_takes(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the hand-written kernel for many rows can run this product."""
     M, K = x.shape
     N = w.shape[0]
-    return (GEMM_TILE and M > GEMM_TILE_ROWS and _bf16_rows_ok(x, w) and N % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0
+    return (GEMM_TILE and M > GEMM_TILE_ROWS and _bf16_rows_ok(x, w) and N % 8 == 0 and x.stride(1) == 1 and x.stride(0) >= K and x.stride(0) % 8 == 0
             and w.is_contiguous() and (N + 256) * K < GEMM_TILE_MOST and (M + 256) * x.stride(0) < GEMM_TILE_MOST)
 
 

@@ -107,3 +107,14 @@ def test_additions_at_any_address():
             got = ops.mm_rows(x, w, bias, act, add1, add2)
             want = ops.mm_rows(x, w, bias, act, add1.clone(), None if add2 is None else add2.clone())
             assert torch.equal(got, want)
+
+
+def test_rows_that_share_memory_are_the_librarys():
+    """One row seen many times, and rows that overlap: the kernel takes rows that lie a row or more apart."""
+    M, N, K = 300, 264, 72
+    x, w = _draw(M, N, K, 8)
+    flat = x.reshape(-1)
+    for rows in (x[:1].expand(M, K), flat.as_strided((M, K), (8, 1))):
+        assert not ops.gemm_tile_takes(rows, w)
+        got, want = ops.mm_rows(rows, w, None, "gelu"), torch.nn.functional.gelu(rows.double() @ w.double().T)
+        assert float((got.double() - want).norm()) <= 2.0 ** -7 * float(want.norm())
