@@ -2029,7 +2029,7 @@ def attn_latent(q_full: torch.Tensor, k_pool: torch.Tensor, block_table, token_s
         _need(ctx.cu_tokens, "cu_tokens", torch.int32, (n + 1,))
         _need(ctx.seq_start, "seq_start", torch.int32, (n,))
         if (LATENT_PROMPT and not ctx.is_decode and out_dtype in (torch.float32, torch.bfloat16)
-                and load_library().pta_attn_latent_prompt_ok(int(rank), D)):
+                and q_full.data_ptr() % 16 == 0 and k_pool.data_ptr() % 16 == 0 and load_library().pta_attn_latent_prompt_ok(int(rank), D)):
             out = torch.empty((M, H, rank), dtype=out_dtype, device=q_full.device)
             _call("pta_attn_latent_prompt", _ptr(out), int(out_dtype == torch.bfloat16), _ptr(q_full), _ptr(k_pool), _ptr(block_table),
                   block_table.shape[1], _ptr(ctx.cu_tokens), _ptr(ctx.seq_start), n, int(max(ctx.new_tokens)), M, H, int(rank),

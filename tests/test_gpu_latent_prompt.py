@@ -67,3 +67,23 @@ def test_scores_that_climb(monkeypatch):
         want = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05)
         got = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05, ctx=ctx)
         assert (got - want).norm() <= 2.0 ** -6 * want.norm()
+
+
+@pytest.mark.parametrize("what", ["queries", "cache"])
+def test_other_addresses_take_the_general_kernel(what):
+    """Queries and cache pages are read sixteen bytes at a time; where they do not lie so, the kernel for all sizes runs."""
+    from pytorch_transformers_amd import ops
+
+    rank, D, T, H = 512, 576, 70, 4
+    g = torch.Generator().manual_seed(9)
+    moved = lambda t: torch.cat([t.reshape(-1)[:2], t.reshape(-1)])[2:].view(t.shape)
+    pool, q = (torch.randn(2, 1, 64, D, generator=g) * 0.7).bfloat16().cuda(), torch.randn(T, H, D, generator=g).cuda()
+    seq, pos = torch.zeros(T, dtype=torch.int32).cuda(), torch.arange(T, dtype=torch.int32).cuda()
+    table = torch.arange(2, dtype=torch.int32).view(1, 2).cuda()
+    ctx = types.SimpleNamespace(cu_tokens=torch.tensor([0, T], dtype=torch.int32).cuda(), seq_start=torch.zeros(1, dtype=torch.int32).cuda(),
+                                new_tokens=[T], max_len=T, is_decode=False)
+    want = ops.attn_latent(q, pool, table, seq, pos, rank, 0.05)
+    q2, pool2 = (moved(q), pool) if what == "queries" else (q, moved(pool))
+    assert (q2.data_ptr() | pool2.data_ptr()) % 16
+    got = ops.attn_latent(q2, pool2, table, seq, pos, rank, 0.05, ctx=ctx)
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()
