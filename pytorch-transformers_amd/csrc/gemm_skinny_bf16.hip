@@ -489,11 +489,14 @@ __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict
 // loads alone.  Normed rows lie in LDS, rounded to bfloat16 as the norm's own launch stores them, and are read from there as the
 // B operand: x passes the address path once a workgroup, not once a wave.  Statistics in 32-bit, mean first.
 // TAIL: a fused query_key_value product taken to its end as by gemm_skinny_tail_kernel.
-// Replays over cold weights, norm and product -> this: 5 rows, 3,120 x 1,040 8.2 -> 5.1 us, 4,160 x 1,040 8.8 -> 6.3, 3,072 x 2,048
-// 10.2 -> 6.7, 8,192 x 2,048 13.6 -> 11.7; 16 rows, 3,072 x 768 9.2 -> 5.4, 3,072 x 2,048 11.4 -> 8.3, 8,192 x 2,048 14.7 -> 15.4.  Eight waves
-// finish the norm sooner, four leave room for a second workgroup on the unit (8,192 x 2,048 at 5 rows: 12.4 and 11.7).
+// Sizes of W alone choose the waves and with them the order of summation: eight, which finish the norm sooner, up to a workgroup
+// a compute unit and a sixteenth, else four, which leave room for a second one (8,192 x 2,048 at 5 rows: 12.4 and 11.7 us).  A wave
+// norms up to four rows then, two at a time (of 2,048 elements one), so that the registers do not run out.
+// Replays over cold weights, norm and product (GELU) -> this, 5 / 8 / 9 / 16 rows: 3,120 x 1,040 9.0 -> 5.1, 9.1 -> 5.2, 9.1 -> 5.7, 9.2
+// -> 6.1; 4,160 x 1,040 9.4 -> 6.3, 9.7 -> 6.8, 9.8 -> 8.7, 10.0 -> 9.4; 6,144 x 1,536 12.6 -> 8.5, 12.8 -> 8.8, 12.9 -> 10.8, 13.6 -> 11.4;
+// 8,192 x 2,048 16.2 -> 11.9, 16.4 -> 12.0, 15.8 -> 15.2, 16.8 -> 16.3.
 template <int NORMED_WAVES, int CH, int RW, bool TAIL>  // CH: groups of 512 elements of a row; RW: rows of x a wave norms
-__global__ __launch_bounds__(NORMED_WAVES * 64) void gemm_normed_kernel(SkinnyProblem p, const float* __restrict__ ln_w,
+__global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_normed_kernel(SkinnyProblem p, const float* __restrict__ ln_w,
                                                                        const float* __restrict__ ln_b, float eps, int M, int K,
                                                                        QkvTail tail) {
     constexpr int STEPS = 8 * CH / NORMED_WAVES;  // steps of 64 elements of K a wave takes
@@ -514,13 +517,17 @@ __global__ __launch_bounds__(NORMED_WAVES * 64) void gemm_normed_kernel(SkinnyPr
     }
     const bf16_t* wrow = p.W + (long)w_row * K;
     const int chunks = K >> 3;
-    uint4 xv[RW][CH];
+    constexpr int RB = RW < 2 || (RW == 4 && CH == 4) ? 1 : 2;  // rows normed at a time: what leaves registers for two workgroups of four waves a unit
+    uint4 xv[RB][CH];
     float gain[CH][8], shift[CH][8];
+    auto load_rows = [&](int b) {
 #pragma unroll
-    for (int i = 0; i < RW; ++i)
+        for (int i = 0; i < RB; ++i)
 #pragma unroll
-        for (int j = 0; j < CH; ++j)
-            xv[i][j] = *reinterpret_cast<const uint4*>(p.x + (long)min(wave + i * NORMED_WAVES, M - 1) * K + min(lane + j * 64, chunks - 1) * 8);
+            for (int j = 0; j < CH; ++j)
+                xv[i][j] = *reinterpret_cast<const uint4*>(p.x + (long)min(wave + (b + i) * NORMED_WAVES, M - 1) * K + min(lane + j * 64, chunks - 1) * 8);
+    };
+    load_rows(0);
 #pragma unroll
     for (int j = 0; j < CH; ++j) {
         const int at = min(lane + j * 64, chunks - 1) * 8;
@@ -538,48 +545,55 @@ __global__ __launch_bounds__(NORMED_WAVES * 64) void gemm_normed_kernel(SkinnyPr
         for (int hf = 0; hf < 2; ++hf)
             a[u][hf].u = *reinterpret_cast<const uint4*>(wrow + min((wave + u * NORMED_WAVES) * 64 + hf * 32 + g * 8, K - 8));
     __builtin_amdgcn_sched_barrier(0);
-    float v[RW][CH][8], sum[RW], mean[RW];
 #pragma unroll
-    for (int i = 0; i < RW; ++i) {
-        sum[i] = 0.f;
+    for (int b = 0; b < RW; b += RB) {
+        float v[RB][CH][8], sum[RB], mean[RB];
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            unpack8(xv[i][j], v[i][j]);
+        for (int i = 0; i < RB; ++i) {
+            sum[i] = 0.f;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) sum[i] += lane + j * 64 < chunks ? v[i][j][e] : 0.f;
-        }
-    }
+            for (int j = 0; j < CH; ++j) {
+                unpack8(xv[i][j], v[i][j]);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-        for (int i = 0; i < RW; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
-#pragma unroll
-    for (int i = 0; i < RW; ++i) {
-        mean[i] = sum[i] / (float)K;
-        sum[i] = 0.f;
-#pragma unroll
-        for (int j = 0; j < CH; ++j)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                v[i][j][e] -= mean[i];
-                sum[i] += lane + j * 64 < chunks ? v[i][j][e] * v[i][j][e] : 0.f;
+                for (int e = 0; e < 8; ++e) sum[i] += lane + j * 64 < chunks ? v[i][j][e] : 0.f;
             }
-    }
+        }
+        if (b + RB < RW) {  // the next rows, which come behind W, while these are normed
+            load_rows(b + RB);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1)
+        for (int o = 32; o > 0; o >>= 1)
 #pragma unroll
-        for (int i = 0; i < RW; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+            for (int i = 0; i < RB; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
 #pragma unroll
-    for (int i = 0; i < RW; ++i) {
-        const int m = wave + i * NORMED_WAVES;
-        if (m >= M) break;
-        const float rstd = 1.0f / sqrtf(sum[i] / (float)K + eps);
+        for (int i = 0; i < RB; ++i) {
+            mean[i] = sum[i] / (float)K;
+            sum[i] = 0.f;
 #pragma unroll
-        for (int j = 0; j < CH; ++j) {
-            float o[8];
+            for (int j = 0; j < CH; ++j)
 #pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = v[i][j][e] * rstd * gain[j][e] + shift[j][e];
-            if (lane + j * 64 < chunks) *reinterpret_cast<uint4*>(rows + m * pitch + (lane + j * 64) * 8) = pack8(o);
+                for (int e = 0; e < 8; ++e) {
+                    v[i][j][e] -= mean[i];
+                    sum[i] += lane + j * 64 < chunks ? v[i][j][e] * v[i][j][e] : 0.f;
+                }
+        }
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+#pragma unroll
+            for (int i = 0; i < RB; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+#pragma unroll
+        for (int i = 0; i < RB; ++i) {
+            const int m = wave + (b + i) * NORMED_WAVES;
+            if (m >= M) break;
+            const float rstd = 1.0f / sqrtf(sum[i] / (float)K + eps);
+#pragma unroll
+            for (int j = 0; j < CH; ++j) {
+                float o[8];
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = v[i][j][e] * rstd * gain[j][e] + shift[j][e];
+                if (lane + j * 64 < chunks) *reinterpret_cast<uint4*>(rows + m * pitch + (lane + j * 64) * 8) = pack8(o);
+            }
         }
     }
     // the barrier waits for LDS alone: W stays on its way
@@ -844,9 +858,9 @@ extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* 
 }
 
 // Whether the two entry points below take so many rows of x, elements of K and rows of W: each workgroup norms the rows again, which
-// pays with two workgroups a compute unit up to eight rows of x, with one up to sixteen
+// pays with up to two workgroups a compute unit.  One answer for up to sixteen rows of x: a batch's size changes no bit of a sequence
 extern "C" int pta_gemm_normed_ok(int M, int N, int K) {
-    return M > 0 && M <= 16 && K > 0 && K % 8 == 0 && K <= 2048 && N > 0 && N <= (M <= 8 ? 32 : 16) * pta_compute_units();
+    return M > 0 && M <= 16 && K > 0 && K % 8 == 0 && K <= 2048 && N > 0 && N <= 32 * pta_compute_units();
 }
 
 template <bool TAIL>
@@ -868,7 +882,8 @@ static int launch_normed(const char* what, const SkinnyProblem& p, const float* 
         constexpr int CH = decltype(ch)::value;
         if (eight && M <= 8) go(gemm_normed_kernel<8, CH, 1, TAIL>);
         else if (eight) go(gemm_normed_kernel<8, CH, 2, TAIL>);
-        else go(gemm_normed_kernel<4, CH, 2, TAIL>);  // (more workgroups than units: up to eight rows)
+        else if (M <= 8) go(gemm_normed_kernel<4, CH, 2, TAIL>);
+        else go(gemm_normed_kernel<4, CH, 4, TAIL>);
     };
     switch ((K + 511) / 512) {
         case 1: by_rows(std::integral_constant<int, 1>{}); break;

@@ -20,9 +20,6 @@ def test_norm_and_product(M, N, K, act):
     from pytorch_transformers_amd import ops
 
     x, w, gain, shift, bias = _draw(M, N, K, M + N + K)
-    if N > 4096 and M > 8:
-        assert not ops.gemm_normed_ok(x, w)
-        return
     assert ops.gemm_normed_ok(x, w)
     got = ops.gemm_normed(x, gain, shift, 1e-5, w, bias, act).double()
     rows = torch.nn.functional.layer_norm(x.double(), (K,), gain.double(), shift.double(), 1e-5).bfloat16().double()
@@ -70,4 +67,17 @@ def test_sizes_it_leaves_to_others():
     from pytorch_transformers_amd import ops
 
     ok = lambda M, N, K: ops.gemm_normed_ok(torch.empty(M, K, dtype=torch.bfloat16, device="cuda"), torch.empty(N, K, dtype=torch.bfloat16, device="cuda"))
-    assert ok(8, 8192, 2048) and ok(16, 4096, 2048) and not ok(9, 4097, 2048) and not ok(17, 64, 64) and not ok(1, 64, 2056) and not ok(1, 64, 12) and not ok(1, 8193, 64)
+    assert ok(8, 8192, 2048) and ok(16, 4096, 2048) and ok(16, 8192, 2048) and not ok(17, 64, 64) and not ok(1, 64, 2056) and not ok(1, 64, 12) and not ok(1, 8193, 64)
+
+
+@pytest.mark.parametrize("N,K", [(64, 64), (4096, 2048), (4352, 1040), (4368, 1536), (8192, 520), (8192, 2048)])
+def test_a_row_has_the_same_bits_in_any_batch(N, K):
+    """Sizes of W alone choose the launch, its waves and so the order of summation: of sixteen rows each is what it is alone."""
+    from pytorch_transformers_amd import ops
+
+    x, w, gain, shift, bias = _draw(16, N, K, N + K)
+    assert all(ops.gemm_normed_ok(x[:m], w) for m in (1, 8, 9, 16))
+    whole = ops.gemm_normed(x, gain, shift, 1e-5, w, bias, "gelu")
+    for rows in (x[:1], x[:8], x[:9], x[:13]):
+        assert torch.equal(ops.gemm_normed(rows, gain, shift, 1e-5, w, bias, "gelu"), whole[:len(rows)])
+    assert torch.equal(ops.gemm_normed(x[9:10].contiguous(), gain, shift, 1e-5, w, bias, "gelu"), whole[9:10])
