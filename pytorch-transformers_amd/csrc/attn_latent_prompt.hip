@@ -16,10 +16,12 @@
 // over all banks: sixteen bytes of 32 rows at one place, and for V^T, by the transposing read (ds_read_tr16: sixteen lanes give the
 // addresses of four rows of sixteen elements and get an element of the four rows each), 32 neighbours of four rows.  The order
 // of keys within a step of 16 of the second product is the one in which the score tile's lanes hold them.
+// A latent that is infinite or undefined changes no bit of a token that does not see it.
 //
-// Measured, two sequences of 1,500 and 1,900 tokens, 16 heads (102 GFLOP): 200 us, 510 TFLOP/s, where attn_latent_mfma.h's kernel
-// takes 585; one of 2,048 134 / 427, eight of 64 to 700 tokens 108 / 235 (there a workgroup's start, its queries above all, takes
-// as long as its keys), one of 100 23 / 38.  Error against 64 bits: that kernel's to five digits.
+// Measured, launches in a row: two sequences of 1,500 and 1,900 tokens, 16 heads (102 GFLOP) 210 us, 490 TFLOP/s, where
+// attn_latent_mfma.h's kernel takes 585; within the request, between other kernels, 231 us.  One of 2,048 132 / 427, eight of 64 to 700
+// tokens 98 / 235 (there a workgroup's start, its queries above all, takes as long as its keys), one of 100 22 / 38.  Error against
+// 64 bits: that kernel's to five digits.
 #include "common.h"
 #include "pta_kernels.h"
 
@@ -40,7 +42,8 @@ typedef float f32x2_t __attribute__((ext_vector_type(2)));
 #define LP_LOADS (LP_STAGE / (256 * 16))
 #define LP_WEIGHTS (LP_STAGES * LP_STAGE)    // after the stages: the waves' weights, 2 KB each
 #define LP_MAXIMA (LP_WEIGHTS + 4 * 2048)    // and their columns' largest scores
-#define LP_LDS (LP_MAXIMA + 4 * 32 * 4)
+#define LP_FLAGS (LP_MAXIMA + 4 * 32 * 4)    // and whether a wave found a value that is infinite or undefined
+#define LP_LDS (LP_FLAGS + 4 * 4)
 #define LP_LOG2E 1.4426950408889634f
 
 struct LatentPromptArgs {
@@ -66,6 +69,9 @@ __device__ __forceinline__ uint32_t lp_pack(float lo, float hi) {
     c.b = __builtin_convertvector(f32x2_t{lo, hi}, bf16x2_t);
     return c.u;
 }
+
+// two neighbours of bfloat16, one of them infinite or undefined
+__device__ __forceinline__ bool lp_special(uint32_t u) { return (u & 0x7f80u) == 0x7f80u || (u & 0x7f800000u) == 0x7f800000u; }
 
 template <int N> __device__ __forceinline__ void lp_wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 
@@ -99,8 +105,11 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
     const int tq = valid ? rr / H : 0, head = valid ? rr - tq * H : 0;
     const int pos_q = valid ? start + tq : -1;  // -1: sees no key
     const long at_row = (long)(t0 + tq) * H + head;
-    const int k_end = start + min(n_new - 1, (row0 + LP_COLS - 1) / H) + 1;  // keys this workgroup walks
-    const int all_see = wrow0 + 31 < columns ? start + wrow0 / H : -1;       // positions up to here every column sees
+    // (quotients come out of vector registers, of which there are none to spare)
+    auto scalar = [](int v) { return __builtin_amdgcn_readfirstlane(v); };
+    const int k_end = scalar(start + min(n_new - 1, (row0 + LP_COLS - 1) / H) + 1);  // keys this workgroup walks
+    const int all_see = scalar(wrow0 + 31 < columns ? start + wrow0 / H : -1);       // positions up to here every column sees
+    const int first_pos = scalar(start + row0 / H);                                  // and every one of the workgroup that is a token's
 
     // staging: place p of a stage (sixteen bytes) is piece (p % 72, turned within its eight) of row p / 72; 32 rows on the same again
     auto turn = [](int r) { return ((r >> 1 & 1) << 2) | ((r >> 2 & 1) << 1) | (r >> 3 & 1); };
@@ -151,6 +160,7 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
         }
     char* weights = lds + LP_WEIGHTS + pair * 4096 + lane * 16;            // [half of the keys][step][lane]
     float* maxima = (float*)(lds + LP_MAXIMA) + pair * 64 + c;             // [half of the keys][column]
+    int* flags = (int*)(lds + LP_FLAGS);
 
     f32x16_t oacc[VT];
 #pragma unroll
@@ -163,7 +173,7 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
     lp_meet();
     for (int b = 0; b < blocks; ++b) {
         const int kb = b * LP_KEYS + 32 * kw;
-        const char* base = lds + (b & 1) * LP_STAGE;
+        char* base = lds + (b & 1) * LP_STAGE;
         if (b + 1 < blocks) fetch(b + 1, (b + 1) & 1);
         f32x16_t sc;
 #pragma unroll
@@ -193,7 +203,21 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
         for (int e = 1; e < 16; ++e) mx = fmaxf(mx, sc[e]);
         mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
         if (h == 0) maxima[kw * 32] = mx;
+        // Rows r0 .. r1 - 1 are seen by some columns of the workgroup only (a few of its last page).  A value among them that is
+        // infinite or undefined must reach those alone, and a weight of zero would not keep it from the others.
+        const int r0 = max(first_pos + 1 - b * LP_KEYS, 0), r1 = min(k_end - b * LP_KEYS, LP_KEYS);
+        if (r0 < r1) {
+            bool found = false;
+            for (int r = r0 + 2 * pair + h; r < r1; r += 4) {
+                const uint4 u = *reinterpret_cast<const uint4*>(base + r * LP_ROW + kw * LP_R + c * 16);
+                found |= lp_special(u.x) || lp_special(u.y) || lp_special(u.z) || lp_special(u.w);
+            }
+            found = __any(found);
+            if (lane == 0) flags[wave] = found;
+        }
         lp_meet();
+        bool special = false;
+        if (r0 < r1) special = __builtin_amdgcn_readfirstlane(flags[0] | flags[1] | flags[2] | flags[3]);
         // The first 32 keys count from the largest score up to them, the other 32 from the largest of all: a block's largest weight
         // is then exactly one in each half (with one reference for the 64, or one that lags behind, fewer weights are, and the
         // result's error against 64 bits grows by 0.5 and by 4 %).  Both waves of the pair see the same numbers.
@@ -230,6 +254,38 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
             *reinterpret_cast<uint4*>(weights + kw * 2048 + k2 * 1024) = pf[0][k2].u;
         }
         if (kw == 0) l_run *= corr_l;
+        if (special) {  // (rare) such values are added where they are seen, by hand, and then stand as zeros for the products
+            lp_meet();  // everyone's weights are there
+            for (int r = r0; r < r1; ++r) {
+                const bf16_t wb = *reinterpret_cast<const bf16_t*>(lds + LP_WEIGHTS + pair * 4096 + (r >> 5) * 2048 + (r >> 4 & 1) * 1024 +
+                                                                   (c + 32 * (r >> 2 & 1)) * 16 + ((r >> 3 & 1) * 4 + (r & 3)) * 2);
+                if (b * LP_KEYS + r > pos_q) continue;
+                const float w = bf16_bits_to_f32(wb);
+#pragma unroll
+                for (int t = 0; t < VT; ++t)
+#pragma unroll
+                    for (int e = 0; e < 16; e += 4) {
+                        const uint2 u = *reinterpret_cast<const uint2*>(base + r * LP_ROW + kw * LP_R + (t >> 1) * 128 +
+                                                                        (((t & 1) * 4 + (e >> 2)) ^ turn(r)) * 16 + h * 8);
+                        if (!(lp_special(u.x) || lp_special(u.y))) continue;
+                        const uint32_t bits[4] = {u.x << 16, u.x & 0xffff0000u, u.y << 16, u.y & 0xffff0000u};
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+                            if ((bits[i] & 0x7f800000u) == 0x7f800000u) oacc[t][e + i] += w * __uint_as_float(bits[i]);
+                    }
+            }
+            lp_meet();
+            for (int i = tid; i < (r1 - r0) * (LP_R / 4); i += 256) {
+                uint2* at = reinterpret_cast<uint2*>(base + (r0 + i / (LP_R / 4)) * LP_ROW + i % (LP_R / 4) * 8);
+                uint2 u = *at;
+                if ((u.x & 0x7f80u) == 0x7f80u) u.x &= 0xffff0000u;
+                if ((u.x & 0x7f800000u) == 0x7f800000u) u.x &= 0xffffu;
+                if ((u.y & 0x7f80u) == 0x7f80u) u.y &= 0xffff0000u;
+                if ((u.y & 0x7f800000u) == 0x7f800000u) u.y &= 0xffffu;
+                *at = u;
+            }
+            lp_meet();
+        }
         LpFrag vf[2][4];  // a tile's four steps of 16 keys
         auto read_v = [&](LpFrag (&dst)[4], int t) {
 #pragma unroll

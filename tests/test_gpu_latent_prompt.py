@@ -87,3 +87,37 @@ def test_other_addresses_take_the_general_kernel(what):
     assert (q2.data_ptr() | pool2.data_ptr()) % 16
     got = ops.attn_latent(q2, pool2, table, seq, pos, rank, 0.05, ctx=ctx)
     assert (got - want).norm() <= 2.0 ** -7 * want.norm()
+
+
+@pytest.mark.parametrize("heads", [1, 3, 16, 70])
+@pytest.mark.parametrize("start,bad,where", [(0, (70,), "value"), (0, (64, 65, 127), "all"), (37, (40, 101, 102), "value"), (0, (1,), "rotated"), (5, (199,), "value")])
+@pytest.mark.parametrize("what", [float("inf"), float("-inf"), float("nan")])
+def test_undefined_latents_stay_with_those_who_see_them(heads, start, bad, where, what):
+    """Infinities in a later token's latent change no bit of the tokens before it, also of those that share its columns' workgroup;
+    the tokens that see one have a result that is undefined."""
+    from pytorch_transformers_amd import ops
+
+    rank, D, T = 512, 576, 200 - start
+    g = torch.Generator().manual_seed(heads + start)
+    rows = (torch.randn(256, D, generator=g) * 0.7).bfloat16()
+    q = (torch.randn(T, heads, D, generator=g) * 1.5).cuda()
+    table = torch.randperm(4, generator=g).int().view(1, 4).cuda()
+    seq, pos = torch.zeros(T, dtype=torch.int32).cuda(), torch.arange(start, 200, dtype=torch.int32).cuda()
+    ctx = types.SimpleNamespace(cu_tokens=torch.tensor([0, T], dtype=torch.int32).cuda(), seq_start=torch.full((1,), start, dtype=torch.int32).cuda(),
+                                new_tokens=[T], max_len=200, is_decode=False)
+
+    def run(rows):
+        pool = torch.empty(4, 1, 64, D, dtype=torch.bfloat16, device="cuda")
+        pool[table[0].long(), 0] = rows.view(4, 64, D).cuda()
+        return ops.attn_latent(q, pool, table, seq, pos, rank, 0.05, ctx=ctx)
+
+    clean = run(rows)
+    for element in {"value": (0, 3, 255, 256, 300, 511), "rotated": (512, 575), "all": (None,)}[where]:
+        dirty = rows.clone()
+        for r in bad:
+            dirty[r, slice(None) if element is None else element] = what
+        got = run(dirty)
+        before = min(bad) - start
+        assert torch.equal(got[:before], clean[:before]) and bool(torch.isfinite(clean).all())
+        if where != "rotated" or what != what:  # (an infinite score may also be a weight of zero)
+            assert not bool(torch.isfinite(got[before:]).all(-1).any())
