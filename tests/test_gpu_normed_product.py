@@ -50,17 +50,23 @@ def test_norm_and_fused_rows_to_their_end(layout, nh, nkv, d, M, rotated):
     inv = 10000.0 ** (-torch.arange(d // 2, device="cuda").float() * 2 / d) if rotated else None
     pos = torch.randint(0, 190, (M,), generator=g).int().cuda()
     seq, table = torch.arange(M).int().cuda(), torch.randperm(3 * M, generator=g).view(M, 3).int().cuda()
-    new = lambda: (torch.full((3 * M, nkv, 64, d), 7.0).bfloat16().cuda(), torch.full((3 * M, nkv, d, 64), 7.0).bfloat16().cuda())
+    new = lambda: (torch.full((3 * M, nkv, 64, d), float("nan")).bfloat16().cuda(), torch.full((3 * M, nkv, d, 64), float("nan")).bfloat16().cuda())
     k0, v0 = new()
     q0 = ops.gemm_skinny_qkv(ops.layernorm(x, gain, shift, 1e-5), w, bias, inv, 0.9, pos, seq, table, k0, v0, nh, nkv, d, layout, True)
     k1, v1 = new()
     q1 = ops.gemm_normed_qkv(x, gain, shift, 1e-5, w, bias, inv, 0.9, pos, seq, table, k1, v1, nh, nkv, d, layout, True)
-    for a, b in ((q0, q1), (k0, k1), (v0, v1)):
-        assert (a.float() - b.float()).norm() <= 2.0 ** -8 * a.float().norm()
-        assert torch.equal(a == 7.0, b == 7.0) or (a.float() - b.float()).abs().max() <= 0.1
+    page, at = table[torch.arange(M, device="cuda"), (pos // 64).long()].long(), (pos % 64).long()
+    rows = lambda k, v: (k[page, :, at], v[page, :, :, at])  # what each token wrote
+    for a, b in zip((q0,) + rows(k0, v0), (q1,) + rows(k1, v1)):
+        a, b = a.float(), b.float()
+        # sums of ~1,000 terms of which a few normed ones are a neighbour (2^-8 of themselves), the results a neighbour in places
+        assert bool(torch.isfinite(a).all()) and (a - b).norm() <= 2.0 ** -8 * a.norm()
+        assert (a - b).abs().max() <= 2.0 ** -6 * a.abs().max()
+    for pool in (k1, v1):  # and nothing else
+        assert int((~pool.isnan()).sum()) == M * nkv * d
     k2, v2 = new()
     ops.gemm_normed_qkv(x, gain, shift, 1e-5, w, bias, inv, 0.9, pos, seq, table, k2, v2, nh, nkv, d, layout, False)
-    assert bool((k2 == 7.0).all()) and bool((v2 == 7.0).all())
+    assert bool(k2.isnan().all()) and bool(v2.isnan().all())
 
 
 def test_sizes_it_leaves_to_others():
