@@ -243,9 +243,11 @@ class PendingProjection:
         return self.linear.partial(self.x)
 
     def additions_cost_a_pass(self) -> bool:
-        """Whether tensors added to this product would be a pass of their own over the result: the vendor
-        library's product of many rows, which has no epilogue of ours, with no bias to add.  The norm that reads
-        the sum next can then form it while it reads (``ResidualSum``)."""
+        """Whether the norm that reads the sum next should form it while it reads (``ResidualSum``): products of many rows with
+        no bias to add.  The library's product has no epilogue of ours, so additions would be a pass of their own over the result.
+        The hand-written kernel for many rows could add in its epilogue, which is no faster.  Output products of mixer and
+        feed-forward, the sum of three and the norm, the sum in the norm / in the epilogue: 512 rows of 4,544 135 / 135 us, 2,048 380 / 379,
+        2,317 420 / 425, 4,740 rows of 8,192 2,501 / 2,545, 895 of 1,040 43 / 47."""
         x, lin = self.x, self.linear
         return (x.dtype == torch.bfloat16 and lin.bias is None and ops.layernorm_sum_ok(lin.out_features)
                 and x.shape[0] >= ops.layernorm_sum_rows_min()
