@@ -127,5 +127,7 @@ class AttentionMixer(Part):
             return PendingProjection(self.out, o)
         return self.out(o, add1=residual)
 
+    forward.reads_projected_alone = True
+
 
 register_part("mixer", "attention", AttentionMixer)

@@ -37,8 +37,11 @@ Optional: a mixer or feed-forward that sets ``can_defer = True`` and is called w
 ``defer=True`` returns its last product not run, as a ``PendingProjection`` (the
 ``Linear`` and its input; residual and additions are then the caller's), and one
 with ``input_projection()`` lets the block run its first product and hand the result
-in as ``projected``.  A block may so run two branches' products in one launch, and
-leave the last ones as 32-bit partial sums (:class:`PartialProduct`) in a
+in as ``projected``.  Where its ``forward`` then reads nothing else of its input, the
+function may say so (``forward.reads_projected_alone = True`` in the class; a subclass
+with a ``forward`` of its own says it again): a block may then have the norm in front run
+inside that product's launch, and pass the rows as they were before the norm.  A block may
+so run two branches' products in one launch, and leave the last ones as 32-bit partial sums (:class:`PartialProduct`) in a
 :class:`ResidualSum` that it returns in place of a tensor.  A norm with
 ``forward_sum(sum, rows=None, other=None, want_x=True) -> (x, normed, normed_other)``
 forms such a sum while it normalises it; a block with ``accepts_sum = True`` takes one

@@ -41,6 +41,17 @@ def _normed(x, norm: Part, other: Optional[Part] = None):
     return x, a, m
 
 
+def _normed_projection(part: Part, x, norm: Part, tail=None, offers: str = "input_projection") -> dict:
+    """``{"projected": ...}``, the first product of ``part`` together with the norm in front of it from one launch
+    (``Linear.normed``), where there is one; else nothing.  The normed rows themselves are nowhere then, so ``part.forward`` has to
+    be one that reads nothing of its input but that product (``reads_projected_alone``)."""
+    if not (isinstance(x, torch.Tensor) and hasattr(part, offers) and getattr(type(part).forward, "reads_projected_alone", False)):
+        return {}
+    linear, how = part.input_projection()
+    projected = None if linear is None else linear.normed(x, norm, **({"tail": tail} if tail is not None else how))
+    return {} if projected is None else {"projected": projected}
+
+
 def _sum_parallel(ffn_out: PendingProjection, mixer_out: PendingProjection, x: torch.Tensor):
     """feed-forward + mixer + residual, in that order, formed now or left to the next norm."""
     both = PendingProjection.partial_pair(ffn_out, mixer_out)
@@ -117,23 +128,16 @@ class SequentialBlock(Part):
 
     def forward(self, x, ctx: StepContext, call):
         # in steps of few tokens each norm rides in the launch of the product behind it
-        kw, projected = {}, None
-        if isinstance(x, torch.Tensor) and hasattr(self.mixer, "projection_tail"):
-            projected = self.mixer.input_projection()[0].normed(x, self.norm_in, tail=lambda: self.mixer.projection_tail(ctx, call))
-        if projected is not None:
-            a, kw["projected"] = x, projected
+        kw = _normed_projection(self.mixer, x, self.norm_in, lambda: self.mixer.projection_tail(ctx, call), "projection_tail")
+        if kw:
+            a = x
         else:
             x, a, _ = _normed(x, self.norm_in)
         if _can_defer(self.mixer):
             r = _sum_sequential(self.mixer.forward(a, ctx, call, defer=True, **kw), x)
         else:
             r = self.mixer.forward(a, ctx, call, residual=x, **kw)
-        kw = {}
-        if isinstance(r, torch.Tensor) and hasattr(self.feed_forward, "input_projection"):
-            linear, how = self.feed_forward.input_projection()
-            projected = linear.normed(r, self.norm_post, **how)
-            if projected is not None:
-                kw["projected"] = projected
+        kw = _normed_projection(self.feed_forward, r, self.norm_post)
         if kw:
             m = r
         else:

@@ -44,6 +44,8 @@ class DenseFeedForward(Part):
             return PendingProjection(self.down, h)
         return self.down(h, add1=as_tensor(add1), add2=as_tensor(add2))
 
+    forward.reads_projected_alone = True
+
 
 class PolyNormFeedForward(Part):
     """``down(act(up(x)))`` without biases, with the activation PolyNorm: over a token's vector z of ``ffn_size`` values,
@@ -133,6 +135,8 @@ class GatedFeedForward(Part):
         F = self.ffn_size
         y = ops.glu(both[:, :F], both[:, F:], self.kind, self.alpha, self.limit)
         return self.down(y, add1=as_tensor(add1), add2=as_tensor(add2))
+
+    forward.reads_projected_alone = True
 
 
 EXPERT_GATES = ("silu", "clamped")  # the kinds of gate that the experts' launches form

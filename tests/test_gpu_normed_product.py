@@ -87,3 +87,55 @@ def test_a_row_has_the_same_bits_in_any_batch(N, K):
     for rows in (x[:1], x[:8], x[:9], x[:13]):
         assert torch.equal(ops.gemm_normed(rows, gain, shift, 1e-5, w, bias, "gelu"), whole[:len(rows)])
     assert torch.equal(ops.gemm_normed(x[9:10].contiguous(), gain, shift, 1e-5, w, bias, "gelu"), whole[9:10])
+
+
+@pytest.mark.parametrize("which", ["mixer", "feed-forward", "no product"])
+def test_parts_that_read_their_input_get_the_normed_rows(which):
+    """A mixer or feed-forward with a ``forward`` of its own may read its input beside the product that it is handed: what it is
+    given is the norm's result then; the library's own parts, which read nothing else, have the norm inside the product's launch."""
+    import test_gpu_parts as TP
+    from pytorch_transformers_amd import ops
+    from pytorch_transformers_amd.cache import PagedCache
+    from pytorch_transformers_amd.engine.spec import CACHE_FULL, CacheGroupSpec, LayerCall
+    from pytorch_transformers_amd.parts import AttentionMixer, DenseFeedForward, LayerNorm, NoPositions, SequentialBlock
+    from pytorch_transformers_amd.parts.base import as_tensor
+
+    H, nh, d, seen = 64, 4, 16, []
+
+    class OwnMixer(AttentionMixer):
+        def forward(self, x, *a, **k):
+            seen.append(x)
+            return super().forward(x, *a, **k)
+
+    class OwnFeedForward(DenseFeedForward):
+        def forward(self, x, *a, **k):
+            seen.append(x)
+            return super().forward(x, *a, **k)
+
+    class NoProduct(DenseFeedForward):
+        def input_projection(self):
+            return None, {}
+
+    def block(mixer, ffn):
+        b = SequentialBlock(mixer("a", H, nh, nh, d, "interleaved", True, NoPositions()), ffn("f", H, 128, bias=True), LayerNorm("n1", H, 1e-5),
+                            LayerNorm("n2", H, 1e-5))
+        TP._fill(b, torch.bfloat16, 3)
+        return b
+
+    x = torch.randn(3, H, generator=torch.Generator().manual_seed(0)).bfloat16().cuda()
+
+    def run(b):
+        cache = PagedCache([CacheGroupSpec("kv", CACHE_FULL, 1, nh, d)], 256, torch.bfloat16, "cuda:0")
+        ctx, _ = TP._ctx(cache, [cache.alloc()], [3], torch.bfloat16)
+        return as_tensor(b.forward(x, ctx, LayerCall(0, "kv", 0))).float()
+
+    want = run(block(AttentionMixer, DenseFeedForward))
+    b = block(OwnMixer if which == "mixer" else AttentionMixer, {"feed-forward": OwnFeedForward, "no product": NoProduct}.get(which, DenseFeedForward))
+    got = run(b)
+    assert (got - want).norm() <= 2.0 ** -7 * want.norm()
+    if which == "mixer":
+        assert torch.equal(seen[0], b.norm_in.forward(x))
+    elif which == "feed-forward":
+        a = seen[0].float()  # rows of a norm: the gain and shift taken off, mean 0 and mean square 1
+        z = (a - b.norm_post.bias) / b.norm_post.weight
+        assert z.mean(1).abs().max() <= 0.02 and (z.pow(2).mean(1) - 1).abs().max() <= 0.05
