@@ -6,6 +6,14 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
+@pytest.fixture(autouse=True)
+def _on():
+    from pytorch_transformers_amd import ops
+
+    if not ops.GEMM_NORMED:
+        pytest.skip("switched off by PTA_GEMM_NORMED=0")
+
+
 def _draw(M, N, K, seed):
     g = torch.Generator().manual_seed(seed)
     r = lambda *s: torch.randn(*s, generator=g).cuda()

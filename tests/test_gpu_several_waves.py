@@ -5,7 +5,7 @@ from types import SimpleNamespace
 
 from pytorch_transformers_amd import ops, tuning
 
-pytestmark = pytest.mark.gpu
+pytestmark = [pytest.mark.gpu, pytest.mark.skipif(bool(ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES), reason="the cut is set by PTA_ATTN_SPLIT or PTA_ATTN_TILES")]
 
 
 @pytest.mark.parametrize("nh,nkv,d", [(13, 13, 80), (71, 1, 64), (4, 2, 16), (64, 8, 64)])

@@ -101,6 +101,8 @@ def test_additions_at_any_address():
     bias = torch.randn(N, generator=torch.Generator().manual_seed(6)).to(DEV)
     wide = torch.randn(2 * M * N + 1, generator=torch.Generator().manual_seed(7)).bfloat16().to(DEV)
     at = lambda off: wide[off:off + M * N].view(M, N)
+    if not ops.GEMM_TILE:
+        pytest.skip("switched off by PTA_GEMM_TILE=0")
     assert ops.gemm_tile_takes(x, w) and ops.gemm_tile_rule(M, N, K)
     for act in (None, "gelu"):
         for add1, add2 in ((at(1), None), (at(0), at(M * N + 1)), (at(3), at(5))):

@@ -17,6 +17,8 @@ def ways(monkeypatch):
     """``ops`` with a table of its own, and the names of what products run in, in order: "tile", or rows of a library product."""
     from pytorch_transformers_amd import ops, tuning
 
+    if not (ops.GEMM_TILE and tuning.MM_CHUNKS):
+        pytest.skip("switched off by PTA_GEMM_TILE=0 or PTA_MM_CHUNKS=0")
     seen, tile, mm = [], ops.gemm_tile_bf16, torch.mm
     monkeypatch.setattr(ops, "gemm_tile_bf16", lambda *a, **k: (seen.append("tile"), tile(*a, **k))[1])
     monkeypatch.setattr(torch, "mm", lambda x, w, **k: (seen.append(x.shape[0]), mm(x, w, **k))[1])
@@ -95,6 +97,8 @@ def test_joined_matrices_are_timed_with_what_follows_them(ways, monkeypatch, act
     from pytorch_transformers_amd.parts import Linear
 
     ops, tuning, _ = ways
+    if not tuning.MM_JOIN:
+        pytest.skip("switched off by PTA_MM_JOIN=0")
     M, N1, N2, K = 600, 72, 136, 200
     g = torch.Generator().manual_seed(2)
     first, second = Linear("a", K, N1, False), Linear("b", K, N2, False)
