@@ -749,10 +749,10 @@ extern "C" int pta_gemm_skinny_bf16(void* y, const void* x, const void* W, const
                 "gemm_skinny_bf16: waves per workgroup must be 0 (choose) or a power of two up to 8, got %d", waves);
     hipStream_t s = (hipStream_t)stream;
     const SkinnyProblem none{nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0, 0};
+    PTA_REQUIRE(!out_f32 || act == PTA_ACT_NONE || act == PTA_ACT_GELU, "gemm_skinny_bf16: activation %d needs a bfloat16 result", act);
     if (!in_kernel(act)) {
         // the kernel's epilogue knows the exact GELU and the squared ReLU only (every activation there would cost it its
         // unrolled loops): the product with its bias first, then activation and additions as a pass over y
-        PTA_REQUIRE(!out_f32, "gemm_skinny_bf16: activation %d needs a bfloat16 result", act);
         const SkinnyProblem plain{y, (const bf16_t*)x, (const bf16_t*)W, bias, nullptr, nullptr, N, PTA_ACT_NONE, 0};
         if (launch_skinny<bf16_t>(plain, none, M, K, variant, waves, s)) return 1;
         return pta_epilogue(y, N, nullptr, add1, add2, M, N, act, PTA_BF16, stream);

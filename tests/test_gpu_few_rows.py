@@ -133,3 +133,15 @@ def test_one_arithmetic_of_the_gate_for_any_rows(kind, F):
         both = ops.gemm_skinny_bf16(x[:16], w)
         got, want = ops.gemm_skinny_glu(x[:16], w, kind, 1.7, 3.0), ops.glu(both[:, :F], both[:, F:], kind, 1.7, 3.0)
         assert (got != want).float().mean() <= 0.01
+
+
+@pytest.mark.parametrize("act", ["relu2", "silu", "gelu_new"])
+@pytest.mark.parametrize("N", [64, 8192])
+def test_activations_of_32_bit_results_are_refused(act, N):
+    """Results in 32-bit are the output head's: they take no activation but the exact GELU."""
+    from pytorch_transformers_amd import ops
+
+    x, w = torch.ones(2, 64).bfloat16().cuda(), torch.ones(N, 64).bfloat16().cuda()
+    with pytest.raises(ops.KernelError, match="needs a bfloat16 result"):
+        ops.gemm_skinny_bf16(x, w, act=act, out_f32=True)
+    assert torch.equal(ops.gemm_skinny_bf16(x, w, act=act, out_f32=False), ops.epilogue_(ops.gemm_skinny_bf16(x, w), None, act))
