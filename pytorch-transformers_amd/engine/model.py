@@ -403,11 +403,9 @@ class CausalLM:
                     self.step(cache, [slot], [[0] * int(T)], "last")
                     cache.free(slot)
                 for b in (int(b) for b in batches):
-                    # one token each: the shape of a decode step; then the same with tokens before it in every
-                    # sequence, one sequence as long as the longest and the others such that the mean comes out
+                    # one token each: the shape of a decode step; then the same with tokens before it in every sequence
                     for longest, mean in [(1, 1)] + pairs:
-                        rest = longest if b == 1 else max(1, min(longest, (mean * b - longest) // (b - 1)))
-                        before = [longest - 1] + [rest - 1] * (b - 1)
+                        before = [n_ - 1 for n_ in tuning.context_lengths(longest, mean, b)]
                         slots = [cache.alloc() for _ in range(b)]
                         grow = [(s_, n_) for s_, n_ in zip(slots, before) if n_ > 0]
                         if grow:

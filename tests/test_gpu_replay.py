@@ -420,6 +420,22 @@ def test_tune_times_whole_steps_with_each_cut_of_the_decode_attention(folders):
     assert torch.equal(run(), before)
 
 
+def test_decode_steps_are_timed_at_unequal_lengths(folders, monkeypatch):
+    """``tune`` with a longest and a mean context times steps whose sequences differ as a service's do, not one long one among equals."""
+    from pytorch_transformers_amd import AutoModelForCausalLM, ops, tuning
+    from pytorch_transformers_amd.engine.model import CausalLM
+
+    model = AutoModelForCausalLM.from_pretrained(folders["C"], dtype="bfloat16")
+    seen = []
+    monkeypatch.setattr(CausalLM, "_time_decode_cuts", lambda self, cache, slots, timed: seen.append([cache.length(s) for s in slots]))
+    try:
+        model.tune(prompt_lens=(), batches=(8,), contexts=(300, (700, 350)))
+    finally:
+        ops.clear_tuning()
+    assert seen == [tuning.context_lengths(300, 300, 8), tuning.context_lengths(700, 350, 8)]
+    assert len(set(seen[1])) == 8 and sum(seen[1]) == 8 * 350
+
+
 def test_logits_of_a_step_outlive_the_next_step(folders):
     """What ``step`` returns is the caller's: the next step, replayed from the same captured graph, writes a
     buffer of its own."""
