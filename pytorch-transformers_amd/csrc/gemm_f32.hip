@@ -1,42 +1,53 @@
-// C[M,N] = act(A[M,K] . W[N,K]^T + bias) + add1 + add2 in true 32-bit, on the 32-bit matrix instruction
-// (v_mfma_f32_16x16x4_f32: products and sums in 32-bit, 154 TFLOP/s dense on this chip; the vector units give half).
+// C[M,N] = act(A[M,K] . W[N,K]^T + bias) + add1 + add2 in 32-bit, on the bfloat16 matrix instruction.
 // The 32-bit path of the whole model runs its projections, feed-forwards and output head through here.
 //
+// Every 32-bit value is the sum of three bfloat16 values, exactly: the nearest one, the nearest one to what is left, and the
+// rest, which has at most eight bits (split8).  Of the nine products of the parts of two values six are formed, the three left
+// out being under 2^-26 of the product of the values; each is exact in 32 bits, and so are the sums.  Six instructions of 16
+// cycles take the place of eight of 32 (v_mfma_f32_16x16x4_f32, 154 TFLOP/s).
+//
+// A value that is infinite, undefined or rounds to an infinite bfloat16 (above 3.39e38) has no such parts.  It leaves the sums
+// it takes part in undefined, and an overflow leaves them infinite: such sums are formed again on the 32-bit instruction
+// (plain_fragment), all others stay as they are.
+//
 // Order of summation.  A row's result is bitwise the same alone and in any batch, so every kernel here sums the products
-// of an output in one order, which K alone decides: K is walked in blocks of sixteen elements (the last one filled up with
+// of an output in one order, which K alone decides: K is walked in blocks of 32 elements (the last one filled up with
 // zeros), the blocks are cut into up to eight segments of equal length, a segment is one chain of matrix instructions
-// (a block is four instructions; each takes one element in four, from 3, 7, 11 and 15 down to 0, 4, 8 and 12, so that a
-// lane's four operands are sixteen consecutive bytes of a row), and the segments' sums are added in order.  Where a row lies in
+// (a block is six of them, the smallest parts first), and the segments' sums are added in order.  Where a row lies in
 // the grid, which kernel runs and how many workgroups share the segments changes nothing.
 //
-// The error against 64 bits, relative to the root of the sum of a row's squared products, is 3.7 x 2^-24 at K = 1,040, 7.2 at
-// 4,544 and 14.3 at 18,176 (rms).  Whether a block's four instructions go down or up makes no difference to it (7.22 and 7.21 at
-// 4,544, 14.31 and 14.31 at 18,176; down was the smaller in 56 of 144 draws): down is what it is, and every kernel has to keep to it.
+// The error against 64 bits, relative to the root of the sum of a row's squared products, in units of 2^-24 (rms): 0.8 at K = 64,
+// 3.1 at 1,040, 6.2 at 4,544 and 13.4 at 18,176.  Chains of the 32-bit instruction over the same segments gave 1.4, 3.7, 7.2 and
+// 14.3: an instruction here adds 32 products at a time, so a chain has fewer roundings.
 //
-// Measured at 4,544 / 18,176 features (one kernel of 64 x 64 tiles on the vector units before): one row of A 986 -> 56 us a
-// product on average (22 us = 3.7 TB/s for 83 MB, 70 to 75 us = 4.4 to 4.7 TB/s for 330 MB); 2,053 rows 26 -> 103 to 131 TFLOP/s.
+// Measured against the 32-bit instruction, microseconds: 2,053 rows by 4,544 x 4,544 703 -> 432 (196 TFLOP/s), by 18,176 x 4,544
+// 2,632 -> 1,640 (207), by 4,544 x 18,176 2,787 -> 1,632 (208); 60 rows by the same 42 -> 35, 146 -> 95, 120 -> 102; one row 21.2
+// -> 21.3, 71 -> 68, 65 -> 65, by 65,024 x 4,544 239 -> 198 (6.0 TB/s).
 //
-// Three ways to the same numbers, by what bounds them:
-//   few rows (M <= 32, with a short K 64): every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight
-//     waves a segment each; W goes from memory straight into the instruction's operands, the sums meet in LDS.
-//   many rows: tiles of 128 x 128 or 64 x 64 through two LDS buffers, bound by the matrix instruction (loads straight to LDS
-//     where rows are sixteen-byte aligned, else through registers).
-//   in between, or N small: too few tiles to fill the chip, so the segments of a tile are shared out over workgroups, whose
+// Three ways to the same numbers, by what bounds them (few_rows, f32_plan):
+//   few rows: every weight is read once and that is the time.
+//   many rows: tiles through two LDS buffers, bound by the matrix cores and the chip's power (8,192 x 8,192 x 4,096: 58 to 62 % of
+//     the cycles at 1.9 GHz).
+//   too few tiles to fill the chip, or to fill its last round: the segments of a tile are shared out over workgroups, whose
 //     sums go to memory and are added by a small launch.
 #include "common.h"
 #include "pta_kernels.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 #define SEGS 8          // segments of K, at most
-#define SKINNY_ROWS 32  // rows of A up to which the kernel for few rows runs
-#define SHARE_K 1024    // K from which segments may be shared out over workgroups
+#define BK 32           // elements of K of a block
+#define MOST_SUMS (32L << 20)           // 32-bit values that the segments' sums of cut tiles may take
+#define MOST_K (0x7f000000 / (256 * 4))  // elements of a row that tiles can address
+#define TILE_GROUP 8    // tiles along A that stand side by side in the order of tiles
 
 struct F32Epilogue {
     const float* bias;
     const float* add1;
     const float* add2;
     int act;
+    int wide;  // rows of C, add1 and add2 are read and written sixteen bytes at a time
 };
 
 __device__ __forceinline__ float finish(float v, const F32Epilogue& e, int n, long at) {
@@ -47,8 +58,30 @@ __device__ __forceinline__ float finish(float v, const F32Epilogue& e, int n, lo
     return v;
 }
 
+// four neighbours of row m of C from column n on, as far as they lie before column `end`
+__device__ __forceinline__ void store4(float* C, f32x4 v, const F32Epilogue& e, int m, int n, int end, int N) {
+    const long at = (long)m * N + n;
+    if (e.wide && n + 4 <= end) {
+        if (e.bias) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] += e.bias[n + j];
+        }
+        if (e.act) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) v[j] = apply_act(v[j], e.act);
+        }
+        if (e.add1) v += *(const f32x4*)(e.add1 + at);
+        if (e.add2) v += *(const f32x4*)(e.add2 + at);
+        *(f32x4*)(C + at) = v;
+        return;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+        if (n + j < end) C[at + j] = finish(v[j], e, n + j, at + j);
+}
+
 // How rows are read: element by element; sixteen bytes at a time (rows sixteen-byte aligned, K a multiple of 4); the same
-// without a look at the end (K a multiple of 16, what every published size is).
+// without a look at the end (K a multiple of 32, what every published size is).
 enum RowLoads { ROW_ELEMENTS, ROW_VECTORS, ROW_WHOLE };
 
 // four consecutive elements of a row from k on, zeros beyond K (ROW_WHOLE: k + 4 <= K is the caller's)
@@ -66,9 +99,72 @@ __device__ __forceinline__ f32x4 load4(const float* row, int k, int K) {
     return v;
 }
 
-__host__ __device__ static inline int seg_blocks(int K) { return ((K + 15) / 16 + SEGS - 1) / SEGS; }
+__host__ __device__ static inline int k_blocks(int K) { return (K + BK - 1) / BK; }
+__host__ __device__ static inline int seg_blocks(int K) { return (k_blocks(K) + SEGS - 1) / SEGS; }
+__host__ __device__ static inline int segments(int K) { return (k_blocks(K) + seg_blocks(K) - 1) / seg_blocks(K); }
+
+// ---- the three parts of a value -------------------------------------------------------------------------------------------
+struct Parts {
+    bf16x8 part[3];  // nearest, next, rest
+};
+
+// A lane's eight elements of a block: k from 4 c on and k from 16 + 4 c on, c = lane / 16 (any order will do that both
+// operands have; this one reads 64 bytes of a row by four lanes).
+__device__ __forceinline__ Parts split8(f32x4 a, f32x4 b) {
+    typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
+    typedef float f32_pair __attribute__((ext_vector_type(2)));
+    union { bf16x8 v[3]; uint32_t u[3][4]; } out;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+#pragma unroll
+        for (int p = 0; p < 3; ++p) {
+            union { bf16_pair h; uint32_t u; } c;
+            c.h = __builtin_convertvector(f32_pair{x, y}, bf16_pair);  // one instruction for the two
+            out.u[p][i] = c.u;
+            if (p < 2) {  // what is left: exact
+                x -= __uint_as_float(c.u << 16);
+                y -= __uint_as_float(c.u & 0xffff0000u);
+            }
+        }
+    }
+    return Parts{{out.v[0], out.v[1], out.v[2]}};
+}
+
+// the six products, the smallest first
+#define TERMS 6
+__device__ constexpr int term_w(int t) { return t == 0 ? 2 : t < 3 ? 1 : 0; }
+__device__ constexpr int term_x(int t) { return t == 3 ? 2 : t == 1 || t == 4 ? 1 : 0; }
+
+__device__ __forceinline__ bool any_not_finite(f32x4 v) {
+    bool bad = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bad |= !(fabsf(v[e]) <= 3.402823466e38f);
+    return __any(bad);
+}
+
+// Sixteen rows of W from n on by sixteen of A from m on, on the 32-bit instruction, one chain over all of K, for what `v` holds
+// that is not finite.
+template <int ROWS>
+__device__ __forceinline__ f32x4 plain_fragment(f32x4 v, const float* A, const float* W, int m, int n, int M, int N, int K) {
+    const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
+    const float* wr = W + (long)min(n + r16, N - 1) * K;
+    const float* xr = A + (long)min(m + r16, M - 1) * K;
+    f32x4 sum = {0.f, 0.f, 0.f, 0.f};
+    for (int k = kq; k < K + kq; k += 16) {
+        const f32x4 w = load4<ROWS == ROW_WHOLE ? ROW_VECTORS : ROWS>(wr, k, K), x = load4<ROWS == ROW_WHOLE ? ROW_VECTORS : ROWS>(xr, k, K);
+#pragma unroll
+        for (int j = 3; j >= 0; --j) sum = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j], x[j], sum, 0, 0, 0);
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+        if (!(fabsf(v[e]) <= 3.402823466e38f)) v[e] = sum[e];
+    return v;
+}
 
 // ---- few rows ---------------------------------------------------------------------------------------------------------
+// Every weight is read once and that is the time.  A workgroup owns up to 32 rows of W and its eight waves a segment each; W
+// goes from memory into registers, its parts into the instruction's operands, the sums meet in LDS.
 // CT: tiles of sixteen rows of A, RT: tiles of sixteen rows of W.  D blocks of K are asked for while the D before them are
 // multiplied: at K = 4,544 and one row of A a compute unit then has some 60 KB on its way.  What is asked for past a segment's
 // end is its last block again, which a cache has (the next segment's first blocks, long gone from the caches, were a sixth of all
@@ -81,7 +177,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
     const int r16 = lane & 15, kq = 4 * (lane >> 4);
     // the rows of W are shared out evenly: a launch takes as long as the compute unit with the most of them
     const int n0 = (int)((long)blockIdx.x * N / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * N / gridDim.x);
-    const int nb = (K + 15) / 16, sb = seg_blocks(K);
+    const int nb = k_blocks(K), sb = seg_blocks(K);
     const int b0 = seg * sb, b1 = min(nb, b0 + sb);
     const float* wr[RT];
     const float* xr[CT];
@@ -95,28 +191,36 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 #pragma unroll
         for (int c = 0; c < CT; ++c) acc[r][c] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    f32x4 w[2][D][RT], x[2][D][CT];
+    f32x4 w[2][D][RT][2], x[2][D][CT][2];
     auto fetch = [&](int buf, int b) {
 #pragma unroll
         for (int i = 0; i < D; ++i) {
-            const int k = 16 * min(b + i, b1 - 1) + kq;  // past the segment: its last block again, not used
+            const int k = BK * min(b + i, b1 - 1) + kq;  // past the segment: its last block again, not used
 #pragma unroll
-            for (int r = 0; r < RT; ++r) w[buf][i][r] = load4<ROWS>(wr[r], k, K);
+            for (int h = 0; h < 2; ++h) {
 #pragma unroll
-            for (int c = 0; c < CT; ++c) x[buf][i][c] = load4<ROWS>(xr[c], k, K);
+                for (int r = 0; r < RT; ++r) w[buf][i][r][h] = load4<ROWS>(wr[r], k + 16 * h, K);
+#pragma unroll
+                for (int c = 0; c < CT; ++c) x[buf][i][c][h] = load4<ROWS>(xr[c], k + 16 * h, K);
+            }
         }
     };
     auto multiply = [&](int buf, int b) {
 #pragma unroll
         for (int i = 0; i < D; ++i) {
             if (b + i < b1) {
+                Parts xs[CT];
 #pragma unroll
-                for (int j = 0; j < 4; ++j)
+                for (int c = 0; c < CT; ++c) xs[c] = split8(x[buf][i][c][0], x[buf][i][c][1]);
 #pragma unroll
-                    for (int r = 0; r < RT; ++r)
+                for (int r = 0; r < RT; ++r) {
+                    const Parts ws = split8(w[buf][i][r][0], w[buf][i][r][1]);
+#pragma unroll
+                    for (int t = 0; t < TERMS; ++t)
 #pragma unroll
                         for (int c = 0; c < CT; ++c)
-                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[buf][i][r][3 - j], x[buf][i][c][3 - j], acc[r][c], 0, 0, 0);
+                            acc[r][c] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws.part[term_w(t)], xs[c].part[term_x(t)], acc[r][c], 0, 0, 0);
+                }
             }
         }
     };
@@ -136,13 +240,10 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
     __syncthreads();
     const int used = (nb + sb - 1) / sb;
     for (int i = threadIdx.x; i < RT * CT * 64; i += 512) {
-        const int t = i >> 6, l = i & 63;
+        const int t = i >> 6, l = i & 63;  // a wave has a tile
         f32x4 v = part[0][t][l];
-        for (int s = 1; s < used; ++s) {
-            const f32x4 p = part[s][t][l];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) v[j] += p[j];
-        }
+        for (int s = 1; s < used; ++s) v += part[s][t][l];
+        if (any_not_finite(v)) v = plain_fragment<ROWS>(v, A, W, 16 * (t % CT), n0 + 16 * (t / CT), M, N, K);
         const int m = 16 * (t % CT) + (l & 15);
         const int n = n0 + 16 * (t / CT) + 4 * (l >> 4);
         if (m < M) {
@@ -154,371 +255,434 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 }
 
 // ---- many rows ----------------------------------------------------------------------------------------------------------
-// A workgroup of four waves, two by two, on a tile of T x T.  A row of a tile is 32 elements of K in LDS, 36 apart: the eight
-// lanes that read together (rows next to each other, sixteen bytes each) then cover every bank once.
-#define BK 32
-#define PITCH 36
+// A workgroup of eight waves (four along the rows of W, two along the rows of A) makes a tile of 64 FP rows of W by 32 FQ rows
+// of A, a block of K at a time.  Values come through registers, are taken apart once for the workgroup and lie in LDS as
+// three planes of rows of 64 bytes, sixteen bytes c of row r at place c ^ (-(r / 4) % 4), so that any sixteen lanes that read
+// together cover every bank once (they are not sixteen neighbours: with c ^ (r / 4 % 4) a third of the cycles were conflicts).  Two buffers, one barrier a block:
+//
+//   columns j = 0 .. FQ - 2: the parts of column j + 1 being read, a share of block b + 1 taken apart into the other buffer,
+//                            block b + 2 asked for
+//   barrier: the other buffer is whole, and everyone has read this one
+//   column FQ - 1: the next block's parts being read as those of this block have been used
+struct F32Tiles {
+    float* C;
+    float* part;  // segments' sums of cut tiles: [segment][tile][wave][fragment][lane][4]
+    const float* A;
+    const float* W;
+    int M, N, K;
+    int tiles_q, tiles_p;  // tiles along the rows of A and of W
+    int whole;             // the first tiles, computed over all of K
+    int share;             // workgroups that share the segments of each of the others
+};
 
-template <int T, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void gemm_f32_tile_kernel(float* __restrict__ C, const float* __restrict__ A,
-                                                               const float* __restrict__ W, F32Epilogue epi, int M, int N,
-                                                               int K, int tiles_m, int tiles_n) {
-    constexpr int F = T / 32;        // tiles of sixteen rows per wave and side
-    constexpr int L = T * 8 / 256;   // sixteen-byte loads per thread and side
-    __shared__ float As[2][T * PITCH];
-    __shared__ float Ws[2][T * PITCH];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int r16 = lane & 15, kq = 4 * (lane >> 4);
-    // workgroups go to the eight dies in turn: give each die a run of tiles that share rows of W, which its L2 then holds
-    const int tiles = tiles_m * tiles_n;
-    const int per = (tiles + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || tile >= tiles) return;
-    const int m0 = (tile % tiles_m) * T, n0 = (tile / tiles_m) * T;
-    const int wn = (wave & 1) * (T / 2), wm = (wave >> 1) * (T / 2);
-    const int nb = (K + 15) / 16, sb = seg_blocks(K);
-    // SPLIT: this workgroup's share of the segments
-    const int used = (nb + sb - 1) / sb;
-    const int s0 = SPLIT ? (int)((long)blockIdx.y * used / gridDim.y) : 0;
-    const int s1 = SPLIT ? (int)((long)(blockIdx.y + 1) * used / gridDim.y) : used;
-    const int b_first = s0 * sb, b_last = min(nb, s1 * sb);
+__device__ __forceinline__ void tile_at(const F32Tiles& job, int t, int& tp, int& tq) {
+    const int per_group = TILE_GROUP * job.tiles_p;
+    const int grp = t / per_group, in = t - grp * per_group;
+    const int width = min(TILE_GROUP, job.tiles_q - grp * TILE_GROUP);
+    tp = in / width;
+    tq = grp * TILE_GROUP + in - tp * width;
+}
 
-    f32x4 acc[F][F], total[F][F];
-#pragma unroll
-    for (int i = 0; i < F; ++i)
-#pragma unroll
-        for (int j = 0; j < F; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+__device__ __forceinline__ void meet() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's reads and writes of LDS are done
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+}
 
-    f32x4 ra[L], rw[L];
-    const float* pa[L];
-    const float* pw[L];
-#pragma unroll
-    for (int i = 0; i < L; ++i) {
-        const int row = (tid + 256 * i) >> 3;
-        pa[i] = A + (long)min(m0 + row, M - 1) * K;
-        pw[i] = W + (long)min(n0 + row, N - 1) * K;
+#define PAST 0x7f000000  // an offset past the end of every tile's rows: such loads give zeros
+
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t buffer_of(const float* p, long values) {
+    return __builtin_amdgcn_make_buffer_rsrc((void*)p, 0, (int)(values * 4), 0x00020000);
+}
+
+static constexpr __host__ __device__ int lds_bytes(int FP, int FQ) { return 2 * 3 * (64 * FP + 32 * FQ) * 64; }
+
+template <int FP, int FQ, int ROWS>
+__global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(F32Tiles job, F32Epilogue epi) {
+    static_assert(lds_bytes(FP, FQ) <= 160 * 1024 && FP * FQ * 8192 <= lds_bytes(FP, FQ), "the blocks and the sums must fit LDS");
+    constexpr int TP = 64 * FP, TQ = 32 * FQ, PLANE = (TP + TQ) * 64, BUF = 3 * PLANE, IP = FP / 2;
+    extern __shared__ __attribute__((aligned(1024))) char lds[];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, c4 = lane >> 4, wp = wave & 3, wq = wave >> 2;
+    const int M = job.M, N = job.N, K = job.K;
+    const int tiles = job.tiles_p * job.tiles_q, nb = k_blocks(K), sb = seg_blocks(K), used = segments(K);
+    // which tile, which segments: workgroups go to the eight dies in turn, each die takes a run of tiles
+    int t, s0 = 0, s1 = used, rest = -1;
+    const int whole8 = (job.whole + 7) >> 3;
+    if ((int)blockIdx.x < whole8 * 8) {
+        t = (blockIdx.x & 7) * whole8 + (blockIdx.x >> 3);
+        if (t >= job.whole) return;
+    } else {
+        const int R = tiles - job.whole, all = R * job.share, per = (all + 7) >> 3;
+        const int i = blockIdx.x - whole8 * 8, at = (i & 7) * per + (i >> 3);
+        if (at >= all) return;
+        const int range = at / R;
+        rest = at - range * R;
+        t = job.whole + rest;
+        s0 = range * used / job.share;
+        s1 = (range + 1) * used / job.share;
     }
-    const int kc = 4 * (tid & 7);
-    auto fetch = [&](int b) {  // blocks b and b + 1
-        const int k = 16 * b + kc;
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            ra[i] = load4<ROW_ELEMENTS>(pa[i], k, K);
-            rw[i] = load4<ROW_ELEMENTS>(pw[i], k, K);
-        }
-    };
-    auto stage = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            const int at = ((tid + 256 * i) >> 3) * PITCH + kc;
-            *(f32x4*)&As[buf][at] = ra[i];
-            *(f32x4*)&Ws[buf][at] = rw[i];
-        }
-    };
-    auto store_all = [&](const f32x4 (&v)[F][F], float* to, bool last) {
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j) {
-                const int n = n0 + wn + 16 * i + kq, m = m0 + wm + 16 * j + r16;
-                if (m >= M) continue;
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (n + e < N) to[(long)m * N + n + e] = last ? finish(v[i][j][e], epi, n + e, (long)m * N + n + e) : v[i][j][e];
-            }
-    };
-    if (b_first < b_last) {
-        fetch(b_first);
-        stage(0);
-        __syncthreads();
-    }
-    int left = sb, segs = 0, buf = 0;  // blocks left of the segment, segments finished
-    for (int b = b_first; b < b_last; b += 2, buf ^= 1) {
-        const bool more = b + 2 < b_last;
-        if (more) fetch(b + 2);
+    int tp, tq;
+    tile_at(job, t, tp, tq);
+    const int n0 = tp * TP, m0 = tq * TQ;
+    const int b0 = s0 * sb, b1 = min(nb, s1 * sb);
+
+    // What a thread brings of a block: eight elements of IP rows of W and, in the first 2 FQ waves, of a row of A.  Rows past the
+    // last one lie past the buffer's end and give zeros, as do elements past K.
+    const int row = threadIdx.x >> 2, kq = 4 * (threadIdx.x & 3);
+    const bool has_x = wave < 2 * FQ;
+    const __amdgpu_buffer_rsrc_t rw = buffer_of(job.W + (long)n0 * K, (long)min(TP, N - n0) * K);
+    const __amdgpu_buffer_rsrc_t rx = buffer_of(job.A + (long)m0 * K, (long)min(TQ, M - m0) * K);
+    const int at_row = (row * K + kq) * 4;
+    const int to = row * 64 + (((threadIdx.x & 3) ^ (-(row >> 2) & 3)) * 16);
+    f32x4 v[IP + 1][2];
+    auto fetch = [&](int i, int b) __attribute__((always_inline)) {
+        if (i == IP && !has_x) return;
+        const int k = BK * min(b, nb - 1);  // past the last block: that one again, not used
+        const __amdgpu_buffer_rsrc_t from = i == IP ? rx : rw;
 #pragma unroll
         for (int h = 0; h < 2; ++h) {
-            if (b + h < b_last) {
-                f32x4 w[F], x[F];
-#pragma unroll
-                for (int i = 0; i < F; ++i) {
-                    w[i] = *(const f32x4*)&Ws[buf][(wn + 16 * i + r16) * PITCH + 16 * h + kq];
-                    x[i] = *(const f32x4*)&As[buf][(wm + 16 * i + r16) * PITCH + 16 * h + kq];
-                }
-#pragma unroll
-                for (int j = 0; j < 4; ++j)
-#pragma unroll
-                    for (int i = 0; i < F; ++i)
-#pragma unroll
-                        for (int c = 0; c < F; ++c)
-                            acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[i][3 - j], x[c][3 - j], acc[i][c], 0, 0, 0);
-                if (--left == 0 || b + h + 1 == b_last) {  // the segment ends: its sum joins the others in their order
-                    if (SPLIT) {
-                        store_all(acc, C + (long)(s0 + segs) * M * N, false);
-                    } else if (segs == 0) {
-#pragma unroll
-                        for (int i = 0; i < F; ++i)
-#pragma unroll
-                            for (int c = 0; c < F; ++c) total[i][c] = acc[i][c];
-                    } else {
-#pragma unroll
-                        for (int i = 0; i < F; ++i)
-#pragma unroll
-                            for (int c = 0; c < F; ++c)
-#pragma unroll
-                                for (int e = 0; e < 4; ++e) total[i][c][e] += acc[i][c][e];
-                    }
-#pragma unroll
-                    for (int i = 0; i < F; ++i)
-#pragma unroll
-                        for (int c = 0; c < F; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-                    ++segs;
-                    left = sb;
-                }
-            }
-        }
-        if (more) {
-            stage(buf ^ 1);  // the other buffer: everyone is past reading it since the last barrier
-            __syncthreads();
-        }
-    }
-    if (!SPLIT) store_all(total, C, true);
-}
-
-// The same tiles where rows can be read sixteen bytes at a time (rows sixteen-byte aligned, K a multiple of 4), loads going
-// straight to LDS.  A row of a tile is 32 elements of K, 128 bytes without a gap: sixteen bytes c of row r lie at place
-// c ^ (r % 8), so that the eight lanes that read together cover every bank once.
-//
-// What bounds it is the matrix instruction (32 cycles each); the kernel above, which stages through registers and reads a
-// block's operands right before their products, keeps it busy 80 % of the time a workgroup is there.  Here operands of a
-// block are read while the block before is multiplied, and the loads of a step have the whole step before it to arrive:
-// 8,192 x 8,192 x 4,096 124 -> 139 TFLOP/s, 2,053 rows by 4,544 x 4,544 90 -> 113, by 18,176 x 4,544 110 -> 131.
-// TAIL: K is no multiple of 16, what a block holds past it has to be zero.
-
-// sixteen bytes a lane from byte `at` of an array of `bytes` into LDS, one lane after the other; zeros from its end on
-__device__ __forceinline__ void to_lds(const float* src, int bytes, float* dst, int at) {
-    const __amdgpu_buffer_rsrc_t r = __builtin_amdgcn_make_buffer_rsrc((void*)src, 0, bytes, 0x00020000);
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 16, at, 0, 0, 0);
-}
-
-template <int T, bool TAIL, bool SPLIT>
-__global__ __launch_bounds__(256, 2) void gemm_f32_stream_kernel(float* __restrict__ C, const float* __restrict__ A,
-                                                                 const float* __restrict__ W, F32Epilogue epi, int M, int N,
-                                                                 int K, int tiles_m, int tiles_n) {
-    constexpr int F = T / 32;       // tiles of sixteen rows per wave and side
-    constexpr int L = T * 8 / 256;  // sixteen-byte loads per thread and side
-    // A's rows, then W's; two arrays, so that the compiler sees which of them a load is on its way to
-    __shared__ __attribute__((aligned(1024))) float lds0[2 * T * BK];
-    __shared__ __attribute__((aligned(1024))) float lds1[2 * T * BK];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r16 = lane & 15, kq = 4 * (lane >> 4);
-    const int tiles = tiles_m * tiles_n;
-    const int per = (tiles + 7) / 8;
-    const int tile = (blockIdx.x & 7) * per + (blockIdx.x >> 3);
-    if ((int)(blockIdx.x >> 3) >= per || tile >= tiles) return;
-    const int m0 = (tile % tiles_m) * T, n0 = (tile / tiles_m) * T;
-    const int wn = (wave & 1) * (T / 2), wm = (wave >> 1) * (T / 2);
-    const int nb = (K + 15) / 16, sb = seg_blocks(K);
-    const int used = (nb + sb - 1) / sb;
-    const int s0 = SPLIT ? (int)((long)blockIdx.y * used / gridDim.y) : 0;
-    const int s1 = SPLIT ? (int)((long)(blockIdx.y + 1) * used / gridDim.y) : used;
-    const int b_first = s0 * sb, b_last = min(nb, s1 * sb);
-
-    f32x4 acc[F][F], total[F][F];
-#pragma unroll
-    for (int i = 0; i < F; ++i)
-#pragma unroll
-        for (int j = 0; j < F; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-    const float* at_a = A + (long)m0 * K;
-    const float* at_w = W + (long)n0 * K;
-    const int bytes_a = min(T, M - m0) * K * 4, bytes_w = min(T, N - n0) * K * 4;
-    const int trow = tid >> 3, kc = 4 * ((tid & 7) ^ (trow & 7));
-    // blocks b and b + 1; rows past the last are zeros, what the second block holds past K is not used; past b_last nothing is read
-    auto fetch = [&](float* buf, int b) __attribute__((always_inline)) {
-        const int k = 16 * b + kc;
-#pragma unroll
-        for (int i = 0; i < L; ++i) {
-            const int at = TAIL && k >= K ? -16 : ((trow + 32 * i) * K + k) * 4;
-            to_lds(at_a, b < b_last ? bytes_a : 0, buf + (32 * i + 8 * wave) * BK, at);
-            to_lds(at_w, b < b_last ? bytes_w : 0, buf + (T + 32 * i + 8 * wave) * BK, at);
-        }
-    };
-    f32x4 w[2][F], x[2][F];
-    const int place[2] = {4 * ((lane >> 4) ^ (r16 & 7)), 4 * ((4 + (lane >> 4)) ^ (r16 & 7))};
-    auto read = [&](const float* buf, int h) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < F; ++i) {
-            x[h][i] = *(const f32x4*)&buf[(wm + 16 * i + r16) * BK + place[h]];
-            w[h][i] = *(const f32x4*)&buf[(T + wn + 16 * i + r16) * BK + place[h]];
-        }
-    };
-    auto store_all = [&](const f32x4 (&v)[F][F], float* to, bool last) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < F; ++i)
-#pragma unroll
-            for (int j = 0; j < F; ++j) {
-                const int n = n0 + wn + 16 * i + kq, m = m0 + wm + 16 * j + r16;
-                if (m >= M) continue;
+            const int at = at_row + (i == IP ? 0 : i * 512 * K);
+            if (ROWS == ROW_ELEMENTS) {
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
-                    if (n + e < N) to[(long)m * N + n + e] = last ? finish(v[i][j][e], epi, n + e, (long)m * N + n + e) : v[i][j][e];
-            }
-    };
-    int left = sb, segs = 0;  // blocks left of the segment, segments finished
-    auto multiply = [&](int h, int b) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-#pragma unroll
-            for (int i = 0; i < F; ++i)
-#pragma unroll
-                for (int c = 0; c < F; ++c)
-                    acc[i][c] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[h][i][3 - j], x[h][c][3 - j], acc[i][c], 0, 0, 0);
-        if (--left == 0 || b + 1 == b_last) {  // the segment ends: its sum joins the others in their order
-            if (SPLIT) {
-                store_all(acc, C + (long)(s0 + segs) * M * N, false);
+                    v[i][h][e] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(from, k + kq + 16 * h + e < K ? at + 4 * e : PAST, (k + 16 * h) * 4, 0));
             } else {
-                const bool first = segs == 0;
+                v[i][h] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, ROWS == ROW_WHOLE || k + kq + 16 * h < K ? at : PAST, (k + 16 * h) * 4, 0));
+            }
+        }
+    };
+    auto stage = [&](int i, int buf) __attribute__((always_inline)) {
+        if (i == IP && !has_x) return;
+        const Parts s = split8(v[i][0], v[i][1]);
+        char* at = lds + buf + (i == IP ? TP * 64 : i * 8192) + to;
 #pragma unroll
-                for (int i = 0; i < F; ++i)
+        for (int p = 0; p < 3; ++p) *(bf16x8*)(at + p * PLANE) = s.part[p];
+    };
+
+    f32x4 acc[FP][FQ], total[FP][FQ];
 #pragma unroll
-                    for (int c = 0; c < F; ++c)
+    for (int i = 0; i < FP; ++i)
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) total[i][c][e] = first ? acc[i][c][e] : total[i][c][e] + acc[i][c][e];
+        for (int j = 0; j < FQ; ++j) acc[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    const int in_row = r16 * 64 + ((c4 ^ (-(r16 >> 2) & 3)) * 16);
+    const int at_w = wp * FP * 1024 + in_row, at_x = TP * 64 + wq * FQ * 1024 + in_row;
+    bf16x8 w[FP][3], x[2][3];
+    auto read_w = [&](int buf, int p) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < FP; ++i) w[i][p] = *(const bf16x8*)(lds + buf + p * PLANE + at_w + i * 1024);
+    };
+    auto read_x = [&](int buf, int j, int set) __attribute__((always_inline)) {
+#pragma unroll
+        for (int p = 0; p < 3; ++p) x[set][p] = *(const bf16x8*)(lds + buf + p * PLANE + at_x + j * 1024);
+    };
+    auto multiply = [&](int j, int set, int term) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < FP; ++i)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[i][term_w(term)], x[set][term_x(term)], acc[i][j], 0, 0, 0);
+    };
+    f32x4* out = nullptr;
+    if (rest >= 0) out = reinterpret_cast<f32x4*>(job.part) + (((long)s0 * (tiles - job.whole) + rest) * 8 + wave) * (FP * FQ * 64) + lane;
+    const long out_step = (long)(tiles - job.whole) * 8 * FP * FQ * 64;
+
+    int left = sb, cur = 0;
+    // a block; `set`: where column 0's parts are
+    auto block = [&](int b, int set) __attribute__((always_inline)) {
+        const int nxt = BUF - cur;
+#pragma unroll
+        for (int j = 0; j < FQ; ++j) {
+            const int s = (set + j) & 1;
+            __builtin_amdgcn_sched_barrier(0);
+            if (j + 1 < FQ) read_x(cur, j + 1, s ^ 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i <= IP; ++i)
+                if (i == j || (i > j && j >= FQ - 2)) {
+                    if (FQ > 1 && j == FQ - 1) continue;
+                    stage(i, nxt);
+                    fetch(i, b + 2);
+                }
+            if (j == FQ - 1) {
+                meet();
+                read_x(nxt, 0, s ^ 1);
+            }
+            __builtin_amdgcn_s_setprio(1);  // whoever multiplies goes first: 4 % at 8,192 x 8,192 x 4,096
+#pragma unroll
+            for (int term = 0; term < TERMS; ++term) {
+                multiply(j, s, term);
+                if (j == FQ - 1 && (term == 0 || term == 2 || term == 5)) {
+                    __builtin_amdgcn_sched_barrier(0);
+                    read_w(nxt, term == 0 ? 2 : term == 2 ? 1 : 0);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+            __builtin_amdgcn_s_setprio(0);
+        }
+        cur = nxt;
+        if (--left == 0 || b + 1 == b1) {  // the segment ends: its sum joins the others in their order
+            if (rest >= 0) {
+#pragma unroll
+                for (int j = 0; j < FQ; ++j)
+#pragma unroll
+                    for (int i = 0; i < FP; ++i) out[(j * FP + i) * 64] = acc[i][j];
+                out += out_step;
+            } else if (b < sb) {
+#pragma unroll
+                for (int i = 0; i < FP; ++i)
+#pragma unroll
+                    for (int j = 0; j < FQ; ++j) total[i][j] = acc[i][j];
+            } else {
+#pragma unroll
+                for (int i = 0; i < FP; ++i)
+#pragma unroll
+                    for (int j = 0; j < FQ; ++j) total[i][j] += acc[i][j];
             }
 #pragma unroll
-            for (int i = 0; i < F; ++i)
+            for (int i = 0; i < FP; ++i)
 #pragma unroll
-                for (int c = 0; c < F; ++c) acc[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
-            ++segs;
+                for (int j = 0; j < FQ; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
             left = sb;
         }
     };
-    // Blocks b and b + 1 out of `cur`.  Everyone has read all of it when its second block is multiplied: then it takes the loads
-    // of the step after next, and the next step's first block is read.
-    auto step = [&](float* cur, const float* next, int b) __attribute__((always_inline)) {
-        read(cur, 1);
-        __builtin_amdgcn_sched_barrier(0);
-        if (b < b_last) multiply(0, b);
-        __builtin_amdgcn_sched_barrier(0);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0x0070);  // this wave's reads of `cur` are done, its loads into `next` have landed
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        fetch(cur, b + 4);
-        read(next, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        if (b + 1 < b_last) multiply(1, b + 1);
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    if (b_first < b_last) {
-        fetch(lds0, b_first);
-        fetch(lds1, b_first + 2);
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_s_waitcnt(0x0070);
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        read(lds0, 0);
-        for (int b = b_first; b < b_last; b += 4) {
-            step(lds0, lds1, b);
-            step(lds1, lds0, b + 2);
-        }
-        __builtin_amdgcn_s_waitcnt(0x0070);  // nothing is on its way to LDS when the workgroup ends
+#pragma unroll
+    for (int i = 0; i <= IP; ++i) fetch(i, b0);
+#pragma unroll
+    for (int i = 0; i <= IP; ++i) {
+        stage(i, 0);
+        fetch(i, b0 + 1);
     }
-    if (!SPLIT) store_all(total, C, true);
+    meet();
+    read_x(0, 0, 0);
+    read_w(0, 2);
+    read_w(0, 1);
+    read_w(0, 0);
+    if (FQ & 1) {
+        for (int b = b0; b < b1; b += 2) {
+            block(b, 0);
+            if (b + 1 < b1) block(b + 1, 1);
+        }
+    } else {
+        for (int b = b0; b < b1; ++b) block(b, 0);
+    }
+    if (rest >= 0) return;
+
+    meet();  // everyone is past reading the last block: a wave's sums change hands through LDS, fragment by fragment
+    f32x4* mine = reinterpret_cast<f32x4*>(lds) + wave * (FP * FQ * 64) + lane;
+#pragma unroll
+    for (int j = 0; j < FQ; ++j)
+#pragma unroll
+        for (int i = 0; i < FP; ++i) mine[(j * FP + i) * 64] = total[i][j];
+#pragma unroll 1
+    for (int f = 0; f < FP * FQ; ++f) {
+        const int m16 = m0 + (wq * FQ + f / FP) * 16, n16 = n0 + (wp * FP + f % FP) * 16;
+        f32x4 u = mine[f * 64];
+        if (any_not_finite(u)) u = plain_fragment<ROWS>(u, job.A, job.W, m16, n16, M, N, K);
+        const int m = m16 + r16, n = n16 + 4 * c4;
+        if (m < M && n < N) store4(job.C, u, epi, m, n, N, N);
+    }
 }
 
-// the segments' sums added in order, and the epilogue
-__global__ void gemm_f32_add_kernel(float* __restrict__ C, const float* __restrict__ part, F32Epilogue epi, int segs, long MN, int N) {
-    const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= MN) return;
-    float v = part[i];
-    for (int s = 1; s < segs; ++s) v += part[(long)s * MN + i];
-    C[i] = finish(v, epi, (int)(i % N), i);
+// the cut tiles: the segments' sums added in order, and the epilogue; a wave has a fragment
+template <int FP, int FQ, int ROWS>
+__global__ __launch_bounds__(256) void gemm_f32_add_kernel(F32Tiles job, F32Epilogue epi) {
+    const int R = job.tiles_p * job.tiles_q - job.whole, used = segments(job.K);
+    const int lane = threadIdx.x & 63, at = blockIdx.x * 4 + (threadIdx.x >> 6);
+    const int rest = at / (8 * FP * FQ), wave = at / (FP * FQ) % 8, j = at % (FP * FQ) / FP, i = at % FP;
+    if (rest >= R) return;
+    int tp, tq;
+    tile_at(job, job.whole + rest, tp, tq);
+    const f32x4* from = reinterpret_cast<const f32x4*>(job.part) + (long)at * 64 + lane;
+    const long step = (long)R * 8 * FP * FQ * 64;
+    f32x4 p[SEGS];
+#pragma unroll
+    for (int s = 0; s < SEGS; ++s) p[s] = from[min(s, used - 1) * step];
+    f32x4 v = p[0];
+#pragma unroll
+    for (int s = 1; s < SEGS; ++s)
+        if (s < used) v += p[s];
+    const int m16 = tq * 32 * FQ + ((wave >> 2) * FQ + j) * 16, n16 = tp * 64 * FP + ((wave & 3) * FP + i) * 16;
+    if (any_not_finite(v)) v = plain_fragment<ROWS>(v, job.A, job.W, m16, n16, job.M, job.N, job.K);
+    const int m = m16 + (lane & 15), n = n16 + 4 * (lane >> 4);
+    if (m < job.M && n < job.N) store4(job.C, v, epi, m, n, job.N, job.N);
 }
 
-// How a product runs: the tile's side (0: the kernel for few rows) and over how many workgroups a tile's segments are shared.
-static void f32_plan(int M, int N, int K, int* tile, int* share) {
-    *tile = 0, *share = 1;
-    // 33 rows by 4,544 x 4,544: 61 us with the kernel for few rows, 36 with shared tiles; 17 rows: 35 and 51; 33 rows by 256 x
-    // 512, whose segments are too short to be shared: 7 and 13
-    if (M <= (K < SHARE_K ? 2 * SKINNY_ROWS : SKINNY_ROWS)) return;
-    const int cus = 256;
-    auto tiles = [&](long t) { return ((M + t - 1) / t) * ((N + t - 1) / t); };
-    auto rounds = [&](long n) { return (double)((n + cus - 1) / cus); };
-    // time of a round: a tile of 128 is four of 64, which read twice as much per product (8,192 x 8,192 x 4,096: 139 and
-    // 134 TFLOP/s; 2,053 x 4,544 x 4,544, where 128 leaves the last round half empty: 101 and 119)
-    const double big = 4.0 * rounds(tiles(128)), small = 1.04 * rounds(tiles(64));
-    *tile = big <= small ? 128 : 64;
-    const int used = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
-    if (*tile == 64 && K >= SHARE_K)  // a chip that is not filled twice: share the segments out
-        while (*share < used && tiles(64) * *share < 2 * cus) *share *= 2;
-    if (*share > used) *share = used;
+// How a product runs: few rows (fp = 0), or tiles of 64 fp rows of W by 32 fq rows of A, the first `whole` of them over all of
+// K, the segments of each of the others shared out over `share` workgroups.  What a choice takes, in microseconds, is put
+// together from measurements at K = 1,024, 4,096 and 8,192 (256 compute units, 64 to 1,024 tiles):
+//   a block of 32 elements of K: `full` with a tile for every compute unit, `half` with a tile for at most half of them, `pair`
+//     with two on a unit, where two fit (0: they do not);
+//   a tile's start and end: `ends`, `cut` for a tile whose K is cut (the difference: tiles of 256 x 128 keep part of the segments'
+//     sums in memory, which costs them 2.5 us a segment);
+//   sums of cut tiles: 4.5 us for the second launch and 0.25 us a megabyte.
+// The smallest sum wins.
+struct F32Plan {
+    int fp, fq, whole, share;
+    double us;
+};
+
+struct F32Costs {
+    double half, full, pair, ends, cut;
+};
+static const F32Costs costs[2][4] = {
+    {{0.56, 0.57, 0.93, 6.0, 6.0}, {0.73, 0.77, 1.39, 7.4, 7.4}, {0.94, 1.01, 0.0, 8.8, 8.8}, {1.10, 1.23, 0.0, 10.5, 10.0}},
+    {{0.92, 0.95, 0.0, 8.0, 8.0}, {1.19, 1.32, 0.0, 10.5, 10.5}, {1.52, 1.76, 0.0, 12.6, 12.0}, {1.84, 2.17, 0.0, 32.0, 12.5}},
+};
+
+// Which products the kernel for few rows has.  Measured, microseconds of few rows and of the best tiles:
+//   N x K            1 row            8 rows           16 rows          17 rows          32 rows
+//   1,024 x 1,024     7.3 /   9.9      7.5 /  10.0      7.7 /  10.0      8.5 /   9.8     10.4 /   9.8
+//   4,096 x 1,024     7.8 /  11.9      8.8 /  12.0      9.7 /  12.1     10.4 /  12.2     12.1 /  11.9
+//   2,048 x 2,048     8.4 /  12.4     10.0 /  12.6     11.5 /  12.6     12.9 /  12.8     16.5 /  12.9
+//   4,544 x 4,544    21.0 /  25.9     23.5 /  25.9     27.0 /  26.3     31.6 /  26.3     36.8 /  26.8
+//   18,176 x 4,544   67.9 /  76.4     74.9 /  76.6     85.9 /  77.5     98.0 /  77.5      116 /  79.3
+//   32,768 x 2,048   61.2 /  61.6     66.3 /  61.9     72.2 /  62.7     80.2 /  63.5     90.3 /  64.3
+//   65,024 x 4,544    213 /   198      237 /   198      266 /   199      297 /   200      344 /   203
+// With a short K, whose segments are a block or two, rows up to 64: 256 x 512 33 rows 8.6 and 9.9, 64 rows 10.5 and 10.0.
+// Tiles address a row by 32-bit offsets (MOST_K).
+static bool few_rows(int M, int N, int K) {
+    if (K > MOST_K) return true;
+    if (K < 1024) return M <= 64;
+    if (K < 2048) return M <= 32;
+    return M <= 16 && N < 32768 && (M <= 12 || (long)N * K < (1L << 24));
 }
 
-// 32-bit values of scratch memory that pta_gemm_f32 needs for this product (0: none)
-extern "C" long pta_gemm_f32_scratch(int M, int N, int K) {
-    if (M <= 0 || N <= 0 || K <= 0) return 0;
-    int tile, share;
-    f32_plan(M, N, K, &tile, &share);
-    if (share <= 1) return 0;
-    return (long)(((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K)) * M * N;
+static F32Plan f32_plan(int M, int N, int K) {
+    F32Plan best{0, 0, 0, 1, 1e30};
+    if (few_rows(M, N, K)) return best;
+    const int units = 256, used = segments(K), blocks = k_blocks(K);
+    for (int fp = 2; fp <= 4; fp += 2)
+        for (int fq = 1; fq <= 4; ++fq) {
+            const F32Costs& c = costs[fp / 2 - 1][fq - 1];
+            const long tiles = (long)((N + 64 * fp - 1) / (64 * fp)) * ((M + 32 * fq - 1) / (32 * fq));
+            const long slots = c.pair > 0.0 ? 2 * units : units;
+            // `groups` workgroups, each on b blocks of K
+            auto time = [&](long groups, int b, double ends) {
+                const double round = b * (c.pair > 0.0 ? c.pair : c.full) + ends;
+                double us = (double)(groups / slots) * round;
+                const long left = groups % slots;
+                if (left > units) us += round;
+                else if (left) us += b * (c.half + (c.full - c.half) * (left > units / 2 ? 2.0 * left / units - 1.0 : 0.0)) + ends;
+                return us;
+            };
+            auto consider = [&](long whole, int share, double us) {
+                if (us < best.us) best = F32Plan{fp, fq, (int)whole, share, us};
+            };
+            consider(tiles, 1, time(tiles, blocks, c.ends));
+            const long left = tiles % slots;
+            if (!left) continue;
+            const double body = time(tiles - left, blocks, c.ends);
+            for (int share = 2; share <= used; ++share) {
+                const int each = (used + share - 1) / share * seg_blocks(K);  // of the workgroup with the most segments
+                if (left * used * fp * fq * 2048 > MOST_SUMS) break;
+                consider(tiles - left, share, body + time(left * share, each, c.cut) + 4.5 + 0.25 * left * used * fp * fq * 8192e-6);
+            }
+        }
+    return best;
 }
 
 template <int ROWS>
-static void launch_few(float* C, const float* A, const float* W, const F32Epilogue& epi, int M, int N, int K, hipStream_t s) {
+static void launch_few(float* C, const float* A, const float* W, F32Epilogue epi, int rows, int N, int K, hipStream_t s) {
     // whole rounds of the 256 compute units, up to 32 rows of W each; small matrices: four rows a workgroup
     int groups = 256 * ((N + 256 * 32 - 1) / (256 * 32));
     if (groups > (N + 3) / 4) groups = (N + 3) / 4;
     const bool two = (N + groups - 1) / groups > 16;
 #define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), dim3(groups), dim3(512), 0, s, C, A, W, epi, M, N, K)
-    if (M <= 16) { if (two) FEW(1, 2, 4); else FEW(1, 1, 4); }
-    else if (M <= 32) { if (two) FEW(2, 2, 4); else FEW(2, 1, 4); }
-    else { if (two) FEW(4, 2, 2); else FEW(4, 1, 2); }
+    for (int at = 0; at < rows; at += 64) {  // more than 64 rows: where tiles cannot address K
+        const int M = rows - at < 64 ? rows - at : 64;
+        if (M <= 16) { if (two) FEW(1, 2, 2); else FEW(1, 1, 2); }
+        else if (M <= 32) { if (two) FEW(2, 2, 2); else FEW(2, 1, 2); }
+        else { if (two) FEW(4, 2, 1); else FEW(4, 1, 1); }
+        A += 64L * K, C += 64L * N;
+        if (epi.add1) epi.add1 += 64L * N;
+        if (epi.add2) epi.add2 += 64L * N;
+    }
 #undef FEW
 }
 
-static void launch_tiles(float* C, float* scratch, const float* A, const float* W, const F32Epilogue& epi, int M, int N, int K,
-                         int tile, int share, bool vec, hipStream_t s) {
-    const int tm = (M + tile - 1) / tile, tn = (N + tile - 1) / tile;
-    const int groups = 8 * ((tm * tn + 7) / 8);
-    // offsets within a tile's rows are 32-bit bytes
-    const bool stream = vec && (long)(128 + 2) * K * 4 < (1L << 31);
-#define LAUNCH(KERNEL, SPLIT, OUT) \
-    hipLaunchKernelGGL(KERNEL, dim3(groups, SPLIT ? share : 1), dim3(256), 0, s, OUT, A, W, epi, M, N, K, tm, tn)
-#define TILE(T, SPLIT, OUT) \
-    do { \
-        if (!stream) LAUNCH((gemm_f32_tile_kernel<T, SPLIT>), SPLIT, OUT); \
-        else if (K % 16) LAUNCH((gemm_f32_stream_kernel<T, true, SPLIT>), SPLIT, OUT); \
-        else LAUNCH((gemm_f32_stream_kernel<T, false, SPLIT>), SPLIT, OUT); \
-    } while (0)
-    if (share > 1) TILE(64, true, scratch);
-    else if (tile == 128) TILE(128, false, C);
-    else TILE(64, false, C);
-#undef TILE
-#undef LAUNCH
-    if (share > 1) {
-        const long mn = (long)M * N;
-        const int segs = ((K + 15) / 16 + seg_blocks(K) - 1) / seg_blocks(K);
-        hipLaunchKernelGGL(gemm_f32_add_kernel, dim3((unsigned)((mn + 255) / 256)), dim3(256), 0, s, C, scratch, epi, segs, mn, N);
+template <int FP, int FQ, int ROWS>
+static int launch_tiles(const F32Tiles& job, const F32Epilogue& epi, hipStream_t s) {
+    const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(gemm_f32_tile_kernel<FP, FQ, ROWS>),
+                                                  hipFuncAttributeMaxDynamicSharedMemorySize, lds_bytes(FP, FQ));
+    PTA_REQUIRE(raised == hipSuccess, "gemm_f32: %d bytes of LDS were refused", lds_bytes(FP, FQ));
+    const int R = job.tiles_p * job.tiles_q - job.whole;
+    const int groups = (job.whole + 7) / 8 * 8 + (R * job.share + 7) / 8 * 8;
+    hipLaunchKernelGGL((gemm_f32_tile_kernel<FP, FQ, ROWS>), dim3(groups), dim3(512), lds_bytes(FP, FQ), s, job, epi);
+    if (R > 0) hipLaunchKernelGGL((gemm_f32_add_kernel<FP, FQ, ROWS>), dim3(R * 2 * FP * FQ), dim3(256), 0, s, job, epi);
+    return pta_check_launch("gemm_f32");
+}
+
+template <int ROWS>
+static int launch_plan(const F32Plan& p, const F32Tiles& job, const F32Epilogue& epi, hipStream_t s) {
+    if (p.fp == 0) {
+        launch_few<ROWS>(job.C, job.A, job.W, epi, job.M, job.N, job.K, s);
+        return pta_check_launch("gemm_f32");
     }
+    switch (p.fp * 8 + p.fq) {
+        case 17: return launch_tiles<2, 1, ROWS>(job, epi, s);
+        case 18: return launch_tiles<2, 2, ROWS>(job, epi, s);
+        case 19: return launch_tiles<2, 3, ROWS>(job, epi, s);
+        case 20: return launch_tiles<2, 4, ROWS>(job, epi, s);
+        case 33: return launch_tiles<4, 1, ROWS>(job, epi, s);
+        case 34: return launch_tiles<4, 2, ROWS>(job, epi, s);
+        case 35: return launch_tiles<4, 3, ROWS>(job, epi, s);
+        default: return launch_tiles<4, 4, ROWS>(job, epi, s);
+    }
+}
+
+static long scratch_values(const F32Plan& p, int M, int N, int K) {
+    if (p.fp == 0) return 0;
+    const long tiles = (long)((N + 64 * p.fp - 1) / (64 * p.fp)) * ((M + 32 * p.fq - 1) / (32 * p.fq));
+    return (tiles - p.whole) * segments(K) * p.fp * p.fq * 2048;
+}
+
+// 32-bit values of scratch memory that pta_gemm_f32 needs for this product (0: none)
+extern "C" long pta_gemm_f32_scratch(int M, int N, int K) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    return scratch_values(f32_plan(M, N, K), M, N, K);
+}
+
+static int f32_run(F32Plan p, float* C, const float* A, const float* W, const float* bias, const float* add1,
+                   const float* add2, int M, int N, int K, int act, float* scratch, void* stream) {
+    PTA_REQUIRE(C && A && W, "gemm_f32: null pointer");
+    PTA_REQUIRE(pta_act_known(act), "gemm_f32: unknown activation %d", act);
+    PTA_REQUIRE(scratch_values(p, M, N, K) == 0 || scratch, "gemm_f32: this product needs scratch memory (pta_gemm_f32_scratch)");
+    bool wide = N % 4 == 0;
+    for (const void* q : {(const void*)C, (const void*)add1, (const void*)add2, (const void*)scratch}) wide = wide && (uintptr_t)q % 16 == 0;
+    const F32Epilogue epi{bias, add1, add2, act, wide};
+    F32Tiles job{C, scratch, A, W, M, N, K, 0, 0, p.whole, p.share};
+    if (p.fp) {
+        job.tiles_q = (M + 32 * p.fq - 1) / (32 * p.fq);
+        job.tiles_p = (N + 64 * p.fp - 1) / (64 * p.fp);
+    }
+    const bool vec = K % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
+    hipStream_t s = (hipStream_t)stream;
+    if (vec && K % BK == 0) return launch_plan<ROW_WHOLE>(p, job, epi, s);
+    if (vec) return launch_plan<ROW_VECTORS>(p, job, epi, s);
+    return launch_plan<ROW_ELEMENTS>(p, job, epi, s);
 }
 
 extern "C" int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, const float* add1,
                             const float* add2, int M, int N, int K, int act, float* scratch, void* stream) {
     PTA_REQUIRE(M > 0 && N > 0 && K > 0, "gemm_f32: sizes must be positive (M=%d N=%d K=%d)", M, N, K);
-    PTA_REQUIRE(C && A && W, "gemm_f32: null pointer");
-    PTA_REQUIRE(pta_act_known(act), "gemm_f32: unknown activation %d", act);
     PTA_REQUIRE(M <= 65535 * 64, "gemm_f32: M=%d is too large for one launch", M);
-    int tile, share;
-    f32_plan(M, N, K, &tile, &share);
-    PTA_REQUIRE(share <= 1 || scratch, "gemm_f32: this product needs scratch memory (pta_gemm_f32_scratch)");
-    const F32Epilogue epi{bias, add1, add2, act};
-    const bool vec = K % 4 == 0 && (uintptr_t)A % 16 == 0 && (uintptr_t)W % 16 == 0;
-    hipStream_t s = (hipStream_t)stream;
-#define BY_ROWS(FN, ...) (vec && K % 16 == 0 ? FN<ROW_WHOLE>(__VA_ARGS__) : vec ? FN<ROW_VECTORS>(__VA_ARGS__) : FN<ROW_ELEMENTS>(__VA_ARGS__))
-    if (tile == 0) BY_ROWS(launch_few, C, A, W, epi, M, N, K, s);
-    else launch_tiles(C, scratch, A, W, epi, M, N, K, tile, share, vec, s);
-#undef BY_ROWS
-    return pta_check_launch("gemm_f32");
+    return f32_run(f32_plan(M, N, K), C, A, W, bias, add1, add2, M, N, K, act, scratch, stream);
+}
+
+// The same with the choice in the caller's hands, for measuring one against another and for tests of each: fp = 0 for the
+// kernel for few rows, else fp 2 or 4 and fq 1 to 4; `room` 32-bit values at scratch.
+extern "C" int pta_gemm_f32_as(float* C, const float* A, const float* W, const float* bias, const float* add1,
+                               const float* add2, int M, int N, int K, int act, int fp, int fq, int whole, int share,
+                               float* scratch, long room, void* stream) {
+    PTA_REQUIRE(M > 0 && N > 0 && K > 0 && M <= 65535 * 64, "gemm_f32: sizes out of range (M=%d N=%d K=%d)", M, N, K);
+    PTA_REQUIRE(fp == 0 || ((fp == 2 || fp == 4) && fq >= 1 && fq <= 4), "gemm_f32: no tiles of 64 x %d by 32 x %d", fp, fq);
+    const F32Plan p{fp, fq, whole, share, 0.0};
+    if (fp) {
+        const long tiles = (long)((N + 64 * fp - 1) / (64 * fp)) * ((M + 32 * fq - 1) / (32 * fq));
+        PTA_REQUIRE(K <= MOST_K && whole >= 0 && whole <= tiles && share >= 1 && share <= segments(K),
+                    "gemm_f32: %d of %ld tiles whole, %d shares of %d segments", whole, tiles, share, segments(K));
+    }
+    PTA_REQUIRE(scratch_values(p, M, N, K) <= room, "gemm_f32: room for %ld sums, %ld are needed", room, scratch_values(p, M, N, K));
+    return f32_run(p, C, A, W, bias, add1, add2, M, N, K, act, scratch, stream);
 }

@@ -133,6 +133,9 @@ int pta_attn_mfma(void* out, const void* q, const void* k_pool, const void* v_po
 long pta_gemm_f32_scratch(int M, int N, int K);
 int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, const float* add1, const float* add2,
                  int M, int N, int K, int act, float* scratch, void* stream);
+// The same with the choice of kernel in the caller's hands (gemm_f32.hip); room: values that scratch holds.
+int pta_gemm_f32_as(float* C, const float* A, const float* W, const float* bias, const float* add1, const float* add2,
+                    int M, int N, int K, int act, int fp, int fq, int whole, int share, float* scratch, long room, void* stream);
 
 // Attention of 32-bit heads of up to 256 elements, a multiple of 4, on the 32-bit matrix instruction: the arguments of
 // pta_attn_generic, and the step's sequences in the tokens' order (cu_tokens null: every token is taken by itself, in any

@@ -1,5 +1,6 @@
 """The 32-bit kernels alone, against 64-bit references: every way a product runs (few rows, tiles, shared segments) and both
 attention kernels, at the edges of their tiles, and the same bits for a row whichever of them it runs in."""
+import ctypes
 import math
 
 import pytest
@@ -40,6 +41,94 @@ def test_products(N, K):
     for m in (1, 2, 16, 17, 33, 64, 65, 128, 300):
         assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w), plain[:m]), f"{m} rows alone and in a batch"
         assert torch.equal(ops.gemm_f32(a[:m].contiguous(), w, bias, "gelu", a1[:m].contiguous(), a2[:m].contiguous()), full[:m])
+
+
+def _product_as(ops, a, w, fp, fq, whole, share):
+    """The product by tiles of 64 ``fp`` rows of w by 32 ``fq`` rows of a (0: few rows), the first ``whole`` over all of K."""
+    (M, K), N = a.shape, w.shape[0]
+    out = torch.full((M, N), 7.0, device="cuda")
+    scratch = torch.empty(16 << 20, dtype=torch.float32, device="cuda")
+    ops._call("pta_gemm_f32_as", ops._ptr(out), ops._ptr(a), ops._ptr(w), ops._ptr(None), ops._ptr(None), ops._ptr(None), M, N, K, 0,
+              fp, fq, whole, share, ops._ptr(scratch), ctypes.c_long(scratch.numel()), ops._stream())
+    return out
+
+
+def _split_tol(a, w):
+    """What the sums in 32 bits may be off by: as test_products."""
+    scale = ((a.double() ** 2) @ (w.double() ** 2).T.contiguous()).sqrt().max().item()
+    return 8 * 2.0 ** -24 * math.sqrt(a.shape[1]) * scale + 1e-30
+
+
+# K: no last block of 32; a last block; rows of sixteen bytes and not; fewer blocks than segments, as many, and more
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (33, 129, 32), (129, 257, 100), (64, 256, 256), (130, 70, 1044), (257, 300, 2050), (70, 520, 4544)])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_products_by_every_way(M, N, K, offset):
+    """Few rows, every size of tile, tiles over all of K, cut ones and both: the same bits, also off sixteen-byte addresses."""
+    ops = _ops()
+    a, w = (_rand(n * K + 1, seed=i)[offset:offset + n * K].view(n, K) for i, n in enumerate((M, N)))
+    want = _product_as(ops, a, w, 0, 0, 0, 1)
+    assert (want.double() - a.double() @ w.double().T).abs().max().item() <= _split_tol(a, w)
+    blocks = -(-K // 32)
+    segments = -(-blocks // -(-blocks // 8))
+    for fp in (2, 4):
+        for fq in (1, 2, 3, 4):
+            tiles = -(-N // (64 * fp)) * -(-M // (32 * fq))
+            for whole, share in {(tiles, 1), (0, 1), (0, segments), (tiles // 2, segments), (0, (segments + 1) // 2)}:
+                assert torch.equal(_product_as(ops, a, w, fp, fq, whole, share), want), (fp, fq, whole, share)
+
+
+def test_product_of_rows_that_tiles_cannot_address():
+    """Rows too long for 32-bit offsets within a tile go by 64 at a time through the kernel for few rows."""
+    ops = _ops()
+    M, N, K = 70, 3, 0x7f000000 // 1024 + 8
+    g = torch.Generator(device="cuda").manual_seed(0)
+    a, w = torch.randn(M, K, generator=g, device="cuda"), torch.randn(N, K, generator=g, device="cuda")
+    a1 = _rand(M, N)
+    got = ops.gemm_f32(a, w, add1=a1)
+    want = a1.double()
+    for k in range(0, K, 1 << 18):
+        want = want + a[:, k:k + (1 << 18)].double() @ w[:, k:k + (1 << 18)].double().T.contiguous()
+    assert (got.double() - want).abs().max().item() <= 8 * 2.0 ** -24 * K  # sqrt(K) eps times the root of a sum of K squares
+    assert torch.equal(ops.gemm_f32(a[65:].contiguous(), w, add1=a1[65:].contiguous()), got[65:])
+
+
+@pytest.mark.parametrize("way", [(0, 0, 0, 1), (2, 1, 64, 1), (4, 4, 64, 1), (2, 2, 0, 7), (4, 3, 0, 3)])
+def test_products_of_values_without_parts(way):
+    """Infinite and undefined values, values that round to an infinite bfloat16, overflow, tiny and huge rows: what 32-bit
+    arithmetic says of them, and no change to any other row."""
+    ops = _ops()
+    M, N, K = 60, 300, 1040
+    a, w = _rand(M, K), _rand(N, K, seed=1)
+    plain = ops.gemm_f32(a, w)
+    b = a.clone()
+    b[3, 5], b[7, 9], b[9, 100], b[11, 3] = math.inf, math.nan, 3.4e38, -math.inf
+    b[9, :100] *= 1e-10  # the large value alone decides the row, and stays in range where |w| < 1
+    b[9, 101:] *= 1e-10
+    b[13] *= 1e-30
+    b[14] *= 1e34
+    b[15] = 3e38 * torch.sign(w[4])  # overflows in column 4, whose products are all positive
+    v = w.clone()
+    v[20, 3] = 0.0
+    fp, fq, whole, share = way
+    if fp:
+        tiles = -(-N // (64 * fp)) * -(-M // (32 * fq))
+        whole = min(whole, tiles)
+    got = _product_as(ops, b, v, fp, fq, whole, share)
+    want = b.double() @ v.double().T
+    row = got[3]
+    assert torch.equal(row, torch.where(v[:, 5] > 0, math.inf, -math.inf))
+    assert torch.isnan(got[7]).all()
+    small = v[:, 100].abs() < 0.99
+    torch.testing.assert_close(got[9][small].double(), want[9][small], rtol=1e-5, atol=0.0)
+    assert torch.isinf(got[9][v[:, 100].abs() > 1.01]).all()
+    other = torch.arange(N, device="cuda") != 20
+    assert torch.equal(got[11][other], torch.where(v[other, 3] > 0, -math.inf, math.inf)) and torch.isnan(got[11][20])
+    for r in (13, 14):
+        scale = (b[r].double() ** 2).sum().sqrt() * (v.double() ** 2).sum(1).sqrt()
+        assert ((got[r].double() - want[r]).abs() <= 8 * 2.0 ** -24 * math.sqrt(K) * scale).all()
+    assert got[15, 4] == math.inf
+    same = [r for r in range(M) if r not in (3, 7, 9, 11, 13, 14, 15)]
+    assert torch.equal(got[same][:, other], plain[same][:, other])
 
 
 def _attention_case(nh, nkv, d, starts, news, window=0, chunk=0, sink=False, slopes=None, spoil=False):
