@@ -26,7 +26,7 @@ ARCH = "gfx950"
 # ... and matrix-core results go to ordinary vector registers: the kernels here do arithmetic on their
 # accumulators between products, and copies to and from the accumulation registers cost more than they save
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Xclang", "-target-feature", "-Xclang",
-         "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form", "-Wno-unused-command-line-argument"]
+         "-packed-fp32-ops", "-mllvm", "-amdgpu-mfma-vgpr-form", "-mllvm", "-amdgpu-kernarg-preload-count=16", "-Wno-unused-command-line-argument"]
 
 
 def sources():
