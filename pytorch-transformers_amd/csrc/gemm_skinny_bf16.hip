@@ -14,6 +14,7 @@
 // the order of summation never depends on M or on what else is in the batch.
 #include "common.h"
 #include "glu.h"
+#include "lds_stream.h"
 #include "pta_kernels.h"
 #include "qkv_tail.h"
 
@@ -21,11 +22,6 @@
 
 #include <algorithm>
 #include <type_traits>
-
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
 
 union Frag {
     uint4 u;
@@ -94,6 +90,21 @@ __device__ __forceinline__ void compute_stage(const Stage<MT, RT, U>& st, f32x4_
             }
 }
 
+// How `items` (rows of W, pairs of them) are shared out evenly to `groups` workgroups: the first `over` have one more than the others.
+// Made on the host: the division by a number of workgroups was 300 instructions at the start of a launch of few microseconds.
+struct Share {
+    int each, over;
+    Share() = default;
+    Share(int items, int groups) : each(groups > 0 ? items / groups : 0), over(groups > 0 ? items % groups : 0) {}
+    __device__ __forceinline__ int begin(int j) const { return j * each + min(j, over); }
+    __device__ __forceinline__ int end(int j) const { return begin(j) + each + (j < over ? 1 : 0); }
+};
+
+// where a workgroup starts in K, for rows of W a power of two long (gemm_skinny_kernel)
+__device__ __forceinline__ int start_step(int rot_stride, int nsteps) {
+    return rot_stride > 0 ? (int)((unsigned)(blockIdx.x * rot_stride) % (unsigned)nsteps) : 0;
+}
+
 // One product of a launch: a launch may carry two that share M and K (a block's two input projections),
 // so that the second one's workgroups fill the chip while the first one's drain.
 struct SkinnyProblem {
@@ -106,6 +117,7 @@ struct SkinnyProblem {
     int N;
     int act;
     int blocks;  // workgroups of this product
+    Share rows;  // of W, over them (pairs of rows where a launch works on those)
 };
 
 // what follows the product, for one feature: bias, activation, additions
@@ -128,11 +140,14 @@ __device__ __forceinline__ void store_feature(OutT* y, const float* bias, int ac
 // first elements of sixteen pairs as its first row tile and their partners as its second (TAIL 1: whole heads in
 // half-split pairs, or no rotation: pair p is elements p and p + d/2, and four pairs in a row are stored as eight
 // bytes; TAIL 2: any rotation that qkv_tail_pair_elements describes, stored element by element).
-template <int MT, int RT, int U, typename OutT, int TAIL = 0>
+template <int MT, int RT, int U, typename OutT, int TAIL = 0, int D = 0>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, SkinnyProblem pb, int M, int K,
                                                           int rot_stride, QkvTail tail) {
     static_assert(!TAIL || (RT == 2 && MT == 1 && sizeof(OutT) == 2), "the query_key_value tail: two row tiles, sixteen rows of x");
-    extern __shared__ f32x4_t part[];  // [S][RT][MT][64]
+    static_assert(D == 0 || MT == 1, "through LDS: sixteen rows of x");
+    // the waves' sums, [RT][MT][64] each; through LDS they take the place of the waves' rings
+    extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];
+    constexpr int WAVE = D == 0 ? RT * MT * 64 : RowStream<RT, D == 0 ? 1 : D>::RING / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4;
     const bool second = (int)blockIdx.x >= pa.blocks;
@@ -144,28 +159,19 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     const bf16_t* __restrict__ add2 = second ? pb.add2 : pa.add2;
     const int N = second ? pb.N : pa.N, act = second ? pb.act : pa.act;
     // the workgroups of a product share its rows evenly: this one has rows n0 .. n1 - 1, at most 16 * RT
-    const int blocks = second ? pb.blocks : pa.blocks, j = (int)blockIdx.x - (second ? pa.blocks : 0);
-    const int n0 = (int)((long)j * N / blocks), n1 = (int)((long)(j + 1) * N / blocks);
-    const bf16_t* wrow[RT];
+    const int j = (int)blockIdx.x - (second ? pa.blocks : 0);
+    const Share mine = second ? pb.rows : pa.rows;
+    const int n0 = mine.begin(j), n1 = mine.end(j);
     const bool tailed = TAIL && !second;
-    // with the tail: workgroup j has pairs s16*16 .. +15 of segment seg (a head's q, k or v)
+    // with the tail: workgroup j has pairs s16*16 .. +15 of segment seg (a head's q, k or v); their elements are its two row tiles
     const int per_seg = TAIL ? tail.d / 32 : 1, seg = j / per_seg, s16 = j % per_seg;
-    int pair_e[2] = {0, 0};  // the two elements of this lane's pair
-    if (TAIL == 1) {
-        pair_e[0] = s16 * 16 + r;
-        pair_e[1] = pair_e[0] + (tail.d >> 1);
-    } else if (TAIL == 2) {
+    auto tail_row = [&](int i, int t) {  // element t of pair i of the sixteen, within the segment
+        if (TAIL == 1) return s16 * 16 + i + (t & 1) * (tail.d >> 1);
+        int e[2] = {0, 0};
         bool rotated;
-        qkv_tail_pair_elements(tail.rot, tail.d, s16 * 16 + r, pair_e[0], pair_e[1], rotated);
-    }
-#pragma unroll
-    for (int t = 0; t < RT; ++t) {
-        const int row = tailed ? seg * tail.d + pair_e[t & 1] : min(n0 + t * 16 + r, n1 - 1);
-        wrow[t] = W + (long)row * K;
-    }
-    // x through a buffer descriptor whose bounds are the M real rows (0x00020000: 32-bit raw data format)
-    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
-
+        qkv_tail_pair_elements(tail.rot, tail.d, s16 * 16 + i, e[0], e[1], rotated);
+        return t & 1 ? e[1] : e[0];
+    };
     f32x4_t acc[RT][MT];
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -176,25 +182,53 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     // Where a row of W is a power of two long, every workgroup walking K from its start would ask the same few
     // memory channels at the same time (K = 4,096: 13 % slower than K = 4,160).  So each starts `rot_stride`
     // steps after its neighbour.  A feature's order of summation follows from N, K and the launch alone.
-    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
-    Stage<MT, RT, U> s0, s1;
-    load_stage<MT, RT, U>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
-    // the scheduling barriers keep the compiler from sinking a stage's loads down to their first
-    // use, which would shrink what is in flight to a load or two
-    for (int step = wave; step < nsteps; step += 2 * U * S) {
-        load_stage<MT, RT, U>(s1, wrow, xres, r, step + U * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<MT, RT, U>(s0, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        load_stage<MT, RT, U>(s0, wrow, xres, r, step + 2 * U * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<MT, RT, U>(s1, acc);
-        __builtin_amdgcn_sched_barrier(0);
+    const int rot = start_step(rot_stride, nsteps);
+    if constexpr (D > 0) {
+        RowStream<RT, D> rows;
+        rows.x = buffer_of(x, M * K * 2);
+#pragma unroll
+        for (int t = 0; t < RT; ++t) {
+            const int first = tailed ? seg * tail.d : min(n0 + t * 16, N - 1), count = tailed ? tail.d : min(16, n1 - n0 - t * 16);
+            rows.w[t] = buffer_of(W + (long)first * K, max(count, 0) * K * 2);
+#pragma unroll
+            for (int l = 0; l < 2; ++l) {
+                const int i = stream_row(lane, l), row = tailed ? tail_row(i, t) : i;
+                rows.w_at[2 * t + l] = row < count ? row * K * 2 : LDS_PAST;
+            }
+        }
+#pragma unroll
+        for (int l = 0; l < 2; ++l) rows.x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 2 : LDS_PAST;
+        f32x4_t sums[RT];
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) sums[rt] = acc[rt][0];
+        rows.run(sums, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, rot);
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) acc[rt][0] = sums[rt];
+    } else {
+        const bf16_t* wrow[RT];
+#pragma unroll
+        for (int t = 0; t < RT; ++t) wrow[t] = W + (long)(tailed ? seg * tail.d + tail_row(r, t) : min(n0 + t * 16 + r, n1 - 1)) * K;
+        // x through a buffer descriptor whose bounds are the M real rows (0x00020000: 32-bit raw data format)
+        __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
+        Stage<MT, RT, U> s0, s1;
+        load_stage<MT, RT, U>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
+        // the scheduling barriers keep the compiler from sinking a stage's loads down to their first
+        // use, which would shrink what is in flight to a load or two
+        for (int step = wave; step < nsteps; step += 2 * U * S) {
+            load_stage<MT, RT, U>(s1, wrow, xres, r, step + U * S, S, g, K, nsteps, rot);
+            __builtin_amdgcn_sched_barrier(0);
+            compute_stage<MT, RT, U>(s0, acc);
+            __builtin_amdgcn_sched_barrier(0);
+            load_stage<MT, RT, U>(s0, wrow, xres, r, step + 2 * U * S, S, g, K, nsteps, rot);
+            __builtin_amdgcn_sched_barrier(0);
+            compute_stage<MT, RT, U>(s1, acc);
+            __builtin_amdgcn_sched_barrier(0);
+        }
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) part[((wave * RT + rt) * MT + mt) * 64 + lane] = acc[rt][mt];
+        for (int mt = 0; mt < MT; ++mt) part[wave * WAVE + (rt * MT + mt) * 64 + lane] = acc[rt][mt];
     __syncthreads();
 
     if constexpr (TAIL) {
@@ -203,7 +237,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
             for (int ln = threadIdx.x; ln < 64; ln += blockDim.x) {
                 f32x4_t lo = part[ln], hi = part[64 + ln];
                 for (int w = 1; w < S; ++w) {
-                    const f32x4_t p = part[(w * 2) * 64 + ln], q = part[(w * 2 + 1) * 64 + ln];
+                    const f32x4_t p = part[w * WAVE + ln], q = part[w * WAVE + 64 + ln];
                     lo[0] += p[0]; lo[1] += p[1]; lo[2] += p[2]; lo[3] += p[3];
                     hi[0] += q[0]; hi[1] += q[1]; hi[2] += q[2]; hi[3] += q[3];
                 }
@@ -274,7 +308,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
         const int ln = item & 63, mt = (item >> 6) % MT, rt = (item >> 6) / MT;
         f32x4_t sum = part[(rt * MT + mt) * 64 + ln];
         for (int w = 1; w < S; ++w) {
-            const f32x4_t p = part[((w * RT + rt) * MT + mt) * 64 + ln];
+            const f32x4_t p = part[w * WAVE + (rt * MT + mt) * 64 + ln];
             sum[0] += p[0]; sum[1] += p[1]; sum[2] += p[2]; sum[3] += p[3];
         }
         const int m = mt * 16 + (ln & 15);
@@ -292,36 +326,30 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
 // rows 0 .. 7 of its one tile, their partners as rows 8 .. 15.  Bound by the launch, not by W: at 3,120 x 1,040 and 5 rows it
 // takes what the product alone takes, and the launch that split, rotated and wrote the cache (4 us a layer) is gone: a
 // model of 24 such layers, 5 sequences, 24 steps and their prompts 34.5 -> 32.2 ms.
+template <int D>
 __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
                                                                const float* __restrict__ bias, int M, int K, int rot_stride,
-                                                               QkvTail tail) {
-    extern __shared__ f32x4_t part[];  // [S][64]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
-    const int r = lane & 15, g = lane >> 4, half = tail.d >> 1;
-    const int pairs = (tail.nh + 2 * tail.nkv) * half;
-    const int p0 = (int)((long)blockIdx.x * pairs / gridDim.x), p1 = (int)((long)(blockIdx.x + 1) * pairs / gridDim.x);
-    const int mine = min(p0 + (r & 7), p1 - 1);  // (places past the end read a pair again)
-    int ea, eb;
-    bool rotated;
-    qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
-    const bf16_t* wrow[1] = {W + (long)(mine / half * tail.d + (r < 8 ? ea : eb)) * K};
-    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
-    f32x4_t acc[1][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}};
-    const int nsteps = (K + 63) >> 6;
-    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
-    Stage<1, 1, 2> s0, s1;
-    load_stage<1, 1, 2>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
-    for (int step = wave; step < nsteps; step += 4 * S) {
-        load_stage<1, 1, 2>(s1, wrow, xres, r, step + 2 * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<1, 1, 2>(s0, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        load_stage<1, 1, 2>(s0, wrow, xres, r, step + 4 * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<1, 1, 2>(s1, acc);
-        __builtin_amdgcn_sched_barrier(0);
+                                                               Share share, QkvTail tail) {
+    extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums
+    constexpr int WAVE = RowStream<1, D>::RING / 16;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6, half = tail.d >> 1;
+    const int p0 = share.begin(blockIdx.x), p1 = share.end(blockIdx.x);
+    const int nsteps = (K + 63) >> 6, first = p0 / half * tail.d;  // row of W that the others are counted from
+    RowStream<1, D> rows;
+    rows.w[0] = buffer_of(W + (long)first * K, min((tail.nh + 2 * tail.nkv) * tail.d - first, 2 * tail.d) * K * 2);
+    rows.x = buffer_of(x, M * K * 2);
+#pragma unroll
+    for (int l = 0; l < 2; ++l) {
+        const int pair = p0 + (lane >> 3);
+        int e[2];
+        bool rotated;
+        qkv_tail_pair_elements(tail.rot, tail.d, pair % half, e[0], e[1], rotated);
+        rows.w_at[l] = pair < p1 ? (pair / half * tail.d + e[l] - first) * K * 2 : LDS_PAST;
+        rows.x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 2 : LDS_PAST;
     }
-    part[wave * 64 + lane] = acc[0][0];
+    f32x4_t acc[1] = {f32x4_t{0.f, 0.f, 0.f, 0.f}};
+    rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, start_step(rot_stride, nsteps));
+    part[wave * WAVE + lane] = acc[0];
     __syncthreads();
     const float* sums = (const float*)part;  // row i of the tile, column m: lane (i / 4) * 16 + m, element i % 4
     for (int item = threadIdx.x; item < 128; item += blockDim.x) {
@@ -329,7 +357,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
         if (m >= M || pair >= p1) continue;
         const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
         float a = sums[at], b = sums[at + 2 * 16 * 4];
-        for (int w = 1; w < S; ++w) a += sums[w * 256 + at], b += sums[w * 256 + at + 2 * 16 * 4];
+        for (int w = 1; w < S; ++w) a += sums[w * WAVE * 4 + at], b += sums[w * WAVE * 4 + at + 2 * 16 * 4];
         qkv_tail_pair(tail, bias, m, pair / half, pair % half, round_to_bf16(a), round_to_bf16(b));
     }
 }
@@ -351,8 +379,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
     const int r = lane & 15, g = lane >> 4, row = r & 7, sub = r >> 3;
     const int half = TAIL ? tail.d >> 1 : 1;
-    const int items = TAIL ? (tail.nh + 2 * tail.nkv) * half : p.N;  // pairs, or rows, that the workgroups share evenly
-    const int n0 = (int)((long)blockIdx.x * items / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * items / gridDim.x);
+    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);  // pairs, or rows
     int w_row = min(n0 + row, n1 - 1);
     if (TAIL) {
         const int mine = min(n0 + (row & 3), n1 - 1);  // (places past the end read a pair again)
@@ -364,7 +391,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
     const bf16_t* wrow = p.W + (long)w_row * K;
     __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, M * K * 2, 0x00020000);
     const int nsteps = (K + 127) >> 7;
-    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
+    const int rot = start_step(rot_stride, nsteps);
     struct Halves {
         Frag a[U][2], b[U][2][BT];
         uint32_t keep[U][2];
@@ -443,33 +470,29 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
 // The input product of a gated feed-forward, W = [gate rows, up rows], with the gate in its epilogue: y[M, F] = glu(x . Wg^T, x . Wu^T)
 // for up to 16 rows.  A workgroup's two row tiles are the same rows of the gate and of the up matrix.  As a pass of its own
 // the gate took 4.5 us behind a product of 13 (2 rows, 2 x 5,504 x 2,048).
+template <int D>
 __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
                                                               const bf16_t* __restrict__ W, int M, int F, int K, int rot_stride, int kind,
-                                                              float alpha, float limit) {
-    extern __shared__ f32x4_t part[];  // [S][2][64]
+                                                              float alpha, float limit, Share share) {
+    extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums, [2][64] each
+    constexpr int WAVE = RowStream<2, D>::RING / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
-    const int r = lane & 15, g = lane >> 4;
-    const int n0 = (int)((long)blockIdx.x * F / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * F / gridDim.x);
-    const int row = min(n0 + r, n1 - 1);
-    const bf16_t* wrow[2] = {W + (long)row * K, W + (long)(F + row) * K};
-    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
-    f32x4_t acc[2][1] = {{f32x4_t{0.f, 0.f, 0.f, 0.f}}, {f32x4_t{0.f, 0.f, 0.f, 0.f}}};
+    const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);
     const int nsteps = (K + 63) >> 6;
-    const int rot = rot_stride > 0 ? (int)(((long)blockIdx.x * rot_stride) % nsteps) : 0;
-    Stage<1, 2, 2> s0, s1;
-    load_stage<1, 2, 2>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
-    for (int step = wave; step < nsteps; step += 4 * S) {
-        load_stage<1, 2, 2>(s1, wrow, xres, r, step + 2 * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<1, 2, 2>(s0, acc);
-        __builtin_amdgcn_sched_barrier(0);
-        load_stage<1, 2, 2>(s0, wrow, xres, r, step + 4 * S, S, g, K, nsteps, rot);
-        __builtin_amdgcn_sched_barrier(0);
-        compute_stage<1, 2, 2>(s1, acc);
-        __builtin_amdgcn_sched_barrier(0);
-    }
+    RowStream<2, D> rows;
+    rows.w[0] = buffer_of(W + (long)n0 * K, (n1 - n0) * K * 2);
+    rows.w[1] = buffer_of(W + (long)(F + n0) * K, (n1 - n0) * K * 2);
+    rows.x = buffer_of(x, M * K * 2);
 #pragma unroll
-    for (int rt = 0; rt < 2; ++rt) part[(wave * 2 + rt) * 64 + lane] = acc[rt][0];
+    for (int l = 0; l < 2; ++l) {
+        const int i = stream_row(lane, l);
+        rows.w_at[l] = rows.w_at[2 + l] = i < n1 - n0 ? i * K * 2 : LDS_PAST;
+        rows.x_at[l] = i < M ? i * K * 2 : LDS_PAST;
+    }
+    f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+    rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, start_step(rot_stride, nsteps));
+#pragma unroll
+    for (int rt = 0; rt < 2; ++rt) part[wave * WAVE + rt * 64 + lane] = acc[rt];
     __syncthreads();
     const float* sums = (const float*)part;  // feature i of a tile, row m of x: lane (i / 4) * 16 + m, element i % 4
     for (int item = threadIdx.x; item < 16 * M; item += blockDim.x) {
@@ -477,7 +500,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict
         if (n0 + i >= n1) continue;
         const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
         float gate = sums[at], up = sums[256 + at];
-        for (int w = 1; w < S; ++w) gate += sums[w * 512 + at], up += sums[w * 512 + 256 + at];
+        for (int w = 1; w < S; ++w) gate += sums[w * WAVE * 4 + at], up += sums[w * WAVE * 4 + 256 + at];
         y[(long)m * F + n0 + i] = f32_to_bf16_bits(glu_value(kind, round_to_bf16(gate), round_to_bf16(up), alpha, limit));
     }
 }
@@ -505,8 +528,7 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
     const int pitch = K + 8;  // sixteen bytes between rows keep the reads of sixteen rows on distinct banks
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int r = lane & 15, g = lane >> 4, half = TAIL ? tail.d >> 1 : 1;
-    const int items = TAIL ? (tail.nh + 2 * tail.nkv) * half : p.N;
-    const int n0 = (int)((long)blockIdx.x * items / gridDim.x), n1 = (int)((long)(blockIdx.x + 1) * items / gridDim.x);
+    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);
     int w_row = min(n0 + r, n1 - 1);
     if (TAIL) {  // as in gemm_skinny_tail_kernel
         const int mine = min(n0 + (r & 7), n1 - 1);
@@ -632,21 +654,39 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
     }
 }
 
-// Waves per workgroup, i.e. how many ways K is split.  Measured on MI355X: long streams per wave beat
-// many short ones, so K is split only when N alone gives too few waves.  It depends on N only, never
-// on M or on the tile variant, so the order of summation is the same for every batch.
-static int pick_split(int N) {
-    const int groups = (N + 31) / 32;
-    if (groups >= 512) return 1;
-    if (groups >= 128) return 2;
-    if (groups >= 32) return 4;
+// Waves per workgroup, i.e. how many ways K is split, by the sizes of W alone, never by M or by the tile variant, so the order of
+// summation is the same for every batch.  Long streams per wave beat many short ones, so K is split where N alone gives too
+// few waves, and where rows are long (each wave then walks fewer rows' pages at a time).  Measured over cold weights, us with 1 / 2 / 4
+// waves, 8 rows of x, by tiles of 32 rows of W: 41,984 x 8,192 129 / 127 / 124, 65,024 x 4,544 108 / 110 / 112, 22,848 x 4,544 42.0 / 39.7 /
+// 43.1, 22,528 x 4,096 36.2 / 35.6 / 38.7, 32,768 x 2,048 26.6 / 28.6 / 32.5, 8,192 x 2,048 11.2 / 8.5 / 8.9, 6,144 x 2,048 11.1 / 7.5 / 7.8; by
+// tiles of sixteen 12,032 x 8,192 38.1 / 39.5 / 37.3, 12,032 x 4,096 20.5 / 21.4 / 21.6, 11,008 x 2,048 11.0 / 11.7 / 12.6.
+static int pick_split(int N, int K) {
+    if (N >= 10240 && K >= 8192) return 4;
+    if (N >= 32768 || (N >= 10240 && N < 16384)) return 1;
+    if (N >= 16384) return K >= 4096 ? 2 : 1;
+    if (N >= 4096) return 2;
+    if (N >= 1024) return 4;
     return 8;
 }
 
+// Whether up to sixteen rows of x go by tiles of sixteen rows of W a wave (else of 32, which read x half as often; the bits are the
+// same): where 32 leave compute units with an uneven share, and for short rows, whose waves spend their time starting.  32 rows -> 16, us:
+// 11,008 x 2,048 12.0 -> 11.0, 12,032 x 8,192 42.0 -> 37.3; 50,001 x 1,040 1 row 28.5 -> 22.5, 8 rows 28.8 -> 26.6, 16 rows 31.0 -> 31.2.
+static bool short_tiles(int N, int K, int M) { return (N >= 10240 && N < 16384) || (N >= 16384 && K <= 2048 && M <= 8); }
+
+// One launch of a kernel whose waves each have a ring in LDS (D > 0): more than 64 KB have to be asked for, on every device
+template <typename Kernel, typename... Args>
+static int launch_rings(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, Args... args) {
+    if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+        return pta_fail("gemm_skinny_bf16: %zu bytes of LDS were refused", lds);
+    hipLaunchKernelGGL(kernel, grid, block, lds, s, args...);
+    return 0;
+}
+
 template <int MT, int RT, int U, typename OutT>
-static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hipStream_t s, bool spread = false) {
+static int launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hipStream_t s, bool spread = false) {
     const int rows = 16 * RT;
-    if (S <= 0) S = pick_split(a.N + b.N);
+    if (S <= 0) S = pick_split(a.N + b.N, K);
     a.blocks = (a.N + rows - 1) / rows;
     b.blocks = (b.N + rows - 1) / rows;
     // A launch takes as long as the compute unit with the most workgroups: 714 workgroups on 256 units take
@@ -665,21 +705,29 @@ static void launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hi
             b.blocks = total - a.blocks;
         }
     }
+    a.rows = Share(a.N, a.blocks);
+    b.rows = Share(b.N, b.blocks);
     const dim3 grid(a.blocks + b.blocks), block(S * 64);
     const size_t lds = (size_t)S * RT * MT * 64 * sizeof(f32x4_t);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);  // rows a multiple of 4 KB long
+    if constexpr (MT == 1 && RT <= 2) if (K <= STREAM_MOST_K) {
+        if (S <= 4) return launch_rings(gemm_skinny_kernel<MT, RT, U, OutT, 0, 4>, grid, block, (size_t)S * RowStream<RT, 4>::RING, s, a, b, M, K, rot_stride, QkvTail{});
+        return launch_rings(gemm_skinny_kernel<MT, RT, U, OutT, 0, 3>, grid, block, (size_t)S * RowStream<RT, 3>::RING, s, a, b, M, K, rot_stride, QkvTail{});
+    }
     hipLaunchKernelGGL((gemm_skinny_kernel<MT, RT, U, OutT>), grid, block, lds, s, a, b, M, K, rot_stride, QkvTail{});
+    return 0;
 }
 
 // where a workgroup has eight rows of W or fewer (N alone decides: one order of summation for any number of rows of x)
 static bool by_halves(int N) { return N <= 8 * pta_compute_units(); }
 
 template <typename OutT, bool TAIL = false>
-static int launch_halves(const SkinnyProblem& p, int M, int K, int S, hipStream_t s, const QkvTail& tail = QkvTail{}) {
+static int launch_halves(SkinnyProblem p, int M, int K, int S, hipStream_t s, const QkvTail& tail = QkvTail{}) {
     const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 4 : 8, units = pta_compute_units();
     if (S <= 0) S = 2;  // four waves 5.9 us at 2,048 x 2,048 and 8 rows, 7.6 at 16, two 5.4 and 6.7; longer rows within 2 %
     const dim3 grid(std::max((items + most - 1) / most, std::min(units, (items + most / 2 - 1) / (most / 2)))), block(S * 64);
+    p.rows = Share(items, (int)grid.x);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 3 : 0);
     auto go = [&](auto kernel, int tiles) { hipLaunchKernelGGL(kernel, grid, block, (size_t)S * tiles * 64 * sizeof(f32x4_t), s, p, M, K, rot, tail); };
@@ -704,26 +752,28 @@ static int launch_skinny(SkinnyProblem a, SkinnyProblem b, int M, int K, int var
     // x 2,048 9.2 -> 9.8, at 16 rows of x 9.9 -> 11.7).
     if (variant == 7 || (variant == 0 && b.N == 0 && by_halves(a.N))) return launch_halves<OutT>(a, M, K, S, s);
     if (variant == 0 && b.N == 0 && pta_gemm_skinny_spread(a.N)) variant = 6;
+    int rc;
     if (M <= 16) {
-        if (variant == 0) variant = 2;
-        if (variant == 1) launch_cfg<1, 1, 4, OutT>(a, b, M, K, S, s);
-        else if (variant == 2) launch_cfg<1, 2, 2, OutT>(a, b, M, K, S, s);
-        else if (variant == 3) launch_cfg<1, 4, 1, OutT>(a, b, M, K, S, s);
-        else if (variant == 4) launch_cfg<1, 4, 2, OutT>(a, b, M, K, S, s);
-        else if (variant == 6) launch_cfg<1, 1, 2, OutT>(a, b, M, K, S, s, true);
-        else launch_cfg<1, 2, 4, OutT>(a, b, M, K, S, s);
+        if (variant == 0) variant = short_tiles(a.N + b.N, K, M) ? 1 : 2;
+        if (variant == 1) rc = launch_cfg<1, 1, 4, OutT>(a, b, M, K, S, s);
+        else if (variant == 2) rc = launch_cfg<1, 2, 2, OutT>(a, b, M, K, S, s);
+        else if (variant == 3) rc = launch_cfg<1, 4, 1, OutT>(a, b, M, K, S, s);
+        else if (variant == 4) rc = launch_cfg<1, 4, 2, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) rc = launch_cfg<1, 1, 2, OutT>(a, b, M, K, S, s, true);
+        else rc = launch_cfg<1, 2, 4, OutT>(a, b, M, K, S, s);
     } else if (M <= 32) {
-        if (variant == 3 || variant == 4) launch_cfg<2, 4, 1, OutT>(a, b, M, K, S, s);
-        else if (variant == 6) launch_cfg<2, 1, 1, OutT>(a, b, M, K, S, s, true);
-        else launch_cfg<2, 2, 1, OutT>(a, b, M, K, S, s);
+        if (variant == 3 || variant == 4) rc = launch_cfg<2, 4, 1, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) rc = launch_cfg<2, 1, 1, OutT>(a, b, M, K, S, s, true);
+        else rc = launch_cfg<2, 2, 1, OutT>(a, b, M, K, S, s);
     } else if (M <= 48) {
-        if (variant == 6) launch_cfg<3, 1, 1, OutT>(a, b, M, K, S, s, true);
-        else launch_cfg<3, 2, 1, OutT>(a, b, M, K, S, s);
+        if (variant == 6) rc = launch_cfg<3, 1, 1, OutT>(a, b, M, K, S, s, true);
+        else rc = launch_cfg<3, 2, 1, OutT>(a, b, M, K, S, s);
     } else {
-        if (variant == 3 || variant == 4) launch_cfg<4, 4, 1, OutT>(a, b, M, K, S, s);
-        else if (variant == 6) launch_cfg<4, 1, 1, OutT>(a, b, M, K, S, s, true);
-        else launch_cfg<4, 2, 1, OutT>(a, b, M, K, S, s);
+        if (variant == 3 || variant == 4) rc = launch_cfg<4, 4, 1, OutT>(a, b, M, K, S, s);
+        else if (variant == 6) rc = launch_cfg<4, 1, 1, OutT>(a, b, M, K, S, s, true);
+        else rc = launch_cfg<4, 2, 1, OutT>(a, b, M, K, S, s);
     }
+    if (rc) return rc;
     return pta_check_launch("gemm_skinny_bf16");
 }
 
@@ -795,15 +845,20 @@ extern "C" int pta_gemm_skinny_pair_qkv_bf16(void* q_out, const void* x1, const 
     b.blocks = (N2 + 31) / 32;
     const int units = pta_compute_units(), natural = a.blocks + b.blocks;
     if (natural > units && natural % units != 0) b.blocks = (natural + units - 1) / units * units - a.blocks;
-    const int S = pick_split(N1 + N2);
+    a.rows = Share(a.N, a.blocks);
+    b.rows = Share(b.N, b.blocks);
+    const int S = pick_split(N1 + N2, K);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
-    if (qkv_tail_plain_pairs(rot, d))
-        hipLaunchKernelGGL((gemm_skinny_kernel<1, 2, 2, bf16_t, 1>), dim3(a.blocks + b.blocks), dim3(S * 64),
-                           (size_t)S * 2 * 64 * sizeof(f32x4_t), (hipStream_t)stream, a, b, M, K, rot_stride, tail);
-    else
-        hipLaunchKernelGGL((gemm_skinny_kernel<1, 2, 2, bf16_t, 2>), dim3(a.blocks + b.blocks), dim3(S * 64),
-                           (size_t)S * 2 * 64 * sizeof(f32x4_t), (hipStream_t)stream, a, b, M, K, rot_stride, tail);
+    auto go = [&](auto kernel, size_t ring) {
+        return launch_rings(kernel, dim3(a.blocks + b.blocks), dim3(S * 64), S * ring, (hipStream_t)stream, a, b, M, K, rot_stride, tail);
+    };
+    const bool plain = qkv_tail_plain_pairs(rot, d);
+    int rc;
+    if (K > STREAM_MOST_K) rc = plain ? go(gemm_skinny_kernel<1, 2, 2, bf16_t, 1>, 2048) : go(gemm_skinny_kernel<1, 2, 2, bf16_t, 2>, 2048);
+    else if (S <= 4) rc = plain ? go(gemm_skinny_kernel<1, 2, 2, bf16_t, 1, 4>, RowStream<2, 4>::RING) : go(gemm_skinny_kernel<1, 2, 2, bf16_t, 2, 4>, RowStream<2, 4>::RING);
+    else rc = plain ? go(gemm_skinny_kernel<1, 2, 2, bf16_t, 1, 3>, RowStream<2, 3>::RING) : go(gemm_skinny_kernel<1, 2, 2, bf16_t, 2, 3>, RowStream<2, 3>::RING);
+    if (rc) return rc;
     if (pta_check_launch("gemm_skinny_pair_qkv_bf16")) return 1;
     if (!in_kernel(act2)) return pta_epilogue(y2, N2, nullptr, nullptr, nullptr, M, N2, act2, PTA_BF16, stream);
     return 0;
@@ -846,14 +901,15 @@ extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* 
                           v_pool, nh, nkv, d, layout, write_cache, M, K, p, tail)) return 1;
     const int N = p.N;
     PTA_REQUIRE(pta_gemm_skinny_spread(N), "gemm_skinny_qkv_bf16: %d rows of W are too many for this launch", N);
+    PTA_REQUIRE(K <= STREAM_MOST_K, "gemm_skinny_qkv_bf16: rows of %d elements are too long for this launch", K);
     if (by_halves(N)) return launch_halves<bf16_t, true>(p, M, K, 0, (hipStream_t)stream, tail);
     const int pairs = N / 2;
     const int blocks = std::max((pairs + 7) / 8, std::min(pta_compute_units(), (pairs + 1) / 2));
-    const int S = pick_split(N);
+    const int S = pick_split(N, K);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
-    hipLaunchKernelGGL(gemm_skinny_tail_kernel, dim3(blocks), dim3(S * 64), (size_t)S * 64 * sizeof(f32x4_t), (hipStream_t)stream,
-                       p.x, p.W, bias, M, K, rot_stride, tail);
+    if (launch_rings(gemm_skinny_tail_kernel<4>, dim3(blocks), dim3(S * 64), (size_t)S * RowStream<1, 4>::RING, (hipStream_t)stream, p.x,
+                     p.W, bias, M, K, rot_stride, Share(pairs, blocks), tail)) return 1;
     return pta_check_launch("gemm_skinny_qkv_bf16");
 }
 
@@ -864,12 +920,13 @@ extern "C" int pta_gemm_normed_ok(int M, int N, int K) {
 }
 
 template <bool TAIL>
-static int launch_normed(const char* what, const SkinnyProblem& p, const float* ln_w, const float* ln_b, float eps, int M, int K,
+static int launch_normed(const char* what, SkinnyProblem p, const float* ln_w, const float* ln_b, float eps, int M, int K,
                          const QkvTail& tail, hipStream_t s) {
     PTA_REQUIRE(pta_gemm_normed_ok(M, p.N, K), "%s: M=%d N=%d K=%d are not for this launch", what, M, p.N, K);
     PTA_REQUIRE(ln_w && ln_b && ((uintptr_t)ln_w % 16) == 0 && ((uintptr_t)ln_b % 16) == 0, "%s: the norm's vectors must be there and 16-byte aligned", what);
     const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 8 : 16, units = pta_compute_units();
     const int groups = std::max((items + most - 1) / most, std::min(units, (items + most / 4 - 1) / (most / 4)));
+    p.rows = Share(items, groups);
     const bool eight = groups <= units + units / 16;
     const int waves = eight ? 8 : 4;
     const size_t lds = waves * 64 * sizeof(f32x4_t) + (size_t)M * (K + 8) * sizeof(bf16_t);
@@ -920,14 +977,18 @@ extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, i
     if (check_skinny("gemm_skinny_glu_bf16", y, x, W, M, F, K, PTA_ACT_NONE)) return 1;
     PTA_REQUIRE(M <= 16, "gemm_skinny_glu_bf16: at most 16 rows, got %d", M);
     PTA_REQUIRE(F < (1 << 30), "gemm_skinny_glu_bf16: %d features are too many", F);
+    PTA_REQUIRE(K <= STREAM_MOST_K, "gemm_skinny_glu_bf16: rows of %d elements are too long for this launch", K);
     PTA_REQUIRE(kind == PTA_GLU_SILU || kind == PTA_GLU_CLAMPED || kind == PTA_GLU_GELU_TANH, "gemm_skinny_glu_bf16: kind %d is not built", kind);
-    const int S = pick_split(2 * F), units = pta_compute_units();
+    const int S = 2 * F >= 16384 ? pick_split(2 * F, K) : 2 * F >= 4096 ? 2 : 2 * F >= 1024 ? 4 : 8, units = pta_compute_units();
     int blocks = (F + 15) / 16;
     if (blocks > units) blocks = (blocks + units - 1) / units * units;  // a whole number of workgroups per unit (launch_cfg)
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
-    hipLaunchKernelGGL(gemm_skinny_glu_kernel, dim3(blocks), dim3(S * 64), (size_t)S * 2 * 64 * sizeof(f32x4_t), (hipStream_t)stream,
-                       (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)W, M, F, K, rot_stride, kind, alpha, limit);
+    auto go = [&](auto kernel, size_t ring) {
+        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)W, M, F, K,
+                            rot_stride, kind, alpha, limit, Share(F, blocks));
+    };
+    if (S <= 4 ? go(gemm_skinny_glu_kernel<4>, RowStream<2, 4>::RING) : go(gemm_skinny_glu_kernel<3>, RowStream<2, 3>::RING)) return 1;
     return pta_check_launch("gemm_skinny_glu_bf16");
 }
 

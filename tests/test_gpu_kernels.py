@@ -98,6 +98,38 @@ def test_gemm_skinny_bf16(M, N, K):
     assert torch.equal(alone, got32[r:r + 1])
 
 
+# N: where the waves a workgroup and the rows of a tile change, and a row more or less; K: less than a step of 64, one, several and a
+# part, and fewer steps than a ring holds
+@pytest.mark.parametrize("N", [1, 17, 1000, 1024, 4095, 4096, 10239, 10240, 16383, 16384, 32768, 32800])
+@pytest.mark.parametrize("K", [8, 64, 72, 264, 2056])
+def test_gemm_skinny_bf16_through_lds(N, K):
+    """Few rows through the waves' rings in LDS: 32-bit sums against 64 bits, the same bits for any number of rows of x."""
+    ops = _ops()
+    x = _rand(16, K, dtype=torch.bfloat16)
+    w = _rand(N, K, seed=1, dtype=torch.bfloat16, scale=0.05)
+    prod = x.double() @ w.double().T
+    got = ops.gemm_skinny_bf16(x, w, out_f32=True)
+    assert float((got.double() - prod).abs().max()) <= 2e-5 * float(prod.abs().max()) + 1e-6
+    for m in (1, 8, 9):
+        assert torch.equal(ops.gemm_skinny_bf16(x[:m].contiguous(), w, out_f32=True), got[:m]), m
+
+
+@pytest.mark.parametrize("M", [1, 20])
+def test_few_row_products_of_very_long_rows(M):
+    """Rows of W beyond what the launches through LDS address (2^20 elements)."""
+    ops = _ops()
+    N, K = 3, (1 << 20) + 8
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w = (torch.randn(n, K, generator=g, device="cuda").bfloat16() for n in (M, N))
+    prod = x.double() @ w.double().T.contiguous()
+    tol = 8 * 2.0 ** -24 * K  # as a chain of K sums of products of size 1: sqrt(K) eps times the root of the sum of K squares
+    assert float((ops.gemm_skinny_bf16(x, w, out_f32=True).double() - prod).abs().max()) <= tol
+    for parts in (1, 3):
+        assert float((ops.gemm_splitk_bf16(x, w, out_f32=True, parts=parts).double() - prod).abs().max()) <= tol
+    part = ops.gemm_splitk_partial(x, w)
+    assert float((part.double().sum(0) - prod).abs().max()) <= tol
+
+
 @pytest.mark.parametrize("M", [1, 9, 17, 32, 33, 50, 64, 65, 81, 96, 100, 128, 129, 200, 256])
 @pytest.mark.parametrize("N,K,parts,rt,sb,depth", [(16, 64, 0, 0, 0, 0), (100, 200, 0, 0, 0, 0), (100, 200, 3, 2, 2, 2),
                                                    (4544, 4544, 0, 0, 0, 0), (250, 18176 // 4, 5, 1, 2, 4),
