@@ -3,20 +3,22 @@
 //
 // With more than 16 rows the activations are no longer negligible beside the weights: a wave that
 // fetched its own x fragments would pull as many bytes of x out of L2 as of W out of HBM.  Here a
-// workgroup of four waves owns 64*RT rows of W (16*RT each) and a range of K, and shares x: the four
-// waves copy the stage's [M, KS] slice of x into LDS together (through registers, one stage ahead,
-// two LDS buffers), and every wave reads its B fragments from there.  W rows go straight from global
-// memory into the A operand registers, one stage ahead of the matrix cores, as in the kernel for
-// few rows.  K is split over gridDim.y workgroups when N alone gives too few of them to occupy the
-// chip; each writes its 32-bit partial tile to `part`, and a second small kernel adds the partials
-// in the order of the ranges and applies bias, activation and additions; with reduce = 0 the partials
+// workgroup of four waves owns 64*RT rows of W (16*RT each) and a range of K, and shares x: a stage is 64
+// elements of K, for which each wave brings its own rows of W and its share of the rows of x straight to LDS
+// (lds_stream.h), D - 1 stages ahead, with one barrier a stage.  K is split over gridDim.y workgroups when N alone
+// gives too few of them to occupy the chip; each writes its 32-bit partial tile to `part`, and a second small kernel
+// adds the partials in the order of the ranges and applies bias, activation and additions; with reduce = 0 the partials
 // are the result, and the kernel that reads them next adds them in the same order.  The split is chosen from N
 // and K alone, so the order of summation does not depend on the batch.
 //
-// Chunks of x past the workgroup's K range, or rows past M, are read through a buffer descriptor at
-// an offset outside its bounds and arrive as zeros; W addresses are clamped into the range instead, so
-// a stage past the end multiplies weights that are already in cache by zeros.
+// Through registers, sixteen rows of W a load, the same ranges took (pairs of products, us, registers -> LDS): 4,544 x 4,544 with
+// 4,544 x 18,176 1 row 42.7 -> 40.5, 32 rows 49.6 -> 45.0; 4,096 x 4,096 with 4,096 x 16,384 39.8 -> 36.1, 46.0 -> 39.3; 9,216 and 32,768 x
+// 8,192 17 rows 156 -> 139, 32 rows 166 -> 144.
+//
+// Chunks of x and W past the workgroup's K range, or rows past M and N, are read through a buffer descriptor at
+// an offset outside its bounds and arrive as zeros.
 #include "common.h"
+#include "lds_stream.h"
 #include "pta_kernels.h"
 #include "qkv_tail.h"
 
@@ -27,15 +29,8 @@
 #include <mutex>
 #include <utility>
 
-typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
-typedef float f32x4_t __attribute__((ext_vector_type(4)));
-typedef int i32x4_t __attribute__((ext_vector_type(4)));
-
-union Frag8 {
-    uint4 u;
-    bf16x8_t v;
-    i32x4_t i;
-};
+// bytes of a stage of 64 elements of K in LDS: four waves' rows of W, and the rows of x by whole loads of each wave
+static constexpr __host__ __device__ int splitk_slot(int MT, int RT) { return RT * 8192 + (MT + 1) / 2 * 4096; }
 
 #define SK_THREADS 256
 #define SK_CHUNK_ROWS 128  // eight tiles of sixteen rows of x: what a workgroup holds
@@ -58,19 +53,27 @@ struct SplitkProblem {
     int direct;           // one range and the epilogue in this kernel
 };
 
-template <int MT, int RT, int U, int D, bool ROT>
+// what follows a whole sum, for one element
+__device__ __forceinline__ void store_whole(void* y, const float* bias, const bf16_t* add1, const bf16_t* add2, int act, int out_f32, int n,
+                                            long o, float v) {
+    if (!out_f32) v = round_to_bf16(v);
+    if (bias) { v += bias[n]; if (!out_f32) v = round_to_bf16(v); }
+    if (act == PTA_ACT_GELU) v = out_f32 ? gelu_erf(v) : gelu_bf16(v);  // other activations: see pta_gemm_splitk_bf16
+    if (add1) v += bf16_bits_to_f32(add1[o]);
+    if (add2) v += bf16_bits_to_f32(add2[o]);
+    if (out_f32) ((float*)y)[o] = v;
+    else ((bf16_t*)y)[o] = f32_to_bf16_bits(v);
+}
+
+template <int MT, int RT, int D, bool ROT>
 __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem pa, SplitkProblem pb, int M, int chunks,
                                                                  int chunk_rows, int rot_stride) {
-    constexpr int KS = U * 64;                       // elements of K per stage
-    constexpr int MP = MT * 16;                      // rows of x, padded to whole tiles
-    constexpr int LDW = KS + 8;                      // LDS row stride: 16 bytes of padding keep 16-byte reads off each other's banks
-    constexpr int PIECES = MP * (KS / 8) / SK_THREADS;  // 16-byte pieces of the x slice per thread
-    constexpr int STEPS = U * 2;                     // 32-element matrix-core steps per stage
-    static_assert(MP * (KS / 8) % SK_THREADS == 0, "the x slice must divide over the threads");
-    static_assert(D % 2 == 0, "stages alternate between two LDS buffers");
-    extern __shared__ __attribute__((aligned(16))) bf16_t xs[];  // [2][MP][LDW]
+    constexpr int NX = (MT + 1) / 2;                 // loads of x per wave and stage (eight rows by 128 bytes each)
+    constexpr int NL = 2 * RT + NX;                  // all of a wave's loads per stage
+    constexpr int SLOT = splitk_slot(MT, RT);        // a stage in LDS: the four waves' rows of W, then x
+    extern __shared__ __attribute__((aligned(1024))) char lds[];  // [D][SLOT]
 
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int r = lane & 15, g = lane >> 4;
     // More rows than a workgroup holds are cut into `chunks` chunks of `chunk_rows`; the workgroups that take the
     // same rows of W for the chunks sit a multiple of eight apart in the grid, so that they start together on one
@@ -107,12 +110,22 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
     const int nkb = (K + 63) >> 6;
     const int kb0 = range * blocks_per_part, kb1 = min(kb0 + blocks_per_part, nkb);
     const int k_begin = kb0 * 64, k_end = min(kb1 * 64, K);
-    const int nstages = (kb1 - kb0 + U - 1) / U;
+    const int nstages = kb1 - kb0;
 
-    const bf16_t* wrow[RT];
+    // rows past the last one lie past the buffers' ends, elements past the range's end are asked for there: zeros, no traffic
+    const int n_rows = max(0, min(16 * RT, N - n_base));
+    const i32x4_t rw = buffer_of(W + (long)min(n_base, N - 1) * K, n_rows * K * 2), rx = buffer_of(x + (long)m0 * K, (m_end - m0) * K * 2);
+    const unsigned to_w = __builtin_amdgcn_readfirstlane(lds_address(lds)) + wave * (RT * 2048);
+    const unsigned to_x = __builtin_amdgcn_readfirstlane(lds_address(lds)) + RT * 8192 + wave * 1024;
+    int w_at[2 * RT], x_at[NX];  // the lane's rows
 #pragma unroll
-    for (int t = 0; t < RT; ++t) wrow[t] = W + (long)min(n_base + t * 16 + r, N - 1) * K;
-    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
+    for (int l = 0; l < 2 * RT; ++l) w_at[l] = ((l >> 1) * 16 + stream_row(lane, l & 1)) * K * 2;
+#pragma unroll
+    for (int l = 0; l < NX; ++l) {
+        const int row = (wave + 4 * l) * 8 + (lane >> 3);
+        x_at[l] = row < m_end - m0 ? row * K * 2 : LDS_PAST;
+    }
+    const int c8[2] = {stream_element(lane, 0), stream_element(lane, 1)};
 
     f32x4_t acc[RT][MT];
 #pragma unroll
@@ -124,80 +137,55 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
     // memory channels at the same time (N = 4,096, K = 16,384: a third slower than K = 16,448).  So each walks its
     // range from a starting stage of its own and wraps round; stages past the last read nothing.  A feature's
     // order of summation follows from N, K and the launch alone.
-    // (ROT is a compile-time choice: the wrap costs the other shapes 5 % of this kernel at 17 to 32 rows.)
     const int rot = ROT && nstages > 0 ? (int)(((long)tile * rot_stride) % nstages) : 0;
-    auto stage_k = [&](int stage) {
-        if (!ROT) return k_begin + stage * KS;
-        if (stage >= nstages) return k_end;
-        int at = stage + rot;
-        at -= at >= nstages ? nstages : 0;
-        return k_begin + at * KS;
-    };
-    auto load_x = [&](int stage, i32x4_t(&xr)[PIECES]) {
-        const int k_stage = stage_k(stage);
+    auto issue = [&](int stage, int slot) {
+        int at = stage;
+        if (ROT) { at += rot; at -= at >= nstages ? nstages : 0; }
+        const int k = k_begin + at * 64;
+        const bool real = stage < nstages;
 #pragma unroll
-        for (int j = 0; j < PIECES; ++j) {
-            const int q = tid + j * SK_THREADS, row = m0 + q / (KS / 8), k = k_stage + (q % (KS / 8)) * 8;
-            const int off = (k < k_end && row < m_end) ? (row * K + k) * 2 : 0x7ffffff0;
-            xr[j] = __builtin_amdgcn_raw_buffer_load_b128(xres, off, 0, 0);
+        for (int l = 0; l < 2 * RT; ++l) {
+            const int ke = k + c8[l & 1];
+            fetch16(rw, to_w + slot + l * 1024, real && ke < k_end ? w_at[l] + ke * 2 : LDS_PAST);
+        }
+#pragma unroll
+        for (int l = 0; l < NX; ++l) {
+            const int ke = k + c8[wave & 1];  // (an even number of loads away from the wave's first: the same half of a tile)
+            fetch16(rx, to_x + slot + l * 4096, real && ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
         }
     };
-    auto store_x = [&](int buf, const i32x4_t(&xr)[PIECES]) {
+    const int in_row = r * 128 + ((g ^ (r >> 1)) & 7) * 16;  // the second 32 elements of a stage: 64 flipped
+    // D - 1 stages are on their way.  One barrier a stage: behind it everyone's share of the stage has landed, and everyone is
+    // past reading the one before, whose place the next loads take.
 #pragma unroll
-        for (int j = 0; j < PIECES; ++j) {
-            const int q = tid + j * SK_THREADS, row = q / (KS / 8), c8 = q % (KS / 8);
-            *reinterpret_cast<i32x4_t*>(&xs[(buf * MP + row) * LDW + c8 * 8]) = xr[j];
-        }
-    };
-    auto load_w = [&](int stage, Frag8(&wr)[STEPS][RT]) {
-        const int k_stage = stage_k(stage) + g * 8;
+    for (int d = 0; d < D - 1; ++d) issue(d, d * SLOT);
+    int cur = 0, free = (D - 1) * SLOT;
+    for (int s = 0; s < nstages; ++s) {
+        wait_reads();
+        wait_loads<(D - 2) * NL>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+        issue(s + D - 1, free);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int j = 0; j < STEPS; ++j) {
-            const int kc = min(k_stage + j * 32, k_end - 8);
+        for (int hf = 0; hf < 2; ++hf) {
+            bf16x8_t w[RT], b[MT];
+            const int at = (in_row ^ (hf * 64)) + cur;
 #pragma unroll
-            for (int t = 0; t < RT; ++t) wr[j][t].u = *reinterpret_cast<const uint4*>(wrow[t] + kc);
-        }
-    };
-    auto compute = [&](int buf, const Frag8(&wr)[STEPS][RT]) {
+            for (int t = 0; t < RT; ++t) w[t] = *reinterpret_cast<const bf16x8_t*>(lds + at + (wave * RT + t) * 2048);
 #pragma unroll
-        for (int j = 0; j < STEPS; ++j) {
-            bf16x8_t b[MT];
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-                b[mt] = *reinterpret_cast<const bf16x8_t*>(&xs[(buf * MP + mt * 16 + r) * LDW + j * 32 + g * 8]);
+            for (int mt = 0; mt < MT; ++mt) b[mt] = *reinterpret_cast<const bf16x8_t*>(lds + at + RT * 8192 + mt * 2048);
 #pragma unroll
             for (int t = 0; t < RT; ++t)
 #pragma unroll
                 for (int mt = 0; mt < MT; ++mt)
-                    acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wr[j][t].v, b[mt], acc[t][mt], 0, 0, 0);
+                    acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], b[mt], acc[t][mt], 0, 0, 0);
         }
-    };
-
-    // D stages of loads are in flight per wave: stage s lives in register set s % D.  x loads are issued
-    // before the W loads of their stage, so that waiting for the next stage's x leaves younger loads in
-    // flight; the scheduling barriers keep the compiler from sinking loads down to their use.
-    i32x4_t xr[D][PIECES];
-    Frag8 w[D][STEPS][RT];
-#pragma unroll
-    for (int d = 0; d < D; ++d) {
-        load_x(d, xr[d]);
-        load_w(d, w[d]);
+        free = cur;
+        cur = cur == (D - 1) * SLOT ? 0 : cur + SLOT;
     }
-    __builtin_amdgcn_sched_barrier(0);
-    store_x(0, xr[0]);
-    __syncthreads();
-    for (int s = 0; s < nstages; s += D) {
-#pragma unroll
-        for (int d = 0; d < D; ++d) {  // stage s + d: LDS buffer d % 2 (D is even)
-            compute(d % 2, w[d]);
-            __builtin_amdgcn_sched_barrier(0);
-            load_x(s + d + D, xr[d]);
-            load_w(s + d + D, w[d]);
-            __builtin_amdgcn_sched_barrier(0);
-            store_x((d + 1) % 2, xr[(d + 1) % D]);
-            __syncthreads();
-        }
-    }
+    wait_loads<0>();  // nothing is on its way to LDS any more
 
     // lane: row m = mt*16 + r of x, columns n_base + t*16 + g*4 + 0..3
 #pragma unroll
@@ -215,17 +203,25 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
                     for (int i = 0; i < 4 && n + i < N; ++i) dst[i] = acc[t][mt][i];
                 continue;
             }
-            for (int i = 0; i < 4 && n + i < N; ++i) {
-                float v = acc[t][mt][i];
-                if (!out_f32) v = round_to_bf16(v);
-                if (bias) { v += bias[n + i]; if (!out_f32) v = round_to_bf16(v); }
-                if (act == PTA_ACT_GELU) v = out_f32 ? gelu_erf(v) : gelu_bf16(v);  // other activations: see pta_gemm_splitk_bf16
-                if (add1) v += bf16_bits_to_f32(add1[o + i]);
-                if (add2) v += bf16_bits_to_f32(add2[o + i]);
-                if (out_f32) ((float*)y)[o + i] = v;
-                else ((bf16_t*)y)[o + i] = f32_to_bf16_bits(v);
-            }
+            for (int i = 0; i < 4 && n + i < N; ++i) store_whole(y, bias, add1, add2, act, out_f32, n + i, o + i, acc[t][mt][i]);
         }
+}
+
+// The same sums for rows too long for 32-bit offsets within a workgroup's rows (STREAM_MOST_K): a wave takes a row of W by a range of
+// K, one row of x after the other.  So that such products run; nothing was done for their speed.
+__global__ __launch_bounds__(64) void gemm_splitk_long_kernel(SplitkProblem p, int M) {
+    const int lane = threadIdx.x, n = blockIdx.x, range = blockIdx.y;
+    const long k0 = (long)range * p.blocks_per_part * 64, k1 = min((long)p.K, k0 + (long)p.blocks_per_part * 64);
+    for (int m = 0; m < M; ++m) {
+        float v = 0.f;
+        for (long k = k0 + lane; k < k1; k += 64) v += bf16_bits_to_f32(p.x[(long)m * p.K + k]) * bf16_bits_to_f32(p.W[(long)n * p.K + k]);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        if (lane != 0) continue;
+        const long o = (long)m * p.N + n;
+        if (p.direct) store_whole(p.y, p.bias, p.add1, p.add2, p.act, p.out_f32, n, o, v);
+        else p.part[(long)range * M * p.N + o] = v;
+    }
 }
 
 // y = act(sum over the parts + bias) + add1 + add2; parts are added in the order of their K ranges
@@ -380,27 +376,7 @@ static SplitkProblem make_problem(void* y, float* part, const void* x, const voi
     return p;
 }
 
-template <int MT, int RT, int U, int D>
-static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
-    const size_t lds = (size_t)2 * MT * 16 * (U * 64 + 8) * sizeof(bf16_t);
-    // rows of W a multiple of 4 KB long are the ones that crowd memory channels: there every workgroup starts at a
-    // stage of its own (PTA_SPLITK_ROT: stages between neighbours, 0 switches it off)
-    static const int rot_env = getenv("PTA_SPLITK_ROT") ? atoi(getenv("PTA_SPLITK_ROT")) : -1;
-    const int rot_stride = rot_env >= 0 ? rot_env : 1;
-    const bool rotate = rot_stride > 0 && (a.K % 2048 == 0 || (b.N > 0 && b.K % 2048 == 0));
-    auto kern = rotate ? gemm_splitk_kernel<MT, RT, U, D, true> : gemm_splitk_kernel<MT, RT, U, D, false>;
-    if (lds > 64 * 1024) {
-        static bool raised[2] = {false, false};  // per instantiation
-        if (!raised[rotate]) {
-            if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
-                return pta_fail("gemm_splitk_bf16: cannot have %zu bytes of LDS", lds);
-            raised[rotate] = true;
-        }
-    }
-    // rows beyond the MT tiles of a workgroup go to further chunks of workgroups, all of the same size
-    const int chunks = (M + MT * 16 - 1) / (MT * 16), chunk_rows = ((M + chunks - 1) / chunks + 15) / 16 * 16;
-    const dim3 grid((a.tiles * a.parts + b.tiles * b.parts) * chunks);
-    hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), lds, s, a, b, M, chunks, chunk_rows, rot_stride);
+static int reduce_parts(const SplitkProblem& a, int M, int reduce, hipStream_t s) {
     if (reduce && a.parts > 1) {
         const long MN = (long)M * a.N;
         hipLaunchKernelGGL(gemm_splitk_reduce_kernel, dim3((unsigned)((MN + 255) / 256)), dim3(256), 0, s, a.y, a.part,
@@ -409,27 +385,48 @@ static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int
     return pta_check_launch("gemm_splitk_bf16");
 }
 
+template <int MT, int RT, int D>
+static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
+    constexpr int lds = D * splitk_slot(MT, RT);
+    static_assert(lds <= 160 * 1024, "the stages must fit the LDS of a compute unit");
+    // rows of W a multiple of 4 KB long are the ones that crowd memory channels: there every workgroup starts at a
+    // stage of its own (PTA_SPLITK_ROT: stages between neighbours, 0 switches it off)
+    static const int rot_env = getenv("PTA_SPLITK_ROT") ? atoi(getenv("PTA_SPLITK_ROT")) : -1;
+    const int rot_stride = rot_env >= 0 ? rot_env : 1;
+    const bool rotate = rot_stride > 0 && (a.K % 2048 == 0 || (b.N > 0 && b.K % 2048 == 0));
+    auto kern = rotate ? gemm_splitk_kernel<MT, RT, D, true> : gemm_splitk_kernel<MT, RT, D, false>;
+    if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
+        return pta_fail("gemm_splitk_bf16: cannot have %d bytes of LDS", lds);
+    if (a.K > STREAM_MOST_K || b.K > STREAM_MOST_K) {
+        for (const SplitkProblem* p : {&a, &b})
+            if (p->N > 0) hipLaunchKernelGGL(gemm_splitk_long_kernel, dim3(p->N, p->parts), dim3(64), 0, s, *p, M);
+        return reduce_parts(a, M, reduce, s);
+    }
+    // rows beyond the MT tiles of a workgroup go to further chunks of workgroups, all of the same size
+    const int chunks = (M + MT * 16 - 1) / (MT * 16), chunk_rows = ((M + chunks - 1) / chunks + 15) / 16 * 16;
+    const dim3 grid((a.tiles * a.parts + b.tiles * b.parts) * chunks);
+    hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), lds, s, a, b, M, chunks, chunk_rows, rot_stride);
+    return reduce_parts(a, M, reduce, s);
+}
+
 // sixteen-row tiles of x that a workgroup holds: all rows up to SK_CHUNK_ROWS, else an even share of them
 static int tiles_per_chunk(int M) {
     const int chunks = (M + SK_CHUNK_ROWS - 1) / SK_CHUNK_ROWS;
     return ((M + chunks - 1) / chunks + 15) / 16;
 }
 
-template <int RT, int U, int D>
+#ifndef SKD
+#define SKD 4
+#endif
+template <int RT, int D = SKD>
 static int launch_rows(int MT, const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
     switch (MT) {
-        case 1: return launch_cfg<1, RT, U, D>(a, b, M, reduce, s);
-        case 2: return launch_cfg<2, RT, U, D>(a, b, M, reduce, s);
-        case 3: return launch_cfg<3, RT, U, D>(a, b, M, reduce, s);
-        case 4: return launch_cfg<4, RT, U, D>(a, b, M, reduce, s);
-        default:
-            // 65 to 128 rows: two stages in flight only (four would not fit the registers)
-            if constexpr (D == 2) {
-                if (MT <= 6) return launch_cfg<6, RT, U, D>(a, b, M, reduce, s);
-                return launch_cfg<8, RT, U, D>(a, b, M, reduce, s);
-            } else {
-                return pta_fail("gemm_splitk_bf16: more than 64 rows run with two stages in flight, not %d", D);
-            }
+        case 1: return launch_cfg<1, RT, D>(a, b, M, reduce, s);
+        case 2: return launch_cfg<2, RT, D>(a, b, M, reduce, s);
+        case 3: return launch_cfg<3, RT, D>(a, b, M, reduce, s);
+        case 4: return launch_cfg<4, RT, D>(a, b, M, reduce, s);
+        case 5: case 6: return launch_cfg<6, RT, D>(a, b, M, reduce, s);
+        default: return launch_cfg<8, RT, D>(a, b, M, reduce, s);
     }
 }
 
@@ -456,7 +453,6 @@ extern "C" int pta_gemm_splitk_bf16(void* y, float* part, const void* x, const v
     PTA_REQUIRE(parts >= 0 && parts <= 64, "gemm_splitk_bf16: parts must be 0 (choose) or 1..64, got %d", parts);
     if (rt == 0) rt = pick_rt(N);
     if (parts == 0) parts = pick_parts(N, K, rt);
-    if (depth == 0 || M > 64) depth = 2;  // measured: more stages in flight per wave do not pay, more workgroups do
     SplitkProblem a = make_problem(y, part, x, W, bias, add1, add2, N, K, act, out_f32, rt, parts, reduce);
     PTA_REQUIRE(a.direct || part, "gemm_splitk_bf16: %d ranges of K need the workspace for partial sums", a.parts);
     // One range of K ends in the matrix kernel itself, whose epilogue knows the exact GELU only (every activation
@@ -471,10 +467,8 @@ extern "C" int pta_gemm_splitk_bf16(void* y, float* part, const void* x, const v
     hipStream_t s = (hipStream_t)stream;
     const int MT = tiles_per_chunk(M);
     int rc;
-    if (rt == 1 && depth == 2) rc = launch_rows<1, 2, 2>(MT, a, none, M, reduce, s);
-    else if (rt == 1) rc = launch_rows<1, 2, 4>(MT, a, none, M, reduce, s);
-    else if (depth == 2) rc = launch_rows<2, 2, 2>(MT, a, none, M, reduce, s);
-    else rc = launch_rows<2, 2, 4>(MT, a, none, M, reduce, s);
+    if (rt == 1) rc = launch_rows<1>(MT, a, none, M, reduce, s);
+    else rc = launch_rows<2>(MT, a, none, M, reduce, s);
     if (rc || !after) return rc;
     return pta_epilogue(y, N, nullptr, add1, add2, M, N, act, PTA_BF16, stream);
 }
@@ -650,8 +644,8 @@ extern "C" int pta_gemm_splitk_pair_bf16(float* part1, const void* x1, const voi
     if (kind == 3) return pta_gemm_stationary_pair_bf16(part1, x1, W1, N1, K1, p1, part2, x2, W2, N2, K2, p2, M, stream);
     const SplitkProblem a = make_problem(nullptr, part1, x1, W1, nullptr, nullptr, nullptr, N1, K1, 0, 0, kind, p1, 0);
     const SplitkProblem b = make_problem(nullptr, part2, x2, W2, nullptr, nullptr, nullptr, N2, K2, 0, 0, kind, p2, 0);
-    if (kind == 2) return launch_rows<2, 2, 2>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
-    return launch_rows<1, 2, 2>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
+    if (kind == 2) return launch_rows<2>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
+    return launch_rows<1>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
 }
 
 // The same pair run to the end: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2) in bfloat16; the two
