@@ -22,7 +22,7 @@
 //
 // Measured against the 32-bit instruction, microseconds: 2,053 rows by 4,544 x 4,544 703 -> 432 (196 TFLOP/s), by 18,176 x 4,544
 // 2,632 -> 1,640 (207), by 4,544 x 18,176 2,787 -> 1,632 (208); 60 rows by the same 42 -> 35, 146 -> 95, 120 -> 102; one row 21.2
-// -> 21.3, 71 -> 68, 65 -> 65, by 65,024 x 4,544 239 -> 198 (6.0 TB/s).
+// -> 19.6, 71 -> 60, 65 -> 65, by 65,024 x 4,544 239 -> 198 (6.0 TB/s).
 //
 // Three ways to the same numbers, by what bounds them (few_rows, f32_plan):
 //   few rows: every weight is read once and that is the time.
@@ -31,6 +31,7 @@
 //   too few tiles to fill the chip, or to fill its last round: the segments of a tile are shared out over workgroups, whose
 //     sums go to memory and are added by a small launch.
 #include "common.h"
+#include "lds_stream.h"
 #include "pta_kernels.h"
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -252,6 +253,109 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
                 if (n + j < n1) C[(long)m * N + n + j] = finish(v[j], epi, n + j, (long)m * N + n + j);
         }
     }
+}
+
+// The same for up to sixteen rows of A where rows are sixteen-byte aligned: rows of W straight to LDS in whole lines (lds_stream.h),
+// D blocks ahead, a wave's segment at a time, and on to the workgroup's next rows without a pause: a workgroup has all the rows of W of a
+// compute unit, in tiles of up to 16 RT.  Sums change hands through LDS, in two places in turn, one barrier a tile.
+// 18,176 x 4,544, us with registers and three rounds of workgroups -> this: 1 row 70.0 -> 60.5 (5.5 TB/s), 16 rows 86.5 -> 67; 4,544 x
+// 18,176 67 -> 65, 83 -> 70; 32,768 x 2,048 59.9 -> 53.9, 72.3 -> 55.6.
+template <int RT, int D>
+struct FewRing {
+    static constexpr int SLOT = (RT + 1) * 2048, RING = D * SLOT, LOADS = 2 * (RT + 1);
+    static constexpr int LDS = SEGS * RING + 2 * SEGS * RT * 1024;
+};
+
+template <int RT, int D>
+__global__ __launch_bounds__(512, 2) void gemm_f32_few_ring_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W,
+                                                                   F32Epilogue epi, int M, int N, int K, int each, int over) {
+    using R = FewRing<RT, D>;
+    extern __shared__ __attribute__((aligned(1024))) char lds[];  // the waves' rings, then the sums, [2][segment][RT][64]
+    const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r16 = lane & 15, g = lane >> 4;
+    const int n0 = blockIdx.x * each + min((int)blockIdx.x, over), rows = each + ((int)blockIdx.x < over ? 1 : 0);
+    const int tiles = (rows + 16 * RT - 1) / (16 * RT), per_tile = (rows + tiles - 1) / tiles;
+    const int nb = k_blocks(K), sb = seg_blocks(K), used = segments(K);
+    const int b0 = seg * sb, b1 = min(nb, b0 + sb);
+    const i32x4_t w = buffer_of(W + (long)n0 * K, rows * K * 4), x = buffer_of(A, M * K * 4);
+    char* ring = lds + seg * R::RING;
+    const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(ring));
+    const int c4[2] = {stream_element(lane, 0) / 2, stream_element(lane, 1) / 2};  // four values where a bfloat16 row has eight
+    int x_at[2], w_at[2 * RT];
+#pragma unroll
+    for (int l = 0; l < 2; ++l) x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 4 : LDS_PAST;
+    auto rows_of = [&](int tile) {
+#pragma unroll
+        for (int l = 0; l < 2 * RT; ++l) {
+            const int i = (l >> 1) * 16 + stream_row(lane, l & 1), row = tile * per_tile + i;
+            w_at[l] = i < per_tile && row < rows ? row * K * 4 : LDS_PAST;
+        }
+    };
+    int p_tile = 0, p_block = b0;  // what is asked for next
+    auto issue = [&](int slot) {
+        const int k = p_block * BK;
+#pragma unroll
+        for (int l = 0; l < R::LOADS; ++l) {
+            const int row_at = l < 2 * RT ? w_at[l] : x_at[l & 1];
+            const int at = p_tile < tiles && p_block < b1 && row_at != LDS_PAST && k + c4[l & 1] < K ? row_at + (k + c4[l & 1]) * 4 : LDS_PAST;
+            fetch16(l < 2 * RT ? w : x, to + slot + l * 1024, at);
+        }
+        if (++p_block >= b1) {
+            p_block = b0;
+            rows_of(++p_tile);
+        }
+    };
+    rows_of(0);
+#pragma unroll
+    for (int d = 0; d < D; ++d) issue(d * R::SLOT);
+    const int in_row = r16 * 128 + ((g ^ (r16 >> 1)) & 7) * 16;  // elements 4 g of a block, and 64 flipped 16 + 4 g
+    f32x4* sums = reinterpret_cast<f32x4*>(lds + SEGS * R::RING);
+    int slot = 0;
+    for (int t = 0; t < tiles; ++t) {
+        f32x4 acc[RT];
+#pragma unroll
+        for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int b = b0; b < b1; ++b) {
+            wait_loads<(D - 1) * R::LOADS>();
+            f32x4 v[RT + 1][2];
+#pragma unroll
+            for (int r = 0; r <= RT; ++r)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) v[r][h] = *reinterpret_cast<const f32x4*>(ring + ((in_row ^ (h * 64)) + slot + r * 2048));
+            wait_reads();
+            __builtin_amdgcn_sched_barrier(0);
+            issue(slot);  // into the slot just read
+            __builtin_amdgcn_sched_barrier(0);
+            const Parts xs = split8(v[RT][0], v[RT][1]);
+#pragma unroll
+            for (int r = 0; r < RT; ++r) {
+                const Parts ws = split8(v[r][0], v[r][1]);
+#pragma unroll
+                for (int term = 0; term < TERMS; ++term)
+                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws.part[term_w(term)], xs.part[term_x(term)], acc[r], 0, 0, 0);
+            }
+            slot = slot == R::RING - R::SLOT ? 0 : slot + R::SLOT;
+        }
+        f32x4* mine = sums + (t & 1) * (SEGS * RT * 64);
+#pragma unroll
+        for (int r = 0; r < RT; ++r) mine[(seg * RT + r) * 64 + lane] = acc[r];
+        wait_reads();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        const int r = (seg - t * RT) & (SEGS - 1);  // the waves take turns at what follows
+        if (r >= RT) continue;
+        f32x4 u = mine[r * 64 + lane];
+        for (int s = 1; s < used; ++s) u += mine[(s * RT + r) * 64 + lane];
+        const int n_end = n0 + min(rows, (t + 1) * per_tile), n16 = n0 + t * per_tile + 16 * r;
+        if (any_not_finite(u)) u = plain_fragment<ROW_VECTORS>(u, A, W, 0, n16, M, N, K);
+        const int n = n16 + 4 * g;
+        if (r16 < M) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (n + j < n_end) C[(long)r16 * N + n + j] = finish(u[j], epi, n + j, (long)r16 * N + n + j);
+        }
+    }
+    wait_loads<0>();  // nothing is on its way to LDS any more
 }
 
 // ---- many rows ----------------------------------------------------------------------------------------------------------
@@ -530,22 +634,22 @@ static const F32Costs costs[2][4] = {
     {{0.92, 0.95, 0.0, 8.0, 8.0}, {1.19, 1.32, 0.0, 10.5, 10.5}, {1.52, 1.76, 0.0, 12.6, 12.0}, {1.84, 2.17, 0.0, 32.0, 12.5}},
 };
 
-// Which products the kernel for few rows has.  Measured, microseconds of few rows and of the best tiles:
+// Which products the kernels for few rows have.  Measured, microseconds of few rows and of the best tiles:
 //   N x K            1 row            8 rows           16 rows          17 rows          32 rows
 //   1,024 x 1,024     7.3 /   9.9      7.5 /  10.0      7.7 /  10.0      8.5 /   9.8     10.4 /   9.8
-//   4,096 x 1,024     7.8 /  11.9      8.8 /  12.0      9.7 /  12.1     10.4 /  12.2     12.1 /  11.9
-//   2,048 x 2,048     8.4 /  12.4     10.0 /  12.6     11.5 /  12.6     12.9 /  12.8     16.5 /  12.9
-//   4,544 x 4,544    21.0 /  25.9     23.5 /  25.9     27.0 /  26.3     31.6 /  26.3     36.8 /  26.8
-//   18,176 x 4,544   67.9 /  76.4     74.9 /  76.6     85.9 /  77.5     98.0 /  77.5      116 /  79.3
-//   32,768 x 2,048   61.2 /  61.6     66.3 /  61.9     72.2 /  62.7     80.2 /  63.5     90.3 /  64.3
-//   65,024 x 4,544    213 /   198      237 /   198      266 /   199      297 /   200      344 /   203
+//   4,096 x 1,024     7.6 /  11.9      7.6 /  12.0      7.8 /  12.1     10.4 /  12.2     12.1 /  11.9
+//   2,048 x 2,048     8.4 /  12.4      9.0 /  12.6      9.2 /  12.6     12.9 /  12.8     16.5 /  12.9
+//   4,544 x 4,544    19.6 /  25.9     21.2 /  25.9     21.5 /  26.3     31.6 /  26.3     36.8 /  26.8
+//   18,176 x 4,544   60.5 /  76.4     63.0 /  76.6     66.9 /  77.5     98.0 /  77.5      116 /  79.3
+//   32,768 x 2,048   53.9 /  61.6     55.4 /  61.9     55.6 /  62.7     80.2 /  63.5     90.3 /  64.3
+//   65,024 x 4,544    199 /   198      206 /   199      217 /   200      297 /   200      344 /   203
 // With a short K, whose segments are a block or two, rows up to 64: 256 x 512 33 rows 8.6 and 9.9, 64 rows 10.5 and 10.0.
 // Tiles address a row by 32-bit offsets (MOST_K).
 static bool few_rows(int M, int N, int K) {
     if (K > MOST_K) return true;
     if (K < 1024) return M <= 64;
     if (K < 2048) return M <= 32;
-    return M <= 16 && N < 32768 && (M <= 12 || (long)N * K < (1L << 24));
+    return M <= 16 && (N < 32768 || K < 4096);
 }
 
 static F32Plan f32_plan(int M, int N, int K) {
@@ -588,6 +692,17 @@ static void launch_few(float* C, const float* A, const float* W, F32Epilogue epi
     int groups = 256 * ((N + 256 * 32 - 1) / (256 * 32));
     if (groups > (N + 3) / 4) groups = (N + 3) / 4;
     const bool two = (N + groups - 1) / groups > 16;
+    // Rings in LDS: their offsets are 32-bit bytes within a workgroup's rows.  Up to sixteen rows of W a unit, whose waves take a block
+    // or two each, they pay from five rows of A on: 2,048 x 2,048 1 row 7.9 us, in rings 8.7, 8 rows 9.6 and 8.8, 16 rows 11.1 and 8.9.
+    const int units = groups < 256 ? groups : 256;  // one workgroup a unit, with its rows of all rounds
+    if (ROWS != ROW_ELEMENTS && rows <= 16 && (two || rows > 4) && (long)(N / units + 1) * K * 4 < LDS_PAST && (long)rows * K * 4 < LDS_PAST) {
+        auto go = [&](auto kernel, int bytes) {
+            if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
+            hipLaunchKernelGGL(kernel, dim3(units), dim3(512), bytes, s, C, A, W, epi, rows, N, K, N / units, N % units);
+            return true;
+        };
+        if (two ? go(gemm_f32_few_ring_kernel<2, 2>, FewRing<2, 2>::LDS) : go(gemm_f32_few_ring_kernel<1, 2>, FewRing<1, 2>::LDS)) return;
+    }
 #define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), dim3(groups), dim3(512), 0, s, C, A, W, epi, M, N, K)
     for (int at = 0; at < rows; at += 64) {  // more than 64 rows: where tiles cannot address K
         const int M = rows - at < 64 ? rows - at : 64;
