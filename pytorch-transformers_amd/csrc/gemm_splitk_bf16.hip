@@ -24,10 +24,12 @@
 
 #include <stdlib.h>
 
+#include <algorithm>
 #include <array>
 #include <map>
 #include <mutex>
 #include <utility>
+#include <vector>
 
 // bytes of a stage of 64 elements of K in LDS: four waves' rows of W, and the rows of x by whole loads of each wave
 static constexpr __host__ __device__ int splitk_slot(int MT, int RT) { return RT * 8192 + (MT + 1) / 2 * 4096; }
@@ -506,6 +508,65 @@ extern "C" int pta_gemm_splitk_pair_fix_parts(int N1, int K1, int N2, int K2, in
     return pta_gemm_splitk_pair_fix(N1, K1, N2, K2, p1, p2, 1);
 }
 
+// What a pair launch with `a` and `b` ranges takes at so many rows, in microseconds: the workgroups are handed to the compute units in
+// turn, as many at a time as LDS has room for (the rest goes to whichever is done first), and the launch takes as long as the unit
+// with the most blocks of 64 elements to pull, or as the chip does for all of them; a workgroup starts and ends in the time of six
+// blocks, uneven ranges cost 2 %, and partial sums are written and read again.  Put together from 1,500 launches of eight pairs of shapes at 8, 32 and 64
+// rows; what it picks takes on average 1 % longer than the fastest of them, at most 5.  Ranges of about 2,304 elements, the rule
+// before, and what this picks, us at 8, 32 and 64 rows (64: before with stationary activations):
+//   4,544 x 4,544 + 4,544 x 18,176   40.8 -> 40.2   42.9 -> 42.7   48.9 -> 43.9    9,216 + 32,768 x 8,192    129.5 -> 128.0   132.3 -> 129.4   148.6 -> 143.3
+//   4,096 x 4,096 + 4,096 x 16,384   36.5 -> 32.9   39.2 -> 33.8   41.4 -> 39.6    8,192 x 8,192 + 32,768    117.9 -> 111.8   127.7 -> 118.4   141.2 -> 139.7
+//   2,048 x 2,048 + 2,048 x 8,192    11.2 -> 10.5   12.8 -> 11.1   15.2 -> 13.3    7,680 + 20,480 x 5,120     54.3 -> 52.6    58.6 -> 60.2    71.6 -> 66.3
+static double pair_us(int N1, int K1, int a, int N2, int K2, int b, int rt, int rows) {
+    const int units = max(1, pta_compute_units()), slots = units * (rt == 1 ? (rows <= 32 ? 3 : 2) : rows <= 16 ? 2 : 1);
+    const double fixed = 6.0;
+    struct Run { int count; double blocks; } runs[4];
+    int n = 0;
+    long groups = 0;
+    double total = 0.0, longest = 0.0, uneven = 0.0;
+    for (int i = 0; i < 2; ++i) {
+        const int N = i ? N2 : N1, K = i ? K2 : K1, p = i ? b : a;
+        const int nkb = (K + 63) / 64, per = (nkb + p - 1) / p, parts = (nkb + per - 1) / per, tiles = (N + 64 * rt - 1) / (64 * rt);
+        runs[n++] = Run{tiles * (parts - 1), per + fixed};
+        runs[n++] = Run{tiles, nkb - (parts - 1) * per + fixed};
+        groups += (long)tiles * parts;
+        if (nkb % parts) uneven += (double)N * K / ((double)N1 * K1 + (double)N2 * K2);
+    }
+    for (const Run& r : runs) {
+        total += r.count * r.blocks;
+        if (r.count) longest = std::max(longest, r.blocks);
+    }
+    std::vector<double> load(units, 0.0);
+    int at = 0;
+    for (const Run& r : runs)
+        for (int j = 0; j < r.count && at < slots; ++j, ++at) load[at % units] += r.blocks;
+    const double mean = total / units;
+    double most = *std::max_element(load.begin(), load.end());
+    if (groups > slots) most = std::max(most, mean + 0.5 * longest);
+    const double bytes = 8192.0 * rt + 0.2 * 4096.0 * (((rows + 15) / 16 + 1) / 2);  // of a block: rows of W, and of x, which come from near by
+    return 4.0 + (1.0 + 0.02 * uneven) * std::max(most * bytes / 26e3, mean * bytes / 22.5e3) + ((double)a * N1 + (double)b * N2) * rows * 4.0 / 3e6;
+}
+
+// Ranges, and tiles of sixteen rows of W a wave, for steps of up to 32 rows (one tile) or of 33 to 64; kept by shape
+static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
+    static std::map<std::array<int, 5>, PairChoice> known;
+    const std::array<int, 5> key{N1, K1, N2, K2, rows};
+    std::lock_guard<std::mutex> hold(pair_parts_lock);
+    const auto it = known.find(key);
+    if (it != known.end()) return it->second;
+    PairChoice best{1, 1, 1};
+    double us = 1e30;
+    for (int rt = 1; rt <= (rows > 32 ? 2 : 1); ++rt)
+        for (int a = 1; a <= 8; ++a)
+            for (int b = 1; b <= 16; ++b) {
+                if (!parts_valid(K1, a) || !parts_valid(K2, b)) continue;
+                const double t = pair_us(N1, K1, a, N2, K2, b, rt, rows);
+                if (t < us) us = t, best = PairChoice{a, b, rt};
+            }
+    if (known.size() >= 1024) known.clear();
+    return known[key] = best;
+}
+
 // returns the row tiles per wave for steps of more than 32 rows
 static int pick_pair_parts(int N1, int K1, int N2, int K2, int* p1, int* p2) {
     {
@@ -517,17 +578,9 @@ static int pick_pair_parts(int N1, int K1, int N2, int K2, int* p1, int* p2) {
             return it->second.rt;
         }
     }
-    const int g1 = (N1 + 63) / 64, g2 = (N2 + 63) / 64;
-    const int range = range_for(min(g1, g2));
-    int a = clamp_parts((K1 + range / 2) / range, K1), b = clamp_parts((K2 + range / 2) / range, K2);
-    const int total = g1 * a + g2 * b;
-    if (total < splitk_target()) {
-        const int more = (splitk_target() + total - 1) / total;
-        a = clamp_parts(a * more, K1);
-        b = clamp_parts(b * more, K2);
-    }
-    *p1 = effective_parts(K1, a);
-    *p2 = effective_parts(K2, b);
+    const PairChoice c = pair_rule(N1, K1, N2, K2, 32);
+    *p1 = c.p1;
+    *p2 = c.p2;
     return 1;
 }
 
@@ -535,7 +588,7 @@ static int pick_pair_parts(int N1, int K1, int N2, int K2, int* p1, int* p2) {
 // ranges of its own, by the class of the step's rows (up to 16, 32, 64, 128).  The rule: ranges of about 1,400
 // elements, of the same length in both products, but no more of them than leave every wave at most the row tiles
 // it can hold with one workgroup per compute unit (past that the launch needs a second round of workgroups).
-// Measured against the staged kernel (us, staged -> stationary with the rule's ranges): K = 4,544 with N = 4,672
+// Measured against the staged kernel of its time, which brought W to registers (us, staged -> stationary with the rule's ranges): K = 4,544 with N = 4,672
 // + 18,176 at 8 / 32 / 64 / 128 rows 45.3 -> 40.5, 47.1 -> 43.1, 58.2 -> 46.5, 75.4 -> 56.0; K = 4,544 + 18,176
 // with N = 4,544: 44.9 -> 41.6, 48.8 -> 44.9, 57.5 -> 48.0, 72.6 -> 55.6; K = 4,096 with N = 6,144 + 16,384: 42.3
 // -> 38.4, 45.6 -> 40.1, 51.7 -> 45.1, 64.8 -> 55.1; K = 8,192 with N = 9,216 + 32,768: 141.8 -> 137.5, 158.5 ->
@@ -549,9 +602,13 @@ static int stationary_class(int M) { return M <= 16 ? 0 : M <= 32 ? 1 : M <= 64 
 struct StationaryChoice { int q1[STATIONARY_CLASSES], q2[STATIONARY_CLASSES]; };  // 0: the staged kernel
 static std::map<std::array<int, 4>, StationaryChoice> pair_stationary_fixed;
 
-// Without a fixed choice the launch is used from 33 rows on (classes 2 and 3): below, the staged kernel with timed
-// ranges is as fast or faster at most shapes.
+// Where one class of a shape is fixed, the others from 33 rows on (classes 2 and 3) have the rule's ranges; without a fixed choice the
+// launch is used from 65 rows on: below, the staged kernel is faster (pair_us), at 128 rows 53 us against its 57 for 4,672 + 18,176 x 4,544,
+// 163 against 167 for 9,216 + 32,768 x 8,192, 54 against 52 for 4,544 x 4,544 + 4,544 x 18,176, 158 against 168 for 8,192 x 8,192 + 32,768.
 #define STATIONARY_RULE_FROM_CLASS 2
+// (At 33 to 64 rows the staged kernel was timed for matrices of 4,096 rows together and more.)
+#define STATIONARY_UNFIXED_FROM_CLASS 3
+#define STAGED_FROM_ROWS 4096
 static void stationary_rule(int N1, int K1, int N2, int K2, int cls, int* q1, int* q2) {
     const int kmin = min(K1, K2), f1 = max(1, (K1 + kmin / 2) / kmin), f2 = max(1, (K2 + kmin / 2) / kmin);
     const long tiles = (long)((N1 + 15) / 16) * f1 + (long)((N2 + 15) / 16) * f2;
@@ -589,6 +646,11 @@ extern "C" int pta_gemm_splitk_pair_fix_stationary(int N1, int K1, int N2, int K
     return 0;
 }
 
+static bool pair_fixed(int N1, int K1, int N2, int K2) {
+    std::lock_guard<std::mutex> hold(pair_parts_lock);
+    return pair_parts_fixed.count({N1, K1, N2, K2}) != 0;
+}
+
 // The ranges of a pair launch of M rows and its kind: 3 with stationary activations, else the tiles of sixteen
 // rows of W per wave of the staged kernel (1 or 2).  M = 0 asks for the staged kernel's ranges.
 static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, int* p2) {
@@ -607,7 +669,14 @@ static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, 
         }
         if (!fixed) {
             q1 = q2 = 0;
-            if (cls >= STATIONARY_RULE_FROM_CLASS) stationary_rule(N1, K1, N2, K2, cls, &q1, &q2);
+            if (cls >= STATIONARY_UNFIXED_FROM_CLASS || (cls == 2 && N1 + N2 < STAGED_FROM_ROWS)) {
+                stationary_rule(N1, K1, N2, K2, cls, &q1, &q2);
+            } else if (cls == 2 && !pair_fixed(N1, K1, N2, K2)) {  // ranges and tiles of its own
+                const PairChoice c = pair_rule(N1, K1, N2, K2, 64);
+                *p1 = c.p1;
+                *p2 = c.p2;
+                return c.rt;
+            }
         }
         if (q1 > 0 && q2 > 0) {
             *p1 = q1;

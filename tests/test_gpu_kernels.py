@@ -379,6 +379,21 @@ def test_gemm_stationary_pair(M, shapes, parts):
         assert float((got - want).abs().max()) <= 2e-5 * float(want.abs().max()) + 1e-6
 
 
+@pytest.mark.parametrize("M", [8, 32, 33, 48, 64])
+@pytest.mark.parametrize("shapes", [((2100, 2112), (2008, 4608)), ((4104, 520), (1000, 520)), ((2048, 2048), (2048, 8192))])
+def test_gemm_splitk_pair_ranges_untuned(shapes, M):
+    """Pairs with the ranges and tile heights that the rule picks: the ranges reported are the ones left, and add up to the product."""
+    ops = _ops()
+    (N1, K1), (N2, K2) = shapes
+    x1, x2 = _rand(M, K1, dtype=torch.bfloat16), _rand(M, K2, seed=5, dtype=torch.bfloat16)
+    w1, w2 = _rand(N1, K1, seed=1, dtype=torch.bfloat16, scale=0.05), _rand(N2, K2, seed=2, dtype=torch.bfloat16, scale=0.05)
+    parts = ops.gemm_splitk_pair_partial(x1, w1, x2, w2)
+    assert tuple(p.shape[0] for p in parts) == ops.gemm_splitk_pair_parts(N1, K1, N2, K2, M)
+    for part, x, w in zip(parts, (x1, x2), (w1, w2)):
+        want = x.double() @ w.double().T
+        assert float((part.double().sum(0) - want).abs().max()) <= 2e-5 * float(want.abs().max())
+
+
 def test_gemm_stationary_pair_refusals_and_dispatch():
     """Rows beyond 128 are refused with a message; a pair launch of up to 128 rows runs with stationary activations
     and the ranges the library reports for the class of its rows; a class can be fixed to other ranges or to the
