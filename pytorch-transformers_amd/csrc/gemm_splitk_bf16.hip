@@ -144,32 +144,19 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
         int at = stage;
         if (ROT) { at += rot; at -= at >= nstages ? nstages : 0; }
         const int k = k_begin + at * 64;
-        const bool real = stage < nstages;
 #pragma unroll
         for (int l = 0; l < 2 * RT; ++l) {
             const int ke = k + c8[l & 1];
-            fetch16(rw, to_w + slot + l * 1024, real && ke < k_end ? w_at[l] + ke * 2 : LDS_PAST);
+            fetch16(rw, to_w + slot + l * 1024, ke < k_end ? w_at[l] + ke * 2 : LDS_PAST);
         }
 #pragma unroll
         for (int l = 0; l < NX; ++l) {
             const int ke = k + c8[wave & 1];  // (an even number of loads away from the wave's first: the same half of a tile)
-            fetch16(rx, to_x + slot + l * 4096, real && ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
+            fetch16(rx, to_x + slot + l * 4096, ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
         }
     };
     const int in_row = r * 128 + ((g ^ (r >> 1)) & 7) * 16;  // the second 32 elements of a stage: 64 flipped
-    // D - 1 stages are on their way.  One barrier a stage: behind it everyone's share of the stage has landed, and everyone is
-    // past reading the one before, whose place the next loads take.
-#pragma unroll
-    for (int d = 0; d < D - 1; ++d) issue(d, d * SLOT);
-    int cur = 0, free = (D - 1) * SLOT;
-    for (int s = 0; s < nstages; ++s) {
-        wait_reads();
-        wait_loads<(D - 2) * NL>();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-        issue(s + D - 1, free);
-        __builtin_amdgcn_sched_barrier(0);
+    auto multiply = [&](int cur) {
 #pragma unroll
         for (int hf = 0; hf < 2; ++hf) {
             bf16x8_t w[RT], b[MT];
@@ -184,10 +171,34 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
                 for (int mt = 0; mt < MT; ++mt)
                     acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], b[mt], acc[t][mt], 0, 0, 0);
         }
+    };
+    // everyone's share of the stage has landed, and everyone is past reading the one before
+    auto meet = [&]() {
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    // D - 1 stages are on their way, one barrier a stage, behind which the next loads take the place of the stage before; the last
+    // D - 1 stages wait for fewer and fewer.
+#pragma unroll
+    for (int d = 0; d < D - 1; ++d)
+        if (d < nstages) issue(d, d * SLOT);
+    int cur = 0, free = (D - 1) * SLOT;
+    for (int s = D - 1; s < nstages; ++s) {
+        wait_reads();
+        wait_loads<(D - 2) * NL>();
+        meet();
+        issue(s, free);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply(cur);
         free = cur;
         cur = cur == (D - 1) * SLOT ? 0 : cur + SLOT;
     }
-    wait_loads<0>();  // nothing is on its way to LDS any more
+    RingTail<NL>::template last_steps<D - 2>(nstages, [&]() {
+        meet();
+        multiply(cur);
+        cur = cur == (D - 1) * SLOT ? 0 : cur + SLOT;
+    });
 
     // lane: row m = mt*16 + r of x, columns n_base + t*16 + g*4 + 0..3
 #pragma unroll
@@ -417,10 +428,7 @@ static int tiles_per_chunk(int M) {
     return ((M + chunks - 1) / chunks + 15) / 16;
 }
 
-#ifndef SKD
-#define SKD 4
-#endif
-template <int RT, int D = SKD>
+template <int RT, int D = 4>
 static int launch_rows(int MT, const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
     switch (MT) {
         case 1: return launch_cfg<1, RT, D>(a, b, M, reduce, s);

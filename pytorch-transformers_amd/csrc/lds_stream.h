@@ -45,6 +45,19 @@ __device__ __forceinline__ int stream_element(int lane, int l) { return ((lane &
 // projection's rotation pairs (two heads of up to 256) too.
 #define STREAM_MOST_K (1 << 20)
 
+template <int LOADS>
+struct RingTail {
+    // the last steps, T + 1 of them if there are so many: each waits until only what is asked for behind it is on its way
+    template <int T, typename Step>
+    static __device__ __forceinline__ void last_steps(int n, Step step) {
+        if (T < n) {
+            wait_loads<T * LOADS>();
+            step();
+        }
+        if constexpr (T > 0) last_steps<T - 1>(n, step);
+    }
+};
+
 // RT tiles of sixteen rows of W and one of x, by steps of 64 elements of K: the wave takes the steps wave, wave + S, ..., D of
 // them on their way at a time.  w: each tile's buffer; w_at, x_at: byte offsets of the lane's rows (stream_row) within their
 // buffers, LDS_PAST for none.  The steps are walked from `rot` on, round.
@@ -54,44 +67,55 @@ struct RowStream {
     i32x4_t w[RT], x;
     int w_at[2 * RT], x_at[2];
 
-    __device__ __forceinline__ void run(f32x4_t (&acc)[RT], const char* ring, int lane, int wave, int S, int K, int nsteps, int rot) const {
+    // S: a power of two.  Loads are asked for as far as there are steps: the last D steps wait for fewer and fewer.
+    __device__ __forceinline__ void run(f32x4_t (&acc)[RT], const char* ring, int lane, int any_wave, int S, int K, int nsteps, int rot) const {
         const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(ring));
+        const int wave = __builtin_amdgcn_readfirstlane(any_wave);
         const int c8[2] = {stream_element(lane, 0), stream_element(lane, 1)};
         auto issue = [&](int step, int slot) {
-            const bool real = step < nsteps;
             int s = step + rot;
             s -= s >= nsteps ? nsteps : 0;
             const int k = s * 64;
 #pragma unroll
             for (int l = 0; l < LOADS; ++l) {
                 const int row_at = l < 2 * RT ? w_at[l] : x_at[l & 1];
-                const int at = real && row_at != LDS_PAST && k + c8[l & 1] < K ? row_at + (k + c8[l & 1]) * 2 : LDS_PAST;
+                const int at = row_at != LDS_PAST && k + c8[l & 1] < K ? row_at + (k + c8[l & 1]) * 2 : LDS_PAST;
                 fetch16(l < 2 * RT ? w[l >> 1] : x, to + slot + l * 1024, at);
             }
         };
-        const int r = lane & 15, g = lane >> 4;
-        const char* mine = ring + r * 128 + ((g ^ (r >> 1)) & 7) * 16;
-#pragma unroll
-        for (int d = 0; d < D; ++d) issue(wave + d * S, d * SLOT);
-        int slot = 0;
-        for (int step = wave; step < nsteps; step += S) {
-            wait_loads<(D - 1) * LOADS>();
-            bf16x8_t a[2][RT + 1];
+        const int in_row = (lane & 15) * 128 + (((lane >> 4) ^ ((lane & 15) >> 1)) & 7) * 16;
+        bf16x8_t a[2][RT + 1];
+        auto read = [&](int slot) {
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
-                for (int t = 0; t <= RT; ++t)
-                    a[hf][t] = *reinterpret_cast<const bf16x8_t*>(ring + (((mine - ring) ^ (hf * 64)) + slot + t * 2048));
-            wait_reads();
-            __builtin_amdgcn_sched_barrier(0);
-            issue(step + D * S, slot);  // into the slot just read
-            __builtin_amdgcn_sched_barrier(0);
+                for (int t = 0; t <= RT; ++t) a[hf][t] = *reinterpret_cast<const bf16x8_t*>(ring + ((in_row ^ (hf * 64)) + slot + t * 2048));
+        };
+        auto multiply = [&]() {
 #pragma unroll
             for (int hf = 0; hf < 2; ++hf)
 #pragma unroll
                 for (int t = 0; t < RT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[hf][t], a[hf][RT], acc[t], 0, 0, 0);
+        };
+        const int n = wave < nsteps ? (nsteps - wave + S - 1) >> __builtin_ctz(S) : 0;  // the wave's steps
+#pragma unroll
+        for (int d = 0; d < D; ++d)
+            if (d < n) issue(wave + d * S, d * SLOT);
+        int slot = 0, step = wave + D * S;
+        for (int i = D; i < n; ++i, step += S) {
+            wait_loads<(D - 1) * LOADS>();
+            read(slot);
+            wait_reads();
+            __builtin_amdgcn_sched_barrier(0);
+            issue(step, slot);  // into the slot just read
+            __builtin_amdgcn_sched_barrier(0);
+            multiply();
             slot = slot == RING - SLOT ? 0 : slot + SLOT;
         }
-        wait_loads<0>();  // nothing is on its way to LDS any more
+        RingTail<LOADS>::template last_steps<D - 1>(n, [&]() {
+            read(slot);
+            multiply();
+            slot = slot == RING - SLOT ? 0 : slot + SLOT;
+        });
     }
 };
