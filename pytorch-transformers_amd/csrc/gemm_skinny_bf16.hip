@@ -362,6 +362,33 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
     }
 }
 
+// What follows the halves kernels' sums: `sums` of wave w from w * stride on, items n0 .. n1 - 1 (rows, or rotation pairs)
+template <bool DIAG, typename OutT, bool TAIL>
+__device__ __forceinline__ void halves_end(const SkinnyProblem& p, const QkvTail& tail, const float* sums, int stride, int S, int M, int n0, int n1) {
+    const int half = TAIL ? tail.d >> 1 : 1;
+    auto sum_of = [&](int m, int i) {  // row i of the eight for row m of x
+        constexpr int OTHER = (32 + (DIAG ? 8 : 0)) * 4;
+        const int at = ((m >> 4) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
+        float v = sums[at] + sums[at + OTHER];
+        for (int w = 1; w < S; ++w) {
+            v += sums[w * stride + at];
+            v += sums[w * stride + at + OTHER];
+        }
+        return v;
+    };
+    if constexpr (TAIL) {
+        for (int item = threadIdx.x; item < 4 * M; item += blockDim.x) {
+            const int m = item >> 2, i = item & 3, pair = n0 + i;
+            if (pair < n1) qkv_tail_pair(tail, p.bias, m, pair / half, pair % half, round_to_bf16(sum_of(m, i)), round_to_bf16(sum_of(m, i + 4)));
+        }
+    } else {
+        for (int item = threadIdx.x; item < 8 * M; item += blockDim.x) {
+            const int m = item >> 3, i = item & 7;
+            if (n0 + i < n1) store_feature<OutT>((OutT*)p.y, p.bias, p.act, p.add1, p.add2, p.N, m, n0 + i, sum_of(m, i));
+        }
+    }
+}
+
 // Small matrices, eight rows of W or fewer a workgroup (N up to eight times the compute units): what bounds such a launch, apart
 // from its start, is not memory but the compute units' address paths, a wave's load taking sixteen cycles whatever it fetches,
 // and with eight rows in a tile of sixteen half of W's loads fetched nothing new.  So a tile is eight rows at two places of K:
@@ -441,30 +468,108 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
         __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt) part[(wave * MT + mt) * 64 + lane] = DIAG ? acc[0] : (g < 2 ? acc[mt * 2] : acc[BT > 1 ? mt * 2 + 1 : 0]);
-    __syncthreads();
-    const float* sums = (const float*)part;
-    auto sum_of = [&](int m, int i) {  // row i of the eight for row m of x
-        constexpr int OTHER = (32 + (DIAG ? 8 : 0)) * 4;
-        const int at = ((m >> 4) * 64 + (i >> 2) * 16 + (m & 15)) * 4 + (i & 3);
-        float v = sums[at] + sums[at + OTHER];
-        for (int w = 1; w < S; ++w) {
-            v += sums[w * MT * 256 + at];
-            v += sums[w * MT * 256 + at + OTHER];
-        }
-        return v;
-    };
-    if constexpr (TAIL) {
-        for (int item = threadIdx.x; item < 4 * M; item += blockDim.x) {
-            const int m = item >> 2, i = item & 3, pair = n0 + i;
-            if (pair < n1) qkv_tail_pair(tail, p.bias, m, pair / half, pair % half, round_to_bf16(sum_of(m, i)), round_to_bf16(sum_of(m, i + 4)));
-        }
-    } else {
-        for (int item = threadIdx.x; item < 8 * M; item += blockDim.x) {
-            const int m = item >> 3, i = item & 7;
-            if (n0 + i < n1) store_feature<OutT>((OutT*)p.y, p.bias, p.act, p.add1, p.add2, p.N, m, n0 + i, sum_of(m, i));
-        }
+    for (int mt = 0; mt < MT; ++mt) {
+        const f32x4_t first_half = acc[mt * (BT / MT)], second_half = acc[mt * (BT / MT) + BT / MT - 1];
+        part[(wave * MT + mt) * 64 + lane] = g < 2 || DIAG ? first_half : second_half;
     }
+    __syncthreads();
+    halves_end<DIAG, OutT, TAIL>(p, tail, (const float*)part, MT * 256, S, M, n0, n1);
+}
+
+// The same through LDS (lds_stream.h): a step of 128 elements of K is two lines of each of the eight rows, and they lie in the slot
+// as the tile's two halves; D steps are on their way.  The sums and their order are the kernel's above, which is left for rows that
+// are too long for the buffers' 32-bit offsets, and for eight waves with more than sixteen rows of x, whose rings LDS cannot hold.
+// Over cold weights, 8 / 16 / 32 / 64 rows of x, from registers -> here, us: 2,048 x 8,192 11.8 -> 8.6, 16.0 -> 10.4, 23.1 -> 13.7, 41.5 ->
+// 21.5; 2,048 x 2,048 6.1 -> 4.6, 7.3 -> 5.0, 9.7 -> 6.1, 15.3 -> 9.0; 1,040 x 4,160 7.5 -> 5.2, 9.8 -> 6.0, 13.8 -> 8.1, 24.1 -> 11.5; 640 x
+// 2,048 5.3 -> 3.9, 6.6 -> 4.3, 9.0 -> 5.4, 14.4 -> 7.3.  What bounds it: with few rows the start and the end (2.3 us for 300 x 72), then
+// the weights (2,048 x 8,192: 3.9 TB/s); with many the reading of x, all of which every workgroup needs (64 rows of 8,192: 1 MB each).
+template <int MT, bool DIAG, int D, typename OutT, bool TAIL>
+__global__ __launch_bounds__(512) void gemm_skinny_halves_ring_kernel(SkinnyProblem p, int M, int K, int rot_stride, QkvTail tail) {
+    static_assert(!DIAG || MT == 1, "both halves of K in a tile: eight rows of x");
+    constexpr int BT = DIAG ? 1 : 2 * MT, SLOT = 2048 * (1 + BT), RING = D * SLOT, LOADS = 2 * (1 + BT), WAVE = RING / 16;
+    extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums, [64] each
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = blockDim.x >> 6;
+    const int r = lane & 15, g = lane >> 4, half = TAIL ? tail.d >> 1 : 1;
+    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);  // pairs, or rows
+    const int nsteps = (K + 127) >> 7, rot = start_step(rot_stride, nsteps);
+    const int row = lane >> 3;  // the row that the lane's sixteen bytes are of
+    int first = n0, at_row;     // of W: the row that the others are counted from, and the lane's
+    if (TAIL) {
+        const int pair = n0 + (row & 3);
+        int e[2];
+        bool rotated;
+        qkv_tail_pair_elements(tail.rot, tail.d, pair % half, e[0], e[1], rotated);
+        first = n0 / half * tail.d;
+        at_row = pair < n1 ? pair / half * tail.d + (row < 4 ? e[0] : e[1]) - first : -1;
+    } else {
+        at_row = n0 + row < n1 ? row : -1;
+    }
+    const i32x4_t w = buffer_of(p.W + (long)first * K, (TAIL ? min((tail.nh + 2 * tail.nkv) * tail.d - first, 2 * tail.d) : n1 - n0) * K * 2);
+    const i32x4_t x = buffer_of(p.x, M * K * 2);
+    const int w_at = at_row >= 0 ? at_row * K * 2 : LDS_PAST;
+    int x_at[2 * MT];
+#pragma unroll
+    for (int i = 0; i < 2 * MT; ++i) x_at[i] = row + 8 * i < M ? (row + 8 * i) * K * 2 : LDS_PAST;
+    const int c8[2] = {stream_element(lane, 0), stream_element(lane, 1)};
+    const char* ring = (const char*)(part + wave * WAVE);
+    const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(ring));
+    auto issue = [&](int step, int slot) {
+        int s = step + rot;
+        s -= s >= nsteps ? nsteps : 0;
+#pragma unroll
+        for (int l = 0; l < LOADS; ++l) {  // W: a half of K a load; x: the same with eight rows, else a half of K a tile
+            const int k = s * 128 + (l < 2 || DIAG ? l & 1 : (l - 2) >> 1 & 1) * 64 + c8[l & 1];
+            const int from = l < 2 ? w_at : x_at[l < 2 || DIAG ? 0 : ((l - 2) >> 2) * 2 + (l & 1)];
+            fetch16(l < 2 ? w : x, to + slot + l * 1024, from != LDS_PAST && k < K ? from + k * 2 : LDS_PAST);
+        }
+    };
+    f32x4_t acc[BT];
+#pragma unroll
+    for (int t = 0; t < BT; ++t) acc[t] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    const int in_row = r * 128 + ((g ^ (r >> 1)) & 7) * 16;
+    bf16x8_t a[2], b[2][BT];
+    auto read = [&](int slot) {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf) {
+            const int at = (in_row ^ (hf * 64)) + slot;
+            a[hf] = *reinterpret_cast<const bf16x8_t*>(ring + at);
+#pragma unroll
+            for (int t = 0; t < BT; ++t) b[hf][t] = *reinterpret_cast<const bf16x8_t*>(ring + at + 2048 * (1 + t));
+        }
+    };
+    auto multiply = [&]() {
+#pragma unroll
+        for (int hf = 0; hf < 2; ++hf)
+#pragma unroll
+            for (int t = 0; t < BT; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[hf], b[hf][t], acc[t], 0, 0, 0);
+    };
+    const int n = wave < nsteps ? (nsteps - wave + S - 1) >> __builtin_ctz(S) : 0;  // the wave's steps
+#pragma unroll
+    for (int d = 0; d < D; ++d)
+        if (d < n) issue(wave + d * S, d * SLOT);
+    int slot = 0, step = wave + D * S;
+    for (int i = D; i < n; ++i, step += S) {
+        wait_loads<(D - 1) * LOADS>();
+        read(slot);
+        wait_reads();
+        __builtin_amdgcn_sched_barrier(0);
+        issue(step, slot);  // into the slot just read
+        __builtin_amdgcn_sched_barrier(0);
+        multiply();
+        slot = slot == RING - SLOT ? 0 : slot + SLOT;
+    }
+    RingTail<LOADS>::template last_steps<D - 1>(n, [&]() {
+        read(slot);
+        multiply();
+        slot = slot == RING - SLOT ? 0 : slot + SLOT;
+    });
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const f32x4_t first_half = acc[mt * (BT / MT)], second_half = acc[mt * (BT / MT) + BT / MT - 1];
+        part[wave * WAVE + mt * 64 + lane] = g < 2 || DIAG ? first_half : second_half;
+    }
+    __syncthreads();
+    halves_end<DIAG, OutT, TAIL>(p, tail, (const float*)part, WAVE * 4, S, M, n0, n1);
 }
 
 // The input product of a gated feed-forward, W = [gate rows, up rows], with the gate in its epilogue: y[M, F] = glu(x . Wg^T, x . Wu^T)
@@ -722,15 +827,38 @@ static int launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hip
 // where a workgroup has eight rows of W or fewer (N alone decides: one order of summation for any number of rows of x)
 static bool by_halves(int N) { return N <= 8 * pta_compute_units(); }
 
+template <int N> using I = std::integral_constant<int, N>;
+
 template <typename OutT, bool TAIL = false>
 static int launch_halves(SkinnyProblem p, int M, int K, int S, hipStream_t s, const QkvTail& tail = QkvTail{}) {
     const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 4 : 8, units = pta_compute_units();
-    if (S <= 0) S = 2;  // four waves 5.9 us at 2,048 x 2,048 and 8 rows, 7.6 at 16, two 5.4 and 6.7; longer rows within 2 %
+    // Waves by N alone, as the order of the sums must not depend on x: four where a workgroup has five rows or fewer and its waves
+    // spend their time starting (8 rows of x, two -> four: 1,040 x 4,160 5.2 -> 4.9 us, 640 x 2,048 3.6 -> 3.2, 1,024 x 4,096 5.1 -> 4.8),
+    // else two (2,048 x 8,192 8.3, four 9.0; 2,048 x 2,048 4.3, four 4.6).
+    if (S <= 0) S = p.N <= 5 * units ? 4 : 2;
     const dim3 grid(std::max((items + most - 1) / most, std::min(units, (items + most / 2 - 1) / (most / 2)))), block(S * 64);
     p.rows = Share(items, (int)grid.x);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 3 : 0);
     auto go = [&](auto kernel, int tiles) { hipLaunchKernelGGL(kernel, grid, block, (size_t)S * tiles * 64 * sizeof(f32x4_t), s, p, M, K, rot, tail); };
+    if (K <= STREAM_MOST_K && (M <= 16 || S <= 4)) {
+        int rc = 0;
+        auto ring = [&](auto kernel, int bytes) { rc = launch_rings(kernel, grid, block, (size_t)S * bytes, s, p, M, K, rot, tail); };
+        auto of_depth = [&](auto tiles, auto few, auto two, auto four, auto eight) {  // loads on their way that LDS has room for
+            constexpr int MT = tiles(), SLOT = 2048 * (few() ? 2 : 1 + 2 * MT);
+            if (S <= 2) ring(gemm_skinny_halves_ring_kernel<MT, few(), two(), OutT, TAIL>, two() * SLOT);
+            else if (S <= 4) ring(gemm_skinny_halves_ring_kernel<MT, few(), four(), OutT, TAIL>, four() * SLOT);
+            else if constexpr (eight() > 0) ring(gemm_skinny_halves_ring_kernel<MT, few(), eight(), OutT, TAIL>, eight() * SLOT);
+        };
+        if (M <= 8) of_depth(I<1>(), std::true_type(), I<6>(), I<6>(), I<4>());
+        else if (M <= 16) of_depth(I<1>(), std::false_type(), I<6>(), I<6>(), I<3>());
+        else if constexpr (!TAIL) {
+            if (M <= 32) of_depth(I<2>(), std::false_type(), I<4>(), I<3>(), I<0>());
+            else if (M <= 48) of_depth(I<3>(), std::false_type(), I<4>(), I<2>(), I<0>());
+            else of_depth(I<4>(), std::false_type(), I<4>(), I<2>(), I<0>());
+        }
+        return rc ? rc : pta_check_launch("gemm_skinny_bf16");
+    }
     if (M <= 8) go(gemm_skinny_halves_kernel<1, true, 2, OutT, TAIL>, 1);
     else if (M <= 16) go(gemm_skinny_halves_kernel<1, false, 2, OutT, TAIL>, 1);
     else if constexpr (!TAIL) {

@@ -114,6 +114,25 @@ def test_gemm_skinny_bf16_through_lds(N, K):
         assert torch.equal(ops.gemm_skinny_bf16(x[:m].contiguous(), w, out_f32=True), got[:m]), m
 
 
+# eight rows of W a workgroup and fewer, up to 64 rows of x: four waves and two, fewer steps than a ring holds, a ring's length and more
+@pytest.mark.parametrize("N", [1, 1279, 1280, 1281, 2048])
+@pytest.mark.parametrize("K", [8, 136, 640, 2056])
+def test_gemm_skinny_bf16_halves_through_lds(N, K):
+    """Every height of the tiles of x has the same bits, and waves that are asked for keep to the sums' rounding."""
+    ops = _ops()
+    x = _rand(64, K, dtype=torch.bfloat16)
+    w = _rand(N, K, seed=1, dtype=torch.bfloat16, scale=0.05)
+    prod = x.double() @ w.double().T.contiguous()
+    tol = 2e-5 * float(prod.abs().max()) + 1e-6
+    got = ops.gemm_skinny_bf16(x, w, out_f32=True)
+    assert float((got.double() - prod).abs().max()) <= tol
+    for m in (1, 8, 9, 16, 17, 32, 33, 48, 49):
+        assert torch.equal(ops.gemm_skinny_bf16(x[:m].contiguous(), w, out_f32=True), got[:m]), m
+        for waves in (1, 8):
+            of = ops.gemm_skinny_bf16(x[:m].contiguous(), w, out_f32=True, waves=waves)
+            assert float((of.double() - prod[:m]).abs().max()) <= tol, (m, waves)
+
+
 @pytest.mark.parametrize("M", [1, 20])
 def test_few_row_products_of_very_long_rows(M):
     """Rows of W beyond what the launches through LDS address (2^20 elements)."""
