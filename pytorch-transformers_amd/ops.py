@@ -1566,6 +1566,14 @@ def gemm_skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     return _bf16_rows_ok(x, w) and 0 < x.shape[0] <= 16
 
 
+def gemm_skinny_small_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
+    """Whether the kernel for few rows is the faster choice also for 17 to 32 rows: eight rows of W a compute unit or fewer,
+    and rows of up to 8,192 elements.  Over cold weights, the decode batch kernel -> this one, 17 / 32 rows, us: 2,048 x 2,048
+    7.8 -> 5.8, 8.1 -> 6.1; 1,040 x 4,160 8.8 -> 7.0, 8.7 -> 8.1; 640 x 2,048 7.2 -> 4.9, 7.4 -> 5.4; 2,048 x 8,192 14.7 -> 13.8, 14.8
+    -> 14.0; but 2,048 x 16,384 20.9 -> 24.7 (every workgroup reads all of x), and at 40 rows 1,040 x 4,160 9.0 -> 9.9."""
+    return 16 < x.shape[0] <= 32 and w.shape[0] <= 8 * compute_units() and w.shape[1] <= 8192 and gemm_splitk_ok(x, w)
+
+
 def gemm_splitk_pair_ok(x1: torch.Tensor, w1: torch.Tensor, x2: torch.Tensor, w2: torch.Tensor) -> bool:
     """Whether the two products run as a pair launch of the decode batch kernel (17 to 256 rows; beyond 128 only
     where the pair was timed faster than the library's two products)."""

@@ -110,7 +110,7 @@ class Linear(Part):
         bias = self.bias if apply_bias else None
         if x.dtype == torch.float32:
             return ops.gemm_f32(x, self.weight, bias, act, add1, add2)
-        if ops.gemm_skinny_ok(x, self.weight):
+        if ops.gemm_skinny_ok(x, self.weight) or ops.gemm_skinny_small_ok(x, self.weight):
             return ops.gemm_skinny_bf16(x, self.weight, bias, act, add1, add2)
         if ops.gemm_splitk_ok(x, self.weight):
             return ops.gemm_splitk_bf16(x, self.weight, bias, act, add1, add2)

@@ -161,6 +161,21 @@ def test_rows_beyond_one_chunk_take_the_way_that_was_timed_faster(monkeypatch):
     assert ops.gemm_splitk_ok(x[:128].contiguous(), first.weight)
 
 
+@pytest.mark.parametrize("M,N,K,few", [(16, 640, 520, False), (17, 640, 520, True), (32, 2048, 2048, True), (33, 640, 520, False),
+                                       (17, 2056, 2048, False), (17, 8, 8192, True), (17, 8, 8200, False)])
+def test_small_matrices_take_up_to_32_rows_as_few(M, N, K, few):
+    """Where the kernel for few rows stands in for the decode batch kernel, and a row, a column and an element further on."""
+    from pytorch_transformers_amd import ops
+    from pytorch_transformers_amd.parts import Linear
+
+    lin = Linear("a", K, N, bias=True)
+    _, ref = _fill(lin, torch.bfloat16, 1)
+    x = _rand(M, K, seed=3).bfloat16().cuda()
+    if ops.compute_units() == 256:
+        assert ops.gemm_skinny_small_ok(x, lin.weight) == few
+    _close(lin(x, act="gelu"), P.gelu(P.linear(x.double().cpu(), ref["a.weight"], ref["a.bias"])), 2e-2, "product")
+
+
 def test_library_product_over_ranges_of_k():
     """A few hundred rows with K long against N: the library's batched product over ranges of K, its 32-bit
     partial sums added in order by the kernel that applies bias, activation and additions.  Which way is
