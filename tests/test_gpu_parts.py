@@ -176,6 +176,20 @@ def test_small_matrices_take_up_to_32_rows_as_few(M, N, K, few):
     _close(lin(x, act="gelu"), P.gelu(P.linear(x.double().cpu(), ref["a.weight"], ref["a.bias"])), 2e-2, "product")
 
 
+@pytest.mark.parametrize("M,N,K,ok", [(17, 8192, 264, True), (64, 8192, 264, True), (65, 8192, 264, False), (17, 8200, 264, False),
+                                      (32, 2000, 64, True), (33, 2000, 64, False), (128, 4096, 1024, True), (128, 4104, 1024, False)])
+def test_products_long_in_n_as_a_decode_batch(M, N, K, ok):
+    """Where the decode batch kernel takes matrices that are long against K, and a row or some columns further on."""
+    from pytorch_transformers_amd import ops
+    from pytorch_transformers_amd.parts import Linear
+
+    lin = Linear("a", K, N, bias=True)
+    _, ref = _fill(lin, torch.bfloat16, 1)
+    x = _rand(M, K, seed=3).bfloat16().cuda()
+    assert ops.gemm_splitk_ok(x, lin.weight) == (ok and M <= ops.SPLITK_MAX_ROWS)
+    _close(lin(x, act="gelu"), P.gelu(P.linear(x.double().cpu(), ref["a.weight"], ref["a.bias"])), 2e-2, "product")
+
+
 def test_library_product_over_ranges_of_k():
     """A few hundred rows with K long against N: the library's batched product over ranges of K, its 32-bit
     partial sums added in order by the kernel that applies bias, activation and additions.  Which way is
