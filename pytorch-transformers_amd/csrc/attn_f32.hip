@@ -74,15 +74,6 @@ __device__ __forceinline__ void load_query(const AttnF32& a, const Column& c, in
     }
 }
 
-__device__ __forceinline__ float across_max(float v) {  // over the four lanes of a column
-    v = fmaxf(v, __shfl_xor(v, 16));
-    return fmaxf(v, __shfl_xor(v, 32));
-}
-__device__ __forceinline__ float across_sum(float v) {
-    v += __shfl_xor(v, 16);
-    return v + __shfl_xor(v, 32);
-}
-
 // One page for CT tiles: m, l and o of its keys alone.  ``seen[c]``: whether column c looks at this page's sequence at all.
 // ``end``: keys of the sequence that any column of the wave sees (what lies behind is whatever the page held before).  ``spare``:
 // LDS of the wave's own for the weights of the page.
@@ -131,7 +122,7 @@ __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, con
                 s[c][t][e] = v;
                 top = fmaxf(top, v);
             }
-        top = across_max(top);
+        top = column_max(top);
         const float base = top == -INFINITY ? 0.f : top;
         float sum = 0.f;
 #pragma unroll
@@ -143,7 +134,7 @@ __device__ __forceinline__ void page_pass(const AttnF32& a, const float* kp, con
                 s[c][t][e] = p;
                 sum += p;
             }
-        m[c] = top, l[c] = across_sum(sum);
+        m[c] = top, l[c] = column_sum(sum);
     }
     const bool ragged = __ballot(!whole) != 0;
 #pragma unroll

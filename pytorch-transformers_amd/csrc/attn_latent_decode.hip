@@ -151,8 +151,7 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
                 p[i] = kb + 16 * wave + 4 * g + i < k1 ? sc[0][i] + sc[1][i] : -INFINITY;
                 top = fmaxf(top, p[i]);
             }
-            top = fmaxf(top, __shfl_xor(top, 16));
-            top = fmaxf(top, __shfl_xor(top, 32));
+            top = column_max(top);
             if (g == 0) stat[wave * 16 + r16] = top;
             __syncthreads();
             const float m_new = fmaxf(fmaxf(fmaxf(stat[r16], stat[16 + r16]), fmaxf(stat[32 + r16], stat[48 + r16])), m_run);
@@ -166,8 +165,7 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
                 sum += bf16_bits_to_f32(w.b[i]);  // the weights as they were rounded
             }
             *(uint2*)(Ps + r16 * 72 + 16 * wave + 4 * g) = w.u;
-            sum += __shfl_xor(sum, 16);
-            sum += __shfl_xor(sum, 32);
+            sum = column_sum(sum);
             if (g == 0) stat[64 + wave * 16 + r16] = sum;
             __syncthreads();
             l_run = l_run * corr + (stat[64 + r16] + stat[80 + r16] + stat[96 + r16] + stat[112 + r16]);

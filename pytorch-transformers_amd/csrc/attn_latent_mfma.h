@@ -199,8 +199,7 @@ __global__ __launch_bounds__(256) void attn_latent_mfma_kernel(const LatentArgs 
                 p[tt * 4 + r] = see ? sc[tt][r] : -INFINITY;
                 m_blk = fmaxf(m_blk, p[tt * 4 + r]);
             }
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 16, 64));
-        m_blk = fmaxf(m_blk, __shfl_xor(m_blk, 32, 64));
+        m_blk = column_max(m_blk);
         const float m_new = fmaxf(m_run, m_blk);
         const bool none = m_new == -INFINITY;  // the column has seen no key yet
         const float corr = none ? 1.f : expf(m_run - m_new);
@@ -236,8 +235,7 @@ __global__ __launch_bounds__(256) void attn_latent_mfma_kernel(const LatentArgs 
                 }
         }
     }
-    float l_tot = l_run + __shfl_xor(l_run, 16, 64);
-    l_tot += __shfl_xor(l_tot, 32, 64);
+    const float l_tot = column_sum(l_run);
     if (!valid) return;
     // oacc[dt][r] is element dt * 16 + g * 4 + r of column j
     if (a.n_splits == 1) {

@@ -201,7 +201,7 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
         float mx = sc[0];
 #pragma unroll
         for (int e = 1; e < 16; ++e) mx = fmaxf(mx, sc[e]);
-        mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        mx = fold_32(mx, LaneMax());
         if (h == 0) maxima[kw * 32] = mx;
         // Rows r0 .. r1 - 1 are seen by some columns of the workgroup only (a few of its last page).  A value among them that is
         // infinite or undefined must reach those alone, and a weight of zero would not keep it from the others.
@@ -320,7 +320,7 @@ __global__ __launch_bounds__(256, 1) void attn_latent_prompt_kernel(const Latent
         lp_wait_loads<0>();  // the next page has landed
         lp_meet();
     }
-    float l = l_run + __shfl_xor(l_run, 32, 64);
+    float l = fold_32(l_run, LaneSum());
     if (h == 0) maxima[kw * 32] = l;
     lp_meet();
     l += maxima[(kw ^ 1) * 32];

@@ -292,8 +292,7 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
         for (int ct = 0; ct < CT; ++ct) {
             if (!__any(mx[ct] > m_raise[ct])) continue;
             float m = mx[ct] * s_mul;
-            m = fmaxf(m, __shfl_xor(m, 16, 64));
-            m = fmaxf(m, __shfl_xor(m, 32, 64));
+            m = column_max(m);
             const float m_new = fmaxf(m_run[ct], m);
             const float corr = __builtin_amdgcn_exp2f(m_run[ct] - (m_new == -INFINITY ? 0.f : m_new));
             lacc[ct][0] *= corr;  // the one row of the sums that is read at the end

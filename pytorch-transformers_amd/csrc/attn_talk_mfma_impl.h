@@ -260,8 +260,7 @@ __global__ __launch_bounds__(64 * MAXW) void attn_talk_mfma_kernel(
             // it is brought up (and what was summed rescaled) only when a score lies more than 2^8 above it
             if (__any(mx > m_raise[ct])) {
                 float m = mx * TALK_LOG2E;
-                m = fmaxf(m, __shfl_xor(m, 16, 64));
-                m = fmaxf(m, __shfl_xor(m, 32, 64));
+                m = column_max(m);
                 const float m_new = fmaxf(m_run[ct], m);
                 const float corr = __builtin_amdgcn_exp2f(m_run[ct] - (m_new == -INFINITY ? 0.f : m_new));
                 lacc[ct][0] *= corr;

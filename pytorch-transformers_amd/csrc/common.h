@@ -71,16 +71,33 @@ template <> struct Io<bf16_t> {
     static __device__ __forceinline__ float round(float v) { return round_to_bf16(v); }
 };
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// Sums and maxima over lanes, for whole waves.  Between the rows of sixteen lanes by the instructions that exchange halves and rows
+// of two registers, within a row by rotated operands: seven instructions in a chain for a wave where __shfl_xor goes through LDS
+// six times, each some hundred cycles and a wait.  The additions and their order are those of v + __shfl_xor(v, o) with o as named: a
+// rotation by o brings lane i the value of lane i ^ o once those of lanes that are 2 o apart are equal.
+struct LaneSum { __device__ __forceinline__ float operator()(float a, float b) const { return a + b; } };
+struct LaneMax { __device__ __forceinline__ float operator()(float a, float b) const { return fmaxf(a, b); } };
+template <typename Op> __device__ __forceinline__ float fold_32(float v, Op op) {  // with lane ^ 32
+    const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+template <typename Op> __device__ __forceinline__ float fold_16(float v, Op op) {  // with lane ^ 16
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return op(__uint_as_float(p[0]), __uint_as_float(p[1]));
 }
+template <int O, typename Op> __device__ __forceinline__ float fold_turned(float v, Op op) {
+    return op(v, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x120 + O, 0xf, 0xf, true)));  // row_ror:O
+}
+template <typename Op> __device__ __forceinline__ float wave_fold(float v, Op op) {
+    v = fold_16(fold_32(v, op), op);
+    v = fold_turned<4>(fold_turned<8>(v, op), op);
+    return fold_turned<1>(fold_turned<2>(v, op), op);
+}
+__device__ __forceinline__ float wave_sum(float v) { return wave_fold(v, LaneSum()); }
+__device__ __forceinline__ float wave_max(float v) { return wave_fold(v, LaneMax()); }
+// over the four lanes that hold a column of a matrix instruction's result
+__device__ __forceinline__ float column_sum(float v) { return fold_32(fold_16(v, LaneSum()), LaneSum()); }
+__device__ __forceinline__ float column_max(float v) { return fold_32(fold_16(v, LaneMax()), LaneMax()); }
 
 // Sum over a block of up to 1024 threads; every thread gets the result.  `red`
 // is LDS of at least 16 floats.  The order of additions depends on the block

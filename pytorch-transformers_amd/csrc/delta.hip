@@ -256,8 +256,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
                 S[i] *= gg.x; S[i + 1] *= gg.y; S[i + 2] *= gg.z; S[i + 3] *= gg.w;
                 u += S[i] * kk.x; u += S[i + 1] * kk.y; u += S[i + 2] * kk.z; u += S[i + 3] * kk.w;
             }
-            u += __shfl_xor(u, 16, 64);
-            u += __shfl_xor(u, 32, 64);
+            u = column_sum(u);
             u = b_s[tt] * (v_s[tt * 64 + pw] - u);
 #pragma unroll
             for (int i = 0; i < NPT; i += 4) {
@@ -265,8 +264,7 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
                 S[i] += kk.x * u; S[i + 1] += kk.y * u; S[i + 2] += kk.z * u; S[i + 3] += kk.w * u;
                 o += S[i] * qq.x; o += S[i + 1] * qq.y; o += S[i + 2] * qq.z; o += S[i + 3] * qq.w;
             }
-            o += __shfl_xor(o, 16, 64);
-            o += __shfl_xor(o, 32, 64);
+            o = column_sum(o);
             if (g4 == 0 && p < P) y[((long)(c0 + tt) * heads + h) * P + p] = o;
         }
     }
@@ -374,10 +372,8 @@ __global__ __launch_bounds__(256) void delta_block_kernel(float* __restrict__ ha
     __syncthreads();
 #pragma unroll
     for (int t = 0; t < 16; ++t) {
-        lk[t] += __shfl_xor(lk[t], 16, 64);
-        lk[t] += __shfl_xor(lk[t], 32, 64);
-        aq[t] += __shfl_xor(aq[t], 16, 64);
-        aq[t] += __shfl_xor(aq[t], 32, 64);
+        lk[t] = column_sum(lk[t]);
+        aq[t] = column_sum(aq[t]);
         if (lane < 16) {
             red[((wave * 2 + 0) * 16 + t) * 16 + st] = lk[t];
             red[((wave * 2 + 1) * 16 + t) * 16 + st] = aq[t];

@@ -690,9 +690,7 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
             __builtin_amdgcn_sched_barrier(0);
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-            for (int i = 0; i < RB; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+        for (int i = 0; i < RB; ++i) sum[i] = wave_sum(sum[i]);
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             mean[i] = sum[i] / (float)K;
@@ -706,9 +704,7 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
                 }
         }
 #pragma unroll
-        for (int o = 32; o > 0; o >>= 1)
-#pragma unroll
-            for (int i = 0; i < RB; ++i) sum[i] += __shfl_xor(sum[i], o, 64);
+        for (int i = 0; i < RB; ++i) sum[i] = wave_sum(sum[i]);
 #pragma unroll
         for (int i = 0; i < RB; ++i) {
             const int m = wave + (b + i) * NORMED_WAVES;

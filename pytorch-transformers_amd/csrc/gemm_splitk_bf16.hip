@@ -228,8 +228,7 @@ __global__ __launch_bounds__(64) void gemm_splitk_long_kernel(SplitkProblem p, i
     for (int m = 0; m < M; ++m) {
         float v = 0.f;
         for (long k = k0 + lane; k < k1; k += 64) v += bf16_bits_to_f32(p.x[(long)m * p.K + k]) * bf16_bits_to_f32(p.W[(long)n * p.K + k]);
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+        v = wave_sum(v);
         if (lane != 0) continue;
         const long o = (long)m * p.N + n;
         if (p.direct) store_whole(p.y, p.bias, p.add1, p.add2, p.act, p.out_f32, n, o, v);

@@ -90,8 +90,7 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(
                 }
             }
             if (MODE != LA_LOCAL) {
-                acc += __shfl_xor(acc, 16, 64);
-                acc += __shfl_xor(acc, 32, 64);
+                acc = column_sum(acc);
                 if (g4 == 0 && p < P) y[(long)(c0 + tt) * heads * P + (long)h * P + p] = acc;
             }
         }

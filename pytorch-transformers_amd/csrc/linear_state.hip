@@ -221,8 +221,7 @@ __global__ __launch_bounds__(MOST) void lin_step_kernel(T* __restrict__ out, lon
                 S[i + 3] = aa.w * S[i + 3] + kk.w * x;
                 o += S[i] * qq.x; o += S[i + 1] * qq.y; o += S[i + 2] * qq.z; o += S[i + 3] * qq.w;
             }
-            o += __shfl_xor(o, 16, 64);
-            o += __shfl_xor(o, 32, 64);
+            o = column_sum(o);
             if (g4 == 0) v_s[tt * PP + pw] = pw < P ? o : 0.f;  // (this wave alone has read that value, and its lanes run together)
         }
         __syncthreads();
@@ -377,8 +376,7 @@ __global__ __launch_bounds__(256) void lin_block_kernel(float* __restrict__ hat,
         }
 #pragma unroll
         for (int t = 0; t < 16; ++t) {
-            aq[t] += __shfl_xor(aq[t], 16, 64);
-            aq[t] += __shfl_xor(aq[t], 32, 64);
+            aq[t] = column_sum(aq[t]);
             if (lane < 16) red[(wave * 16 + t) * 16 + st] = aq[t];
         }
         __syncthreads();  // q' has been read by all: Q^ takes its place

@@ -429,8 +429,7 @@ __global__ __launch_bounds__(256) void ssm_scan_kernel(float* __restrict__ y, co
                 }
             }
             if (MODE != SSM_LOCAL) {
-                acc += __shfl_xor(acc, 16, 64);
-                acc += __shfl_xor(acc, 32, 64);
+                acc = column_sum(acc);
                 if (q == 0 && p < P) y[(long)(c0 + tt) * inner + (long)h * P + p] = acc + Dh * xv;
             }
         }
