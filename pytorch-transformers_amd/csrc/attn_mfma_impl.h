@@ -66,10 +66,6 @@ __device__ __forceinline__ float max3(float a, float b, float c) {
     return r;
 }
 
-#ifndef PTA_ATTN_DEPTH
-#define PTA_ATTN_DEPTH 2  // register buffers of a wave that walks its keys alone (measured: four gain 15 % on one
-                          // long range and lose as much on ranges of 64 to 256 keys, which are the ones chosen)
-#endif
 #define PTA_LOG2E 1.4426950408889634f
 
 template <int DT>
@@ -177,7 +173,6 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
     const int lo_last = WIN ? lowest_key(max_qpos) : 0;            // lowest key the last column sees
     const int k_begin = max(n_splits > 1 ? split * split_size : 0, lo_first & ~31);
     const int k_end = !active ? 0 : n_splits > 1 ? min(max_qpos + 1, split * split_size + split_size) : max_qpos + 1;
-    const int kb_last = (kv_len - 1) & ~31;  // the last block that has a page
     // below this key index no column of this wave masks anything (columns are ordered by token)
     const int min_lim = min(start + col0 / g + 1, k_end);
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
@@ -338,14 +333,13 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
     };
 
     if constexpr (W == 1) {
-        // all of a block at once (a block past k_end changes nothing)
+        // all of a block at once
         auto use_block = [&](KvBlock<DT>& b, int kb) {
-            if (kb + 32 > kv_len || kb >= k_end) {
+            if (kb + 32 > kv_len) {
                 // positions past the sequence's end were never written; whatever lies there must not reach the
-                // sum, not even with weight zero.  A block past this wave's range was loaded from a clamped
-                // address and is dropped whole.
+                // sum, not even with weight zero
 #pragma unroll
-                for (int dt = 0; dt < DT; ++dt) keep_below(b.v[dt].u, kb + gq * 8, kb >= k_end ? 0 : kv_len);
+                for (int dt = 0; dt < DT; ++dt) keep_below(b.v[dt].u, kb + gq * 8, kv_len);
             }
             f32x4_t sacc[2][CT];
             AFrag pf[CT];
@@ -356,15 +350,17 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
             weights(sacc, pf);
             values(b.v, pf);
         };
-        // NB register buffers: while one block is used, the loads of the next NB - 1 are in flight (a wave alone
-        // has nothing else to hide the memory's latency behind).  Addresses past the last block are clamped to
-        // it, and such a block is not used.
-        constexpr int NB = DT <= 4 ? PTA_ATTN_DEPTH : 2;
+        // Two register buffers: while one block is used, the loads of the next are in flight (a wave alone has nothing else to hide
+        // the memory's latency behind), and what is not used is not asked for: a block loaded past the wave's last costs as
+        // much as one that counts (launches over cold caches, us, the next block always loaded -> only where there is one: 13 heads on
+        // 13 of 80, 5 sequences of 40 / 210 / 320 keys 6.2 -> 5.5, 8.1 -> 6.9, 9.4 -> 8.3; 71 on 1 of 64, 8 of 100 6.0 -> 5.1; 32 on 8 of 128, 32 of
+        // 100 / 270 10.3 -> 7.8, 13.2 -> 12.2).  The loads stand in straight lines of code, not behind
+        // conditions: where ways with and without a load meet, the compiler waits for all of them.
         constexpr int STEP = 32 * KS;  // from one block of this wave to its next
-        KvBlock<DT> b[NB];
+        KvBlock<DT> b0, b1;
         const int k_first = k_begin + 32 * kw;
         const int n_mine = k_first < k_end ? (k_end - k_first + STEP - 1) / STEP : 0;  // blocks of this wave
-        auto blk = [&](int j) { return j < n_mine ? min(k_first + STEP * j, kb_last) : kb_last; };
+        auto blk = [&](int j) { return k_first + STEP * j; };
         auto page_of = [&](int kb) {
             if constexpr (!WIN) {
                 if (kb >> 6 == first_key >> 6) return (long)first_page;
@@ -372,18 +368,30 @@ __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
             }
             return (long)bt[kb >> 6];
         };
+        auto load = [&](KvBlock<DT>& to, int j) {
+            load_block<DT>(to, blk(j), page_of(blk(j)), k_pool, v_pool, nkv, kvh, c, gq);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto use = [&](KvBlock<DT>& from, int j) {
+            use_block(from, blk(j));
+            __builtin_amdgcn_sched_barrier(0);
+        };
         if (n_mine > 0) {
-#pragma unroll
-            for (int i = 0; i < NB - 1; ++i) load_block<DT>(b[i], blk(i), page_of(blk(i)), k_pool, v_pool, nkv, kvh, c, gq);
-        }
-        for (int j = 0; j < n_mine; j += NB) {
-#pragma unroll
-            for (int i = 0; i < NB; ++i) {
-                load_block<DT>(b[(i + NB - 1) % NB], blk(j + i + NB - 1), page_of(blk(j + i + NB - 1)), k_pool, v_pool, nkv, kvh, c, gq);
-                __builtin_amdgcn_sched_barrier(0);
-                if (j + i < n_mine) use_block(b[i], blk(j + i));
-                __builtin_amdgcn_sched_barrier(0);
+            load(b0, 0);
+            int j = 0;
+            for (; j + 2 < n_mine; j += 2) {
+                load(b1, j + 1);
+                use(b0, j);
+                load(b0, j + 2);
+                use(b1, j + 1);
             }
+            if (j + 1 < n_mine) {
+                load(b1, j + 1);
+                use(b0, j);
+                b0 = b1;
+                ++j;
+            }
+            use(b0, j);
         }
     } else {
         // The workgroup's waves walk the keys of its last column together, a stage of SK keys (one or two
