@@ -4,14 +4,19 @@
 //
 // A workgroup of S waves owns 16*RT rows of W and all of K.  Its waves take the 64-element K-steps
 // round robin (wave w: steps w, w + S, ...), so neighbouring waves read neighbouring 128-byte lines
-// of the same rows.  A wave works in stages of U steps and always has the next stage's loads in
-// flight while the matrix cores consume the current one (two register buffers), so every wave
-// keeps 2*U*RT KB of W on its way from HBM for as long as it runs.  W rows are the A operand of
-// v_mfma_f32_16x16x32_bf16 (lane: row = lane % 16, eight consecutive k at (lane / 16) * 8, one
+// of the same rows.  Up to sixteen rows of x (64 with a small matrix) a wave brings whole lines of its rows of W and of x straight to a
+// ring of its own in LDS, several steps ahead, and reads the operands of v_mfma_f32_16x16x32_bf16 from there (lds_stream.h: why, and what
+// it measured).  More rows of x, and rows of W too long for the buffers' offsets, go by registers: a wave works in
+// stages of U steps and always has the next stage's loads in flight while the matrix cores consume the current one (two
+// register buffers); W rows are the A operand (lane: row = lane % 16, eight consecutive k at (lane / 16) * 8, one
 // 16-byte load straight from global memory), x rows are the B operand (same shape, buffer loads whose
-// bounds are the M real rows, so the padding rows of the tile read zeros and cost no traffic).  The S partial tiles are summed through LDS in wave order, then bias,
-// activation and additions are applied and the tile is stored.  S is chosen from N and K alone, so
+// bounds are the M real rows, so the padding rows of the tile read zeros and cost no traffic).  The S partial tiles are summed through
+// LDS in wave order, then bias, activation and additions are applied and the tile is stored.  S is chosen from N and K alone, so
 // the order of summation never depends on M or on what else is in the batch.
+//
+// What is left between a launch and the rate of its loads (22,848 x 4,544, one row, 207 MB: 38.2 us from launch to launch): workgroups start
+// within 0.5 us and set up for 0.5, their rings end between 26 and 36 us after the first start (5.9 TB/s over the whole), sums and store take 0.8,
+// and the next launch starts 1.1 later.  One load of x a step instead of two, where x has eight rows or fewer, changed nothing.
 #include "common.h"
 #include "glu.h"
 #include "lds_stream.h"

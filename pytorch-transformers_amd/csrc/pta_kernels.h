@@ -193,8 +193,8 @@ int pta_gemm_normed_qkv_bf16(void* q_out, const void* x, const float* ln_w, cons
 
 // The same product for a batch of up to 128 rows that shares x through LDS and may split K over workgroups:
 // `part` is a 32-bit workspace [parts, M, N], needed when parts > 1 or reduce = 0.  rt (row tiles per wave),
-// parts, stage_blocks (64-element blocks of K per stage) and depth (stages in flight) are tuning knobs (0:
-// chosen from N and K alone); pta_gemm_splitk_parts tells the number of ranges that choice gives.
+// parts are tuning knobs (0: chosen from N and K alone); pta_gemm_splitk_parts tells the number of ranges that choice
+// gives.  stage_blocks (0, 2) and depth (0, 2, 4) are checked and change nothing.
 // With reduce = 0 the product is left as the partial sums (y may be null; bias, act and additions are not
 // applied).  Ranges that would be empty are dropped: ceil(nkb / ceil(nkb / parts)) remain, nkb = ceil(K / 64).
 int pta_gemm_splitk_bf16(void* y, float* part, const void* x, const void* W, const float* bias, const void* add1,

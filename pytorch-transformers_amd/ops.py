@@ -1219,7 +1219,8 @@ def gemm_splitk_bf16(x: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1
                      out_f32: bool = False, rt: int = 0, parts: int = 0, stage_blocks: int = 0,
                      depth: int = 0) -> torch.Tensor:
     """act(x @ w.T + bias) + add1 + add2 for a batch of at most 128 rows of bfloat16: x shared through LDS,
-    K split over workgroups where N gives too few of them."""
+    K split over workgroups where N gives too few of them.  ``stage_blocks`` (0, 2) and ``depth`` (0, 2, 4) are checked and
+    change nothing: a stage is 64 elements of K, and three stages are on their way."""
     _need(x, "x", torch.bfloat16)
     _need(w, "w", torch.bfloat16)
     M, K = x.shape
