@@ -8,8 +8,8 @@
 //   latent_values    merges a token's ranges and takes the result through the head's value expansion
 //
 // What bounds a layer here is launches and chains of dependent loads, not bytes: 16 heads, R = 512, dr = 64, 8 sequences of 64 to
-// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 27 in three (4.7,
-// 15 and 6.8).
+// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 26 in three (4.7,
+// 14 and 6.8).
 #include "attn_latent_token.h"
 
 typedef __bf16 ld_bf16x8 __attribute__((ext_vector_type(8)));
@@ -74,6 +74,7 @@ struct LatentPages {
 };
 
 #define LP_PIECES 20  // D <= 640
+#define LP_QUERIES 5  // pieces of sixteen queries a thread takes: 16 D / 8 / 256
 
 // TILES: sixteen-element tiles of the value part a wave holds (its quarter of them)
 template <int TILES>
@@ -107,15 +108,30 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
             for (int j = 0; j < LP_PIECES; ++j)
                 if (j < per) pre[j] = page[256 * j];
         };
-        fetch(k0);
-        {   // queries, scaled and rounded, once for the four waves
+        // Queries, scaled and rounded, once for the four waves: all asked for before the page, whose place the block table
+        // has yet to tell, and in LDS while it comes (a piece after the other behind the page: 15.0 us where this takes 13.9, 16 heads, R = 512, 8
+        // sequences of 64 to 700 keys)
+        float4 lo[LP_QUERIES], hi[LP_QUERIES];
+        {
             int c = row0, e = at0;
-            for (int i = tid; i < 16 * pieces; i += 256) {
-                const float* src = a.q + ((long)s * a.H + min(h0 + c, a.H - 1)) * D + 8 * e;
-                const float4 lo = *(const float4*)src, hi = *(const float4*)(src + 4);
-                const float v[8] = {lo.x * a.scale, lo.y * a.scale, lo.z * a.scale, lo.w * a.scale,
-                                    hi.x * a.scale, hi.y * a.scale, hi.z * a.scale, hi.w * a.scale};
-                *(uint4*)(Qs + c * P + 8 * e) = pack8(v);
+#pragma unroll
+            for (int j = 0; j < LP_QUERIES; ++j) {
+                const float* src = a.q + ((long)s * a.H + min(h0 + min(c, 15), a.H - 1)) * D + 8 * e;
+                lo[j] = *(const float4*)src, hi[j] = *(const float4*)(src + 4);
+                c += step_row, e += step_at;
+                if (e >= pieces) e -= pieces, ++c;
+            }
+        }
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(k0);
+        __builtin_amdgcn_sched_barrier(0);
+        {
+            int c = row0, e = at0;
+#pragma unroll
+            for (int j = 0; j < LP_QUERIES; ++j) {
+                const float v[8] = {lo[j].x * a.scale, lo[j].y * a.scale, lo[j].z * a.scale, lo[j].w * a.scale,
+                                    hi[j].x * a.scale, hi[j].y * a.scale, hi[j].z * a.scale, hi[j].w * a.scale};
+                if (tid + 256 * j < 16 * pieces) *(uint4*)(Qs + c * P + 8 * e) = pack8(v);
                 c += step_row, e += step_at;
                 if (e >= pieces) e -= pieces, ++c;
             }
