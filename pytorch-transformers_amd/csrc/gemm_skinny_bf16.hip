@@ -326,6 +326,10 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     }
 }
 
+// Heads that hold rotation pairs p0 .. p1 - 1, `half` pairs a head: what a workgroup's buffer of W has to span.  Two for up to eight
+// pairs of heads of fourteen elements and more; eight pairs of heads of two lie in eight.
+__device__ __forceinline__ int heads_of(int p0, int p1, int half) { return (p1 - 1) / half - p0 / half + 1; }
+
 // A fused query_key_value product on its own, taken to its end by its epilogue (qkv_tail.h), for matrices whose rows are spread
 // over all compute units (``launch_skinny``): a workgroup has up to eight neighbouring rotation pairs, the first elements as
 // rows 0 .. 7 of its one tile, their partners as rows 8 .. 15.  Bound by the launch, not by W: at 3,120 x 1,040 and 5 rows it
@@ -341,7 +345,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
     const int p0 = share.begin(blockIdx.x), p1 = share.end(blockIdx.x);
     const int nsteps = (K + 63) >> 6, first = p0 / half * tail.d;  // row of W that the others are counted from
     RowStream<1, D> rows;
-    rows.w[0] = buffer_of(W + (long)first * K, min((tail.nh + 2 * tail.nkv) * tail.d - first, 2 * tail.d) * K * 2);
+    rows.w[0] = buffer_of(W + (long)first * K, heads_of(p0, p1, half) * tail.d * K * 2);
     rows.x = buffer_of(x, M * K * 2);
 #pragma unroll
     for (int l = 0; l < 2; ++l) {
@@ -509,7 +513,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_ring_kernel(SkinnyProb
     } else {
         at_row = n0 + row < n1 ? row : -1;
     }
-    const i32x4_t w = buffer_of(p.W + (long)first * K, (TAIL ? min((tail.nh + 2 * tail.nkv) * tail.d - first, 2 * tail.d) : n1 - n0) * K * 2);
+    const i32x4_t w = buffer_of(p.W + (long)first * K, (TAIL ? heads_of(n0, n1, half) * tail.d : n1 - n0) * K * 2);
     const i32x4_t x = buffer_of(p.x, M * K * 2);
     const int w_at = at_row >= 0 ? at_row * K * 2 : LDS_PAST;
     int x_at[2 * MT];

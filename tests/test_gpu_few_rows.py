@@ -59,6 +59,14 @@ def test_fused_rows_to_their_end(layout, nh, nkv, d, M, rotation):
     assert bool((k2 == 7.0).all()) and bool((v2 == 7.0).all())
 
 
+# heads so short that a workgroup's rotation pairs (four up to N = 2,048, then eight) lie in three heads and more; of 12 in two
+@pytest.mark.parametrize("layout,nh,nkv,d", [("grouped", 171, 171, 2), ("tail", 1026, 1, 2), ("grouped", 171, 171, 4), ("grouped", 256, 256, 4), ("tail", 340, 1, 6),
+                                             ("grouped", 129, 129, 8), ("tail", 383, 1, 8), ("tail", 306, 1, 10), ("tail", 170, 1, 12)])
+@pytest.mark.parametrize("rotation", ["none", "half", "interleaved part"])
+def test_fused_rows_of_short_heads(layout, nh, nkv, d, rotation):
+    test_fused_rows_to_their_end(layout, nh, nkv, d, 5, rotation)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 40, 72), (8, 8192, 2048), (16, 1048, 520)])
 def test_squared_relu_in_the_epilogue(M, N, K):
     """Bias, squared ReLU and an addition in the launch itself: the bits of the product with its bias, taken to its end by hand."""
