@@ -1,14 +1,14 @@
 // C[M,N] = act(A[M,K] . W[N,K]^T + bias) + add1 + add2 in 32-bit, on the bfloat16 matrix instruction.
 // The 32-bit path of the whole model runs its projections, feed-forwards and output head through here.
 //
-// Every 32-bit value is the sum of three bfloat16 values, exactly: the nearest one, the nearest one to what is left, and the
-// rest, which has at most eight bits (split8).  Of the nine products of the parts of two values six are formed, the three left
-// out being under 2^-26 of the product of the values; each is exact in 32 bits, and so are the sums.  Six instructions of 16
-// cycles take the place of eight of 32 (v_mfma_f32_16x16x4_f32, 154 TFLOP/s).
+// A value times 2^16 is the sum of three bfloat16 values, exactly: the nearest one, the nearest one to what is left, and the rest,
+// which has at most eight bits (split8).  (Without the factor the parts of values under 2^-110 would fall below bfloat16's smallest, 2^-133.
+// With it those of the smallest value, 2^-149, do not.)  Of the nine products of the parts of two values six are formed, each exact in
+// 32 bits.  The three left out, next times rest twice and rest times rest, come to 2^-24 of the product of the values at most, 2^-27.4 in
+// the root of the mean square.  Six instructions of 16 cycles take the place of eight of 32 (v_mfma_f32_16x16x4_f32, 154 TFLOP/s).
 //
-// A value that is infinite, undefined or rounds to an infinite bfloat16 (above 3.39e38) has no such parts.  It leaves the sums
-// it takes part in undefined, and an overflow leaves them infinite: such sums are formed again on the 32-bit instruction
-// (plain_fragment), all others stay as they are.
+// A value of 2^111 and more, infinite or undefined, has no such parts and leaves the sums it takes part in undefined; sums of 2^96 and more
+// leave the range.  Those are formed on the 32-bit instruction (whole_sum); all others stay as they are.
 //
 // Order of summation.  A row's result is bitwise the same alone and in any batch, so every kernel here sums the products
 // of an output in one order, which K alone decides: K is walked in blocks of 32 elements (the last one filled up with
@@ -20,9 +20,9 @@
 // 3.1 at 1,040, 6.2 at 4,544 and 13.4 at 18,176.  Chains of the 32-bit instruction over the same segments gave 1.4, 3.7, 7.2 and
 // 14.3: an instruction here adds 32 products at a time, so a chain has fewer roundings.
 //
-// Measured against the 32-bit instruction, microseconds: 2,053 rows by 4,544 x 4,544 703 -> 432 (196 TFLOP/s), by 18,176 x 4,544
-// 2,632 -> 1,640 (207), by 4,544 x 18,176 2,787 -> 1,632 (208); 60 rows by the same 42 -> 35, 146 -> 95, 120 -> 102; one row 21.2
-// -> 19.6, 71 -> 60, 65 -> 65, by 65,024 x 4,544 239 -> 198 (6.0 TB/s).
+// Measured against the 32-bit instruction, microseconds: 2,053 rows by 4,544 x 4,544 703 -> 446 (190 TFLOP/s), by 18,176 x 4,544
+// 2,632 -> 1,650 (205), by 4,544 x 18,176 2,787 -> 1,640 (207); 60 rows by the same 42 -> 33, 146 -> 94, 120 -> 103; one row 21.2
+// -> 19.8, 71 -> 60, 65 -> 65, by 65,024 x 4,544 239 -> 198 (6.0 TB/s).  (The factor costs the tiles 4 %: 424, 1,620 and 1,570 us without.)
 //
 // Three ways to the same numbers, by what bounds them (few_rows, f32_plan):
 //   few rows: every weight is read once and that is the time.
@@ -105,25 +105,48 @@ __host__ __device__ static inline int seg_blocks(int K) { return (k_blocks(K) + 
 __host__ __device__ static inline int segments(int K) { return (k_blocks(K) + seg_blocks(K) - 1) / seg_blocks(K); }
 
 // ---- the three parts of a value -------------------------------------------------------------------------------------------
+#define SCALE 0x1p16f    // of both operands
+#define UNSCALE 0x1p-32f  // of their sums
+
 struct Parts {
     bf16x8 part[3];  // nearest, next, rest
 };
 
+typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
+union PairBits {
+    bf16_pair h;
+    uint32_t u;
+};
+// (kept from the compiler, which would give -1 below as an inline constant, and the instruction reads that as the 32-bit one)
+__device__ __forceinline__ bf16_pair pair_in_register(uint32_t bits) {
+    PairBits p;
+    p.u = bits;
+    asm("" : "+s"(p.u));
+    return p.h;
+}
+
 // A lane's eight elements of a block: k from 4 c on and k from 16 + 4 c on, c = lane / 16 (any order will do that both
-// operands have; this one reads 64 bytes of a row by four lanes).
+// operands have; this one reads 64 bytes of a row by four lanes).  DOT: what is left behind the first part is made by one instruction a
+// value, the dot product of the two parts with (-1, 0) or (0, -1) added to the value (exact, as the subtraction is, which takes two).
+// A wave of the few-row kernels has nothing to do meanwhile (18,176 elements a row, one row: 67.3 us, 64.7 so, 64.2 without
+// the factor; for both parts 65.8); beside many matrix instructions it is the slower one (2,053 rows by 4,544 x 18,176 1,640 us, 1,930 so).
+template <bool DOT>
 __device__ __forceinline__ Parts split8(f32x4 a, f32x4 b) {
-    typedef __bf16 bf16_pair __attribute__((ext_vector_type(2)));
     typedef float f32_pair __attribute__((ext_vector_type(2)));
+    const bf16_pair first = pair_in_register(0x0000bf80u), second = pair_in_register(0xbf800000u);
     union { bf16x8 v[3]; uint32_t u[3][4]; } out;
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
-        float x = i < 2 ? a[2 * i] : b[2 * i - 4], y = i < 2 ? a[2 * i + 1] : b[2 * i - 3];
+        float x = SCALE * (i < 2 ? a[2 * i] : b[2 * i - 4]), y = SCALE * (i < 2 ? a[2 * i + 1] : b[2 * i - 3]);
 #pragma unroll
         for (int p = 0; p < 3; ++p) {
-            union { bf16_pair h; uint32_t u; } c;
+            PairBits c;
             c.h = __builtin_convertvector(f32_pair{x, y}, bf16_pair);  // one instruction for the two
             out.u[p][i] = c.u;
-            if (p < 2) {  // what is left: exact
+            if (p == 0 && DOT) {
+                x = __builtin_amdgcn_fdot2_f32_bf16(c.h, first, x, false);
+                y = __builtin_amdgcn_fdot2_f32_bf16(c.h, second, y, false);
+            } else if (p < 2) {
                 x -= __uint_as_float(c.u << 16);
                 y -= __uint_as_float(c.u & 0xffff0000u);
             }
@@ -137,17 +160,18 @@ __device__ __forceinline__ Parts split8(f32x4 a, f32x4 b) {
 __device__ constexpr int term_w(int t) { return t == 0 ? 2 : t < 3 ? 1 : 0; }
 __device__ constexpr int term_x(int t) { return t == 3 ? 2 : t == 1 || t == 4 ? 1 : 0; }
 
-__device__ __forceinline__ bool any_not_finite(f32x4 v) {
-    bool bad = false;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) bad |= !(fabsf(v[e]) <= 3.402823466e38f);
-    return __any(bad);
-}
-
-// Sixteen rows of W from n on by sixteen of A from m on, on the 32-bit instruction, one chain over all of K, for what `v` holds
-// that is not finite.
+// The sums of sixteen rows of W from n on by sixteen of A from m on, from those of the parts; what of them is not finite as
+// one chain over all of K on the 32-bit instruction.
 template <int ROWS>
-__device__ __forceinline__ f32x4 plain_fragment(f32x4 v, const float* A, const float* W, int m, int n, int M, int N, int K) {
+__device__ __forceinline__ f32x4 whole_sum(f32x4 v, const float* A, const float* W, int m, int n, int M, int N, int K) {
+    bool out[4], any = false;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        out[e] = !(fabsf(v[e]) <= 3.402823466e38f);
+        any |= out[e];
+        v[e] *= UNSCALE;
+    }
+    if (!__any(any)) return v;
     const int lane = threadIdx.x & 63, r16 = lane & 15, kq = 4 * (lane >> 4);
     const float* wr = W + (long)min(n + r16, N - 1) * K;
     const float* xr = A + (long)min(m + r16, M - 1) * K;
@@ -159,7 +183,7 @@ __device__ __forceinline__ f32x4 plain_fragment(f32x4 v, const float* A, const f
     }
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        if (!(fabsf(v[e]) <= 3.402823466e38f)) v[e] = sum[e];
+        if (out[e]) v[e] = sum[e];
     return v;
 }
 
@@ -212,10 +236,10 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
             if (b + i < b1) {
                 Parts xs[CT];
 #pragma unroll
-                for (int c = 0; c < CT; ++c) xs[c] = split8(x[buf][i][c][0], x[buf][i][c][1]);
+                for (int c = 0; c < CT; ++c) xs[c] = split8<true>(x[buf][i][c][0], x[buf][i][c][1]);
 #pragma unroll
                 for (int r = 0; r < RT; ++r) {
-                    const Parts ws = split8(w[buf][i][r][0], w[buf][i][r][1]);
+                    const Parts ws = split8<true>(w[buf][i][r][0], w[buf][i][r][1]);
 #pragma unroll
                     for (int t = 0; t < TERMS; ++t)
 #pragma unroll
@@ -244,7 +268,7 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
         const int t = i >> 6, l = i & 63;  // a wave has a tile
         f32x4 v = part[0][t][l];
         for (int s = 1; s < used; ++s) v += part[s][t][l];
-        if (any_not_finite(v)) v = plain_fragment<ROWS>(v, A, W, 16 * (t % CT), n0 + 16 * (t / CT), M, N, K);
+        v = whole_sum<ROWS>(v, A, W, 16 * (t % CT), n0 + 16 * (t / CT), M, N, K);
         const int m = 16 * (t % CT) + (l & 15);
         const int n = n0 + 16 * (t / CT) + 4 * (l >> 4);
         if (m < M) {
@@ -326,10 +350,10 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_few_ring_kernel(float* __rest
             __builtin_amdgcn_sched_barrier(0);
             issue(slot);  // into the slot just read
             __builtin_amdgcn_sched_barrier(0);
-            const Parts xs = split8(v[RT][0], v[RT][1]);
+            const Parts xs = split8<true>(v[RT][0], v[RT][1]);
 #pragma unroll
             for (int r = 0; r < RT; ++r) {
-                const Parts ws = split8(v[r][0], v[r][1]);
+                const Parts ws = split8<true>(v[r][0], v[r][1]);
 #pragma unroll
                 for (int term = 0; term < TERMS; ++term)
                     acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws.part[term_w(term)], xs.part[term_x(term)], acc[r], 0, 0, 0);
@@ -347,7 +371,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_few_ring_kernel(float* __rest
         f32x4 u = mine[r * 64 + lane];
         for (int s = 1; s < used; ++s) u += mine[(s * RT + r) * 64 + lane];
         const int n_end = n0 + min(rows, (t + 1) * per_tile), n16 = n0 + t * per_tile + 16 * r;
-        if (any_not_finite(u)) u = plain_fragment<ROW_VECTORS>(u, A, W, 0, n16, M, N, K);
+        u = whole_sum<ROW_VECTORS>(u, A, W, 0, n16, M, N, K);
         const int n = n16 + 4 * g;
         if (r16 < M) {
 #pragma unroll
@@ -459,7 +483,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(F32Tiles job, F32
     };
     auto stage = [&](int i, int buf) __attribute__((always_inline)) {
         if (i == IP && !has_x) return;
-        const Parts s = split8(v[i][0], v[i][1]);
+        const Parts s = split8<false>(v[i][0], v[i][1]);
         char* at = lds + buf + (i == IP ? TP * 64 : i * 8192) + to;
 #pragma unroll
         for (int p = 0; p < 3; ++p) *(bf16x8*)(at + p * PLANE) = s.part[p];
@@ -582,7 +606,7 @@ __global__ __launch_bounds__(512, 2) void gemm_f32_tile_kernel(F32Tiles job, F32
     for (int f = 0; f < FP * FQ; ++f) {
         const int m16 = m0 + (wq * FQ + f / FP) * 16, n16 = n0 + (wp * FP + f % FP) * 16;
         f32x4 u = mine[f * 64];
-        if (any_not_finite(u)) u = plain_fragment<ROWS>(u, job.A, job.W, m16, n16, M, N, K);
+        u = whole_sum<ROWS>(u, job.A, job.W, m16, n16, M, N, K);
         const int m = m16 + r16, n = n16 + 4 * c4;
         if (m < M && n < N) store4(job.C, u, epi, m, n, N, N);
     }
@@ -607,7 +631,7 @@ __global__ __launch_bounds__(256) void gemm_f32_add_kernel(F32Tiles job, F32Epil
     for (int s = 1; s < SEGS; ++s)
         if (s < used) v += p[s];
     const int m16 = tq * 32 * FQ + ((wave >> 2) * FQ + j) * 16, n16 = tp * 64 * FP + ((wave & 3) * FP + i) * 16;
-    if (any_not_finite(v)) v = plain_fragment<ROWS>(v, job.A, job.W, m16, n16, job.M, job.N, job.K);
+    v = whole_sum<ROWS>(v, job.A, job.W, m16, n16, job.M, job.N, job.K);
     const int m = m16 + (lane & 15), n = n16 + 4 * (lane >> 4);
     if (m < job.M && n < job.N) store4(job.C, v, epi, m, n, job.N, job.N);
 }

@@ -700,8 +700,8 @@ def attn_talk(q: torch.Tensor, k_pool, v_pool, block_table, token_seq, token_pos
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, add2=None) -> torch.Tensor:
-    """act(a @ w.T + bias) + add1 + add2 of 32-bit values (taken apart into three bfloat16 each, exactly), in 32-bit sums
-    with a fixed order."""
+    """act(a @ w.T + bias) + add1 + add2 of 32-bit values, in 32-bit sums with a fixed order.  A value is taken apart into three
+    bfloat16, exactly; what of two values' product is left out is 2^-24 of it at most (2^-27.4 rms)."""
     _need(a, "a", torch.float32)
     _need(w, "w", torch.float32)
     M, K = a.shape

@@ -133,6 +133,31 @@ def test_products_of_values_without_parts(way):
     assert torch.equal(got[same][:, other], plain[same][:, other])
 
 
+def _as_way(M, N, way):
+    fp, fq, whole, share = way
+    return (fp, fq, min(whole, -(-N // (64 * fp)) * -(-M // (32 * fq))) if fp else whole, share)
+
+
+# down to the smallest 32-bit value, whose parts as bfloat16 exist only beside a factor
+@pytest.mark.parametrize("way", [(0, 0, 0, 1), (2, 1, 64, 1), (4, 4, 64, 1), (2, 2, 0, 7), (4, 3, 0, 3)])
+@pytest.mark.parametrize("side", ["a", "w"])
+def test_products_of_small_values(way, side):
+    """Rows of tiny values, of either operand, against large ones: every result relative to its own products."""
+    ops = _ops()
+    M, N, K = 60, 300, 1040
+    small, large = _rand(M if side == "a" else N, K), _rand(N if side == "a" else M, K, seed=1) * 1e30
+    powers = [-20, -30, -32, -33, -34, -35, -36, -37, -38, -40, -44]
+    small[:len(powers)] = (small[:len(powers)].double() * 10.0 ** torch.tensor(powers, device="cuda").double()[:, None]).float()
+    small[20, ::2] *= 1e-36  # beside others
+    a, w = (small, large) if side == "a" else (large, small)
+    got = _product_as(ops, a, w, *_as_way(M, N, way))
+    want = a.double() @ w.double().T
+    scale = ((a.double() ** 2) @ (w.double() ** 2).T).sqrt()
+    assert ((got.double() - want).abs() <= 8 * 2.0 ** -24 * math.sqrt(K) * scale).all()
+    few = ops.gemm_f32(a[:16].contiguous(), w)
+    assert torch.equal(few, got[:16])
+
+
 def _attention_case(nh, nkv, d, starts, news, window=0, chunk=0, sink=False, slopes=None, spoil=False):
     """(queries, pools, table, token arrays, 64-bit result); pages hold NaN where nothing was written."""
     g = torch.Generator().manual_seed(nh * 100 + d)
