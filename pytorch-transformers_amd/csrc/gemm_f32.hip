@@ -8,7 +8,8 @@
 // the root of the mean square.  Six instructions of 16 cycles take the place of eight of 32 (v_mfma_f32_16x16x4_f32, 154 TFLOP/s).
 //
 // A value of 2^111 and more, infinite or undefined, has no such parts and leaves the sums it takes part in undefined; sums of 2^96 and more
-// leave the range.  Those are formed on the 32-bit instruction (whole_sum); all others stay as they are.
+// leave the range.  Those, and all with K under SHORT_K, are formed on the 32-bit instruction (whole_sum); all others stay as they
+// are.
 //
 // Order of summation.  A row's result is bitwise the same alone and in any batch, so every kernel here sums the products
 // of an output in one order, which K alone decides: K is walked in blocks of 32 elements (the last one filled up with
@@ -160,14 +161,20 @@ __device__ __forceinline__ Parts split8(f32x4 a, f32x4 b) {
 __device__ constexpr int term_w(int t) { return t == 0 ? 2 : t < 3 ? 1 : 0; }
 __device__ constexpr int term_x(int t) { return t == 3 ? 2 : t == 1 || t == 4 ? 1 : 0; }
 
-// The sums of sixteen rows of W from n on by sixteen of A from m on, from those of the parts; what of them is not finite as
-// one chain over all of K on the 32-bit instruction.
+// Products so short take the 32-bit instruction: what the six products of parts leave out is more than its roundings.  The error against 64
+// bits in 2^-24 (rms), 32-bit instruction and parts, of normal values relative to the root of the sum of squared products / of values
+// over ten orders of magnitude relative to the sum of absolute products: K = 1 0.42 / 0.42 and 0.58 / 0.58, 2 0.53 / 0.49 and 0.56 / 0.57, 4
+// 0.67 / 0.60 and 0.53 / 0.61, 5 0.74 / 0.64 and 0.57 / 0.64, 6 0.79 / 0.69 and 0.57 / 0.64, 8 0.91 / 0.76 and 0.56 / 0.65.
+#define SHORT_K 6
+
+// The sums of sixteen rows of W from n on by sixteen of A from m on, from those of the parts; what of them is not finite, and all
+// of a short K, as one chain over all of K on the 32-bit instruction.
 template <int ROWS>
 __device__ __forceinline__ f32x4 whole_sum(f32x4 v, const float* A, const float* W, int m, int n, int M, int N, int K) {
     bool out[4], any = false;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        out[e] = !(fabsf(v[e]) <= 3.402823466e38f);
+        out[e] = K < SHORT_K || !(fabsf(v[e]) <= 3.402823466e38f);
         any |= out[e];
         v[e] *= UNSCALE;
     }

@@ -158,6 +158,22 @@ def test_products_of_small_values(way, side):
     assert torch.equal(few, got[:16])
 
 
+@pytest.mark.parametrize("K", [1, 2, 3, 4, 5, 6, 8, 16])
+@pytest.mark.parametrize("M", [1, 16, 60, 200])
+def test_short_products(M, K):
+    """Rows of a few elements: one product is that of 32-bit arithmetic, and several are off by no more than its chain of
+    roundings, each under 2^-23 of what has been summed."""
+    ops = _ops()
+    a, w = _rand(M, K), _rand(300, K, seed=1)
+    got = ops.gemm_f32(a, w)
+    if K == 1:
+        assert torch.equal(got, a * w[:, 0])
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    assert ((got.double() - want).abs() <= K * 2.0 ** -23 * size).all()
+    for way in ((0, 0, 0, 1), (2, 1, 64, 1), (4, 4, 0, 1)):
+        assert torch.equal(_product_as(ops, a, w, *_as_way(M, 300, way)), got)
+
+
 def _attention_case(nh, nkv, d, starts, news, window=0, chunk=0, sink=False, slopes=None, spoil=False):
     """(queries, pools, table, token arrays, 64-bit result); pages hold NaN where nothing was written."""
     g = torch.Generator().manual_seed(nh * 100 + d)
