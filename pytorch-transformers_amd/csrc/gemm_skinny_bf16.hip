@@ -95,6 +95,29 @@ __device__ __forceinline__ void compute_stage(const Stage<MT, RT, U>& st, f32x4_
             }
 }
 
+// A wave's steps of K, two stages of registers in turn: rows of W from the lane's addresses, so rows of any length
+template <int MT, int RT, int U>
+__device__ __forceinline__ void by_registers(f32x4_t (&acc)[RT][MT], const bf16_t* const (&wrow)[RT], const bf16_t* x, int lane, int wave,
+                                             int S, int M, int K, int nsteps, int rot) {
+    // x through a buffer descriptor whose bounds are the M real rows (0x00020000: 32-bit raw data format)
+    const __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
+    const int r = lane & 15, g = lane >> 4;
+    Stage<MT, RT, U> s0, s1;
+    load_stage<MT, RT, U>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
+    // the scheduling barriers keep the compiler from sinking a stage's loads down to their first
+    // use, which would shrink what is in flight to a load or two
+    for (int step = wave; step < nsteps; step += 2 * U * S) {
+        load_stage<MT, RT, U>(s1, wrow, xres, r, step + U * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<MT, RT, U>(s0, acc);
+        __builtin_amdgcn_sched_barrier(0);
+        load_stage<MT, RT, U>(s0, wrow, xres, r, step + 2 * U * S, S, g, K, nsteps, rot);
+        __builtin_amdgcn_sched_barrier(0);
+        compute_stage<MT, RT, U>(s1, acc);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+}
+
 // How `items` (rows of W, pairs of them) are shared out evenly to `groups` workgroups: the first `over` have one more than the others.
 // Made on the host: the division by a number of workgroups was 300 instructions at the start of a launch of few microseconds.
 struct Share {
@@ -154,7 +177,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];
     constexpr int WAVE = D == 0 ? RT * MT * 64 : RowStream<RT, D == 0 ? 1 : D>::RING / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
-    const int r = lane & 15, g = lane >> 4;
+    const int r = lane & 15;
     const bool second = (int)blockIdx.x >= pa.blocks;
     OutT* __restrict__ y = (OutT*)(second ? pb.y : pa.y);
     const bf16_t* __restrict__ x = second ? pb.x : pa.x;
@@ -213,22 +236,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
         const bf16_t* wrow[RT];
 #pragma unroll
         for (int t = 0; t < RT; ++t) wrow[t] = W + (long)(tailed ? seg * tail.d + tail_row(r, t) : min(n0 + t * 16 + r, n1 - 1)) * K;
-        // x through a buffer descriptor whose bounds are the M real rows (0x00020000: 32-bit raw data format)
-        __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, M * K * 2, 0x00020000);
-        Stage<MT, RT, U> s0, s1;
-        load_stage<MT, RT, U>(s0, wrow, xres, r, wave, S, g, K, nsteps, rot);
-        // the scheduling barriers keep the compiler from sinking a stage's loads down to their first
-        // use, which would shrink what is in flight to a load or two
-        for (int step = wave; step < nsteps; step += 2 * U * S) {
-            load_stage<MT, RT, U>(s1, wrow, xres, r, step + U * S, S, g, K, nsteps, rot);
-            __builtin_amdgcn_sched_barrier(0);
-            compute_stage<MT, RT, U>(s0, acc);
-            __builtin_amdgcn_sched_barrier(0);
-            load_stage<MT, RT, U>(s0, wrow, xres, r, step + 2 * U * S, S, g, K, nsteps, rot);
-            __builtin_amdgcn_sched_barrier(0);
-            compute_stage<MT, RT, U>(s1, acc);
-            __builtin_amdgcn_sched_barrier(0);
-        }
+        by_registers<MT, RT, U>(acc, wrow, x, lane, wave, S, M, K, nsteps, rot);
     }
 #pragma unroll
     for (int rt = 0; rt < RT; ++rt)
@@ -340,25 +348,38 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
                                                                const float* __restrict__ bias, int M, int K, int rot_stride,
                                                                Share share, QkvTail tail) {
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums
-    constexpr int WAVE = RowStream<1, D>::RING / 16;
+    constexpr int WAVE = D == 0 ? 64 : RowStream<1, D == 0 ? 1 : D>::RING / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6, half = tail.d >> 1;
     const int p0 = share.begin(blockIdx.x), p1 = share.end(blockIdx.x);
-    const int nsteps = (K + 63) >> 6, first = p0 / half * tail.d;  // row of W that the others are counted from
-    RowStream<1, D> rows;
-    rows.w[0] = buffer_of(W + (long)first * K, heads_of(p0, p1, half) * tail.d * K * 2);
-    rows.x = buffer_of(x, M * K * 2);
-#pragma unroll
-    for (int l = 0; l < 2; ++l) {
-        const int pair = p0 + (lane >> 3);
+    const int nsteps = (K + 63) >> 6, rot = start_step(rot_stride, nsteps);
+    auto row_of = [&](int pair, int second) {  // of W: an element of a pair
         int e[2];
         bool rotated;
         qkv_tail_pair_elements(tail.rot, tail.d, pair % half, e[0], e[1], rotated);
-        rows.w_at[l] = pair < p1 ? (pair / half * tail.d + e[l] - first) * K * 2 : LDS_PAST;
-        rows.x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 2 : LDS_PAST;
+        return pair / half * tail.d + (second ? e[1] : e[0]);
+    };
+    f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    if constexpr (D > 0) {
+        const int first = p0 / half * tail.d;  // row of W that the others are counted from
+        RowStream<1, D> rows;
+        rows.w[0] = buffer_of(W + (long)first * K, heads_of(p0, p1, half) * tail.d * K * 2);
+        rows.x = buffer_of(x, M * K * 2);
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+            const int pair = p0 + (lane >> 3);
+            rows.w_at[l] = pair < p1 ? (row_of(pair, l) - first) * K * 2 : LDS_PAST;
+            rows.x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 2 : LDS_PAST;
+        }
+        f32x4_t acc[1] = {sum};
+        rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, rot);
+        sum = acc[0];
+    } else {  // (places past the end read a pair again)
+        const bf16_t* wrow[1] = {W + (long)row_of(min(p0 + (lane & 7), p1 - 1), lane >> 3 & 1) * K};
+        f32x4_t acc[1][1] = {{sum}};
+        by_registers<1, 1, 2>(acc, wrow, x, lane, wave, S, M, K, nsteps, rot);
+        sum = acc[0][0];
     }
-    f32x4_t acc[1] = {f32x4_t{0.f, 0.f, 0.f, 0.f}};
-    rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, start_step(rot_stride, nsteps));
-    part[wave * WAVE + lane] = acc[0];
+    part[wave * WAVE + lane] = sum;
     __syncthreads();
     const float* sums = (const float*)part;  // row i of the tile, column m: lane (i / 4) * 16 + m, element i % 4
     for (int item = threadIdx.x; item < 128; item += blockDim.x) {
@@ -589,22 +610,30 @@ __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict
                                                               const bf16_t* __restrict__ W, int M, int F, int K, int rot_stride, int kind,
                                                               float alpha, float limit, Share share) {
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums, [2][64] each
-    constexpr int WAVE = RowStream<2, D>::RING / 16;
+    constexpr int WAVE = D == 0 ? 128 : RowStream<2, D == 0 ? 1 : D>::RING / 16;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
     const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);
-    const int nsteps = (K + 63) >> 6;
-    RowStream<2, D> rows;
-    rows.w[0] = buffer_of(W + (long)n0 * K, (n1 - n0) * K * 2);
-    rows.w[1] = buffer_of(W + (long)(F + n0) * K, (n1 - n0) * K * 2);
-    rows.x = buffer_of(x, M * K * 2);
-#pragma unroll
-    for (int l = 0; l < 2; ++l) {
-        const int i = stream_row(lane, l);
-        rows.w_at[l] = rows.w_at[2 + l] = i < n1 - n0 ? i * K * 2 : LDS_PAST;
-        rows.x_at[l] = i < M ? i * K * 2 : LDS_PAST;
-    }
+    const int nsteps = (K + 63) >> 6, rot = start_step(rot_stride, nsteps);
     f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
-    rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, start_step(rot_stride, nsteps));
+    if constexpr (D > 0) {
+        RowStream<2, D> rows;
+        rows.w[0] = buffer_of(W + (long)n0 * K, (n1 - n0) * K * 2);
+        rows.w[1] = buffer_of(W + (long)(F + n0) * K, (n1 - n0) * K * 2);
+        rows.x = buffer_of(x, M * K * 2);
+#pragma unroll
+        for (int l = 0; l < 2; ++l) {
+            const int i = stream_row(lane, l);
+            rows.w_at[l] = rows.w_at[2 + l] = i < n1 - n0 ? i * K * 2 : LDS_PAST;
+            rows.x_at[l] = i < M ? i * K * 2 : LDS_PAST;
+        }
+        rows.run(acc, (const char*)(part + wave * WAVE), lane, wave, S, K, nsteps, rot);
+    } else {
+        const int row = min(n0 + (lane & 15), n1 - 1);
+        const bf16_t* wrow[2] = {W + (long)row * K, W + (long)(F + row) * K};
+        f32x4_t sums[2][1] = {{acc[0]}, {acc[1]}};
+        by_registers<1, 2, 2>(sums, wrow, x, lane, wave, S, M, K, nsteps, rot);
+        acc[0] = sums[0][0], acc[1] = sums[1][0];
+    }
 #pragma unroll
     for (int rt = 0; rt < 2; ++rt) part[wave * WAVE + rt * 64 + lane] = acc[rt];
     __syncthreads();
@@ -1034,15 +1063,16 @@ extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* 
                           v_pool, nh, nkv, d, layout, write_cache, M, K, p, tail)) return 1;
     const int N = p.N;
     PTA_REQUIRE(pta_gemm_skinny_spread(N), "gemm_skinny_qkv_bf16: %d rows of W are too many for this launch", N);
-    PTA_REQUIRE(K <= STREAM_MOST_K, "gemm_skinny_qkv_bf16: rows of %d elements are too long for this launch", K);
     if (by_halves(N)) return launch_halves<bf16_t, true>(p, M, K, 0, (hipStream_t)stream, tail);
     const int pairs = N / 2;
     const int blocks = std::max((pairs + 7) / 8, std::min(pta_compute_units(), (pairs + 1) / 2));
     const int S = pick_split(N, K);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
-    if (launch_rings(gemm_skinny_tail_kernel<4>, dim3(blocks), dim3(S * 64), (size_t)S * RowStream<1, 4>::RING, (hipStream_t)stream, p.x,
-                     p.W, bias, M, K, rot_stride, Share(pairs, blocks), tail)) return 1;
+    auto go = [&](auto kernel, size_t ring) {
+        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, p.x, p.W, bias, M, K, rot_stride, Share(pairs, blocks), tail);
+    };
+    if (K > STREAM_MOST_K ? go(gemm_skinny_tail_kernel<0>, 1024) : go(gemm_skinny_tail_kernel<4>, RowStream<1, 4>::RING)) return 1;
     return pta_check_launch("gemm_skinny_qkv_bf16");
 }
 
@@ -1110,7 +1140,6 @@ extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, i
     if (check_skinny("gemm_skinny_glu_bf16", y, x, W, M, F, K, PTA_ACT_NONE)) return 1;
     PTA_REQUIRE(M <= 16, "gemm_skinny_glu_bf16: at most 16 rows, got %d", M);
     PTA_REQUIRE(F < (1 << 30), "gemm_skinny_glu_bf16: %d features are too many", F);
-    PTA_REQUIRE(K <= STREAM_MOST_K, "gemm_skinny_glu_bf16: rows of %d elements are too long for this launch", K);
     PTA_REQUIRE(kind == PTA_GLU_SILU || kind == PTA_GLU_CLAMPED || kind == PTA_GLU_GELU_TANH, "gemm_skinny_glu_bf16: kind %d is not built", kind);
     const int S = 2 * F >= 16384 ? pick_split(2 * F, K) : 2 * F >= 4096 ? 2 : 2 * F >= 1024 ? 4 : 8, units = pta_compute_units();
     int blocks = (F + 15) / 16;
@@ -1121,7 +1150,8 @@ extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, i
         return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)W, M, F, K,
                             rot_stride, kind, alpha, limit, Share(F, blocks));
     };
-    if (S <= 4 ? go(gemm_skinny_glu_kernel<4>, RowStream<2, 4>::RING) : go(gemm_skinny_glu_kernel<3>, RowStream<2, 3>::RING)) return 1;
+    if (K > STREAM_MOST_K ? go(gemm_skinny_glu_kernel<0>, 2048)
+                          : S <= 4 ? go(gemm_skinny_glu_kernel<4>, RowStream<2, 4>::RING) : go(gemm_skinny_glu_kernel<3>, RowStream<2, 3>::RING)) return 1;
     return pta_check_launch("gemm_skinny_glu_bf16");
 }
 

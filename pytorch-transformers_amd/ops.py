@@ -1365,7 +1365,7 @@ def gemm_splitk_pair_qkv(x1: torch.Tensor, w_qkv: torch.Tensor, bias_qkv, inv_fr
 def gemm_skinny_qkv_ok(x: torch.Tensor, w_qkv: torch.Tensor, d: int) -> bool:
     """Whether the product of few rows takes a fused query_key_value projection on its own to its end: matrices whose rows
     are spread over all compute units (larger ones keep their tiles, and the launch behind them)."""
-    return (QKV_TAIL and gemm_skinny_ok(x, w_qkv) and d % 2 == 0 and d <= 256 and w_qkv.shape[1] <= STREAM_MOST_K
+    return (QKV_TAIL and gemm_skinny_ok(x, w_qkv) and d % 2 == 0 and d <= 256
             and bool(load_library().pta_gemm_skinny_spread(int(w_qkv.shape[0]))))
 
 
@@ -1556,9 +1556,6 @@ def layernorm_sum(terms, H: int, *, w=None, b=None, eps: float = 0.0, w2=None, b
 def _bf16_rows_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     return (x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.shape[1] % 8 == 0
             and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
-
-
-STREAM_MOST_K = 1 << 20  # elements of a row of W that the launches through LDS address (lds_stream.h)
 
 
 def gemm_skinny_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
@@ -2208,7 +2205,7 @@ def glu(gate: torch.Tensor, up: torch.Tensor, kind: str = "silu", alpha: float =
 
 def gemm_skinny_glu_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the product of few rows forms the gate of a feed-forward itself: ``w`` the gate's rows, then as many of the other."""
-    return gemm_skinny_ok(x, w) and w.shape[0] % 2 == 0 and w.shape[0] > 0 and w.shape[1] <= STREAM_MOST_K
+    return gemm_skinny_ok(x, w) and w.shape[0] % 2 == 0 and w.shape[0] > 0
 
 
 def gemm_skinny_glu_pays(x: torch.Tensor, w: torch.Tensor) -> bool:

@@ -67,6 +67,50 @@ def test_fused_rows_of_short_heads(layout, nh, nkv, d, rotation):
     test_fused_rows_to_their_end(layout, nh, nkv, d, 5, rotation)
 
 
+LONG = (1 << 20) + 8  # elements of a row beyond what the launches through LDS address
+
+
+# heads of one tile a workgroup, whose halves are eight rows, and of sixteen
+@pytest.mark.parametrize("layout,nh,nkv,d", [("tail", 4, 1, 6), ("tail", 30, 1, 66)])
+def test_fused_rows_of_very_long_rows(layout, nh, nkv, d):
+    """The fused product taken to its end where rows of W go by registers: queries and cache pages within the product's rounding."""
+    from pytorch_transformers_amd import ops
+
+    if not ops.QKV_TAIL:
+        pytest.skip("switched off by PTA_QKV_TAIL=0")
+    M, N = 3, (nh + 2 * nkv) * d
+    g = torch.Generator(device="cuda").manual_seed(d)
+    x, w = torch.randn(M, LONG, generator=g, device="cuda").bfloat16(), torch.randn(N, LONG, generator=g, device="cuda").bfloat16()
+    pos, seq, table = (torch.tensor(v, dtype=torch.int32, device="cuda") for v in ([5, 70, 130], [0, 1, 2], [[0, 1, 2], [3, 4, 5], [6, 7, 8]]))
+    assert ops.gemm_skinny_qkv_ok(x, w, d)
+    new = lambda: (torch.full((9, nkv, 64, d), 7.0).bfloat16().cuda(), torch.full((9, nkv, d, 64), 7.0).bfloat16().cuda())
+    k0, v0 = new()
+    q0 = ops.qkv_rope_cache(ops.gemm_skinny_bf16(x, w), None, None, 1.0, pos, seq, table, k0, v0, nh, nkv, d, layout)
+    k1, v1 = new()
+    q1 = ops.gemm_skinny_qkv(x, w, None, None, 1.0, pos, seq, table, k1, v1, nh, nkv, d, layout, True)
+    for got, want in ((q1, q0), (k1, k0), (v1, v0)):  # sums in another order: a neighbour where they are rounded, the sums' roundings beside
+        got, want = got.float(), want.float()
+        assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + 8 * 2.0 ** -24 * LONG).all()
+    assert bool((k1 == 7.0).eq(k0 == 7.0).all()) and bool((v1 == 7.0).eq(v0 == 7.0).all())
+
+
+def test_the_gate_of_very_long_rows():
+    """As test_the_gate_in_the_epilogue, by registers."""
+    from pytorch_transformers_amd import ops
+
+    M, F = 2, 24
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w = torch.randn(M, LONG, generator=g, device="cuda").bfloat16(), (0.002 * torch.randn(2 * F, LONG, generator=g, device="cuda")).bfloat16()
+    assert ops.gemm_skinny_glu_ok(x, w)
+    got = ops.gemm_skinny_glu(x, w, "silu", 1.7, 3.0).float()
+    both = ops.gemm_skinny_bf16(x, w).float()
+    gate, up = both[:, :F], both[:, F:]
+    want = torch.nn.functional.silu(gate) * up
+    # a neighbour of either half, and the sums' roundings at values of some 0.002 sqrt(K) = 2
+    tol = 2.0 ** -7 * (1.3 * gate.abs() * (up.abs() + 1) + gate.abs() * up.abs() + want.abs()) + 1e-3
+    assert bool(((got - want).abs() <= tol).all())
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 40, 72), (8, 8192, 2048), (16, 1048, 520)])
 def test_squared_relu_in_the_epilogue(M, N, K):
     """Bias, squared ReLU and an addition in the launch itself: the bits of the product with its bias, taken to its end by hand."""
