@@ -220,19 +220,32 @@ __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem p
         }
 }
 
-// The same sums for rows too long for 32-bit offsets within a workgroup's rows (STREAM_MOST_K): a wave takes a row of W by a range of
-// K, one row of x after the other.  So that such products run; nothing was done for their speed.
+// The same sums for rows too long for 32-bit offsets within a wave's rows of W (32 rows of 2^25 elements, 16 of 2^26), at most 31 of x: a
+// wave takes a row of W by a range of K, four rows of x at a time.
 __global__ __launch_bounds__(64) void gemm_splitk_long_kernel(SplitkProblem p, int M) {
     const int lane = threadIdx.x, n = blockIdx.x, range = blockIdx.y;
     const long k0 = (long)range * p.blocks_per_part * 64, k1 = min((long)p.K, k0 + (long)p.blocks_per_part * 64);
-    for (int m = 0; m < M; ++m) {
-        float v = 0.f;
-        for (long k = k0 + lane; k < k1; k += 64) v += bf16_bits_to_f32(p.x[(long)m * p.K + k]) * bf16_bits_to_f32(p.W[(long)n * p.K + k]);
-        v = wave_sum(v);
-        if (lane != 0) continue;
-        const long o = (long)m * p.N + n;
-        if (p.direct) store_whole(p.y, p.bias, p.add1, p.add2, p.act, p.out_f32, n, o, v);
-        else p.part[(long)range * M * p.N + o] = v;
+    for (int m0 = 0; m0 < M; m0 += 4) {
+        float v[4] = {0.f, 0.f, 0.f, 0.f};
+        for (long k = k0 + lane * 8; k < k1; k += 512) {  // K is a multiple of 8
+            float w[8];
+            unpack8(*reinterpret_cast<const uint4*>(p.W + (long)n * p.K + k), w);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float x[8];
+                unpack8(*reinterpret_cast<const uint4*>(p.x + (long)min(m0 + i, M - 1) * p.K + k), x);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[i] += x[e] * w[e];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            v[i] = wave_sum(v[i]);
+            if (lane != 0 || m0 + i >= M) continue;
+            const long o = (long)(m0 + i) * p.N + n;
+            if (p.direct) store_whole(p.y, p.bias, p.add1, p.add2, p.act, p.out_f32, n, o, v[i]);
+            else p.part[(long)range * M * p.N + o] = v[i];
+        }
     }
 }
 
@@ -409,7 +422,8 @@ static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int
     auto kern = rotate ? gemm_splitk_kernel<MT, RT, D, true> : gemm_splitk_kernel<MT, RT, D, false>;
     if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return pta_fail("gemm_splitk_bf16: cannot have %d bytes of LDS", lds);
-    if (a.K > STREAM_MOST_K || b.K > STREAM_MOST_K) {
+    // (x lies within 32-bit offsets: check_splitk)
+    if ((long)std::max(a.K, b.K) * 16 * RT * 2 >= LDS_PAST) {
         for (const SplitkProblem* p : {&a, &b})
             if (p->N > 0) hipLaunchKernelGGL(gemm_splitk_long_kernel, dim3(p->N, p->parts), dim3(64), 0, s, *p, M);
         return reduce_parts(a, M, reduce, s);

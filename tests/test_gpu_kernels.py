@@ -149,6 +149,21 @@ def test_few_row_products_of_very_long_rows(M):
     assert float((part.double().sum(0) - prod).abs().max()) <= tol
 
 
+# the longest rows that lie within 32-bit offsets, 32 rows of W a wave, and ones past them
+@pytest.mark.parametrize("K", [(1 << 25) - 8, (1 << 25) + 8])
+def test_gemm_splitk_of_the_longest_rows(K):
+    ops = _ops()
+    M, N = 19, 33
+    g = torch.Generator(device="cuda").manual_seed(0)
+    x, w = (torch.randn(n, K, generator=g, device="cuda", dtype=torch.bfloat16) for n in (M, N))
+    want = torch.zeros(M, N, dtype=torch.float64, device="cuda")
+    for k in range(0, K, 1 << 22):
+        want += x[:, k:k + (1 << 22)].double() @ w[:, k:k + (1 << 22)].double().T.contiguous()
+    tol = 8 * 2.0 ** -24 * K  # as test_few_row_products_of_very_long_rows
+    for parts in (1, 5):
+        assert float((ops.gemm_splitk_bf16(x, w, out_f32=True, rt=2, parts=parts).double() - want).abs().max()) <= tol
+
+
 @pytest.mark.parametrize("M", [1, 9, 17, 32, 33, 50, 64, 65, 81, 96, 100, 128, 129, 200, 256])
 @pytest.mark.parametrize("N,K,parts,rt,sb,depth", [(16, 64, 0, 0, 0, 0), (100, 200, 0, 0, 0, 0), (100, 200, 3, 2, 2, 2),
                                                    (4544, 4544, 0, 0, 0, 0), (250, 18176 // 4, 5, 1, 2, 4),
