@@ -79,7 +79,6 @@ class TuningTable:
         for k, v in data.get("pair_parts", {}).items():
             s1, s2 = shapes(k)
             cut = (int(v[0]), int(v[1]), int(v[2]) if len(v) > 2 else 1)
-            _unfix_pair(s1, s2)
             _fix_pair(s1, s2, cut)
             self.pair_parts[(s1, s2)] = cut
         for k, v in data.get("pair_stationary", {}).items():
@@ -114,12 +113,10 @@ def _unfix_pair(s1, s2) -> None:
 
 
 def _fix_pair(s1, s2, cut) -> None:
-    """Fix (ranges, ranges, row tiles per wave) for a pair of shapes in the kernel library, unless it is the rule's
-    own choice (nothing is fixed for the shapes when this is called)."""
+    """Fix (ranges, ranges, row tiles per wave) for a pair of shapes in the kernel library: also where they are the rule's for
+    some rows, which has others for steps of 33 to 64 rows."""
     a, b, rt = cut
-    rule = ops.gemm_splitk_pair_parts(s1[0], s1[1], s2[0], s2[1])
-    if (a, b, rt) != tuple(rule) + (1,) and ops.load_library().pta_gemm_splitk_pair_fix(
-            int(s1[0]), int(s1[1]), int(s2[0]), int(s2[1]), int(a), int(b), int(rt)):
+    if ops.load_library().pta_gemm_splitk_pair_fix(int(s1[0]), int(s1[1]), int(s2[0]), int(s2[1]), int(a), int(b), int(rt)):
         raise ops.KernelError(f"tuning table: {a} and {b} ranges of K with {rt} row tiles are not valid for the pair "
                               f"{tuple(s1)}, {tuple(s2)}")
 
@@ -748,8 +745,7 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
         if t24 <= 1.03 * small[0]:
             chosen = cands[i]
             break
-    if chosen != cands[0]:
-        fix(chosen)
+    fix(chosen)
     _active.pair_parts[key] = chosen
     # the launch with stationary activations against that choice, per class of rows
     chosen_st = []
@@ -787,8 +783,8 @@ def gemm_splitk_pair_parts_rule(N1: int, K1: int, N2: int, K2: int):
     kept = _active.pair_parts.get(((int(N1), int(K1)), (int(N2), int(K2))))
     lib.pta_gemm_splitk_pair_fix(int(N1), int(K1), int(N2), int(K2), 0, 0, 1)
     rule = ops.gemm_splitk_pair_parts(N1, K1, N2, K2)
-    if kept is not None and tuple(kept) != rule + (1,):
-        lib.pta_gemm_splitk_pair_fix(int(N1), int(K1), int(N2), int(K2), int(kept[0]), int(kept[1]), int(kept[2]))
+    if kept is not None:
+        _fix_pair((N1, K1), (N2, K2), kept)
     return rule
 
 
