@@ -623,13 +623,12 @@ static int stationary_class(int M) { return M <= 16 ? 0 : M <= 32 ? 1 : M <= 64 
 struct StationaryChoice { int q1[STATIONARY_CLASSES], q2[STATIONARY_CLASSES]; };  // 0: the staged kernel
 static std::map<std::array<int, 4>, StationaryChoice> pair_stationary_fixed;
 
-// Where one class of a shape is fixed, the others from 33 rows on (classes 2 and 3) have the rule's ranges; without a fixed choice the
-// launch is used from 65 rows on: below, the staged kernel is faster (pair_us), at 128 rows 53 us against its 57 for 4,672 + 18,176 x 4,544,
-// 163 against 167 for 9,216 + 32,768 x 8,192, 54 against 52 for 4,544 x 4,544 + 4,544 x 18,176, 158 against 168 for 8,192 x 8,192 + 32,768.
-#define STATIONARY_RULE_FROM_CLASS 2
-// (At 33 to 64 rows the staged kernel was timed for matrices of 4,096 rows together and more.)
-#define STATIONARY_UNFIXED_FROM_CLASS 3
+// Where no choice is fixed the launch is used from 65 rows on: below, the staged kernel is faster (pair_us), at 128 rows 53 us against its
+// 57 for 4,672 + 18,176 x 4,544, 163 against 167 for 9,216 + 32,768 x 8,192, 54 against 52 for 4,544 x 4,544 + 4,544 x 18,176, 158 against
+// 168 for 8,192 x 8,192 + 32,768.  (At 33 to 64 rows the staged kernel was timed for matrices of 4,096 rows together and more.)
 #define STAGED_FROM_ROWS 4096
+static bool stationary_unfixed(int N1, int N2, int cls) { return cls >= 3 || (cls == 2 && N1 + N2 < STAGED_FROM_ROWS); }
+
 static void stationary_rule(int N1, int K1, int N2, int K2, int cls, int* q1, int* q2) {
     const int kmin = min(K1, K2), f1 = max(1, (K1 + kmin / 2) / kmin), f2 = max(1, (K2 + kmin / 2) / kmin);
     const long tiles = (long)((N1 + 15) / 16) * f1 + (long)((N2 + 15) / 16) * f2;
@@ -659,7 +658,8 @@ extern "C" int pta_gemm_splitk_pair_fix_stationary(int N1, int K1, int N2, int K
     auto it = pair_stationary_fixed.find(key);
     if (it == pair_stationary_fixed.end()) {
         StationaryChoice c{};
-        for (int i = STATIONARY_RULE_FROM_CLASS; i < STATIONARY_CLASSES; ++i) stationary_rule(N1, K1, N2, K2, i, &c.q1[i], &c.q2[i]);
+        for (int i = 0; i < STATIONARY_CLASSES; ++i)  // the other classes stay as they are
+            if (stationary_unfixed(N1, N2, i)) stationary_rule(N1, K1, N2, K2, i, &c.q1[i], &c.q2[i]);
         it = pair_stationary_fixed.emplace(key, c).first;
     }
     it->second.q1[cls] = q1;
@@ -677,7 +677,7 @@ static bool pair_fixed(int N1, int K1, int N2, int K2) {
 static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, int* p2) {
     if (M >= 1 && M <= STATIONARY_MAX_ROWS && K1 % 8 == 0 && K2 % 8 == 0) {
         const int cls = stationary_class(M);
-        int q1, q2;
+        int q1 = 0, q2 = 0;
         bool fixed = false;
         {
             std::lock_guard<std::mutex> hold(pair_parts_lock);
@@ -688,21 +688,17 @@ static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, 
                 fixed = true;
             }
         }
-        if (!fixed) {
-            q1 = q2 = 0;
-            if (cls >= STATIONARY_UNFIXED_FROM_CLASS || (cls == 2 && N1 + N2 < STAGED_FROM_ROWS)) {
-                stationary_rule(N1, K1, N2, K2, cls, &q1, &q2);
-            } else if (cls == 2 && !pair_fixed(N1, K1, N2, K2)) {  // ranges and tiles of its own
-                const PairChoice c = pair_rule(N1, K1, N2, K2, 64);
-                *p1 = c.p1;
-                *p2 = c.p2;
-                return c.rt;
-            }
-        }
+        if (!fixed && stationary_unfixed(N1, N2, cls)) stationary_rule(N1, K1, N2, K2, cls, &q1, &q2);
         if (q1 > 0 && q2 > 0) {
             *p1 = q1;
             *p2 = q2;
             return 3;
+        }
+        if (cls == 2 && !stationary_unfixed(N1, N2, cls) && !pair_fixed(N1, K1, N2, K2)) {  // ranges and tiles of its own
+            const PairChoice c = pair_rule(N1, K1, N2, K2, 64);
+            *p1 = c.p1;
+            *p2 = c.p2;
+            return c.rt;
         }
     }
     const int rt = pick_pair_parts(N1, K1, N2, K2, p1, p2);

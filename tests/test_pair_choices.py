@@ -38,3 +38,22 @@ def test_recorded_ranges_hold_at_every_row_count(table, shape):
         assert _ranges(shape, 0, 8, 24, 48, 64) == [cut] * 5
     table.clear_tuning()
     assert _ranges(shape, 24, 48) == [few, middle]
+
+
+@pytest.mark.parametrize("shape", SHAPES + [(328, 2112, 200, 4608)])
+@pytest.mark.parametrize("cls", range(4))
+def test_a_class_of_rows_leaves_the_others(table, shape, cls):
+    """Where one class of rows is fixed, to the staged kernel or to ranges of the stationary one, the others have what they have without;
+    and the staged kernel runs with the rule's ranges of its rows."""
+    from pytorch_transformers_amd import ops
+
+    rows = (8, 24, 48, 100)
+    plain, fix = _ranges(shape, *rows), ops.load_library().pta_gemm_splitk_pair_fix_stationary
+    staged = [plain[i] if i < 2 or (i == 2 and shape in SHAPES) else _ranges(shape, 0)[0] for i in range(4)]
+    try:
+        for cut, want in (((0, 0), staged[cls]), ((1, 1), (1, 1))):
+            assert fix(*shape, cls, *cut) == 0
+            assert _ranges(shape, *rows) == [want if i == cls else plain[i] for i in range(4)]
+    finally:
+        fix(*shape, -1, 0, 0)
+    assert _ranges(shape, *rows) == plain
