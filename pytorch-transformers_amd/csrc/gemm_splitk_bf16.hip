@@ -502,10 +502,15 @@ extern "C" int pta_gemm_splitk_bf16(void* y, float* part, const void* x, const v
 // fastest (N = 4,096 with K = 4,096 and 16,384 at 64 rows: 2 and 7 ranges by the rule; 4 and 8 make the
 // decode step 7 % faster, 2 and 10 make it 3 % slower with as many workgroups), so the Python side times them once.
 struct PairChoice { int p1, p2, rt; };
-static std::map<std::array<int, 4>, PairChoice> pair_parts_fixed;
+struct PairFixed { PairChoice few, middle; };  // for 33 to 64 rows of wide matrices (staged_middle), and for all others; p1 = 0: the rule's
+static std::map<std::array<int, 4>, PairFixed> pair_parts_fixed;
 static std::mutex pair_parts_lock;
 
 static bool parts_valid(int K, int p) { return p >= 1 && clamp_parts(p, K) == p && effective_parts(K, p) == p; }
+
+// (At 33 to 64 rows the staged kernel was timed for matrices of 4,096 rows together and more.)
+#define STAGED_FROM_ROWS 4096
+static bool staged_middle(int N1, int N2) { return N1 + N2 >= STAGED_FROM_ROWS; }
 
 // Fixes, for every later pair launch of this shape, the ranges of K of the two products and how many tiles of
 // sixteen rows of W a wave holds in steps of more than 32 rows (rt 1 or 2: 64 or 128 rows of W a workgroup; the
@@ -521,12 +526,21 @@ extern "C" int pta_gemm_splitk_pair_fix(int N1, int K1, int N2, int K2, int p1, 
         return 0;
     }
     if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2)) return 1;
-    pair_parts_fixed[key] = {p1, p2, rt};
+    pair_parts_fixed[key] = {{p1, p2, rt}, {p1, p2, rt}};
     return 0;
 }
 
 extern "C" int pta_gemm_splitk_pair_fix_parts(int N1, int K1, int N2, int K2, int p1, int p2) {
     return pta_gemm_splitk_pair_fix(N1, K1, N2, K2, p1, p2, 1);
+}
+
+// The same for steps of 33 to 64 rows alone, of matrices for which those have ranges of their own (else 1).
+extern "C" int pta_gemm_splitk_pair_fix_middle(int N1, int K1, int N2, int K2, int p1, int p2, int rt) {
+    if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || !staged_middle(N1, N2)) return 1;
+    if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2)) return 1;
+    std::lock_guard<std::mutex> hold(pair_parts_lock);
+    pair_parts_fixed[{N1, K1, N2, K2}].middle = {p1, p2, rt};  // (a new entry's others are the rule's)
+    return 0;
 }
 
 // What a pair launch with `a` and `b` ranges takes at so many rows, in microseconds: the workgroups are handed to the compute units in
@@ -588,21 +602,19 @@ static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
     return known[key] = best;
 }
 
-// returns the row tiles per wave for steps of more than 32 rows
-static int pick_pair_parts(int N1, int K1, int N2, int K2, int* p1, int* p2) {
+// the staged kernel's ranges, and its tiles of sixteen rows of W a wave, for a step of so many rows (0: up to 32)
+static int pick_pair_parts(int N1, int K1, int N2, int K2, int M, int* p1, int* p2) {
+    const bool middle = M > 32 && M <= 64 && staged_middle(N1, N2);
+    PairChoice c{0, 0, 1};
     {
         std::lock_guard<std::mutex> hold(pair_parts_lock);
         const auto it = pair_parts_fixed.find({N1, K1, N2, K2});
-        if (it != pair_parts_fixed.end()) {
-            *p1 = it->second.p1;
-            *p2 = it->second.p2;
-            return it->second.rt;
-        }
+        if (it != pair_parts_fixed.end()) c = middle ? it->second.middle : it->second.few;
     }
-    const PairChoice c = pair_rule(N1, K1, N2, K2, 32);
+    if (c.p1 == 0) c = pair_rule(N1, K1, N2, K2, middle ? 64 : 32);
     *p1 = c.p1;
     *p2 = c.p2;
-    return 1;
+    return M > 32 ? c.rt : 1;
 }
 
 // Steps of up to 128 rows may run with the activations stationary (gemm_stationary_bf16.hip), which cuts K into
@@ -625,9 +637,8 @@ static std::map<std::array<int, 4>, StationaryChoice> pair_stationary_fixed;
 
 // Where no choice is fixed the launch is used from 65 rows on: below, the staged kernel is faster (pair_us), at 128 rows 53 us against its
 // 57 for 4,672 + 18,176 x 4,544, 163 against 167 for 9,216 + 32,768 x 8,192, 54 against 52 for 4,544 x 4,544 + 4,544 x 18,176, 158 against
-// 168 for 8,192 x 8,192 + 32,768.  (At 33 to 64 rows the staged kernel was timed for matrices of 4,096 rows together and more.)
-#define STAGED_FROM_ROWS 4096
-static bool stationary_unfixed(int N1, int N2, int cls) { return cls >= 3 || (cls == 2 && N1 + N2 < STAGED_FROM_ROWS); }
+// 168 for 8,192 x 8,192 + 32,768.
+static bool stationary_unfixed(int N1, int N2, int cls) { return cls >= 3 || (cls == 2 && !staged_middle(N1, N2)); }
 
 static void stationary_rule(int N1, int K1, int N2, int K2, int cls, int* q1, int* q2) {
     const int kmin = min(K1, K2), f1 = max(1, (K1 + kmin / 2) / kmin), f2 = max(1, (K2 + kmin / 2) / kmin);
@@ -667,11 +678,6 @@ extern "C" int pta_gemm_splitk_pair_fix_stationary(int N1, int K1, int N2, int K
     return 0;
 }
 
-static bool pair_fixed(int N1, int K1, int N2, int K2) {
-    std::lock_guard<std::mutex> hold(pair_parts_lock);
-    return pair_parts_fixed.count({N1, K1, N2, K2}) != 0;
-}
-
 // The ranges of a pair launch of M rows and its kind: 3 with stationary activations, else the tiles of sixteen
 // rows of W per wave of the staged kernel (1 or 2).  M = 0 asks for the staged kernel's ranges.
 static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, int* p2) {
@@ -694,20 +700,20 @@ static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, 
             *p2 = q2;
             return 3;
         }
-        if (cls == 2 && !stationary_unfixed(N1, N2, cls) && !pair_fixed(N1, K1, N2, K2)) {  // ranges and tiles of its own
-            const PairChoice c = pair_rule(N1, K1, N2, K2, 64);
-            *p1 = c.p1;
-            *p2 = c.p2;
-            return c.rt;
-        }
     }
-    const int rt = pick_pair_parts(N1, K1, N2, K2, p1, p2);
-    return M > 32 ? rt : 1;
+    return pick_pair_parts(N1, K1, N2, K2, M, p1, p2);
 }
 
 extern "C" int pta_gemm_splitk_pair_parts(int N1, int K1, int N2, int K2, int M, int* p1, int* p2) {
     if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || M < 0) return pta_fail("gemm_splitk_pair_parts: sizes must be positive");
     pick_pair_parts_rows(N1, K1, N2, K2, M, p1, p2);
+    return 0;
+}
+
+// The same, and how the launch runs: 1 or 2, tiles of sixteen rows of W a wave of the staged kernel; 3, with stationary activations.
+extern "C" int pta_gemm_splitk_pair_way(int N1, int K1, int N2, int K2, int M, int* p1, int* p2, int* way) {
+    if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || M < 0) return pta_fail("gemm_splitk_pair_way: sizes must be positive");
+    *way = pick_pair_parts_rows(N1, K1, N2, K2, M, p1, p2);
     return 0;
 }
 

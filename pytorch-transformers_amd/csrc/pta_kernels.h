@@ -245,6 +245,10 @@ int pta_gemm_splitk_pair_fix_parts(int N1, int K1, int N2, int K2, int p1, int p
 // the same, and how many tiles of sixteen rows of W a wave holds in steps of more than 32 rows (rt 1 or 2, i.e. 64
 // or 128 rows of W a workgroup); the ranges decide the order of summation, the tile height does not
 int pta_gemm_splitk_pair_fix(int N1, int K1, int N2, int K2, int p1, int p2, int rt);
+// the same for steps of 33 to 64 rows alone, where those have ranges of their own (matrices of 4,096 rows together and more; else 1)
+int pta_gemm_splitk_pair_fix_middle(int N1, int K1, int N2, int K2, int p1, int p2, int rt);
+// what pta_gemm_splitk_pair_parts gives, and how the launch runs: 1 or 2, the staged kernel's rt; 3, with stationary activations
+int pta_gemm_splitk_pair_way(int N1, int K1, int N2, int K2, int M, int* parts1, int* parts2, int* way);
 // The same two partial products for 1 to 128 rows with the activations stationary (gemm_stationary_bf16.hip):
 // about one workgroup per compute unit, each wave keeping the sums of its row tiles in registers while the
 // workgroup walks its range of K in phases of LDS-resident slices of x.  parts1 and parts2 ranges of K

@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_stationary_rule", "pta_gemm_tile_plan")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -1263,6 +1263,14 @@ def gemm_splitk_pair_parts(N1: int, K1: int, N2: int, K2: int, M: int = 0):
     p1, p2 = ctypes.c_int(0), ctypes.c_int(0)
     _call("pta_gemm_splitk_pair_parts", int(N1), int(K1), int(N2), int(K2), int(M), ctypes.byref(p1), ctypes.byref(p2))
     return p1.value, p2.value
+
+
+def gemm_splitk_pair_way(N1: int, K1: int, N2: int, K2: int, M: int):
+    """``gemm_splitk_pair_parts``, and how the launch runs: 1 or 2, the kernel that walks K in stages with so many tiles of
+    sixteen rows of W a wave; 3, with stationary activations."""
+    p1, p2, way = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
+    _call("pta_gemm_splitk_pair_way", int(N1), int(K1), int(N2), int(K2), int(M), ctypes.byref(p1), ctypes.byref(p2), ctypes.byref(way))
+    return p1.value, p2.value, way.value
 
 
 STATIONARY_CLASS_ROWS = (16, 32, 64, 128)  # a pair launch's rows count by the first of these that holds them

@@ -34,7 +34,9 @@ class TuningTable:
     FIELDS = ("pair_parts", "pair_stationary", "splitk_rows", "mm_plans", "mm_joined", "mm_ksplit", "mm_tiles", "decode_plans")
 
     def __init__(self, data: Optional[dict] = None):
-        self.pair_parts: dict = {}  # (shape of w1, shape of w2) -> (ranges, ranges, row tiles per wave) in use
+        # (shape of w1, shape of w2) -> (ranges, ranges, row tiles per wave) in use, and another three where steps of 33 to 64
+        # rows have theirs
+        self.pair_parts: dict = {}
         # (shape of w1, shape of w2) -> per class of rows the (ranges, ranges) of the launch with stationary
         # activations, (0, 0) where the staged kernel stays
         self.pair_stationary: dict = {}
@@ -57,7 +59,7 @@ class TuningTable:
         hence the same bits."""
         key = lambda t: ",".join("x".join(str(int(v)) for v in (p if isinstance(p, tuple) else (p,))) for p in t)
         return {
-            "pair_parts": {key(k): list(v) for k, v in self.pair_parts.items()},  # ranges, ranges, row tiles per wave
+            "pair_parts": {key(k): list(v) for k, v in self.pair_parts.items()},  # ranges, ranges, row tiles per wave (and again)
             "pair_stationary": {key(k): [list(c) for c in v] for k, v in self.pair_stationary.items()},  # per class of rows
             "splitk_rows": {key(k): int(v) for k, v in self.splitk_rows.items()},
             "mm_plans": {key(k): list(v) for k, v in self.mm_plans.items()},
@@ -78,7 +80,7 @@ class TuningTable:
         flat = lambda k: tuple(int(p) for p in k.split(","))
         for k, v in data.get("pair_parts", {}).items():
             s1, s2 = shapes(k)
-            cut = (int(v[0]), int(v[1]), int(v[2]) if len(v) > 2 else 1)
+            cut = tuple(int(n) for n in v) if len(v) != 2 else (int(v[0]), int(v[1]), 1)
             _fix_pair(s1, s2, cut)
             self.pair_parts[(s1, s2)] = cut
         for k, v in data.get("pair_stationary", {}).items():
@@ -113,12 +115,14 @@ def _unfix_pair(s1, s2) -> None:
 
 
 def _fix_pair(s1, s2, cut) -> None:
-    """Fix (ranges, ranges, row tiles per wave) for a pair of shapes in the kernel library: also where they are the rule's for
-    some rows, which has others for steps of 33 to 64 rows."""
-    a, b, rt = cut
-    if ops.load_library().pta_gemm_splitk_pair_fix(int(s1[0]), int(s1[1]), int(s2[0]), int(s2[1]), int(a), int(b), int(rt)):
-        raise ops.KernelError(f"tuning table: {a} and {b} ranges of K with {rt} row tiles are not valid for the pair "
-                              f"{tuple(s1)}, {tuple(s2)}")
+    """Fix (ranges, ranges, row tiles per wave) for a pair of shapes in the kernel library, and the second three for steps of 33
+    to 64 rows: also where they are the rule's for some rows, which has others for those."""
+    lib, shapes = ops.load_library(), (int(s1[0]), int(s1[1]), int(s2[0]), int(s2[1]))
+    refused = len(cut) not in (3, 6) or lib.pta_gemm_splitk_pair_fix(*shapes, *(int(n) for n in cut[:3]))
+    if not refused and len(cut) == 6:
+        refused = lib.pta_gemm_splitk_pair_fix_middle(*shapes, *(int(n) for n in cut[3:]))
+    if refused:
+        raise ops.KernelError(f"tuning table: ranges of K and row tiles {tuple(cut)} are not valid for the pair {tuple(s1)}, {tuple(s2)}")
 
 
 def _fix_stationary(s1, s2, cuts) -> None:
@@ -649,49 +653,65 @@ def joined_mm_pays(x: torch.Tensor, joined: torch.Tensor, n_first: int, bias1=No
     return _active.mm_joined[key]
 
 
-# Ranges of K for the pairs of a shape: the kernel library's rule gives a choice; when timing is on, its neighbours
-# are timed once per shape, at 64 rows, with cold caches, and one that is at least 3 % faster is kept for every
-# later launch (PTA_PAIR_TUNE=0 switches this off).
+# Ranges of K for the pairs of a shape: the kernel library's rule gives a choice per class of rows; when timing is on,
+# its neighbours are timed once per shape, with cold caches, at rows of the class, and one that is at least 3 % faster is kept for
+# every later launch of the class (PTA_PAIR_TUNE=0 switches this off).
 PAIR_TUNE = os.environ.get("PTA_PAIR_TUNE", "1") != "0"
 PAIR_TUNE_MARGIN = 0.97
-PAIR_TUNE_ROWS = int(os.environ.get("PTA_PAIR_TUNE_ROWS", "64"))  # rows of the timed launches (17 to 128)
+PAIR_TUNE_ROWS = int(os.environ.get("PTA_PAIR_TUNE_ROWS", "64"))  # the larger of the two counts timed for 33 to 64 rows
+
+
+def pick_way(times, margin: float) -> int:
+    """The way to take, by times[count of rows][way]: the first, which is the rule's, unless another is no slower at any count
+    and faster by the margin over them together; then the fastest of those."""
+    total = [sum(t[i] for t in times) for i in range(len(times[0]))]
+    ok = [i for i in range(1, len(total)) if total[i] < margin * total[0] and all(t[i] <= t[0] for t in times)]
+    return min(ok, key=lambda i: total[i]) if ok else 0
 
 
 def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
-    """Once per pair of shapes, while timing is on: time the pair launch with the rule's ranges of K, with their
-    neighbours, and with workgroups of 128 rows of W (which load the activations half as often, have half as many
-    workgroups and so want more ranges), at 64 rows with cold caches; keep the fastest in the kernel library if it
-    beats the rule's by the margin and is no slower than the rule's at 24 rows (where the tile height does not
-    apply, but the ranges do).  ``_pair_parts_tuned`` says what is in use: (ranges, ranges, row tiles per wave).
-    Then, at 8, 32, 64 and 128 rows (one count per class of rows), the launch with stationary activations is timed
-    against the winner with one to six ranges of the shorter K (and as many times more of the longer), each
-    with what reads its partial sums behind it (the norm that adds them, where the two products have one width; else
-    a charge for the ranges' bytes): the fastest is fixed for the class, or the staged kernel where that is not
-    beaten by 2 % (``_pair_stationary_tuned``)."""
+    """Once per pair of shapes, while timing is on: the pair launch with the ranges of K that the rule has for the rows, and with
+    neighbours of them, with cold caches; ``pick_way`` says which is kept.  Up to 32 rows are timed at 8 and 32; 33 to 64 rows,
+    where they have ranges of their own, at 40 and 64, and with workgroups of 128 rows of W (which load the activations half as
+    often, have half as many workgroups and so want more ranges); those are timed at 128 rows too, with the ranges of few rows.  Then, at 8, 32, 64 and 128 rows (one count per class of
+    rows), the launch with stationary activations is timed against the winner with one to six ranges of the shorter K
+    (and as many times more of the longer): whichever of the two the rule takes for the class stays unless it is beaten by 2 %.
+    All with what reads the partial sums behind the launch (the norm that adds them, where the two products have one width;
+    else a charge for the ranges' bytes).  ``TuningTable.pair_parts`` and ``pair_stationary`` keep what is in use.
+
+    The rule's choice for the class is what has to be beaten, at rows of the class, because ranges that are 14 % faster at 64 rows may be
+    slower at 8 (4,544 x 4,544 + 4,544 x 18,176, where a single timing at 64 rows chose for all: a step of 7B layers 3.07 -> 3.17 ms at 8
+    sequences, 3.61 -> 3.68 at 32)."""
     key = (tuple(w1.shape), tuple(w2.shape))
     if not PAIR_TUNE or key in _active.pair_parts or not may_time():
         return
     lib = ops.load_library()
     (N1, K1), (N2, K2) = w1.shape, w2.shape
-    a0, b0 = ops.gemm_splitk_pair_parts(N1, K1, N2, K2)
-    fix = lambda c: lib.pta_gemm_splitk_pair_fix(int(N1), int(K1), int(N2), int(K2), int(c[0]), int(c[1]), int(c[2]))
-    forget = lambda: lib.pta_gemm_splitk_pair_fix(int(N1), int(K1), int(N2), int(K2), 0, 0, 1)
-    fix_st = lambda cls, c: lib.pta_gemm_splitk_pair_fix_stationary(int(N1), int(K1), int(N2), int(K2), int(cls), int(c[0]), int(c[1]))
-    for cls in range(len(ops.STATIONARY_CLASS_ROWS)):
+    shapes = (int(N1), int(K1), int(N2), int(K2))
+    class_rows = (8, 32, 64, 128)
+    rules = [ops.gemm_splitk_pair_way(*shapes, rows) for rows in class_rows]  # nothing is fixed for the shapes yet
+    few, middle = rules[0], rules[2] if rules[2][2] != 3 else None
+    fix = lambda c: lib.pta_gemm_splitk_pair_fix(*shapes, int(c[0]), int(c[1]), int(c[2]))
+    forget = lambda: lib.pta_gemm_splitk_pair_fix(*shapes, 0, 0, 1)
+    fix_st = lambda cls, c: lib.pta_gemm_splitk_pair_fix_stationary(*shapes, int(cls), int(c[0]), int(c[1]))
+    for cls in range(len(class_rows)):
         fix_st(cls, (0, 0))  # the launches timed first are the staged kernel's
-    cands = [(a0, b0, 1)] + [(a, b, 1) for a in range(max(1, a0 - 1), a0 + 3) for b in range(max(1, b0 - 2), b0 + 3)
-                             if (a, b) != (a0, b0)]
-    tall = lambda p: sorted({max(1, p - 1), p, p + 1, max(1, 2 * p - 1), 2 * p, 2 * p + 1})
-    cands += [(a, b, 2) for a in tall(a0) for b in tall(b0)]
-    cands = [c for c in cands if fix(c) == 0]
-    xs = {rows: [torch.randn((rows, K), dtype=torch.float32, device=w1.device).to(torch.bfloat16) for K in (K1, K2)]
-          for rows in sorted({PAIR_TUNE_ROWS, 24, 8, 32, 64, 128})}
-    xs_bf16 = {rows: torch.zeros((rows, N1), dtype=torch.bfloat16, device=w1.device) for rows in xs}
+    near = lambda a0, b0: [(a, b, 1) for a in range(max(1, a0 - 1), a0 + 3) for b in range(max(1, b0 - 2), b0 + 3)]
+    tall = lambda a0, b0: [(a, b, 2) for a in sorted({max(1, a0 - 1), a0, a0 + 1, max(1, 2 * a0 - 1), 2 * a0, 2 * a0 + 1})
+                           for b in sorted({max(1, b0 - 1), b0, b0 + 1, max(1, 2 * b0 - 1), 2 * b0, 2 * b0 + 1})]
+    ways = lambda rule, others: [rule] + [c for c in dict.fromkeys(others) if c != rule and fix(c) == 0]  # those that the kernel takes
+    few_ways = ways(few, near(*few[:2]))
+    middle_ways = ways(middle, near(*middle[:2]) + near(*few[:2]) + tall(*middle[:2]) + tall(*few[:2])) if middle else []
+    larger = min(64, max(41, PAIR_TUNE_ROWS))
+    counts = {rows: [torch.randn((rows, K), dtype=torch.float32, device=w1.device).to(torch.bfloat16) for K in (K1, K2)]
+              for rows in sorted({*class_rows, 40, larger})}
+    xs_bf16 = {rows: torch.zeros((rows, N1), dtype=torch.bfloat16, device=w1.device) for rows in counts}
     kmin = min(K1, K2)
     f1, f2 = max(1, (K1 + kmin // 2) // kmin), max(1, (K2 + kmin // 2) // kmin)
-    st_cands = [(b * f1, b * f2) for b in (1, 2, 3, 4, 6) if b * f1 <= 16 and b * f2 <= 16 and fix_st(0, (b * f1, b * f2)) == 0]
+    st_cands = [(b * f1, b * f2) for b in (1, 2, 3, 4, 6) if b * f1 <= 16 and b * f2 <= 16]
+    st_cands = [c for c in dict.fromkeys([r[:2] for r in rules if r[2] == 3] + st_cands) if fix_st(0, c) == 0]
     fix_st(0, (0, 0))
-    most = [max([c[i] for c in cands] + [c[i] for c in st_cands] + [16]) for i in (0, 1)]
+    most = [max([c[i] for c in few_ways + middle_ways] + [c[i] for c in st_cands] + [16]) for i in (0, 1)]
     parts = [torch.empty((most[i], 128, N), dtype=torch.float32, device=w1.device) for i, N in enumerate((N1, N2))]
     # A launch is timed over several copies of the matrices in turn (more bytes than the memory-side cache holds),
     # back to back between two events: every launch reads its matrices from memory, as in a model, and no gap of
@@ -700,7 +720,18 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
     n_copies = max(2, min(6, int(640e6 // copy_bytes) + 1))
     copies = [(w1, w2)] + [(w1.clone(), w2.clone()) for _ in range(n_copies - 1)]
 
-    def timed_ways(chosen, rows, rounds=3, fix=fix, read=None):
+    # Two products of the same width are a block's last ones, and what reads their partial sums next is the norm
+    # that adds them: it is launched behind every timed launch, so that a launch pays for
+    # the ranges it leaves to be added and for how it leaves them (all at once at its end, or as it goes).
+    norm_w = (torch.ones(N1, dtype=torch.float32, device=w1.device)
+              if N1 == N2 and ops.layernorm_sum_ok(N1) and os.environ.get("PTA_PAIR_TUNE_READER", "1") != "0" else None)
+
+    def read_sums(c, rows):
+        views = [parts[i].view(-1)[:int(c[i]) * rows * N].view(int(c[i]), rows, N) for i, N in enumerate((N1, N2))]
+        ops.layernorm_sum([(views[1], None), (views[0], None), xs_bf16[rows]], N1, w=norm_w, b=norm_w, eps=1e-5)
+
+    def timed_ways(chosen, rows, fix, rounds=4):
+        """Milliseconds of a launch and of reading its sums, for each of the ways (ranges, ranges, ..) that ``fix`` sets."""
         best = [float("inf")] * len(chosen)
         for r in range(rounds + 1):  # the first round warms up
             for j, c in enumerate(chosen):
@@ -708,72 +739,57 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
                 start, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
                 start.record()
                 for a, b in copies:
-                    ops._call("pta_gemm_splitk_pair_bf16", ops._ptr(parts[0]), ops._ptr(xs[rows][0]), ops._ptr(a), int(N1), int(K1),
-                          ops._ptr(parts[1]), ops._ptr(xs[rows][1]), ops._ptr(b), int(N2), int(K2), rows, ops._stream())
-                    if read is not None:
-                        read(c, rows)
+                    ops._call("pta_gemm_splitk_pair_bf16", ops._ptr(parts[0]), ops._ptr(counts[rows][0]), ops._ptr(a), int(N1), int(K1),
+                          ops._ptr(parts[1]), ops._ptr(counts[rows][1]), ops._ptr(b), int(N2), int(K2), rows, ops._stream())
+                    if norm_w is not None:
+                        read_sums(c, rows)
                 end.record()
                 end.synchronize()
                 if r > 0:
                     best[j] = min(best[j], start.elapsed_time(end) / len(copies))
-        return best
+        # (what reads partial sums afterwards takes some 8 TB/s worth of them)
+        return best if norm_w is not None else [t + (c[0] * N1 + c[1] * N2) * rows * 4 / 8e12 * 1e3 for t, c in zip(best, chosen)]
 
-    # Two products of the same width are a block's last ones, and what reads their partial sums next is the norm
-    # that adds them: it is launched behind every timed launch of the comparison below, so that a launch pays for
-    # the ranges it leaves to be added and for how it leaves them (all at once at its end, or as it goes).
-    norm_w = (torch.ones(N1, dtype=torch.float32, device=w1.device)
-              if N1 == N2 and ops.layernorm_sum_ok(N1) and os.environ.get("PTA_PAIR_TUNE_READER", "1") != "0" else None)
+    say = (lambda text: print(f"[pta tune] pair {key}: {text}", flush=True)) if os.environ.get("PTA_TUNE_VERBOSE") else (lambda text: None)
 
-    def read_sums(c, rows):
-        views = [parts[i].view(-1)[:int(c[-2 + i]) * rows * N].view(int(c[-2 + i]), rows, N) for i, N in enumerate((N1, N2))]
-        ops.layernorm_sum([(views[1], None), (views[0], None), xs_bf16[rows]], N1, w=norm_w, b=norm_w, eps=1e-5)
+    def choose(found, label, rows):
+        times = [timed_ways(found, n, fix) for n in rows]
+        i = pick_way(times, PAIR_TUNE_MARGIN)
+        show = lambda j: f"{found[j]} " + " / ".join(f"{t[j] * 1e3:.1f}" for t in times)
+        say(f"{label}: rule {show(0)} us; fastest " + ", ".join(show(j) for j in sorted(range(len(found)), key=lambda j: sum(t[j] for t in times))[:5]) +
+            f" -> {found[i]}")
+        return found[i]
 
-    try:
-        times = timed_ways(cands, PAIR_TUNE_ROWS)
-        order = sorted(range(len(cands)), key=lambda i: times[i])
-        short = [0] + [i for i in order if i != 0 and times[i] < PAIR_TUNE_MARGIN * times[0]][:3]
-        small = timed_ways([cands[i] for i in short], 24) if len(short) > 1 else [0.0]
-    finally:
-        forget()
-    if os.environ.get("PTA_TUNE_VERBOSE"):
-        print(f"[pta tune] pair {key}: rule {cands[0]} {times[0] * 1e3:.1f} us at {PAIR_TUNE_ROWS} rows; fastest " +
-              ", ".join(f"{cands[i]} {times[i] * 1e3:.1f}" for i in order[:6]) +
-              (f"; at 24 rows {[round(t * 1e3, 1) for t in small]} for {[cands[i] for i in short]}" if len(short) > 1 else ""),
-              flush=True)
-    chosen = cands[0]
-    for i, t24 in zip(short[1:], small[1:]):  # fastest first
-        if t24 <= 1.03 * small[0]:
-            chosen = cands[i]
-            break
-    fix(chosen)
-    _active.pair_parts[key] = chosen
-    # the launch with stationary activations against that choice, per class of rows
     chosen_st = []
     try:
-        for cls, rows in enumerate((8, 32, 64, 128)):
-            fix_st(cls, (0, 0))
-            # what reads the partial sums afterwards pays for every range (measured: some 8 TB/s worth of them), so
-            # a launch is charged for its ranges' bytes at that rate on top of its own time
-            read = read_sums if norm_w is not None else None
-            slices_ms = (lambda c: 0.0) if read else (lambda c: (c[0] * N1 + c[1] * N2) * rows * 4 / 8e12 * 1e3)
-            t_staged = timed_ways([chosen[:2]], rows, fix=lambda c: None, read=read)[0] + slices_ms(chosen)
-            t_st = (timed_ways([(cls,) + c for c in st_cands], rows, fix=lambda a: fix_st(a[0], a[1:]), read=read)
-                    if st_cands else [])
-            t_st = [t + slices_ms(c) for t, c in zip(t_st, st_cands)]
+        a, b, _ = choose(few_ways, "8 / 32 rows", (8, 32))
+        cut = choose([(a, b, 1), (a, b, 2)], "128 rows", (128,))  # (the tile height counts beyond 32 rows)
+        if middle:
+            cut = cut + choose(middle_ways, f"40 / {larger} rows", (40, larger))
+        _fix_pair(*key, cut)
+        # the launch with stationary activations against that choice, per class of rows
+        for cls, rows in enumerate(class_rows):
             # the fewest ranges among those within 1.5 % of the fastest: what separates them is less than a box
             # varies, and fewer ranges leave whatever reads them next less to read
-            best = (min((i for i in range(len(st_cands)) if t_st[i] <= 1.015 * min(t_st)), key=lambda i: st_cands[i])
-                    if st_cands else -1)
-            keep = st_cands[best] if best >= 0 and t_st[best] < 0.98 * t_staged else (0, 0)
+            staged = ops.gemm_splitk_pair_parts(*shapes, rows)
+            t_staged = timed_ways([staged], rows, lambda c: fix_st(cls, (0, 0)))[0]
+            t_st = timed_ways(st_cands, rows, lambda c: fix_st(cls, c)) if st_cands else []
+            best = min((i for i in range(len(st_cands)) if t_st[i] <= 1.015 * min(t_st)), key=lambda i: st_cands[i]) if st_cands else -1
+            found = [((0, 0), t_staged)] + ([(st_cands[best], t_st[best])] if best >= 0 else [])
+            if rules[cls][2] == 3:  # the rule's ranges first
+                found.insert(0, (rules[cls][:2], t_st[st_cands.index(rules[cls][:2])]))
+            keep = found[pick_way([[t for _, t in found]], 0.98)][0]
             chosen_st.append(keep)
-            if os.environ.get("PTA_TUNE_VERBOSE"):
-                print(f"[pta tune] pair {key} at {rows} rows (with the reading of the partial sums): staged {t_staged * 1e3:.1f} us; stationary " +
-                      ", ".join(f"{c} {t * 1e3:.1f}" for c, t in zip(st_cands, t_st)) + f" -> {keep}", flush=True)
-    finally:
-        while len(chosen_st) < len(ops.STATIONARY_CLASS_ROWS):
-            chosen_st.append((0, 0))
-        for cls, c in enumerate(chosen_st):
-            fix_st(cls, c)
+            fix_st(cls, (0, 0))
+            say(f"at {rows} rows: staged {t_staged * 1e3:.1f} us; stationary " + ", ".join(f"{c} {t * 1e3:.1f}" for c, t in zip(st_cands, t_st)) +
+                f"; rule {rules[cls]} -> {keep}")
+    except BaseException:
+        forget()
+        fix_st(-1, (0, 0))
+        raise
+    for cls, c in enumerate(chosen_st):
+        fix_st(cls, c)
+    _active.pair_parts[key] = cut
     _active.pair_stationary[key] = tuple(chosen_st)
 
 

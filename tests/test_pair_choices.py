@@ -40,6 +40,35 @@ def test_recorded_ranges_hold_at_every_row_count(table, shape):
     assert _ranges(shape, 24, 48) == [few, middle]
 
 
+@pytest.mark.parametrize("shape", SHAPES)
+def test_ranges_of_33_to_64_rows_are_their_own(table, shape):
+    """A table with ranges for both: neither reaches the other's rows, and the table as data brings both back; what the kernel does not
+    take is refused."""
+    from pytorch_transformers_amd import ops
+
+    lib = ops.load_library()
+    first = {"pair_parts": {_key(shape): [2, 1, 1, 4, 2, 2]}, "pair_stationary": {_key(shape): [[0, 0]] * 4}}
+    table.load_tuning(first)
+    for _ in range(2):
+        assert [ops.gemm_splitk_pair_way(*shape, M) for M in (8, 24, 33, 64, 65, 200)] == [(2, 1, 1), (2, 1, 1), (4, 2, 2), (4, 2, 2), (2, 1, 1), (2, 1, 1)]
+        kept = table.tuning_table()
+        assert kept["pair_parts"] == first["pair_parts"]
+        table.clear_tuning()
+        table.load_tuning(kept)
+    for wrong in ([2, 1, 1, 4, 2, 3], [2, 1, 1, 4, 17, 1], [2, 1, 1, 4]):
+        with pytest.raises(ops.KernelError, match="not valid"):
+            table.load_tuning({"pair_parts": {_key(shape): wrong}})
+    assert lib.pta_gemm_splitk_pair_fix_middle(328, 2112, 200, 4608, 1, 3, 1) == 1, "small matrices have none of their own there"
+
+
+@pytest.mark.parametrize("times,kept", [([[5.0, 4.0, 3.0]], 2), ([[5.0, 4.9]], 0), ([[5.0, 3.0], [5.0, 5.1]], 0), ([[5.0, 4.5, 3.0], [5.0, 5.0, 5.1]], 1),
+                                        ([[5.0]], 0), ([[5.0, 4.0], [5.0, 4.0]], 1)])
+def test_the_rule_stays_unless_beaten_at_every_count_of_rows(times, kept):
+    from pytorch_transformers_amd import tuning
+
+    assert tuning.pick_way(times, 0.97) == kept
+
+
 @pytest.mark.parametrize("shape", SHAPES + [(328, 2112, 200, 4608)])
 @pytest.mark.parametrize("cls", range(4))
 def test_a_class_of_rows_leaves_the_others(table, shape, cls):
