@@ -1591,9 +1591,10 @@ def gemm_splitk_ok(x: torch.Tensor, w: torch.Tensor) -> bool:
     """Whether the kernel for a decode batch of 17 to 128 rows is the faster choice.  Measured at K = 4,544 and
     K = 18,176: it beats the vendor library except where N is long against K (the feed-forward's first matrix
     and the output head), which give the library enough row tiles to fill the chip; those of small matrices do not
-    (``_splitk_small``)."""
+    (``_splitk_small``; rows that lie apart or share memory, which ``mm_rows`` takes and this kernel does not, stay with it)."""
     return (_bf16_rows_ok(x, w) and 16 < x.shape[0] <= tuning.SPLITK_MAX_ROWS
-            and (w.shape[0] < 2 * w.shape[1] or _splitk_small(x.shape[0], *w.shape)) and tuning.splitk_rows_ok(x, w))
+            and (w.shape[0] < 2 * w.shape[1] or (_splitk_small(x.shape[0], *w.shape) and x.is_cuda and x.is_contiguous() and w.is_contiguous()))
+            and tuning.splitk_rows_ok(x, w))
 
 
 def _splitk_small(M: int, N: int, K: int) -> bool:

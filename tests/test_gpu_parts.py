@@ -190,6 +190,26 @@ def test_products_long_in_n_as_a_decode_batch(M, N, K, ok):
     _close(lin(x, act="gelu"), P.gelu(P.linear(x.double().cpu(), ref["a.weight"], ref["a.bias"])), 2e-2, "product")
 
 
+@pytest.mark.parametrize("M", [17, 24, 64, 128])
+@pytest.mark.parametrize("rows", ["apart", "shared", "columns of a transposed matrix"])
+def test_products_long_in_n_of_rows_that_lie_apart(M, rows):
+    """Inputs whose rows lie apart or share memory, of a matrix that the decode batch kernel takes from rows side by side: taken as by
+    ``mm_rows``, and a query_key_value tail is the caller's."""
+    from types import SimpleNamespace
+
+    from pytorch_transformers_amd import ops
+    from pytorch_transformers_amd.parts import Linear
+
+    N, K = 1024, 264
+    lin = Linear("a", K, N, bias=True)
+    _, ref = _fill(lin, torch.bfloat16, 1)
+    wide = _rand(M, K + 8, seed=3).bfloat16().cuda()
+    x = {"apart": wide[:, :K], "shared": wide[:1, :K].expand(M, K), "columns of a transposed matrix": wide[:, :K].t().contiguous().t()}[rows]
+    assert not x.is_contiguous() and ops.gemm_splitk_ok(x.contiguous(), lin.weight) and not ops.gemm_splitk_ok(x, lin.weight)
+    assert lin.with_tail(x, SimpleNamespace(head_dim=64)) is None
+    _close(lin(x, act="gelu"), P.gelu(P.linear(x.double().cpu(), ref["a.weight"], ref["a.bias"])), 2e-2, "product")
+
+
 def test_library_product_over_ranges_of_k():
     """A few hundred rows with K long against N: the library's batched product over ranges of K, its 32-bit
     partial sums added in order by the kernel that applies bias, activation and additions.  Which way is
