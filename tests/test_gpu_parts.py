@@ -200,7 +200,7 @@ def test_products_long_in_n_of_rows_that_lie_apart(M, rows):
     from pytorch_transformers_amd import ops
     from pytorch_transformers_amd.parts import Linear
 
-    N, K = 1024, 264
+    N, K = 2064, 1032
     lin = Linear("a", K, N, bias=True)
     _, ref = _fill(lin, torch.bfloat16, 1)
     wide = _rand(M, K + 8, seed=3).bfloat16().cuda()
