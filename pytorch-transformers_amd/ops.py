@@ -1601,7 +1601,9 @@ def _splitk_small(M: int, N: int, K: int) -> bool:
     """N long against K, up to 8,192: over cold weights, ``mm_rows`` -> the decode batch kernel, 17 / 64 rows, us: 4,160 x 1,040 13.4 ->
     7.5, 13.5 -> 10.2; 3,072 x 1,536 12.1 -> 7.5, 12.4 -> 9.1; 8,192 x 2,048 15.8 -> 12.2, 16.3 -> 15.7.  Beyond M N = 2^19 the tiles
     win again (8,192 x 2,048 at 96 rows 19.2 -> 19.4, 6,144 x 2,048 at 128 18.4 -> 21.0, 11,008 x 2,048 at 48 18.9 -> 20.2), and with
-    short rows sooner (8,192 x 256 at 64 7.0 -> 5.8, at 96 6.8 -> 7.1; 2,048 x 64 at 32 3.9 -> 3.3, at 64 4.0 -> 4.4)."""
+    short rows sooner (8,192 x 256 at 64 7.0 -> 5.8, at 96 6.8 -> 7.1; 2,048 x 64 at 32 3.9 -> 3.3, at 64 4.0 -> 4.4).  Rows count by
+    their next multiple of eight, to which a captured step is padded: it takes the way of the same step run directly."""
+    M = (M + 7) // 8 * 8
     return M <= (32 if K < 256 else 64 if K < 1024 else 128) and N <= min(8192, (1 << 19) // M)
 
 
