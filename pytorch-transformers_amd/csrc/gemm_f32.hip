@@ -686,7 +686,7 @@ static bool few_rows(int M, int N, int K) {
 static F32Plan f32_plan(int M, int N, int K) {
     F32Plan best{0, 0, 0, 1, 1e30};
     if (few_rows(M, N, K)) return best;
-    const int units = 256, used = segments(K), blocks = k_blocks(K);
+    const int units = pta_compute_units(), used = segments(K), blocks = k_blocks(K);
     for (int fp = 2; fp <= 4; fp += 2)
         for (int fq = 1; fq <= 4; ++fq) {
             const F32Costs& c = costs[fp / 2 - 1][fq - 1];
@@ -719,13 +719,14 @@ static F32Plan f32_plan(int M, int N, int K) {
 
 template <int ROWS>
 static void launch_few(float* C, const float* A, const float* W, F32Epilogue epi, int rows, int N, int K, hipStream_t s) {
-    // whole rounds of the 256 compute units, up to 32 rows of W each; small matrices: four rows a workgroup
-    int groups = 256 * ((N + 256 * 32 - 1) / (256 * 32));
+    // whole rounds of the compute units, up to 32 rows of W each; small matrices: four rows a workgroup
+    const int all = pta_compute_units();
+    int groups = all * ((N + all * 32 - 1) / (all * 32));
     if (groups > (N + 3) / 4) groups = (N + 3) / 4;
     const bool two = (N + groups - 1) / groups > 16;
     // Rings in LDS: their offsets are 32-bit bytes within a workgroup's rows.  Up to sixteen rows of W a unit, whose waves take a block
     // or two each, they pay from five rows of A on: 2,048 x 2,048 1 row 7.9 us, in rings 8.7, 8 rows 9.6 and 8.8, 16 rows 11.1 and 8.9.
-    const int units = groups < 256 ? groups : 256;  // one workgroup a unit, with its rows of all rounds
+    const int units = groups < all ? groups : all;  // one workgroup a unit, with its rows of all rounds
     if (ROWS != ROW_ELEMENTS && rows <= 16 && (two || rows > 4) && (long)(N / units + 1) * K * 4 < LDS_PAST && (long)rows * K * 4 < LDS_PAST) {
         auto go = [&](auto kernel, int bytes) {
             if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;

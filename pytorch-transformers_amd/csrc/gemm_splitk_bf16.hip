@@ -8,8 +8,9 @@
 // (lds_stream.h), D - 1 stages ahead, with one barrier a stage.  K is split over gridDim.y workgroups when N alone
 // gives too few of them to occupy the chip; each writes its 32-bit partial tile to `part`, and a second small kernel
 // adds the partials in the order of the ranges and applies bias, activation and additions; with reduce = 0 the partials
-// are the result, and the kernel that reads them next adds them in the same order.  The split is chosen from N
-// and K alone, so the order of summation does not depend on the batch.
+// are the result, and the kernel that reads them next adds them in the same order.  The split of a product on its own is chosen
+// from N and K alone, so its order of summation does not depend on the batch; pairs have one for steps of up to 32 rows, one for
+// 33 to 64 and one for more.
 //
 // Through registers, sixteen rows of W a load, the same ranges took (pairs of products, us, registers -> LDS): 4,544 x 4,544 with
 // 4,544 x 18,176 1 row 42.7 -> 40.5, 32 rows 49.6 -> 45.0; 4,096 x 4,096 with 4,096 x 16,384 39.8 -> 36.1, 46.0 -> 39.3; 9,216 and 32,768 x
@@ -410,8 +411,9 @@ static int reduce_parts(const SplitkProblem& a, int M, int reduce, hipStream_t s
     return pta_check_launch("gemm_splitk_bf16");
 }
 
-template <int MT, int RT, int D>
+template <int MT, int RT>
 static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
+    constexpr int D = 4;  // stages in LDS
     constexpr int lds = D * splitk_slot(MT, RT);
     static_assert(lds <= 160 * 1024, "the stages must fit the LDS of a compute unit");
     // rows of W a multiple of 4 KB long are the ones that crowd memory channels: there every workgroup starts at a
@@ -441,15 +443,15 @@ static int tiles_per_chunk(int M) {
     return ((M + chunks - 1) / chunks + 15) / 16;
 }
 
-template <int RT, int D = 4>
+template <int RT>
 static int launch_rows(int MT, const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
     switch (MT) {
-        case 1: return launch_cfg<1, RT, D>(a, b, M, reduce, s);
-        case 2: return launch_cfg<2, RT, D>(a, b, M, reduce, s);
-        case 3: return launch_cfg<3, RT, D>(a, b, M, reduce, s);
-        case 4: return launch_cfg<4, RT, D>(a, b, M, reduce, s);
-        case 5: case 6: return launch_cfg<6, RT, D>(a, b, M, reduce, s);
-        default: return launch_cfg<8, RT, D>(a, b, M, reduce, s);
+        case 1: return launch_cfg<1, RT>(a, b, M, reduce, s);
+        case 2: return launch_cfg<2, RT>(a, b, M, reduce, s);
+        case 3: return launch_cfg<3, RT>(a, b, M, reduce, s);
+        case 4: return launch_cfg<4, RT>(a, b, M, reduce, s);
+        case 5: case 6: return launch_cfg<6, RT>(a, b, M, reduce, s);
+        default: return launch_cfg<8, RT>(a, b, M, reduce, s);
     }
 }
 

@@ -42,7 +42,7 @@ __device__ __forceinline__ int stream_row(int lane, int l) { return l * 8 + (lan
 __device__ __forceinline__ int stream_element(int lane, int l) { return ((lane & 7) ^ ((4 * l + (lane >> 4)) & 7)) * 8; }
 
 // Elements of a row that this takes: the rows of a tile lie within 32-bit bytes of each other, those of a query_key_value
-// projection's rotation pairs (two heads of up to 256) too.
+// projection's rotation pairs (up to 512 rows apart) too.
 #define STREAM_MOST_K (1 << 20)
 
 template <int LOADS>

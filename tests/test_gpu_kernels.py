@@ -169,7 +169,8 @@ def test_gemm_splitk_of_the_longest_rows(K):
                                                    (4544, 4544, 0, 0, 0, 0), (250, 18176 // 4, 5, 1, 2, 4),
                                                    (1000, 1096, 1, 2, 2, 4), (333, 2056, 4, 1, 2, 2)])
 def test_gemm_splitk_bf16(M, N, K, parts, rt, sb, depth):
-    """The batch product with x shared through LDS: every row tile count, stage depth and split of K."""
+    """The batch product with x shared through LDS: every row tile count and split of K.  (Blocks a stage and stages in flight, which
+    an earlier kernel had a choice of, are accepted and change nothing.)"""
     ops = _ops()
     x = _rand(M, K, dtype=torch.bfloat16)
     w = _rand(N, K, seed=1, dtype=torch.bfloat16, scale=0.05)
