@@ -291,99 +291,159 @@ __global__ __launch_bounds__(512, CT * RT <= 2 ? 2 : 1) void gemm_f32_few_kernel
 // compute unit, in tiles of up to 16 RT.  Sums change hands through LDS, in two places in turn, one barrier a tile.
 // 18,176 x 4,544, us with registers and three rounds of workgroups -> this: 1 row 70.0 -> 60.5 (5.5 TB/s), 16 rows 86.5 -> 67; 4,544 x
 // 18,176 67 -> 65, 83 -> 70; 32,768 x 2,048 59.9 -> 53.9, 72.3 -> 55.6.
+//
+// Two products of the same rows of A in one launch (PRODUCTS 2: a block's query_key_value and first feed-forward matrix, or the last
+// matrices of both branches, whose K and A differ): a workgroup has its share of the rows of both and its rings go on from the first to the
+// second as from tile to tile, so that one launch starts and ends where two did.  With `add_first` (matrices of one N) the first's
+// results, bias and activation done, lie in LDS until the second's have them added.  us on their own -> so, 1 / 8 / 16 rows: 4,672 and 18,176 by
+// 4,544 85.4 -> 80.4, 90.7 -> 85.5, 95.5 -> 90.7; 4,544 by 4,544 and by 18,176 95.6 -> 87.7, 94.7 -> 85.7, 97.2 -> 89.3; 2,048 by 2,048
+// and by 8,192 33.8 -> 31.7, 36.9 -> 31.8, 37.7 -> 32.9; 3,072 and 4,096 by 1,024 14.2 -> 11.7, 13.4 -> 11.7, 13.5 -> 11.9.  Of the
+// 80.4 some 73 are the loads; taking values apart is not all hidden beside them (a third block on its way changed nothing).
 template <int RT, int D>
 struct FewRing {
     static constexpr int SLOT = (RT + 1) * 2048, RING = D * SLOT, LOADS = 2 * (RT + 1);
     static constexpr int LDS = SEGS * RING + 2 * SEGS * RT * 1024;
 };
 
-template <int RT, int D>
-__global__ __launch_bounds__(512, 2) void gemm_f32_few_ring_kernel(float* __restrict__ C, const float* __restrict__ A, const float* __restrict__ W,
-                                                                   F32Epilogue epi, int M, int N, int K, int each, int over) {
+struct F32Few {
+    float* C;
+    const float* A;
+    const float* W;
+    F32Epilogue epi;
+    int N, K;
+    int each, over;  // rows of W a workgroup has, and how many of the first workgroups have one more
+};
+
+template <int PRODUCTS>
+struct F32FewJob {
+    F32Few of[PRODUCTS];
+};
+
+template <int RT, int D, int PRODUCTS>
+__global__ __launch_bounds__(512, 2) void gemm_f32_few_ring_kernel(F32FewJob<PRODUCTS> job, int M, int add_first) {
     using R = FewRing<RT, D>;
-    extern __shared__ __attribute__((aligned(1024))) char lds[];  // the waves' rings, then the sums, [2][segment][RT][64]
+    extern __shared__ __attribute__((aligned(1024))) char lds[];  // the waves' rings, the sums, [2][segment][RT][64], the first's results
     const int lane = threadIdx.x & 63, seg = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, g = lane >> 4;
-    const int n0 = blockIdx.x * each + min((int)blockIdx.x, over), rows = each + ((int)blockIdx.x < over ? 1 : 0);
-    const int tiles = (rows + 16 * RT - 1) / (16 * RT), per_tile = (rows + tiles - 1) / tiles;
-    const int nb = k_blocks(K), sb = seg_blocks(K), used = segments(K);
-    const int b0 = seg * sb, b1 = min(nb, b0 + sb);
-    const i32x4_t w = buffer_of(W + (long)n0 * K, rows * K * 4), x = buffer_of(A, M * K * 4);
     char* ring = lds + seg * R::RING;
+    f32x4* sums = reinterpret_cast<f32x4*>(lds + SEGS * R::RING);
+    float* kept = reinterpret_cast<float*>(lds + R::LDS);  // [row of the workgroup][16]
     const unsigned to = __builtin_amdgcn_readfirstlane(lds_address(ring));
     const int c4[2] = {stream_element(lane, 0) / 2, stream_element(lane, 1) / 2};  // four values where a bfloat16 row has eight
-    int x_at[2], w_at[2 * RT];
-#pragma unroll
-    for (int l = 0; l < 2; ++l) x_at[l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 4 : LDS_PAST;
-    auto rows_of = [&](int tile) {
+    struct Mine {  // what a workgroup, and of its K this wave, has of a product
+        int n0, rows, tiles, per_tile, b0, blocks;
+    };
+    auto mine_of = [&](const F32Few& p) {
+        Mine m;
+        m.n0 = blockIdx.x * p.each + min((int)blockIdx.x, p.over);
+        m.rows = p.each + ((int)blockIdx.x < p.over ? 1 : 0);
+        m.tiles = max((m.rows + 16 * RT - 1) / (16 * RT), 1);
+        m.per_tile = (m.rows + m.tiles - 1) / m.tiles;
+        m.b0 = seg * seg_blocks(p.K);
+        m.blocks = max(min(k_blocks(p.K) - m.b0, seg_blocks(p.K)), 1);  // (a wave without a segment multiplies a block of zeros)
+        return m;
+    };
+    // what is asked for next: a block of a tile of a product
+    const float *w_from, *x_from;
+    int w_bytes, x_bytes;
+    Mine next;
+    int K, product = -1, tile = 0, block = 0, row_at[R::LOADS];  // rows of W, and of A behind them
+    auto rows_of = [&]() {
 #pragma unroll
         for (int l = 0; l < 2 * RT; ++l) {
-            const int i = (l >> 1) * 16 + stream_row(lane, l & 1), row = tile * per_tile + i;
-            w_at[l] = i < per_tile && row < rows ? row * K * 4 : LDS_PAST;
+            const int i = (l >> 1) * 16 + stream_row(lane, l & 1), row = tile * next.per_tile + i;
+            row_at[l] = i < next.per_tile && row < next.rows ? row * K * 4 : LDS_PAST;
         }
     };
-    int p_tile = 0, p_block = b0;  // what is asked for next
-    auto issue = [&](int slot) {
-        const int k = p_block * BK;
+    auto next_product = [&]() {
+        if (++product == PRODUCTS) return;
+        const F32Few& p = job.of[product];
+        next = mine_of(p);
+        K = p.K;
+        w_from = p.W + (long)next.n0 * K, w_bytes = next.rows * K * 4;
+        x_from = p.A, x_bytes = M * K * 4;
+        tile = block = 0;
+        rows_of();
 #pragma unroll
-        for (int l = 0; l < R::LOADS; ++l) {
-            const int row_at = l < 2 * RT ? w_at[l] : x_at[l & 1];
-            const int at = p_tile < tiles && p_block < b1 && row_at != LDS_PAST && k + c4[l & 1] < K ? row_at + (k + c4[l & 1]) * 4 : LDS_PAST;
-            fetch16(l < 2 * RT ? w : x, to + slot + l * 1024, at);
-        }
-        if (++p_block >= b1) {
-            p_block = b0;
-            rows_of(++p_tile);
+        for (int l = 0; l < 2; ++l) row_at[2 * RT + l] = stream_row(lane, l) < M ? stream_row(lane, l) * K * 4 : LDS_PAST;
+    };
+    auto issue = [&](int slot) {
+        const i32x4_t w = buffer_of(w_from, w_bytes), x = buffer_of(x_from, x_bytes);
+        const int k = product < PRODUCTS ? (next.b0 + block) * BK : K;
+#pragma unroll
+        for (int l = 0; l < R::LOADS; ++l)
+            fetch16(l < 2 * RT ? w : x, to + slot + l * 1024, row_at[l] != LDS_PAST && k + c4[l & 1] < K ? row_at[l] + (k + c4[l & 1]) * 4 : LDS_PAST);
+        if (product < PRODUCTS && ++block == next.blocks) {
+            block = 0;
+            if (++tile < next.tiles) rows_of();
+            else next_product();
         }
     };
-    rows_of(0);
+    next_product();
 #pragma unroll
     for (int d = 0; d < D; ++d) issue(d * R::SLOT);
     const int in_row = r16 * 128 + ((g ^ (r16 >> 1)) & 7) * 16;  // elements 4 g of a block, and 64 flipped 16 + 4 g
-    f32x4* sums = reinterpret_cast<f32x4*>(lds + SEGS * R::RING);
-    int slot = 0;
-    for (int t = 0; t < tiles; ++t) {
-        f32x4 acc[RT];
+    int slot = 0, turn = 0;  // tiles so far, of both products
+#pragma unroll 1
+    for (int q = 0; q < PRODUCTS; ++q) {
+        const F32Few& p = job.of[q];
+        const Mine mine = mine_of(p);
+        const int used = segments(p.K);
+        for (int t = 0; t < mine.tiles; ++t, ++turn) {
+            f32x4 acc[RT];
 #pragma unroll
-        for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
-        for (int b = b0; b < b1; ++b) {
-            wait_loads<(D - 1) * R::LOADS>();
-            f32x4 v[RT + 1][2];
+            for (int r = 0; r < RT; ++r) acc[r] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < mine.blocks; ++b) {
+                wait_loads<(D - 1) * R::LOADS>();
+                f32x4 v[RT + 1][2];
 #pragma unroll
-            for (int r = 0; r <= RT; ++r)
+                for (int r = 0; r <= RT; ++r)
 #pragma unroll
-                for (int h = 0; h < 2; ++h) v[r][h] = *reinterpret_cast<const f32x4*>(ring + ((in_row ^ (h * 64)) + slot + r * 2048));
-            wait_reads();
-            __builtin_amdgcn_sched_barrier(0);
-            issue(slot);  // into the slot just read
-            __builtin_amdgcn_sched_barrier(0);
-            const Parts xs = split8<true>(v[RT][0], v[RT][1]);
+                    for (int h = 0; h < 2; ++h) v[r][h] = *reinterpret_cast<const f32x4*>(ring + ((in_row ^ (h * 64)) + slot + r * 2048));
+                wait_reads();
+                __builtin_amdgcn_sched_barrier(0);
+                issue(slot);  // into the slot just read
+                __builtin_amdgcn_sched_barrier(0);
+                const Parts xs = split8<true>(v[RT][0], v[RT][1]);
 #pragma unroll
-            for (int r = 0; r < RT; ++r) {
-                const Parts ws = split8<true>(v[r][0], v[r][1]);
+                for (int r = 0; r < RT; ++r) {
+                    const Parts ws = split8<true>(v[r][0], v[r][1]);
 #pragma unroll
-                for (int term = 0; term < TERMS; ++term)
-                    acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws.part[term_w(term)], xs.part[term_x(term)], acc[r], 0, 0, 0);
+                    for (int term = 0; term < TERMS; ++term)
+                        acc[r] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws.part[term_w(term)], xs.part[term_x(term)], acc[r], 0, 0, 0);
+                }
+                slot = slot == R::RING - R::SLOT ? 0 : slot + R::SLOT;
             }
-            slot = slot == R::RING - R::SLOT ? 0 : slot + R::SLOT;
-        }
-        f32x4* mine = sums + (t & 1) * (SEGS * RT * 64);
+            f32x4* meet_at = sums + (turn & 1) * (SEGS * RT * 64);
 #pragma unroll
-        for (int r = 0; r < RT; ++r) mine[(seg * RT + r) * 64 + lane] = acc[r];
-        wait_reads();
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        const int r = (seg - t * RT) & (SEGS - 1);  // the waves take turns at what follows
-        if (r >= RT) continue;
-        f32x4 u = mine[r * 64 + lane];
-        for (int s = 1; s < used; ++s) u += mine[(s * RT + r) * 64 + lane];
-        const int n_end = n0 + min(rows, (t + 1) * per_tile), n16 = n0 + t * per_tile + 16 * r;
-        u = whole_sum<ROW_VECTORS>(u, A, W, 0, n16, M, N, K);
-        const int n = n16 + 4 * g;
-        if (r16 < M) {
+            for (int r = 0; r < RT; ++r) meet_at[(seg * RT + r) * 64 + lane] = acc[r];
+            wait_reads();
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const int r = (seg - turn * RT) & (SEGS - 1);  // the waves take turns at what follows
+            if (r >= RT) continue;
+            f32x4 u = meet_at[r * 64 + lane];
+            for (int s = 1; s < used; ++s) u += meet_at[(s * RT + r) * 64 + lane];
+            const int end = min(mine.rows, (t + 1) * mine.per_tile), at16 = t * mine.per_tile + 16 * r;
+            u = whole_sum<ROW_VECTORS>(u, p.A, p.W, 0, mine.n0 + at16, M, p.N, p.K);
+            const bool keep = PRODUCTS > 1 && q == 0 && add_first;
+            if (r16 < M) {
 #pragma unroll
-            for (int j = 0; j < 4; ++j)
-                if (n + j < n_end) C[(long)r16 * N + n + j] = finish(u[j], epi, n + j, (long)r16 * N + n + j);
+                for (int j = 0; j < 4; ++j) {
+                    const int i = at16 + 4 * g + j, n = mine.n0 + i;  // (read a barrier and more after it was kept)
+                    if (i >= end) continue;
+                    if (PRODUCTS > 1 && q == 1 && add_first) {
+                        F32Epilogue bare = p.epi;
+                        bare.add1 = bare.add2 = nullptr;
+                        const float v = finish(u[j], bare, n, 0) + kept[i * 16 + r16];
+                        p.C[(long)r16 * p.N + n] = p.epi.add1 ? v + p.epi.add1[(long)r16 * p.N + n] : v;
+                    } else {
+                        const float v = finish(u[j], p.epi, n, (long)r16 * p.N + n);
+                        if (keep) kept[i * 16 + r16] = v;
+                        else p.C[(long)r16 * p.N + n] = v;
+                    }
+                }
+            }
         }
     }
     wait_loads<0>();  // nothing is on its way to LDS any more
@@ -728,12 +788,13 @@ static void launch_few(float* C, const float* A, const float* W, F32Epilogue epi
     // or two each, they pay from five rows of A on: 2,048 x 2,048 1 row 7.9 us, in rings 8.7, 8 rows 9.6 and 8.8, 16 rows 11.1 and 8.9.
     const int units = groups < all ? groups : all;  // one workgroup a unit, with its rows of all rounds
     if (ROWS != ROW_ELEMENTS && rows <= 16 && (two || rows > 4) && (long)(N / units + 1) * K * 4 < LDS_PAST && (long)rows * K * 4 < LDS_PAST) {
+        const F32Few p{C, A, W, epi, N, K, N / units, N % units};
         auto go = [&](auto kernel, int bytes) {
             if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, bytes) != hipSuccess) return false;
-            hipLaunchKernelGGL(kernel, dim3(units), dim3(512), bytes, s, C, A, W, epi, rows, N, K, N / units, N % units);
+            hipLaunchKernelGGL(kernel, dim3(units), dim3(512), bytes, s, F32FewJob<1>{{p}}, rows, 0);
             return true;
         };
-        if (two ? go(gemm_f32_few_ring_kernel<2, 2>, FewRing<2, 2>::LDS) : go(gemm_f32_few_ring_kernel<1, 2>, FewRing<1, 2>::LDS)) return;
+        if (two ? go(gemm_f32_few_ring_kernel<2, 2, 1>, FewRing<2, 2>::LDS) : go(gemm_f32_few_ring_kernel<1, 2, 1>, FewRing<1, 2>::LDS)) return;
     }
 #define FEW(CT, RT, D) hipLaunchKernelGGL((gemm_f32_few_kernel<CT, RT, D, ROWS>), dim3(groups), dim3(512), 0, s, C, A, W, epi, M, N, K)
     for (int at = 0; at < rows; at += 64) {  // more than 64 rows: where tiles cannot address K
@@ -817,7 +878,57 @@ extern "C" int pta_gemm_f32(float* C, const float* A, const float* W, const floa
     return f32_run(f32_plan(M, N, K), C, A, W, bias, add1, add2, M, N, K, act, scratch, stream);
 }
 
-// The same with the choice in the caller's hands, for measuring one against another and for tests of each: fp = 0 for the
+// How two products of up to sixteen rows run in one launch, or none (units 0) where they do not: each of them one that the kernels for
+// few rows have, rows sixteen-byte aligned, 32-bit offsets within a workgroup's rows, and the first's results in what LDS is left.
+struct F32PairPlan {
+    int units, tiles;  // workgroups, and tiles of sixteen rows of W that their rings hold
+    int lds;
+};
+
+static F32PairPlan f32_pair_plan(int M, int N1, int K1, int N2, int K2, bool add_first) {
+    const F32PairPlan none{0, 0, 0};
+    if (M < 1 || M > 16 || N1 < 1 || N2 < 1 || K1 < 1 || K2 < 1 || K1 % 4 || K2 % 4 || (add_first && N1 != N2)) return none;
+    if (!few_rows(M, N1, K1) || !few_rows(M, N2, K2)) return none;
+    const int most = N1 > N2 ? N1 : N2;
+    F32PairPlan p;
+    p.units = pta_compute_units();
+    if (p.units > (most + 3) / 4) p.units = (most + 3) / 4;  // small matrices: four rows a workgroup
+    p.tiles = (most + p.units - 1) / p.units > 16 ? 2 : 1;
+    const int rings = p.tiles == 2 ? FewRing<2, 2>::LDS : FewRing<1, 2>::LDS;
+    const long kept = add_first ? (N1 / p.units + 1) * 64L : 0;
+    if (rings + kept > 160 * 1024) return none;
+    for (const long bytes : {(N1 / p.units + 1L) * K1 * 4, (N2 / p.units + 1L) * K2 * 4, (long)M * K1 * 4, (long)M * K2 * 4})
+        if (bytes >= LDS_PAST) return none;
+    p.lds = rings + (int)kept;
+    return p;
+}
+
+extern "C" int pta_gemm_f32_pair_ok(int M, int N1, int K1, int N2, int K2, int add_first) {
+    return f32_pair_plan(M, N1, K1, N2, K2, add_first != 0).units > 0;
+}
+
+// C1 = act1(A1 . W1^T + bias1) and C2 = act2(A2 . W2^T + bias2), or with C1 null the one result C2 = act2(A2 . W2^T + bias2) +
+// act1(A1 . W1^T + bias1) + add, from one launch: the values that pta_gemm_f32 gives, bit by bit.
+extern "C" int pta_gemm_f32_pair(float* C1, const float* A1, const float* W1, const float* bias1, int N1, int K1, int act1,
+                                 float* C2, const float* A2, const float* W2, const float* bias2, int N2, int K2, int act2,
+                                 const float* add, int M, void* stream) {
+    PTA_REQUIRE(A1 && W1 && C2 && A2 && W2, "gemm_f32_pair: null pointer");
+    PTA_REQUIRE(pta_act_known(act1) && pta_act_known(act2), "gemm_f32_pair: unknown activation %d or %d", act1, act2);
+    PTA_REQUIRE(!C1 || !add, "gemm_f32_pair: an addition goes with the sum of the two");
+    for (const void* q : {(const void*)A1, (const void*)W1, (const void*)A2, (const void*)W2})
+        PTA_REQUIRE((uintptr_t)q % 16 == 0, "gemm_f32_pair: rows must be 16-byte aligned");
+    const F32PairPlan p = f32_pair_plan(M, N1, K1, N2, K2, !C1);
+    PTA_REQUIRE(p.units > 0, "gemm_f32_pair: no launch for %d rows by %d x %d and %d x %d", M, N1, K1, N2, K2);
+    const F32Few a{C1, A1, W1, F32Epilogue{bias1, nullptr, nullptr, act1, 0}, N1, K1, N1 / p.units, N1 % p.units};
+    const F32Few b{C2, A2, W2, F32Epilogue{bias2, add, nullptr, act2, 0}, N2, K2, N2 / p.units, N2 % p.units};
+    auto kernel = p.tiles == 2 ? gemm_f32_few_ring_kernel<2, 2, 2> : gemm_f32_few_ring_kernel<1, 2, 2>;
+    PTA_REQUIRE(hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, p.lds) == hipSuccess,
+                "gemm_f32_pair: %d bytes of LDS were refused", p.lds);
+    hipLaunchKernelGGL(kernel, dim3(p.units), dim3(512), p.lds, (hipStream_t)stream, F32FewJob<2>{{a, b}}, M, C1 ? 0 : 1);
+    return pta_check_launch("gemm_f32_pair");
+}
+
+// pta_gemm_f32 with the choice in the caller's hands, for measuring one against another and for tests of each: fp = 0 for the
 // kernel for few rows, else fp 2 or 4 and fq 1 to 4; `room` 32-bit values at scratch.
 extern "C" int pta_gemm_f32_as(float* C, const float* A, const float* W, const float* bias, const float* add1,
                                const float* add2, int M, int N, int K, int act, int fp, int fq, int whole, int share,

@@ -14,7 +14,7 @@
 
 #include <stdint.h>
 
-#define PTA_ABI_VERSION 20
+#define PTA_ABI_VERSION 21
 
 #ifdef __cplusplus
 extern "C" {
@@ -136,6 +136,11 @@ int pta_gemm_f32(float* C, const float* A, const float* W, const float* bias, co
 // The same with the choice of kernel in the caller's hands (gemm_f32.hip); room: values that scratch holds.
 int pta_gemm_f32_as(float* C, const float* A, const float* W, const float* bias, const float* add1, const float* add2,
                     int M, int N, int K, int act, int fp, int fq, int whole, int share, float* scratch, long room, void* stream);
+// Two such products of the same M rows from one launch, C1 and C2, or with C1 null their sum and `add` (may be null) as C2; the values of
+// the products on their own, bit by bit.  pta_gemm_f32_pair_ok: whether there is a launch for these sizes (add_first: for the sum).
+int pta_gemm_f32_pair_ok(int M, int N1, int K1, int N2, int K2, int add_first);
+int pta_gemm_f32_pair(float* C1, const float* A1, const float* W1, const float* bias1, int N1, int K1, int act1, float* C2,
+                      const float* A2, const float* W2, const float* bias2, int N2, int K2, int act2, const float* add, int M, void* stream);
 
 // Attention of 32-bit heads of up to 256 elements, a multiple of 4, on the 32-bit matrix instruction: the arguments of
 // pta_attn_generic, and the step's sequences in the tokens' order (cu_tokens null: every token is taken by itself, in any

@@ -25,7 +25,7 @@ QKV_LAYOUT_CODES = {"grouped": 0, "tail": 1, "interleaved": 2}
 ACT_CODES = {None: 0, "none": 0, "linear": 0, "gelu": 1, "gelu_python": 1, "gelu_new": 2, "gelu_pytorch_tanh": 2,
              "gelu_fast": 2, "gelu_accurate": 2, "quick_gelu": 3, "relu": 4, "relu2": 5, "relu6": 6, "silu": 7, "swish": 7,
              "sigmoid": 8, "tanh": 9, "leaky_relu": 10, "mish": 11, "gelu_10": 12, "laplace": 13}
-ABI_VERSION = 20
+ABI_VERSION = 21
 PAIRING_CODES = {"half": 0, "interleaved": 1}  # PtaPairing: elements (i, i + rotary_dim / 2) or (2i, 2i + 1)
 BIAS_OF_CODES = {"key": 0, "distance": 1}  # PtaBiasOf: the slope times the key's position, or times key - query position
 
@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -188,6 +188,9 @@ def _entry_cost(name: str, a) -> tuple:
         return gemm(a[19], (a[14] + 2 * a[15]) * a[16], a[20])
     if name == "pta_gemm_f32":
         return gemm(a[6], a[7], a[8], 4)
+    if name == "pta_gemm_f32_pair":
+        one, two = gemm(a[15], a[4], a[5], 4), gemm(a[15], a[11], a[12], 4)
+        return (one[0] + two[0], one[1] + two[1])
     if name == "pta_layernorm_sum":
         return ((a[4] + a[7]) * float(a[17]) * a[19] * 4, 0.0)
     if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_latent_decode", "pta_attn_latent_mfma", "pta_attn_latent_prompt", "pta_attn_latent", "pta_attn_talk",
@@ -718,6 +721,43 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, a
     scratch = torch.empty(need, dtype=torch.float32, device=a.device) if need else None
     _call("pta_gemm_f32", _ptr(out), _ptr(a), _ptr(w), _ptr(bias), _ptr(add1), _ptr(add2), M, N, K, ACT_CODES[act],
           _ptr(scratch), _stream())
+    return out
+
+
+def gemm_f32_pair_ok(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: torch.Tensor, add_first: bool = False) -> bool:
+    """Whether ``gemm_f32_pair`` (with ``add_first``: ``gemm_f32_pair_sum``) has a launch for these: up to sixteen rows of each."""
+    if not all(t.dtype == torch.float32 and t.dim() == 2 and t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0
+               for t in (a1, w1, a2, w2)):
+        return False
+    if a1.shape[0] != a2.shape[0] or a1.shape[0] > 16 or a1.shape[1] != w1.shape[1] or a2.shape[1] != w2.shape[1]:
+        return False
+    return bool(load_library().pta_gemm_f32_pair_ok(a1.shape[0], w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], int(add_first)))
+
+
+def _gemm_f32_pair(out1, out2, a1, w1, bias1, act1, a2, w2, bias2, act2, add) -> None:
+    for name, t in (("a1", a1), ("w1", w1), ("a2", a2), ("w2", w2)):
+        _need(t, name, torch.float32)
+    M, (N1, K1), (N2, K2) = a1.shape[0], w1.shape, w2.shape
+    _need(a1, "a1", shape=(M, K1))
+    _need(a2, "a2", shape=(M, K2))
+    for name, t, shape in (("bias1", bias1, (N1,)), ("bias2", bias2, (N2,)), ("add", add, (M, N2))):
+        if t is not None:
+            _need(t, name, torch.float32, shape)
+    _call("pta_gemm_f32_pair", _ptr(out1), _ptr(a1), _ptr(w1), _ptr(bias1), N1, K1, ACT_CODES[act1], _ptr(out2), _ptr(a2), _ptr(w2),
+          _ptr(bias2), N2, K2, ACT_CODES[act2], _ptr(add), M, _stream())
+
+
+def gemm_f32_pair(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: torch.Tensor, bias1=None, act1=None, bias2=None, act2=None):
+    """``(act1(a1 @ w1.T + bias1), act2(a2 @ w2.T + bias2))`` as ``gemm_f32`` gives them, from one launch, where ``gemm_f32_pair_ok``."""
+    both = [torch.empty((a1.shape[0], w.shape[0]), dtype=torch.float32, device=a1.device) for w in (w1, w2)]
+    _gemm_f32_pair(both[0], both[1], a1, w1, bias1, act1, a2, w2, bias2, act2, None)
+    return both[0], both[1]
+
+
+def gemm_f32_pair_sum(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: torch.Tensor, bias1=None, bias2=None, add=None):
+    """``(a2 @ w2.T + bias2) + (a1 @ w1.T + bias1) + add``, added in that order as ``gemm_f32`` with additions does, from one launch."""
+    out = torch.empty((a1.shape[0], w2.shape[0]), dtype=torch.float32, device=a1.device)
+    _gemm_f32_pair(None, out, a1, w1, bias1, None, a2, w2, bias2, None, add)
     return out
 
 

@@ -57,6 +57,9 @@ def _sum_parallel(ffn_out: PendingProjection, mixer_out: PendingProjection, x: t
     both = PendingProjection.partial_pair(ffn_out, mixer_out)
     if both is not None:
         return ResidualSum([both[0], both[1], x])
+    formed = PendingProjection.pair_sum(ffn_out, mixer_out, x)
+    if formed is not None:
+        return formed
     p = ffn_out.partial()
     if p is not None:
         return ResidualSum([p, mixer_out.partial() or mixer_out.run(), x])

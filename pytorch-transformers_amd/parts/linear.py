@@ -153,12 +153,14 @@ class Linear(Part):
         decode kernels (same rows, no additions); else None.  ``tail`` (a ``QkvTail``) says what the caller will
         do with the first result; where the launch can do that itself, the first result comes back as
         ``TailDone(queries)``."""
-        if not (x1.dtype == torch.bfloat16 and x1.shape[0] == x2.shape[0]):
-            return None
-        if any(k not in ("act", "apply_bias") for k in list(kw1) + list(kw2)):
+        if x1.shape[0] != x2.shape[0] or any(k not in ("act", "apply_bias") for k in list(kw1) + list(kw2)):
             return None
         b1 = first.bias if kw1.get("apply_bias", True) else None
         b2 = second.bias if kw2.get("apply_bias", True) else None
+        if ops.gemm_f32_pair_ok(x1, first.weight, x2, second.weight):
+            return ops.gemm_f32_pair(x1, first.weight, x2, second.weight, b1, kw1.get("act"), b2, kw2.get("act"))
+        if x1.dtype != torch.bfloat16:
+            return None
         if (tail is not None and x1.shape == x2.shape and kw1.get("act") is None
                 and ops.gemm_skinny_pair_qkv_ok(x1, first.weight, second.weight, tail.head_dim)):
             q, y2 = ops.gemm_skinny_pair_qkv(
@@ -252,6 +254,14 @@ class PendingProjection:
         return (x.dtype == torch.bfloat16 and lin.bias is None and ops.layernorm_sum_ok(lin.out_features)
                 and x.shape[0] >= ops.layernorm_sum_rows_min()
                 and not ops.gemm_skinny_ok(x, lin.weight) and not ops.gemm_splitk_ok(x, lin.weight))
+
+    @staticmethod
+    def pair_sum(last: "PendingProjection", first: "PendingProjection", x: torch.Tensor) -> Optional[torch.Tensor]:
+        """``last + first + x``, added in that order, from one launch, or None where there is none (32-bit, few rows)."""
+        a, b = first, last
+        if x.dtype != torch.float32 or not ops.gemm_f32_pair_ok(a.x, a.linear.weight, b.x, b.linear.weight, add_first=True):
+            return None
+        return ops.gemm_f32_pair_sum(a.x, a.linear.weight, b.x, b.linear.weight, a.linear.bias, b.linear.bias, x)
 
     @staticmethod
     def partial_pair(first: "PendingProjection", second: "PendingProjection"):

@@ -336,3 +336,38 @@ def test_a_prompt_beside_single_tokens_costs_what_the_two_cost():
 
     apart = us([(1000, 1)] * 32) + us([(0, 64)])
     assert us([(1000, 1)] * 32 + [(0, 64)]) <= 4 * apart + 50
+
+
+@pytest.mark.parametrize("M,N1,K1,N2,K2", [(1, 4672, 4544, 18176, 4544), (16, 4544, 4544, 4544, 18176), (7, 36, 64, 1000, 68),
+                                           (2, 3, 1024, 4100, 8), (16, 8193, 260, 8193, 28), (5, 2064, 2048, 2064, 1028)])
+def test_two_products_in_one_launch_are_the_products_on_their_own(M, N1, K1, N2, K2):
+    """Bit by bit, with biases, activations and the sum of the two: workgroups with rows of one matrix alone, waves without a segment of
+    one K, one tile of sixteen rows and two."""
+    ops = _ops()
+    g = torch.Generator(device="cuda").manual_seed(M + N1 + K2)
+    draw = lambda *shape: torch.randn(shape, generator=g, device="cuda")
+    a1, w1, b1, a2, w2, b2 = draw(M, K1), draw(N1, K1), draw(N1), draw(M, K2), draw(N2, K2), draw(N2)
+    assert ops.gemm_f32_pair_ok(a1, w1, a2, w2)
+    got = ops.gemm_f32_pair(a1, w1, a2, w2, b1, None, b2, "gelu")
+    assert torch.equal(got[0], ops.gemm_f32(a1, w1, b1))
+    assert torch.equal(got[1], ops.gemm_f32(a2, w2, b2, "gelu"))
+    if N1 == N2:
+        x = draw(M, N2)
+        first = ops.gemm_f32(a1, w1, b1)
+        for bias, add in ((b2, x), (None, None)):
+            assert torch.equal(ops.gemm_f32_pair_sum(a1, w1, a2, w2, b1, bias, add), ops.gemm_f32(a2, w2, bias, None, first, add))
+        big = a1.clone()
+        big[0, 3] = float("inf")  # a sum that is formed on the 32-bit instruction
+        want = ops.gemm_f32(a2, w2, None, None, ops.gemm_f32(big, w1), None)
+        assert torch.equal(torch.nan_to_num(ops.gemm_f32_pair_sum(big, w1, a2, w2)), torch.nan_to_num(want))
+
+
+def test_pairs_that_have_no_launch():
+    w = lambda n, k: torch.empty((n, k), device="cuda")
+    ok = _ops().gemm_f32_pair_ok
+    assert not ok(w(17, 2048), w(64, 2048), w(17, 2048), w(64, 2048))  # more rows than the rings take
+    assert not ok(w(1, 6), w(64, 6), w(1, 8), w(64, 8))  # rows that are no multiple of sixteen bytes
+    assert not ok(w(1, 64), w(64, 64), w(2, 64), w(64, 64))
+    assert not ok(w(1, 64), w(64, 64), w(1, 64), w(60, 64), add_first=True)
+    assert not ok(w(1, 8192), w(32768, 8192), w(1, 8192), w(64, 8192))  # a matrix that goes by tiles
+    assert not ok(w(1, 64).bfloat16(), w(64, 64).bfloat16(), w(1, 64).bfloat16(), w(64, 64).bfloat16())
