@@ -74,3 +74,33 @@ def test_a_capture_without_memory(monkeypatch, make, failures):
     assert torch.equal(got, want) and len(captures) == failures + 1
     assert [(g.graph is not None, g.direct) for g in cache._decode_graphs.values()] == [(True, 0)]
     assert sorted(cache.length(s) for s in range(2)) == [7, 9]
+
+
+@pytest.mark.parametrize("make", [_model, _stateful])
+@pytest.mark.parametrize("failures", [0, 1, 2])
+def test_a_shape_captured_before_is_captured_first(monkeypatch, make, failures):
+    """In a second cache the step of a known shape is captured and replayed, with no launch of its own; where the capture finds no
+    memory twice, the steps are launched directly, and each once: states that layers keep move on by one token a step."""
+    from pytorch_transformers_amd.engine import model as engine
+
+    model = make()
+    want, _ = _steps(model, 6)
+    monkeypatch.setattr(engine, "DIRECT_STEPS", 2)
+    forward, left, calls = model.forward_tokens, [failures], []
+
+    def short_of_memory(*args):
+        out = forward(*args)
+        calls.append(torch.cuda.is_current_stream_capturing())
+        if calls[-1] and left[0]:
+            left[0] -= 1
+            raise torch.cuda.OutOfMemoryError("no memory")
+        return out
+
+    monkeypatch.setattr(model, "forward_tokens", short_of_memory)
+    got, cache = _steps(model, 6)
+    assert torch.equal(got, want)
+    # the prompts' step, then captures; with no memory twice: three steps directly, and the next is captured and replayed
+    assert calls == [False] + {0: [True], 1: [True, True], 2: [True, True, False, False, False, True]}[failures]
+    assert [(g.graph is not None, g.direct) for g in cache._decode_graphs.values()] == [(True, 0)]
+    model.tune(table=model.tune(table={}))  # choices may have changed: the next step of the shape sets up what they need
+    assert not model._captured_shapes
