@@ -182,7 +182,7 @@ def generate(model, prompts: Sequence[Sequence[int]], generation_config: Optiona
     # Steps ahead of the host: where nothing of a step's decisions needs more than the tokens themselves, the next
     # step is launched from the tokens on the device before the host has read them.
     ahead = (bool(getattr(model, "steps_ahead", False)) and getattr(sampler, "needs_histories", True) is False
-             and not want_scores and not want_logits and streamer is None and not stop_strings
+             and not want_scores and streamer is None and not stop_strings
              and cfg.max_time is None and not keep_slots and not logits_processor and not stopping_criteria)
     pad = 0 if cfg.pad_token_id is None else int(cfg.pad_token_id)
     custom = dict(extra_processors=logits_processor, pad_token_id=pad) if logits_processor else {}
@@ -208,7 +208,7 @@ def generate(model, prompts: Sequence[Sequence[int]], generation_config: Optiona
         try:
             if ahead:
                 _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, out_tokens, new_budget,
-                              padded_len, done_with, first_draw)
+                              padded_len, done_with, first_draw, out_logits)
                 live = []
             while live:
                 logits = model.step(cache, [slot_of[i] for i in live], [feed[i] for i in live], "last")
@@ -327,7 +327,7 @@ def _step_extras(sampler, step: int, new_budget: int) -> dict:
 
 
 def _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, out_tokens, new_budget, padded_len,
-                  done_with, first_draw) -> None:
+                  done_with, first_draw, out_logits=None) -> None:
     """One batch, with every step launched before the host has seen the tokens of the step before it.
 
     The tokens of a step stay on the device (``sampler.sample(..., ahead=True)``) and the next step takes them
@@ -336,7 +336,7 @@ def _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, ou
     reads: its keys and values went into a slot that is given back, and whatever takes the slot's pages next is
     launched later on the same stream.  A sequence that ends by its length is known beforehand and never takes
     part in a step too many.  The tokens are those of the loop that waits after every step: a sequence's result
-    does not depend on what else is in its batch.
+    does not depend on what else is in its batch.  ``out_logits``: per sequence, the list that is to have its steps' logits.
     """
     from ..cache.paged import CacheFull
 
@@ -350,13 +350,14 @@ def _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, ou
 
     step_no = 0  # the number of the token that `pending` holds for each of its sequences
     seqs = list(batch)
-    pending = choose(model.step(cache, [slot_of[i] for i in seqs], [feed[i] for i in seqs], "last"), seqs, 0)
+    held = model.step(cache, [slot_of[i] for i in seqs], [feed[i] for i in seqs], "last")
+    pending = choose(held, seqs, 0)  # the tokens chosen from the rows of `held`
     rows = list(range(len(seqs)))  # the rows of `pending` whose sequences live, as far as the host knows
     while True:
         nxt = None
         if step_no + 1 < new_budget:  # (else every sequence ends with the pending token)
             try:
-                logits = model.step(cache, [slot_of[i] for i in seqs], pending.take(rows), "last", own_logits=False)
+                logits = model.step(cache, [slot_of[i] for i in seqs], pending.take(rows), "last", own_logits=out_logits is not None)
             except CacheFull:
                 logits = None  # no room to go on before knowing who has ended: wait for the tokens first
             if logits is not None:
@@ -367,6 +368,8 @@ def _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, ou
         for at, (row, i) in enumerate(zip(rows, seqs)):
             tok = int(tokens[row])
             out_tokens[i].append(tok)
+            if out_logits is not None:
+                out_logits[i].append(held[row])  # (a step's logits are a tensor of their own)
             if tok in eos or step_no >= new_budget:
                 done_with(i, slot_of.pop(i))
             else:
@@ -379,7 +382,7 @@ def _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, ou
             pending, rows = choose(logits, survivors, step_no), list(range(len(survivors)))
         else:
             pending, rows = nxt, on
-        seqs = survivors
+        seqs, held = survivors, logits
 
 
 def _ends_with_stop(tokenizer, new_tokens: Sequence[int], stop_strings: Sequence[str]) -> bool:

@@ -353,6 +353,23 @@ def test_a_step_ahead_that_finds_no_room_waits_for_the_tokens_and_goes_on_with_w
     assert ("step", None) in log[1:]  # the step that waited
 
 
+def test_logits_are_kept_ahead_of_the_host_as_by_the_loop_that_waits():
+    """The same rows for every sequence, also where sequences end at different steps and where a step finds no room."""
+    a, b = [1] * 60, [2] * 62
+    for prompts, eos, room in (([[1, 2, 3], [20, 5], [9]], 12, None), ([a, b], expected(a, 3)[-1], 128)):
+        outs = []
+        for model, sampler in ((ScriptedModel(), ArgmaxSampler([eos])), (AheadModel(log := []), AheadSampler(log, [eos]))):
+            cache = None if room is None else model.new_cache(room, max_slots=2)
+            outs.append(generate(model, prompts, GenerationConfig(max_new_tokens=6, eos_token_id=eos, output_logits=True,
+                                                                  return_dict_in_generate=True), sampler=sampler, cache=cache))
+        assert any(what == "step from" for what, _ in log)
+        waits, ahead = outs
+        assert waits.sequences == ahead.sequences and len({len(rows) for rows in waits.logits}) > 1
+        for seq, p, one, two in zip(waits.sequences, prompts, waits.logits, ahead.logits):
+            assert len(one) == len(two) == len(seq) - len(p)
+            assert all(torch.equal(torch.as_tensor(x), torch.as_tensor(y)) for x, y in zip(one, two))
+
+
 def test_what_needs_the_tokens_on_the_host_keeps_the_loop_that_waits():
     class Reads(AheadSampler):
         needs_histories = True
