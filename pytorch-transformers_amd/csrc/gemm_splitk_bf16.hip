@@ -18,9 +18,7 @@
 //
 // Chunks of x and W past the workgroup's K range, or rows past M and N, are read through a buffer descriptor at
 // an offset outside its bounds and arrive as zeros.
-#include "common.h"
-#include "lds_stream.h"
-#include "pta_kernels.h"
+#include "gemm_splitk_attn.h"
 #include "qkv_tail.h"
 
 #include <stdlib.h>
@@ -32,193 +30,10 @@
 #include <utility>
 #include <vector>
 
-// bytes of a stage of 64 elements of K in LDS: four waves' rows of W, and the rows of x by whole loads of each wave
-static constexpr __host__ __device__ int splitk_slot(int MT, int RT) { return RT * 8192 + (MT + 1) / 2 * 4096; }
-
-#define SK_THREADS 256
-#define SK_CHUNK_ROWS 128  // eight tiles of sixteen rows of x: what a workgroup holds
-#define SK_MAX_ROWS 256
-
-// One product of a launch.  A launch may carry two that share M (a block's two output projections, left
-// as partial sums): the workgroups of the second follow those of the first in a one-dimensional grid.
-struct SplitkProblem {
-    void* y;
-    float* part;
-    const bf16_t* x;
-    const bf16_t* W;
-    const float* bias;
-    const bf16_t* add1;
-    const bf16_t* add2;
-    int N, K, act, out_f32;
-    int blocks_per_part;  // 64-element blocks of K per range
-    int tiles;            // workgroups along N
-    int parts;            // ranges of K
-    int direct;           // one range and the epilogue in this kernel
-};
-
-// what follows a whole sum, for one element
-__device__ __forceinline__ void store_whole(void* y, const float* bias, const bf16_t* add1, const bf16_t* add2, int act, int out_f32, int n,
-                                            long o, float v) {
-    if (!out_f32) v = round_to_bf16(v);
-    if (bias) { v += bias[n]; if (!out_f32) v = round_to_bf16(v); }
-    if (act == PTA_ACT_GELU) v = out_f32 ? gelu_erf(v) : gelu_bf16(v);  // other activations: see pta_gemm_splitk_bf16
-    if (add1) v += bf16_bits_to_f32(add1[o]);
-    if (add2) v += bf16_bits_to_f32(add2[o]);
-    if (out_f32) ((float*)y)[o] = v;
-    else ((bf16_t*)y)[o] = f32_to_bf16_bits(v);
-}
-
 template <int MT, int RT, int D, bool ROT>
 __global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem pa, SplitkProblem pb, int M, int chunks,
                                                                  int chunk_rows, int rot_stride) {
-    constexpr int NX = (MT + 1) / 2;                 // loads of x per wave and stage (eight rows by 128 bytes each)
-    constexpr int NL = 2 * RT + NX;                  // all of a wave's loads per stage
-    constexpr int SLOT = splitk_slot(MT, RT);        // a stage in LDS: the four waves' rows of W, then x
-    extern __shared__ __attribute__((aligned(1024))) char lds[];  // [D][SLOT]
-
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int r = lane & 15, g = lane >> 4;
-    // More rows than a workgroup holds are cut into `chunks` chunks of `chunk_rows`; the workgroups that take the
-    // same rows of W for the chunks sit a multiple of eight apart in the grid, so that they start together on one
-    // die and all but the first find W in its cache.
-    const int first_blocks = pa.tiles * pa.parts;
-    int block = (int)blockIdx.x, chunk = 0;
-    if (chunks > 1) {
-        const int per_chunk = (int)gridDim.x / chunks, whole = per_chunk / 8 * 8, rest = per_chunk - whole;
-        if (block < whole * chunks) {
-            chunk = (block >> 3) % chunks;
-            block = block / (8 * chunks) * 8 + (block & 7);
-        } else {
-            const int t = block - whole * chunks;
-            chunk = t / rest;
-            block = whole + t % rest;
-        }
-    }
-    const int m0 = chunk * chunk_rows, m_end = min(M, m0 + chunk_rows);
-    const bool second = block >= first_blocks;
-    void* __restrict__ y = second ? pb.y : pa.y;
-    float* __restrict__ part = second ? pb.part : pa.part;
-    const bf16_t* __restrict__ x = second ? pb.x : pa.x;
-    const bf16_t* __restrict__ W = second ? pb.W : pa.W;
-    const float* __restrict__ bias = second ? pb.bias : pa.bias;
-    const bf16_t* __restrict__ add1 = second ? pb.add1 : pa.add1;
-    const bf16_t* __restrict__ add2 = second ? pb.add2 : pa.add2;
-    const int N = second ? pb.N : pa.N, K = second ? pb.K : pa.K, act = second ? pb.act : pa.act;
-    const int out_f32 = second ? pb.out_f32 : pa.out_f32, direct = second ? pb.direct : pa.direct;
-    const int blocks_per_part = second ? pb.blocks_per_part : pa.blocks_per_part;
-    const int tiles = second ? pb.tiles : pa.tiles;
-    const int idx = block - (second ? first_blocks : 0);
-    const int tile = idx % tiles, range = idx / tiles;  // neighbours share a range of K: its x slice stays in L2
-    const int n_base = tile * (64 * RT) + wave * (16 * RT);
-    const int nkb = (K + 63) >> 6;
-    const int kb0 = range * blocks_per_part, kb1 = min(kb0 + blocks_per_part, nkb);
-    const int k_begin = kb0 * 64, k_end = min(kb1 * 64, K);
-    const int nstages = kb1 - kb0;
-
-    // rows past the last one lie past the buffers' ends, elements past the range's end are asked for there: zeros, no traffic
-    const int n_rows = max(0, min(16 * RT, N - n_base));
-    const i32x4_t rw = buffer_of(W + (long)min(n_base, N - 1) * K, n_rows * K * 2), rx = buffer_of(x + (long)m0 * K, (m_end - m0) * K * 2);
-    const unsigned to_w = __builtin_amdgcn_readfirstlane(lds_address(lds)) + wave * (RT * 2048);
-    const unsigned to_x = __builtin_amdgcn_readfirstlane(lds_address(lds)) + RT * 8192 + wave * 1024;
-    int w_at[2 * RT], x_at[NX];  // the lane's rows
-#pragma unroll
-    for (int l = 0; l < 2 * RT; ++l) w_at[l] = ((l >> 1) * 16 + stream_row(lane, l & 1)) * K * 2;
-#pragma unroll
-    for (int l = 0; l < NX; ++l) {
-        const int row = (wave + 4 * l) * 8 + (lane >> 3);
-        x_at[l] = row < m_end - m0 ? row * K * 2 : LDS_PAST;
-    }
-    const int c8[2] = {stream_element(lane, 0), stream_element(lane, 1)};
-
-    f32x4_t acc[RT][MT];
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[t][mt] = f32x4_t{0.f, 0.f, 0.f, 0.f};
-
-    // Where a row of W is a power of two long, workgroups that walk the same range of K in step ask the same few
-    // memory channels at the same time (N = 4,096, K = 16,384: a third slower than K = 16,448).  So each walks its
-    // range from a starting stage of its own and wraps round; stages past the last read nothing.  A feature's
-    // order of summation follows from N, K and the launch alone.
-    const int rot = ROT && nstages > 0 ? (int)(((long)tile * rot_stride) % nstages) : 0;
-    auto issue = [&](int stage, int slot) {
-        int at = stage;
-        if (ROT) { at += rot; at -= at >= nstages ? nstages : 0; }
-        const int k = k_begin + at * 64;
-#pragma unroll
-        for (int l = 0; l < 2 * RT; ++l) {
-            const int ke = k + c8[l & 1];
-            fetch16(rw, to_w + slot + l * 1024, ke < k_end ? w_at[l] + ke * 2 : LDS_PAST);
-        }
-#pragma unroll
-        for (int l = 0; l < NX; ++l) {
-            const int ke = k + c8[wave & 1];  // (an even number of loads away from the wave's first: the same half of a tile)
-            fetch16(rx, to_x + slot + l * 4096, ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
-        }
-    };
-    const int in_row = r * 128 + ((g ^ (r >> 1)) & 7) * 16;  // the second 32 elements of a stage: 64 flipped
-    auto multiply = [&](int cur) {
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-            bf16x8_t w[RT], b[MT];
-            const int at = (in_row ^ (hf * 64)) + cur;
-#pragma unroll
-            for (int t = 0; t < RT; ++t) w[t] = *reinterpret_cast<const bf16x8_t*>(lds + at + (wave * RT + t) * 2048);
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt) b[mt] = *reinterpret_cast<const bf16x8_t*>(lds + at + RT * 8192 + mt * 2048);
-#pragma unroll
-            for (int t = 0; t < RT; ++t)
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    acc[t][mt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t], b[mt], acc[t][mt], 0, 0, 0);
-        }
-    };
-    // everyone's share of the stage has landed, and everyone is past reading the one before
-    auto meet = [&]() {
-        __builtin_amdgcn_s_barrier();
-        asm volatile("" ::: "memory");
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    // D - 1 stages are on their way, one barrier a stage, behind which the next loads take the place of the stage before; the last
-    // D - 1 stages wait for fewer and fewer.
-#pragma unroll
-    for (int d = 0; d < D - 1; ++d)
-        if (d < nstages) issue(d, d * SLOT);
-    int cur = 0, free = (D - 1) * SLOT;
-    for (int s = D - 1; s < nstages; ++s) {
-        wait_reads();
-        wait_loads<(D - 2) * NL>();
-        meet();
-        issue(s, free);
-        __builtin_amdgcn_sched_barrier(0);
-        multiply(cur);
-        free = cur;
-        cur = cur == (D - 1) * SLOT ? 0 : cur + SLOT;
-    }
-    RingTail<NL>::template last_steps<D - 2>(nstages, [&]() {
-        meet();
-        multiply(cur);
-        cur = cur == (D - 1) * SLOT ? 0 : cur + SLOT;
-    });
-
-    // lane: row m = mt*16 + r of x, columns n_base + t*16 + g*4 + 0..3
-#pragma unroll
-    for (int t = 0; t < RT; ++t)
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int m = m0 + mt * 16 + r, n = n_base + t * 16 + g * 4;
-            if (m >= m_end || n >= N) continue;
-            const long o = (long)m * N + n;
-            if (!direct) {
-                const long at = (long)range * M * N + o;
-                float* dst = part + at;
-                if (n + 3 < N && (at & 3) == 0) *reinterpret_cast<f32x4_t*>(dst) = acc[t][mt];
-                else
-                    for (int i = 0; i < 4 && n + i < N; ++i) dst[i] = acc[t][mt][i];
-                continue;
-            }
-            for (int i = 0; i < 4 && n + i < N; ++i) store_whole(y, bias, add1, add2, act, out_f32, n + i, o + i, acc[t][mt][i]);
-        }
+    splitk_body<MT, RT, D, ROT>(pa, pb, M, chunks, chunk_rows, rot_stride, (int)blockIdx.x, (int)gridDim.x, NoGate{});
 }
 
 // The same sums for rows too long for 32-bit offsets within a wave's rows of W (32 rows of 2^25 elements, 16 of 2^26), at most 31 of x: a
@@ -411,21 +226,30 @@ static int reduce_parts(const SplitkProblem& a, int M, int reduce, hipStream_t s
     return pta_check_launch("gemm_splitk_bf16");
 }
 
+// rows of W a multiple of 4 KB long are the ones that crowd memory channels: there every workgroup starts at a
+// stage of its own (PTA_SPLITK_ROT: stages between neighbours, 0 switches it off)
+static int rotation_stride() {
+    static const int env = getenv("PTA_SPLITK_ROT") ? atoi(getenv("PTA_SPLITK_ROT")) : -1;
+    return env >= 0 ? env : 1;
+}
+static bool rotated(const SplitkProblem& a, const SplitkProblem& b) {
+    return rotation_stride() > 0 && (a.K % 2048 == 0 || (b.N > 0 && b.K % 2048 == 0));
+}
+
+// (x lies within 32-bit offsets: check_splitk)
+static bool rows_too_long(const SplitkProblem& a, const SplitkProblem& b, int rt) { return (long)std::max(a.K, b.K) * 16 * rt * 2 >= LDS_PAST; }
+
 template <int MT, int RT>
 static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
     constexpr int D = 4;  // stages in LDS
     constexpr int lds = D * splitk_slot(MT, RT);
     static_assert(lds <= 160 * 1024, "the stages must fit the LDS of a compute unit");
-    // rows of W a multiple of 4 KB long are the ones that crowd memory channels: there every workgroup starts at a
-    // stage of its own (PTA_SPLITK_ROT: stages between neighbours, 0 switches it off)
-    static const int rot_env = getenv("PTA_SPLITK_ROT") ? atoi(getenv("PTA_SPLITK_ROT")) : -1;
-    const int rot_stride = rot_env >= 0 ? rot_env : 1;
-    const bool rotate = rot_stride > 0 && (a.K % 2048 == 0 || (b.N > 0 && b.K % 2048 == 0));
+    const int rot_stride = rotation_stride();
+    const bool rotate = rotated(a, b);
     auto kern = rotate ? gemm_splitk_kernel<MT, RT, D, true> : gemm_splitk_kernel<MT, RT, D, false>;
     if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return pta_fail("gemm_splitk_bf16: cannot have %d bytes of LDS", lds);
-    // (x lies within 32-bit offsets: check_splitk)
-    if ((long)std::max(a.K, b.K) * 16 * RT * 2 >= LDS_PAST) {
+    if (rows_too_long(a, b, RT)) {
         for (const SplitkProblem* p : {&a, &b})
             if (p->N > 0) hipLaunchKernelGGL(gemm_splitk_long_kernel, dim3(p->N, p->parts), dim3(64), 0, s, *p, M);
         return reduce_parts(a, M, reduce, s);
@@ -740,6 +564,53 @@ extern "C" int pta_gemm_splitk_pair_bf16(float* part1, const void* x1, const voi
     const SplitkProblem b = make_problem(nullptr, part2, x2, W2, nullptr, nullptr, nullptr, N2, K2, 0, 0, kind, p2, 0);
     if (kind == 2) return launch_rows<2>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
     return launch_rows<1>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
+}
+
+// Whether a decode step's attention of so many heads may ride in the launch of a pair: one of the staged kernel's, for steps of up to 64
+// rows, heads of 64 elements.
+extern "C" int pta_gemm_splitk_pair_attn_ok(int N1, int K1, int N2, int K2, int M, int nh, int nkv, int d) {
+    if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || M <= 0 || M > RIDE_MOST_ROWS || nkv <= 0 || nh <= 0 || nh % nkv || d != 16 * RIDE_HEAD ||
+        (long)nh * d != K2 || K1 % 8 || K2 % 8)
+        return 0;
+    int p1, p2;
+    const int rt = pick_pair_parts_rows(N1, K1, N2, K2, M, &p1, &p2);
+    return rt != 3 && (long)std::max(K1, K2) * 32 * 2 < LDS_PAST;
+}
+
+// The pair with the attention that its second product takes (x2 [M, nh d] is written here): pta_attn_mfma of one token a sequence,
+// whole contexts, `waves` (1 or 4) on a piece's keys; sync: groups of sixteen heads x nkv x M zeros; owners: -1, or how many of attention's
+// workgroups the launch is to begin with (the products' do the others).
+extern "C" int pta_gemm_splitk_pair_attn(float* part1, const void* x1, const void* W1, int N1, int K1, float* part2, void* x2,
+                                         const void* W2, int N2, int K2, int M, const void* q, const void* k_pool, const void* v_pool,
+                                         const int* block_table, int bt_stride, const int* cu_tokens, const int* seq_start,
+                                         const PtaScoreBias* score_bias, int nh, int nkv, int d, float scale, const float* sink, int waves,
+                                         int* sync, int owners, void* stream) {
+    PTA_REQUIRE(waves == 1 || waves == RIDE_WAVES, "gemm_splitk_pair_attn: 1 or %d waves on the keys of a piece, got %d", RIDE_WAVES, waves);
+    if (check_splitk("gemm_splitk_pair_attn", x1, W1, M, N1, K1)) return 1;
+    if (check_splitk("gemm_splitk_pair_attn", x2, W2, M, N2, K2)) return 1;
+    PTA_REQUIRE(pta_gemm_splitk_pair_attn_ok(N1, K1, N2, K2, M, nh, nkv, d), "gemm_splitk_pair_attn: no launch for %d rows by %d x %d and %d x %d, %d heads on %d of %d",
+                M, N1, K1, N2, K2, nh, nkv, d);
+    PTA_REQUIRE(part1 && part2 && sync && q && k_pool && v_pool && block_table && cu_tokens && seq_start, "gemm_splitk_pair_attn: null pointer");
+    for (const void* p : {q, k_pool, v_pool, (const void*)x2})
+        PTA_REQUIRE((uintptr_t)p % 16 == 0, "gemm_splitk_pair_attn: pointers must be 16-byte aligned");
+    int bias_mode = 0;
+    if (pta_score_bias_mode("gemm_splitk_pair_attn", score_bias, &bias_mode)) return 1;
+    const float* slopes = score_bias ? score_bias->slopes : nullptr;
+    int p1, p2;
+    const int rt = pick_pair_parts_rows(N1, K1, N2, K2, M, &p1, &p2);
+    const SplitkProblem a = make_problem(nullptr, part1, x1, W1, nullptr, nullptr, nullptr, N1, K1, 0, 0, rt, p1, 0);
+    const SplitkProblem b = make_problem(nullptr, part2, x2, W2, nullptr, nullptr, nullptr, N2, K2, 0, 0, rt, p2, 0);
+    AttnRide ride{};
+    ride.attn = AttnArgs{(bf16_t*)x2, (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_table, bt_stride, cu_tokens, seq_start,
+                         slopes, bias_mode, nh, nkv, scale * PTA_LOG2E, slopes ? PTA_LOG2E * score_bias->scale : 0.f, sink,
+                         pta_head_rows_of(nullptr, nh, d)};
+    ride.groups = (nh / nkv + 15) / 16;
+    ride.n_seqs = M;
+    const int pieces = ride.groups * nkv * M;
+    ride.tasks = waves == 1 ? (pieces + RIDE_WAVES - 1) / RIDE_WAVES : pieces;
+    ride.owners = owners < 0 || owners > ride.tasks ? ride.tasks : owners;
+    ride.sync = sync;
+    return pta_splitk_attn_launch(a, b, M, rt, rotated(a, b), rotation_stride(), waves > 1, ride, (hipStream_t)stream);
 }
 
 // The same pair run to the end: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2) in bfloat16; the two

@@ -269,6 +269,15 @@ int pta_gemm_stationary_rule(int N1, int K1, int N2, int K2, int cls, int* q1, i
 int pta_gemm_splitk_pair_bf16(float* part1, const void* x1, const void* W1, int N1, int K1, float* part2,
                               const void* x2, const void* W2, int N2, int K2, int M, void* stream);
 
+// The same pair with the attention that its second product takes in the same launch (gemm_splitk_attn.hip): x2 [M, nh d] is written.  One token a
+// sequence, heads of 64, up to 64 sequences, waves (1 or 4) on the keys of sixteen heads.  sync: (sixteens of heads of a KV head) x nkv x M
+// 32-bit zeros; owners: -1, or how many of the attention's workgroups the launch begins with (the products' workgroups do the others: for tests).
+int pta_gemm_splitk_pair_attn_ok(int N1, int K1, int N2, int K2, int M, int nh, int nkv, int d);
+int pta_gemm_splitk_pair_attn(float* part1, const void* x1, const void* W1, int N1, int K1, float* part2, void* x2, const void* W2, int N2,
+                              int K2, int M, const void* q, const void* k_pool, const void* v_pool, const int* block_table, int bt_stride,
+                              const int* cu_tokens, const int* seq_start, const PtaScoreBias* score_bias, int nh, int nkv, int d, float scale,
+                              const float* sink, int waves, int* sync, int owners, void* stream);
+
 // the same pair run to the end: y1 = act1(x1 . W1^T + bias1), y2 = act2(x2 . W2^T + bias2), bfloat16
 int pta_gemm_splitk_pair_reduced_bf16(void* y1, float* part1, const void* x1, const void* W1, const float* bias1, int N1,
                                       int K1, int act1, void* y2, float* part2, const void* x2, const void* W2,

@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok", "pta_gemm_splitk_pair_attn_ok")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -824,6 +824,47 @@ def attn_mfma(q: torch.Tensor, k_pool, v_pool, block_table, cu_tokens, seq_start
 
 
 
+class LateAttention:
+    """Attention of a decode step that has not run yet, into ``out`` [tokens, heads * head size]: ``run`` runs it as ``attention`` does,
+    ``gemm_splitk_pair_attn`` in the launch of the products behind it."""
+
+    def __init__(self, q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: float, waves: int = 4, **how):
+        """``waves``: on the keys of sixteen heads, in the launch that it may wait for (1 or 4)."""
+        self.waves = waves
+        self.q, self.k_pool, self.v_pool, self.block_table, self.ctx = q, k_pool, v_pool, block_table, ctx
+        self.slopes, self.scale, self.how = slopes, scale, how
+        M, nh, d = q.shape
+        self.out = torch.empty((M, nh * d), dtype=q.dtype, device=q.device)
+
+    def run(self) -> None:
+        attention(self.q, self.k_pool, self.v_pool, self.block_table, self.ctx, self.slopes, self.scale, into=(self.out, self.q.shape[2], 1.0),
+                  **self.how)
+
+    def sync(self, words: int) -> torch.Tensor:
+        """``words`` 32-bit zeros of the step's, which the launch that takes them leaves as it likes: cleared for many launches at a time."""
+        words = (words + 31) // 32 * 32  # (lines of their own)
+        room, at = self.ctx.extras.get("late_sync", (None, 0))
+        if room is None or at + words > room.shape[0]:
+            room, at = torch.zeros((32 * words,), dtype=torch.int32, device=self.q.device), 0
+        self.ctx.extras["late_sync"] = (room, at + words)
+        return room[at:at + words]
+
+
+def late_attention_waves(q: torch.Tensor, k_pool, ctx) -> int:
+    """0, or the waves on a piece's keys with which a decode step's attention waits for the launch of the products behind it
+    (``gemm_splitk_pair_attn``, ``tuning.late_waves``)."""
+    if not (ctx.is_decode and attn_mfma_ok(q) and q.shape[2] == LATE_HEAD and q.shape[0] <= LATE_MOST_ROWS):
+        return 0
+    shape = (ctx.n_seqs, q.shape[1], k_pool.shape[1], q.shape[2], ctx.max_len, getattr(ctx, "mean_len", 0))
+    waves = tuning.late_waves(*shape)
+    if waves and tuning.short_cut(ctx.max_len) is None:
+        tuning.note_decode_launch(*shape, late=True)
+    return waves
+
+
+LATE_HEAD, LATE_MOST_ROWS = 64, 64  # what gemm_splitk_attn.hip is built for
+
+
 def attention(q: torch.Tensor, k_pool, v_pool, block_table, ctx, slopes, scale: float, window: int = 0,
               alibi_exact: bool = False, bias_of: str = "key", bias_scale: Optional[float] = None,
               chunk: int = 0, sink: Optional[torch.Tensor] = None, into=None) -> torch.Tensor:
@@ -1340,6 +1381,47 @@ def gemm_splitk_pair_partial(x1: torch.Tensor, w1: torch.Tensor, x2: torch.Tenso
     part2 = torch.empty((p2, M, N2), dtype=torch.float32, device=x1.device)
     _call("pta_gemm_splitk_pair_bf16", _ptr(part1), _ptr(x1), _ptr(w1), N1, K1, _ptr(part2), _ptr(x2), _ptr(w2), N2, K2,
           M, _stream())
+    return part1, part2
+
+
+def gemm_splitk_pair_attn_ok(x1: torch.Tensor, w1: torch.Tensor, late: LateAttention, w2: torch.Tensor) -> bool:
+    """Whether ``gemm_splitk_pair_attn`` has a launch for these (which ``gemm_partial_pair_ok`` takes, with ``late.out`` as the second input)."""
+    _, nh, d = late.q.shape
+    return bool(load_library().pta_gemm_splitk_pair_attn_ok(w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], x1.shape[0], nh,
+                                                            late.k_pool.shape[1], d))
+
+
+def gemm_splitk_pair_attn(x1: torch.Tensor, w1: torch.Tensor, late: LateAttention, w2: torch.Tensor, owners: int = -1):
+    """``gemm_splitk_pair_partial(x1, w1, late.out, w2)`` with ``late`` run in the same launch.  ``owners``: how many of attention's workgroups
+    the launch begins with (-1: all of them; the others are done by workgroups that wait for them)."""
+    x2, q, ctx = late.out, late.q, late.ctx
+    for name, t in (("x1", x1), ("w1", w1), ("x2", x2), ("w2", w2), ("q", q)):
+        _need(t, name, torch.bfloat16)
+    M, nh, d = q.shape
+    (N1, K1), (N2, K2) = w1.shape, w2.shape
+    if x1.shape != (M, K1) or K2 != nh * d:
+        raise KernelError(f"a pair shares M: x1 {tuple(x1.shape)}, w1 {tuple(w1.shape)}, attention {tuple(q.shape)}, w2 {tuple(w2.shape)}")
+    nkv = late.k_pool.shape[1]
+    _need_pools(late.k_pool, late.v_pool, torch.bfloat16, nkv, d)
+    _need(late.block_table, "block_table", torch.int32)
+    if late.block_table.shape[0] != M:
+        raise KernelError(f"attention of {M} tokens, one a sequence, but the table has {late.block_table.shape[0]} sequences")
+    _need(ctx.cu_tokens, "cu_tokens", torch.int32, (M + 1,))
+    _need(ctx.seq_start, "seq_start", torch.int32, (M,))
+    how = late.how
+    sink = how.get("sink")
+    if sink is not None:
+        _need(sink, "sink", torch.float32, (nh,))
+    bias_scale = how.get("bias_scale")
+    bias = _score_bias_arg(late.slopes, nh, how.get("bias_of", "key"), not how.get("alibi_exact", False), d ** -0.5 if bias_scale is None else bias_scale)
+    tuning.tune_pair_parts(w1, w2)
+    p1, p2 = gemm_splitk_pair_parts(N1, K1, N2, K2, M)
+    part1 = torch.empty((p1, M, N1), dtype=torch.float32, device=q.device)
+    part2 = torch.empty((p2, M, N2), dtype=torch.float32, device=q.device)
+    sync = late.sync((nh // nkv + 15) // 16 * nkv * M)
+    _call("pta_gemm_splitk_pair_attn", _ptr(part1), _ptr(x1), _ptr(w1), N1, K1, _ptr(part2), _ptr(x2), _ptr(w2), N2, K2, M, _ptr(q),
+          _ptr(late.k_pool), _ptr(late.v_pool), _ptr(late.block_table), late.block_table.shape[1], _ptr(ctx.cu_tokens), _ptr(ctx.seq_start), bias,
+          nh, nkv, d, ctypes.c_float(late.scale), _ptr(sink), int(late.waves), _ptr(sync), int(owners), _stream())
     return part1, part2
 
 

@@ -118,6 +118,11 @@ class AttentionMixer(Part):
             fused = projected if projected is not None else self.qkv(x, apply_bias=False)
             q = self.projection_tail(ctx, call).run(fused)
         bias = as_score_bias(self.positions.score_bias(), self.head_dim)
+        waves = ops.late_attention_waves(q, k_pool, ctx) if defer and self.window == 0 else 0
+        if waves:
+            how = {} if bias is None else dict(alibi_exact=not bias.bf16, bias_of=bias.of, bias_scale=bias.scale)
+            late = ops.LateAttention(q, k_pool, v_pool, table, ctx, None if bias is None else bias.slopes, self.scale, waves=waves, **how)
+            return PendingProjection(self.out, late.out, late)
         if bias is None:
             o = ops.attention(q, k_pool, v_pool, table, ctx, None, self.scale, self.window)
         else:

@@ -235,8 +235,16 @@ class PendingProjection:
     its epilogue (``run``), left as partial sums for the next norm (``partial``), or together with the
     other branch's in one launch (``partial_pair``)."""
 
-    def __init__(self, linear: Linear, x: torch.Tensor):
-        self.linear, self.x = linear, x
+    def __init__(self, linear: Linear, x: torch.Tensor, late=None):
+        """``late`` (an ``ops.LateAttention``): what ``x`` is still to be filled by; it runs when ``x`` is asked for."""
+        self.linear, self._x, self.late = linear, x, late
+
+    @property
+    def x(self) -> torch.Tensor:
+        if self.late is not None:
+            late, self.late = self.late, None
+            late.run()
+        return self._x
 
     def run(self, add1=None, add2=None) -> torch.Tensor:
         return self.linear(self.x, add1=add1, add2=add2)
@@ -267,10 +275,14 @@ class PendingProjection:
     def partial_pair(first: "PendingProjection", second: "PendingProjection"):
         """Both as partial sums from one launch, or None where that does not apply."""
         a, b = first, second
-        if not (a.x.dtype == torch.bfloat16 and ops.layernorm_sum_ok(a.linear.out_features)
-                and ops.gemm_partial_pair_ok(a.x, a.linear.weight, b.x, b.linear.weight)):
+        if not (a._x.dtype == torch.bfloat16 and ops.layernorm_sum_ok(a.linear.out_features)
+                and ops.gemm_partial_pair_ok(a._x, a.linear.weight, b._x, b.linear.weight)):
             return None
-        pa, pb = ops.gemm_splitk_pair_partial(a.x, a.linear.weight, b.x, b.linear.weight)
+        if a.late is None and b.late is not None and ops.gemm_splitk_pair_attn_ok(a._x, a.linear.weight, b.late, b.linear.weight):
+            late, b.late = b.late, None
+            pa, pb = ops.gemm_splitk_pair_attn(a._x, a.linear.weight, late, b.linear.weight)
+        else:
+            pa, pb = ops.gemm_splitk_pair_partial(a.x, a.linear.weight, b.x, b.linear.weight)
         return PartialProduct(pa, a.linear.bias), PartialProduct(pb, b.linear.bias)
 
 

@@ -274,6 +274,39 @@ def decode_key(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_le
     return (n, int(n_heads), int(n_kv_heads), int(head_dim), bound, mean)
 
 
+def late_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0) -> int:
+    """0, or the waves (1 or 4) on the keys of sixteen heads with which a decode step's attention goes in the launch of the products behind it,
+    where there is such a launch (``ops.gemm_splitk_pair_attn``).  Whole contexts: a piece, sixteen heads of a KV head, occupies a
+    workgroup, or a wave of one, for as long as its keys take behind the stream of weights, and every workgroup of attention is one less for that
+    stream.  Microseconds a layer against launches apart, one wave / four:
+
+                                        1 sequence       8               16              32              64
+        71 heads on 1 of 64, 60 keys    -3.3 / -3.2   -3.2 / -1.5     -2.5 / -0.5     -1.7 / +0.1     -2.0 / -0.5
+                            150 keys    -4.3 / -4.1   -3.9 / -2.1     -3.5 / -0.8     -3.1 / +0.2     -0.2 / -1.2
+                            900 keys      +4 / -6.4    +52 / -5.1      +50 / -1.2      +32 / -1.8       +8 / -1.4
+                          1,900 keys    +134 / -7.3   +132 / -7.1     +130 / +2.4     +121 / +2.7      +45 / +11.6
+        128 on 8 of 64, 60 keys         -3.2 / -3.2   -2.4 / -1.4     +0.5 / +0.3     -0.2 / -2.6     +0.9 / +3.7
+                       150 keys         -2.6 / +6.4   -0.8 / -1.2     +1.1 / -2.4     +1.6 / -1.4     +2.2 / +1.9
+                       900 keys          +10 / -4.0    +10 / -1.0       +6 / -5.6      +10 / -4.7     +8.5 / +5.4
+                     1,900 keys         +107 / +2.1   +110 / +3.1     +103 / +1.8      +98 / -9.2      +13 / +6.1
+
+    So a wave alone up to ``SHORT_CONTEXT`` where the heads of a KV head fill several pieces (whose waves share its keys), else four; beyond that four
+    waves, up to 2,048 keys where there are few pieces of several a KV head, up to 1,024 where a KV head is one piece.  A cut that was fixed
+    (``set_decode_plan``) goes before the rule."""
+    key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
+    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
+        return 0
+    n, bound = key[0], key[4]
+    groups = (n_heads // n_kv_heads + 15) // 16
+    pieces = n * n_kv_heads * groups
+    if max_len <= SHORT_CONTEXT:
+        return 1 if groups > 1 and pieces <= 320 else 4 if pieces <= 256 else 0
+    cut = _active.decode_plans.get(key)
+    if cut is not None:
+        return 4 if cut[0] == 1 and cut[1] >= max_len and cut[2] == 4 else 0
+    return 4 if (bound <= 2048 and pieces <= 40 if groups > 1 else bound <= 1024 and pieces <= 256) else 0
+
+
 def decode_plan(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0):
     """How a decode launch is cut: (column tiles per wave, keys per workgroup, waves per workgroup); a size that
     covers the context means one workgroup per sequence and head group, which writes the result itself.  The
@@ -342,12 +375,15 @@ def _shared_keys_rule(n: int, n_heads: int, n_kv_heads: int, head_dim: int, boun
 
 
 _decode_keys_seen: set = set()  # what decode launches asked ``decode_plan`` for while timing was on
+_decode_keys_late: set = set()  # of those, where attention went in the launch of the products behind it (``late_waves``)
 
 
-def note_decode_launch(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0) -> None:
+def note_decode_launch(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0, late: bool = False) -> None:
     """While timing is on: remember that a decode launch of this shape ran, for ``CausalLM.tune`` to time its cuts."""
     if may_time():
-        _decode_keys_seen.add(decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len))
+        key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
+        _decode_keys_seen.add(key)
+        (_decode_keys_late.add if late else _decode_keys_late.discard)(key)
 
 
 def take_decode_keys() -> list:
@@ -372,7 +408,8 @@ def decode_plan_candidates(key) -> list:
     most = min(groups, int(lib.pta_attn_decode_max_tiles(d)))
     rule = _decode_plan(n, nh, nkv, d, bound, mean, most) + (1,)
     # what runs where nothing was timed comes first: the caller measures the others against it
-    cuts = [c for c in (_several_waves_rule(*key), _shared_keys_rule(*key), rule) if c is not None]
+    late = (1, bound, 4) if tuple(key) in _decode_keys_late else None
+    cuts = [c for c in dict.fromkeys((late, _several_waves_rule(*key), _shared_keys_rule(*key), rule)) if c is not None]
     want = [(rule[0], rule[1] * 2, 1), (rule[0], rule[1] // 2, 1), (max(1, rule[0] - 1), rule[1], 1),
             (min(most, rule[0] + 1), rule[1], 1)]
     want += [(t, size, w) for t in (1, min(2, most)) for w in (4, 8) for size in (bound, 1024, 512)]
