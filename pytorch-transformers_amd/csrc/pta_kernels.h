@@ -345,6 +345,11 @@ int pta_ssm_scan(float* y, const float* xbc, const void* dt_in, long dt_ld, cons
                  const float* Dp, float* state, long state_ld, float* chunk_state, float* chunk_decay,
                  const int* cu_tokens, const int* seq_slot, int n_seqs, int heads, int P, int N, int G, int chunk,
                  int max_chunks, int dtype, void* stream);
+// conv_silu, ssm_scan and the gated RMS norm (a mean a group of heads) of one token a sequence in one launch (ssm_step.hip); heads of 64
+int pta_ssm_step_ok(int heads, int P, int N, int G, int K);
+int pta_ssm_step(void* out, const void* proj, long ld, const float* conv_w, const float* conv_b, float* tail, long tail_ld,
+                 const float* dt_bias, const float* A_log, const float* D, float* state, long state_ld, const float* norm_w, float offset,
+                 float eps, const int* cu_tokens, const int* seq_slot, int n_seqs, int heads, int N, int G, int K, int dtype, void* stream);
 
 // ---- attention over a cache of latents (attn_latent.hip) ----------------------------------------------------------
 int pta_attn_latent_sizes_ok(int H, int dn, int dr, int R);

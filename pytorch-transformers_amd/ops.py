@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok", "pta_gemm_splitk_pair_attn_ok")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok", "pta_gemm_splitk_pair_attn_ok", "pta_ssm_step_ok")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -1960,6 +1960,39 @@ def ssm_scan(xbc: torch.Tensor, dt: torch.Tensor, dt_bias, a_log, d_skip, state:
               _ptr(state), ctypes.c_long(state_ld), _ptr(chunk_state), _ptr(chunk_decay), _ptr(cu_tokens), _ptr(seq_slot),
               n, heads, head_dim, state_rows, groups, chunk, chunks, dtype_code(dt.dtype), _stream())
     return y
+
+
+def ssm_step_ok(state: torch.Tensor, heads: int, head_dim: int, state_rows: int, groups: int, taps: int, norm_groups: int) -> bool:
+    """Whether ``ssm_step`` has a launch for these sizes and this table of states."""
+    return (norm_groups == groups and state.data_ptr() % 16 == 0 and state.stride(0) % 4 == 0
+            and bool(load_library().pta_ssm_step_ok(int(heads), int(head_dim), int(state_rows), int(groups), int(taps))))
+
+
+def ssm_step(proj: torch.Tensor, conv_w, conv_b, dt_bias, a_log, d_skip, row: torch.Tensor, norm_w, offset: float, eps: float, cu_tokens, seq_slot,
+             heads: int, head_dim: int, state_rows: int, groups: int) -> torch.Tensor:
+    """A decode step of the state-space mixer, one token a sequence: ``conv_silu``, ``ssm_scan`` and the gated ``rmsnorm`` (``groups`` parts of
+    a row) in one launch.  ``proj`` ``[tokens, gate | inputs | B | C | dt]``; ``row`` ``[slots, state | tail of the convolution]`` (32-bit) is
+    moved on.  Returns the normed rows ``[tokens, heads * head_dim]`` in ``proj``'s type."""
+    inner, n = heads * head_dim, seq_slot.numel()
+    C, K = conv_w.shape
+    cut = heads * state_rows * head_dim
+    if C != inner + 2 * groups * state_rows:
+        raise KernelError(f"a convolution of {C} channels for {heads} heads of {head_dim} and {groups} groups of {state_rows} rows")
+    ld = _rows_of(proj, "proj", inner + C + heads)
+    _need(conv_w, "conv_w", torch.float32)
+    if conv_b is not None:
+        _need(conv_b, "conv_b", torch.float32, (C,))
+    for name, t, size in (("dt_bias", dt_bias, heads), ("A_log", a_log, heads), ("D", d_skip, heads), ("norm_w", norm_w, inner)):
+        _need(t, name, torch.float32, (size,))
+    _need(seq_slot, "seq_slot", torch.int32, (n,))
+    _need(cu_tokens, "cu_tokens", torch.int32, (n + 1,))
+    state_ld = _need_state(row, cut + (K - 1) * C)
+    tail = row[:, cut:]
+    out = torch.empty((proj.shape[0], inner), dtype=proj.dtype, device=proj.device)
+    _call("pta_ssm_step", _ptr(out), _ptr(proj), ctypes.c_long(ld), _ptr(conv_w), _ptr(conv_b), _ptr(tail), ctypes.c_long(state_ld), _ptr(dt_bias),
+          _ptr(a_log), _ptr(d_skip), _ptr(row), ctypes.c_long(state_ld), _ptr(norm_w), ctypes.c_float(offset), ctypes.c_float(eps), _ptr(cu_tokens),
+          _ptr(seq_slot), n, heads, state_rows, groups, K, dtype_code(proj.dtype), _stream())
+    return out
 
 
 # ---- attention over a cache of latents ---------------------------------------------------------------------------

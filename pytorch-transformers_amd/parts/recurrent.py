@@ -106,6 +106,10 @@ class StateSpaceMixer(Part):
         row = ctx.cache.state_layer(call.cache_group, call.cache_layer)
         cut = self.heads * self.state_rows * self.head_dim
         proj = self.inp(x)
+        if ctx.is_decode and ops.ssm_step_ok(row, self.heads, self.head_dim, self.state_rows, self.groups, self.taps, self.norm.groups):
+            normed = ops.ssm_step(proj, self.conv_w, self.conv_b, self.dt_bias, self.a_log, self.d_skip, row, self.norm.weight, self.norm.offset,
+                                  self.norm.eps, ctx.cu_tokens, ctx.seq_slot, self.heads, self.head_dim, self.state_rows, self.groups)
+            return self.out(normed, add1=residual)
         gate = proj[:, :self.inner]
         xbc = ops.conv_silu(proj[:, self.inner:self.inner + self.channels], self.conv_w, self.conv_b, row[:, cut:],
                             ctx.cu_tokens, ctx.token_seq, ctx.seq_slot)
