@@ -8,8 +8,8 @@
 //   latent_values    merges a token's ranges and takes the result through the head's value expansion
 //
 // What bounds a layer here is launches and chains of dependent loads, not bytes: 16 heads, R = 512, dr = 64, 8 sequences of 64 to
-// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 26 in three (4.7,
-// 14 and 6.8).
+// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 21 in three (4.7,
+// 9.3 and 6.8).
 #include "attn_latent_token.h"
 
 typedef __bf16 ld_bf16x8 __attribute__((ext_vector_type(8)));
@@ -109,8 +109,8 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
                 if (j < per) pre[j] = page[256 * j];
         };
         // Queries, scaled and rounded, once for the four waves: all asked for before the page, whose place the block table
-        // has yet to tell, and in LDS while it comes (a piece after the other behind the page: 15.0 us where this takes 13.9, 16 heads, R = 512, 8
-        // sequences of 64 to 700 keys)
+        // has yet to tell, and in LDS while it comes (a piece after the other behind the page: 1.1 us more, 16 heads, R = 512, 8 sequences of
+        // 64 to 700 keys)
         float4 lo[LP_QUERIES], hi[LP_QUERIES];
         {
             int c = row0, e = at0;
@@ -154,13 +154,18 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
             ld_f32x4 sc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
             const bf16_t* kr = Ks + (16 * wave + r16) * P + g * 8;
             const bf16_t* qr = Qs + r16 * P + g * 8;
-#pragma unroll 4
-            for (int c = 0; c < D / 32; ++c) {
+            auto step = [&](ld_f32x4& sum, int c) {
                 LdFrag k, q;
                 k.u = *(const uint4*)(kr + 32 * c);
                 q.u = *(const uint4*)(qr + 32 * c);
-                sc[c & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, q.v, sc[c & 1], 0, 0, 0);
-            }
+                sum = __builtin_amdgcn_mfma_f32_16x16x32_bf16(k.v, q.v, sum, 0, 0, 0);
+            };
+            // The even pieces' sum and the odd ones', each by its own name.  Told apart by an index they kept the loop one step long, and a step took
+            // 670 cycles (the sum moved in and out of place, a trip to LDS and back): 12,000 of the launch's 25,700 went there, and 1,600 go now (18 pieces).
+            // With latent_values, 16 heads, R = 512, dr = 64: 8 sequences of 64 to 700 keys 17.8 -> 13.1 us, 2 of 1,900 19.4 -> 14.7, 16 of 4,000 48.0 -> 29.7.
+#pragma unroll 3
+            for (int c = 0; c + 1 < D / 32; c += 2) step(sc[0], c), step(sc[1], c + 1);
+            if (D / 32 % 2) step(sc[0], D / 32 - 1);
             float p[4], top = -INFINITY;
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
