@@ -135,6 +135,7 @@ extern "C" int pta_attn_mfma(void* out, const void* q, const void* k_pool, const
     PTA_REQUIRE(n_splits == 1 || (split_size > 0 && split_size % 64 == 0 && po && pm && pl),
                 "attn_mfma: splitting needs a split size that is a multiple of 64 and buffers for partial results");
     PTA_REQUIRE((long)n_seqs * n_splits <= 65535 && nkv <= 65535, "attn_mfma: too many sequences x splits for one launch");
+    PTA_REQUIRE(nh / nkv <= 65535 && bt_stride >= 0 && bt_stride < 1 << 30, "attn_mfma: %d heads on a KV head, rows of %d pages: too many", nh / nkv, bt_stride);
     PTA_REQUIRE(((uintptr_t)q % 16) == 0 && ((uintptr_t)k_pool % 16) == 0 && ((uintptr_t)v_pool % 16) == 0 &&
                     ((uintptr_t)out % 8) == 0, "attn_mfma: pointers must be 16-byte aligned");
     const PtaHeadRows rows = pta_head_rows_of(head_rows, nh, d);

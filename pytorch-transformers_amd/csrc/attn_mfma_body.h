@@ -1,15 +1,19 @@
 // What a workgroup of the attention kernel does (attn_mfma_impl.h), as text, because a launch of another kind carries it too
-// (gemm_splitk_attn.hip) and the compiler did not survive it as a function at every head size.  Which workgroup it is stands in ATTN_X, ATTN_Y and
-// ATTN_Z of ATTN_NX by .. by ATTN_NZ; ATTN_INSIDE: it is part of a launch of another kind.
+// (gemm_splitk_attn.hip) and the compiler did not survive it as a function at every head size.  Which workgroup it is stands in ATTN_X (of ATTN_NX),
+// ATTN_Y and ATTN_Z; ATTN_INSIDE: it is part of a launch of another kind.
     constexpr int D = DT * 16;
-    const int window = WIN ? window_arg : 0;
-    const int chunk = WIN ? chunk_arg : 0;  // blocks of positions that a token does not see out of (0: none)
+    int window = 0, chunk = 0;  // chunk: blocks of positions that a token does not see out of (0: none)
+    if constexpr (WIN) {
+        ATTN_LATE(more);
+        window = more.window_arg, chunk = more.chunk_arg;
+    }
     // the lowest key that a token at position t sees: never decreasing in t
     auto lowest_key = [&](int t) {
         int lo = window > 0 ? max(0, t - window + 1) : 0;
         if (chunk > 0) lo = max(lo, t / chunk * chunk);
         return lo;
     };
+    auto token_of = [&](int col) { return KS > 1 || ATTN_INSIDE ? 0 : col / g; };  // (launches for one token a sequence)
     constexpr int DS = (DT + 1) / 2;   // 32-wide steps over the head dimension
     constexpr int CHUNKS = D / 8;      // 16-byte chunks in a row of d elements
     static_assert(KS == 1 || W == 1, "waves either share key blocks or divide them");
@@ -20,51 +24,55 @@
     // start first, and the last ones, which are short or empty for most sequences, fill the launch's end.  (Sequence-
     // major, 32 sequences of 16,405 keys in ranges of 1,024 left two whole ranges to start when the first ones ended:
     // 45.8 us against 30.3 us at 16,384 keys.)
-    const int n_seqs_z = ATTN_NZ / n_splits;
-    const int seq = ATTN_Z % n_seqs_z, split = ATTN_Z / n_seqs_z;
-    const int kvh = ATTN_Y, g = nh / nkv;
+    int seq = ATTN_Z, split = 0, range0 = 0, range1 = 0;
+    if (many_ranges) {
+        ATTN_LATE(more);
+        seq = ATTN_Z % more.n_seqs, split = ATTN_Z / more.n_seqs, range0 = split * more.split_size, range1 = range0 + more.split_size;
+    }
+    const int kvh = ATTN_Y;
     // The pages of a lone wave's first two blocks are looked up beside the sequence's length, not behind it: one round trip less in
     // a decode step's chain of them (an entry past the sequence's pages is read but not used).
     const int* bt = block_table + (long)seq * bt_stride;
-    const int first_key = (n_splits > 1 ? split * split_size : 0) + 32 * kw;
+    const int first_key = range0 + 32 * kw;
     int first_page = 0, next_page = 0;
     if constexpr (W == 1 && !WIN) {
         first_page = bt[min(first_key >> 6, bt_stride - 1)];
         next_page = bt[min((first_key + 32 * KS) >> 6, bt_stride - 1)];
     }
-    const int t0 = cu_tokens[seq], n_new = cu_tokens[seq + 1] - t0, start = seq_start[seq];
+    int t0 = cu_tokens[seq], t1 = cu_tokens[seq + 1], start = seq_start[seq];
     if constexpr (W == 1 && !WIN) {
         // (behind another part of a launch, which writes memory, the entries come by vector loads)
         if constexpr (ATTN_INSIDE) first_page = __builtin_amdgcn_readfirstlane(first_page), next_page = __builtin_amdgcn_readfirstlane(next_page);
-        else asm volatile("" : "+s"(first_page), "+s"(next_page));
+        else asm volatile("" : "+s"(first_page), "+s"(next_page), "+s"(t0), "+s"(t1), "+s"(start));
     }
+    const int n_new = t1 - t0;
     const int ncols = n_new * g, n_groups = (ncols + 16 * CT * W - 1) / (16 * CT * W);
     // Column groups are handed out last first: late tokens see the most keys, and the longest work should
     // start first so that the launch ends evenly.  A paired launch has half the workgroups, and each takes a
     // late group and then the early group that mirrors it: under the causal mask the two together see as
     // many keys as any other pair, so a launch whose workgroups are all resident at once ends evenly too.
     for (int pass = 0; pass <= paired; ++pass) {
-    int group = (int)(ATTN_NX - 1 - ATTN_X);
+    int group = (W > 1 ? (int)ATTN_NX : n_groups) - 1 - (int)ATTN_X;  // (a sequence with fewer groups than the launch has room for: none below 0)
     if (paired) {
         const int late = n_groups - 1 - (int)ATTN_X, early = (int)ATTN_X;
         if (late < early || (pass == 1 && late == early)) return;
         group = pass == 0 ? late : early;
     }
     const int wg_col0 = group * (16 * CT * W);
-    if (wg_col0 >= ncols) return;
+    if (wg_col0 >= ncols || wg_col0 < 0) return;
     const int col0 = wg_col0 + wave * (16 * CT);
     const bool active = col0 < ncols;  // W > 1: a wave past the last column still loads and waits with the others
     const int last_col = min(ncols, col0 + 16 * CT) - 1;
-    const int max_qpos = start + last_col / g;
+    const int max_qpos = start + token_of(last_col);
     const int kv_len = start + n_new;
     // with a window a column at position t sees keys t - window + 1 .. t; this wave starts at the block of
     // the first key its first column sees (earlier pages may be gone), and at its range's start if split
-    const int lo_first = WIN ? lowest_key(start + col0 / g) : 0;   // lowest key any column sees
+    const int lo_first = WIN ? lowest_key(start + token_of(col0)) : 0;   // lowest key any column sees
     const int lo_last = WIN ? lowest_key(max_qpos) : 0;            // lowest key the last column sees
-    const int k_begin = max(n_splits > 1 ? split * split_size : 0, lo_first & ~31);
-    const int k_end = !active ? 0 : n_splits > 1 ? min(max_qpos + 1, split * split_size + split_size) : max_qpos + 1;
+    const int k_begin = WIN ? max(range0, lo_first & ~31) : range0;
+    const int k_end = !active ? 0 : many_ranges ? min(max_qpos + 1, range1) : max_qpos + 1;
     // below this key index no column of this wave masks anything (columns are ordered by token)
-    const int min_lim = min(start + col0 / g + 1, k_end);
+    const int min_lim = min(start + token_of(col0) + 1, k_end);
     const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
     // in the last 32-wide step of an odd number of 16-wide tiles, the upper half of the lanes has no data
     const uint32_t tail_keep = (DT % 2 == 1 && (DS - 1) * 4 + gq >= CHUNKS) ? 0u : 0xffffffffu;
@@ -76,17 +84,16 @@
     for (int ct = 0; ct < CT; ++ct) {
         const int col = col0 + ct * 16 + c;
         const int colc = min(col, ncols - 1);
-        const int t = colc / g;
+        const int t = token_of(colc);
         tok[ct] = t0 + t;
-        head[ct] = kvh * g + colc % g;
+        head[ct] = kvh * g + colc - t * g;
         qpos[ct] = col < ncols ? start + t : -1;  // -1: every key is masked for a column that does not exist
-        slope[ct] = slopes ? slopes[head[ct]] : 0.f;
         const bf16_t* qp = q + ((long)tok[ct] * nh + head[ct]) * D;
 #pragma unroll
         for (int ds = 0; ds < DS; ++ds) {
             const int chunk = ds * 4 + gq;
             qf[ct][ds].u = *reinterpret_cast<const uint4*>(qp + min(chunk, CHUNKS - 1) * 8);
-            if (chunk >= CHUNKS) qf[ct][ds].u = zero4;
+            if (W > 1 && chunk >= CHUNKS) qf[ct][ds].u = zero4;
         }
     }
 
@@ -109,11 +116,30 @@
 
     // AL says at compile time whether there is ALiBi (0: none, 1: there is; 2: whatever the launch brings), so
     // that the kernels for prompts, which are bound by their instruction stream, branch on nothing in it.
-    const bool has_alibi = AL == 2 ? slopes != nullptr : AL == 1;
     // Scores are kept in units of log 2 (the scale carries log2 e), so that the exponential is the hardware's
     // exp2.  Without ALiBi the products are left unscaled, and the scale rides in the one multiply-add in front
     // of the exponential: s_mul is what a settled score is still to be multiplied by (positive).
-    const float s_mul = has_alibi ? 1.0f : scale;
+    // What none of a lone wave's first loads of keys hangs on is read behind them.
+    const float *slopes = nullptr, *sink = nullptr;
+    float scale = 0.f, alibi_mul = 0.f, s_mul = 1.f;
+    int bias_mode = 0, ranges = 1;
+    bool has_alibi = AL == 1;
+    bf16_t* out = nullptr;
+    float *po = nullptr, *pm = nullptr, *pl = nullptr;
+    PtaHeadRows rows;
+    auto read_more = [&]() {
+        ATTN_LATE(more);
+        slopes = more.slopes, sink = more.sink, scale = more.scale, alibi_mul = more.alibi_mul, bias_mode = more.bias_mode, ranges = more.ranges;
+        out = more.out, po = more.po, pm = more.pm, pl = more.pl;
+        rows.ld = more.rows.ld, rows.head = more.rows.head, rows.keep = more.rows.keep, rows.mult = more.rows.mult;
+        if (AL == 2) has_alibi = slopes != nullptr;
+        s_mul = has_alibi ? 1.0f : scale;
+        const float* of = slopes ? slopes : reinterpret_cast<const float*>(q);  // (a launch without slopes reads something and leaves it)
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) slope[ct] = of[head[ct]];
+    };
+    constexpr bool FIRST = W > 1 || WIN || CT > 2;  // (of several tiles the registers run short, and these words would be kept in them all the while)
+    if constexpr (FIRST) read_more();
 
     // The work on a block of 32 keys, in the four pieces that the loops below put together:
     // the products S^T = K . Q^T of the block, raw
@@ -127,9 +153,13 @@
 #pragma unroll
             for (int ct = 0; ct < CT; ++ct) {
                 f32x4_t acc = f32x4_t{0.f, 0.f, 0.f, 0.f};
+                AFrag q_last = qf[ct][DS - 1];
+                if (W == 1 && DT % 2 == 1) {  // (where q is loaded, a lone wave would wait for it before it asks for the first keys)
+                    q_last.u.x &= tail_keep; q_last.u.y &= tail_keep; q_last.u.z &= tail_keep; q_last.u.w &= tail_keep;
+                }
 #pragma unroll
                 for (int ds = 0; ds < DS; ++ds)
-                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ds == DS - 1 ? k_last.v : k[tt][ds].v, qf[ct][ds].v, acc, 0, 0, 0);
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ds == DS - 1 ? k_last.v : k[tt][ds].v, ds == DS - 1 ? q_last.v : qf[ct][ds].v, acc, 0, 0, 0);
                 sacc[tt][ct] = acc;
             }
         }
@@ -274,6 +304,7 @@
         };
         if (n_mine > 0) {
             load(b0, 0);
+            if constexpr (!FIRST) read_more();
             int j = 0;
             for (; j + 2 < n_mine; j += 2) {
                 load(b1, j + 1);
@@ -288,7 +319,7 @@
                 ++j;
             }
             use(b0, j);
-        }
+        } else if constexpr (!FIRST) read_more();
     } else {
         // The workgroup's waves walk the keys of its last column together, a stage of SK keys (one or two
         // blocks) between barriers.  A stage goes global memory -> registers (one stage ahead) -> one of two
@@ -306,10 +337,10 @@
         const int tid = threadIdx.x;
         const int wg_last_col = min(ncols, wg_col0 + 16 * CT * W) - 1;
         // (a launch that cuts the keys into ranges walks its own range only)
-        const int k_end_wg = n_splits > 1 ? min(start + wg_last_col / g + 1, split * split_size + split_size)
+        const int k_end_wg = many_ranges ? min(start + wg_last_col / g + 1, range1)
                                           : start + wg_last_col / g + 1;
         const int k_begin_wg = max(WIN ? lowest_key(start + wg_col0 / g) & ~(SK - 1) : 0,
-                                   n_splits > 1 ? split * split_size : 0);
+                                   range0);
         const int ks_last = (kv_len - 1) & ~(SK - 1);  // the last stage that has a page
         static_assert(PER <= 2, "a thread moves at most two pieces of keys and two of values per stage");
         static_assert(PTA_PAGE % SK == 0, "a stage lies in one page");
@@ -409,25 +440,28 @@
         __syncthreads();
 #pragma unroll
         for (int ct = 0; ct < CT; ++ct) {
+            float mx = -INFINITY, l = 0.f, wgt[KS];
+#pragma unroll
+            for (int w = 0; w < KS; ++w) wgt[w] = sm[(w * CT + ct) * 16 + c];
+#pragma unroll
+            for (int w = 0; w < KS; ++w) mx = fmaxf(mx, wgt[w]);
+#pragma unroll
+            for (int w = 0; w < KS; ++w) {
+                wgt[w] = wgt[w] == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(wgt[w] - mx);
+                l += wgt[w] * sl[(w * CT + ct) * 16 + c];
+            }
+            if (sink && !many_ranges) l += __builtin_amdgcn_exp2f(sink[head[ct]] * PTA_LOG2E - mx);
 #pragma unroll
             for (int dt = 0; dt < DT; ++dt) {
                 if ((ct * DT + dt) % KS != kw || qpos[ct] < 0) continue;
-                float mx = -INFINITY;
-#pragma unroll
-                for (int w = 0; w < KS; ++w) mx = fmaxf(mx, sm[(w * CT + ct) * 16 + c]);
-                float l = 0.f;
                 float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
 #pragma unroll
                 for (int w = 0; w < KS; ++w) {
-                    const float mw = sm[(w * CT + ct) * 16 + c];
-                    const float wgt = mw == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mw - mx);
                     const float4 o = so[((w * CT + ct) * DT + dt) * 64 + lane];
-                    l += wgt * sl[(w * CT + ct) * 16 + c];
-                    acc.x += wgt * o.x; acc.y += wgt * o.y; acc.z += wgt * o.z; acc.w += wgt * o.w;
+                    acc.x += wgt[w] * o.x; acc.y += wgt[w] * o.y; acc.z += wgt[w] * o.z; acc.w += wgt[w] * o.w;
                 }
                 const long row = (long)tok[ct] * nh + head[ct];
-                if (n_splits == 1) {
-                    if (sink) l += __builtin_amdgcn_exp2f(sink[head[ct]] * PTA_LOG2E - mx);
+                if (!many_ranges) {
                     const float inv = rows.mult / l;
                     uint2 w2;
                     w2.x = pack_bf16(acc.x * inv, acc.y * inv);
@@ -435,10 +469,10 @@
                     if (dt * 16 + gq * 4 < rows.keep)
                         store4(out + (long)tok[ct] * rows.ld + (long)head[ct] * rows.head + dt * 16 + gq * 4, w2);
                 } else {
-                    *reinterpret_cast<float4*>(po + (row * n_splits + split) * D + dt * 16 + gq * 4) = acc;
+                    *reinterpret_cast<float4*>(po + (row * ranges + split) * D + dt * 16 + gq * 4) = acc;
                     if (dt == 0 && gq == 0) {
-                        pm[row * n_splits + split] = mx;
-                        pl[row * n_splits + split] = l;
+                        pm[row * ranges + split] = mx;
+                        pl[row * ranges + split] = l;
                     }
                 }
             }
@@ -449,7 +483,7 @@
         float l = lacc[ct][0];
         if (qpos[ct] < 0) continue;
         const long row = (long)tok[ct] * nh + head[ct];
-        if (n_splits == 1) {
+        if (!many_ranges) {
             if (sink) l += __builtin_amdgcn_exp2f(sink[head[ct]] * PTA_LOG2E - m_run[ct]);
             const float inv = rows.mult / l;
             bf16_t* o = out + (long)tok[ct] * rows.ld + (long)head[ct] * rows.head;
@@ -465,15 +499,15 @@
             // does not read past the last range that has one.  A range before a window is followed by ranges
             // that count, so it is read with weight zero and must hold numbers: the (zero) sums are written.
             if (k_begin < k_end || WIN) {
-                float* o = po + (row * n_splits + split) * D;
+                float* o = po + (row * ranges + split) * D;
 #pragma unroll
                 for (int dt = 0; dt < DT; ++dt)
                     *reinterpret_cast<float4*>(o + dt * 16 + gq * 4) =
                         make_float4(oacc[dt][ct][0], oacc[dt][ct][1], oacc[dt][ct][2], oacc[dt][ct][3]);
             }
             if (gq == 0) {
-                pm[row * n_splits + split] = m_run[ct];
-                pl[row * n_splits + split] = l;
+                pm[row * ranges + split] = m_run[ct];
+                pl[row * ranges + split] = l;
             }
         }
     }

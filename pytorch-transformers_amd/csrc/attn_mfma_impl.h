@@ -34,6 +34,7 @@
 #include "pta_kernels.h"
 #include "score_bias.h"
 
+#include <stddef.h>
 #include <stdlib.h>
 
 #include <algorithm>
@@ -98,6 +99,34 @@ __device__ __forceinline__ void load_block(KvBlock<DT>& b, int kb, long page,
         b.v[dt].u = *reinterpret_cast<const uint4*>(vpage + (long)(dt * 16 + c) * PTA_PAGE + in_page + gq * 8);
 }
 
+// what the kernel looks at later: read where it is used
+struct AttnMore {
+    int n_seqs, ranges, split_size, bias_mode, window_arg, chunk_arg;
+    float scale, alibi_mul;
+    const float* slopes;
+    bf16_t* out;
+    float *po, *pm, *pl;
+    const float* sink;
+    PtaHeadRows rows;
+};
+
+// A launch's arguments, as the kernel takes them.  What comes first and packed is in registers when a workgroup starts, fourteen words of it: what keys
+// and queries are found by.  The others are a load away, which over cold caches takes 0.7 us, and the compiler moves such loads to the front, where the
+// first others that are waited for (the block table's, the lengths') are then waited for with them.  So the kernel reads them from where they lie, where it says so.
+// With all in its order and asked for at the front, 5 sequences of 40 to 325 keys, 13 heads of 80, took 8.6 us a launch in a step, and take 7.5.
+struct AttnKernelArgs {
+    const int *block_table, *cu_tokens, *seq_start;
+    const bf16_t *k_pool, *v_pool, *q;
+    uint32_t heads, table;  // heads of a KV head << 16 | KV heads; pages in a row of the table, and in the two highest bits whether there are ranges and `paired`
+    AttnMore more;
+};
+typedef const __attribute__((address_space(4))) AttnMore& AttnLate;
+__device__ __forceinline__ AttnLate attn_late() {
+    const __attribute__((address_space(4))) char* at = (const __attribute__((address_space(4))) char*)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(at));
+    return *(const __attribute__((address_space(4))) AttnMore*)(at + offsetof(AttnKernelArgs, more));
+}
+
 // W = 1: a workgroup is one wave, which loads its keys and values straight from global memory.
 // W > 1 (prompts; one token per sequence with many heads on a KV head): W waves with neighbouring column groups
 // walk the keys together and share every block through LDS, so that a block crosses the vector memory path once
@@ -109,25 +138,25 @@ __device__ __forceinline__ void load_block(KvBlock<DT>& b, int kb, long page,
 // OCC: waves that a SIMD is to hold at least (the registers a wave may use follow from it; 1: as many as it likes).
 template <int DT, int CT, int W, bool WIN, int KS = 1, int AL = 2, int OCC = 1>
 __global__ __launch_bounds__(64 * W * KS, OCC) void attn_mfma_kernel(
-    bf16_t* __restrict__ out, float* __restrict__ po, float* __restrict__ pm, float* __restrict__ pl,
-    const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pool, const bf16_t* __restrict__ v_pool,
-    const int* __restrict__ block_table, int bt_stride, const int* __restrict__ cu_tokens,
-    const int* __restrict__ seq_start, const float* __restrict__ slopes, int bias_mode, int nh, int nkv, float scale,
-    float alibi_mul,
-    int split_size, int n_splits, int window_arg, int chunk_arg, int paired, const float* __restrict__ sink, PtaHeadRows rows) {
+    const int* __restrict__ block_table, const int* __restrict__ cu_tokens, const int* __restrict__ seq_start, const bf16_t* __restrict__ k_pool,
+    const bf16_t* __restrict__ v_pool, const bf16_t* __restrict__ q, uint32_t heads, uint32_t table,
+    const AttnMore) {  // AttnKernelArgs
+    const int g = heads >> 16, nkv = heads & 0xffff, nh = g * nkv, bt_stride = table & 0x3fffffff;
+    const bool many_ranges = table >> 31;
+    const int paired = KS > 1 ? 0 : table >> 30 & 1;
 #define ATTN_X blockIdx.x
 #define ATTN_Y blockIdx.y
 #define ATTN_Z blockIdx.z
 #define ATTN_NX gridDim.x
-#define ATTN_NZ gridDim.z
 #define ATTN_INSIDE 0
+#define ATTN_LATE(more) AttnLate more = attn_late()
 #include "attn_mfma_body.h"
 #undef ATTN_X
 #undef ATTN_Y
 #undef ATTN_Z
 #undef ATTN_NX
-#undef ATTN_NZ
 #undef ATTN_INSIDE
+#undef ATTN_LATE
 }
 
 struct AttnLaunch {
@@ -168,9 +197,10 @@ static void launch_attn(const AttnLaunch& a) {
             told[dev] = true;
         }
     }
-    hipLaunchKernelGGL(kern, grid, dim3(64 * W * KS), lds, a.s, a.out, a.po, a.pm, a.pl, a.q, a.k_pool, a.v_pool,
-                       a.block_table, a.bt_stride, a.cu_tokens, a.seq_start, a.slopes, a.bias_mode, a.nh, a.nkv,
-                       a.scale * PTA_LOG2E, PTA_LOG2E * a.bias_scale, a.split_size, a.n_splits, a.window, a.chunk, paired, a.sink, a.rows);
+    hipLaunchKernelGGL(kern, grid, dim3(64 * W * KS), lds, a.s, a.block_table, a.cu_tokens, a.seq_start, a.k_pool, a.v_pool, a.q,
+                       (uint32_t)g << 16 | (uint32_t)a.nkv, (uint32_t)a.bt_stride | (a.n_splits > 1 ? 1u << 31 : 0u) | (uint32_t)paired << 30,
+                       AttnMore{a.n_seqs, a.n_splits, a.split_size, a.bias_mode, a.window, a.chunk, a.scale * PTA_LOG2E, PTA_LOG2E * a.bias_scale, a.slopes,
+                                a.out, a.po, a.pm, a.pl, a.sink, a.rows});
 }
 
 // column tiles (of sixteen query heads of one KV head) that one wave of a decode launch holds at most:

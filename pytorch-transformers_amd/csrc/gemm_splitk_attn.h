@@ -10,16 +10,10 @@
 
 // attn_mfma_kernel's arguments for one token a sequence and whole contexts
 struct AttnArgs {
-    bf16_t* out;
     const bf16_t *q, *k_pool, *v_pool;
-    const int* block_table;
-    int bt_stride;
-    const int *cu_tokens, *seq_start;
-    const float* slopes;
-    int bias_mode, nh, nkv;
-    float scale, alibi_mul;
-    const float* sink;
-    PtaHeadRows rows;
+    const int *block_table, *cu_tokens, *seq_start;
+    int bt_stride, nh, nkv;
+    AttnMore more;
 };
 
 struct AttnRide {

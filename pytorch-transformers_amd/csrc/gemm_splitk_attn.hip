@@ -48,22 +48,18 @@ struct RideGate {
 
 // sixteen heads of a KV head of a sequence
 template <int DT, int CT, int W, bool WIN, int KS, int AL>
-__device__ __forceinline__ void attend_to(const AttnArgs& a, int n_seqs, int place_x, int place_y, int place_z, int groups) {
-    bf16_t* const out = a.out;
-    float *const po = nullptr, *const pm = nullptr, *const pl = nullptr;
+__device__ __forceinline__ void attend_to(const AttnArgs& a, int place_x, int place_y, int place_z, int groups) {
     const bf16_t *const q = a.q, *const k_pool = a.k_pool, *const v_pool = a.v_pool;
     const int *const block_table = a.block_table, *const cu_tokens = a.cu_tokens, *const seq_start = a.seq_start;
-    const float *const slopes = a.slopes, *const sink = a.sink;
-    const int bt_stride = a.bt_stride, bias_mode = a.bias_mode, nh = a.nh, nkv = a.nkv;
-    const float scale = a.scale, alibi_mul = a.alibi_mul;
-    constexpr int split_size = 0, n_splits = 1, window_arg = 0, chunk_arg = 0, paired = 0;
-    const PtaHeadRows rows = a.rows;
+    const int bt_stride = a.bt_stride, nh = a.nh, nkv = a.nkv, g = nh / nkv;
+    constexpr int paired = 0;
+    constexpr bool many_ranges = false;
 #define ATTN_X place_x
 #define ATTN_Y place_y
 #define ATTN_Z place_z
 #define ATTN_NX groups
-#define ATTN_NZ n_seqs
 #define ATTN_INSIDE 1
+#define ATTN_LATE(more) const AttnMore& more = a.more
 #include "attn_mfma_body.h"
 }
 
@@ -72,7 +68,7 @@ template <int KS>
 __device__ __forceinline__ void attend(const AttnRide& ride, int t) {
     const int piece = KS > 1 ? t : t * RIDE_WAVES + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), rest = piece / ride.groups;
     if (rest < ride.attn.nkv * ride.n_seqs)
-        attend_to<RIDE_HEAD, 1, 1, false, KS, 2>(ride.attn, ride.n_seqs, piece % ride.groups, rest % ride.attn.nkv, rest / ride.attn.nkv, ride.groups);
+        attend_to<RIDE_HEAD, 1, 1, false, KS, 2>(ride.attn, piece % ride.groups, rest % ride.attn.nkv, rest / ride.attn.nkv, ride.groups);
     wait_loads<0>();  // stores, too, are counted: this wave's have arrived
     __syncthreads();
     if (threadIdx.x == 0) __hip_atomic_store(ride.sync + t, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

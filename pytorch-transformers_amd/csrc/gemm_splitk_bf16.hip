@@ -601,9 +601,9 @@ extern "C" int pta_gemm_splitk_pair_attn(float* part1, const void* x1, const voi
     const SplitkProblem a = make_problem(nullptr, part1, x1, W1, nullptr, nullptr, nullptr, N1, K1, 0, 0, rt, p1, 0);
     const SplitkProblem b = make_problem(nullptr, part2, x2, W2, nullptr, nullptr, nullptr, N2, K2, 0, 0, rt, p2, 0);
     AttnRide ride{};
-    ride.attn = AttnArgs{(bf16_t*)x2, (const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_table, bt_stride, cu_tokens, seq_start,
-                         slopes, bias_mode, nh, nkv, scale * PTA_LOG2E, slopes ? PTA_LOG2E * score_bias->scale : 0.f, sink,
-                         pta_head_rows_of(nullptr, nh, d)};
+    ride.attn = AttnArgs{(const bf16_t*)q, (const bf16_t*)k_pool, (const bf16_t*)v_pool, block_table, cu_tokens, seq_start, bt_stride, nh, nkv,
+                         AttnMore{M, 1, 0, bias_mode, 0, 0, scale * PTA_LOG2E, slopes ? PTA_LOG2E * score_bias->scale : 0.f, slopes, (bf16_t*)x2,
+                                  nullptr, nullptr, nullptr, sink, pta_head_rows_of(nullptr, nh, d)}};
     ride.groups = (nh / nkv + 15) / 16;
     ride.n_seqs = M;
     const int pieces = ride.groups * nkv * M;
