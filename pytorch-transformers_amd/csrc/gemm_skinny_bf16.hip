@@ -126,6 +126,27 @@ struct Share {
     Share(int items, int groups) : each(groups > 0 ? items / groups : 0), over(groups > 0 ? items % groups : 0) {}
     __device__ __forceinline__ int begin(int j) const { return j * each + min(j, over); }
     __device__ __forceinline__ int end(int j) const { return begin(j) + each + (j < over ? 1 : 0); }
+    // in a word: up to 63 items a group, and fewer groups than a launch may have threads for
+    __host__ __device__ __forceinline__ uint32_t packed() const { return (uint32_t)each << 26 | (uint32_t)over; }
+    static __device__ __forceinline__ Share of(uint32_t word) {
+        Share s;
+        s.each = word >> 26, s.over = word & 0x3ffffff;
+        return s;
+    }
+};
+
+// The kernels here take what their loads of W and x are found by first, in the fourteen words that are in registers when a workgroup starts: the
+// arguments behind them are a load away, 0.7 us over cold caches, and what is asked for at the front the first loads wait for.  (With the problem's struct
+// first, 24 layers of four such launches, 1,040 wide, 24 steps of 5 rows: 21.8 ms, this way 21.0: 0.35 us a launch.)  How a workgroup walks, in a word: its waves, a head's elements (with a QkvTail; the sign: its pairs are
+// those that lie half a head apart), and where in K it starts.
+struct Walk {
+    int waves, d, rot_stride;
+    bool plain;
+    static uint32_t packed(int waves, int rot_stride, int d = 0, bool plain = false) {
+        return (uint32_t)waves | (uint32_t)d << 4 | (plain ? 1u << 15 : 0u) | (uint32_t)rot_stride << 16;
+    }
+    __device__ __forceinline__ Walk(uint32_t word)
+        : waves(word & 15), d(word >> 4 & 0x7ff), rot_stride(word >> 16), plain((word >> 15 & 1) != 0) {}
 };
 
 // where a workgroup starts in K, for rows of W a power of two long (gemm_skinny_kernel)
@@ -169,32 +190,29 @@ __device__ __forceinline__ void store_feature(OutT* y, const float* bias, int ac
 // half-split pairs, or no rotation: pair p is elements p and p + d/2, and four pairs in a row are stored as eight
 // bytes; TAIL 2: any rotation that qkv_tail_pair_elements describes, stored element by element).
 template <int MT, int RT, int U, typename OutT, int TAIL = 0, int D = 0>
-__global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, SkinnyProblem pb, int M, int K,
-                                                          int rot_stride, QkvTail tail) {
+__global__ __launch_bounds__(512) void gemm_skinny_kernel(const bf16_t* __restrict__ xa, const bf16_t* __restrict__ Wa, const bf16_t* __restrict__ xb,
+                                                          const bf16_t* __restrict__ Wb, int M, int K, int blocks_a, uint32_t share_a,
+                                                          uint32_t share_b, uint32_t how, SkinnyProblem pa, SkinnyProblem pb, QkvTail tail) {
     static_assert(!TAIL || (RT == 2 && MT == 1 && sizeof(OutT) == 2), "the query_key_value tail: two row tiles, sixteen rows of x");
     static_assert(D == 0 || MT == 1, "through LDS: sixteen rows of x");
     // the waves' sums, [RT][MT][64] each; through LDS they take the place of the waves' rings
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];
     constexpr int WAVE = D == 0 ? RT * MT * 64 : RowStream<RT, D == 0 ? 1 : D>::RING / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const Walk walk(how);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = walk.waves, head = walk.d;
     const int r = lane & 15;
-    const bool second = (int)blockIdx.x >= pa.blocks;
-    OutT* __restrict__ y = (OutT*)(second ? pb.y : pa.y);
-    const bf16_t* __restrict__ x = second ? pb.x : pa.x;
-    const bf16_t* __restrict__ W = second ? pb.W : pa.W;
-    const float* __restrict__ bias = second ? pb.bias : pa.bias;
-    const bf16_t* __restrict__ add1 = second ? pb.add1 : pa.add1;
-    const bf16_t* __restrict__ add2 = second ? pb.add2 : pa.add2;
-    const int N = second ? pb.N : pa.N, act = second ? pb.act : pa.act;
+    const bool second = (int)blockIdx.x >= blocks_a;
+    const bf16_t* __restrict__ x = second ? xb : xa;
+    const bf16_t* __restrict__ W = second ? Wb : Wa;
     // the workgroups of a product share its rows evenly: this one has rows n0 .. n1 - 1, at most 16 * RT
-    const int j = (int)blockIdx.x - (second ? pa.blocks : 0);
-    const Share mine = second ? pb.rows : pa.rows;
+    const int j = (int)blockIdx.x - (second ? blocks_a : 0);
+    const Share mine = Share::of(second ? share_b : share_a);
     const int n0 = mine.begin(j), n1 = mine.end(j);
     const bool tailed = TAIL && !second;
     // with the tail: workgroup j has pairs s16*16 .. +15 of segment seg (a head's q, k or v); their elements are its two row tiles
-    const int per_seg = TAIL ? tail.d / 32 : 1, seg = j / per_seg, s16 = j % per_seg;
+    const int per_seg = TAIL ? head / 32 : 1, seg = j / per_seg, s16 = j % per_seg;
     auto tail_row = [&](int i, int t) {  // element t of pair i of the sixteen, within the segment
-        if (TAIL == 1) return s16 * 16 + i + (t & 1) * (tail.d >> 1);
+        if (TAIL == 1) return s16 * 16 + i + (t & 1) * (head >> 1);
         int e[2] = {0, 0};
         bool rotated;
         qkv_tail_pair_elements(tail.rot, tail.d, s16 * 16 + i, e[0], e[1], rotated);
@@ -210,13 +228,13 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     // Where a row of W is a power of two long, every workgroup walking K from its start would ask the same few
     // memory channels at the same time (K = 4,096: 13 % slower than K = 4,160).  So each starts `rot_stride`
     // steps after its neighbour.  A feature's order of summation follows from N, K and the launch alone.
-    const int rot = start_step(rot_stride, nsteps);
+    const int rot = start_step(walk.rot_stride, nsteps);
     if constexpr (D > 0) {
         RowStream<RT, D> rows;
         rows.x = buffer_of(x, M * K * 2);
 #pragma unroll
         for (int t = 0; t < RT; ++t) {
-            const int first = tailed ? seg * tail.d : min(n0 + t * 16, N - 1), count = tailed ? tail.d : min(16, n1 - n0 - t * 16);
+            const int first = tailed ? seg * head : min(n0 + t * 16, n1 - 1), count = tailed ? head : min(16, n1 - n0 - t * 16);
             rows.w[t] = buffer_of(W + (long)first * K, max(count, 0) * K * 2);
 #pragma unroll
             for (int l = 0; l < 2; ++l) {
@@ -235,7 +253,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     } else {
         const bf16_t* wrow[RT];
 #pragma unroll
-        for (int t = 0; t < RT; ++t) wrow[t] = W + (long)(tailed ? seg * tail.d + tail_row(r, t) : min(n0 + t * 16 + r, n1 - 1)) * K;
+        for (int t = 0; t < RT; ++t) wrow[t] = W + (long)(tailed ? seg * head + tail_row(r, t) : min(n0 + t * 16 + r, n1 - 1)) * K;
         by_registers<MT, RT, U>(acc, wrow, x, lane, wave, S, M, K, nsteps, rot);
     }
 #pragma unroll
@@ -244,10 +262,15 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
         for (int mt = 0; mt < MT; ++mt) part[wave * WAVE + (rt * MT + mt) * 64 + lane] = acc[rt][mt];
     __syncthreads();
 
+    OutT* __restrict__ y = (OutT*)(second ? pb.y : pa.y);
+    const float* __restrict__ bias = second ? pb.bias : pa.bias;
+    const bf16_t* __restrict__ add1 = second ? pb.add1 : pa.add1;
+    const bf16_t* __restrict__ add2 = second ? pb.add2 : pa.add2;
+    const int N = second ? pb.N : pa.N, act = second ? pb.act : pa.act;
     if constexpr (TAIL) {
         if (tailed) {
             // thread ln: token m = ln % 16, features i0 .. i0+3 of the segment's lower half and their partners
-            for (int ln = threadIdx.x; ln < 64; ln += blockDim.x) {
+            for (int ln = threadIdx.x; ln < 64; ln += S * 64) {
                 f32x4_t lo = part[ln], hi = part[64 + ln];
                 for (int w = 1; w < S; ++w) {
                     const f32x4_t p = part[w * WAVE + ln], q = part[w * WAVE + 64 + ln];
@@ -317,7 +340,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
         }
     }
     // item (rt, mt, ln): outputs of row m = mt*16 + ln%16, columns n0 + rt*16 + (ln/16)*4 + 0..3
-    for (int item = threadIdx.x; item < RT * MT * 64; item += blockDim.x) {
+    for (int item = threadIdx.x; item < RT * MT * 64; item += S * 64) {
         const int ln = item & 63, mt = (item >> 6) % MT, rt = (item >> 6) / MT;
         f32x4_t sum = part[(rt * MT + mt) * 64 + ln];
         for (int w = 1; w < S; ++w) {
@@ -334,6 +357,17 @@ __global__ __launch_bounds__(512) void gemm_skinny_kernel(SkinnyProblem pa, Skin
     }
 }
 
+// the two elements of a rotation pair, within their head
+__device__ __forceinline__ void tail_elements(const Walk& walk, const QkvTail& tail, int pair, int (&e)[2]) {
+    bool rotated;
+    if (walk.plain) {
+        e[0] = pair, e[1] = pair + (walk.d >> 1);
+        return;
+    }
+    asm volatile("");  // (a branch: what is read there is not among the first arguments)
+    qkv_tail_pair_elements(tail.rot, walk.d, pair, e[0], e[1], rotated);
+}
+
 // Heads that hold rotation pairs p0 .. p1 - 1, `half` pairs a head: what a workgroup's buffer of W has to span.  Two for up to eight
 // pairs of heads of fourteen elements and more; eight pairs of heads of two lie in eight.
 __device__ __forceinline__ int heads_of(int p0, int p1, int half) { return (p1 - 1) / half - p0 / half + 1; }
@@ -344,25 +378,25 @@ __device__ __forceinline__ int heads_of(int p0, int p1, int half) { return (p1 -
 // takes what the product alone takes, and the launch that split, rotated and wrote the cache (4 us a layer) is gone: a
 // model of 24 such layers, 5 sequences, 24 steps and their prompts 34.5 -> 32.2 ms.
 template <int D>
-__global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W,
-                                                               const float* __restrict__ bias, int M, int K, int rot_stride,
-                                                               Share share, QkvTail tail) {
+__global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int K,
+                                                               uint32_t items, uint32_t how, const float* __restrict__ bias, QkvTail tail) {
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums
     constexpr int WAVE = D == 0 ? 64 : RowStream<1, D == 0 ? 1 : D>::RING / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6, half = tail.d >> 1;
+    const Walk walk(how);
+    const Share share = Share::of(items);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = walk.waves, head = walk.d, half = head >> 1;
     const int p0 = share.begin(blockIdx.x), p1 = share.end(blockIdx.x);
-    const int nsteps = (K + 63) >> 6, rot = start_step(rot_stride, nsteps);
+    const int nsteps = (K + 63) >> 6, rot = start_step(walk.rot_stride, nsteps);
     auto row_of = [&](int pair, int second) {  // of W: an element of a pair
         int e[2];
-        bool rotated;
-        qkv_tail_pair_elements(tail.rot, tail.d, pair % half, e[0], e[1], rotated);
-        return pair / half * tail.d + (second ? e[1] : e[0]);
+        tail_elements(walk, tail, pair % half, e);
+        return pair / half * head + (second ? e[1] : e[0]);
     };
     f32x4_t sum = f32x4_t{0.f, 0.f, 0.f, 0.f};
     if constexpr (D > 0) {
-        const int first = p0 / half * tail.d;  // row of W that the others are counted from
+        const int first = p0 / half * head;  // row of W that the others are counted from
         RowStream<1, D> rows;
-        rows.w[0] = buffer_of(W + (long)first * K, heads_of(p0, p1, half) * tail.d * K * 2);
+        rows.w[0] = buffer_of(W + (long)first * K, heads_of(p0, p1, half) * head * K * 2);
         rows.x = buffer_of(x, M * K * 2);
 #pragma unroll
         for (int l = 0; l < 2; ++l) {
@@ -382,7 +416,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_tail_kernel(const bf16_t* __r
     part[wave * WAVE + lane] = sum;
     __syncthreads();
     const float* sums = (const float*)part;  // row i of the tile, column m: lane (i / 4) * 16 + m, element i % 4
-    for (int item = threadIdx.x; item < 128; item += blockDim.x) {
+    for (int item = threadIdx.x; item < 128; item += S * 64) {
         const int m = item & 15, i = item >> 4, pair = p0 + i;
         if (m >= M || pair >= p1) continue;
         const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
@@ -407,12 +441,12 @@ __device__ __forceinline__ void halves_end(const SkinnyProblem& p, const QkvTail
         return v;
     };
     if constexpr (TAIL) {
-        for (int item = threadIdx.x; item < 4 * M; item += blockDim.x) {
+        for (int item = threadIdx.x; item < 4 * M; item += S * 64) {
             const int m = item >> 2, i = item & 3, pair = n0 + i;
             if (pair < n1) qkv_tail_pair(tail, p.bias, m, pair / half, pair % half, round_to_bf16(sum_of(m, i)), round_to_bf16(sum_of(m, i + 4)));
         }
     } else {
-        for (int item = threadIdx.x; item < 8 * M; item += blockDim.x) {
+        for (int item = threadIdx.x; item < 8 * M; item += S * 64) {
             const int m = item >> 3, i = item & 7;
             if (n0 + i < n1) store_feature<OutT>((OutT*)p.y, p.bias, p.act, p.add1, p.add2, p.N, m, n0 + i, sum_of(m, i));
         }
@@ -429,26 +463,28 @@ __device__ __forceinline__ void halves_end(const SkinnyProblem& p, const QkvTail
 // TAIL: a fused query_key_value product taken to its end as by gemm_skinny_tail_kernel; rows 0 .. 3 are the first elements of up
 // to four rotation pairs, rows 4 .. 7 their partners.
 template <int MT, bool DIAG, int U, typename OutT, bool TAIL>
-__global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p, int M, int K, int rot_stride, QkvTail tail) {
+__global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(const bf16_t* __restrict__ x_rows, const bf16_t* __restrict__ W, int M, int K, uint32_t items,
+                                                                 uint32_t how, SkinnyProblem p, QkvTail tail) {
     static_assert(!DIAG || MT == 1, "both halves of K in a tile: eight rows of x");
     constexpr int BT = DIAG ? 1 : 2 * MT;  // fragments of x a half step
     extern __shared__ f32x4_t part[];      // [S][MT][64]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const Walk walk(how);
+    const Share share = Share::of(items);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = walk.waves;
     const int r = lane & 15, g = lane >> 4, row = r & 7, sub = r >> 3;
-    const int half = TAIL ? tail.d >> 1 : 1;
-    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);  // pairs, or rows
+    const int half = TAIL ? walk.d >> 1 : 1;
+    const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);  // pairs, or rows
     int w_row = min(n0 + row, n1 - 1);
     if (TAIL) {
         const int mine = min(n0 + (row & 3), n1 - 1);  // (places past the end read a pair again)
-        int ea, eb;
-        bool rotated;
-        qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
-        w_row = mine / half * tail.d + (row < 4 ? ea : eb);
+        int e[2];
+        tail_elements(walk, tail, mine % half, e);
+        w_row = mine / half * walk.d + (row < 4 ? e[0] : e[1]);
     }
-    const bf16_t* wrow = p.W + (long)w_row * K;
-    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)p.x, 0, M * K * 2, 0x00020000);
+    const bf16_t* wrow = W + (long)w_row * K;
+    __amdgpu_buffer_rsrc_t xres = __builtin_amdgcn_make_buffer_rsrc((void*)x_rows, 0, M * K * 2, 0x00020000);
     const int nsteps = (K + 127) >> 7;
-    const int rot = start_step(rot_stride, nsteps);
+    const int rot = start_step(walk.rot_stride, nsteps);
     struct Halves {
         Frag a[U][2], b[U][2][BT];
         uint32_t keep[U][2];
@@ -514,28 +550,30 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_kernel(SkinnyProblem p
 // 2,048 5.3 -> 3.9, 6.6 -> 4.3, 9.0 -> 5.4, 14.4 -> 7.3.  What bounds it: with few rows the start and the end (2.3 us for 300 x 72), then
 // the weights (2,048 x 8,192: 3.9 TB/s); with many the reading of x, all of which every workgroup needs (64 rows of 8,192: 1 MB each).
 template <int MT, bool DIAG, int D, typename OutT, bool TAIL>
-__global__ __launch_bounds__(512) void gemm_skinny_halves_ring_kernel(SkinnyProblem p, int M, int K, int rot_stride, QkvTail tail) {
+__global__ __launch_bounds__(512) void gemm_skinny_halves_ring_kernel(const bf16_t* __restrict__ x_rows, const bf16_t* __restrict__ W, int M, int K, uint32_t items,
+                                                                 uint32_t how, SkinnyProblem p, QkvTail tail) {
     static_assert(!DIAG || MT == 1, "both halves of K in a tile: eight rows of x");
     constexpr int BT = DIAG ? 1 : 2 * MT, SLOT = 2048 * (1 + BT), RING = D * SLOT, LOADS = 2 * (1 + BT), WAVE = RING / 16;
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums, [64] each
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = blockDim.x >> 6;
-    const int r = lane & 15, g = lane >> 4, half = TAIL ? tail.d >> 1 : 1;
-    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);  // pairs, or rows
-    const int nsteps = (K + 127) >> 7, rot = start_step(rot_stride, nsteps);
+    const Walk walk(how);
+    const Share share = Share::of(items);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), S = walk.waves;
+    const int r = lane & 15, g = lane >> 4, half = TAIL ? walk.d >> 1 : 1;
+    const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);  // pairs, or rows
+    const int nsteps = (K + 127) >> 7, rot = start_step(walk.rot_stride, nsteps);
     const int row = lane >> 3;  // the row that the lane's sixteen bytes are of
     int first = n0, at_row;     // of W: the row that the others are counted from, and the lane's
     if (TAIL) {
         const int pair = n0 + (row & 3);
         int e[2];
-        bool rotated;
-        qkv_tail_pair_elements(tail.rot, tail.d, pair % half, e[0], e[1], rotated);
-        first = n0 / half * tail.d;
-        at_row = pair < n1 ? pair / half * tail.d + (row < 4 ? e[0] : e[1]) - first : -1;
+        tail_elements(walk, tail, pair % half, e);
+        first = n0 / half * walk.d;
+        at_row = pair < n1 ? pair / half * walk.d + (row < 4 ? e[0] : e[1]) - first : -1;
     } else {
         at_row = n0 + row < n1 ? row : -1;
     }
-    const i32x4_t w = buffer_of(p.W + (long)first * K, (TAIL ? heads_of(n0, n1, half) * tail.d : n1 - n0) * K * 2);
-    const i32x4_t x = buffer_of(p.x, M * K * 2);
+    const i32x4_t w = buffer_of(W + (long)first * K, (TAIL ? heads_of(n0, n1, half) * walk.d : n1 - n0) * K * 2);
+    const i32x4_t x = buffer_of(x_rows, M * K * 2);
     const int w_at = at_row >= 0 ? at_row * K * 2 : LDS_PAST;
     int x_at[2 * MT];
 #pragma unroll
@@ -606,14 +644,15 @@ __global__ __launch_bounds__(512) void gemm_skinny_halves_ring_kernel(SkinnyProb
 // for up to 16 rows.  A workgroup's two row tiles are the same rows of the gate and of the up matrix.  As a pass of its own
 // the gate took 4.5 us behind a product of 13 (2 rows, 2 x 5,504 x 2,048).
 template <int D>
-__global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict__ y, const bf16_t* __restrict__ x,
-                                                              const bf16_t* __restrict__ W, int M, int F, int K, int rot_stride, int kind,
-                                                              float alpha, float limit, Share share) {
+__global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, int M, int F, int K,
+                                                              uint32_t items, uint32_t how, bf16_t* __restrict__ y, int kind, float alpha, float limit) {
     extern __shared__ __attribute__((aligned(1024))) f32x4_t part[];  // the waves' rings, and then their sums, [2][64] each
     constexpr int WAVE = D == 0 ? 128 : RowStream<2, D == 0 ? 1 : D>::RING / 16;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = blockDim.x >> 6;
+    const Walk walk(how);
+    const Share share = Share::of(items);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, S = walk.waves;
     const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);
-    const int nsteps = (K + 63) >> 6, rot = start_step(rot_stride, nsteps);
+    const int nsteps = (K + 63) >> 6, rot = start_step(walk.rot_stride, nsteps);
     f32x4_t acc[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
     if constexpr (D > 0) {
         RowStream<2, D> rows;
@@ -638,7 +677,7 @@ __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict
     for (int rt = 0; rt < 2; ++rt) part[wave * WAVE + rt * 64 + lane] = acc[rt];
     __syncthreads();
     const float* sums = (const float*)part;  // feature i of a tile, row m of x: lane (i / 4) * 16 + m, element i % 4
-    for (int item = threadIdx.x; item < 16 * M; item += blockDim.x) {
+    for (int item = threadIdx.x; item < 16 * M; item += S * 64) {
         const int m = item >> 4, i = item & 15;
         if (n0 + i >= n1) continue;
         const int at = ((i >> 2) * 16 + m) * 4 + (i & 3);
@@ -662,25 +701,18 @@ __global__ __launch_bounds__(512) void gemm_skinny_glu_kernel(bf16_t* __restrict
 // -> 6.1; 4,160 x 1,040 9.4 -> 6.3, 9.7 -> 6.8, 9.8 -> 8.7, 10.0 -> 9.4; 6,144 x 1,536 12.6 -> 8.5, 12.8 -> 8.8, 12.9 -> 10.8, 13.6 -> 11.4;
 // 8,192 x 2,048 16.2 -> 11.9, 16.4 -> 12.0, 15.8 -> 15.2, 16.8 -> 16.3.
 template <int NORMED_WAVES, int CH, int RW, bool TAIL>  // CH: groups of 512 elements of a row; RW: rows of x a wave norms
-__global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_normed_kernel(SkinnyProblem p, const float* __restrict__ ln_w,
-                                                                       const float* __restrict__ ln_b, float eps, int M, int K,
-                                                                       QkvTail tail) {
+__global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_normed_kernel(
+    const bf16_t* __restrict__ x, const bf16_t* __restrict__ W, const float* __restrict__ ln_w, const float* __restrict__ ln_b, int M, int K, uint32_t items,
+    uint32_t how, float eps, SkinnyProblem p, QkvTail tail) {
     constexpr int STEPS = 8 * CH / NORMED_WAVES;  // steps of 64 elements of K a wave takes
     extern __shared__ f32x4_t part[];  // [waves][64], then the normed rows [M][K + 8]
     bf16_t* rows = (bf16_t*)(part + NORMED_WAVES * 64);
     const int pitch = K + 8;  // sixteen bytes between rows keep the reads of sixteen rows on distinct banks
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int r = lane & 15, g = lane >> 4, half = TAIL ? tail.d >> 1 : 1;
-    const int n0 = p.rows.begin(blockIdx.x), n1 = p.rows.end(blockIdx.x);
-    int w_row = min(n0 + r, n1 - 1);
-    if (TAIL) {  // as in gemm_skinny_tail_kernel
-        const int mine = min(n0 + (r & 7), n1 - 1);
-        int ea, eb;
-        bool rotated;
-        qkv_tail_pair_elements(tail.rot, tail.d, mine % half, ea, eb, rotated);
-        w_row = mine / half * tail.d + (r < 8 ? ea : eb);
-    }
-    const bf16_t* wrow = p.W + (long)w_row * K;
+    const Walk walk(how);
+    const Share share = Share::of(items);
+    const int r = lane & 15, g = lane >> 4, half = TAIL ? walk.d >> 1 : 1;
+    const int n0 = share.begin(blockIdx.x), n1 = share.end(blockIdx.x);
     const int chunks = K >> 3;
     constexpr int RB = RW < 2 || (RW == 4 && CH == 4) ? 1 : 2;  // rows normed at a time: what leaves registers for two workgroups of four waves a unit
     uint4 xv[RB][CH];
@@ -690,7 +722,7 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
         for (int i = 0; i < RB; ++i)
 #pragma unroll
             for (int j = 0; j < CH; ++j)
-                xv[i][j] = *reinterpret_cast<const uint4*>(p.x + (long)min(wave + (b + i) * NORMED_WAVES, M - 1) * K + min(lane + j * 64, chunks - 1) * 8);
+                xv[i][j] = *reinterpret_cast<const uint4*>(x + (long)min(wave + (b + i) * NORMED_WAVES, M - 1) * K + min(lane + j * 64, chunks - 1) * 8);
     };
     load_rows(0);
 #pragma unroll
@@ -703,6 +735,14 @@ __global__ __launch_bounds__(NORMED_WAVES * 64, RW == 4 ? 2 : 1) void gemm_norme
         }
     }
     __builtin_amdgcn_sched_barrier(0);
+    int w_row = min(n0 + r, n1 - 1);
+    if (TAIL) {  // as in gemm_skinny_tail_kernel
+        const int mine = min(n0 + (r & 7), n1 - 1);
+        int e[2];
+        tail_elements(walk, tail, mine % half, e);
+        w_row = mine / half * walk.d + (r < 8 ? e[0] : e[1]);
+    }
+    const bf16_t* wrow = W + (long)w_row * K;
     Frag a[STEPS][2];
 #pragma unroll
     for (int u = 0; u < STEPS; ++u)
@@ -822,6 +862,14 @@ static int launch_rings(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStr
     return 0;
 }
 
+// gemm_skinny_kernel, in the order that it takes its arguments in
+template <typename Kernel>
+static int launch_two(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, const SkinnyProblem& a, const SkinnyProblem& b, int M, int K, int rot_stride,
+                      const QkvTail& tail = QkvTail{}) {
+    return launch_rings(kernel, grid, block, lds, s, a.x, a.W, b.x, b.W, M, K, a.blocks, a.rows.packed(), b.rows.packed(),
+                        Walk::packed((int)block.x / 64, rot_stride, tail.d), a, b, tail);
+}
+
 template <int MT, int RT, int U, typename OutT>
 static int launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hipStream_t s, bool spread = false) {
     const int rows = 16 * RT;
@@ -851,10 +899,10 @@ static int launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hip
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);  // rows a multiple of 4 KB long
     if constexpr (MT == 1 && RT <= 2) if (K <= STREAM_MOST_K) {
-        if (S <= 4) return launch_rings(gemm_skinny_kernel<MT, RT, U, OutT, 0, 4>, grid, block, (size_t)S * RowStream<RT, 4>::RING, s, a, b, M, K, rot_stride, QkvTail{});
-        return launch_rings(gemm_skinny_kernel<MT, RT, U, OutT, 0, 3>, grid, block, (size_t)S * RowStream<RT, 3>::RING, s, a, b, M, K, rot_stride, QkvTail{});
+        if (S <= 4) return launch_two(gemm_skinny_kernel<MT, RT, U, OutT, 0, 4>, grid, block, (size_t)S * RowStream<RT, 4>::RING, s, a, b, M, K, rot_stride);
+        return launch_two(gemm_skinny_kernel<MT, RT, U, OutT, 0, 3>, grid, block, (size_t)S * RowStream<RT, 3>::RING, s, a, b, M, K, rot_stride);
     }
-    hipLaunchKernelGGL((gemm_skinny_kernel<MT, RT, U, OutT>), grid, block, lds, s, a, b, M, K, rot_stride, QkvTail{});
+    launch_two(gemm_skinny_kernel<MT, RT, U, OutT>, grid, block, lds, s, a, b, M, K, rot_stride);
     return 0;
 }
 
@@ -874,10 +922,11 @@ static int launch_halves(SkinnyProblem p, int M, int K, int S, hipStream_t s, co
     p.rows = Share(items, (int)grid.x);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 3 : 0);
-    auto go = [&](auto kernel, int tiles) { hipLaunchKernelGGL(kernel, grid, block, (size_t)S * tiles * 64 * sizeof(f32x4_t), s, p, M, K, rot, tail); };
+    const uint32_t how = Walk::packed(S, rot, tail.d, TAIL && qkv_tail_plain_pairs(tail.rot, tail.d));
+    auto go = [&](auto kernel, int tiles) { hipLaunchKernelGGL(kernel, grid, block, (size_t)S * tiles * 64 * sizeof(f32x4_t), s, p.x, p.W, M, K, p.rows.packed(), how, p, tail); };
     if (K <= STREAM_MOST_K && (M <= 16 || S <= 4)) {
         int rc = 0;
-        auto ring = [&](auto kernel, int bytes) { rc = launch_rings(kernel, grid, block, (size_t)S * bytes, s, p, M, K, rot, tail); };
+        auto ring = [&](auto kernel, int bytes) { rc = launch_rings(kernel, grid, block, (size_t)S * bytes, s, p.x, p.W, M, K, p.rows.packed(), how, p, tail); };
         auto of_depth = [&](auto tiles, auto few, auto two, auto four, auto eight) {  // loads on their way that LDS has room for
             constexpr int MT = tiles(), SLOT = 2048 * (few() ? 2 : 1 + 2 * MT);
             if (S <= 2) ring(gemm_skinny_halves_ring_kernel<MT, few(), two(), OutT, TAIL>, two() * SLOT);
@@ -1013,7 +1062,7 @@ extern "C" int pta_gemm_skinny_pair_qkv_bf16(void* q_out, const void* x1, const 
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
     auto go = [&](auto kernel, size_t ring) {
-        return launch_rings(kernel, dim3(a.blocks + b.blocks), dim3(S * 64), S * ring, (hipStream_t)stream, a, b, M, K, rot_stride, tail);
+        return launch_two(kernel, dim3(a.blocks + b.blocks), dim3(S * 64), S * ring, (hipStream_t)stream, a, b, M, K, rot_stride, tail);
     };
     const bool plain = qkv_tail_plain_pairs(rot, d);
     int rc;
@@ -1070,7 +1119,8 @@ extern "C" int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* 
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
     auto go = [&](auto kernel, size_t ring) {
-        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, p.x, p.W, bias, M, K, rot_stride, Share(pairs, blocks), tail);
+        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, p.x, p.W, M, K, Share(pairs, blocks).packed(),
+                            Walk::packed(S, rot_stride, d, qkv_tail_plain_pairs(tail.rot, d)), bias, tail);
     };
     if (K > STREAM_MOST_K ? go(gemm_skinny_tail_kernel<0>, 1024) : go(gemm_skinny_tail_kernel<4>, RowStream<1, 4>::RING)) return 1;
     return pta_check_launch("gemm_skinny_qkv_bf16");
@@ -1096,7 +1146,8 @@ static int launch_normed(const char* what, SkinnyProblem p, const float* ln_w, c
     bool refused = false;
     auto go = [&](auto kernel) {
         if (lds > 64 * 1024) refused = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess;
-        if (!refused) hipLaunchKernelGGL(kernel, dim3(groups), dim3(waves * 64), lds, s, p, ln_w, ln_b, eps, M, K, tail);
+        if (!refused) hipLaunchKernelGGL(kernel, dim3(groups), dim3(waves * 64), lds, s, p.x, p.W, ln_w, ln_b, M, K, p.rows.packed(),
+                                         Walk::packed(waves, 0, tail.d, TAIL && qkv_tail_plain_pairs(tail.rot, tail.d)), eps, p, tail);
     };
     auto by_rows = [&](auto ch) {
         constexpr int CH = decltype(ch)::value;
@@ -1147,8 +1198,8 @@ extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, i
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
     auto go = [&](auto kernel, size_t ring) {
-        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (bf16_t*)y, (const bf16_t*)x, (const bf16_t*)W, M, F, K,
-                            rot_stride, kind, alpha, limit, Share(F, blocks));
+        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)W, M, F, K, Share(F, blocks).packed(),
+                            Walk::packed(S, rot_stride), (bf16_t*)y, kind, alpha, limit);
     };
     if (K > STREAM_MOST_K ? go(gemm_skinny_glu_kernel<0>, 2048)
                           : S <= 4 ? go(gemm_skinny_glu_kernel<4>, RowStream<2, 4>::RING) : go(gemm_skinny_glu_kernel<3>, RowStream<2, 3>::RING)) return 1;
