@@ -102,24 +102,33 @@ __device__ __forceinline__ float column_max(float v) { return fold_32(fold_16(v,
 // Sum over a block of up to 1024 threads; every thread gets the result.  `red`
 // is LDS of at least 16 floats.  The order of additions depends on the block
 // size only.
-__device__ __forceinline__ float block_sum(float v, float* red) {
+__device__ __forceinline__ float block_sum(float v, float* red, int nw) {  // nw: the block's waves
     v = wave_sum(v);
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
-    float t = 0.f;
-    for (int i = 0; i < nw; ++i) t += red[i];
+    // all of them asked for at once, what no wave wrote too: a loop of as many as there are waits for LDS in every turn
+    float w[16], t = 0.f;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = red[i];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t = i < nw ? t + w[i] : t;
     return t;
 }
+__device__ __forceinline__ float block_sum(float v, float* red) { return block_sum(v, red, (blockDim.x + 63) >> 6); }
 __device__ __forceinline__ float block_max(float v, float* red) {
     v = wave_max(v);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, nw = (blockDim.x + 63) >> 6;
     __syncthreads();
     if (lane == 0) red[wave] = v;
     __syncthreads();
-    float t = red[0];
-    for (int i = 1; i < nw; ++i) t = fmaxf(t, red[i]);
+    float w[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) w[i] = red[i];
+    float t = w[0];
+#pragma unroll
+    for (int i = 1; i < 16; ++i) t = i < nw ? fmaxf(t, w[i]) : t;
     return t;
 }
 

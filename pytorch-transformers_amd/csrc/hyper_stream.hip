@@ -14,6 +14,7 @@
 #include "pta_kernels.h"
 
 #include <algorithm>
+#include <type_traits>
 
 #define HYPER_MAX_STREAMS 8
 
@@ -28,6 +29,14 @@ template <> struct Vec<4> {
         v[0] = bf16_bits_to_f32((bf16_t)(q.x & 0xffffu)); v[1] = bf16_bits_to_f32((bf16_t)(q.x >> 16));
         v[2] = bf16_bits_to_f32((bf16_t)(q.y & 0xffffu)); v[3] = bf16_bits_to_f32((bf16_t)(q.y >> 16));
     }
+    // as it lies in memory: where loads come one behind the other with branches between, words widened at once are waited for at each
+    static __device__ __forceinline__ void ld(const float* p, float4& q) { q = *reinterpret_cast<const float4*>(p); }
+    static __device__ __forceinline__ void ld(const bf16_t* p, uint2& q) { q = *reinterpret_cast<const uint2*>(p); }
+    static __device__ __forceinline__ void widen(const float4& q, float (&v)[4]) { v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w; }
+    static __device__ __forceinline__ void widen(const uint2& q, float (&v)[4]) {
+        v[0] = bf16_bits_to_f32((bf16_t)(q.x & 0xffffu)); v[1] = bf16_bits_to_f32((bf16_t)(q.x >> 16));
+        v[2] = bf16_bits_to_f32((bf16_t)(q.y & 0xffffu)); v[3] = bf16_bits_to_f32((bf16_t)(q.y >> 16));
+    }
     static __device__ __forceinline__ void st(float* p, const float (&v)[4]) {
         *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
     }
@@ -38,6 +47,8 @@ template <> struct Vec<4> {
 };
 template <> struct Vec<1> {
     template <typename T> static __device__ __forceinline__ void ld(const T* p, float (&v)[1]) { v[0] = Io<T>::ld(p); }
+    template <typename T> static __device__ __forceinline__ void ld(const T* p, T& q) { q = *p; }
+    template <typename T> static __device__ __forceinline__ void widen(const T& q, float (&v)[1]) { v[0] = Io<T>::ld(&q); }
     template <typename T> static __device__ __forceinline__ void st(T* p, const float (&v)[1]) { Io<T>::st(p, v[0]); }
 };
 
@@ -144,46 +155,67 @@ __global__ __launch_bounds__(1024) void hyper_norm_kernel(HyperArgs a) {
 // The same where a row has a chunk of V features for each thread of a workgroup (4,096 features) and the convolution up to ONCE_TAPS taps: what every
 // published width is.  A step of a few tokens is one chain, and all that does not hang on the norm is asked for at its start: the streams' weights, which the
 // loop above loads again behind every store, the norm's, the taps and the sequence's tail, whose row is two look-ups away.  2,048 features, four
-// streams, four taps, 2 tokens: 6.6 -> 5.3 us.
+// streams, four taps, 2 tokens, in a step: 6.6 us, 5.3 with the loads at the start, 3.6 with none of them behind a wait: a result in 16 bits that is widened where it
+// is loaded, a look-up or a weight of the streams that comes by a vector load, an argument that is not there yet each waited for all before it.
 #define ONCE_TAPS 4
 
+// What its first loads are found by comes first and packed, in the fourteen words that are in registers when a workgroup starts.  sizes: features | taps
+// << 16 | whether rows are picked << 31.
 template <typename T, int S, int V>
-__global__ __launch_bounds__(1024) void hyper_norm_once_kernel(HyperArgs a) {
+__global__ __launch_bounds__(1024) void hyper_norm_once_kernel(const float* __restrict__ xs_in, const T* __restrict__ y, const float* __restrict__ norm_w,
+                                                               const float* __restrict__ conv, const int* __restrict__ token_seq, uint32_t x_row,
+                                                               uint32_t x_stream, uint32_t y_ld, uint32_t sizes, const int* __restrict__ seq_slot,
+                                                               const float* __restrict__ mixes, const float* __restrict__ outs, const float* __restrict__ ins,
+                                                               const int* __restrict__ rows, HyperArgs a) {
     __shared__ float red[16];
-    const int m = blockIdx.x, H = a.H;
-    const bool live = (int)threadIdx.x * V < H, normed = a.h || a.n_out;
+    const int m = blockIdx.x, H = sizes & 0xffff, K = sizes >> 16 & 0xff, waves = max(1, ((H + V - 1) / V + 63) / 64);
+    const bool live = (int)threadIdx.x * V < H, normed = norm_w != nullptr;
     const int i = live ? threadIdx.x * V : 0;
-    const long src = a.rows ? a.rows[m] : m;
-    float* tl = a.conv && a.K > 1 ? a.tail + (long)a.seq_slot[a.token_seq[m]] * a.tail_ld : nullptr;
-    float mix[S][S], to[S], from[S];
-#pragma unroll
-    for (int t = 0; t < S; ++t) {
-        from[t] = a.in ? a.in[t] : 1.f;
-        to[t] = a.y ? a.out[t] : 0.f;
-#pragma unroll
-        for (int s = 0; s < S; ++s) mix[s][t] = a.y ? a.mix[s * S + t] : 0.f;
+    long src = m;
+    if (sizes >> 31) {
+        asm volatile("");
+        src = rows[m];
     }
     float xs[S][V], yv[V], w[V], taps[ONCE_TAPS][V], before[ONCE_TAPS][V];
 #pragma unroll
-    for (int s = 0; s < S; ++s) Vec<V>::ld(a.x + src * a.x_row + s * a.x_stream + i, xs[s]);
-    if (a.y) Vec<V>::ld((const T*)a.y + src * a.y_ld + i, yv);
-    if (normed) Vec<V>::ld(a.w + i, w);
-    if (a.conv) {
+    for (int s = 0; s < S; ++s) Vec<V>::ld(xs_in + src * x_row + (long)s * x_stream + i, xs[s]);
+    typename std::conditional<V == 1, T, typename std::conditional<sizeof(T) == 4, float4, uint2>::type>::type yq;
+    if (y) Vec<V>::ld(y + src * y_ld + i, yq);
+    if (normed) Vec<V>::ld(norm_w + i, w);
+    if (conv) {
 #pragma unroll
-        for (int k = 0; k < ONCE_TAPS; ++k) Vec<V>::ld(a.conv + (long)min(k, a.K - 1) * H + i, taps[k]);
-        if (tl) {
-#pragma unroll
-            for (int k = 0; k + 1 < ONCE_TAPS; ++k) Vec<V>::ld(tl + (long)min(k, a.K - 2) * H + i, before[k]);
-        }
+        for (int k = 0; k < ONCE_TAPS; ++k) Vec<V>::ld(conv + (long)min(k, K - 1) * H + i, taps[k]);
     }
     __builtin_amdgcn_sched_barrier(0);
+    float mix[S][S], to[S], from[S];
+#pragma unroll
+    for (int t = 0; t < S; ++t) from[t] = 1.f;
+    if (ins) {
+#pragma unroll
+        for (int t = 0; t < S; ++t) from[t] = ins[t];
+    }
+    if (y) {
+#pragma unroll
+        for (int t = 0; t < S; ++t) {
+            to[t] = outs[t];
+#pragma unroll
+            for (int s = 0; s < S; ++s) mix[s][t] = mixes[s * S + t];
+        }
+    }
+    float* tl = conv && K > 1 ? a.tail + (long)seq_slot[token_seq[m]] * a.tail_ld : nullptr;
+    if (tl) {
+#pragma unroll
+        for (int k = 0; k + 1 < ONCE_TAPS; ++k) Vec<V>::ld(tl + (long)min(k, K - 2) * H + i, before[k]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (y) Vec<V>::widen(yq, yv);
     float u[V], ss = 0.f;
 #pragma unroll
     for (int v = 0; v < V; ++v) u[v] = 0.f;
 #pragma unroll
     for (int t = 0; t < S; ++t) {
         float xt[V];
-        if (a.y) {
+        if (y) {
 #pragma unroll
             for (int v = 0; v < V; ++v) xt[v] = 0.f;
 #pragma unroll
@@ -204,30 +236,30 @@ __global__ __launch_bounds__(1024) void hyper_norm_once_kernel(HyperArgs a) {
     if (!normed) return;
 #pragma unroll
     for (int v = 0; v < V; ++v) ss += live ? u[v] * u[v] : 0.f;
-    const float inv = 1.0f / sqrtf(block_sum(ss, red) / (float)H + a.eps);
+    const float inv = 1.0f / sqrtf(block_sum(ss, red, waves) / (float)H + a.eps);
     if (!live) return;
     float n[V], h[V];
 #pragma unroll
     for (int v = 0; v < V; ++v) h[v] = n[v] = u[v] * inv * (a.offset + w[v]);
     if (a.n_out) Vec<V>::st(a.n_out + (long)m * H + i, n);
     if (!a.h) return;
-    if (a.conv) {
+    if (conv) {
         float acc[V];
 #pragma unroll
         for (int v = 0; v < V; ++v) acc[v] = 0.f;
 #pragma unroll
         for (int k = 0; k < ONCE_TAPS; ++k) {
-            if (k + 1 < a.K) {
+            if (k + 1 < K) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) acc[v] += taps[k][v] * before[k][v];
                 if (k > 0) Vec<V>::st(tl + (long)(k - 1) * H + i, before[k]);  // each input moves one place towards the oldest
             }
-            if (k + 1 == a.K) {
+            if (k + 1 == K) {
 #pragma unroll
                 for (int v = 0; v < V; ++v) h[v] += acc[v] + taps[k][v] * n[v];
             }
         }
-        if (a.K > 1) Vec<V>::st(tl + (long)(a.K - 2) * H + i, n);
+        if (K > 1) Vec<V>::st(tl + (long)(K - 2) * H + i, n);
     }
     Vec<V>::st((T*)a.h + (long)m * H + i, h);
 }
@@ -237,9 +269,12 @@ static int hyper_launch_s(const HyperArgs& a, int M, bool wide, hipStream_t s) {
     const int per = wide ? 4 : 1;
     const dim3 block(std::min(1024, std::max(64, ((a.H + per - 1) / per + 63) / 64 * 64)));
     const size_t lds = (size_t)a.H * sizeof(float);
-    if (a.H <= per * (int)block.x && (!a.conv || a.K <= ONCE_TAPS)) {
-        if (wide) hipLaunchKernelGGL((hyper_norm_once_kernel<T, S, 4>), dim3(M), block, 0, s, a);
-        else hipLaunchKernelGGL((hyper_norm_once_kernel<T, S, 1>), dim3(M), block, 0, s, a);
+    const bool near = a.x_row <= 0xffffffffL && a.x_stream <= 0xffffffffL && a.y_ld <= 0xffffffffL;
+    if (near && a.H <= per * (int)block.x && (!a.conv || a.K <= ONCE_TAPS)) {
+        const uint32_t sizes = (uint32_t)a.H | (uint32_t)(a.conv ? a.K : 0) << 16 | (a.rows ? 1u << 31 : 0u);
+        hipLaunchKernelGGL((wide ? hyper_norm_once_kernel<T, S, 4> : hyper_norm_once_kernel<T, S, 1>), dim3(M), block, 0, s, a.x, (const T*)a.y,
+                           a.h || a.n_out ? a.w : nullptr, a.conv, a.token_seq, (uint32_t)a.x_row, (uint32_t)a.x_stream, (uint32_t)a.y_ld, sizes, a.seq_slot, a.mix, a.out, a.in,
+                           a.rows, a);
         return pta_check_launch("hyper_norm");
     }
     if (wide) hipLaunchKernelGGL((hyper_norm_kernel<T, S, 4>), dim3(M), block, lds, s, a);
