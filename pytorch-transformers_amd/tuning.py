@@ -332,27 +332,30 @@ def decode_plan(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_l
 
 
 def several_waves_cut(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0):
-    """The cut of an untuned decode launch whose contexts are at most 1,024 keys and 512 on average: four waves of a workgroup
-    walk the whole context between them and merge in LDS, which leaves no ranges to merge by a launch of their own; or None,
-    where ``decode_plan`` decides.  Launch and merge, replayed over twelve caches in turn, the rule's ranges -> this, at 210
-    / 320 / 500 keys: 13 heads on 13 of 80, 5 sequences 10.8 -> 8.1, 11.1 -> 9.5, 11.6 -> 11.0 us, 16 sequences 11.8 -> 9.0, 12.5 ->
-    10.9, 15.8 -> 14.2, 32 (416 workgroups) 13.4 -> 13.7, 16.1 -> 17.2, 22.5 -> 20.5; 71 on 1 of 64, 8 sequences 7.9 -> 6.2,
-    8.5 -> 7.9, 9.1 -> 9.1; 128 on 8 of 64, 32 sequences 11.1 -> 7.7, 12.5 -> 9.3, 15.2 -> 13.2, 64 (512 workgroups) 10.1 -> 11.4, 11.7 ->
-    14.0, 16.6 -> 19.5.  Heads of 128 carry twice the sums through LDS: 32 on 8, 16 sequences 10.0 -> 9.8, 11.4 -> 12.1, 14.8 ->
-    16.2, 32 sequences 14.6 -> 12.9, 16.2 -> 15.3, 21.9 -> 20.6.  Shared keys (``_shared_keys_rule``) -> this where both
-    apply: 71 on 1 of 64, 33 sequences 7.9 -> 6.6, 11.8 -> 7.4, 12.3 -> 8.4, 48 sequences 7.9 -> 7.1, 12.4 -> 8.1, 12.8 -> 9.4, 64
-    (320 workgroups) 8.0 -> 9.9, 13.1 -> 11.6, 13.5 -> 13.9; 64 on 1 of 128, 33 sequences 10.1 -> 9.4, 14.5 -> 11.0, 15.0 ->
-    13.3, 64 sequences 10.2 -> 10.7, 16.0 -> 13.0, 16.6 -> 15.8.  One answer for 33 to 64 sequences (``decode_key``): it wins
-    everywhere but at the most sequences of one range of 256 keys."""
+    """The cut of an untuned decode launch whose whole contexts four waves of a workgroup walk between them, merging in LDS, which leaves no
+    ranges to merge by a launch of their own; or None, where ``decode_plan`` decides.  Launch and merge, replayed over eight
+    caches in turn, the rule's ranges -> this, us:
+
+    - contexts of at most 1,024 keys and 512 on average, at 220 / 500 keys: 13 heads on 13 of 80, 1 sequence 7.6 -> 5.2, 7.9 -> 6.7, 5 8.1 -> 5.8,
+      9.1 -> 7.4, 16 9.2 -> 6.9, 12.9 -> 9.5, 32 (416 workgroups) 9.0 -> 8.9, 17.2 -> 17.1; 71 on 1 of 64, 8 sequences 7.9 -> 5.3, 8.7 -> 7.7, 64
+      (320) 13.0 -> 8.0, 13.9 -> 12.4; 128 on 8 of 64, 32 sequences 11.2 -> 6.4, 13.6 -> 9.3, 64 (512) 8.9 -> 8.6, 16.7 -> 16.2.  Heads of 128 carry twice
+      the sums through LDS: 32 on 8, 8 sequences (64) 8.7 -> 7.5, 9.7 -> 11.4, 16 (128) 9.6 -> 7.6, 12.9 -> 11.7, 32 12.1 -> 9.0, 21.2 -> 16.3.
+    - of at most 1,024 and more than 512 on average, heads up to 80, where workgroups are about as many as compute units, at 900 keys: 208 workgroups
+      (13 on 13 of 80, 16 sequences) 20.3 -> 15.2; 256 (32 on 8 of 64, 32 sequences) 20.4 -> 14.9, (128 on 8) 20.3 -> 14.9; 104 to 128, which
+      the same count of sequences (``decode_key``) stands for, 11.9 -> 10.1 to 15.6 -> 11.1.  With 320 it is 14.9 -> 18.8, with 416 27.0 either way,
+      with 40 8.9 -> 10.3; and up to 2,048 keys 128 to 160 lose (16.4 -> 18.4 at 1,500) where 208 to 256 win (26.5 -> 22.0), under one count."""
     key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
     return None if key in _active.decode_plans else _several_waves_rule(*key)
 
 
 def _several_waves_rule(n: int, n_heads: int, n_kv_heads: int, head_dim: int, bound: int, mean: int):
-    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES or bound > 1024 or mean > 512:
+    if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES or bound > 1024 or not ops.load_library().pta_attn_decode_waves_ok(head_dim, 1, 4):
         return None
     groups = n * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)  # workgroups of the launch
-    if groups > 320 or (head_dim > 80 and groups < 192) or not ops.load_library().pta_attn_decode_waves_ok(head_dim, 1, 4):
+    if mean <= 512:
+        if groups > 320 or (head_dim > 80 and groups < 128):
+            return None
+    elif head_dim > 80 or not 192 <= groups <= 256:
         return None
     return (1, bound, 4)
 
