@@ -150,69 +150,124 @@ __device__ __forceinline__ void st4(bf16_t* p, const float (&v)[4]) {
                                               (uint32_t)f32_to_bf16_bits(v[2]) | ((uint32_t)f32_to_bf16_bits(v[3]) << 16));
 }
 
+// four neighbouring elements as they lie in memory: what is widened where it is loaded is waited for at the next branch, with all before it
+template <typename T> struct Raw4;
+template <> struct Raw4<float> {
+    float4 q;
+    __device__ __forceinline__ void load(const float* p) { q = *reinterpret_cast<const float4*>(p); }
+    __device__ __forceinline__ void widen(float (&v)[4]) const { v[0] = q.x; v[1] = q.y; v[2] = q.z; v[3] = q.w; }
+};
+template <> struct Raw4<bf16_t> {
+    uint2 q;
+    __device__ __forceinline__ void load(const bf16_t* p) { q = *reinterpret_cast<const uint2*>(p); }
+    __device__ __forceinline__ void widen(float (&v)[4]) const {
+        v[0] = bf16_bits_to_f32((bf16_t)(q.x & 0xffffu)); v[1] = bf16_bits_to_f32((bf16_t)(q.x >> 16));
+        v[2] = bf16_bits_to_f32((bf16_t)(q.y & 0xffffu)); v[3] = bf16_bits_to_f32((bf16_t)(q.y >> 16));
+    }
+};
+
 // The same where rows can be read four elements at a time (C times four a thread, at most 8,192 a group).  In a step of a
 // few rows the launch is one chain (load, sum over the workgroup, store) and its length is instructions as much as trips to
 // memory: 2,048 features of 8 rows 3.4 -> 2.4 us (with a gate 4.5 -> 2.9); of 2,000 rows 9.5 -> 6.0 us.
-template <typename TI, typename T, int C>
-__global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(T* __restrict__ out_narrow, float* __restrict__ out_wide,
-                                                           const TI* __restrict__ x, long x_ld, const T* __restrict__ gate,
-                                                           long gate_ld, const int* __restrict__ rows, const float* __restrict__ w,
-                                                           float offset, int group_len, float eps,
-                                                           const float* __restrict__ residual, float mult, int H,
-                                                           const float* __restrict__ planes, long plane,
-                                                           const float* __restrict__ coef, int count, float* __restrict__ mix_wide) {
+// What the loads are found by comes first and packed, in the fourteen words that are in registers when a workgroup starts; the others are a load away.
+// sizes: a group's elements, | planes << 16, | 1 << 30 with a gate, | 1 << 31 where rows are picked.  MIX > 0: a sum of streams is wanted, and its first MIX
+// planes (fewer: the last again, so that the wait for the row counts the loads behind it) are asked for with the row.  Behind the norm they came one
+// after the other: 8 rows of 2,048 with 2 / 5 / 9 planes 2.70, 3.05, 3.07 -> 2.54, 2.65, 3.02 us over warm caches; 192 such norms of a request, half of them with
+// planes, 9.00 -> 8.87 ms.
+#define MOST_PLANES 255
+
+template <typename TI, typename T, int C, int MIX>
+__global__ __launch_bounds__(1024) void rmsnorm_vec_kernel(
+    const TI* __restrict__ x, const float* __restrict__ w, const float* __restrict__ residual, const float* __restrict__ planes,
+    const float* __restrict__ coef, uint32_t x_ld, uint32_t plane, int H, uint32_t sizes, const T* __restrict__ gate, long gate_ld,
+    const int* __restrict__ rows, T* __restrict__ out_narrow, float* __restrict__ out_wide, float* __restrict__ mix_wide, float offset, float eps, float mult) {
     __shared__ float red[16];
-    const int m = blockIdx.x, g = blockIdx.y;
-    const long src = rows ? rows[m] : m;
+    const int m = blockIdx.x, g = blockIdx.y, group_len = sizes & 0xffff, before = MIX ? (int)(sizes >> 16 & 0xff) - 1 : 0;
+    const int threads = ((group_len / 4 + 63) / 64 * 64 / C + 63) / 64 * 64;
+    const bool gated = sizes >> 30 & 1;
+    long src = m;
+    if (sizes >> 31) {
+        asm volatile("");
+        src = rows[m];
+    }
     const TI* xr = x + src * x_ld + (long)g * group_len;
-    const T* gr = gate ? gate + src * gate_ld + (long)g * group_len : nullptr;
     const float* wr = w + (long)g * group_len;
     const float* rr = residual ? residual + src * H + (long)g * group_len : nullptr;
     const long o = (long)m * H + (long)g * group_len;
-    float v[C][4], z[C][4], wv[C][4], rv[C][4];
+    constexpr int AHEAD = MIX ? MIX : 1;
+    float v[C][4], cf[AHEAD];
+    Raw4<TI> xq[C];
+    Raw4<T> gq[C];
+    Raw4<float> wq[C], rq[C], pq[C][AHEAD];
 #pragma unroll
-    for (int c = 0; c < C; ++c) {
-        const int i = 4 * (threadIdx.x + c * blockDim.x);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[c][e] = z[c][e] = 0.f;
-        if (i < group_len) {
-            ld4(xr + i, v[c]);
-            if (gr) ld4(gr + i, z[c]);
-            ld4(wr + i, wv[c]);
-            if (rr) ld4(rr + i, rv[c]);
+    for (int c = 0; c < C; ++c) {  // (a thread past the group's end reads its start)
+        const int i = 4 * (threadIdx.x + c * threads), at = i < group_len ? i : 0;
+        xq[c].load(xr + at);
+        wq[c].load(wr + at);
+        if (rr) rq[c].load(rr + at);
+        if (gated) {
+            asm volatile("");
+            gq[c].load(gate + src * gate_ld + (long)g * group_len + at);
         }
+#pragma unroll
+        for (int j = 0; j < MIX; ++j) pq[c][j].load(planes + (long)max(min(j, before - 1), 0) * plane + o + at);
+    }
+#pragma unroll
+    for (int j = 0; j < MIX; ++j) cf[j] = coef[min(j, before)];
+    float own = MIX ? coef[before] : 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("" ::"s"(out_narrow), "s"(out_wide), "s"(mix_wide), "s"(offset), "s"(eps), "s"(mult));  // asked for here, not where they are used
+    if constexpr (MIX > 0) {
+        asm volatile("" : "+s"(own));
+#pragma unroll
+        for (int j = 0; j < MIX; ++j) asm volatile("" : "+s"(cf[j]));
     }
     float ss = 0.f;
 #pragma unroll
     for (int c = 0; c < C; ++c) {
+        const bool in = 4 * ((int)threadIdx.x + c * threads) < group_len;
+        xq[c].widen(v[c]);
+        if (gated) {
+            float z[4];
+            gq[c].widen(z);
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
-            if (gr) v[c][e] *= z[c][e] / (1.0f + expf(-z[c][e]));
+            for (int e = 0; e < 4; ++e) v[c][e] *= z[e] / (1.0f + expf(-z[e]));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[c][e] = in ? v[c][e] : 0.f;
         ss += (v[c][0] * v[c][0] + v[c][1] * v[c][1]) + (v[c][2] * v[c][2] + v[c][3] * v[c][3]);
     }
-    ss = block_sum(ss, red);
+    ss = block_sum(ss, red, threads / 64);
     const float inv = 1.0f / sqrtf(ss / (float)group_len + eps);
 #pragma unroll
     for (int c = 0; c < C; ++c) {
-        const int i = 4 * (threadIdx.x + c * blockDim.x);
+        const int i = 4 * (threadIdx.x + c * threads);
         if (i >= group_len) continue;
-        float n[4];
+        float n[4], wv[4], rv[4];
+        wq[c].widen(wv);
+        if (rr) rq[c].widen(rv);
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
-            n[e] = v[c][e] * inv * (offset + wv[c][e]);
-            if (rr) n[e] = rv[c][e] + mult * n[e];
+            n[e] = v[c][e] * inv * (offset + wv[e]);
+            if (rr) n[e] = rv[e] + mult * n[e];
         }
         if (out_wide) st4(out_wide + o + i, n);
-        if (planes) {
+        if constexpr (MIX > 0) {
             float acc[4] = {0.f, 0.f, 0.f, 0.f}, pv[4];
-#pragma unroll 8
-            for (int j = 0; j + 1 < count; ++j) {
+#pragma unroll
+            for (int j = 0; j < AHEAD; ++j)
+                if (j < before) {
+                    pq[c][j].widen(pv);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[e] += cf[j] * pv[e];
+                }
+            for (int j = AHEAD; j < before; ++j) {
                 ld4(planes + (long)j * plane + o + i, pv);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[e] += coef[j] * pv[e];
             }
 #pragma unroll
-            for (int e = 0; e < 4; ++e) n[e] = acc[e] + coef[count - 1] * n[e];
+            for (int e = 0; e < 4; ++e) n[e] = acc[e] + own * n[e];
             st4(mix_wide + o + i, n);
         }
         if (out_narrow) st4(out_narrow + o + i, n);
@@ -241,12 +296,18 @@ extern "C" int pta_rmsnorm(void* out_narrow, float* out_wide, const void* x, int
     // reads its row twice.
     auto on = [](const void* p, size_t bytes) { return (uintptr_t)p % bytes == 0; };
     const size_t narrow = dtype == PTA_F32 ? 16 : 8;
-    if (L % 4 == 0 && L >= 512 && L <= 8192 && x_ld % 4 == 0 && (!gate || gate_ld % 4 == 0) && plane % 4 == 0 && on(w, 16) && on(residual, 16) &&
+    const bool near = x_ld <= 0xffffffffL && plane <= 0xffffffffL && (!planes || count <= MOST_PLANES);
+    if (near && L % 4 == 0 && L >= 512 && L <= 8192 && x_ld % 4 == 0 && (!gate || gate_ld % 4 == 0) && plane % 4 == 0 && on(w, 16) && on(residual, 16) &&
         on(out_wide, 16) && on(planes, 16) && on(mix_wide, 16) && on(gate, narrow) && on(out_narrow, narrow) &&
         on(x, x_wide ? 16 : narrow)) {
         const int threads = (L / 4 + 63) / 64 * 64;
-#define RMS_VEC(TX, T, C) hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, T, C>), grid, dim3((threads / C + 63) / 64 * 64), 0, s, RMS_ARGS(T, TX, T))
-#define RMS_VEC_C(TX, T) if (threads <= 1024) RMS_VEC(TX, T, 1); else RMS_VEC(TX, T, 2)
+        const uint32_t sizes = (uint32_t)L | (planes ? (uint32_t)count << 16 : 0u) | (gate ? 1u << 30 : 0u) | (rows ? 1u << 31 : 0u);
+#define RMS_VEC(TX, T, C, MIX) hipLaunchKernelGGL((rmsnorm_vec_kernel<TX, T, C, MIX>), grid, dim3((threads / C + 63) / 64 * 64), 0, s, (const TX*)x, w, \
+                                                  residual, planes, coef, (uint32_t)x_ld, (uint32_t)plane, H, sizes, (const T*)gate, gate_ld, rows, \
+                                                  (T*)out_narrow, out_wide, mix_wide, offset, eps, mult)
+#define RMS_VEC_C(TX, T) if (threads > 1024) { if (planes) RMS_VEC(TX, T, 2, 2); else RMS_VEC(TX, T, 2, 0); } \
+                         else if (!planes) RMS_VEC(TX, T, 1, 0); else if (count <= 3) RMS_VEC(TX, T, 1, 2); \
+                         else if (count <= 5) RMS_VEC(TX, T, 1, 4); else RMS_VEC(TX, T, 1, 7)
         if (dtype == PTA_F32) { RMS_VEC_C(float, float); }
         else if (x_wide) { RMS_VEC_C(float, bf16_t); }
         else { RMS_VEC_C(bf16_t, bf16_t); }
