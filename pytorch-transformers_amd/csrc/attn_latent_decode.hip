@@ -8,8 +8,8 @@
 //   latent_values    merges a token's ranges and takes the result through the head's value expansion
 //
 // What bounds a layer here is launches and chains of dependent loads, not bytes: 16 heads, R = 512, dr = 64, 8 sequences of 64 to
-// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 21 in three (4.7,
-// 9.3 and 6.8).
+// 700 keys took 72 us a layer in eight launches (two of them the vendor library's, three copies), and takes 20 in three (4.6,
+// 9.2 and 5.8).
 #include "attn_latent_token.h"
 
 typedef __bf16 ld_bf16x8 __attribute__((ext_vector_type(8)));
@@ -59,43 +59,41 @@ __global__ __launch_bounds__(256) void latent_queries_kernel(float* __restrict__
 }
 
 // ---- pages --------------------------------------------------------------------------------------------------------------
-struct LatentPages {
-    float* po;  // [M, H, splits, R] sums of weights times rows, not normed
-    float* pm;  // [M, H, splits] maxima
-    float* pl;  // [M, H, splits] sums of weights
-    const float* q;  // [M, H, D]
-    const bf16_t* k_pool;
-    const int* block_table;
-    int bt_stride;
-    const int* seq_start;
-    int H, R, D;
-    float scale;
-    int size, splits;  // keys a range (whole pages), ranges
-};
-
 #define LP_PIECES 20  // D <= 640
 #define LP_QUERIES 5  // pieces of sixteen queries a thread takes: 16 D / 8 / 256
 
 // TILES: sixteen-element tiles of the value part a wave holds (its quarter of them)
 template <int TILES>
-__global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) {
+__global__ __launch_bounds__(256) void latent_pages_kernel(
+    // what a workgroup's loads are found by: the first fourteen words, which are in registers when it starts
+    const float* __restrict__ queries,  // [M, H, D]
+    const bf16_t* __restrict__ k_pool, const int* __restrict__ block_table, const int* __restrict__ seq_start, int bt_stride, int size, int splits, int H, int D,
+    int R,  // size: keys a range (whole pages); splits: ranges
+    float scale,
+    float* __restrict__ po,    // [M, H, splits, R] sums of weights times rows, not normed
+    float* __restrict__ pm,    // [M, H, splits] maxima
+    float* __restrict__ pl) {  // [M, H, splits] sums of weights
     extern __shared__ __attribute__((aligned(16))) bf16_t lds[];
-    const int D = a.D, P = D + 8;      // row distance in LDS: neighbouring rows start in other banks
+    const int P = D + 8;               // row distance in LDS: neighbouring rows start in other banks
     bf16_t* Ks = lds;                  // [64][P]
     bf16_t* Qs = Ks + 64 * P;          // [16][P]
     bf16_t* Ps = Qs + 16 * P;          // [16 columns][72] weights of the page's keys
     float* stat = (float*)(Ps + 16 * 72);  // [4][16] maxima, [4][16] sums
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, r16 = lane & 15, g = lane >> 4;
     const int s = blockIdx.z, split = blockIdx.y, h0 = blockIdx.x * 16;
-    const int nkeys = a.seq_start[s] + 1, k0 = split * a.size, k1 = min(nkeys, k0 + a.size);
-    const long row = (long)s * a.H + h0 + r16;  // this lane's column (a head past H: read as the last one, not kept)
-    const bool there = h0 + r16 < a.H;
+    const int k0 = split * size;
+    // the range's first page beside the sequence's length, not behind it (an entry past the sequence's pages is read but not used)
+    const int* bt = block_table + (long)s * bt_stride;
+    int first_page = bt[min(k0 / PTA_PAGE, bt_stride - 1)], nkeys = seq_start[s] + 1;
+    asm volatile("" : "+s"(first_page), "+s"(nkeys));
+    const int k1 = min(nkeys, k0 + size);
+    const long row = (long)s * H + h0 + r16;  // this lane's column (a head past H: read as the last one, not kept)
+    const bool there = h0 + r16 < H;
     ld_f32x4 acc[TILES];
 #pragma unroll
     for (int i = 0; i < TILES; ++i) acc[i] = ld_f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
     if (k0 < k1) {
-        const int* bt = a.block_table + (long)s * a.bt_stride;
         const int pieces = D / 8, per = pieces / 4;  // sixteen-byte pieces of a row (D is a multiple of 32), of a page per thread
         // Piece tid + 256 j of a page's 64 rows, which are one run of memory, lies in row (tid + 256 j) / pieces: the row and the
         // piece in it are moved on instead of divided for.  All of a page's loads are in flight together, the next page's
@@ -103,20 +101,19 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
         const int step_row = 256 / pieces, step_at = 256 % pieces, row0 = tid / pieces, at0 = tid % pieces;
         uint4 pre[LP_PIECES];
         auto fetch = [&](int kb) {
-            const uint4* page = (const uint4*)(a.k_pool + (long)bt[kb / PTA_PAGE] * PTA_PAGE * D) + tid;
+            const uint4* page = (const uint4*)(k_pool + (long)(kb == k0 ? first_page : bt[kb / PTA_PAGE]) * PTA_PAGE * D) + tid;
 #pragma unroll
             for (int j = 0; j < LP_PIECES; ++j)
                 if (j < per) pre[j] = page[256 * j];
         };
-        // Queries, scaled and rounded, once for the four waves: all asked for before the page, whose place the block table
-        // has yet to tell, and in LDS while it comes (a piece after the other behind the page: 1.1 us more, 16 heads, R = 512, 8 sequences of
-        // 64 to 700 keys)
+        // Queries, scaled and rounded, once for the four waves: all asked for before the page and in LDS while it comes (a piece after the other behind
+        // the page: 1.1 us more, 16 heads, R = 512, 8 sequences of 64 to 700 keys)
         float4 lo[LP_QUERIES], hi[LP_QUERIES];
         {
             int c = row0, e = at0;
 #pragma unroll
             for (int j = 0; j < LP_QUERIES; ++j) {
-                const float* src = a.q + ((long)s * a.H + min(h0 + min(c, 15), a.H - 1)) * D + 8 * e;
+                const float* src = queries + ((long)s * H + min(h0 + min(c, 15), H - 1)) * D + 8 * e;
                 lo[j] = *(const float4*)src, hi[j] = *(const float4*)(src + 4);
                 c += step_row, e += step_at;
                 if (e >= pieces) e -= pieces, ++c;
@@ -129,8 +126,8 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
             int c = row0, e = at0;
 #pragma unroll
             for (int j = 0; j < LP_QUERIES; ++j) {
-                const float v[8] = {lo[j].x * a.scale, lo[j].y * a.scale, lo[j].z * a.scale, lo[j].w * a.scale,
-                                    hi[j].x * a.scale, hi[j].y * a.scale, hi[j].z * a.scale, hi[j].w * a.scale};
+                const float v[8] = {lo[j].x * scale, lo[j].y * scale, lo[j].z * scale, lo[j].w * scale,
+                                    hi[j].x * scale, hi[j].y * scale, hi[j].z * scale, hi[j].w * scale};
                 if (tid + 256 * j < 16 * pieces) *(uint4*)(Qs + c * P + 8 * e) = pack8(v);
                 c += step_row, e += step_at;
                 if (e >= pieces) e -= pieces, ++c;
@@ -198,7 +195,7 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
             for (int i = 0; i < TILES; ++i) {
                 // by the transposing read: sixteen lanes give the addresses of four rows of sixteen elements and get an element of
                 // the four rows each, lanes g keys 8 g .. + 3, then + 4 .. + 7 (R is whole tiles; one past it reads the last again)
-                const bf16_t* vr = Ks + (g * 8 + (r16 >> 2)) * P + min((wave * TILES + i) * 16, a.R - 16) + (r16 & 3) * 4;
+                const bf16_t* vr = Ks + (g * 8 + (r16 >> 2)) * P + min((wave * TILES + i) * 16, R - 16) + (r16 & 3) * 4;
                 LdFrag v[2];
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
@@ -212,13 +209,13 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
         }
     }
     if (!there) return;
-    const long at = row * a.splits + split;
-    if (wave == 0 && g == 0) a.pm[at] = m_run, a.pl[at] = l_run;
+    const long at = row * splits + split;
+    if (wave == 0 && g == 0) pm[at] = m_run, pl[at] = l_run;
     if (k0 >= k1) return;  // (its maximum says so: nothing else of it is read)
 #pragma unroll
     for (int i = 0; i < TILES; ++i) {
         const int el = (wave * TILES + i) * 16 + 4 * g;
-        if (el < a.R) *(ld_f32x4*)(a.po + at * a.R + el) = acc[i];
+        if (el < R) *(ld_f32x4*)(po + at * R + el) = acc[i];
     }
 }
 
@@ -233,9 +230,8 @@ __global__ __launch_bounds__(256) void latent_pages_kernel(const LatentPages a) 
 #define LV_AHEAD 16
 
 template <int TOK>
-__global__ __launch_bounds__(256) void latent_values_kernel(bf16_t* __restrict__ out, const float* __restrict__ po,
-                                                            const float* __restrict__ pm, const float* __restrict__ pl,
-                                                            const bf16_t* __restrict__ up_v, int M, int H, int R, int V, int splits) {
+__global__ __launch_bounds__(256) void latent_values_kernel(const bf16_t* __restrict__ up_v, const float* __restrict__ pm, const float* __restrict__ pl,
+                                                            const float* __restrict__ po, int M, int H, int R, int V, int splits, bf16_t* __restrict__ out) {
     extern __shared__ __attribute__((aligned(16))) bf16_t lat[];  // [TOK][R + 8], then weights [TOK][splits]
     const int P = R + 8, h = blockIdx.x, v0 = blockIdx.y * 32, m0 = blockIdx.z * TOK;
     float* w_s = (float*)(lat + TOK * P);
@@ -252,6 +248,15 @@ __global__ __launch_bounds__(256) void latent_values_kernel(bf16_t* __restrict__
     // a wave a token: e^(m_s - max) / sum
     for (int t = wave; t < TOK; t += 4) {
         const long row = (long)min(m0 + t, M - 1) * H + h;
+        if (splits <= 64) {  // a lane a range: both of its numbers in one trip
+            const int at = min(lane, splits - 1);
+            const float l = pl[row * splits + at], any = pm[row * splits + at], m = lane < splits ? any : -INFINITY;
+            const float top = wave_max(m), e = m == -INFINITY ? 0.f : expf(m - top), sum = wave_sum(e * l);
+            const int last = (int)wave_max(m == -INFINITY ? 0.f : (float)(lane + 1));
+            if (lane == 0) live[t] = last;
+            if (lane < splits) w_s[t * splits + lane] = e * (1.0f / sum);
+            continue;
+        }
         float top = -INFINITY, sum = 0.f;
         int last = 0;
         for (int s = lane; s < splits; s += 64) {
@@ -358,14 +363,14 @@ extern "C" int pta_latent_decode(void* out, float* po, float* pm, float* pl, con
     PTA_REQUIRE((((uintptr_t)po | (uintptr_t)q | (uintptr_t)k_pool | (uintptr_t)up_v) % 16) == 0, "latent_decode: pointers must be sixteen-byte aligned");
     hipStream_t s = (hipStream_t)stream;
     const int D = R + dr;
-    const LatentPages a{po, pm, pl, q, (const bf16_t*)k_pool, block_table, bt_stride, seq_start, H, R, D, scale, size, splits};
     const size_t lds = (size_t)(80 * (D + 8) + 16 * 72) * sizeof(bf16_t) + 128 * sizeof(float);
     const dim3 grid((H + 15) / 16, splits, M);
 #define LP(T) do { \
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(latent_pages_kernel<T>), \
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024); \
         PTA_REQUIRE(raised == hipSuccess, "latent_decode: %zu bytes of LDS were refused", lds); \
-        hipLaunchKernelGGL(latent_pages_kernel<T>, grid, dim3(256), lds, s, a); \
+        hipLaunchKernelGGL(latent_pages_kernel<T>, grid, dim3(256), lds, s, q, (const bf16_t*)k_pool, block_table, seq_start, bt_stride, size, splits, H, D, R, \
+                           scale, po, pm, pl); \
     } while (0)
     if (R <= 64) LP(1);
     else if (R <= 128) LP(2);
@@ -383,7 +388,7 @@ extern "C" int pta_latent_decode(void* out, float* po, float* pm, float* pl, con
         static const hipError_t raised = hipFuncSetAttribute(reinterpret_cast<const void*>(latent_values_kernel<T>), \
                                                              hipFuncAttributeMaxDynamicSharedMemorySize, 112 * 1024); \
         PTA_REQUIRE(raised == hipSuccess, "latent_decode: %zu bytes of LDS were refused", vlds); \
-        hipLaunchKernelGGL(latent_values_kernel<T>, vgrid, dim3(256), vlds, s, (bf16_t*)out, po, pm, pl, (const bf16_t*)up_v, M, H, R, V, splits); \
+        hipLaunchKernelGGL(latent_values_kernel<T>, vgrid, dim3(256), vlds, s, (const bf16_t*)up_v, pm, pl, po, M, H, R, V, splits, (bf16_t*)out); \
     } while (0)
     if (tok == 2) LV(2);
     else if (tok == 4) LV(4);

@@ -60,14 +60,30 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
     if (unit >= 2 * G + 2 * heads) return;
     if (unit >= 2 * G + heads) {  // a head's decays and step size
         const int h = unit - 2 * G - heads;
-        const float rate = expf(A_log[h]);
-        for (int e = lane; e < N; e += PTA_WAVE) {
-            const int at = h * N + e;
-            const float bias = dt_bias[at];
-            for (int m = m0; m < m1; ++m)
-                g[(long)m * heads * N + at] = expf(-rate * softplus_32(Io<T>::ld(a + (long)m * a_ld + at) + bias));
+        const float a_log = A_log[h];
+        // everything asked for as it lies in memory, then used: four elements of each token a lane at a time
+        const T b_raw = b[(long)(m0 + min(lane, m1 - m0 - 1)) * b_ld + h];
+        for (int e0 = lane; e0 - lane < N; e0 += 4 * PTA_WAVE) {
+            float bias[4];
+            T a_raw[4][TOK];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int at = h * N + min(e0 + r * PTA_WAVE, N - 1);
+                bias[r] = dt_bias[at];
+#pragma unroll
+                for (int t = 0; t < TOK; ++t) a_raw[r][t] = a[(long)min(m0 + t, m1 - 1) * a_ld + at];
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = e0 + r * PTA_WAVE;
+                if (e >= N) break;
+#pragma unroll
+                for (int t = 0; t < TOK; ++t)
+                    if (m0 + t < m1) g[(long)(m0 + t) * heads * N + h * N + e] = expf(-expf(a_log) * softplus_32(Io<T>::ld(&a_raw[r][t]) + bias[r]));
+            }
         }
-        if (lane < m1 - m0) beta[(long)(m0 + lane) * heads + h] = 1.0f / (1.0f + expf(-Io<T>::ld(b + (long)(m0 + lane) * b_ld + h)));
+        if (lane < m1 - m0) beta[(long)(m0 + lane) * heads + h] = 1.0f / (1.0f + expf(-Io<T>::ld(&b_raw)));
         return;
     }
     const bool is_v = unit >= 2 * G, is_q = unit < G;
@@ -77,6 +93,52 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(
     const int C = 2 * G * N + heads * P;
     // whether every input of these tokens is a row of this step: they are then asked for all at once
     const bool inside = TOK > 1 && m1 - m0 == TOK && token_seq[m0] == token_seq[m1 - 1] && m0 - cu_tokens[token_seq[m0]] >= K - 1;
+    if (TOK == 1 && KMAX <= 4 && move_tail) {  // a sequence's one token: its inputs are the tail and its own row
+        const float* tl_in = tail + (K > 1 ? (long)seq_slot[token_seq[m0]] * tail_ld : 0L);
+        float* tl = const_cast<float*>(tl_in);
+        for (int e0 = 0; e0 < len; e0 += 4 * PTA_WAVE) {
+            // the taps, the inputs before and the token's own, all on their way before the first is used or moved on (with a store of the tail behind
+            // each load the next load waited for it; 2 tokens, 16 heads of 128 in a step 7.9 -> 4.1 us)
+            float w[4][KMAX], before[4][KMAX];
+            T own[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = min(e0 + lane + r * PTA_WAVE, len - 1);
+                own[r] = src[(long)m0 * ld + e];
+#pragma unroll
+                for (int kk = 0; kk < KMAX; ++kk) {  // (fewer taps: the first again, left out below)
+                    const int k = max(kk - (KMAX - K), 0);
+                    w[r][kk] = conv[(long)k * C + c0 + e];
+                    if (kk + 1 < KMAX && K > 1) before[r][kk] = tl_in[(long)min(k, K - 2) * C + c0 + e];
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            float y[4], ss = 0.f;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int c = c0 + e0 + lane + r * PTA_WAVE;
+                y[r] = 0.f;
+                if (e0 + lane + r * PTA_WAVE >= len) continue;
+                float acc = 0.f;
+#pragma unroll
+                for (int kk = 0; kk < KMAX; ++kk) {
+                    if (kk < KMAX - K) continue;
+                    const float x = kk + 1 < KMAX ? before[r][kk] : Io<T>::ld(&own[r]);
+                    acc += w[r][kk] * x;
+                    if (kk > KMAX - K) tl[(long)(kk - 1 - (KMAX - K)) * C + c] = x;
+                }
+                y[r] = acc / (1.0f + expf(-acc));
+                ss += y[r] * y[r];
+            }
+            const float by = is_v ? 1.0f : (is_q ? q_scale : 1.0f) / sqrtf(wave_sum(ss) + norm_eps);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int e = e0 + lane + r * PTA_WAVE;
+                if (e < len) qkv[(long)m0 * C + c0 + e] = y[r] * by;
+            }
+        }
+        return;
+    }
     for (int e0 = 0; e0 < len; e0 += 4 * PTA_WAVE) {  // (heads of q and k fit one round)
         float w[4][KMAX];
 #pragma unroll
@@ -234,14 +296,17 @@ __global__ __launch_bounds__(256) void delta_step_kernel(
         for (int i = threadIdx.x; i < cnt * 4 * NPT; i += 256) {
             const int tt = i / (4 * NPT), n = i - tt * (4 * NPT);
             const int at = tt * NP + (n / NPT) * GS + n % NPT;
-            const float* row = qkv + (long)(c0 + tt) * C + kh * N + n;
-            g_s[at] = n < N ? g[((long)(c0 + tt) * heads + h) * N + n] : 0.f;
-            k_s[at] = n < N ? row[(long)G * N] : 0.f;
-            q_s[at] = n < N ? row[0] : 0.f;
+            const int in = min(n, N - 1);  // (read in any case: values that are chosen where they are loaded come one after the other)
+            const float* row = qkv + (long)(c0 + tt) * C + kh * N + in;
+            const float gv = g[((long)(c0 + tt) * heads + h) * N + in], kv = row[(long)G * N], qv = row[0];
+            g_s[at] = n < N ? gv : 0.f;
+            k_s[at] = n < N ? kv : 0.f;
+            q_s[at] = n < N ? qv : 0.f;
         }
         for (int i = threadIdx.x; i < cnt * 64; i += 256) {
             const int tt = i >> 6, pp = i & 63;
-            v_s[i] = p0 + pp < P ? qkv[(long)(c0 + tt) * C + 2 * G * N + h * P + p0 + pp] : 0.f;
+            const float vv = qkv[(long)(c0 + tt) * C + 2 * G * N + h * P + min(p0 + pp, P - 1)];
+            v_s[i] = p0 + pp < P ? vv : 0.f;
         }
         if (threadIdx.x < cnt) b_s[threadIdx.x] = beta[(long)(c0 + threadIdx.x) * heads + h];
         __syncthreads();

@@ -26,38 +26,54 @@ __global__ __launch_bounds__(64) void head_norm_rope_cache_kernel(
     const T* src = (kind == 0 ? q_in : kind == 1 ? k_in : v_in) + (long)m * in_ld + (long)head * d;
     const float* w = kind == 0 ? q_w : kind == 1 ? k_w : nullptr;
     const bool normed = kind == 2 ? v_norm != 0 : qk_norm != 0;
-    const int pos = token_pos[m];
-    float x[4], ss = 0.f;
+    // The head's elements, the norm's weights, the position and the sequence, then what hangs on those two, the page and the frequencies: all before the
+    // first is used (where each was, it was a trip of its own: 2 tokens of 16 heads of 128 on 2 in a step 4.7 -> 4.3 us)
+    float x[4], wv[4], ss = 0.f, freqs[4];
+    T raw[4];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
-        const int i = lane + r * PTA_WAVE;
-        x[r] = i < d ? Io<T>::ld(src + i) : 0.f;
+        const int i = min(lane + r * PTA_WAVE, d - 1);
+        raw[r] = src[i];
+        if (w) wv[r] = w[i];
+    }
+    const int pos = token_pos[m], seq = token_seq[m];
+    const int R = (kind != 2 && rot.inv_freq) ? rot.rotary_dim : 0, half = R >> 1;
+    // the pair that element i < R is in
+    auto pair_of = [&](int i) { return rot.pairing == PTA_PAIR_INTERLEAVED ? i >> 1 : i < half ? i : i - half; };
+    if (R) {
+        const float* freq = rot.inv_freq + (rot.inv_freq_ld ? (long)seq * rot.inv_freq_ld : 0L);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) freqs[r] = freq[pair_of(min(lane + r * PTA_WAVE, R - 1))];
+    }
+    int table = 0;
+    if (kind != 0) table = block_table[(long)seq * bt_stride + pos / PTA_PAGE];
+    __builtin_amdgcn_sched_barrier(0);
+    const long page = table;
+    const int in_page = pos % PTA_PAGE;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        x[r] = lane + r * PTA_WAVE < d ? Io<T>::ld(&raw[r]) : 0.f;
         ss += x[r] * x[r];
     }
     const float inv = normed ? rsqrtf(wave_sum(ss) / (float)d + eps) : 1.f;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int i = lane + r * PTA_WAVE;
-        if (i < d) x[r] = x[r] * inv * (w ? w[i] : 1.f);
+        if (i < d) x[r] = x[r] * inv * (w ? wv[r] : 1.f);
         y_s[i] = i < d ? x[r] : 0.f;
     }
     __syncthreads();
-    const int R = (kind != 2 && rot.inv_freq) ? rot.rotary_dim : 0, half = R >> 1;
-    const float* freq = R ? rot.inv_freq + (rot.inv_freq_ld ? (long)token_seq[m] * rot.inv_freq_ld : 0L) : nullptr;
-    long page = 0;
-    if (kind != 0) page = block_table[(long)token_seq[m] * bt_stride + pos / PTA_PAGE];
-    const int in_page = pos % PTA_PAGE;
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
         const int i = lane + r * PTA_WAVE;
         if (i >= D) continue;
         float y = i < d ? x[r] : 0.f;
         if (i < R) {
-            int p, other;  // the pair's index, and the element this one is rotated with
-            float sign;    // -1 for the pair's first element, +1 for its second
-            if (rot.pairing == PTA_PAIR_INTERLEAVED) { p = i >> 1; other = i ^ 1; sign = (i & 1) ? 1.f : -1.f; }
-            else { p = i < half ? i : i - half; other = i < half ? i + half : i - half; sign = i < half ? -1.f : 1.f; }
-            const float ang = (float)pos * freq[p];
+            int other;   // the element this one is rotated with
+            float sign;  // -1 for the pair's first element, +1 for its second
+            if (rot.pairing == PTA_PAIR_INTERLEAVED) { other = i ^ 1; sign = (i & 1) ? 1.f : -1.f; }
+            else { other = i < half ? i + half : i - half; sign = i < half ? -1.f : 1.f; }
+            const float ang = (float)pos * freqs[r];
             y = y * (cosf(ang) * rot.cs_scale) + sign * y_s[other] * (sinf(ang) * rot.cs_scale);
         }
         if (kind == 0) Io<T>::st(q_out + ((long)m * nh + head) * D + i, y);

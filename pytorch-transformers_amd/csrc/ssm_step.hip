@@ -47,11 +47,15 @@ __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __res
     constexpr int MINE = (MOST + 63) / 64;  // with one head a group
     constexpr int AHEAD = 2;                // of a thread with seven heads and more
     auto channel = [&](int i) { return i < per * P ? g * per * P + i : i < per * P + N ? inner + g * N + i - per * P : inner + (a.G + g) * N + i - per * P - N; };
-    float w[AHEAD][K], old[AHEAD][K - 1], now[AHEAD], bias[AHEAD];
+    // (as they lie in memory, and a bias from somewhere where there is none: a value widened, or chosen, where it is loaded is waited for
+    // there, one channel behind the other and the state behind them all)
+    float w[AHEAD][K], old[AHEAD][K - 1], bias[AHEAD];
+    T now[AHEAD], z_raw[4];
+    const float* biases = a.conv_b ? a.conv_b : a.conv_w;
     auto fetch = [&](int u, int i) {
         const int c = channel(min(i, channels - 1));
-        now[u] = Io<T>::ld(row + inner + c);
-        bias[u] = a.conv_b ? a.conv_b[c] : 0.f;
+        now[u] = row[inner + c];
+        bias[u] = biases[c];
 #pragma unroll
         for (int k = 0; k < K; ++k) w[u][k] = a.conv_w[(long)c * K + k];
 #pragma unroll
@@ -60,21 +64,23 @@ __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __res
     auto form = [&](int u, int i) {
         if (i >= channels) return;
         const int c = channel(i);
-        float acc = bias[u];
+        float acc = a.conv_b ? bias[u] : 0.f;
+        const float x = Io<T>::ld(&now[u]);
 #pragma unroll
         for (int k = 0; k + 1 < K; ++k) acc += w[u][k] * old[u][k];
-        acc += w[u][K - 1] * now[u];
+        acc += w[u][K - 1] * x;
         chan[i] = acc / (1.0f + expf(-acc));
 #pragma unroll
-        for (int k = 0; k + 1 < K; ++k) tail[(long)k * C + c] = k + 2 < K ? old[u][k + 1] : now[u];
+        for (int k = 0; k + 1 < K; ++k) tail[(long)k * C + c] = k + 2 < K ? old[u][k + 1] : x;
     };
 #pragma unroll
     for (int u = 0; u < AHEAD; ++u) fetch(u, threadIdx.x + u * blockDim.x);
-    const float dt_raw = Io<T>::ld(row + inner + C + h), A = a.A_log[h], dt_b = a.dt_bias[h], skip = a.D[h];
-    float z[4], nw[4];
+    const T dt_raw = row[inner + C + h];
+    const float A = a.A_log[h], dt_b = a.dt_bias[h], skip = a.D[h];
+    float nw[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        z[e] = Io<T>::ld(row + h * P + col + e);
+        z_raw[e] = row[h * P + col + e];
         nw[e] = a.norm_w[h * P + col + e];
     }
     __builtin_amdgcn_sched_barrier(0);
@@ -92,7 +98,7 @@ __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __res
     __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    const float dt = step_softplus(dt_raw + dt_b), dA = expf(-expf(A) * dt);
+    const float dt = step_softplus(Io<T>::ld(&dt_raw) + dt_b), dA = expf(-expf(A) * dt);
     const float4 xv = *reinterpret_cast<const float4*>(chan + wave * P + col);
     const float4 dx = make_float4(dt * xv.x, dt * xv.y, dt * xv.z, dt * xv.w);
     const float4* B = reinterpret_cast<const float4*>(chan + per * P + q * NPT);
@@ -111,7 +117,8 @@ __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __res
     float v[4], ss = 0.f;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-        v[e] = y[e] * (z[e] / (1.0f + expf(-z[e])));
+        const float z = Io<T>::ld(&z_raw[e]);
+        v[e] = y[e] * (z / (1.0f + expf(-z)));
         ss += v[e] * v[e];
     }
     ss = wave_sum(q == 0 ? ss : 0.f);  // (the four quarters hold the same columns' results)
