@@ -75,12 +75,12 @@ __device__ __forceinline__ void attend(const AttnRide& ride, int t) {
 }
 
 template <int MT, int RT, bool ROT, int KS>
-__global__ __launch_bounds__(SK_THREADS, RT == 2 ? 1 : MT > 2 ? 2 : 3) void gemm_splitk_attn_kernel(SplitkProblem pa, SplitkProblem pb, int M,
+__global__ __launch_bounds__(SK_WAVES * 64, RT == 2 ? 1 : MT > 2 ? 2 : 3) void gemm_splitk_attn_kernel(SplitkProblem pa, SplitkProblem pb, int M,
                                                                                                    int rot_stride, AttnRide ride) {
     __shared__ int seen;
     if ((int)blockIdx.x < ride.owners) return attend<KS>(ride, blockIdx.x);
     const int block = (int)blockIdx.x - ride.owners, blocks = pa.tiles * pa.parts + pb.tiles * pb.parts;
-    if (splitk_body<MT, RT, 4, ROT>(pa, pb, M, 1, M, rot_stride, block, blocks, RideGate{ride, &seen})) return;
+    if (splitk_body<MT, RT, 4, ROT, SK_WAVES>(pa, pb, M, 1, M, rot_stride, block, blocks, RideGate{ride, &seen})) return;
     for (int t = 0; t < ride.tasks; ++t) {
         if (threadIdx.x == 0) seen = is_done(ride.sync + t);
         __syncthreads();
@@ -89,17 +89,17 @@ __global__ __launch_bounds__(SK_THREADS, RT == 2 ? 1 : MT > 2 ? 2 : 3) void gemm
         if (!done) attend<KS>(ride, t);
     }
     __syncthreads();
-    splitk_body<MT, RT, 4, ROT>(pa, pb, M, 1, M, rot_stride, block, blocks, NoGate{});
+    splitk_body<MT, RT, 4, ROT, SK_WAVES>(pa, pb, M, 1, M, rot_stride, block, blocks, NoGate{});
 }
 
 template <int MT, int RT, int KS>
 static int launch(const SplitkProblem& a, const SplitkProblem& b, int M, bool rotate, int rot_stride, const AttnRide& ride, hipStream_t s) {
-    constexpr int stages = 4 * splitk_slot(MT, RT), keys = (int)key_split_lds(RIDE_HEAD, 1, KS), lds = stages > keys ? stages : keys;
+    constexpr int stages = 4 * splitk_slot(MT, RT, SK_WAVES), keys = (int)key_split_lds(RIDE_HEAD, 1, KS), lds = stages > keys ? stages : keys;
     static_assert(lds <= 158 * 1024, "the stages must fit the LDS of a compute unit");
     auto kern = rotate ? gemm_splitk_attn_kernel<MT, RT, true, KS> : gemm_splitk_attn_kernel<MT, RT, false, KS>;
     if (lds > 60 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return pta_fail("gemm_splitk_pair_attn: cannot have %d bytes of LDS", lds);
-    hipLaunchKernelGGL(kern, dim3(ride.owners + a.tiles * a.parts + b.tiles * b.parts), dim3(SK_THREADS), lds, s, a, b, M, rot_stride, ride);
+    hipLaunchKernelGGL(kern, dim3(ride.owners + a.tiles * a.parts + b.tiles * b.parts), dim3(SK_WAVES * 64), lds, s, a, b, M, rot_stride, ride);
     return pta_check_launch("gemm_splitk_pair_attn");
 }
 

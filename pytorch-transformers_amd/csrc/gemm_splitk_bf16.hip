@@ -30,10 +30,10 @@
 #include <utility>
 #include <vector>
 
-template <int MT, int RT, int D, bool ROT>
-__global__ __launch_bounds__(SK_THREADS) void gemm_splitk_kernel(SplitkProblem pa, SplitkProblem pb, int M, int chunks,
+template <int MT, int RT, int D, bool ROT, int NW>
+__global__ __launch_bounds__(NW * 64) void gemm_splitk_kernel(SplitkProblem pa, SplitkProblem pb, int M, int chunks,
                                                                  int chunk_rows, int rot_stride) {
-    splitk_body<MT, RT, D, ROT>(pa, pb, M, chunks, chunk_rows, rot_stride, (int)blockIdx.x, (int)gridDim.x, NoGate{});
+    splitk_body<MT, RT, D, ROT, NW>(pa, pb, M, chunks, chunk_rows, rot_stride, (int)blockIdx.x, (int)gridDim.x, NoGate{});
 }
 
 // The same sums for rows too long for 32-bit offsets within a wave's rows of W (32 rows of 2^25 elements, 16 of 2^26), at most 31 of x: a
@@ -202,6 +202,12 @@ extern "C" int pta_gemm_splitk_parts(int N, int K, int parts, int rt) {
     return effective_parts(K, parts > 0 ? parts : pick_parts(N, K, rt));
 }
 
+// How a pair runs: 1 or 2, workgroups of four waves with so many tiles of sixteen rows of W each; 3, with stationary activations; 4, of six waves with
+// a tile each.
+#define PAIR_STATIONARY 3
+#define PAIR_SIX 4
+static int tile_rows(int kind) { return kind == PAIR_SIX ? 16 * SK_SIX : 64 * kind; }  // of W, of a workgroup
+
 static SplitkProblem make_problem(void* y, float* part, const void* x, const void* W, const float* bias,
                                   const void* add1, const void* add2, int N, int K, int act, int out_f32, int rt,
                                   int parts, int reduce) {
@@ -212,7 +218,7 @@ static SplitkProblem make_problem(void* y, float* part, const void* x, const voi
     const int nkb = (K + 63) / 64;
     p.blocks_per_part = (nkb + parts - 1) / parts;
     p.parts = (nkb + p.blocks_per_part - 1) / p.blocks_per_part;  // ranges that are not empty
-    p.tiles = (N + 64 * rt - 1) / (64 * rt);
+    p.tiles = (N + tile_rows(rt) - 1) / tile_rows(rt);
     p.direct = reduce && p.parts == 1;
     return p;
 }
@@ -239,14 +245,14 @@ static bool rotated(const SplitkProblem& a, const SplitkProblem& b) {
 // (x lies within 32-bit offsets: check_splitk)
 static bool rows_too_long(const SplitkProblem& a, const SplitkProblem& b, int rt) { return (long)std::max(a.K, b.K) * 16 * rt * 2 >= LDS_PAST; }
 
-template <int MT, int RT>
+template <int MT, int RT, int NW = SK_WAVES>
 static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int reduce, hipStream_t s) {
     constexpr int D = 4;  // stages in LDS
-    constexpr int lds = D * splitk_slot(MT, RT);
+    constexpr int lds = D * splitk_slot(MT, RT, NW);
     static_assert(lds <= 160 * 1024, "the stages must fit the LDS of a compute unit");
     const int rot_stride = rotation_stride();
     const bool rotate = rotated(a, b);
-    auto kern = rotate ? gemm_splitk_kernel<MT, RT, D, true> : gemm_splitk_kernel<MT, RT, D, false>;
+    auto kern = rotate ? gemm_splitk_kernel<MT, RT, D, true, NW> : gemm_splitk_kernel<MT, RT, D, false, NW>;
     if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)
         return pta_fail("gemm_splitk_bf16: cannot have %d bytes of LDS", lds);
     if (rows_too_long(a, b, RT)) {
@@ -257,7 +263,7 @@ static int launch_cfg(const SplitkProblem& a, const SplitkProblem& b, int M, int
     // rows beyond the MT tiles of a workgroup go to further chunks of workgroups, all of the same size
     const int chunks = (M + MT * 16 - 1) / (MT * 16), chunk_rows = ((M + chunks - 1) / chunks + 15) / 16 * 16;
     const dim3 grid((a.tiles * a.parts + b.tiles * b.parts) * chunks);
-    hipLaunchKernelGGL(kern, grid, dim3(SK_THREADS), lds, s, a, b, M, chunks, chunk_rows, rot_stride);
+    hipLaunchKernelGGL(kern, grid, dim3(NW * 64), lds, s, a, b, M, chunks, chunk_rows, rot_stride);
     return reduce_parts(a, M, reduce, s);
 }
 
@@ -351,7 +357,7 @@ extern "C" int pta_gemm_splitk_pair_fix(int N1, int K1, int N2, int K2, int p1, 
         pair_parts_fixed.erase(key);
         return 0;
     }
-    if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2)) return 1;
+    if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2 && rt != PAIR_SIX)) return 1;
     pair_parts_fixed[key] = {{p1, p2, rt}, {p1, p2, rt}};
     return 0;
 }
@@ -363,7 +369,7 @@ extern "C" int pta_gemm_splitk_pair_fix_parts(int N1, int K1, int N2, int K2, in
 // The same for steps of 33 to 64 rows alone, of matrices for which those have ranges of their own (else 1).
 extern "C" int pta_gemm_splitk_pair_fix_middle(int N1, int K1, int N2, int K2, int p1, int p2, int rt) {
     if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || !staged_middle(N1, N2)) return 1;
-    if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2)) return 1;
+    if (!parts_valid(K1, p1) || !parts_valid(K2, p2) || (rt != 1 && rt != 2 && rt != PAIR_SIX)) return 1;
     std::lock_guard<std::mutex> hold(pair_parts_lock);
     pair_parts_fixed[{N1, K1, N2, K2}].middle = {p1, p2, rt};  // (a new entry's others are the rule's)
     return 0;
@@ -379,7 +385,7 @@ extern "C" int pta_gemm_splitk_pair_fix_middle(int N1, int K1, int N2, int K2, i
 //   4,096 x 4,096 + 4,096 x 16,384   36.5 -> 32.9   39.2 -> 33.8   41.4 -> 39.6    8,192 x 8,192 + 32,768    117.9 -> 111.8   127.7 -> 118.4   141.2 -> 139.7
 //   2,048 x 2,048 + 2,048 x 8,192    11.2 -> 10.5   12.8 -> 11.1   15.2 -> 13.3    7,680 + 20,480 x 5,120     54.3 -> 52.6    58.6 -> 60.2    71.6 -> 66.3
 static double pair_us(int N1, int K1, int a, int N2, int K2, int b, int rt, int rows) {
-    const int units = max(1, pta_compute_units()), slots = units * (rt == 1 ? (rows <= 32 ? 3 : 2) : rows <= 16 ? 2 : 1);
+    const int units = max(1, pta_compute_units()), slots = units * (rt == 1 ? (rows <= 32 ? 3 : 2) : rows <= 16 && rt == 2 ? 2 : 1);
     const double fixed = 6.0;
     struct Run { int count; double blocks; } runs[4];
     int n = 0;
@@ -387,7 +393,7 @@ static double pair_us(int N1, int K1, int a, int N2, int K2, int b, int rt, int 
     double total = 0.0, longest = 0.0, uneven = 0.0;
     for (int i = 0; i < 2; ++i) {
         const int N = i ? N2 : N1, K = i ? K2 : K1, p = i ? b : a;
-        const int nkb = (K + 63) / 64, per = (nkb + p - 1) / p, parts = (nkb + per - 1) / per, tiles = (N + 64 * rt - 1) / (64 * rt);
+        const int nkb = (K + 63) / 64, per = (nkb + p - 1) / p, parts = (nkb + per - 1) / per, tiles = (N + tile_rows(rt) - 1) / tile_rows(rt);
         runs[n++] = Run{tiles * (parts - 1), per + fixed};
         runs[n++] = Run{tiles, nkb - (parts - 1) * per + fixed};
         groups += (long)tiles * parts;
@@ -404,11 +410,15 @@ static double pair_us(int N1, int K1, int a, int N2, int K2, int b, int rt, int 
     const double mean = total / units;
     double most = *std::max_element(load.begin(), load.end());
     if (groups > slots) most = std::max(most, mean + 0.5 * longest);
-    const double bytes = 8192.0 * rt + 0.2 * 4096.0 * (((rows + 15) / 16 + 1) / 2);  // of a block: rows of W, and of x, which come from near by
+    const double bytes = 128.0 * tile_rows(rt) + 0.2 * 4096.0 * (((rows + 15) / 16 + 1) / 2);  // of a block: rows of W, and of x, which come from near by
     return 4.0 + (1.0 + 0.02 * uneven) * std::max(most * bytes / 26e3, mean * bytes / 22.5e3) + ((double)a * N1 + (double)b * N2) * rows * 4.0 / 3e6;
 }
 
-// Ranges, and tiles of sixteen rows of W a wave, for steps of up to 32 rows (one tile) or of 33 to 64; kept by shape
+// Ranges, and tiles of sixteen rows of W a wave, for steps of up to 32 rows (one tile) or of 33 to 64; kept by shape.  96 rows of W on six waves, at 33 to 64
+// rows, are for where 64 or 128 leave compute units idle or with twice the rows of others, as a unit pulls some 25 GB/s whatever is on its
+// way: 4,672 + 18,176 x 4,544 (179 workgroups of 128 rows, 239 of 96), us at 33 / 48 / 64 rows 41.2 -> 38.7, 43.0 -> 39.4, 45.6 -> 41.5; 6,144 + 16,384 x 4,096
+// 38.1 -> 37.7, 38.7 -> 38.3, 40.6 -> 39.5.  They read x more often, and are taken where the time says 5 % less: at 4 % less (4,544 x 4,544 + 18,176) they
+// are 2 % the faster at 33 rows and none at 64, at none less (9,216 + 32,768 x 8,192) 3 % the slower.
 static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
     static std::map<std::array<int, 5>, PairChoice> known;
     const std::array<int, 5> key{N1, K1, N2, K2, rows};
@@ -417,13 +427,15 @@ static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
     if (it != known.end()) return it->second;
     PairChoice best{1, 1, 1};
     double us = 1e30;
-    for (int rt = 1; rt <= (rows > 32 ? 2 : 1); ++rt)
+    for (int rt : {1, 2, PAIR_SIX}) {
+        if (rt > 1 && rows <= 32) continue;
         for (int a = 1; a <= 8; ++a)
             for (int b = 1; b <= 16; ++b) {
                 if (!parts_valid(K1, a) || !parts_valid(K2, b)) continue;
                 const double t = pair_us(N1, K1, a, N2, K2, b, rt, rows);
-                if (t < us) us = t, best = PairChoice{a, b, rt};
+                if (t < (rt == PAIR_SIX ? 0.95 * us : us)) us = t, best = PairChoice{a, b, rt};
             }
+    }
     if (known.size() >= 1024) known.clear();
     return known[key] = best;
 }
@@ -440,7 +452,7 @@ static int pick_pair_parts(int N1, int K1, int N2, int K2, int M, int* p1, int* 
     if (c.p1 == 0) c = pair_rule(N1, K1, N2, K2, middle ? 64 : 32);
     *p1 = c.p1;
     *p2 = c.p2;
-    return M > 32 ? c.rt : 1;
+    return M <= 32 || (M > 64 && c.rt == PAIR_SIX) ? 1 : c.rt;
 }
 
 // Steps of up to 128 rows may run with the activations stationary (gemm_stationary_bf16.hip), which cuts K into
@@ -524,7 +536,7 @@ static int pick_pair_parts_rows(int N1, int K1, int N2, int K2, int M, int* p1, 
         if (q1 > 0 && q2 > 0) {
             *p1 = q1;
             *p2 = q2;
-            return 3;
+            return PAIR_STATIONARY;
         }
     }
     return pick_pair_parts(N1, K1, N2, K2, M, p1, p2);
@@ -559,9 +571,10 @@ extern "C" int pta_gemm_splitk_pair_bf16(float* part1, const void* x1, const voi
     PTA_REQUIRE(part1 && part2, "gemm_splitk_pair_bf16: null workspace");
     int p1, p2;
     const int kind = pick_pair_parts_rows(N1, K1, N2, K2, M, &p1, &p2);
-    if (kind == 3) return pta_gemm_stationary_pair_bf16(part1, x1, W1, N1, K1, p1, part2, x2, W2, N2, K2, p2, M, stream);
+    if (kind == PAIR_STATIONARY) return pta_gemm_stationary_pair_bf16(part1, x1, W1, N1, K1, p1, part2, x2, W2, N2, K2, p2, M, stream);
     const SplitkProblem a = make_problem(nullptr, part1, x1, W1, nullptr, nullptr, nullptr, N1, K1, 0, 0, kind, p1, 0);
     const SplitkProblem b = make_problem(nullptr, part2, x2, W2, nullptr, nullptr, nullptr, N2, K2, 0, 0, kind, p2, 0);
+    if (kind == PAIR_SIX) return M <= 48 ? launch_cfg<3, 1, SK_SIX>(a, b, M, 0, (hipStream_t)stream) : launch_cfg<4, 1, SK_SIX>(a, b, M, 0, (hipStream_t)stream);
     if (kind == 2) return launch_rows<2>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
     return launch_rows<1>(tiles_per_chunk(M), a, b, M, 0, (hipStream_t)stream);
 }
@@ -574,7 +587,9 @@ extern "C" int pta_gemm_splitk_pair_attn_ok(int N1, int K1, int N2, int K2, int 
         return 0;
     int p1, p2;
     const int rt = pick_pair_parts_rows(N1, K1, N2, K2, M, &p1, &p2);
-    return rt != 3 && (long)std::max(K1, K2) * 32 * 2 < LDS_PAST;
+    // (Workgroups of six waves are one a compute unit and fill the chip: attention's would take the places of the second product's, whose 71 blocks then
+    // start late.  64 sequences of 60 keys, 71 heads on one, 4,544 x 4,544 and 4,544 x 18,176: 50 us, with workgroups of 128 rows 48.)
+    return rt != PAIR_STATIONARY && rt != PAIR_SIX && (long)std::max(K1, K2) * 32 * 2 < LDS_PAST;
 }
 
 // The pair with the attention that its second product takes (x2 [M, nh d] is written here): pta_attn_mfma of one token a sequence,

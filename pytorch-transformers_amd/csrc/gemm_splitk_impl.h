@@ -6,10 +6,11 @@
 #include "lds_stream.h"
 #include "pta_kernels.h"
 
-// bytes of a stage of 64 elements of K in LDS: four waves' rows of W, and the rows of x by whole loads of each wave
-static constexpr __host__ __device__ int splitk_slot(int MT, int RT) { return RT * 8192 + (MT + 1) / 2 * 4096; }
+// bytes of a stage of 64 elements of K in LDS: the waves' rows of W, and the rows of x by whole loads of each wave (NW: waves, an even number)
+static constexpr __host__ __device__ int splitk_slot(int MT, int RT, int NW) { return NW * RT * 2048 + (2 * MT + NW - 1) / NW * NW * 1024; }
 
-#define SK_THREADS 256
+#define SK_WAVES 4
+#define SK_SIX 6  // waves of a workgroup that has 96 rows of W
 #define SK_CHUNK_ROWS 128  // eight tiles of sixteen rows of x: what a workgroup holds
 #define SK_MAX_ROWS 256
 
@@ -50,12 +51,13 @@ struct NoGate {
 
 // Workgroup `block` of `blocks`.  With a gate that may be closed, x is asked for once the gate is open, and W of the first stages before
 // that; false where the gate has used LDS meanwhile and the workgroup is to be begun again.
-template <int MT, int RT, int D, bool ROT, typename Gate>
+template <int MT, int RT, int D, bool ROT, int NW, typename Gate>
 __device__ __forceinline__ bool splitk_body(const SplitkProblem& pa, const SplitkProblem& pb, int M, int chunks, int chunk_rows,
                                             int rot_stride, int block, int blocks, const Gate& gate) {
-    constexpr int NX = (MT + 1) / 2;                 // loads of x per wave and stage (eight rows by 128 bytes each)
+    constexpr int NX = (2 * MT + NW - 1) / NW;       // loads of x per wave and stage (eight rows by 128 bytes each)
     constexpr int NL = 2 * RT + NX;                  // all of a wave's loads per stage
-    constexpr int SLOT = splitk_slot(MT, RT);        // a stage in LDS: the four waves' rows of W, then x
+    constexpr int SLOT = splitk_slot(MT, RT, NW);    // a stage in LDS: the waves' rows of W, then x
+    static_assert(NW % 2 == 0, "a wave's loads of x are all the same half of a tile");
     extern __shared__ __attribute__((aligned(1024))) char lds[];  // [D][SLOT]
 
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -91,7 +93,7 @@ __device__ __forceinline__ bool splitk_body(const SplitkProblem& pa, const Split
     const int tiles = second ? pb.tiles : pa.tiles;
     const int idx = block - (second ? first_blocks : 0);
     const int tile = idx % tiles, range = idx / tiles;  // neighbours share a range of K: its x slice stays in L2
-    const int n_base = tile * (64 * RT) + wave * (16 * RT);
+    const int n_base = tile * (NW * 16 * RT) + wave * (16 * RT);
     const int nkb = (K + 63) >> 6;
     const int kb0 = range * blocks_per_part, kb1 = min(kb0 + blocks_per_part, nkb);
     const int k_begin = kb0 * 64, k_end = min(kb1 * 64, K);
@@ -101,13 +103,13 @@ __device__ __forceinline__ bool splitk_body(const SplitkProblem& pa, const Split
     const int n_rows = max(0, min(16 * RT, N - n_base));
     const i32x4_t rw = buffer_of(W + (long)min(n_base, N - 1) * K, n_rows * K * 2), rx = buffer_of(x + (long)m0 * K, (m_end - m0) * K * 2);
     const unsigned to_w = __builtin_amdgcn_readfirstlane(lds_address(lds)) + wave * (RT * 2048);
-    const unsigned to_x = __builtin_amdgcn_readfirstlane(lds_address(lds)) + RT * 8192 + wave * 1024;
+    const unsigned to_x = __builtin_amdgcn_readfirstlane(lds_address(lds)) + NW * RT * 2048 + wave * 1024;
     int w_at[2 * RT], x_at[NX];  // the lane's rows
 #pragma unroll
     for (int l = 0; l < 2 * RT; ++l) w_at[l] = ((l >> 1) * 16 + stream_row(lane, l & 1)) * K * 2;
 #pragma unroll
     for (int l = 0; l < NX; ++l) {
-        const int row = (wave + 4 * l) * 8 + (lane >> 3);
+        const int row = (wave + NW * l) * 8 + (lane >> 3);
         x_at[l] = row < m_end - m0 ? row * K * 2 : LDS_PAST;
     }
     const int c8[2] = {stream_element(lane, 0), stream_element(lane, 1)};
@@ -141,7 +143,7 @@ __device__ __forceinline__ bool splitk_body(const SplitkProblem& pa, const Split
 #pragma unroll
         for (int l = 0; l < NX; ++l) {
             const int ke = k + c8[wave & 1];  // (an even number of loads away from the wave's first: the same half of a tile)
-            fetch16(rx, to_x + slot + l * 4096, ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
+            fetch16(rx, to_x + slot + l * (NW * 1024), ke < k_end && x_at[l] != LDS_PAST ? x_at[l] + ke * 2 : LDS_PAST);
         }
     };
     auto issue = [&](int stage, int slot) {
@@ -157,7 +159,7 @@ __device__ __forceinline__ bool splitk_body(const SplitkProblem& pa, const Split
 #pragma unroll
             for (int t = 0; t < RT; ++t) w[t] = *reinterpret_cast<const bf16x8_t*>(lds + at + (wave * RT + t) * 2048);
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) b[mt] = *reinterpret_cast<const bf16x8_t*>(lds + at + RT * 8192 + mt * 2048);
+            for (int mt = 0; mt < MT; ++mt) b[mt] = *reinterpret_cast<const bf16x8_t*>(lds + at + NW * RT * 2048 + mt * 2048);
 #pragma unroll
             for (int t = 0; t < RT; ++t)
 #pragma unroll

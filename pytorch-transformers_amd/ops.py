@@ -1348,7 +1348,7 @@ def gemm_splitk_pair_parts(N1: int, K1: int, N2: int, K2: int, M: int = 0):
 
 def gemm_splitk_pair_way(N1: int, K1: int, N2: int, K2: int, M: int):
     """``gemm_splitk_pair_parts``, and how the launch runs: 1 or 2, the kernel that walks K in stages with so many tiles of
-    sixteen rows of W a wave; 3, with stationary activations."""
+    sixteen rows of W a wave; 3, with stationary activations; 4, the first of these by workgroups of six waves with a tile each."""
     p1, p2, way = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_int(0)
     _call("pta_gemm_splitk_pair_way", int(N1), int(K1), int(N2), int(K2), int(M), ctypes.byref(p1), ctypes.byref(p2), ctypes.byref(way))
     return p1.value, p2.value, way.value

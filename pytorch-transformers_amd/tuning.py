@@ -739,9 +739,10 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
     near = lambda a0, b0: [(a, b, 1) for a in range(max(1, a0 - 1), a0 + 3) for b in range(max(1, b0 - 2), b0 + 3)]
     tall = lambda a0, b0: [(a, b, 2) for a in sorted({max(1, a0 - 1), a0, a0 + 1, max(1, 2 * a0 - 1), 2 * a0, 2 * a0 + 1})
                            for b in sorted({max(1, b0 - 1), b0, b0 + 1, max(1, 2 * b0 - 1), 2 * b0, 2 * b0 + 1})]
+    six = lambda a0, b0: [(a, b, 4) for a in range(max(1, a0 - 1), a0 + 2) for b in range(max(1, b0 - 1), b0 + 2)]
     ways = lambda rule, others: [rule] + [c for c in dict.fromkeys(others) if c != rule and fix(c) == 0]  # those that the kernel takes
     few_ways = ways(few, near(*few[:2]))
-    middle_ways = ways(middle, near(*middle[:2]) + near(*few[:2]) + tall(*middle[:2]) + tall(*few[:2])) if middle else []
+    middle_ways = ways(middle, near(*middle[:2]) + near(*few[:2]) + tall(*middle[:2]) + tall(*few[:2]) + six(*middle[:2])) if middle else []
     larger = min(64, max(41, PAIR_TUNE_ROWS))
     counts = {rows: [torch.randn((rows, K), dtype=torch.float32, device=w1.device).to(torch.bfloat16) for K in (K1, K2)]
               for rows in sorted({*class_rows, 40, larger})}
