@@ -1385,7 +1385,9 @@ def gemm_splitk_pair_partial(x1: torch.Tensor, w1: torch.Tensor, x2: torch.Tenso
 
 
 def gemm_splitk_pair_attn_ok(x1: torch.Tensor, w1: torch.Tensor, late: LateAttention, w2: torch.Tensor) -> bool:
-    """Whether ``gemm_splitk_pair_attn`` has a launch for these (which ``gemm_partial_pair_ok`` takes, with ``late.out`` as the second input)."""
+    """Whether ``gemm_splitk_pair_attn`` has a launch for these (which ``gemm_partial_pair_ok`` takes, with ``late.out`` as the second input).
+    A pair that has not been timed is timed here, while timing is on: the answer depends on what that chooses."""
+    tuning.tune_pair_parts(w1, w2)
     _, nh, d = late.q.shape
     return bool(load_library().pta_gemm_splitk_pair_attn_ok(w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], x1.shape[0], nh,
                                                             late.k_pool.shape[1], d))
@@ -1414,7 +1416,6 @@ def gemm_splitk_pair_attn(x1: torch.Tensor, w1: torch.Tensor, late: LateAttentio
         _need(sink, "sink", torch.float32, (nh,))
     bias_scale = how.get("bias_scale")
     bias = _score_bias_arg(late.slopes, nh, how.get("bias_of", "key"), not how.get("alibi_exact", False), d ** -0.5 if bias_scale is None else bias_scale)
-    tuning.tune_pair_parts(w1, w2)
     p1, p2 = gemm_splitk_pair_parts(N1, K1, N2, K2, M)
     part1 = torch.empty((p1, M, N1), dtype=torch.float32, device=q.device)
     part2 = torch.empty((p2, M, N2), dtype=torch.float32, device=q.device)

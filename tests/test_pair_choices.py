@@ -86,3 +86,40 @@ def test_a_class_of_rows_leaves_the_others(table, shape, cls):
     finally:
         fix(*shape, -1, 0, 0)
     assert _ranges(shape, *rows) == plain
+
+
+@pytest.mark.parametrize("rows,fix", [(40, "six"), (64, "six"), (64, "stationary"), (8, "stationary")])
+def test_whether_attention_rides_is_asked_once_the_pair_is_timed(monkeypatch, rows, fix):
+    """Timing may give the pair a launch that carries no attention: the answer has to be the one that holds after it."""
+    import types
+
+    import torch
+    from pytorch_transformers_amd import ops, tuning
+
+    (N1, K1), (N2, K2) = shapes = (4544, 18176), (4544, 4544)
+    lib = ops.load_library()
+    empty = lambda *shape: torch.empty(shape, dtype=torch.bfloat16, device="meta")
+    x1, w1, w2 = empty(rows, K1), empty(N1, K1), empty(N2, K2)
+    late = types.SimpleNamespace(q=empty(rows, 71, 64), k_pool=empty(1, 1, 64, 64))
+    cls = [16, 32, 64, 128].index(min(n for n in (16, 32, 64, 128) if n >= rows))
+
+    def timed(*weights):
+        assert [tuple(w.shape) for w in weights] == list(shapes)
+        if fix == "six":
+            assert lib.pta_gemm_splitk_pair_fix_stationary(N1, K1, N2, K2, cls, 0, 0) == 0
+            assert lib.pta_gemm_splitk_pair_fix_middle(N1, K1, N2, K2, 3, 1, 4) == 0
+        else:
+            assert lib.pta_gemm_splitk_pair_fix_stationary(N1, K1, N2, K2, cls, 4, 1) == 0
+
+    before = ops.gemm_splitk_pair_way(N1, K1, N2, K2, rows)
+    try:
+        assert lib.pta_gemm_splitk_pair_fix(N1, K1, N2, K2, 1, 1, 1) == 0
+        assert lib.pta_gemm_splitk_pair_fix_stationary(N1, K1, N2, K2, cls, 0, 0) == 0
+        monkeypatch.setattr(tuning, "tune_pair_parts", lambda *weights: None)
+        assert ops.gemm_splitk_pair_attn_ok(x1, w1, late, w2)
+        monkeypatch.setattr(tuning, "tune_pair_parts", timed)
+        assert not ops.gemm_splitk_pair_attn_ok(x1, w1, late, w2)
+    finally:
+        lib.pta_gemm_splitk_pair_fix(N1, K1, N2, K2, 0, 0, 1)
+        lib.pta_gemm_splitk_pair_fix_stationary(N1, K1, N2, K2, -1, 0, 0)
+    assert ops.gemm_splitk_pair_way(N1, K1, N2, K2, rows) == before
