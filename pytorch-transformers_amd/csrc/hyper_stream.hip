@@ -235,8 +235,8 @@ __global__ __launch_bounds__(1024) void hyper_norm_once_kernel(const float* __re
     if (a.u_out && live) Vec<V>::st(a.u_out + (long)m * H + i, u);
     if (!normed) return;
 #pragma unroll
-    for (int v = 0; v < V; ++v) ss += live ? u[v] * u[v] : 0.f;
-    const float inv = 1.0f / sqrtf(block_sum(ss, red, waves) / (float)H + a.eps);
+    for (int v = 0; v < V; ++v) ss = __builtin_fmaf(u[v], u[v], ss);  // (with a choice in the sum it would be a product and an addition: other bits than the loop's)
+    const float inv = 1.0f / sqrtf(block_sum(live ? ss : 0.f, red, waves) / (float)H + a.eps);
     if (!live) return;
     float n[V], h[V];
 #pragma unroll
