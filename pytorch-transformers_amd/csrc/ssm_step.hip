@@ -27,15 +27,20 @@ struct SsmStep {
     float offset, eps;
     const int *cu_tokens, *seq_slot;
     int heads, G;
+    int four;  // the norm's sum as of rows that are read four elements at a time
 };
 
 __device__ __forceinline__ float step_softplus(float x) { return x > 20.f ? x : log1pf(expf(x)); }
 
+// dA S + dx b for a lane's row i, as pta_ssm_scan rounds it: every fourth row has the decay's product in the fused operation, the others the input's
+__device__ __forceinline__ float moved(int i, float dA, float S, float dx, float b) {
+    return i % 4 == 0 ? __builtin_fmaf(dA, S, dx * b) : __builtin_fmaf(dx, b, dA * S);
+}
+
 template <typename T, int NPT, int K>
 __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __restrict__ out, const T* __restrict__ proj, long ld, SsmStep a) {
     constexpr int N = 4 * NPT, P = STEP_P, MOST = STEP_MOST_HEADS * P + 2 * N;
-    __shared__ __attribute__((aligned(16))) float chan[MOST];  // the group's channels: x of its heads, B, C
-    __shared__ float red[STEP_MOST_HEADS];
+    __shared__ __attribute__((aligned(16))) float chan[MOST];  // the group's channels: x of its heads (then what is normed), B, C
     const int s = blockIdx.y, g = blockIdx.x, per = a.heads / a.G;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, q = lane >> 4, col = (lane & 15) * 4;
     const int inner = a.heads * P, C = inner + 2 * a.G * N, channels = per * P + 2 * N, h = g * per + wave;
@@ -109,25 +114,38 @@ __global__ __launch_bounds__(STEP_MOST_HEADS * 64) void ssm_step_kernel(T* __res
         const float4 b4 = B[i >> 2], c4 = Cv[i >> 2];
         const float b = (i & 3) == 0 ? b4.x : (i & 3) == 1 ? b4.y : (i & 3) == 2 ? b4.z : b4.w;
         const float c = (i & 3) == 0 ? c4.x : (i & 3) == 1 ? c4.y : (i & 3) == 2 ? c4.z : c4.w;
-        S[i].x = dA * S[i].x + dx.x * b; S[i].y = dA * S[i].y + dx.y * b; S[i].z = dA * S[i].z + dx.z * b; S[i].w = dA * S[i].w + dx.w * b;
+        S[i] = make_float4(moved(i, dA, S[i].x, dx.x, b), moved(i, dA, S[i].y, dx.y, b), moved(i, dA, S[i].z, dx.z, b), moved(i, dA, S[i].w, dx.w, b));
         acc.x += S[i].x * c; acc.y += S[i].y * c; acc.z += S[i].z * c; acc.w += S[i].w * c;
         *reinterpret_cast<float4*>(sb + i * P) = S[i];
     }
     const float y[4] = {column_sum(acc.x) + skip * xv.x, column_sum(acc.y) + skip * xv.y, column_sum(acc.z) + skip * xv.z, column_sum(acc.w) + skip * xv.w};
-    float v[4], ss = 0.f;
+    float v[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
         const float z = Io<T>::ld(&z_raw[e]);
         v[e] = y[e] * (z / (1.0f + expf(-z)));
-        ss += v[e] * v[e];
     }
-    ss = wave_sum(q == 0 ? ss : 0.f);  // (the four quarters hold the same columns' results)
-    if (lane == 0) red[wave] = ss;
+    if (q == 0) *reinterpret_cast<float4*>(chan + wave * P + col) = make_float4(v[0], v[1], v[2], v[3]);  // (x there was this wave's alone)
     __builtin_amdgcn_s_waitcnt(0xc07f);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    ss = red[0];
-    for (int i = 1; i < per; ++i) ss += red[i];
+    // Every wave forms the group's sum of squares, in the order in which pta_rmsnorm does: its threads have four neighbours each, or one element and
+    // the one 256 further on, its waves' sums are added in turn.
+    float ss = 0.f;
+    if (a.four) {
+#pragma unroll
+        for (int w = 0; w < 2; ++w) {
+            const float4 u = *reinterpret_cast<const float4*>(chan + 4 * (64 * w + lane));
+            ss += wave_sum(__builtin_fmaf(u.x, u.x, u.y * u.y) + __builtin_fmaf(u.z, u.z, u.w * u.w));
+        }
+    } else {
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            const int at = 64 * w + lane;
+            const float lo = at < per * P ? chan[at] : 0.f, hi = at + 256 < per * P ? chan[at + 256] : 0.f;
+            ss += wave_sum(__builtin_fmaf(lo, lo, hi * hi));
+        }
+    }
     const float inv = 1.0f / sqrtf(ss / (float)(per * P) + a.eps);
     if (q != 0) return;
     T* to = out + (long)a.cu_tokens[s] * inner + h * P + col;
@@ -151,7 +169,9 @@ extern "C" int pta_ssm_step(void* out, const void* proj, long ld, const float* c
                 "ssm_step: rows lie closer together than they are long");
     PTA_REQUIRE(((uintptr_t)state % 16) == 0 && state_ld % 4 == 0, "ssm_step: rows of state must be 16-byte aligned");
     PTA_REQUIRE(dtype == PTA_F32 || dtype == PTA_BF16, "ssm_step: unknown dtype %d", dtype);
-    const SsmStep a{conv_w, conv_b, tail, tail_ld, dt_bias, A_log, D, state, state_ld, norm_w, offset, eps, cu_tokens, seq_slot, heads, G};
+    // where pta_rmsnorm reads a group of 512 and its gate so
+    const int four = heads / G * STEP_P == 512 && ld % 4 == 0 && (uintptr_t)proj % (dtype == PTA_F32 ? 16 : 8) == 0 && (uintptr_t)norm_w % 16 == 0;
+    const SsmStep a{conv_w, conv_b, tail, tail_ld, dt_bias, A_log, D, state, state_ld, norm_w, offset, eps, cu_tokens, seq_slot, heads, G, four};
     const dim3 grid(G, n_seqs), block(heads / G * 64);
 #define STEP(T, NPT, K_) hipLaunchKernelGGL((ssm_step_kernel<T, NPT, K_>), grid, block, 0, (hipStream_t)stream, (T*)out, (const T*)proj, ld, a)
 #define STEP_K(T, NPT) if (K == 2) STEP(T, NPT, 2); else if (K == 3) STEP(T, NPT, 3); else STEP(T, NPT, 4)
