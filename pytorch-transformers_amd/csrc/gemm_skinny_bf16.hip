@@ -118,22 +118,39 @@ __device__ __forceinline__ void by_registers(f32x4_t (&acc)[RT][MT], const bf16_
     }
 }
 
+#define SHARE_BITS 26
+#define SHARE_MOST 63  // in the bits above
+
 // How `items` (rows of W, pairs of them) are shared out evenly to `groups` workgroups: the first `over` have one more than the others.
 // Made on the host: the division by a number of workgroups was 300 instructions at the start of a launch of few microseconds.
+// In a launch's arguments it is a word, `each` in the six highest bits and `over` in the others: a group has up to 64 items, so 64 for every one is said as 63
+// and one more for all of them, and a launch has fewer groups than 2^26 (of a wave each: 2^32 threads).
 struct Share {
     int each, over;
     Share() = default;
-    Share(int items, int groups) : each(groups > 0 ? items / groups : 0), over(groups > 0 ? items % groups : 0) {}
-    __device__ __forceinline__ int begin(int j) const { return j * each + min(j, over); }
-    __device__ __forceinline__ int end(int j) const { return begin(j) + each + (j < over ? 1 : 0); }
-    // in a word: up to 63 items a group, and fewer groups than a launch may have threads for
-    __host__ __device__ __forceinline__ uint32_t packed() const { return (uint32_t)each << 26 | (uint32_t)over; }
-    static __device__ __forceinline__ Share of(uint32_t word) {
+    Share(int items, int groups) : each(groups > 0 ? items / groups : 0), over(groups > 0 ? items % groups : 0) {
+        if (each == SHARE_MOST + 1 && over == 0) each = SHARE_MOST, over = groups;
+    }
+    __host__ __device__ __forceinline__ int begin(int j) const { return j * each + (j < over ? j : over); }
+    __host__ __device__ __forceinline__ int end(int j) const { return begin(j) + each + (j < over ? 1 : 0); }
+    bool fits() const { return each <= SHARE_MOST && over < 1 << SHARE_BITS; }
+    uint32_t packed() const { return (uint32_t)each << SHARE_BITS | (uint32_t)over; }
+    static __host__ __device__ __forceinline__ Share of(uint32_t word) {
         Share s;
-        s.each = word >> 26, s.over = word & 0x3ffffff;
+        s.each = word >> SHARE_BITS, s.over = word & ((1u << SHARE_BITS) - 1);
         return s;
     }
 };
+
+// Where workgroup j of `groups` finds its share of `items` to begin and end, as a launch's word says it.
+extern "C" int pta_gemm_skinny_share(int items, int groups, int j, int* begin, int* end) {
+    PTA_REQUIRE(items > 0 && groups > 0 && j >= 0 && j < groups, "gemm_skinny_share: workgroup %d of %d for %d items", j, groups, items);
+    const Share made(items, groups);
+    PTA_REQUIRE(made.fits(), "gemm_skinny_share: %d items for each of %d workgroups are more than a word says", items / groups, groups);
+    const Share read = Share::of(made.packed());
+    *begin = read.begin(j), *end = read.end(j);
+    return 0;
+}
 
 // The kernels here take what their loads of W and x are found by first, in the fourteen words that are in registers when a workgroup starts: the
 // arguments behind them are a load away, 0.7 us over cold caches, and what is asked for at the front the first loads wait for.  (With the problem's struct
@@ -866,6 +883,7 @@ static int launch_rings(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStr
 template <typename Kernel>
 static int launch_two(Kernel kernel, dim3 grid, dim3 block, size_t lds, hipStream_t s, const SkinnyProblem& a, const SkinnyProblem& b, int M, int K, int rot_stride,
                       const QkvTail& tail = QkvTail{}) {
+    PTA_REQUIRE(a.rows.fits() && b.rows.fits(), "gemm_skinny_bf16: %d workgroups are too many for one launch", (int)grid.x);
     return launch_rings(kernel, grid, block, lds, s, a.x, a.W, b.x, b.W, M, K, a.blocks, a.rows.packed(), b.rows.packed(),
                         Walk::packed((int)block.x / 64, rot_stride, tail.d), a, b, tail);
 }
@@ -902,8 +920,7 @@ static int launch_cfg(SkinnyProblem a, SkinnyProblem b, int M, int K, int S, hip
         if (S <= 4) return launch_two(gemm_skinny_kernel<MT, RT, U, OutT, 0, 4>, grid, block, (size_t)S * RowStream<RT, 4>::RING, s, a, b, M, K, rot_stride);
         return launch_two(gemm_skinny_kernel<MT, RT, U, OutT, 0, 3>, grid, block, (size_t)S * RowStream<RT, 3>::RING, s, a, b, M, K, rot_stride);
     }
-    launch_two(gemm_skinny_kernel<MT, RT, U, OutT>, grid, block, lds, s, a, b, M, K, rot_stride);
-    return 0;
+    return launch_two(gemm_skinny_kernel<MT, RT, U, OutT>, grid, block, lds, s, a, b, M, K, rot_stride);
 }
 
 // where a workgroup has eight rows of W or fewer (N alone decides: one order of summation for any number of rows of x)
@@ -920,6 +937,7 @@ static int launch_halves(SkinnyProblem p, int M, int K, int S, hipStream_t s, co
     if (S <= 0) S = p.N <= 5 * units ? 4 : 2;
     const dim3 grid(std::max((items + most - 1) / most, std::min(units, (items + most / 2 - 1) / (most / 2)))), block(S * 64);
     p.rows = Share(items, (int)grid.x);
+    PTA_REQUIRE(p.rows.fits(), "gemm_skinny_bf16: %d workgroups are too many for one launch", (int)grid.x);
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 3 : 0);
     const uint32_t how = Walk::packed(S, rot, tail.d, TAIL && qkv_tail_plain_pairs(tail.rot, tail.d));
@@ -1140,6 +1158,7 @@ static int launch_normed(const char* what, SkinnyProblem p, const float* ln_w, c
     const int items = TAIL ? p.N / 2 : p.N, most = TAIL ? 8 : 16, units = pta_compute_units();
     const int groups = std::max((items + most - 1) / most, std::min(units, (items + most / 4 - 1) / (most / 4)));
     p.rows = Share(items, groups);
+    PTA_REQUIRE(p.rows.fits(), "%s: %d workgroups are too many for one launch", what, groups);
     const bool eight = groups <= units + units / 16;
     const int waves = eight ? 8 : 4;
     const size_t lds = waves * 64 * sizeof(f32x4_t) + (size_t)M * (K + 8) * sizeof(bf16_t);
@@ -1197,8 +1216,10 @@ extern "C" int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, i
     if (blocks > units) blocks = (blocks + units - 1) / units * units;  // a whole number of workgroups per unit (launch_cfg)
     static const int rot_env = getenv("PTA_SKINNY_ROT") ? atoi(getenv("PTA_SKINNY_ROT")) : -1;
     const int rot_stride = rot_env >= 0 ? rot_env : (K % 2048 == 0 ? 5 : 0);
+    const Share rows(F, blocks);
+    PTA_REQUIRE(rows.fits(), "gemm_skinny_glu_bf16: %d workgroups are too many for one launch", blocks);
     auto go = [&](auto kernel, size_t ring) {
-        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)W, M, F, K, Share(F, blocks).packed(),
+        return launch_rings(kernel, dim3(blocks), dim3(S * 64), S * ring, (hipStream_t)stream, (const bf16_t*)x, (const bf16_t*)W, M, F, K, rows.packed(),
                             Walk::packed(S, rot_stride), (bf16_t*)y, kind, alpha, limit);
     };
     if (K > STREAM_MOST_K ? go(gemm_skinny_glu_kernel<0>, 2048)

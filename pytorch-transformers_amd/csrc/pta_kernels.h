@@ -182,6 +182,8 @@ int pta_gemm_skinny_spread(int N);
 int pta_gemm_skinny_qkv_bf16(void* q_out, const void* x, const void* W, const float* bias, const PtaRotation* rotation,
                              const int* token_pos, const int* token_seq, const int* block_table, int bt_stride, void* k_pool,
                              void* v_pool, int nh, int nkv, int d, int layout, int write_cache, int M, int K, void* stream);
+// items [*begin, *end) are workgroup j's of a launch that shares them out to `groups` (host only)
+int pta_gemm_skinny_share(int items, int groups, int j, int* begin, int* end);
 
 // y [M, F] = glu(x . Wg^T, x . Wu^T), W = [Wg, Wu] [2 F, K], for up to 16 rows; kinds as pta_glu's
 int pta_gemm_skinny_glu_bf16(void* y, const void* x, const void* W, int M, int F, int K, int kind, float alpha, float limit, void* stream);
