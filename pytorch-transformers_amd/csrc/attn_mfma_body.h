@@ -192,9 +192,10 @@
                     if (kb + 8 * gq + j >= lim || kb + 8 * gq + j < lo) sacc[j >> 2][ct][j & 3] = -INFINITY;
             }
             const f32x4_t s0 = sacc[0][ct], s1 = sacc[1][ct];
-            const float mx3 = max3(s1[2], s1[3], max3(s0[0], s0[1], s0[2]));
-            mx[ct] = max3(s0[3], s1[0], s1[1]);
-            mx[ct] = max3(mx[ct], mx3, mx3);
+            constexpr bool PLAIN = W == 1 && CT == 4 && DT == 8;
+            const float mx3 = max3<PLAIN>(s1[2], s1[3], max3<PLAIN>(s0[0], s0[1], s0[2]));
+            mx[ct] = max3<PLAIN>(s0[3], s1[0], s1[1]);
+            mx[ct] = max3<PLAIN>(mx[ct], mx3, mx3);
         }
     };
     // The running maximum is only a reference point for the exponentials, shared by the four lanes of a column;

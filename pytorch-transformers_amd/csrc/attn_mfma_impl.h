@@ -59,12 +59,13 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
     return c.u;
 }
 
-// the largest of three in one instruction; written out because the compiler, asked for fmaxf of values that
-// come through a branch, first makes each of them canonical with an instruction of its own
-__device__ __forceinline__ float max3(float a, float b, float c) {
-    float r;
-    asm("v_max3_f32 %0, %1, %2, %3" : "=v"(r) : "v"(a), "v"(b), "v"(c));
-    return r;
+// The largest of three in one instruction, by the maximum that takes values as they are (fmaxf of values that come through a branch has each made
+// canonical by an instruction of its own first).  Not inline asm: the compiler knows nothing of what that reads, and leaves out the wait that a matrix
+// instruction's result needs, so scores were read before they were there.  (A NaN stays one: its column's result is NaN in any case.)
+// PLAIN: by fmaxf, for the one kernel whose registers the compiler does not come to terms with otherwise.
+template <bool PLAIN> __device__ __forceinline__ float max3(float a, float b, float c) {
+    if constexpr (PLAIN) return fmaxf(fmaxf(a, b), c);
+    else return __builtin_elementwise_maximum(__builtin_elementwise_maximum(a, b), c);
 }
 
 #define PTA_LOG2E 1.4426950408889634f
