@@ -54,8 +54,8 @@ __global__ __launch_bounds__(1024) void gated_heads_kernel(const TX* __restrict_
         if (w && N <= GATED_EACH * threads) {
 #pragma unroll
             for (int u = 0; u < GATED_EACH; ++u) {
-                const float v = Io<TX>::ld(&xq[u]);
-                ss += i0 + u * threads < N ? v * v : 0.f;
+                const float v = i0 + u * threads < N ? Io<TX>::ld(&xq[u]) : 0.f;  // (a choice between sums would leave a product and an addition)
+                ss = __builtin_fmaf(v, v, ss);
             }
             inv = rsqrtf(block_sum(ss, red, threads / 64) / (float)N + eps);
         }
@@ -313,7 +313,10 @@ __global__ __launch_bounds__(256) void head_norm_gate_kernel(const float* __rest
         }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) ss += lane + r * PTA_WAVE < dv ? xv[r] * xv[r] : 0.f;
+        for (int r = 0; r < 4; ++r) {
+            const float v = lane + r * PTA_WAVE < dv ? xv[r] : 0.f;
+            ss = __builtin_fmaf(v, v, ss);
+        }
         const float inv = 1.0f / sqrtf(wave_sum(ss) / (float)dv + eps);
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
