@@ -1386,8 +1386,9 @@ def gemm_splitk_pair_partial(x1: torch.Tensor, w1: torch.Tensor, x2: torch.Tenso
 
 def gemm_splitk_pair_attn_ok(x1: torch.Tensor, w1: torch.Tensor, late: LateAttention, w2: torch.Tensor) -> bool:
     """Whether ``gemm_splitk_pair_attn`` has a launch for these (which ``gemm_partial_pair_ok`` takes, with ``late.out`` as the second input).
-    A pair that has not been timed is timed here, while timing is on: the answer depends on what that chooses."""
-    tuning.tune_pair_parts(w1, w2)
+    A pair that has not been timed is timed here, while timing is on: the answer depends on what that
+    chooses, and the choice on what a launch that carries the attention saves."""
+    tuning.tune_pair_parts(w1, w2, late)
     _, nh, d = late.q.shape
     return bool(load_library().pta_gemm_splitk_pair_attn_ok(w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], x1.shape[0], nh,
                                                             late.k_pool.shape[1], d))

@@ -15,6 +15,7 @@ this module are also reachable as attributes of ``ops``.
 """
 from __future__ import annotations
 
+import copy
 import functools
 import os
 from typing import Optional
@@ -709,7 +710,69 @@ def pick_way(times, margin: float) -> int:
     return min(ok, key=lambda i: total[i]) if ok else 0
 
 
-def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
+RIDE_KEYS = 150  # of every sequence, where a pair is timed with the attention that it may carry
+
+
+def ride_gain(copies, late, x1: torch.Tensor, stream: torch.Tensor, norm_w: torch.Tensor) -> float:
+    """Milliseconds that the pair's launch saves by carrying a decode step's attention (``ops.gemm_splitk_pair_attn``), against attention in
+    a launch of its own, with the ranges that are fixed for the pair: 0 where it does not carry it.  ``copies``: pairs of matrices, each read from memory;
+    ``late``: what the step that is timed would hand over (an ``ops.LateAttention``), whose heads are taken with contexts of ``RIDE_KEYS``
+    for as many sequences as ``x1`` has rows.  The norm of ``stream`` and both products follows either way.  Replays of captured
+    launches are timed, because the host takes longer for two launches than a small pair does."""
+    rows, (nh, d), nkv = x1.shape[0], late.q.shape[1:], late.k_pool.shape[1]
+    (N1, K1), (N2, K2) = copies[0][0].shape, copies[0][1].shape
+    waves = late_waves(rows, nh, nkv, d, RIDE_KEYS, RIDE_KEYS) if rows <= ops.LATE_MOST_ROWS else 0
+    if not waves or not ops.load_library().pta_gemm_splitk_pair_attn_ok(N1, K1, N2, K2, rows, nh, nkv, d):
+        return 0.0
+    pages = (RIDE_KEYS + 63) // 64
+    draw = lambda *shape: torch.randn(shape, device=x1.device).to(torch.bfloat16)
+    count = lambda *a: torch.arange(*a, dtype=torch.int32, device=x1.device)
+    start = torch.full((rows,), RIDE_KEYS - 1, dtype=torch.int32, device=x1.device)
+    ctx = copy.copy(late.ctx)
+    ctx.n_seqs = ctx.n_tokens = rows
+    ctx.token_seq, ctx.cu_tokens, ctx.token_pos, ctx.seq_start = count(rows), count(rows + 1), start, start
+    ctx.new_tokens, ctx.is_decode, ctx.max_len, ctx.mean_len, ctx.extras = [1] * rows, True, RIDE_KEYS, RIDE_KEYS, {}
+    trial = ops.LateAttention(draw(rows, nh, d), draw(rows * pages, nkv, 64, d), draw(rows * pages, nkv, d, 64), count(rows * pages).view(rows, pages),
+                              ctx, late.slopes, late.scale, waves=waves, **late.how)
+
+    parts = [torch.empty((p, rows, N), dtype=torch.float32, device=x1.device)
+             for p, N in zip(ops.gemm_splitk_pair_parts(N1, K1, N2, K2, rows), (N1, N2))]
+
+    def apart(a, b):
+        trial.run()
+        ops._call("pta_gemm_splitk_pair_bf16", ops._ptr(parts[0]), ops._ptr(x1), ops._ptr(a), int(N1), int(K1), ops._ptr(parts[1]),
+                  ops._ptr(trial.out), ops._ptr(b), int(N2), int(K2), rows, ops._stream())
+        return parts
+
+    def together(a, b):
+        return ops.gemm_splitk_pair_attn(x1, a, trial, b)
+
+    def ms(way) -> float:
+        def run():
+            ctx.extras.clear()  # (marks that are clear when a launch starts are cleared in the capture)
+            for a, b in copies:
+                first, second = way(a, b)
+                ops.layernorm_sum([(second, None), (first, None), stream], N1, w=norm_w, b=norm_w, eps=1e-5)
+
+        run()
+        torch.cuda.synchronize(x1.device)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            run()
+        best = float("inf")
+        for _ in range(6):
+            begin, end = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            best = min(best, begin.elapsed_time(end) / len(copies))
+        return best
+
+    return ms(apart) - ms(together)
+
+
+def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor, late=None) -> None:
     """Once per pair of shapes, while timing is on: the pair launch with the ranges of K that the rule has for the rows, and with
     neighbours of them, with cold caches; ``pick_way`` says which is kept.  Up to 32 rows are timed at 8 and 32; 33 to 64 rows,
     where they have ranges of their own, at 40 and 64, and with workgroups of 128 rows of W (which load the activations half as
@@ -717,7 +780,9 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
     rows), the launch with stationary activations is timed against the winner with one to six ranges of the shorter K
     (and as many times more of the longer): whichever of the two the rule takes for the class stays unless it is beaten by 2 %.
     All with what reads the partial sums behind the launch (the norm that adds them, where the two products have one width;
-    else a charge for the ranges' bytes).  ``TuningTable.pair_parts`` and ``pair_stationary`` keep what is in use.
+    else a charge for the ranges' bytes).  Where the step's attention may go in the pair's launch (``late``, an ``ops.LateAttention``), a way that
+    cannot carry it (six waves, stationary activations) is charged what that saves (``ride_gain``).  ``TuningTable.pair_parts`` and
+    ``pair_stationary`` keep what is in use.
 
     The rule's choice for the class is what has to be beaten, at rows of the class, because ranges that are 14 % faster at 64 rows may be
     slower at 8 (4,544 x 4,544 + 4,544 x 18,176, where a single timing at 64 rows chose for all: a step of 7B layers 3.07 -> 3.17 ms at 8
@@ -793,8 +858,22 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
 
     say = (lambda text: print(f"[pta tune] pair {key}: {text}", flush=True)) if os.environ.get("PTA_TUNE_VERBOSE") else (lambda text: None)
 
+    def saved(rows):  # by the launch that carries attention, with what is fixed now
+        if late is None or norm_w is None or ops._timing is not None:
+            return 0.0
+        gain = ride_gain(copies, late, counts[rows][0], xs_bf16[rows], norm_w)
+        if gain:
+            say(f"at {rows} rows: attention in the launch saves {gain * 1e3:.1f} us")
+        return gain
+
     def choose(found, label, rows):
         times = [timed_ways(found, n, fix) for n in rows]
+        carry = [c[2] != 4 for c in found]
+        if any(carry) and not all(carry):
+            for n, t in zip(rows, times):
+                fix(found[min((j for j, c in enumerate(carry) if c), key=lambda j: t[j])])
+                gain = saved(n)
+                t[:] = [v if c else v + gain for v, c in zip(t, carry)]
         i = pick_way(times, PAIR_TUNE_MARGIN)
         show = lambda j: f"{found[j]} " + " / ".join(f"{t[j] * 1e3:.1f}" for t in times)
         say(f"{label}: rule {show(0)} us; fastest " + ", ".join(show(j) for j in sorted(range(len(found)), key=lambda j: sum(t[j] for t in times))[:5]) +
@@ -814,11 +893,12 @@ def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
             # varies, and fewer ranges leave whatever reads them next less to read
             staged = ops.gemm_splitk_pair_parts(*shapes, rows)
             t_staged = timed_ways([staged], rows, lambda c: fix_st(cls, (0, 0)))[0]
+            gain = saved(rows) if st_cands else 0.0
             t_st = timed_ways(st_cands, rows, lambda c: fix_st(cls, c)) if st_cands else []
             best = min((i for i in range(len(st_cands)) if t_st[i] <= 1.015 * min(t_st)), key=lambda i: st_cands[i]) if st_cands else -1
-            found = [((0, 0), t_staged)] + ([(st_cands[best], t_st[best])] if best >= 0 else [])
+            found = [((0, 0), t_staged)] + ([(st_cands[best], t_st[best] + gain)] if best >= 0 else [])
             if rules[cls][2] == 3:  # the rule's ranges first
-                found.insert(0, (rules[cls][:2], t_st[st_cands.index(rules[cls][:2])]))
+                found.insert(0, (rules[cls][:2], t_st[st_cands.index(rules[cls][:2])] + gain))
             keep = found[pick_way([[t for _, t in found]], 0.98)][0]
             chosen_st.append(keep)
             fix_st(cls, (0, 0))
