@@ -15,6 +15,7 @@ from typing import Dict, Optional, Sequence
 import ctypes
 import gc
 import os
+import threading
 import weakref
 
 import numpy as np
@@ -103,6 +104,7 @@ def _capture_stream(index: int) -> "torch.cuda.Stream":
 # 2.0 to 2.2 ms with it before every capture, 1.87 to 1.88 before every eighth, 1.84 to 1.88 without (and 2 MiB more a call).
 _dropped_graphs: Dict[int, int] = {}
 DROPPED_GRAPHS = 8
+_ran_here = threading.local()  # per thread, because libraries keep their handles so: ``CausalLM._captured_shapes`` of every model
 DIRECT_STEPS = 64  # steps of a shape that are launched directly after a capture that found no memory, before the next attempt
 
 
@@ -237,9 +239,10 @@ class _DecodeGraph:
         # capture; its result is the step's result.  The capture that follows records launches and runs nothing.  A model that has
         # had a step of this shape captured before (in another cache) has no such setting up to do: its step is captured first and
         # then replayed, which spares the host a second pass over the launches (two 32-bit layers, six tokens: of 1.84 ms a call 0.24).
+        # That holds for the thread that ran it, whose libraries are set up, and while choices between kernels stay as they were.
         shape = (self.n, self.len_bound, self.mean_bound)
         captured = self.model._captured_shapes
-        if shape in captured and self.direct == 0:
+        if shape in captured and self.direct == 0 and not tuning.may_time():
             if self._try_capture():
                 self.graph.replay()
                 return self.logits
@@ -316,12 +319,22 @@ class CausalLM:
         self.tuning = tuning.TuningTable()
         #: run steps in which every sequence brings one token as replays of a captured HIP graph
         self.use_graphs = bool(spec.supports_graphs)
-        #: shapes of decode steps (``_DecodeGraph``) that ran directly and were captured since the choices between kernels last changed
-        self._captured_shapes: set = set()
         #: ``layer_hook(i, x)`` is called after entry ``i`` of the run order with the residual stream
         #: ``[tokens, hidden]`` as a tensor (for dumps when a mismatch is being looked for); while it is set, steps
         #: are launched directly, never replayed from a captured graph
         self.layer_hook = None
+
+    @property
+    def _captured_shapes(self) -> set:
+        """Shapes of decode steps (``_DecodeGraph``) that ran directly in this thread and were captured since choices between kernels last
+        changed."""
+        models = getattr(_ran_here, "models", None)
+        if models is None:
+            models = _ran_here.models = weakref.WeakKeyDictionary()
+        kept = models.get(self)
+        if kept is None or kept[0] != tuning.changes():
+            kept = models[self] = (tuning.changes(), set())
+        return kept[1]
 
     def _move_constants(self) -> None:
         seen = set()
@@ -396,7 +409,6 @@ class CausalLM:
         Steps never time anything by themselves (unless PTA_TUNE=1 is set): untuned, they take the built-in
         choice, and logits are the same bits in every process."""
         tuning.activate(self.tuning)
-        self._captured_shapes.clear()
         if table is not None:
             if isinstance(table, (str, os.PathLike)):
                 import json

@@ -77,6 +77,7 @@ class TuningTable:
         if unknown:
             raise ValueError(f"a tuning table has the sections {list(self.FIELDS)}; this one also holds {unknown}")
         activate(self)
+        _note_change()
         shapes = lambda k: tuple(tuple(int(v) for v in p.split("x")) for p in k.split(","))
         flat = lambda k: tuple(int(p) for p in k.split(","))
         for k, v in data.get("pair_parts", {}).items():
@@ -104,11 +105,25 @@ class TuningTable:
 
     def clear(self) -> None:
         """Back to the built-in defaults for every shape."""
+        _note_change()
         if self is _active:
             _release(self)
         for d in (self.pair_stationary, self.pair_parts, self.splitk_rows, self.mm_plans, self.mm_costs, self.mm_times,
                   self.mm_joined, self.mm_ksplit, self.mm_tiles, self.decode_plans):
             d.clear()
+
+
+_changes = 0  # times that a choice of some table was set or may have been timed
+
+
+def changes() -> int:
+    """A number that grows when choices change: what ran under another number may have run otherwise."""
+    return _changes
+
+
+def _note_change() -> None:
+    global _changes
+    _changes += 1
 
 
 def _unfix_pair(s1, s2) -> None:
@@ -458,6 +473,7 @@ def context_lengths(longest: int, mean: int, n: int) -> list:
 
 def set_decode_plan(key, cut=None) -> None:
     """Fix the cut of the decode launches that ``key`` counts (None: back to the rule)."""
+    _note_change()
     if cut is None:
         _active.decode_plans.pop(tuple(key), None)
     else:
@@ -479,6 +495,7 @@ class live_tuning:
     def __exit__(self, *exc):
         global TUNE_LIVE
         TUNE_LIVE = self._old
+        _note_change()
         return False
 
 
