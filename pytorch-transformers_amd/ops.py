@@ -193,6 +193,8 @@ def _entry_cost(name: str, a) -> tuple:
         return (one[0] + two[0], one[1] + two[1])
     if name == "pta_layernorm_sum":
         return ((a[4] + a[7]) * float(a[17]) * a[19] * 4, 0.0)
+    if name == "pta_gemm_splitk_pair_attn":  # both matrices, and what attention in a launch of its own reads
+        return both(both(gemm(a[10], a[3], a[4]), gemm(a[10], a[8], a[9])), _entry_cost("pta_attn_mfma", a))
     if name in ("pta_attn_mfma", "pta_attn_generic", "pta_attn_f32", "pta_latent_decode", "pta_attn_latent_mfma", "pta_attn_latent_prompt", "pta_attn_latent", "pta_attn_talk",
                 "pta_attn_talk_mfma"):
         # (a model with two kinds of attention says each kind's figures under the entry point's name)
@@ -215,6 +217,11 @@ def _entry_cost(name: str, a) -> tuple:
     if name == "pta_ssm_scan":  # the convolution's output in, y out, both 32-bit
         M, inner = float(timing_hint.get("rows", 0)), float(a[14] * a[15])
         return (M * (2 * inner + 2 * a[17] * a[16]) * 4.0, 4.0 * M * inner * a[16])
+    if name == "pta_ssm_step":  # the state and the convolution's tail in and out (32-bit), the product's row in, the normed one out
+        n, heads, N, G, K, e = float(a[17]), a[18], a[19], a[20], a[21], (4.0 if a[22] == F32 else 2.0)
+        inner = heads * 64
+        C = inner + 2 * G * N
+        return (n * (8.0 * (inner * N + (K - 1) * C) + (2 * inner + C + heads) * e), 4.0 * n * inner * N)
     if name == "pta_head_project":
         M, H, K, O = float(a[9]), a[10], a[11], a[12]
         return (H * K * O * (4.0 if a[13] == F32 else 2.0) + M * H * (K + O) * 4.0, 2.0 * M * H * K * O)
