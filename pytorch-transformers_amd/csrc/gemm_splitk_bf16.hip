@@ -612,6 +612,23 @@ extern "C" int pta_gemm_splitk_pair_attn_ok(int N1, int K1, int N2, int K2, int 
     return rt != PAIR_STATIONARY && rt != PAIR_SIX && (long)std::max(K1, K2) * 32 * 2 < LDS_PAST;
 }
 
+// What decides whether the products of such a launch hide the attention (`tuning.late_pays` has the lines): rounds, the workgroups a compute unit has
+// at most, and slack, the blocks (64 elements of K by 64 rows of W, a third of a microsecond each, as a unit pulls some 25 GB/s) that a unit has more of the
+// first product's than of the second's, which wait for attention.
+extern "C" int pta_gemm_splitk_pair_attn_room(int N1, int K1, int N2, int K2, int M, int* rounds, int* slack) {
+    if (N1 <= 0 || K1 <= 0 || N2 <= 0 || K2 <= 0 || M <= 0) return pta_fail("gemm_splitk_pair_attn_room: sizes must be positive");
+    int p1, p2;
+    const int rt = pick_pair_parts_rows(N1, K1, N2, K2, M, &p1, &p2);
+    *rounds = *slack = 0;
+    if (rt == PAIR_STATIONARY || rt == PAIR_SIX) return 0;
+    const SplitkProblem a = make_problem(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N1, K1, 0, 0, rt, p1, 0);
+    const SplitkProblem b = make_problem(nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, N2, K2, 0, 0, rt, p2, 0);
+    const int units = max(1, pta_compute_units());
+    *rounds = (a.tiles * a.parts + b.tiles * b.parts + units - 1) / units;
+    *slack = *rounds * rt * (a.blocks_per_part - b.blocks_per_part);
+    return 0;
+}
+
 // The pair with the attention that its second product takes (x2 [M, nh d] is written here): pta_attn_mfma of one token a sequence,
 // whole contexts, `waves` (1 or 4) on a piece's keys; sync: groups of sixteen heads x nkv x M zeros; owners: -1, or how many of attention's
 // workgroups the launch is to begin with (the products' do the others).

@@ -113,7 +113,7 @@ def _call(name: str, *args) -> None:
 # cannot be recorded into a captured step.  ``timing_hint`` carries what an entry point's arguments do not say
 # (how many cached keys and values an attention launch reads, the arithmetic of a prompt's attention).
 _timing = None
-_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok", "pta_gemm_splitk_pair_attn_ok", "pta_ssm_step_ok")  # entry points that launch nothing
+_HOST_ENTRIES = ("pta_attn_f32_plan", "pta_gemm_splitk_pair_parts", "pta_gemm_splitk_pair_way", "pta_gemm_stationary_rule", "pta_gemm_tile_plan", "pta_gemm_f32_pair_ok", "pta_gemm_splitk_pair_attn_ok", "pta_gemm_splitk_pair_attn_room", "pta_ssm_step_ok")  # entry points that launch nothing
 timing_hint = {"attn_bytes": 0, "attn_flops": 0}
 
 
@@ -1395,10 +1395,19 @@ def gemm_splitk_pair_attn_ok(x1: torch.Tensor, w1: torch.Tensor, late: LateAtten
     """Whether ``gemm_splitk_pair_attn`` has a launch for these (which ``gemm_partial_pair_ok`` takes, with ``late.out`` as the second input).
     A pair that has not been timed is timed here, while timing is on: the answer depends on what that
     chooses, and the choice on what a launch that carries the attention saves."""
-    tuning.tune_pair_parts(w1, w2, late)
+    tuning.tune_pair_carrying(w1, w2, late)
+    tuning.tune_pair_parts(w1, w2)
     _, nh, d = late.q.shape
     return bool(load_library().pta_gemm_splitk_pair_attn_ok(w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], x1.shape[0], nh,
                                                             late.k_pool.shape[1], d))
+
+
+def late_attention_pays(late: LateAttention, w1: torch.Tensor, w2: torch.Tensor) -> bool:
+    """Whether the pair of products has the room for ``late`` in its launch (``tuning.late_pays``), which takes it (``gemm_splitk_pair_attn_ok``)."""
+    ctx, (M, nh, d) = late.ctx, late.q.shape
+    rounds, slack = ctypes.c_int(0), ctypes.c_int(0)
+    _call("pta_gemm_splitk_pair_attn_room", *(int(n) for n in (*w1.shape, *w2.shape)), int(M), ctypes.byref(rounds), ctypes.byref(slack))
+    return tuning.late_pays(ctx.n_seqs, nh, late.k_pool.shape[1], d, ctx.max_len, getattr(ctx, "mean_len", 0), rounds.value, slack.value)
 
 
 def gemm_splitk_pair_attn(x1: torch.Tensor, w1: torch.Tensor, late: LateAttention, w2: torch.Tensor, owners: int = -1):

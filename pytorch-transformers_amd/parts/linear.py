@@ -278,7 +278,8 @@ class PendingProjection:
         if not (a._x.dtype == torch.bfloat16 and ops.layernorm_sum_ok(a.linear.out_features)
                 and ops.gemm_partial_pair_ok(a._x, a.linear.weight, b._x, b.linear.weight)):
             return None
-        if a.late is None and b.late is not None and ops.gemm_splitk_pair_attn_ok(a._x, a.linear.weight, b.late, b.linear.weight):
+        if (a.late is None and b.late is not None and ops.gemm_splitk_pair_attn_ok(a._x, a.linear.weight, b.late, b.linear.weight)
+                and ops.late_attention_pays(b.late, a.linear.weight, b.linear.weight)):
             late, b.late = b.late, None
             pa, pb = ops.gemm_splitk_pair_attn(a._x, a.linear.weight, late, b.linear.weight)
         else:

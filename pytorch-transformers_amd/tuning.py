@@ -292,23 +292,23 @@ def decode_key(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_le
 
 def late_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0) -> int:
     """0, or the waves (1 or 4) on the keys of sixteen heads with which a decode step's attention goes in the launch of the products behind it,
-    where there is such a launch (``ops.gemm_splitk_pair_attn``).  Whole contexts: a piece, sixteen heads of a KV head, occupies a
-    workgroup, or a wave of one, for as long as its keys take behind the stream of weights, and every workgroup of attention is one less for that
-    stream.  Microseconds a layer against launches apart, one wave / four:
+    where there is such a launch (``ops.gemm_splitk_pair_attn``) and its products leave the room (``late_pays``).  Whole contexts: a piece,
+    sixteen heads of a KV head, occupies a workgroup, or a wave of one, for as long as its keys take behind the stream of weights, and every
+    workgroup of attention is one less for that stream.  Microseconds a layer against launches apart, one wave / four:
 
                                         1 sequence       8               16              32              64
-        71 heads on 1 of 64, 60 keys    -3.3 / -3.2   -3.2 / -1.5     -2.5 / -0.5     -1.7 / +0.1     -2.0 / -0.5
-                            150 keys    -4.3 / -4.1   -3.9 / -2.1     -3.5 / -0.8     -3.1 / +0.2     -0.2 / -1.2
-                            900 keys      +4 / -6.4    +52 / -5.1      +50 / -1.2      +32 / -1.8       +8 / -1.4
-                          1,900 keys    +134 / -7.3   +132 / -7.1     +130 / +2.4     +121 / +2.7      +45 / +11.6
-        128 on 8 of 64, 60 keys         -3.2 / -3.2   -2.4 / -1.4     +0.5 / +0.3     -0.2 / -2.6     +0.9 / +3.7
-                       150 keys         -2.6 / +6.4   -0.8 / -1.2     +1.1 / -2.4     +1.6 / -1.4     +2.2 / +1.9
-                       900 keys          +10 / -4.0    +10 / -1.0       +6 / -5.6      +10 / -4.7     +8.5 / +5.4
-                     1,900 keys         +107 / +2.1   +110 / +3.1     +103 / +1.8      +98 / -9.2      +13 / +6.1
+        71 heads on 1 of 64, 60 keys    -2.3 / -2.3   -1.3 / -0.1     -0.3 / +0.8     +0.6 / +2.3     -0.8 / +0.6
+                            150 keys    -3.1 / -3.4   -2.6 / -0.8     -1.5 / +0.9     -1.3 / +0.9     +1.2 / +0.5
+                            900 keys    +4.5 / -5.3    +11 / -3.8     +9.9 / +0.1     +7.7 / +0.9      +12 / +2.3
+                          1,900 keys     +38 / -6.4    +48 / -5.5      +47 / +2.5      +45 / +4.6      +48 / +16
+        128 on 8 of 64, 60 keys         -1.4 / -1.3   -1.2 / -0.3     +0.7 / +0.4     +1.5 / +0.7     -2.0 / +3.3
+                       150 keys         -1.1 / -2.8   -0.4 / -0.8     +2.6 / -0.5     +2.2 / -0.5     +0.3 / +4.5
+                       900 keys          +10 / -3.1    +12 / -1.2     +7.7 / -4.7      +13 / -0.9     +6.2 / +5.5
+                     1,900 keys          +29 / +1.7    +27 / +2.7      +27 / +1.6      +15 / -9.5     +4.4 / +2.9
 
     So a wave alone up to ``SHORT_CONTEXT`` where the heads of a KV head fill several pieces (whose waves share its keys), else four; beyond that four
-    waves, up to 2,048 keys where there are few pieces of several a KV head, up to 1,024 where a KV head is one piece.  A cut that was fixed
-    (``set_decode_plan``) goes before the rule."""
+    waves, up to 2,048 keys where there are few pieces of several a KV head, up to 1,024 where a KV head is one piece.  (One answer for 33 to 64
+    sequences: 40 to 56 of 30 to 190 keys are -1.0 to -4.7, 64 from -0.8 to +3.0.)  A cut that was fixed (``set_decode_plan``) goes before the rule."""
     key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
     if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
         return 0
@@ -321,6 +321,25 @@ def late_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_le
     if cut is not None:
         return 4 if cut[0] == 1 and cut[1] >= max_len and cut[2] == 4 else 0
     return 4 if (bound <= 2048 and pieces <= 40 if groups > 1 else bound <= 1024 and pieces <= 256) else 0
+
+
+def late_pays(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int, rounds: int, slack: int) -> bool:
+    """Whether the products of a pair's launch hide the attention that ``late_waves`` would have it carry: the second's workgroups wait for it, and the
+    launch ends later where they have as much to do as the first's.  ``slack``: the blocks of a third of a microsecond that a compute unit has
+    less of theirs; ``rounds``: the workgroups a unit has.  Microseconds a layer against launches apart, 1 / 8 / 32 sequences, by slack:
+
+        150 keys   0: +0.1 / +1.1 / +2.1 (of 28 to 31)    11: -3.0 / -1.5 / -1.5 (of 40)    16: -3.4 / -2.9 / -2.0 (of 20)    22: -4.2 / -1.9 / -1.8 (of 42)
+        500        0: +1.1 / +2.2 / +4.0                  11: -1.5 / +0.8 / +1.5            16: -2.1 / -1.2 / -0.6            22: -3.6 / -0.8 / -0.7
+        900        0: +4.4 / +5.0 / +4.8                  16: +0.7 / +1.8 / +1.9            22: -1.3 / +0.9 / +2.5            32: -3.2 / -0.6 / -0.8
+        1,900      0: +13 / +13 / +13                     22: +6.6 / +6.8 / +11             48: +1.4 / +1.3                   154: -6.4 / -5.5 / +4.6
+
+    So 8 blocks for a short context, 16 for one of 512 keys on average and 20 beyond, 64 past 1,024 keys.  Few pieces beside two workgroups a unit
+    find room without: 96 heads on 8, 480 workgroups, one sequence -2.0 at 30 keys to -5.0 at 900; 80 on 1, 8 sequences, +0.0 to +0.5."""
+    n, _, _, _, bound, mean = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
+    pieces = n * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+    if rounds > 1 and pieces <= 40 and bound <= 1024:
+        return True
+    return slack >= (8 if max_len <= SHORT_CONTEXT else 64 if bound > 1024 else 16 if mean <= 512 else 20)
 
 
 def decode_plan(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0):
@@ -751,7 +770,8 @@ def ride_gain(copies, late, x1: torch.Tensor, stream: torch.Tensor, norm_w: torc
     ctx.new_tokens, ctx.is_decode, ctx.max_len, ctx.mean_len, ctx.extras = [1] * rows, True, RIDE_KEYS, RIDE_KEYS, {}
     trial = ops.LateAttention(draw(rows, nh, d), draw(rows * pages, nkv, 64, d), draw(rows * pages, nkv, d, 64), count(rows * pages).view(rows, pages),
                               ctx, late.slopes, late.scale, waves=waves, **late.how)
-
+    if not ops.late_attention_pays(trial, *copies[0]):
+        return 0.0
     parts = [torch.empty((p, rows, N), dtype=torch.float32, device=x1.device)
              for p, N in zip(ops.gemm_splitk_pair_parts(N1, K1, N2, K2, rows), (N1, N2))]
 
@@ -789,7 +809,12 @@ def ride_gain(copies, late, x1: torch.Tensor, stream: torch.Tensor, norm_w: torc
     return ms(apart) - ms(together)
 
 
-def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor, late=None) -> None:
+def tune_pair_parts(w1: torch.Tensor, w2: torch.Tensor) -> None:
+    """``tune_pair_carrying`` of a pair whose launch carries nothing else."""
+    tune_pair_carrying(w1, w2, None)
+
+
+def tune_pair_carrying(w1: torch.Tensor, w2: torch.Tensor, late) -> None:
     """Once per pair of shapes, while timing is on: the pair launch with the ranges of K that the rule has for the rows, and with
     neighbours of them, with cold caches; ``pick_way`` says which is kept.  Up to 32 rows are timed at 8 and 32; 33 to 64 rows,
     where they have ranges of their own, at 40 and 64, and with workgroups of 128 rows of W (which load the activations half as

@@ -92,7 +92,7 @@ def test_a_decode_step_takes_the_launch(monkeypatch):
     from pytorch_transformers_amd import AutoModelForCausalLM, FalconConfig, ops, tuning
 
     cfg = FalconConfig(num_hidden_layers=3, hidden_size=1024, num_attention_heads=16, multi_query=True, new_decoder_architecture=False, parallel_attn=True,
-                       vocab_size=512, ffn_hidden_size=4096, alibi=False, bias=False)
+                       vocab_size=512, ffn_hidden_size=16384, alibi=False, bias=False)
     model = AutoModelForCausalLM.from_config(cfg, seed=0, std=0.05, dtype="bfloat16", device="cuda:0")
     calls = []
     launch = ops.gemm_splitk_pair_attn

@@ -6,7 +6,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-SHAPE = (1088, 4352, 1088, 1088)  # N, K of a block's last matrices, 17 heads of 64 on one KV head
+SHAPE = (1024, 16384, 1024, 1024)  # N, K of a block's last matrices, 16 heads of 64 on one KV head
 
 
 @pytest.fixture
@@ -29,7 +29,7 @@ def _late(M):
     i32 = lambda *a: torch.arange(*a, dtype=torch.int32, device="cuda")
     ctx = types.SimpleNamespace(cu_tokens=i32(M + 1), seq_start=torch.full((M,), 20, dtype=torch.int32, device="cuda"), n_seqs=M, n_tokens=M, max_len=21, mean_len=21,
                                 is_decode=True, new_tokens=[1] * M, extras={})
-    return ops.LateAttention(draw(M, 17, 64), draw(M, 1, 64, 64), draw(M, 1, 64, 64), i32(M).view(M, 1), ctx, None, 0.125, waves=1)
+    return ops.LateAttention(draw(M, 16, 64), draw(M, 1, 64, 64), draw(M, 1, 64, 64), i32(M).view(M, 1), ctx, None, 0.125, waves=1)
 
 
 def _timed(ops, tuning, M=8):
@@ -39,7 +39,7 @@ def _timed(ops, tuning, M=8):
     with tuning.live_tuning():
         ops.gemm_splitk_pair_attn_ok(x1, w1, late, w2)
     ops.release_flush()
-    return lambda rows: bool(ops.load_library().pta_gemm_splitk_pair_attn_ok(*SHAPE, rows, 17, 1, 64))
+    return lambda rows: bool(ops.load_library().pta_gemm_splitk_pair_attn_ok(*SHAPE, rows, 16, 1, 64))
 
 
 @pytest.mark.parametrize("gain,carried", [(1e3, True), (-1e3, False)])
