@@ -9,7 +9,8 @@
 // A layer's decode step, us, launches apart -> this: 4,544 x 18,176 with 71 heads on one KV head, 1 / 8 / 16 / 32 sequences of 150 keys 102 -> 97.4,
 // 104 -> 100.6, 107.5 -> 104.1, 118.4 -> 115.3 (a wave on a piece's keys), 1 and 8 of 1,900 105 -> 97.5, 109.8 -> 102.7 (four waves, and
 // no merge of ranges); the attention alone takes 4.7 to 8 us there, the merge 4.4.  What is lost of it are the places that attention's workgroups have on
-// the compute units, each for a chain of loads that wait behind the stream: many pieces ride no longer (tuning.py has the line).
+// the compute units, each for a chain of loads that wait behind the stream: many pieces ride no longer, nor any where both
+// products keep a unit about as long, which then ends with the attention instead of beside it (tuning.py has both lines).
 //
 // The wait ends whatever order workgroups start in: one that has looked for a while does what of attention it does not find done itself, which
 // writes the values that stand there or will.
@@ -61,6 +62,12 @@ __device__ __forceinline__ void attend_to(const AttnArgs& a, int place_x, int pl
 #define ATTN_INSIDE 1
 #define ATTN_LATE(more) const AttnMore& more = a.more
 #include "attn_mfma_body.h"
+#undef ATTN_X
+#undef ATTN_Y
+#undef ATTN_Z
+#undef ATTN_NX
+#undef ATTN_INSIDE
+#undef ATTN_LATE
 }
 
 // workgroup t's worth of pieces; KS: waves that share a piece's keys

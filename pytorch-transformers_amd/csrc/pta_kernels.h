@@ -275,6 +275,8 @@ int pta_gemm_splitk_pair_bf16(float* part1, const void* x1, const void* W1, int 
 // sequence, heads of 64, up to 64 sequences, waves (1 or 4) on the keys of sixteen heads.  sync: (sixteens of heads of a KV head) x nkv x M
 // 32-bit zeros; owners: -1, or how many of the attention's workgroups the launch begins with (the products' workgroups do the others: for tests).
 int pta_gemm_splitk_pair_attn_ok(int N1, int K1, int N2, int K2, int M, int nh, int nkv, int d);
+// what tells whether the products hide the attention (tuning.py has the line): rounds, the workgroups that a compute unit has, rounded up; slack, the
+// blocks (64 rows of W, 64 of K) that it has more of the first product than of the second.  0 and 0 where the pair runs in a way that carries none.
 int pta_gemm_splitk_pair_attn_room(int N1, int K1, int N2, int K2, int M, int* rounds, int* slack);
 int pta_gemm_splitk_pair_attn(float* part1, const void* x1, const void* W1, int N1, int K1, float* part2, void* x2, const void* W2, int N2,
                               int K2, int M, const void* q, const void* k_pool, const void* v_pool, const int* block_table, int bt_stride,

@@ -36,7 +36,7 @@ def test_a_step_is_the_launches_one_after_the_other(seqs, heads, groups, N, K, d
     (want, one), (got, two), table, slots = _both(seqs, heads, groups, N, K, dtype)
     cut = heads * N * 64
     assert torch.equal(one[:, cut:], two[:, cut:])  # the tail is moved, not formed
-    # the same sums of N terms in 32 bits, which may be contracted otherwise: N rounding steps at most
+    # sums of N terms in 32 bits: N rounding steps at most (the bits, where heads of a group are a power of two: below)
     torch.testing.assert_close(two[:, :cut], one[:, :cut], rtol=4e-6, atol=4e-6)
     tol = N * 2.0 ** -24 * 8 if dtype == torch.float32 else 2.0 ** -8
     torch.testing.assert_close(got.float(), want.float(), rtol=tol, atol=tol * want.float().abs().max().item())
