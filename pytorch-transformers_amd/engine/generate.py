@@ -206,7 +206,9 @@ def generate(model, prompts: Sequence[Sequence[int]], generation_config: Optiona
         live = list(batch)
         step_no = 0
         try:
-            if ahead:
+            # (one token whose logits are wanted: there is no next step to launch, and waiting for the tokens themselves is
+            # shorter: two 32-bit layers, a batch of 8: 600 us a call, the other way 640)
+            if ahead and (out_logits is None or new_budget > 1):
                 _decode_ahead(model, cache, sampler, cfg, eos, ids, batch, slot_of, feed, out_tokens, new_budget,
                               padded_len, done_with, first_draw, out_logits)
                 live = []

@@ -325,6 +325,18 @@ def test_steps_ahead_choose_the_same_tokens_and_wait_for_none_before_the_next_st
             assert any(what == "step from" for what, _ in log)
 
 
+def test_one_token_with_its_logits_is_not_chosen_ahead_of_the_host():
+    prompts = [[1, 2, 3], [20, 5], [7, 7, 7, 7], [9]]
+    for new, ahead in ((1, False), (2, True)):
+        cfg = GenerationConfig(max_new_tokens=new, output_logits=True, return_dict_in_generate=True)
+        want = generate(ScriptedModel(), prompts, cfg, batch_size=3, sampler=ArgmaxSampler())
+        log = []
+        got = generate(AheadModel(log), prompts, cfg, batch_size=3, sampler=AheadSampler(log))
+        assert got.sequences == want.sequences
+        assert all(torch.equal(a, b) for one, two in zip(got.logits, want.logits) for a, b in zip(one, two))
+        assert any(what == "read" for what, _ in log) == ahead
+
+
 def test_a_sequence_that_ends_on_a_stop_token_takes_part_in_one_step_too_many_and_one_that_ends_by_length_in_none():
     log = []
     m = AheadModel(log)
