@@ -733,10 +733,12 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor, bias=None, act=None, add1=None, a
 
 def gemm_f32_pair_ok(a1: torch.Tensor, w1: torch.Tensor, a2: torch.Tensor, w2: torch.Tensor, add_first: bool = False) -> bool:
     """Whether ``gemm_f32_pair`` (with ``add_first``: ``gemm_f32_pair_sum``) has a launch for these: up to sixteen rows of each."""
+    if a1.dtype != torch.float32 or a1.shape[0] > 16:  # first, as it costs least: a prompt of two 32-bit layers asks four times, 4 us each
+        return False
     if not all(t.dtype == torch.float32 and t.dim() == 2 and t.is_cuda and t.is_contiguous() and t.data_ptr() % 16 == 0
                for t in (a1, w1, a2, w2)):
         return False
-    if a1.shape[0] != a2.shape[0] or a1.shape[0] > 16 or a1.shape[1] != w1.shape[1] or a2.shape[1] != w2.shape[1]:
+    if a1.shape[0] != a2.shape[0] or a1.shape[1] != w1.shape[1] or a2.shape[1] != w2.shape[1]:
         return False
     return bool(load_library().pta_gemm_f32_pair_ok(a1.shape[0], w1.shape[0], w1.shape[1], w2.shape[0], w2.shape[1], int(add_first)))
 
