@@ -258,9 +258,8 @@ static int rotation_stride() {
     static const int env = getenv("PTA_SPLITK_ROT") ? atoi(getenv("PTA_SPLITK_ROT")) : -1;
     return env >= 0 ? env : 1;
 }
-static bool rotated(const SplitkProblem& a, const SplitkProblem& b) {
-    return rotation_stride() > 0 && (a.K % 2048 == 0 || (b.N > 0 && b.K % 2048 == 0));
-}
+static bool crowding(int K) { return rotation_stride() > 0 && K % 2048 == 0; }
+static bool rotated(const SplitkProblem& a, const SplitkProblem& b) { return crowding(a.K) || (b.N > 0 && crowding(b.K)); }
 
 // (x lies within 32-bit offsets: check_splitk)
 static bool rows_too_long(const SplitkProblem& a, const SplitkProblem& b, int rt) { return (long)std::max(a.K, b.K) * 16 * rt * 2 >= LDS_PAST; }
@@ -436,9 +435,10 @@ static double pair_us(int N1, int K1, int a, int N2, int K2, int b, int rt, int 
 
 // Ranges, and tiles of sixteen rows of W a wave, for steps of up to 32 rows (one tile) or of 33 to 64; kept by shape.  96 rows of W on six waves, at 33 to 64
 // rows, are for where 64 or 128 leave compute units idle or with twice the rows of others, as a unit pulls some 25 GB/s whatever is on its
-// way: 4,672 + 18,176 x 4,544 (179 workgroups of 128 rows, 239 of 96), us at 33 / 48 / 64 rows 41.2 -> 38.7, 43.0 -> 39.4, 45.6 -> 41.5; 6,144 + 16,384 x 4,096
-// 38.1 -> 37.7, 38.7 -> 38.3, 40.6 -> 39.5.  They read x more often, and are taken where the time says 5 % less: at 4 % less (4,544 x 4,544 + 18,176) they
-// are 2 % the faster at 33 rows and none at 64, at none less (9,216 + 32,768 x 8,192) 3 % the slower.
+// way: 4,672 + 18,176 x 4,544 (179 workgroups of 128 rows, 239 of 96), us at 33 / 48 / 64 rows 41.2 -> 38.7, 43.0 -> 39.4, 45.6 -> 41.5.  They read x more often,
+// and are taken where the time says 5 % less: at 4 % less (4,544 x 4,544 + 18,176) they are 2 % the faster at 33 rows and none at 64, at none less (9,216 + 32,768 x
+// 8,192) 3 % the slower.  Nor where each tile walks K from a place of its own, which another height of the tiles would change the sums by: 6,144 + 16,384 x 4,096
+// took 38.1 -> 37.7, 38.7 -> 38.3, 40.6 -> 39.5, and steps of 40 and 64 rows of eight such layers 22.47 -> 22.33 and 24.65 -> 24.43 ms, no more than runs differ by.
 static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
     static std::map<std::array<int, 5>, PairChoice> known;
     const std::array<int, 5> key{N1, K1, N2, K2, rows};
@@ -448,7 +448,7 @@ static PairChoice pair_rule(int N1, int K1, int N2, int K2, int rows) {
     PairChoice best{1, 1, 1};
     double us = 1e30;
     for (int rt : {1, 2, PAIR_SIX}) {
-        if (rt > 1 && rows <= 32) continue;
+        if ((rt > 1 && rows <= 32) || (rt == PAIR_SIX && (crowding(K1) || crowding(K2)))) continue;
         for (int a = 1; a <= 8; ++a)
             for (int b = 1; b <= 16; ++b) {
                 if (!parts_valid(K1, a) || !parts_valid(K2, b)) continue;
