@@ -306,9 +306,12 @@ def late_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_le
                        900 keys          +10 / -3.1    +12 / -1.2     +7.7 / -4.7      +13 / -0.9     +6.2 / +5.5
                      1,900 keys          +29 / +1.7    +27 / +2.7      +27 / +1.6      +15 / -9.5     +4.4 / +2.9
 
-    So a wave alone up to ``SHORT_CONTEXT`` where the heads of a KV head fill several pieces (whose waves share its keys), else four; beyond that four
-    waves, up to 2,048 keys where there are few pieces of several a KV head, up to 1,024 where a KV head is one piece.  (One answer for 33 to 64
-    sequences: 40 to 56 of 30 to 190 keys are -1.0 to -4.7, 64 from -0.8 to +3.0.)  A cut that was fixed (``set_decode_plan``) goes before the rule."""
+    So a wave alone up to ``SHORT_CONTEXT``, which is the cut of the launch apart there (``short_cut``), so that a result is the same whether it rides: with
+    up to 320 pieces where the heads of a KV head fill several (whose waves share its keys), with up to 64 where a KV head is one: at 30 / 100 / 190 keys 128 on 8
+    of 1 sequence -2.1 / -1.4 / -2.9 (four waves -1.7 / -3.1 / -3.4), of 8 -1.3 / -0.6 / -1.0 (-0.6 / -1.0 / -1.5), of 12 +0.0 / +1.8 / -0.1; 48 on 6 of 8 -1.1 / -2.3 / -3.6
+    (-0.6 / -1.3 / -2.6).  Beyond that four waves, up to 2,048 keys where there are few pieces of several a KV head, up to 1,024 where a KV head is one piece.  (One
+    answer for 33 to 64 sequences: 40 to 56 of 30 to 190 keys are -1.0 to -4.7, 64 from -0.8 to +3.0.)  A cut that was fixed (``set_decode_plan``) goes
+    before the rule."""
     key = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
     if ops.ATTN_FORCE_SPLIT or ops.ATTN_FORCE_TILES:
         return 0
@@ -316,7 +319,7 @@ def late_waves(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_le
     groups = (n_heads // n_kv_heads + 15) // 16
     pieces = n * n_kv_heads * groups
     if max_len <= SHORT_CONTEXT:
-        return 1 if groups > 1 and pieces <= 320 else 4 if pieces <= 256 else 0
+        return 1 if pieces <= (320 if groups > 1 else 64) else 0
     cut = _active.decode_plans.get(key)
     if cut is not None:
         return 4 if cut[0] == 1 and cut[1] >= max_len and cut[2] == 4 else 0
@@ -333,13 +336,17 @@ def late_pays(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len
         900        0: +4.4 / +5.0 / +4.8                  16: +0.7 / +1.8 / +1.9            22: -1.3 / +0.9 / +2.5            32: -3.2 / -0.6 / -0.8
         1,900      0: +13 / +13 / +13                     22: +6.6 / +6.8 / +11             48: +1.4 / +1.3                   154: -6.4 / -5.5 / +4.6
 
-    So 8 blocks for a short context, 16 for one of 512 keys on average and 20 beyond, 64 past 1,024 keys.  Few pieces beside two workgroups a unit
-    find room without: 96 heads on 8, 480 workgroups, one sequence -2.0 at 30 keys to -5.0 at 900; 80 on 1, 8 sequences, +0.0 to +0.5."""
+    So 8 blocks for a short context, 16 for one of 512 keys on average and 20 beyond, 64 past 1,024 keys.  The 11 and 16 are of four waves on the keys of a KV head
+    of one piece, which take one up to ``SHORT_CONTEXT`` and want 16 then: at 150 keys 11: +0.2 / +1.2, 16: -3.2 / +0.5 (of 20), 22: -1.2 / +0.0.  Few pieces
+    beside two workgroups a unit find room without: 96 heads on 8, 480 workgroups, one sequence -2.0 at 30 keys to -5.0 at 900; 80 on 1, 8 sequences, +0.0 to +0.5."""
     n, _, _, _, bound, mean = decode_key(n_seqs, n_heads, n_kv_heads, head_dim, max_len, mean_len)
-    pieces = n * n_kv_heads * ((n_heads // n_kv_heads + 15) // 16)
+    groups = (n_heads // n_kv_heads + 15) // 16
+    pieces = n * n_kv_heads * groups
     if rounds > 1 and pieces <= 40 and bound <= 1024:
         return True
-    return slack >= (8 if max_len <= SHORT_CONTEXT else 64 if bound > 1024 else 16 if mean <= 512 else 20)
+    if max_len <= SHORT_CONTEXT:
+        return slack >= (8 if groups > 1 else 16)
+    return slack >= (64 if bound > 1024 else 16 if mean <= 512 else 20)
 
 
 def decode_plan(n_seqs: int, n_heads: int, n_kv_heads: int, head_dim: int, max_len: int, mean_len: int = 0):

@@ -55,3 +55,15 @@ def test_ways_that_carry_nothing_have_no_room():
         lib.pta_gemm_splitk_pair_fix(*shapes, 0, 0, 1)
         lib.pta_gemm_splitk_pair_fix_stationary(*shapes, -1, 0, 0)
     assert lib.pta_gemm_splitk_pair_attn_room(0, 64, 64, 64, 1, ctypes.byref(ctypes.c_int()), ctypes.byref(ctypes.c_int())) != 0
+
+
+@pytest.mark.parametrize("nh,nkv", [(71, 1), (16, 1), (128, 8), (64, 8), (32, 8), (13, 13), (48, 6)])
+def test_short_contexts_are_cut_as_by_a_launch_apart(nh, nkv):
+    """Whether attention rides changes no result: up to so many keys a launch apart has one wave on the keys of sixteen heads."""
+    from pytorch_transformers_amd import tuning
+
+    for keys in (1, 60, tuning.SHORT_CONTEXT):
+        bound = tuning.context_bound(keys)
+        assert tuning.short_cut(bound)[2] == 1
+        waves = [tuning.late_waves(n, nh, nkv, 64, bound, keys) for n in (1, 2, 4, 5, 8, 16, 33, 64)]
+        assert set(waves) <= {0, 1} and waves[0] == 1 and waves == sorted(waves, reverse=True)
