@@ -6,8 +6,8 @@
 // which start at once, and ends with those of b, which ask for their first rows of W and then wait until all of attention is done, as
 // it then long is.
 //
-// A layer's decode step, us, launches apart -> this: 4,544 x 18,176 with 71 heads on one KV head, 1 / 8 / 16 / 32 sequences of 150 keys 102 -> 97.4,
-// 104 -> 100.6, 107.5 -> 104.1, 118.4 -> 115.3 (a wave on a piece's keys), 1 and 8 of 1,900 105 -> 97.5, 109.8 -> 102.7 (four waves, and
+// Attention, the pair and the norm behind it, us, launches apart -> this: 4,544 x 18,176 with 71 heads on one KV head, 1 / 8 / 16 / 32 sequences of 150 keys
+// 48.6 -> 45.5, 49.6 -> 47.5, 50.9 -> 49.2, 54.1 -> 52.4 (a wave on a piece's keys), 1 and 8 of 1,900 51.7 -> 46.1, 55.3 -> 50.3 (four waves, and
 // no merge of ranges); the attention alone takes 4.7 to 8 us there, the merge 4.4.  What is lost of it are the places that attention's workgroups have on
 // the compute units, each for a chain of loads that wait behind the stream: many pieces ride no longer, nor any where both
 // products keep a unit about as long, which then ends with the attention instead of beside it (tuning.py has both lines).
